@@ -658,8 +658,20 @@ int ilt_mm_q8_mma2(uint64_t stream, const int8_t* w0, const uint16_t* d0, float*
   // a matrix of no rows (or a null one) takes no part, as in the reference's grid
   const int8_t* ws[3] = {w0, w1, w2}; const uint16_t* ds[3] = {d0, d1, d2}; float* ys[3] = {y0, y1, y2};
   const float* bs[3] = {b0, b1, b2}; const int rows[3] = {rows0, rows1, rows2};
+  // few tokens: the matrices in one launch
+  const uint8_t* fw[3]; const uint16_t* fd[3]; float* fy[3]; const float* fb[3]; int fr[3], fm[3], nm = 0;
   for (int i = 0; i < 3; i++) {
     ILT_REQUIRE(rows[i] >= 0);
+    if (rows[i] == 0 || !ws[i]) continue;
+    ILT_REQUIRE(ds[i] && ys[i] && ((uintptr_t)ws[i] & 15) == 0);
+    fw[nm] = (const uint8_t*)ws[i]; fd[nm] = ds[i]; fy[nm] = ys[i]; fb[nm] = bs[i]; fr[nm] = rows[i]; fm[nm] = ILT_Q8_0; nm++;
+  }
+  if (nm > 1 && n > 0) {
+    ILT_REQUIRE(xq && xs && ((uintptr_t)xq & 15) == 0 && cols > 0 && cols % 32 == 0);
+    const hipError_t e = ilt_k_gemm_i8_few(nm, fm, fw, fd, fr, fy, fb, cols, xq, xs, nullptr, n, acc, S(stream));
+    if (e != hipErrorNotSupported) return (int)e;
+  }
+  for (int i = 0; i < 3; i++) {
     if (rows[i] == 0 || !ws[i]) continue;
     const int e = ilt_mm_q8(stream, ws[i], ds[i], xq, xs, ys[i], bs[i], rows[i], cols, n, acc);
     if (e != ILT_OK) return e;
@@ -705,7 +717,10 @@ int ilt_mm_k_n(uint64_t stream, int type, const void* w0, float* y0, const float
   if (nm == 0 || n == 0) return ILT_OK;
   ILT_REQUIRE(xq && xd && bsums && ((uintptr_t)xq & 15) == 0);
   const long long row_bytes = (long long)cols / 256 * block_bytes(fmt);
-  const hipError_t e = ilt_k_gemm_i8_planes_n(fmt, nm, ws, rows, ys, bs, row_bytes, cols, xq, xd, bsums, n, acc, S(stream));
+  const int fmts[3] = {fmt, fmt, fmt};
+  hipError_t e = ilt_k_gemm_i8_few(nm, fmts, ws, nullptr, rows, ys, bs, cols, xq, xd, bsums, n, acc, S(stream));
+  if (e != hipErrorNotSupported) return (int)e;
+  e = ilt_k_gemm_i8_planes_n(fmt, nm, ws, rows, ys, bs, row_bytes, cols, xq, xd, bsums, n, acc, S(stream));
   if (e != hipErrorNotSupported) return (int)e;
   for (int i = 0; i < nm; i++) {
     const int r = ilt_mm_k(stream, type, ws[i], xq, xd, bsums, ys[i], bs[i], rows[i], cols, n, acc);

@@ -159,6 +159,11 @@ hipError_t ilt_k_moe_sum_rows(int d, int nu, int ntok, const float* down, const 
 hipError_t ilt_k_gemm_i8(int fmt, const uint8_t* w, const uint16_t* wd, long long row_bytes, int rows, int cols,
                          const int8_t* xq, const float* xs, const int* bsums, int ntok, float* y, const float* bias,
                          int acc, hipStream_t st, long long ldy = 0);
+// The same for a few tokens (kernels_gemm_few.hip): up to four matrices, all Q8_0 or Q4_K and Q6_K in any mix, in one launch.
+// hipErrorNotSupported, and nothing launched, where the shapes are not that kernel's.  ldy 0: each matrix's rows.
+hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws, const uint16_t* const* wds, const int* rows, float* const* ys,
+                             const float* const* biases, int cols, const int8_t* xq, const float* xs, const int* bsums, int ntok, int acc,
+                             hipStream_t st, long long ldy = 0);
 // Q6_K, Q4_K and Q2_K, exact, on the pipelined kernel (kernels_gemm_bf16.hip): scale * quant as int8 planes
 hipError_t ilt_k_gemm_i8_planes(int fmt, const uint8_t* w, long long row_bytes, int rows, int cols, const int8_t* xq, const float* xd,
                                 const int* bsums, int ntok, float* y, const float* bias, int acc, hipStream_t st, long long ldy = 0);

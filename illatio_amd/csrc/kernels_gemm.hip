@@ -434,6 +434,10 @@ hipError_t ilt_k_gemm_i8(int fmt, const uint8_t* w, const uint16_t* wd, long lon
   // as int8 planes, the same bits.  ILT_I8_PLANES (tests): "0" never, "1" whenever the format allows.
   const char* force = getenv("ILT_I8_PLANES");
   const int forced = force ? atoi(force) : -1;
+  {
+    const hipError_t e = ilt_k_gemm_i8_few(1, &fmt, &w, &wd, &rows, &y, &bias, cols, xq, xs, bsums, ntok, acc, st, ldy);
+    if (e != hipErrorNotSupported) return e;
+  }
   const bool fits = rows < (1 << 21) && ldy < (1 << 21) && (long long)rows * row_bytes < 0x7FFFFFFFLL;      // the pipelined kernels' 32-bit offsets
   if (fits && (fmt == ILT_Q6_K || fmt == ILT_Q4_K || fmt == ILT_Q2_K) && cols % 256 == 0 && forced != 0 && (forced == 1 || (ntok >= 96 && rows >= 128)))
     return ilt_k_gemm_i8_planes(fmt, w, row_bytes, rows, cols, xq, xs, bsums, ntok, y, bias, acc, st, ldy);
