@@ -1084,6 +1084,147 @@ int ilt_dense_decode(uint64_t stream, const ilt_dense_model* m, const int32_t* t
   return ILT_OK;
 }
 
+// ---- a prompt's chunk through the dense decoder ----------------------------------------------------
+namespace {
+// X (n rows of cols floats; normed by W first unless null) quantized into each format A holds
+int chunk_quant(uint64_t st, const float* x, const float* w, const ilt_dense_act& a, int cols, float eps, int n) {
+  int e;
+  if (a.xq && (e = w ? ilt_rmsnorm_q8(st, x, w, nullptr, a.xq, a.xs, nullptr, cols, eps, n, 0)
+                     : ilt_quant_q8(st, x, a.xq, a.xs, nullptr, (int64_t)n * cols / 32))) return e;
+  if (a.kq && (e = w ? ilt_rmsnorm_q8k(st, x, w, nullptr, a.kq, a.kd, a.ksum, cols, eps, n, 0)
+                     : ilt_quant_q8k(st, x, a.kq, a.kd, a.ksum, (int64_t)n * cols / 256))) return e;
+  return ILT_OK;
+}
+struct ChunkMat { const ilt_dense_mat* w; float* y; const float* bias; };
+int chunk_mul_one(uint64_t st, const ChunkMat& c, const ilt_dense_act& a, int n, int acc) {
+  const ilt_dense_mat& w = *c.w;
+  if (w.gguf_type == ILT_TYPE_Q8_0) return ilt_mm_q8(st, (const int8_t*)w.w, w.wd, a.xq, a.xs, c.y, c.bias, w.rows, w.cols, n, acc);
+  return ilt_mm_k(st, w.gguf_type == ILT_TYPE_Q4_K ? 0 : w.gguf_type == ILT_TYPE_Q6_K ? 2 : -1, w.w, a.kq, a.kd, a.ksum, c.y, c.bias, w.rows, w.cols, n, acc);
+}
+// Up to three products sharing their activations.  Few tokens: one launch.  Else the K-quant matrices of one type in one
+// launch, and what that leaves -- the launches after the first -- on the work's second stream (Q+K is 320 workgroups at 512
+// tokens and V 64: side by side they take what Q+K takes).
+int chunk_mul(const ilt_dense_work& W, int nm, const ChunkMat* c, const ilt_dense_act& a, int n, int acc) {
+  if (nm > 1) {
+    int fmts[3], rows[3]; const uint8_t* ws[3]; const uint16_t* wds[3]; float* ys[3]; const float* bs[3];
+    bool one = true;
+    for (int i = 0; i < nm; i++) {
+      const ilt_dense_mat& w = *c[i].w;
+      fmts[i] = w.gguf_type; rows[i] = w.rows; ws[i] = (const uint8_t*)w.w; wds[i] = w.wd; ys[i] = c[i].y; bs[i] = c[i].bias;
+      one &= w.rows > 0 && w.cols == c[0].w->cols;
+    }
+    const bool q8 = fmts[0] == ILT_TYPE_Q8_0;
+    if (one && (q8 ? a.xq && a.xs : a.kq && a.kd && a.ksum)) {
+      const hipError_t e = ilt_k_gemm_i8_few(nm, fmts, ws, wds, rows, ys, bs, c[0].w->cols, q8 ? a.xq : a.kq, q8 ? a.xs : a.kd, a.ksum, n, acc, S(W.stream));
+      if (e != hipErrorNotSupported) return (int)e;
+    }
+  }
+  bool done[3] = {false, false, false}, beside = false, first = true;
+  // the launch of the first matrix is queued last, so that the others' are on the second stream before it fills the GPU
+  for (int pass = 0; pass < 2; pass++)
+    for (int i = pass == 0 ? 1 : 0; i < nm; i++) {
+      if (done[i]) continue;
+      const ilt_dense_mat& w = *c[i].w;
+      const bool k = w.gguf_type != ILT_TYPE_Q8_0;
+      auto same = [&](int j) { return k && c[j].w->gguf_type == w.gguf_type && c[j].w->cols == w.cols; };
+      if (pass == 0 && same(0)) continue;                   // goes with the first
+      uint64_t st = W.stream;
+      if (pass == 0 && W.second) {
+        if (!beside) {
+          ILT_TRY(hipEventRecord(E(W.forked), S(W.stream)));
+          ILT_TRY(hipStreamWaitEvent(S(W.second), E(W.forked), 0));
+          beside = true;
+        }
+        st = W.second;
+      }
+      ChunkMat g[3]; int ng = 0;
+      for (int j = i; j < nm; j++) if (!done[j] && (j == i || same(j))) { g[ng++] = c[j]; done[j] = true; }
+      int e;
+      if (ng > 1) {
+        const ilt_dense_mat none = {}; const ChunkMat z = {&none, nullptr, nullptr};
+        const ChunkMat& g2 = ng > 2 ? g[2] : z;
+        e = ilt_mm_k_n(st, w.gguf_type == ILT_TYPE_Q4_K ? 0 : w.gguf_type == ILT_TYPE_Q6_K ? 2 : -1, g[0].w->w, g[0].y, g[0].bias, g[0].w->rows, g[1].w->w, g[1].y,
+                       g[1].bias, g[1].w->rows, g2.w->w, g2.y, g2.bias, g2.w->rows, a.kq, a.kd, a.ksum, w.cols, n, acc);
+      } else e = chunk_mul_one(st, g[0], a, n, acc);
+      if (e) return e;
+      if (pass == 1 && first) {
+        first = false;
+        if (beside) ILT_TRY(hipEventRecord(E(W.joined), S(W.second)));
+      }
+    }
+  if (beside) ILT_TRY(hipStreamWaitEvent(S(W.stream), E(W.joined), 0));
+  return ILT_OK;
+}
+}  // namespace
+
+int ilt_dense_chunk(const ilt_dense_model* m, int nparts, const ilt_dense_work* works, const int32_t* tokens, const int* ntok, int pos,
+                    int want_logits, const uint64_t* events) {
+  ILT_REQUIRE(m && works && tokens && ntok && nparts >= 1 && (nparts == 1 || events) && m->layers && m->nl > 0 && pos >= 0 && m->rope);
+  ILT_REQUIRE(!want_logits || (m->logits && m->output_norm));
+  int total = 0;
+  for (int j = 0; j < nparts; j++) {
+    ILT_REQUIRE(ntok[j] >= 1 && works[j].x && works[j].q && works[j].k && works[j].v && works[j].att && works[j].fa && works[j].fb);
+    total += ntok[j];
+  }
+  ILT_REQUIRE(pos + total <= m->nctx);
+  for (int t = 0; t < total; t++) ILT_REQUIRE(tokens[t] >= 0 && tokens[t] < m->embd.rows);
+  const int qd = m->nh * m->hd;
+  int e;
+  if (nparts > 1) {
+    const uint64_t* ends = events + (size_t)(nparts - 1) * m->nl;
+    ILT_TRY(hipEventRecord(E(ends[0]), S(works[0].stream)));
+    for (int j = 1; j < nparts; j++) ILT_TRY(hipStreamWaitEvent(S(works[j].stream), E(ends[0]), 0));
+  }
+  for (int j = 0, t0 = 0; j < nparts; t0 += ntok[j], j++) {
+    const ilt_dense_mat& w = m->embd;
+    ILT_REQUIRE(w.w && w.cols == m->d && block_bytes(w.gguf_type) && m->d % block_weights(w.gguf_type) == 0 && (w.gguf_type != ILT_Q8_0 || w.wd));
+    const long long rb = w.gguf_type == ILT_Q8_0 ? w.cols : (long long)w.cols / 256 * block_bytes(w.gguf_type);
+    ILT_TRY(ilt_k_dequant_ids(w.gguf_type, (const uint8_t*)w.w, w.wd, tokens + t0, ntok[j], m->d, rb, works[j].x, S(works[j].stream)));
+  }
+  for (int l = 0; l < m->nl; l++) {
+    const ilt_dense_layer& L = m->layers[l];
+    for (int j = 0, p = pos; j < nparts; p += ntok[j], j++) {
+      const ilt_dense_work& W = works[j];
+      const int n = ntok[j];
+      if ((e = chunk_quant(W.stream, W.x, L.attn_norm, W.act[0], m->d, m->eps, n))) return e;
+      const ChunkMat qkv[3] = {{&L.wq, W.q, L.bq}, {&L.wk, W.k, L.bk}, {&L.wv, W.v, L.bv}};
+      if ((e = chunk_mul(W, 3, qkv, W.act[0], n, 0))) return e;
+      if ((e = ilt_qk_rope(W.stream, W.q, W.k, W.v, L.q_norm, L.k_norm, m->rope, L.kc, L.vc, m->nh, m->nkv, m->hd, m->rd, p, m->eps, m->neox, n))) return e;
+      if (j < nparts - 1) ILT_TRY(hipEventRecord(E(events[(size_t)j * m->nl + l]), S(W.stream)));
+      for (int i = 0; i < j; i++) ILT_TRY(hipStreamWaitEvent(S(W.stream), E(events[(size_t)i * m->nl + l]), 0));
+    }
+    for (int j = 0, p = pos; j < nparts; p += ntok[j], j++) {
+      const ilt_dense_work& W = works[j];
+      const int n = ntok[j];
+      if ((e = ilt_attn_rows(W.stream, W.q, L.kc, L.vc, W.att, m->nh, m->nkv, m->hd, p, n, p + n <= 8192 ? W.scores : nullptr))) return e;
+      if ((e = chunk_quant(W.stream, W.att, nullptr, W.act[1], qd, 0.0f, n))) return e;
+      if ((e = chunk_mul_one(W.stream, {&L.wo, W.x, nullptr}, W.act[1], n, 1))) return e;
+      if ((e = chunk_quant(W.stream, W.x, L.ffn_norm, W.act[0], m->d, m->eps, n))) return e;
+      const ChunkMat gu[2] = {{&L.gate, W.fa, nullptr}, {&L.up, W.fb, nullptr}};
+      if ((e = chunk_mul(W, 2, gu, W.act[0], n, 0))) return e;
+      const ilt_dense_act& f = W.act[2];
+      if (f.kq && !f.xq) {
+        if ((e = ilt_swiglu_quant_q8k(W.stream, W.fa, W.fb, f.kq, f.kd, f.ksum, (int64_t)n * m->ffn / 256))) return e;
+      } else {
+        if ((e = ilt_swiglu(W.stream, W.fa, W.fb, (int64_t)n * m->ffn))) return e;
+        if ((e = chunk_quant(W.stream, W.fa, nullptr, f, m->ffn, 0.0f, n))) return e;
+      }
+      if ((e = chunk_mul_one(W.stream, {&L.down, W.x, nullptr}, f, n, 1))) return e;
+    }
+  }
+  if (want_logits) {
+    const ilt_mv_desc head = mv_of(m->output, m->logits);
+    const ilt_dense_work& W = works[nparts - 1];
+    if ((e = ilt_mv_multi_norm(W.stream, 1, &head, m->d, W.x + (size_t)(ntok[nparts - 1] - 1) * m->d, m->output_norm, m->eps, 0, 1, 0))) return e;
+  }
+  for (int j = 1; j < nparts; j++) {
+    const uint64_t end = events[(size_t)(nparts - 1) * m->nl + j];
+    ILT_TRY(hipEventRecord(E(end), S(works[j].stream)));
+    ILT_TRY(hipStreamWaitEvent(S(works[0].stream), E(end), 0));
+  }
+  return ILT_OK;
+}
+
 // rope-table (model.lisp:218-231) for positions pos0 .. pos0 + n - 1, on the host: a position's head_dim/2 cosines
 // then head_dim/2 sines, theta advanced by repeated single-float multiplication, theta-scale, cos and sin through
 // double and rounded to single as SBCL evaluates them.  The only float arithmetic this file does: model constants,

@@ -139,6 +139,9 @@ hipError_t ilt_k_read_through(const unsigned long long* srcs, const unsigned lon
                               hipStream_t st);
 hipError_t ilt_k_dequant_rows(int fmt, const uint8_t* w, const uint16_t* wd, const int* rows_idx, long long nrows,
                               int cols, long long row_bytes, float* out, hipStream_t st);
+// rows host_ids[0..n) (host memory, read during the call) of the matrix as floats
+hipError_t ilt_k_dequant_ids(int fmt, const uint8_t* w, const uint16_t* wd, const int* host_ids, int n, int cols, long long row_bytes, float* out,
+                             hipStream_t st);
 
 hipError_t ilt_k_route(int ne, int nu, int hash, float scale, int has_bias, const float* logits, const float* bias,
                        const int* tid2eid, const uint32_t* tokens, uint32_t* sel, float* wout, int ntok, hipStream_t st);

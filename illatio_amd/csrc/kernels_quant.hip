@@ -201,6 +201,17 @@ __global__ __launch_bounds__(256) void dequant_rows_kernel(int fmt, const u8* __
     out[n * cols + col] = dequant_one(fmt, wrow, wdrow, col);
 }
 
+// The rows of up to 512 ids that come with the launch: a prompt's embedding without the ids' copy to the device and the
+// wait that a copy from ordinary host memory is (a chunk's launches stay queued one after another).
+struct RowIds { int id[512]; };
+__global__ __launch_bounds__(256) void dequant_ids_kernel(int fmt, const u8* __restrict__ w, const u16* __restrict__ wd, RowIds ids, int cols,
+                                                          long long row_bytes, float* __restrict__ out) {
+  const long long n = blockIdx.y, r = ids.id[blockIdx.y];
+  const u8* wrow = w + r * row_bytes;
+  const u16* wdrow = wd ? wd + r * (cols >> 5) : nullptr;
+  for (int col = blockIdx.x * 256 + threadIdx.x; col < cols; col += gridDim.x * 256)
+    out[n * cols + col] = dequant_one(fmt, wrow, wdrow, col);
+}
 
 // y[t*y_stride + r] = W[r] . x[t*x_stride ..] for an F16 matrix and float activations (the router's product,
 // ds4f_mm.cu:253; CPU: f32mm!, ds4f.lisp:278-293).  Each dot is F32-DOT16's (tensor.lisp:370-378): column i's
@@ -312,6 +323,18 @@ hipError_t ilt_k_dequant_rows(int fmt, const uint8_t* w, const uint16_t* wd, con
     hipLaunchKernelGGL(dequant_rows_kernel, dim3(gx, gy), dim3(256), 0, st, fmt, w, wd,
                        rows_idx ? rows_idx + n0 : nullptr, cols, row_bytes, out + n0 * cols);
     if (!rows_idx) w += 65535 * row_bytes, wd = wd ? wd + 65535LL * (cols >> 5) : nullptr;
+  }
+  return hipGetLastError();
+}
+
+hipError_t ilt_k_dequant_ids(int fmt, const uint8_t* w, const uint16_t* wd, const int* host_ids, int n, int cols, long long row_bytes, float* out,
+                             hipStream_t st) {
+  const unsigned gx = (unsigned)min((cols + 255) / 256, 64);
+  for (int n0 = 0; n0 < n; n0 += 512) {
+    RowIds ids = {};
+    const int k = min(n - n0, 512);
+    for (int i = 0; i < k; i++) ids.id[i] = host_ids[n0 + i];
+    hipLaunchKernelGGL(dequant_ids_kernel, dim3(gx, k), dim3(256), 0, st, fmt, w, wd, ids, cols, row_bytes, out + (long long)n0 * cols);
   }
   return hipGetLastError();
 }

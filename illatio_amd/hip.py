@@ -266,6 +266,14 @@ def hip_stream_sync(stream):
     call("ilt_stream_sync", C.c_uint64(stream))
 
 
+def second_of(dev):
+    """DEV with its second stream and the two events of fork and join, made when they are first wanted."""
+    if getattr(dev, "second", None) is None:
+        dev.second = hip_stream_create(dev)
+        dev.forked, dev.joined = hip_event_create(dev), hip_event_create(dev)
+    return dev
+
+
 class beside:
     """with beside(dev): what is queued inside goes to DEV's second stream, which first waits for everything DEV's
     stream holds so far; rejoin(dev) then makes DEV's stream wait for it.  For launches that do not depend on each
@@ -276,10 +284,7 @@ class beside:
         self.dev = dev
 
     def __enter__(self):
-        dev = self.dev
-        if getattr(dev, "second", None) is None:
-            dev.second = hip_stream_create(dev)
-            dev.forked, dev.joined = hip_event_create(dev), hip_event_create(dev)
+        dev = second_of(self.dev)
         hip_event_record(dev.forked, dev.stream)
         hip_stream_wait(dev.second, dev.forked)
         self.main, dev.stream = dev.stream, dev.second

@@ -77,6 +77,14 @@ class _Model(C.Structure):
                [(n, C.c_uint64) for n in ("x", "q", "k", "v", "att", "fa", "scores", "logits")]
 
 
+class _Act(C.Structure):
+    _fields_ = [(n, C.c_uint64) for n in ("xq", "xs", "kq", "kd", "ksum")]
+
+
+class _WorkC(C.Structure):
+    _fields_ = [(n, C.c_uint64) for n in ("stream", "second", "forked", "joined", "x", "q", "k", "v", "att", "fa", "fb", "scores")] + [("act", _Act * 3)]
+
+
 def _mat(w):
     return _Mat(w.type, w.rows, w.cols, w.qs.ptr, w.d.ptr if w.d else 0)
 
@@ -140,7 +148,7 @@ class DenseModel:
             raise ValueError("the bf16 prefill multiplies K-quant matrices; this model has Q8_0 ones")
         # the buffers a chunk goes through the layers in (more sets, each on a stream of its own, are made when the
         # parts of a chunk first go side by side: eval_tokens)
-        self.work, self.more_work, self._keys_ev, self._join_ev = self._work_set(dev, chunk), [], [], []
+        self.work, self.more_work, self._events = self._work_set(dev, chunk), [], []
         w = self.work
         self.x, self.q, self.k, self.v, self.att, self.fa, self.fb = w.x, w.q, w.k, w.v, w.att, w.fa, w.fb
         self.tokens, self.scores, self.acts, self.xb = w.tokens, w.scores, w.acts, w.xb
@@ -193,14 +201,32 @@ class DenseModel:
         n = len(tokens)
         if n < 1 or n > self.chunk or self.pos + n > self.nctx:
             raise ValueError(f"{n} tokens at position {self.pos}: the chunk holds {self.chunk}, the context {self.nctx}")
-        for _ in self._steps(tokens, self.pos, logits, self.work):
-            pass
+        if n > 1 and self.prefill == "exact":
+            self._chunk([tokens], logits, [self.work])
+        else:
+            for _ in self._steps(tokens, self.pos, logits, self.work):
+                pass
         self.pos += n
         return self.logits
 
+    def _chunk(self, parts, logits, works, events=None):
+        """An exact chunk, PARTS (lists of tokens) in WORKS, queued by one call into the library (ilt_dense_chunk): the
+        launches of a layer from Python, a call each, took the host 0.5 ms a layer, twice what a short prompt takes the GPU."""
+        c, ptr = self.c, lambda b: b.ptr if b is not None else 0
+        cw = (_WorkC * len(works))()
+        for j, w in enumerate(works):
+            dev = hip.second_of(w.dev) if dense.BESIDE else w.dev
+            acts = [_Act(*[ptr(b) for b in (a.xq, a.xs, a.kq, a.kd, a.ksum)]) for a in (w.acts[c["d"]], w.acts[self.qd], w.acts[c["ffn"]])]
+            side = (dev.second, dev.forked, dev.joined) if dense.BESIDE else (0, 0, 0)
+            cw[j] = _WorkC(dev.stream, *side, w.x.ptr, w.q.ptr, w.k.ptr, w.v.ptr, w.att.ptr, w.fa.ptr, w.fb.ptr, w.scores.ptr, (_Act * 3)(*acts))
+        ids = np.ascontiguousarray([t for part in parts for t in part], np.int32)
+        hip.call("ilt_dense_chunk", C.byref(self._cmodel), C.c_int(len(parts)), cw, ids.ctypes.data_as(C.c_void_p), (C.c_int * len(parts))(*map(len, parts)),
+                 C.c_int(self.pos), C.c_int(1 if logits else 0), (C.c_uint64 * len(events))(*events) if events else None)
+
     def _steps(self, tokens, pos, logits, W):
-        """forward_n's launches for TOKENS at positions POS.. in the work set W, as a generator: it yields ("keys", layer)
-        when a layer's keys and values are queued for the caches and ("layer", layer) when the layer is."""
+        """forward_n's launches for one token, or for a chunk through the bf16 products, TOKENS at positions POS.. in the work set
+        W, as a generator: it yields ("keys", layer) when a layer's keys and values are queued for the caches and
+        ("layer", layer) when the layer is."""
         dev, c, n = W.dev, self.c, len(tokens)
         d, ffn, hd, nh, nkv, eps = c["d"], c["ffn"], c["hd"], c["nh"], c["nkv"], c["eps"]
         S = C.c_uint64(dev.stream)
@@ -211,7 +237,6 @@ class DenseModel:
             hip.call("ilt_dense_decode", S, C.byref(self._cmodel), P(W.tokens), C.c_int(pos), C.c_int(1 if logits else 0))
             return
         dense.embed(dev, self.embd, W.tokens, W.x, n, d)
-        fast = self.prefill != "exact" and n > 1
         slabs = self.prefill == "bf16-resident"
 
         def mul_fast(li, parts, act, acc=False):
@@ -237,25 +262,13 @@ class DenseModel:
                 for pt in parts:
                     run(*pt)
 
-        def gated():
-            """The chunk's gated activations as the down product reads them: swiglu and the quantizer in one launch, or
-            (a model with Q8_0 matrices) one after the other."""
-            a = dense.swiglu_quantize_act(dev, W.fa, W.fb, W.acts[ffn], n)
-            if a is None:
-                hip.call("ilt_swiglu", S, P(W.fa), P(W.fb), C.c_int64(n * ffn))
-                a = dense.quantize_act(dev, W.fa, W.acts[ffn], n=n)
-            return a
-
         for li, L in enumerate(self.layers):
             if n == 1:
                 dense.qkv_mul(dev, L["wq"], L["wk"], L["wv"], None, W.q, W.k, W.v, L["bq"], L["bk"], L["bv"], xf=W.x,
                               norm=(L["attn_norm"], eps))
             else:
                 a = dense.rmsnorm_q8(dev, W.x, L["attn_norm"], W.acts[d], d, eps, n=n)
-                if fast:
-                    mul_fast(li, [("wq", W.q, L["bq"]), ("wk", W.k, L["bk"]), ("wv", W.v, L["bv"])], a)
-                else:
-                    dense.cmat_mul_n(dev, [(L["wq"], W.q, L["bq"]), (L["wk"], W.k, L["bk"]), (L["wv"], W.v, L["bv"])], a, n)
+                mul_fast(li, [("wq", W.q, L["bq"]), ("wk", W.k, L["bk"]), ("wv", W.v, L["bv"])], a)
             if n == 1 and scratch is not None:
                 hip.call("ilt_attn_step", S, P(W.q), P(W.k), P(W.v), P(L["q_norm"]), P(L["k_norm"]), P(self.rope), P(L["kc"]), P(L["vc"]),
                          P(W.att), C.c_int(nh), C.c_int(nkv), C.c_int(hd), C.c_int(hd), C.c_int(pos), C.c_float(eps),
@@ -271,15 +284,10 @@ class DenseModel:
                 dense.mv_multi(dev, [(L["wo"], W.x, None)], xf=W.att, acc=True)
                 dense.glu_mul(dev, L["gate"], L["up"], None, W.fa, xf=W.x, norm=(L["ffn_norm"], eps))
                 dense.mv_multi(dev, [(L["down"], W.x, None)], xf=W.fa, acc=True)
-            elif fast:
+            else:
                 mul_fast(li, [("wo", W.x, None)], dense.quantize_act(dev, W.att, W.acts[self.qd], n=n), acc=True)
                 mul_fast(li, [("gate", W.fa, None), ("up", W.fb, None)], dense.rmsnorm_q8(dev, W.x, L["ffn_norm"], W.acts[d], d, eps, n=n))
-                mul_fast(li, [("down", W.x, None)], gated(), acc=True)
-            else:
-                dense.cmat_mul(dev, L["wo"], dense.quantize_act(dev, W.att, W.acts[self.qd], n=n), W.x, n=n, acc=True)
-                a = dense.rmsnorm_q8(dev, W.x, L["ffn_norm"], W.acts[d], d, eps, n=n)
-                dense.cmat_mul_n(dev, [(L["gate"], W.fa, None), (L["up"], W.fb, None)], a, n)
-                dense.cmat_mul(dev, L["down"], gated(), W.x, n=n, acc=True)
+                mul_fast(li, [("down", W.x, None)], dense.swiglu_quantize_act(dev, W.fa, W.fb, W.acts[ffn], n), acc=True)
             yield ("layer", li)
         if logits:
             last = hip.DBuf(W.x.ptr + 4 * (n - 1) * d, 4 * d, dev)
@@ -325,29 +333,36 @@ class DenseModel:
             dev2 = copy.copy(dev)
             dev2.stream, dev2.second = hip.hip_stream_create(dev), None
             self.more_work.append(self._work_set(dev2, ((self.chunk + 1) // 2 + 127) // 128 * 128))      # (a part: up to half a chunk, rounded up to whole tiles of 128 tokens)
-        while len(self._keys_ev) < k:
-            self._keys_ev.append([hip.hip_event_create(dev) for _ in self.layers])
-            self._join_ev.append(hip.hip_event_create(dev))
         works = [self.work] + self.more_work[:k - 1]
-        hip.hip_event_record(self._join_ev[0], dev.stream)            # the other streams after what this one holds so far
+        parts = [tokens[j * per:(j + 1) * per] for j in range(k)]
+        # (the events of a chunk of k parts: one a part but the last and layer, then one a part)
+        nl = len(self.layers)
+        while len(self._events) < (k - 1) * nl + k:
+            self._events.append(hip.hip_event_create(dev))
+        if self.prefill == "exact":
+            self._chunk(parts, logits, works, self._events[:(k - 1) * nl + k])
+            self.pos += n
+            return self.logits
+        ends = self._events[(k - 1) * nl:]
+        hip.hip_event_record(ends[0], dev.stream)                     # the other streams after what this one holds so far
         for w in works[1:]:
-            hip.hip_stream_wait(w.dev.stream, self._join_ev[0])
-        gens = [self._steps(tokens[j * per:(j + 1) * per], self.pos + j * per, logits and j == k - 1, works[j]) for j in range(k)]
-        for li in range(len(self.layers)):
+            hip.hip_stream_wait(w.dev.stream, ends[0])
+        gens = [self._steps(parts[j], self.pos + j * per, logits and j == k - 1, works[j]) for j in range(k)]
+        for li in range(nl):
             for j in range(k):
                 assert next(gens[j]) == ("keys", li)
                 if j < k - 1:
-                    hip.hip_event_record(self._keys_ev[j][li], works[j].dev.stream)
+                    hip.hip_event_record(self._events[j * nl + li], works[j].dev.stream)
                 for i in range(j):
-                    hip.hip_stream_wait(works[j].dev.stream, self._keys_ev[i][li])
+                    hip.hip_stream_wait(works[j].dev.stream, self._events[i * nl + li])
             for j in range(k):
                 assert next(gens[j]) == ("layer", li)
         for g in gens:
             for _ in g:
                 pass
         for j in range(1, k):
-            hip.hip_event_record(self._join_ev[j], works[j].dev.stream)
-            hip.hip_stream_wait(dev.stream, self._join_ev[j])
+            hip.hip_event_record(ends[j], works[j].dev.stream)
+            hip.hip_stream_wait(dev.stream, ends[j])
         self.pos += n
         return self.logits
 
@@ -404,8 +419,8 @@ class DenseModel:
                 hip.hip_event_destroy(w.dev.forked)
                 hip.hip_event_destroy(w.dev.joined)
             hip.hip_stream_destroy(w.dev.stream)
-        for e in [e for evs in self._keys_ev for e in evs] + self._join_ev:
+        for e in self._events:
             hip.hip_event_destroy(e)
-        self.more_work, self._keys_ev, self._join_ev = [], [], []
+        self.more_work, self._events = [], []
         for b in self.wb.values():
             hip.hip_free(b)

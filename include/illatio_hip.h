@@ -389,6 +389,28 @@ typedef struct ilt_dense_model {
   float *x, *q, *k, *v, *att, *fa, *scores, *logits;          /* d, nh*hd, nkv*hd, nkv*hd, nh*hd, ffn, nh*((pos+4)&~3), vocab floats */
 } ilt_dense_model;
 int ilt_dense_decode(uint64_t stream, const ilt_dense_model* m, const int32_t* token, int pos, int want_logits);
+/* A prompt's chunk through the whole decoder in one call, each token with the bits of its own ilt_dense_decode: what
+   cuda-forward-n queues for several tokens (cuda-dense.lisp:380-432) -- embedding, then per layer the norm and quantizer,
+   the Q/K/V products, qk_rope, attn_rows, wo onto the residual, the norm, gate and up, the gated activation, down -- and
+   (want_logits) the last token's output norm and head into m->logits.  The chunk's tokens are positions pos .. ; they come
+   as nparts consecutive parts, part j ntok[j] token ids at tokens + the parts before it (host memory, read during the
+   call) in buffers and on a stream of its own (works[j]), its attention in a layer waiting for the earlier parts' keys
+   and values of that layer: events[j * nl + l], recorded on part j's stream (j < nparts - 1).  More than one part:
+   works[1..]'s streams first wait for what works[0]'s holds (events behind the keys' ones: events[(nparts - 1) * nl] is
+   recorded for that), and works[0]'s waits for part j's end, events[(nparts - 1) * nl + j].  One part: events may be null.
+   second, forked, joined: a stream beside the work's own and two events, for products that share their activations and
+   do not fill the GPU one by one, or zeros (all on the one stream).  act[0] holds the quantized activations of width d,
+   act[1] of nh * hd, act[2] of ffn, in the formats their matrices take (Q8_0's xq and xs, the K-quants' kq, kd and ksum;
+   a format nobody takes: nulls).  scores: ntok * nh * ((pos + ntok + 3) & ~3) floats for contexts of up to 8192
+   positions, not read past that.  No counterpart in the reference, whose host queues the launches one by one. */
+typedef struct ilt_dense_act { int8_t* xq; float* xs; int8_t* kq; float* kd; int32_t* ksum; } ilt_dense_act;
+typedef struct ilt_dense_work {
+  uint64_t stream, second, forked, joined;
+  float *x, *q, *k, *v, *att, *fa, *fb, *scores;
+  ilt_dense_act act[3];
+} ilt_dense_work;
+int ilt_dense_chunk(const ilt_dense_model* m, int nparts, const ilt_dense_work* works, const int32_t* tokens, const int* ntok, int pos,
+                    int want_logits, const uint64_t* events);
 int ilt_swiglu(uint64_t stream, float* a, const float* b, int64_t n);
 /* ilt_swiglu followed by ilt_quant_q8k in one launch, for a prompt chunk whose gated activations only the down product
    reads (GLU-MUL's "swiglu" launch, cuda-dense.lisp:338-339, and the quantizing launch that follows it in
