@@ -533,6 +533,27 @@ __device__ __forceinline__ void stage_q8k_from_f32(const float* __restrict__ x, 
 // NP passes of the workgroup's first 256 threads over the blocks' float4s from c0 on: every pass's loads are asked for
 // before the first is quantized (a pass a trip to memory otherwise), without a branch around any of them (past the
 // end: the last float4 again; nothing is stored for it).
+// One float4 of a block, number C of N8, weighted already: its block's scale by the block's eight lanes, and its four quants.
+__device__ __forceinline__ void q8_store(const float4& w, int c, int n8, int f16_scale, i8* lxq, float* lxs, int* xsum) {
+  float amax = fmaxf(fmaxf(fabsf(w.x), fabsf(w.y)), fmaxf(fabsf(w.z), fabsf(w.w)));
+  amax = fmaxf(amax, ilt_dppf<ILT_DPP_XOR1>(amax));
+  amax = fmaxf(amax, ilt_dppf<ILT_DPP_XOR2>(amax));
+  amax = fmaxf(amax, ilt_dppf<ILT_DPP_HALF_MIRROR>(amax));
+  const float d = amax / 127.0f;
+  const float id = d == 0.0f ? 0.0f : 1.0f / d;
+  const int q0 = (int)rintf(w.x * id), q1 = (int)rintf(w.y * id), q2 = (int)rintf(w.z * id), q3 = (int)rintf(w.w * id);
+  const int qs = xsum ? ilt_sum8(q0 + q1 + q2 + q3) : 0;
+  if (c < n8) {
+    *(int*)(lxq + 4 * c) = (q0 & 0xFF) | ((q1 & 0xFF) << 8) | ((q2 & 0xFF) << 16) | ((q3 & 0xFF) << 24);
+    if ((c & 7) == 0) {
+      lxs[c >> 3] = f16_scale ? __half2float(__float2half_rn(d)) : d;
+      if (xsum) xsum[c >> 3] = qs;
+    }
+  }
+}
+__device__ __forceinline__ float4 norm_weighted(const float4& x, float nscale, const float4& n) {
+  return make_float4((x.x * nscale) * n.x, (x.y * nscale) * n.y, (x.z * nscale) * n.z, (x.w * nscale) * n.w);
+}
 template <int NP>
 __device__ __forceinline__ void stage_q8_passes(const float* __restrict__ x, int n8, int c0, int f16_scale, i8* lxq, float* lxs, int* xsum,
                                                 const float* __restrict__ nw, float nscale, float* __restrict__ h, int tid, int nthreads) {
@@ -549,24 +570,10 @@ __device__ __forceinline__ void stage_q8_passes(const float* __restrict__ x, int
     const int c = c0 + i * nthreads + tid;
     float4 w = v[i];
     if (nw) {
-      w = make_float4((w.x * nscale) * n[i].x, (w.y * nscale) * n[i].y, (w.z * nscale) * n[i].z, (w.w * nscale) * n[i].w);
+      w = norm_weighted(w, nscale, n[i]);
       if (h && c < n8) *(float4*)(h + 4 * c) = w;
     }
-    float amax = fmaxf(fmaxf(fabsf(w.x), fabsf(w.y)), fmaxf(fabsf(w.z), fabsf(w.w)));
-    amax = fmaxf(amax, ilt_dppf<ILT_DPP_XOR1>(amax));
-    amax = fmaxf(amax, ilt_dppf<ILT_DPP_XOR2>(amax));
-    amax = fmaxf(amax, ilt_dppf<ILT_DPP_HALF_MIRROR>(amax));
-    const float d = amax / 127.0f;
-    const float id = d == 0.0f ? 0.0f : 1.0f / d;
-    const int q0 = (int)rintf(w.x * id), q1 = (int)rintf(w.y * id), q2 = (int)rintf(w.z * id), q3 = (int)rintf(w.w * id);
-    const int qs = xsum ? ilt_sum8(q0 + q1 + q2 + q3) : 0;
-    if (c < n8) {
-      *(int*)(lxq + 4 * c) = (q0 & 0xFF) | ((q1 & 0xFF) << 8) | ((q2 & 0xFF) << 16) | ((q3 & 0xFF) << 24);
-      if ((c & 7) == 0) {
-        lxs[c >> 3] = f16_scale ? __half2float(__float2half_rn(d)) : d;
-        if (xsum) xsum[c >> 3] = qs;
-      }
-    }
+    q8_store(w, c, n8, f16_scale, lxq, lxs, xsum);
   }
 }
 // TID, NTHREADS: the threads that stage (a multiple of 8, eight lanes a block), numbered from 0: the workgroup's first
@@ -1010,6 +1017,28 @@ __device__ __forceinline__ float norm_scale_stagers(double part, const float* __
   return 1.0f / sqrtf((float)v);
 }
 
+// Q8_0 activations normalized first, by the kStagers waves: up to 1,024 NP floats, x and the norm's weights in registers
+// from the one time they are read (read again after the squares they would come in behind the row waves' loads).
+constexpr int kQ8NormCols = 4096;
+template <int NP>
+__device__ __forceinline__ void stage_q8_normed(const float* __restrict__ x, const float* __restrict__ nw, int cols, float eps, int seq, int f16_scale,
+                                                i8* lxq, float* lxs, u32* meet) {
+  const int n8 = cols / 4, tid = (int)threadIdx.x;
+  float4 v[NP], n[NP];
+  double sq = 0.0;
+#pragma unroll
+  for (int i = 0; i < NP; i++) {
+    const int cc = min(256 * i + tid, n8 - 1);
+    v[i] = *(const float4*)(x + 4 * cc);
+    n[i] = *(const float4*)(nw + 4 * cc);
+  }
+#pragma unroll
+  for (int i = 0; i < NP; i++) sq += 256 * i + tid < n8 ? sq4(v[i]) : 0.0;
+  const float nscale = norm_scale_stagers(sq, x, cols, eps, seq, meet);
+#pragma unroll
+  for (int i = 0; i < NP; i++) q8_store(norm_weighted(v[i], nscale, n[i]), 256 * i + tid, n8, f16_scale, lxq, lxs, nullptr);
+}
+
 // Calls f(integral_constant<int, FMT>) for the format FMT of a matrix.
 template <int FSET, typename F>
 __device__ __forceinline__ void with_format(int fmt, F&& f) {
@@ -1124,6 +1153,9 @@ __global__ __launch_bounds__(kStreamThreads) void gemv_stream_kernel(IltGemvPara
         const int e = k * 64 + lane;
         if (e < p.route.ne) { r_lg[k] = p.route.logits[e]; if (p.route.bias) r_bs[k] = p.route.bias[e]; }
       }
+    } else if (p.xf && p.norm_w) {
+      if (p.cols <= 1024) stage_q8_normed<1>(p.xf, p.norm_w, p.cols, p.eps, p.norm_seq, p.f16_scale, lxq, lxs, s_meet);
+      else stage_q8_normed<kQ8NormCols / 1024>(p.xf, p.norm_w, p.cols, p.eps, p.norm_seq, p.f16_scale, lxq, lxs, s_meet);
     } else if (p.xf) {
       if (routing) stage_q8_from_f32(p.xf, S, p.f16_scale, lxq, lxs, nullptr, nullptr, 1.0f, nullptr, (int)threadIdx.x - 64, 64 * (kStagers - 1));
       else stage_q8_from_f32(p.xf, S, p.f16_scale, lxq, lxs);
@@ -1399,7 +1431,7 @@ static hipError_t gemv_stream_launch(IltGemvParams& p, int fset, int nz, hipStre
   if (experts ? !(fset == ILT_IQ2_XXS || fset == ILT_Q2_K) : !(fset == 0 || fset == ILT_Q4_K || fset == ILT_Q6_K || q8)) return hipErrorNotSupported;
   if (p.group_rows > 0 || (!experts && nz != 1) || (!experts && !q8 && p.glu > 1) || (experts && (p.norm_w || !(p.x_stride == 0 || p.x_stride == p.cols))))
     return hipErrorNotSupported;
-  if (q8 && (p.norm_w || (p.cols / 32) % 2 != 0)) return hipErrorNotSupported;      // the scales go four bytes at a time
+  if (q8 && ((p.norm_w && (p.cols > kQ8NormCols || p.route.logits)) || (p.cols / 32) % 2 != 0)) return hipErrorNotSupported;      // (the scales go four bytes at a time)
   const int S = q8 ? p.cols / 32 : p.cols / 256;
   const int nx = p.x_stride ? nz : 1;
   if (!q8 && (p.xf && p.norm_w ? S > 64 : (long)S * nx > 64 * 3)) return hipErrorNotSupported;
