@@ -716,11 +716,11 @@ int ilt_mm_k_n(uint64_t stream, int type, const void* w0, float* y0, const float
   }
   if (nm == 0 || n == 0) return ILT_OK;
   ILT_REQUIRE(xq && xd && bsums && ((uintptr_t)xq & 15) == 0);
-  const long long row_bytes = (long long)cols / 256 * block_bytes(fmt);
   const int fmts[3] = {fmt, fmt, fmt};
   hipError_t e = ilt_k_gemm_i8_few(nm, fmts, ws, nullptr, rows, ys, bs, cols, xq, xd, bsums, n, acc, S(stream));
   if (e != hipErrorNotSupported) return (int)e;
-  e = ilt_k_gemm_i8_planes_n(fmt, nm, ws, rows, ys, bs, row_bytes, cols, xq, xd, bsums, n, acc, S(stream));
+  const char* planes = getenv("ILT_I8_PLANES");
+  if (!(planes && planes[0] == '0')) e = ilt_k_gemm_i8_reg(nm, fmts, ws, rows, ys, bs, cols, xq, xd, bsums, n, acc, S(stream));
   if (e != hipErrorNotSupported) return (int)e;
   for (int i = 0; i < nm; i++) {
     const int r = ilt_mm_k(stream, type, ws[i], xq, xd, bsums, ys[i], bs[i], rows[i], cols, n, acc);
@@ -1115,7 +1115,8 @@ int chunk_mul(const ilt_dense_work& W, int nm, const ChunkMat* c, const ilt_dens
     }
     const bool q8 = fmts[0] == ILT_TYPE_Q8_0;
     if (one && (q8 ? a.xq && a.xs : a.kq && a.kd && a.ksum)) {
-      const hipError_t e = ilt_k_gemm_i8_few(nm, fmts, ws, wds, rows, ys, bs, c[0].w->cols, q8 ? a.xq : a.kq, q8 ? a.xs : a.kd, a.ksum, n, acc, S(W.stream));
+      hipError_t e = ilt_k_gemm_i8_few(nm, fmts, ws, wds, rows, ys, bs, c[0].w->cols, q8 ? a.xq : a.kq, q8 ? a.xs : a.kd, a.ksum, n, acc, S(W.stream));
+      if (e == hipErrorNotSupported && !q8) e = ilt_k_gemm_i8_reg(nm, fmts, ws, rows, ys, bs, c[0].w->cols, a.kq, a.kd, a.ksum, n, acc, S(W.stream));
       if (e != hipErrorNotSupported) return (int)e;
     }
   }

@@ -430,17 +430,20 @@ hipError_t ilt_k_gemm_i8(int fmt, const uint8_t* w, const uint16_t* wd, long lon
   if (ntok <= 0 || rows <= 0) return hipSuccess;
   if (ldy == 0) ldy = rows;
   if (ldy < rows) return hipErrorInvalidValue;
-  // Q6_K, Q4_K and Q2_K with enough tokens and rows to fill 128 x 128 tiles: the pipelined kernel with scale * quant
-  // as int8 planes, the same bits.  ILT_I8_PLANES (tests): "0" never, "1" whenever the format allows.
+  // The kernels of few tokens and of operands in registers (Q6_K, Q4_K) have rules of their own; Q2_K and Q8_0 with enough
+  // tokens and rows to fill 128 x 128 tiles take pipelined kernels, the same bits.  ILT_I8_PLANES (tests): "0" none of
+  // them, "1" the pipelined ones and the registers' whenever the format allows.
   const char* force = getenv("ILT_I8_PLANES");
   const int forced = force ? atoi(force) : -1;
   {
-    const hipError_t e = ilt_k_gemm_i8_few(1, &fmt, &w, &wd, &rows, &y, &bias, cols, xq, xs, bsums, ntok, acc, st, ldy);
+    hipError_t e = ilt_k_gemm_i8_few(1, &fmt, &w, &wd, &rows, &y, &bias, cols, xq, xs, bsums, ntok, acc, st, ldy);
+    if (e == hipErrorNotSupported && forced != 0)
+      e = ilt_k_gemm_i8_reg(1, &fmt, &w, &rows, &y, &bias, cols, xq, xs, bsums, ntok, acc, st, ldy);
     if (e != hipErrorNotSupported) return e;
   }
   const bool fits = rows < (1 << 21) && ldy < (1 << 21) && (long long)rows * row_bytes < 0x7FFFFFFFLL;      // the pipelined kernels' 32-bit offsets
-  if (fits && (fmt == ILT_Q6_K || fmt == ILT_Q4_K || fmt == ILT_Q2_K) && cols % 256 == 0 && forced != 0 && (forced == 1 || (ntok >= 96 && rows >= 128)))
-    return ilt_k_gemm_i8_planes(fmt, w, row_bytes, rows, cols, xq, xs, bsums, ntok, y, bias, acc, st, ldy);
+  if (fits && fmt == ILT_Q2_K && cols % 256 == 0 && forced != 0 && (forced == 1 || (ntok >= 96 && rows >= 128)))
+    return ilt_k_gemm_i8_planes(w, row_bytes, rows, cols, xq, xs, bsums, ntok, y, bias, acc, st, ldy);
   if (fits && fmt == ILT_Q8_0 && cols % 64 == 0 && forced != 0 && (forced == 1 || (ntok >= 96 && rows >= 128)))
     return ilt_k_gemm_i8_q8(w, wd, rows, cols, xq, xs, ntok, y, bias, acc, st, ldy);
   GemmParams p = {};

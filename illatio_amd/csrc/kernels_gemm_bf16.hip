@@ -31,6 +31,7 @@
 // The same pipeline also carries the exact product (gemm_i8p_kernel, further down): scale * quant
 // as int8 planes on v_mfma_i32_32x32x32_i8, the bits of the CPU path's MATMUL!.
 #include "ilt_device.h"
+#include "ilt_gemm_tile.h"
 #include "ilt_iq2xxs_tables.h"
 #include "ilt_kernels.h"
 #include <stdlib.h>
@@ -41,11 +42,9 @@ namespace {
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 
 constexpr int KS = 32;                 // columns per step
-constexpr int GR = 8;                  // row tiles per block of tiles sharing an L2
 
 __device__ const u64 bf_grid_dev[256] = { ILT_IQ2XXS_GRID_VALUES };
 
@@ -191,33 +190,6 @@ __device__ __forceinline__ void dequant16_pk<ILT_IQ2_XXS>(const WRaw<ILT_IQ2_XXS
   }
 }
 
-struct BfParams {
-  const u8* w;                               // dense
-  const u64* ptrs; long long add;            // grouped: expert z's matrix at ptrs[z] + add
-  const u32* counts; const u32* bases; int ne;
-  int rows, cols; long long row_bytes;
-  const u16* x;                              // bf16 activations, cols per token (the gathered rows when grouped)
-  const u32* rmap;                           // grouped: row i of the groups is x's row rmap[i] (null: row i)
-  float* y; const float* bias; int acc; int ntok;
-  long long ldy;                             // floats from a token's results to the next token's in y (rows, unless p covers a part of the rows)
-  // several matrices of one format on the same tokens in one launch (gemm_i8p_kernel, dense): matrix m's row tiles follow
-  // matrix m-1's; rows = the tiles of all of them together times 128 until the workgroup has found its matrix
-  int nmulti; const u8* mw[3]; int mrows[3]; float* my[3]; const float* mbias[3];
-  // the grouped gate and up products with the gated activation (gemm_bf16_regb_kernel<FMT, true>): rows = the width of
-  // each; up's matrix at ptrs[z] + add + up_delta; mid[i][r] = bf16((silu(gate) * up) * wrow[i]), clamped as d4_swiglu_w does
-  unsigned up_delta; const float* wrow; float clamp; u16* mid;
-  // the exact product (gemm_i8p_kernel): x = the tokens' Q8_K quants (a byte a column), with their block scales and sums of 16
-  const float* xd; const int* bsums;
-  // Q8_0 (gemm_i8q_kernel): w = the quants (a byte a weight, rows of cols bytes), wdq their f16 scales, xd the tokens' scales (one per 32)
-  const u16* wdq;
-  // the planes made beforehand (gemm_i8pp_kernel): w = the hi plane, wlo the lo plane (a byte a weight, rows of cols bytes), wdf = d per row and super-block
-  const u8* wlo; const float* wdf;
-  // the columns split over workgroups (gemm_bf16_kernel, dense): workgroups from split_from on take the tiles from
-  // split_from on, ksplit of them a tile, each a run of the super-blocks, and leave their sums in part (a tile of TM x TN
-  // floats each, token after token); bf16_split_sum_kernel adds a tile's parts in order and writes y.  ksplit 0: none
-  int ksplit, split_from; float* part;
-};
-
 template <int TM, int TN, int NXS, int NWS> struct Smem {
   __align__(16) u8 xs[NXS][TN * KS * 2];
   __align__(16) u8 ws[NWS][TM * KS * 2];
@@ -232,113 +204,6 @@ template <int TM, int TN, int NXS, int NWS> struct Smem {
 // in 8 (or 16) different 16-byte columns.
 __device__ __forceinline__ u32 slab_swz(int r) { return (((r >> 1) ^ (r >> 3)) & 1) | (((r >> 2) & 1) << 1); }
 __device__ __forceinline__ u32 slab_off(int r, int p) { return (u32)(4 * r + (p ^ slab_swz(r))) * 16; }
-
-// ---- a wave's results to y ----
-// Patch (a, b), register r of a lane: token wt0 + 32a + 8*(r/4) + 4*lh + r%4, row wr0 + 32b + l32
-// of the tile, so a store instruction writes 32 consecutive rows of two tokens.  With one
-// workgroup on a CU nothing else runs while it stores, so the loop is kept to an address add
-// and a store per value and has no branches: the stores go through a buffer descriptor that
-// ends with the tile's last token, which drops what lies past it, and a lane whose row the
-// matrix does not have starts 2 GiB out.  (ldy * 1024 < 2^31, checked by the host.)
-template <int NA, int NB, bool BIAS, bool ACC>
-__device__ __forceinline__ void store_patches(const v16f (&acc)[NA][NB], const BfParams& p, __amdgpu_buffer_rsrc_t ry, int r0,
-                                              int wt0, int wr0, int l32, int lh) {
-  const u32 rows4 = (u32)p.ldy * 4;
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
-    const int row = r0 + wr0 + 32 * b + l32;
-    const bool ok = row < p.rows;
-    const u32 base = ok ? (u32)((wt0 + 4 * lh) * (int)p.ldy + row) * 4 : 0x80000000u;
-    float bv = 0.0f;
-    if (BIAS) bv = ok ? p.bias[row] : 0.0f;
-#pragma unroll
-    for (int a = 0; a < NA; a++) {
-      float old[16];
-      if (ACC) {
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-          old[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ry, base + (u32)(32 * a + 8 * (r >> 2) + (r & 3)) * rows4, 0, 0));
-      }
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        float v = acc[a][b][r];
-        if (BIAS) v = v + bv;
-        if (ACC) v = old[r] + v;
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, v), ry, base + (u32)(32 * a + 8 * (r >> 2) + (r & 3)) * rows4, 0, 0);
-      }
-    }
-  }
-}
-
-template <int NA, int NB>
-__device__ __forceinline__ void store_tile(const v16f (&acc)[NA][NB], const BfParams& p, long tok0, int ntok, int r0,
-                                           int wt0, int wr0, int l32, int lh) {
-  // (ntok may come out of LDS: the same in every lane, said so to the compiler)
-  const u32 ybytes = ((u32)(__builtin_amdgcn_readfirstlane(ntok) - 1) * (u32)p.ldy + (u32)p.rows) * 4;
-  const __amdgpu_buffer_rsrc_t ry = ilt_rsrc(ilt_uniform_ptr(p.y + tok0 * p.ldy), ybytes);
-  if (p.bias) {
-    if (p.acc) store_patches<NA, NB, true, true>(acc, p, ry, r0, wt0, wr0, l32, lh);
-    else store_patches<NA, NB, true, false>(acc, p, ry, r0, wt0, wr0, l32, lh);
-  } else {
-    if (p.acc) store_patches<NA, NB, false, true>(acc, p, ry, r0, wt0, wr0, l32, lh);
-    else store_patches<NA, NB, false, false>(acc, p, ry, r0, wt0, wr0, l32, lh);
-  }
-}
-
-// Which tile a workgroup takes: row tile rt, tokens tok0 .. tok0+ntok-1 (of expert z's group,
-// with w its matrix, when grouped).  Tiles are numbered so that the eight XCDs' workgroups (the
-// hardware deals them round-robin) each walk a contiguous run, GR row tiles of one token tile
-// after another.  False: none (the grid is rounded up).  S: scan[256], tile_z, tile_t0, tile_n.
-// (dense) tile number s of the NT x NR: its row tile and its first token
-__device__ __forceinline__ void tile_place(int s, int NT, int NR, int& rt, int& tt) {
-  const int rg = s / (GR * NT), rem = s - rg * GR * NT, nr = min(GR, NR - rg * GR);
-  tt = rem / nr;
-  rt = rg * GR + (rem - tt * nr);
-}
-
-// LIMIT >= 0: only the tiles before it are dealt out (a multiple of 8; the workgroups from it on take parts of the rest)
-template <int TM, int TN, typename SM>
-__device__ __forceinline__ bool pick_tile(const BfParams& p, SM& S, long& tok0, int& ntok, int& rt, const u8*& w, int limit = -1) {
-  const int t = threadIdx.x;
-  const int NR = (p.rows + TM - 1) / TM;
-  int NT;
-  if (p.ptrs) {
-    if (t < 256) S.scan[t] = t < p.ne ? (p.counts[t] + TN - 1) / TN : 0;
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-      const u32 v = (t < 256 && t >= off) ? S.scan[t - off] : 0;
-      __syncthreads();
-      if (t < 256) S.scan[t] += v;
-      __syncthreads();
-    }
-    NT = (int)S.scan[255];
-  } else {
-    NT = (p.ntok + TN - 1) / TN;
-  }
-  const int total = limit >= 0 ? limit : NT * NR, per = (total + 7) / 8;
-  const int L = blockIdx.x, j = L >> 3;
-  const int s = (L & 7) * per + j;
-  if (j >= per || s >= total) return false;
-  int tt;
-  tile_place(s, NT, NR, rt, tt);
-  if (p.ptrs) {
-    if (t < p.ne) {
-      const u32 incl = S.scan[t], tiles = (p.counts[t] + TN - 1) / TN, excl = incl - tiles;
-      if ((u32)tt >= excl && (u32)tt < incl) {
-        S.tile_z = t;
-        S.tile_t0 = (int)(p.bases[t] + ((u32)tt - excl) * TN);
-        S.tile_n = (int)min((u32)TN, p.counts[t] - ((u32)tt - excl) * TN);
-      }
-    }
-    __syncthreads();
-    tok0 = S.tile_t0; ntok = S.tile_n;
-    w = (const u8*)(p.ptrs[S.tile_z] + p.add);
-  } else {
-    tok0 = (long)tt * TN;
-    ntok = min(TN, p.ntok - (int)tok0);
-  }
-  return true;
-}
 
 // TM rows x TN tokens per workgroup; wave w: rows 32*NB*(w/2).., tokens (TN/2)*(w%2)..: NA x NB
 // patches of 32x32.  NB = 2: 2*TM threads, two per row (a thread dequantizes 16 weights a step);
@@ -1083,18 +948,6 @@ __global__ __launch_bounds__(4 * TM, TM == 128 ? 1 : 2) void gemm_i8p_kernel(BfP
 
   long tok0; int ntok, rt; const u8* w = p.w;
   if (!pick_tile<TM, TN>(p, S, tok0, ntok, rt, w)) return;
-  if constexpr (!GROUPED) {
-    if (p.nmulti > 1) {                                      // which of the launch's matrices the row tile belongs to
-      const int n0 = (p.mrows[0] + TM - 1) / TM, n1 = n0 + (p.mrows[1] + TM - 1) / TM;
-      const int m = rt < n0 ? 0 : rt < n1 ? 1 : 2;
-      rt -= m == 0 ? 0 : m == 1 ? n0 : n1;
-      w = m == 0 ? p.mw[0] : m == 1 ? p.mw[1] : p.mw[2];
-      p.rows = m == 0 ? p.mrows[0] : m == 1 ? p.mrows[1] : p.mrows[2];
-      p.y = m == 0 ? p.my[0] : m == 1 ? p.my[1] : p.my[2];
-      p.bias = m == 0 ? p.mbias[0] : m == 1 ? p.mbias[1] : p.mbias[2];
-      p.ldy = p.rows;
-    }
-  }
   const int r0 = rt * TM;
   int* const cxo = (int*)S.wdm;                              // IQ2_XXS: cx for the even groups, this for the odd ones
   if constexpr (FMT == ILT_IQ2_XXS) {
@@ -2106,30 +1959,15 @@ static int i8p_tile_rows(long long tiles128) {
   return (tiles128 < 384 || (tiles128 < 1024 && rem != 0 && rem < 128)) ? 64 : 128;
 }
 
-template <bool GROUPED>
-static hipError_t launch_i8p(int fmt, const BfParams& p, long long token_tiles, hipStream_t st, int tm = 128) {
-  if ((fmt != ILT_Q6_K && fmt != ILT_Q4_K && fmt != ILT_Q2_K && fmt != ILT_IQ2_XXS) || p.cols % 256 != 0 || (long long)p.rows * 1024 >= 0x7FFFFFFFLL)
-    return hipErrorInvalidValue;
+static bool i8p_grid(const BfParams& p, long long token_tiles, int tm, dim3& grid) {
+  if (p.cols % 256 != 0 || (long long)p.rows * 1024 >= 0x7FFFFFFFLL) return false;
   const long long total = token_tiles * ((p.rows + tm - 1) / tm), per = (total + 7) / 8;
-  if (per * 8 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)(per * 8));
-  if constexpr (!GROUPED) {
-    if (tm == 64) {
-      if (fmt == ILT_Q6_K) hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q6_K, false, 64>), grid, dim3(256), 0, st, p);
-      else if (fmt == ILT_Q4_K) hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q4_K, false, 64>), grid, dim3(256), 0, st, p);
-      else if (fmt == ILT_Q2_K) hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q2_K, false, 64>), grid, dim3(256), 0, st, p);
-      else hipLaunchKernelGGL((gemm_i8p_kernel<ILT_IQ2_XXS, false, 64>), grid, dim3(256), 0, st, p);
-      return hipGetLastError();
-    }
-  }
-  if (fmt == ILT_Q6_K) hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q6_K, GROUPED>), grid, dim3(512), 0, st, p);
-  else if (fmt == ILT_Q4_K) hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q4_K, GROUPED>), grid, dim3(512), 0, st, p);
-  else if (fmt == ILT_Q2_K) hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q2_K, GROUPED>), grid, dim3(512), 0, st, p);
-  else hipLaunchKernelGGL((gemm_i8p_kernel<ILT_IQ2_XXS, GROUPED>), grid, dim3(512), 0, st, p);
-  return hipGetLastError();
+  if (per * 8 > 0x7FFFFFFFLL) return false;
+  grid = dim3((unsigned)(per * 8));
+  return true;
 }
 
-hipError_t ilt_k_gemm_i8_planes(int fmt, const uint8_t* w, long long row_bytes, int rows, int cols, const int8_t* xq, const float* xd,
+hipError_t ilt_k_gemm_i8_planes(const uint8_t* w, long long row_bytes, int rows, int cols, const int8_t* xq, const float* xd,
                                 const int* bsums, int ntok, float* y, const float* bias, int acc, hipStream_t st, long long ldy) {
   if (ntok <= 0 || rows <= 0) return hipSuccess;
   if (ldy == 0) ldy = rows;
@@ -2138,31 +1976,12 @@ hipError_t ilt_k_gemm_i8_planes(int fmt, const uint8_t* w, long long row_bytes, 
   p.w = w; p.rows = rows; p.cols = cols; p.row_bytes = row_bytes; p.x = (const u16*)xq; p.xd = xd; p.bsums = bsums;
   p.y = y; p.bias = bias; p.acc = acc; p.ntok = ntok; p.ldy = ldy;
   const long long tt = (ntok + 127) / 128;
-  return launch_i8p<false>(fmt, p, tt, st, i8p_tile_rows(tt * ((rows + 127) / 128)));
-}
-
-// Up to three matrices of one format (Q6_K, Q4_K, Q2_K) on the same tokens in one launch: their row tiles one after
-// another, so that matrices too small to fill the chip on their own share it (Q/K/V, gate and up of a prompt's chunk).
-// hipErrorNotSupported: the caller launches them one by one.
-hipError_t ilt_k_gemm_i8_planes_n(int fmt, int nmat, const uint8_t* const* ws, const int* rows, float* const* ys, const float* const* biases,
-                                  long long row_bytes, int cols, const int8_t* xq, const float* xd, const int* bsums, int ntok, int acc,
-                                  hipStream_t st) {
-  if (nmat < 2 || nmat > 3 || ntok < 96 || (fmt != ILT_Q6_K && fmt != ILT_Q4_K && fmt != ILT_Q2_K) || cols % 256 != 0) return hipErrorNotSupported;
-  BfParams p = {};
-  long long tiles128 = 0;
-  for (int m = 0; m < nmat; m++) {
-    if (rows[m] < 128 || rows[m] >= (1 << 21) || (long long)rows[m] * row_bytes >= 0x7FFFFFFFLL) return hipErrorNotSupported;
-    p.mw[m] = ws[m]; p.mrows[m] = rows[m]; p.my[m] = ys[m]; p.mbias[m] = biases ? biases[m] : nullptr;
-    tiles128 += (rows[m] + 127) / 128;
-  }
-  if (tiles128 * 128 >= (1 << 21)) return hipErrorNotSupported;
-  const int tm = i8p_tile_rows(tiles128 * ((ntok + 127) / 128));
-  long long tiles = 0;
-  for (int m = 0; m < nmat; m++) tiles += (rows[m] + tm - 1) / tm;
-  p.nmulti = nmat;
-  p.w = ws[0]; p.rows = (int)(tiles * tm); p.cols = cols; p.row_bytes = row_bytes; p.x = (const u16*)xq; p.xd = xd; p.bsums = bsums;
-  p.y = ys[0]; p.acc = acc; p.ntok = ntok; p.ldy = rows[0];
-  return launch_i8p<false>(fmt, p, (ntok + 127) / 128, st, tm);
+  const int tm = i8p_tile_rows(tt * ((rows + 127) / 128));
+  dim3 grid;
+  if (!i8p_grid(p, tt, tm, grid)) return hipErrorInvalidValue;
+  if (tm == 64) hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q2_K, false, 64>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q2_K, false>), grid, dim3(512), 0, st, p);
+  return hipGetLastError();
 }
 
 hipError_t ilt_k_planes_i8(int fmt, const uint8_t* w, long long row_bytes, int rows, int cols, uint8_t* wh, uint8_t* wl, float* wdf,
@@ -2219,7 +2038,16 @@ hipError_t ilt_k_gemm_i8_planes_id(int fmt, const uint64_t* ptrs, long long add,
   p.ptrs = ptrs; p.add = add; p.counts = counts; p.bases = bases; p.ne = ne;
   p.rows = rows; p.cols = cols; p.row_bytes = row_bytes; p.x = (const u16*)xq; p.xd = xd; p.bsums = bsums;
   p.y = y; p.ntok = (int)total_rows; p.ldy = rows;
-  return launch_i8p<true>(fmt, p, total_rows / 128 + ne, st);
+  dim3 grid;
+  if (!i8p_grid(p, total_rows / 128 + ne, 128, grid)) return hipErrorInvalidValue;
+  switch (fmt) {
+    case ILT_Q6_K: hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q6_K, true>), grid, dim3(512), 0, st, p); break;
+    case ILT_Q4_K: hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q4_K, true>), grid, dim3(512), 0, st, p); break;
+    case ILT_Q2_K: hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q2_K, true>), grid, dim3(512), 0, st, p); break;
+    case ILT_IQ2_XXS: hipLaunchKernelGGL((gemm_i8p_kernel<ILT_IQ2_XXS, true>), grid, dim3(512), 0, st, p); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
 }
 
 hipError_t ilt_k_cvt_bf16_slabs(const float* x, uint16_t* out, int n, int cols, hipStream_t st) {

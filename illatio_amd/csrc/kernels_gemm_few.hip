@@ -426,12 +426,14 @@ hipError_t few_dispatch(FewParams& p, int forced, hipStream_t st) {
 }  // namespace
 
 // Up to four matrices (all Q8_0, or Q4_K and Q6_K in any mix) on the same quantized tokens in one launch.
-// hipErrorNotSupported (nothing launched) where the shapes are not this kernel's.  Against the pipelined kernels, which
-// want 96 tokens and 128 rows and take a tile's time whether or not the tiles fill the chip, the line lies at the number of
-// 32 x 32 tiles that take as long (1,024 Q4_K: 4096 x 2560 on 256 tokens 29.5 against 39.7 us, on 512 55.7 against 42.9;
-// 800 Q6_K: 2560 x 9728 on 256 tokens 86 against 103, on 512 134 against 108; 640 Q8_0: 4864 x 896 on 128 tokens 16.8
-// against 18.6, on 256 25 against 20).  Below 96 tokens the other kernel is the one of 64 x 64 tiles, two to eight times
-// slower at every shape measured.  ILT_I8_FEW (tests): "0" never, "1" always, "2", "4", "8" always, that cut.
+// hipErrorNotSupported (nothing launched) where the shapes are not this kernel's.  Against the kernel with the weights in
+// operand registers (kernels_gemm_reg.hip), whose tiles of 128 tokens take their time however few the tokens are, the line
+// lies at the number of 32 x 32 tiles that take as long (Q4_K: 2560 x 4096 on 192 tokens, 480 tiles: 25 against 33 us, on 256,
+// 640: 38 against 33; 19456 x 2560 on 24, 608: 22 against 32, on 48, 1,216: 37 against 33; Q6_K: 2560 x 9728 on 192, 480: 63
+// against 75, on 256: 91 against 75; 9728 x 2560 on 24, 304: 21 against 23, on 48: 32 against 23).  With up to 32 tokens the
+// other kernel does four times the work for nothing, with up to 16 eight times.  Q8_0 against the pipelined kernel of its own,
+// which wants 96 tokens and 128 rows: 640 tiles (4864 x 896 on 128 tokens 16.8 against 18.6, on 256 25 against 20).
+// ILT_I8_FEW (tests): "0" never, "1" always, "2", "4", "8" always, that cut.
 hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws, const uint16_t* const* wds, const int* rows, float* const* ys,
                              const float* const* biases, int cols, const int8_t* xq, const float* xs, const int* bsums, int ntok, int acc,
                              hipStream_t st, long long ldy) {
@@ -458,7 +460,8 @@ hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws
   }
   tiles32 *= (ntok + 31) / 32;
   if (tiles32 > 0x3FFFFFFF) return hipErrorNotSupported;
-  if (forced < 0 && ntok >= 96 && !small && tiles32 > (fset == ILT_Q8_0 ? 640 : fset == ILT_Q6_K ? 800 : 1024)) return hipErrorNotSupported;
+  const long long line = ntok <= 32 ? 1250 : fset == ILT_Q4_K ? 620 : fset == ILT_Q6_K ? 480 : 550;
+  if (forced < 0 && !small && (fset == ILT_Q8_0 ? ntok >= 96 && tiles32 > 640 : ntok > 16 && tiles32 > line)) return hipErrorNotSupported;
   switch (fset) {
     case ILT_Q8_0: return few_dispatch<ILT_Q8_0>(p, forced, st);
     case ILT_Q4_K: return few_dispatch<ILT_Q4_K>(p, forced, st);

@@ -1,0 +1,448 @@
+// The exact prefill product of many tokens, the weights made in the matrix cores' operand registers: Y[t][r] = W[r].x_t, W in
+// GGUF Q4_K / Q6_K blocks, every result with the CPU path's bits (MATMUL!: kquant.lisp:180-236, batch.lisp:128).
+//
+// What bounds it: the vector ALU and the matrix cores together (gfx950 issues a multiply or an add of two waves in the time a
+// third of an MFMA takes, and an MFMA hides permutes and 16-bit arithmetic but only half of the plain float work beside it),
+// and the latencies between them.  A super-block of 256 columns leaves one integer a result, however it comes about, and two
+// (Q4_K: four) roundings after it; the integer goes through v_mfma_i32_32x32x32_i8 as two planes:
+//   Q4_K: a scale is two digits, sc = 8 sh + sl, and q * digit is at most 105: four bytes times a digit is one 16-bit packed
+//         multiply with no carry between them.  isum = 8 * (sh q . xq) + (sl q . xq).
+//   Q6_K: T = sc (q - 32) = 256 hi + lo with lo signed: 16-bit fields, one packed multiply-add for two weights.
+// The minimums (Q4_K) are one f16 product of the tokens' sums of 32, in two parts of seven bits, with the 6-bit minimums:
+// whole numbers below 2^21, exact in its single-precision sums.
+//
+// A wave takes 32 rows and holds a whole super-block of them as operands (64 registers), so a weight is unpacked once for the
+// wave's 64 or 128 tokens and nothing of it passes through LDS twice; the rows' blocks come into LDS as they are (direct
+// loads of consecutive bytes: the same bytes as 16-byte loads a lane, of 32 rows each, cost the memory pipeline four times
+// as much and half the kernel's time), the tokens' quants beside them, 64 tokens' room at a time, so that two workgroups of
+// four waves fit a CU and one's start and end run beside the other's middle.  Everything is one step ahead: while patch a's
+// products run, patch a-1's integer sums become float terms, and with a block's last patch each group's operands are replaced
+// by the next block's as soon as they have been multiplied.  Two barriers a super-block, loads half a super-block ahead.
+// A patch's float work beside its MFMAs one result after another left every instruction waiting for the one before it; two
+// results go step by step side by side, and what a step wants from LDS is asked for a step before.
+//
+// Measured against the kernel of 64-column steps with planes through LDS that this one replaced (us; Q4_K 19456 x 2560 on 256,
+// 512, 2048 tokens; 2560 x 4096 on 512; Q6_K 2560 x 9728 on 512; 17408 x 5120 on 4096): 88 -> 54, 137 -> 82, 583 -> 278;
+// 62 -> 40; 110 -> 79; 1,400 -> 985 (741 TFLOP/s).
+#include "ilt_device.h"
+#include "ilt_gemm_tile.h"
+#include "ilt_kernels.h"
+#include <stdlib.h>
+#include <type_traits>
+
+namespace {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef unsigned short v2u __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ u32 wordr(const int4& v, int i) { return (u32)(i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w); }
+__device__ __forceinline__ v2u as2(u32 v) { return __builtin_bit_cast(v2u, v); }
+__device__ __forceinline__ u32 asw(v2u v) { return __builtin_bit_cast(u32, v); }
+// half H of the two 16-bit fields of V, in both
+template <int H> __device__ __forceinline__ v2u splat(u32 v) { const v2u a = as2(v); return v2u{a[H], a[H]}; }
+
+__device__ __forceinline__ float4 lds_f4(const float* p) {
+  const int4 v = ilt_lds_ld16(p);
+  return make_float4(__builtin_bit_cast(float, v.x), __builtin_bit_cast(float, v.y), __builtin_bit_cast(float, v.z), __builtin_bit_cast(float, v.w));
+}
+
+template <int FMT> struct RegW;
+
+template <> struct RegW<ILT_Q4_K> {
+  static constexpr int BLOCK = 144;
+  static constexpr bool MINS = true;
+  static constexpr int SH = 3;              // isum = (hi sums << SH) + (lo sums)
+  struct Block { u32 sc[2]; float d, dm; v8h mins; };
+  struct Quants { int4 q[2]; };
+  // In LDS: the quants of eight rows a kilobyte, piece p of row r at p ^ (r >> 1 & 7); behind them a header a row.
+  static constexpr int LOADS = 5, LBYTES = 5120;             // direct loads, bytes of LDS for 32 rows
+  struct At { u32 a, b, h; };
+  static __device__ __forceinline__ At place(u32 row_bytes, int lane) {
+    const u32 pc = 16 * (u32)((lane & 7) ^ ((lane >> 4) & 3)), rr = (u32)(lane >> 3) * row_bytes + 16;
+    return At{rr + pc, rr + (pc ^ 64), (u32)(lane & 31) * row_bytes};
+  }
+  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t rw, const At& at, u32 row_bytes, u32 base, u8* dst) {
+    if (i < 4) __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 1024 * i), 16, i & 1 ? at.b : at.a, base + 8 * i * row_bytes, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 4096), 16, at.h, base, 0, 0);
+  }
+  static __device__ __forceinline__ void block(Block& o, const u8* src, int l32, int) {
+    const int4 h = ilt_lds_ld16(src + 4096 + 16 * l32);
+    o.d = ilt_h2f((u16)((u32)h.x & 0xFFFF));
+    o.dm = ilt_h2f((u16)((u32)h.x >> 16));
+    const u32 a = (u32)h.y, b = (u32)h.z, c = (u32)h.w;                          // get_scale_min_k4, four groups a word
+    o.sc[0] = a & 0x3F3F3F3Fu; o.sc[1] = (c & 0x0F0F0F0Fu) | ((a >> 2) & 0x30303030u);
+    const u32 mn[2] = { b & 0x3F3F3F3Fu, ((c >> 4) & 0x0F0F0F0Fu) | ((b >> 2) & 0x30303030u) };
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const v2h k = {(_Float16)1024.0f, (_Float16)1024.0f};
+      const v2h m01 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0, mn[i], 0x0C010C00u) | 0x64006400u) - k;
+      const v2h m23 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0, mn[i], 0x0C030C02u) | 0x64006400u) - k;
+      o.mins[4 * i] = m01[0]; o.mins[4 * i + 1] = m01[1]; o.mins[4 * i + 2] = m23[0]; o.mins[4 * i + 3] = m23[1];
+    }
+  }
+  // the quants of groups g and g + 1 (g even)
+  static __device__ __forceinline__ void quants(Quants& o, const u8* src, int g, int l32, int lh) {
+    if (g % 2 == 0) o.q[(g >> 1) & 1] = ilt_lds_ld16(src + 128 * l32 + 16 * ((g + lh) ^ ((l32 >> 1) & 7)));
+  }
+  static __device__ __forceinline__ void quants_now(Quants&, const u8*, int, int, int) {}
+  static __device__ __forceinline__ void group(const Block& b, const Quants& r, int g, int, v4i& hi, v4i& lo) {
+    const v2u l = splat<0>((b.sc[g >> 2] >> (8 * (g & 3))) & 7), h = splat<0>((b.sc[g >> 2] >> (8 * (g & 3) + 3)) & 7);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const u32 w = wordr(r.q[(g >> 1) & 1], k);
+      const v2u n = as2((g % 2 ? w >> 4 : w) & 0x0F0F0F0Fu);
+      lo[k] = (int)asw(n * l);
+      hi[k] = (int)asw(n * h);
+    }
+  }
+};
+
+template <> struct RegW<ILT_Q6_K> {
+  static constexpr int BLOCK = ILT_Q6K_STRIDE;
+  static constexpr bool MINS = false;
+  static constexpr int SH = 8;
+  struct Block { int4 sc; float d, dm; v8h mins; };
+  struct Quants { int4 l[2], h; };
+  // In LDS: four rows a kilobyte and 64 bytes, piece p of row r at p ^ (r & 3) of its 256; piece 13 the block's last 16 bytes.
+  static constexpr int LOADS = 8, LBYTES = 8704;
+  struct At { u32 a; };
+  static __device__ __forceinline__ At place(u32 row_bytes, int lane) {
+    return At{(u32)(lane >> 4) * row_bytes + min(16u * (u32)((lane & 15) ^ (lane >> 4)), 196u)};
+  }
+  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t rw, const At& at, u32 row_bytes, u32 base, u8* dst) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 1088 * i), 16, at.a, base + 4 * i * row_bytes, 0, 0);
+  }
+  static __device__ __forceinline__ const u8* row_of(const u8* src, int l32) { return src + (l32 >> 2) * 1088 + (l32 & 3) * 256; }
+  static __device__ __forceinline__ void block(Block& o, const u8* src, int l32, int) {
+    const u8* row = row_of(src, l32);
+    o.sc = ilt_lds_ld16(row + 16 * (12 ^ (l32 & 3)));
+    o.d = ilt_h2f(*ILT_LDS_PTR(const u16, row + 16 * (13 ^ (l32 & 3)) + 12));
+  }
+  // what group g needs that no group before it has brought: groups g and g + 2 of a half share 16 bytes of low bits, a half's
+  // four groups 16 bytes of high ones
+  static __device__ __forceinline__ void quants(Quants& o, const u8* src, int g, int l32, int lh) {
+    const u8* row = row_of(src, l32);
+    const int x = l32 & 3, n = g >> 2;
+    if (g % 4 < 2) o.l[g % 4] = ilt_lds_ld16(row + 16 * ((4 * n + 2 * (g % 4) + lh) ^ x));
+  }
+  // (the high ones once the last of the half before has been made)
+  static __device__ __forceinline__ void quants_now(Quants& o, const u8* src, int g, int l32, int lh) {
+    if (g % 4 == 0) o.h = ilt_lds_ld16(row_of(src, l32) + 16 * ((8 + 2 * (g >> 2) + lh) ^ (l32 & 3)));
+  }
+  static __device__ __forceinline__ void group(const Block& b, const Quants& r, int g, int lh, v4i& hi, v4i& lo) {
+    const int j = g & 3;                             // columns 32g + 16lh ..: scale 2g + lh
+    const int s = (int)(i8)((wordr(b.sc, g >> 1) >> (8 * lh)) >> (16 * (g & 1)));
+    const u32 kk = (u32)(128 - 32 * s);
+    const v2u s2 = {(unsigned short)s, (unsigned short)s}, k2 = {(unsigned short)kk, (unsigned short)kk};
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const u32 w = wordr(r.l[j & 1], k), qh = wordr(r.h, k);
+      const u32 v = ((j >> 1 ? w >> 4 : w) & 0x0F0F0F0Fu) | ((j < 2 ? qh << (4 - 2 * j) : qh >> (2 * j - 4)) & 0x30303030u);
+      const u32 te = asw(as2(v & 0x00FF00FFu) * s2 + k2), to = asw((as2(v) >> 8) * s2 + k2);
+      hi[k] = (int)__builtin_amdgcn_perm(to, te, 0x07030501u);
+      lo[k] = (int)(__builtin_amdgcn_perm(to, te, 0x06020400u) ^ 0x80808080u);
+    }
+  }
+};
+
+template <int TN, int RAW, bool MINS> struct RegSmem {
+  // the tokens' quants of a super-block: four tokens a kilobyte and 64 bytes, piece p of token t at p ^ (t & 3) of its 256
+  __align__(16) u8 xs[TN / 4 * 1088];
+  __align__(16) u8 ms[3][MINS ? TN * 32 : 16];          // the sums of 32 as halves: eight times 128 * (sum >> 7), eight times sum & 127
+  __align__(16) u8 ws[RAW];                 // the rows' blocks
+  float xd[3][TN];
+};
+template <int FMT, int WR, int WT> constexpr int raw_bytes() { return (WT == 1 ? 1 : 2) * WR * RegW<FMT>::LBYTES; }
+
+// Rows r0 .. of one matrix (rows of them, results to y) x tokens tok0 .. tok0 + ntok - 1: WR x WT waves of 32 rows x 32 NP tokens
+template <int FMT, int NP, int WR, int WT>
+__device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0, long tok0, int ntok, unsigned char* smem) {
+  using F = RegW<FMT>;
+  constexpr int TN = 32 * NP * WT, THREADS = 64 * WR * WT;
+  constexpr int NI = TN / (8 * WR * WT);             // direct loads of a wave a super-block's half of the tokens (four tokens each)
+  constexpr int NW = (F::LOADS + WT - 1) / WT;       // and of the rows' blocks
+  static_assert((NP == 2 || NP == 4) && 2 * TN == THREADS, "a thread a half token's sums");
+  using Smem = RegSmem<TN, raw_bytes<FMT, WR, WT>(), F::MINS>;
+  Smem& S = *(Smem*)smem;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int nsb = p.cols / 256;
+  const int l32 = lane & 31, lh = lane >> 5;
+  const int wr0 = 32 * (wave % WR), wt0 = 32 * NP * (wave / WR);
+  const __amdgpu_buffer_rsrc_t rw = ilt_rsrc(ilt_uniform_ptr(w), (u32)p.rows * (u32)(nsb * F::BLOCK));
+  const u32 row_bytes = (u32)(nsb * F::BLOCK), wbase = (u32)(r0 + wr0) * row_bytes;      // (past the matrix's rows: zeros)
+  const typename F::At at = F::place(row_bytes, lane);
+  const int wg = wave % WR, wq = wave / WR;          // the wave's group of rows, its place among those that share it
+  auto issue_w = [&](int sb, int buf) {
+    u8* const dst = S.ws + ((WT == 1 ? 0 : buf) * WR + wg) * F::LBYTES;
+#pragma unroll
+    for (int i = 0; i < NW; i++)
+      if (F::LOADS % WT == 0 || wq * NW + i < F::LOADS) F::issue(wq * NW + i, rw, at, row_bytes, wbase + (u32)sb * F::BLOCK, dst);
+  };
+  const u8* xbase = (const u8*)ilt_uniform_ptr((const i8*)p.x + tok0 * (long)p.cols);
+  // (past the tile's tokens: zeros)
+  const __amdgpu_buffer_rsrc_t rx = ilt_rsrc(xbase, (u32)(__builtin_amdgcn_readfirstlane(ntok) * p.cols));
+  const u32 xlane = (u32)(lane >> 4) * (u32)p.cols, xpiece = 16 * (u32)((lane & 15) ^ (lane >> 4));
+  // half H of the tokens: the first or the second NP / 2 patches of every wave's
+  auto issue_x = [&](int sb, int h) {
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      const int j = wave * NI + i, q = j / (4 * NP), k4 = 8 * NP * q + 4 * NP * h + j % (4 * NP);      // tokens 4 k4 .. + 3
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (ILT_LDS void*)(S.xs + k4 * 1088), 16, xlane + xpiece, k4 * 4 * p.cols + sb * 256, 0, 0);
+    }
+  };
+  // the tokens' scales and sums of 32 of a super-block, through registers
+  const __amdgpu_buffer_rsrc_t rd = ilt_rsrc(ilt_uniform_ptr(p.xd + tok0 * nsb), (u32)(__builtin_amdgcn_readfirstlane(ntok) * nsb) * 4);
+  const __amdgpu_buffer_rsrc_t rb = ilt_rsrc(ilt_uniform_ptr(p.bsums + (F::MINS ? tok0 * (p.cols >> 4) : 0)), F::MINS ? (u32)(__builtin_amdgcn_readfirstlane(ntok) * (p.cols >> 4)) * 4 : 0);
+  float c_yd; int4 c_bs[2];
+  const u32 ctok = (u32)((t >> 1) * nsb);            // (past the tile's tokens: zeros)
+  auto load_consts = [&](int sb) {
+    c_yd = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, ctok * 4, sb * 4, 0));
+    if constexpr (F::MINS) {
+      const u32 o = ctok * 64 + 32 * (t & 1);
+      const ilt_v4i a = __builtin_amdgcn_raw_buffer_load_b128(rb, o, sb * 64, 0), b = __builtin_amdgcn_raw_buffer_load_b128(rb, o + 16, sb * 64, 0);
+      c_bs[0] = make_int4(a.x, a.y, a.z, a.w); c_bs[1] = make_int4(b.x, b.y, b.z, b.w);
+    }
+  };
+  auto store_consts = [&](int buf) {
+    if ((t & 1) == 0) S.xd[buf][t >> 1] = c_yd;
+    if constexpr (F::MINS) {
+      const int s[4] = { c_bs[0].x + c_bs[0].y, c_bs[0].z + c_bs[0].w, c_bs[1].x + c_bs[1].y, c_bs[1].z + c_bs[1].w };
+      _Float16 hh[4], ll[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) { hh[k] = (_Float16)(float)(s[k] & ~127); ll[k] = (_Float16)(float)(s[k] & 127); }
+      _Float16* const dst = (_Float16*)(S.ms[buf] + 32 * (t >> 1)) + 4 * (t & 1);
+      __builtin_memcpy(dst, hh, 8);
+      __builtin_memcpy(dst + 8, ll, 8);
+    }
+  };
+  v16f sum[NP][1];
+#pragma unroll
+  for (int a = 0; a < NP; a++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) sum[a][0][r] = 0.0f;
+  const u32 x0 = (u32)((wt0 + l32) >> 2) * 1088 + (u32)(l32 & 3) * 256 + 16 * (u32)(lh ^ (l32 & 3)), x1 = x0 ^ 32;
+  const u8* const wsrc = S.ws + wg * F::LBYTES;
+  v4i hi[8], lo[8];
+  typename F::Block blk;
+  issue_w(0, 0);
+  issue_x(0, 0);
+  load_consts(0);
+  store_consts(0);
+  if (t < TN) S.xd[2][t] = 0.0f;                     // (the block before the first: nothing)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the direct loads have landed
+  ilt_barrier_lds();
+  F::block(blk, wsrc, l32, lh);
+  {
+    typename F::Quants qs;
+#pragma unroll
+    for (int g = 0; g < 8; g++) { F::quants(qs, wsrc, g, l32, lh); F::quants_now(qs, wsrc, g, l32, lh); F::group(blk, qs, g, lh, hi[g], lo[g]); }
+  }
+  // integer sums: of the patch being multiplied, and of the one before as they are, or put together where registers are short
+  constexpr bool TIGHT = NP == 4;
+  v16i X[TIGHT ? 1 : 2], Y[TIGHT ? 1 : 2], P;
+#pragma unroll
+  for (int r = 0; r < 16; r++) { if (TIGHT) P[r] = 0; else { X[1][r] = 0; Y[1][r] = 0; } }
+  v16f im = {};                                      // and of the minimums
+  float dprev = 0.0f, dmprev = 0.0f;
+  int c0 = 0, c1 = 1, c2 = 2;                        // where the tokens' constants of this block, the next and the one before are
+  // Patch a of the block: its products, and beside them the terms of the patch before it and, with the last patch, the next
+  // block's operands, each group's as soon as this block's have been multiplied.
+  auto patch = [&](auto ac, const u8* wnext) {
+    constexpr int a = decltype(ac)::value, par = a & 1, pa = (a + NP - 1) % NP;
+    constexpr bool last = a == NP - 1;
+    v16i &XC = X[TIGHT ? 0 : par], &YC = Y[TIGHT ? 0 : par], &XP = X[TIGHT ? 0 : par ^ 1], &YP = Y[TIGHT ? 0 : par ^ 1];
+    const float dp = a == 0 ? dprev : blk.d, dmp = a == 0 ? dmprev : blk.dm;
+    const float* const xp = S.xd[a == 0 ? c2 : c0] + wt0 + 32 * pa + 4 * lh;
+    auto frag = [&](int g) { return __builtin_bit_cast(v4i, ilt_lds_ld16(S.xs + (g & 1 ? x1 : x0) + 8704 * a + 64 * (g >> 1))); };
+    const v16i zi = {};
+    typename F::Block nb = {};
+    typename F::Quants qs;
+    v4i f0 = frag(0), f1 = frag(1);
+    float4 yp = lds_f4(xp), yn;
+    v8h sums;
+    if constexpr (last) { F::block(nb, wnext, l32, lh); F::quants(qs, wnext, 0, l32, lh); }
+#pragma unroll
+    for (int g = 0; g < 8; g++) {
+      const v4i f = f0;
+      f0 = f1;
+      // (what the next step wants from LDS is asked for before this one's products)
+      if (g < 6) f1 = frag(g + 2);
+      if (last) F::quants_now(qs, wnext, g, l32, lh);
+      if (last && g < 7) F::quants(qs, wnext, g + 1, l32, lh);
+      if (g % 2 == 0 && g < 6) yn = lds_f4(xp + 4 * g + 8);
+      if (F::MINS && g == 6) sums = __builtin_bit_cast(v8h, ilt_lds_ld16(S.ms[c0] + 32 * (wt0 + 32 * a + l32) + 16 * lh));
+      __builtin_amdgcn_sched_barrier(0);
+      XC = __builtin_amdgcn_mfma_i32_32x32x32_i8(f, hi[g], g ? XC : zi, 0, 0, 0);
+      YC = __builtin_amdgcn_mfma_i32_32x32x32_i8(f, lo[g], g ? YC : zi, 0, 0, 0);
+      // two results' terms, step by step side by side (one after the other every instruction waits for the one before it)
+      {
+        const int r = 2 * g;
+        const float y0 = r & 2 ? yp.z : yp.x, y1 = r & 2 ? yp.w : yp.y;
+        const int i0 = TIGHT ? P[r] : (XP[r] << F::SH) + YP[r], i1 = TIGHT ? P[r + 1] : (XP[r + 1] << F::SH) + YP[r + 1];
+        float b0 = y0 * dp, b1 = y1 * dp, f0_ = (float)i0, f1_ = (float)i1, s0 = sum[pa][0][r], s1 = sum[pa][0][r + 1];
+        if constexpr (F::MINS) {
+          float a0 = y0 * dmp, a1 = y1 * dmp;
+          asm volatile("" : "+v"(a0), "+v"(a1), "+v"(b0), "+v"(b1), "+v"(f0_), "+v"(f1_));
+          a0 = a0 * im[r]; a1 = a1 * im[r + 1]; b0 = b0 * f0_; b1 = b1 * f1_;
+          asm volatile("" : "+v"(a0), "+v"(a1), "+v"(b0), "+v"(b1));
+          s0 = s0 - a0; s1 = s1 - a1;
+          asm volatile("" : "+v"(s0), "+v"(s1));
+        } else {
+          asm volatile("" : "+v"(b0), "+v"(b1), "+v"(f0_), "+v"(f1_));
+          b0 = b0 * f0_; b1 = b1 * f1_;
+          asm volatile("" : "+v"(b0), "+v"(b1));
+        }
+        sum[pa][0][r] = s0 + b0; sum[pa][0][r + 1] = s1 + b1;
+      }
+      if (g % 2 == 1) yp = yn;
+      // (pinned here: the compiler would put all of it off to the block's end, where nothing runs beside it)
+      asm volatile("" : "+v"(sum[pa][0]));
+      if constexpr (last) {
+        F::group(nb, qs, g, lh, hi[g], lo[g]);
+        asm volatile("" : "+v"(hi[g]), "+v"(lo[g]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (F::MINS) {
+      const v16f zf = {};
+      im = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, blk.mins, zf, 0, 0, 0);
+    }
+    if constexpr (TIGHT) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) P[r] = (XC[r] << F::SH) + YC[r];
+      asm volatile("" : "+v"(P));
+    }
+    if constexpr (last) { dprev = blk.d; dmprev = blk.dm; blk = nb; }
+  };
+#pragma unroll 1
+  for (int sb = 0; sb < nsb; sb++) {
+    const int nx = min(sb + 1, nsb - 1), nbuf = (sb + 1) & 1;       // (the last block's again, for nobody)
+    using std::integral_constant;
+    __builtin_amdgcn_sched_barrier(0);
+    issue_x(sb, 1);                                  // (the block before's second half has been multiplied)
+    issue_w(nx, nbuf);                               // (and this block's operands are made)
+    load_consts(nx);
+    __builtin_amdgcn_sched_barrier(0);
+    const u8* const wnext = wsrc + (WT == 1 ? 0 : nbuf) * WR * F::LBYTES;
+    patch(integral_constant<int, 0>{}, wnext);
+    if constexpr (NP == 4) patch(integral_constant<int, 1>{}, wnext);
+    store_consts(c1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    ilt_barrier_lds();
+    __builtin_amdgcn_sched_barrier(0);
+    issue_x(nx, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (NP == 4) {
+      patch(integral_constant<int, 2>{}, wnext);
+      patch(integral_constant<int, 3>{}, wnext);
+    } else {
+      patch(integral_constant<int, 1>{}, wnext);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    ilt_barrier_lds();
+    const int c = c2; c2 = c0; c0 = c1; c1 = c;
+  }
+  {
+    const float* const xp = S.xd[c2] + wt0 + 32 * (NP - 1) + 4 * lh;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      if constexpr (F::MINS) sum[NP - 1][0][r] = sum[NP - 1][0][r] - (xp[8 * (r >> 2) + (r & 3)] * dmprev) * im[r];
+      sum[NP - 1][0][r] = sum[NP - 1][0][r] + (xp[8 * (r >> 2) + (r & 3)] * dprev) * (float)(TIGHT ? P[r] : (X[TIGHT ? 0 : 1][r] << F::SH) + Y[TIGHT ? 0 : 1][r]);
+    }
+  }
+  store_tile<NP, 1>(sum, p, tok0, ntok, r0, wt0, wr0, l32, lh);
+}
+
+struct NoScan { u32 scan[1]; int tile_z, tile_t0, tile_n; };      // (tiles of groups only)
+
+// FSET: the matrices' format, or 0 where Q4_K and Q6_K meet in a launch
+template <int FSET, int NP, int WR, int WT>
+__global__ __launch_bounds__(64 * WR * WT, 2) void gemm_i8r_kernel(BfParams p) {
+  constexpr int TM = 32 * WR, TN = 32 * NP * WT;
+  extern __shared__ __align__(16) unsigned char smem[];
+  long tok0; int ntok, rt; const u8* w = p.w;
+  if (!pick_tile<TM, TN>(p, *(NoScan*)smem, tok0, ntok, rt, w)) return;
+  // which of the launch's matrices the row tile belongs to
+  const int n0 = (p.mrows[0] + TM - 1) / TM, n1 = n0 + (p.mrows[1] + TM - 1) / TM;
+  const int m = rt < n0 ? 0 : rt < n1 ? 1 : 2;
+  rt -= m == 0 ? 0 : m == 1 ? n0 : n1;
+  w = m == 0 ? p.mw[0] : m == 1 ? p.mw[1] : p.mw[2];
+  p.rows = m == 0 ? p.mrows[0] : m == 1 ? p.mrows[1] : p.mrows[2];
+  p.y = m == 0 ? p.my[0] : m == 1 ? p.my[1] : p.my[2];
+  p.bias = m == 0 ? p.mbias[0] : m == 1 ? p.mbias[1] : p.mbias[2];
+  if (p.nmulti > 1) p.ldy = p.rows;
+  const int fmt = m == 0 ? p.mfmt[0] : m == 1 ? p.mfmt[1] : p.mfmt[2];
+  if constexpr (FSET != 0) reg_tile<FSET, NP, WR, WT>(p, w, rt * TM, tok0, ntok, smem);
+  else if (fmt == ILT_Q4_K) reg_tile<ILT_Q4_K, NP, WR, WT>(p, w, rt * TM, tok0, ntok, smem);
+  else reg_tile<ILT_Q6_K, NP, WR, WT>(p, w, rt * TM, tok0, ntok, smem);
+}
+
+template <int FMT, int NP, int WR, int WT> constexpr size_t reg_smem() {
+  constexpr int TN = 32 * NP * WT;
+  if constexpr (FMT != 0) return sizeof(RegSmem<TN, raw_bytes<FMT, WR, WT>(), RegW<FMT>::MINS>);
+  else return reg_smem<ILT_Q4_K, NP, WR, WT>() > reg_smem<ILT_Q6_K, NP, WR, WT>() ? reg_smem<ILT_Q4_K, NP, WR, WT>() : reg_smem<ILT_Q6_K, NP, WR, WT>();
+}
+
+template <int FSET, int NP, int WR, int WT>
+hipError_t launch_i8r(BfParams& p, hipStream_t st) {
+  constexpr int TM = 32 * WR, TN = 32 * NP * WT;
+  constexpr size_t smem = reg_smem<FSET, NP, WR, WT>();
+  static_assert(2 * smem <= 160 * 1024, "two workgroups a CU");
+  static bool attr_set[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  if (!attr_set[dev]) {            // more dynamic LDS than the default 64 KB: asked for once per device
+    const hipError_t e = hipFuncSetAttribute((const void*)gemm_i8r_kernel<FSET, NP, WR, WT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return e;
+    attr_set[dev] = true;
+  }
+  long long tiles = 0;
+  for (int m = 0; m < p.nmulti; m++) tiles += (p.mrows[m] + TM - 1) / TM;
+  p.rows = (int)(tiles * TM);
+  const long long total = (long long)((p.ntok + TN - 1) / TN) * tiles, per = (total + 7) / 8;
+  if (per * 8 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((gemm_i8r_kernel<FSET, NP, WR, WT>), dim3((unsigned)(per * 8)), dim3(64 * WR * WT), smem, st, p);
+  return hipGetLastError();
+}
+
+template <int FSET>
+hipError_t dispatch_i8r(BfParams& p, bool big, hipStream_t st) {
+  return big ? launch_i8r<FSET, 4, 4, 1>(p, st) : launch_i8r<FSET, 2, 2, 2>(p, st);
+}
+
+}  // namespace
+
+// Up to three matrices (Q4_K, Q6_K in any mix) on the same tokens in one launch, their row tiles one after another.
+// hipErrorNotSupported, and nothing launched, where the shapes are not this kernel's.  128 rows x 128 tokens a workgroup from
+// 150 such tiles on; fewer leave CUs idle, and 64 x 128 (each weight unpacked twice, for 64 tokens at a time) fills twice
+// as many: Q6_K 2560 x 9728 on 512 tokens, 80 tiles: 79 against 104 us; on 1,024, 160: 124 against 112; Q4_K 2560 x 4096 the
+// same 39 against 49, 54 against 53; 19456 x 2560 on 128, 152: 36.4 against 35.5.  ILT_I8_TM (tests): 64 or 128 rows whatever the shape.
+hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws, const int* rows, float* const* ys, const float* const* biases,
+                             int cols, const int8_t* xq, const float* xd, const int* bsums, int ntok, int acc, hipStream_t st, long long ldy) {
+  if (nmat < 1 || nmat > 3 || ntok < 1 || cols < 256 || cols % 256 != 0 || (long long)cols * 128 >= 0x7FFFFFFFLL) return hipErrorNotSupported;
+  BfParams p = {};
+  long long tiles128 = 0;
+  int fset = fmts[0];
+  for (int m = 0; m < nmat; m++) {
+    if (fmts[m] != ILT_Q4_K && fmts[m] != ILT_Q6_K) return hipErrorNotSupported;
+    if (fmts[m] != fset) fset = 0;
+    const long long bytes = (long long)rows[m] * (cols / 256) * (fmts[m] == ILT_Q4_K ? 144 : ILT_Q6K_STRIDE);
+    if (rows[m] < 1 || bytes >= 0x7FFFFFFFLL || (((uintptr_t)ws[m]) & 3) || rows[m] >= (1 << 21)) return hipErrorNotSupported;      // 32-bit offsets
+    p.mw[m] = ws[m]; p.mrows[m] = rows[m]; p.my[m] = ys[m]; p.mbias[m] = biases ? biases[m] : nullptr; p.mfmt[m] = fmts[m];
+    tiles128 += (rows[m] + 127) / 128;
+  }
+  p.ldy = nmat > 1 || ldy == 0 ? rows[0] : ldy;
+  if (p.ldy < rows[0] || p.ldy >= (1 << 21) || tiles128 * 128 >= (1 << 30)) return hipErrorNotSupported;
+  p.nmulti = nmat; p.cols = cols; p.x = (const u16*)xq; p.xd = xd; p.bsums = bsums; p.acc = acc; p.ntok = ntok;
+  const char* force = getenv("ILT_I8_TM");
+  const int forced = force ? atoi(force) : 0;
+  const bool big = forced ? forced == 128 : tiles128 * ((ntok + 127) / 128) >= 150;
+  switch (fset) {
+    case ILT_Q4_K: return dispatch_i8r<ILT_Q4_K>(p, big, st);
+    case ILT_Q6_K: return dispatch_i8r<ILT_Q6_K>(p, big, st);
+    default: return dispatch_i8r<0>(p, big, st);
+  }
+}
