@@ -343,7 +343,8 @@ int ilt_d4_mvq8(uint64_t stream, int rows, int cols, int group_rows, const int8_
 static int gemv_experts(uint64_t stream, int fmt, int ncols, int nrows, int row_bytes, int64_t add, int64_t add_up,
                         int x_stride, int y_stride, const uint64_t* ptrs, int nz, const int8_t* xq, const float* xd,
                         const int32_t* bsums, const float* xf, const float* wts, float clamp, float* dst,
-                        const uint32_t* sel = nullptr, const uint32_t* counts = nullptr, const uint32_t* bases = nullptr) {
+                        const uint32_t* sel = nullptr, const uint32_t* counts = nullptr, const uint32_t* bases = nullptr,
+                        const uint32_t* xrow = nullptr) {
   ILT_REQUIRE(nrows >= 0 && nz >= 0 && ncols > 0 && ncols % 256 == 0 && row_bytes == ncols / 256 * block_bytes(fmt));
   if (nrows == 0 || nz == 0) return ILT_OK;
   ILT_REQUIRE(ptrs && dst && add >= 0 && (add & 1) == 0 && (add_up < 0 || (add_up & 1) == 0) && x_stride % 256 == 0 && x_stride >= 0);
@@ -359,7 +360,7 @@ static int gemv_experts(uint64_t stream, int fmt, int ncols, int nrows, int row_
   }
   p.ptrs = ptrs; p.sel = sel; p.cols = ncols;
   p.xq = xq; p.xs = xd; p.bsums = bsums; p.xf = xf; p.x_stride = x_stride; p.y_stride = y_stride;
-  p.counts = counts; p.bases = bases;
+  p.counts = counts; p.bases = bases; p.xrow = xrow;
   return (int)ilt_gemv_launch(p, nz, S(stream));
 }
 
@@ -642,6 +643,53 @@ int ilt_d4_ffn_step_noalloc(uint64_t stream, int ne, int nu, int d, int ff, floa
   // Every piece of the layout is written in full by the launch that produces it before a later
   // launch reads it, so nothing of the previous call's contents has to be cleared.
   return step_run(stream, ws, ne, nu, d, ff, scale, clamp, wt, logits, bias, x, moe);
+}
+
+namespace {
+struct SmallLayout { uint64_t rexp, xrow, wrow, smap, xq, xs, sg, su, mq, ms, sout, bm, bd, total; };
+SmallLayout small_layout(int n, int nu, int d, int ff) {
+  const uint64_t rows = (uint64_t)n * nu;
+  SmallLayout l; uint64_t o = 0;
+  auto take = [&](uint64_t bytes) { const uint64_t at = o; o += up256(bytes); return at; };
+  l.rexp = take(4 * rows); l.xrow = take(4 * rows); l.wrow = take(4 * rows); l.smap = take(4 * rows);
+  l.xq = take((uint64_t)n * d); l.xs = take((uint64_t)n * d / 8);
+  l.sg = take(4ull * n * ff); l.su = take(4ull * n * ff);
+  l.mq = take((uint64_t)n * ff); l.ms = take((uint64_t)n * ff / 8);
+  l.sout = take(4ull * n * d); l.bm = take(4 * rows * ff); l.bd = take(4 * rows * d);
+  l.total = o;
+  return l;
+}
+}  // namespace
+
+uint64_t ilt_d4_ffn_small_workspace(int n, int nu, int d, int ff) {
+  if (n < 1 || n > 9 || nu < 1 || d < 1 || ff < 1 || nu > 64 || d > (1 << 20) || ff > (1 << 20)) return 0;
+  return small_layout(n, nu, d, ff).total;
+}
+
+int ilt_d4_ffn_small(uint64_t stream, void* wsp, uint64_t ws_bytes, int n, int ne, int nu, int d, int ff, float scale, float clamp,
+                     const ilt_ffn_step_weights* wt, const float* logits, const float* bias, const float* x, float* moe) {
+  ILT_TRY((hipError_t)step_args_ok(ne, nu, d, ff, wt, logits, x, moe));
+  ILT_REQUIRE(n >= 1 && n <= 9 && wsp && ((uintptr_t)wsp & 255) == 0 && ws_bytes >= small_layout(n, nu, d, ff).total && ((uintptr_t)x & 15) == 0);
+  const SmallLayout l = small_layout(n, nu, d, ff);
+  uint8_t* const ws = (uint8_t*)wsp;
+  uint32_t *rexp = (uint32_t*)(ws + l.rexp), *xrow = (uint32_t*)(ws + l.xrow), *smap = (uint32_t*)(ws + l.smap);
+  float *wrow = (float*)(ws + l.wrow), *xs = (float*)(ws + l.xs), *sg = (float*)(ws + l.sg), *su = (float*)(ws + l.su), *ms = (float*)(ws + l.ms);
+  float *sout = (float*)(ws + l.sout), *bm = (float*)(ws + l.bm), *bd = (float*)(ws + l.bd);
+  int8_t *xq = (int8_t*)(ws + l.xq), *mq = (int8_t*)(ws + l.mq);
+  const int rows = n * nu, grb = d / 256 * 66, drb = ff / 256 * 84;
+  int e;
+  ILT_TRY(ilt_k_small_route(ne, nu, scale, logits, bias, n, rexp, xrow, wrow, smap, S(stream)));
+  // the shared expert: its matrices once for all the tokens
+  ILT_TRY(ilt_k_quant_q8(x, xq, xs, nullptr, (long long)n * d / 32, 0, S(stream)));
+  if ((e = ilt_mm_q8_mma2(stream, wt->sgate_q, wt->sgate_d, sg, nullptr, ff, wt->sup_q, wt->sup_d, su, nullptr, ff, nullptr, nullptr, nullptr, nullptr, 0,
+                          xq, xs, d, n, 0))) return e;
+  ILT_TRY(ilt_k_swiglu_w(n, ff, clamp, sg, su, nullptr, nullptr, mq, ms, S(stream)));
+  if ((e = ilt_mm_q8(stream, wt->sdown_q, wt->sdown_d, mq, ms, sout, nullptr, d, ff, n, 0))) return e;
+  // the routed experts, a slot a (token, slot) row, an expert's rows one after another
+  if ((e = gemv_experts(stream, ILT_IQ2_XXS, d, ff, grb, 0, wt->gate_bytes, d, ff, wt->slots, rows, nullptr, nullptr, nullptr, x, wrow, clamp, bm, rexp,
+                        nullptr, nullptr, xrow))) return e;
+  if ((e = gemv_experts(stream, ILT_Q2_K, ff, d, drb, 2 * wt->gate_bytes, -1, ff, d, wt->slots, rows, nullptr, nullptr, nullptr, bm, nullptr, 0.0f, bd, rexp))) return e;
+  return (int)ilt_k_moe_sum_rows(d, nu, n, bd, smap, sout, moe, S(stream));
 }
 
 int ilt_mm_q8(uint64_t stream, const int8_t* wq, const uint16_t* wd, const int8_t* xq, const float* xs, float* y,

@@ -108,6 +108,7 @@ struct IltGemvParams {
   // cache for the rows after the first (the counts / bases of the reference's d4_mv_*, ds4f.cu:762-772); null = row y
   const uint32_t* counts;
   const uint32_t* bases;
+  const uint32_t* xrow;      // grid y works on row xrow[y] of the activations (the looping variant only); null = row y
 };
 
 // The kernel is chosen by the matrices' formats (mat[i].fmt): one format, or Q4_K and Q6_K mixed.
@@ -145,6 +146,10 @@ hipError_t ilt_k_dequant_ids(int fmt, const uint8_t* w, const uint16_t* wd, cons
 
 hipError_t ilt_k_route(int ne, int nu, int hash, float scale, int has_bias, const float* logits, const float* bias,
                        const int* tid2eid, const uint32_t* tokens, uint32_t* sel, float* wout, int ntok, hipStream_t st);
+// A short pass's routing and grouping in one launch (ntok <= 16, ntok * nu <= 1024): the (token, slot) rows in the order of their
+// experts, row i on expert rexp[i] of token xrow[i] with weight wrow[i]; smap[token * nu + slot] = the row
+hipError_t ilt_k_small_route(int ne, int nu, float scale, const float* logits, const float* bias, int ntok, uint32_t* rexp, uint32_t* xrow,
+                             float* wrow, uint32_t* smap, hipStream_t st);
 hipError_t ilt_k_group_zero(int ne, uint32_t* counts, hipStream_t st);
 hipError_t ilt_k_group_count(int n, int ne, int nu, const uint32_t* sel, uint32_t* counts, uint32_t* rank, hipStream_t st);
 hipError_t ilt_k_group_scan(int n, int ne, int nu, const uint32_t* counts, uint32_t* bases, hipStream_t st);

@@ -23,6 +23,30 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_kernel(int ntok, int n
                  hash == 1 ? tid2eid + (long long)tokens[t] * nu : nullptr, sel + (long long)t * nu, wout + (long long)t * nu, s_idx[wv], s_sc[wv]);
 }
 
+// A short pass's routing and grouping, one workgroup: wave t routes token t into LDS, then thread r finds its (token, slot)
+// row's place among all of them ordered by expert (at most a hundred rows in earnest: counting the smaller ones is a few
+// microseconds less than the counters, the scan and the scatter as launches of their own, 7 + 15 us of a pass's launches).
+template <int K>
+__global__ __launch_bounds__(1024) void small_route_kernel(int ntok, int ne, int nu, float scale, const float* __restrict__ logits,
+                                                           const float* __restrict__ bias, u32* __restrict__ rexp, u32* __restrict__ xrow,
+                                                           float* __restrict__ wrow, u32* __restrict__ smap) {
+  __shared__ u32 s_idx[16][64];
+  __shared__ float s_sc[16][64];
+  __shared__ u32 sel[1024];
+  __shared__ float w[1024];
+  const int lane = threadIdx.x & 63, t = threadIdx.x >> 6;
+  if (t < ntok)
+    route_token<K>(lane, ne, nu, scale, logits + (long long)t * ne, bias, nullptr, sel + t * nu, w + t * nu, s_idx[t], s_sc[t]);
+  __syncthreads();
+  const int n = ntok * nu;
+  for (int r = threadIdx.x; r < n; r += blockDim.x) {
+    const u32 e = sel[r];
+    int at = 0;
+    for (int i = 0; i < n; i++) at += sel[i] < e || (sel[i] == e && i < r);
+    rexp[at] = e; xrow[at] = (u32)(r / nu); wrow[at] = w[r]; smap[r] = (u32)at;
+  }
+}
+
 __global__ void group_zero_kernel(int ne, u32* counts) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e < ne) counts[e] = 0u;
@@ -87,7 +111,7 @@ __global__ void gather_rows_kernel(int d, int nrows, const float* __restrict__ s
   *(float4*)(x + gid) = *(const float4*)(src + (long long)map[r] * d + j);
 }
 
-// mid[r][j] = (silu(g) * u) * w[r], g and u clamped first when clamp > 1e-6
+// mid[r][j] = (silu(g) * u) * w[r] (no w: weights of one), g and u clamped first when clamp > 1e-6
 // (d4-routed!, ds4f.lisp:1016-1019); quantized to Q8_0 with a float scale as well when xq
 // is given (the shared expert's down projection takes Q8_0 activations).
 __global__ __launch_bounds__(256) void swiglu_w_kernel(long long total, int ff, float clamp, const float* __restrict__ g,
@@ -99,8 +123,9 @@ __global__ __launch_bounds__(256) void swiglu_w_kernel(long long total, int ff, 
   if (live) {
     float gv = g[i], uv = u[i];
     if (clamp > 1e-6f) { gv = fminf(gv, clamp); uv = fmaxf(-clamp, fminf(uv, clamp)); }
-    v = (ilt_silu(gv) * uv) * w[i / ff];
-    mid[i] = v;
+    v = ilt_silu(gv) * uv;
+    if (w) v = v * w[i / ff];
+    if (mid) mid[i] = v;
   }
   if (xq) {
     float amax = ilt_max16(fabsf(v));
@@ -189,6 +214,16 @@ hipError_t ilt_k_route(int ne, int nu, int hash, float scale, int has_bias, cons
   if (k <= 1) ROUTE_LAUNCH(1); else if (k <= 2) ROUTE_LAUNCH(2); else if (k <= 4) ROUTE_LAUNCH(4);
   else if (k <= 8) ROUTE_LAUNCH(8); else ROUTE_LAUNCH(16);
 #undef ROUTE_LAUNCH
+  return hipGetLastError();
+}
+
+hipError_t ilt_k_small_route(int ne, int nu, float scale, const float* logits, const float* bias, int ntok, uint32_t* rexp, uint32_t* xrow,
+                             float* wrow, uint32_t* smap, hipStream_t st) {
+  if (ntok < 1 || ntok > 16 || ne < 1 || ne > 1024 || nu < 1 || nu > 64 || nu > ne || ntok * nu > 1024) return hipErrorInvalidValue;
+  const dim3 block(64 * ntok);
+#define SR(K) hipLaunchKernelGGL(small_route_kernel<K>, dim3(1), block, 0, st, ntok, ne, nu, scale, logits, bias, rexp, xrow, wrow, smap)
+  if (ne <= 64) SR(1); else if (ne <= 128) SR(2); else if (ne <= 256) SR(4); else if (ne <= 512) SR(8); else SR(16);
+#undef SR
   return hipGetLastError();
 }
 

@@ -12,6 +12,7 @@ experts, D4-ROUTED!, ds4f.lisp:994-1037; Q8_0 with a float scale for the shared 
 D4-SHARED!, :1039-1048), not left as floats as its CUDA kernels take them.
 """
 import ctypes as C
+import threading
 
 import numpy as np
 
@@ -44,6 +45,24 @@ class ExpertPool:
                 ctypes.memmove(self.host_buf + i * self.slot_bytes, host[e].ctypes.data, self.slot_bytes)
                 hip.hip_zero(hip.DBuf(self.slot_ptr_device(e), self.slot_bytes, dev))      # the device slot plays no part
         self.ptrs = hip.hip_upload_new(dev, np.array([self.slot_ptr(e) for e in range(ne)], np.uint64))
+        self._spare, self._lock = [], threading.Lock()
+
+    def lend(self, nbytes):
+        """A workspace of at least NBYTES for a call that waits for its launches: one given back before, or a new one."""
+        with self._lock:
+            b = self._spare.pop() if self._spare else None
+        if b is not None and b.bytes < nbytes:
+            hip.hip_free(b)
+            b = None
+        return b or hip.hip_alloc(self.dev, nbytes, zero=False)
+
+    def give_back(self, b):
+        """Keep B for the next call: two at most (two callers at a time), until free()."""
+        with self._lock:
+            if len(self._spare) < 2:
+                self._spare.append(b)
+                return
+        hip.hip_free(b)
 
     def slot_ptr_device(self, e):
         return self.pool.ptr + int(e) * self.slot_bytes
@@ -57,6 +76,8 @@ class ExpertPool:
         hip.hip_sync(self.dev)
         hip.hip_free(self.pool)
         hip.hip_free(self.ptrs)
+        while self._spare:
+            hip.hip_free(self._spare.pop())
         if self.host_buf:
             hip.hip_host_free(self.host_buf)
             self.host_buf = 0
@@ -289,14 +310,30 @@ def ffn_small(dev, pool, sh, logits, norm2, n, ne, nu, scale, clamp, bias=None, 
     """The FFN past the router for a short pass's N <= 9 tokens (DK-FFN-SMALL,
     cuda-ds4f-spec.lisp:30-100: a speculative step's verification), every token with decode's
     bits.  The reference routes on the CPU and hands each expert its tokens' rows through
-    counts/bases; here d4_route leaves sel and the weights on the device and the expert
-    kernels take one slot per (token, slot) row, row t*nu + j on expert sel[t*nu + j]: the
-    gathered rows, gate+up+gated activation of all rows in one launch, their downs in one, the
-    sums in slot order with the shared expert's (d4_mvq8n for its three products).  Returns
-    MOE (N x d).  GROUPED "counts": DK-FFN-SMALL's own launches with its argument lists
+    counts/bases; here one call (ilt_d4_ffn_small) queues eight launches: the routing leaves the
+    (token, slot) rows on the device in the order of their experts, so that an expert's matrices come
+    from memory once for all its tokens, and the expert kernels take one slot per row.  Returns
+    MOE (N x d), a new DBuf, when it is there.  GROUPED "counts": DK-FFN-SMALL's own launches with its argument lists
     (cuda-ds4f-spec.lisp:82-88) -- d4_gather_rows, d4_mv_iq2_xxs for the gates and again for the ups,
     d4_swiglu_w, d4_mv_q2_k, each expert kernel over all NE slots with the counts and bases that
     d4_group_* left on the device (an expert nobody chose has a count of 0)."""
+    if grouped == "counts":
+        return _ffn_small_counts(dev, pool, sh, logits, norm2, n, ne, nu, scale, clamp, bias)
+    f = hip.lib().ilt_d4_ffn_small_workspace
+    f.restype = C.c_uint64
+    moe, ws = hip.hip_alloc(dev, 4 * n * pool.d, zero=False), pool.lend(int(f(C.c_int(n), C.c_int(nu), C.c_int(pool.d), C.c_int(pool.ff))))
+    wt = step_weights(pool, sh)
+    try:
+        hip.call("ilt_d4_ffn_small", C.c_uint64(dev.stream), C.c_uint64(ws.ptr), C.c_uint64(ws.bytes), C.c_int(n), C.c_int(ne), C.c_int(nu),
+                 C.c_int(pool.d), C.c_int(pool.ff), C.c_float(scale), C.c_float(clamp), C.byref(wt), C.c_uint64(logits.ptr),
+                 C.c_uint64(bias.ptr if bias is not None else 0), C.c_uint64(norm2.ptr), C.c_uint64(moe.ptr))
+        hip.hip_sync(dev)
+    finally:
+        pool.give_back(ws)
+    return moe
+
+
+def _ffn_small_counts(dev, pool, sh, logits, norm2, n, ne, nu, scale, clamp, bias):
     d, ff = pool.d, pool.ff
     rows = n * nu
     gb = pool.gate_bytes
@@ -314,44 +351,20 @@ def ffn_small(dev, pool, sh, logits, norm2, n, ne, nu, scale, clamp, bias=None, 
     hip.launch(dev, "d4_mvq8n", (d + 3) // 4, 128, [d, ff, d, n, ff, d, sh.down.qs, sh.down.d, qm_q, qm_s, sout])
     # the routed experts: row r = (token r / nu, slot r % nu)
     sel, w = route(dev, logits, n, ne, nu, scale, bias)
-    extra = []
-    if grouped == "counts":
-        g = group_rows(dev, sel, w, n, ne, nu)
-        rmap, smap, wrow = g["rmap"], g["smap"], g["wrow"]
-        x, bg, bu = A(dev, 4 * rows * d), A(dev, 4 * rows * ff), A(dev, 4 * rows * ff)
-        bm, bd, moe = A(dev, 4 * rows * ff), A(dev, 4 * rows * d), A(dev, 4 * n * d)
-        hip.launch(dev, "d4_gather_rows", (rows * d + 255) // 256, 256, [d, rows, norm2, rmap, x])
-        for add, out in ((0, bg), (gb, bu)):
-            hip.launch(dev, "d4_mv_iq2_xxs", ((ff + 7) // 8, 1, ne), 64,
-                       [d, ff, pool.grb, hip.I64(add), d, ff, pool.ptrs, None, x, out, g["counts"], g["bases"]])
-        hip.launch(dev, "d4_swiglu_w", (rows * ff + 255) // 256, 256, [rows, ff, float(clamp), bg, bu, wrow, bm, None, None])
-        hip.launch(dev, "d4_mv_q2_k", ((d + 7) // 8, 1, ne), 64,
-                   [ff, d, pool.drb, hip.I64(2 * gb), ff, d, pool.ptrs, None, bm, bd, g["counts"], g["bases"]])
-        hip.launch(dev, "d4_moe_sum_rows", (n * d + 255) // 256, 256, [d, nu, n, bd, smap, sout, moe])
-        hip.hip_sync(dev)
-        for b in [qn_q, qn_s, sg, su, smid, qm_q, qm_s, sout, one, sel, w, x, bg, bu, bm, bd] + list(g.values()):
-            hip.hip_free(b)
-        return moe
-    if grouped:
-        # GROUPED: the rows grouped by expert on the device (d4_group_*), an expert's rows one after another, so its
-        # matrices come from memory once for all its tokens: what the reference's counts / bases arguments give
-        g = group_rows(dev, sel, w, n, ne, nu)
-        rmap, smap, wrow = g["rmap"], g["smap"], g["wrow"]
-        rexp = A(dev, 4 * rows)
-        hip.launch(dev, "d4_rows_expert", (rows + 255) // 256, 256, [rows, sel, smap, rexp])
-        extra = [rexp] + [v for k, v in g.items() if k not in ("rmap", "smap")]
-    else:
-        rmap = hip.hip_upload_new(dev, (np.arange(rows) // nu).astype(np.uint32))
-        smap = hip.hip_upload_new(dev, np.arange(rows, dtype=np.uint32))
-        rexp, wrow = sel, w
-    x, bm, bd, moe = A(dev, 4 * rows * d), A(dev, 4 * rows * ff), A(dev, 4 * rows * d), A(dev, 4 * n * d)
+    g = group_rows(dev, sel, w, n, ne, nu)
+    rmap, smap, wrow = g["rmap"], g["smap"], g["wrow"]
+    x, bg, bu = A(dev, 4 * rows * d), A(dev, 4 * rows * ff), A(dev, 4 * rows * ff)
+    bm, bd, moe = A(dev, 4 * rows * ff), A(dev, 4 * rows * d), A(dev, 4 * n * d)
     hip.launch(dev, "d4_gather_rows", (rows * d + 255) // 256, 256, [d, rows, norm2, rmap, x])
-    hip.launch(dev, "d4_mv_glu_iq2_xxs", ((ff + 7) // 8, 1, rows), 64,
-               [d, ff, pool.grb, hip.I64(0), hip.I64(gb), d, ff, pool.ptrs, rexp, x, wrow, float(clamp), bm])
-    hip.launch(dev, "d4_mv_q2_k_f32", ((d + 7) // 8, 1, rows), 64, [ff, d, pool.drb, hip.I64(2 * gb), ff, d, pool.ptrs, rexp, bm, bd])
+    for add, out in ((0, bg), (gb, bu)):
+        hip.launch(dev, "d4_mv_iq2_xxs", ((ff + 7) // 8, 1, ne), 64,
+                   [d, ff, pool.grb, hip.I64(add), d, ff, pool.ptrs, None, x, out, g["counts"], g["bases"]])
+    hip.launch(dev, "d4_swiglu_w", (rows * ff + 255) // 256, 256, [rows, ff, float(clamp), bg, bu, wrow, bm, None, None])
+    hip.launch(dev, "d4_mv_q2_k", ((d + 7) // 8, 1, ne), 64,
+               [ff, d, pool.drb, hip.I64(2 * gb), ff, d, pool.ptrs, None, bm, bd, g["counts"], g["bases"]])
     hip.launch(dev, "d4_moe_sum_rows", (n * d + 255) // 256, 256, [d, nu, n, bd, smap, sout, moe])
     hip.hip_sync(dev)
-    for b in [qn_q, qn_s, sg, su, smid, qm_q, qm_s, sout, one, sel, w, rmap, smap, x, bm, bd] + extra:
+    for b in [qn_q, qn_s, sg, su, smid, qm_q, qm_s, sout, one, sel, w, x, bg, bu, bm, bd] + list(g.values()):
         hip.hip_free(b)
     return moe
 

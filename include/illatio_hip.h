@@ -268,6 +268,14 @@ typedef struct ilt_ffn_step_weights {
 uint64_t ilt_d4_ffn_step_workspace(int nu, int d, int ff);
 int ilt_d4_ffn_step(uint64_t stream, void* ws, uint64_t ws_bytes, int ne, int nu, int d, int ff, float scale, float clamp,
                     const ilt_ffn_step_weights* wt, const float* logits, const float* bias, const float* x, float* moe);
+/* The same for a short pass's n <= 9 tokens (DK-FFN-SMALL, cuda-ds4f-spec.lisp:30-100: a speculative step's verification):
+   logits n x ne, x n x d, moe n x d, every token with ilt_d4_ffn_step's bits.  Eight launches on stream: the routing and the
+   rows' order by expert, the shared expert's quantizer, gate and up, gated activation and down (its matrices read once for
+   all the tokens), the routed experts' gate/up/activation and down over the n * nu (token, slot) rows, the sums.  Nothing is
+   allocated, freed or waited for; ws as above, ilt_d4_ffn_small_workspace bytes. */
+uint64_t ilt_d4_ffn_small_workspace(int n, int nu, int d, int ff);
+int ilt_d4_ffn_small(uint64_t stream, void* ws, uint64_t ws_bytes, int n, int ne, int nu, int d, int ff, float scale, float clamp,
+                     const ilt_ffn_step_weights* wt, const float* logits, const float* bias, const float* x, float* moe);
 /* Measurement only (no counterpart in the reference): the calling thread's next ilt_d4_ffn_step calls record
    events[i] (ilt_event_create's handles, n <= 8) on the stream before their launch i and the one after their last
    launch behind it, so that a bench can time the step's launches as the step queues them; n = 0 switches it off. */
