@@ -26,7 +26,7 @@ struct BfParams {
   // the grouped gate and up products with the gated activation (gemm_bf16_regb_kernel<FMT, true>): rows = the width of
   // each; up's matrix at ptrs[z] + add + up_delta; mid[i][r] = bf16((silu(gate) * up) * wrow[i]), clamped as d4_swiglu_w does
   unsigned up_delta; const float* wrow; float clamp; u16* mid;
-  // the exact product (gemm_i8p_kernel): x = the tokens' Q8_K quants (a byte a column), with their block scales and sums of 16
+  // the exact products (gemm_i8r_kernel): x = the tokens' Q8_K quants (a byte a column), with their block scales and sums of 16
   const float* xd; const int* bsums;
   // Q8_0 (gemm_i8q_kernel): w = the quants (a byte a weight, rows of cols bytes), wdq their f16 scales, xd the tokens' scales (one per 32)
   const u16* wdq;

@@ -124,6 +124,9 @@ unsigned long long ilt_k_streamed_launches();      // decode products launched a
 hipError_t ilt_k_quant_q8(const float* x, int8_t* xq, float* xs, int* xsum, long long nblocks, int f16_scale, hipStream_t st);
 hipError_t ilt_k_quant_q8k(const float* x, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st);
 hipError_t ilt_k_swiglu_quant_q8k(const float* gate, const float* up, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st);
+// d4_swiglu_w and quantize-q8k! of its rows in one
+hipError_t ilt_k_swiglu_w_quant_q8k(int nrows, int ff, float clamp, const float* gate, const float* up, const float* wrow, int8_t* xq, float* xd, int* bsums,
+                                    hipStream_t st);
 // ntok rows of cols floats, x_stride floats apart, quantized into packed rows: quantize-q8! (k 0) or quantize-q8k! (k 1)
 hipError_t ilt_k_quant_rows(int k, const float* x, int8_t* xq, float* xs, int* bsums, long long ntok, int cols, long long x_stride,
                             int f16_scale, hipStream_t st);
@@ -157,6 +160,7 @@ hipError_t ilt_k_group_scatter(int n, int ne, int nu, const uint32_t* sel, const
                                const float* w, uint32_t* rmap, uint32_t* smap, float* wrow, hipStream_t st);
 hipError_t ilt_k_rows_expert(int n, const uint32_t* sel, const uint32_t* smap, uint32_t* rexp, hipStream_t st);
 hipError_t ilt_k_gather_rows(int d, int nrows, const float* src, const uint32_t* map, float* x, hipStream_t st);
+hipError_t ilt_k_gather_q8k(int d, int nrows, const int8_t* xq, const float* xd, const uint32_t* map, int8_t* oq, float* od, hipStream_t st);
 hipError_t ilt_k_swiglu_w(int n, int ff, float clamp, const float* g, const float* u, const float* w, float* mid,
                           int8_t* xq, float* xs, hipStream_t st);
 hipError_t ilt_k_moe_sum(int d, int k, const float* down, const float* shared_, float* moe, const uint32_t* perm, hipStream_t st);
@@ -172,13 +176,10 @@ hipError_t ilt_k_gemm_i8(int fmt, const uint8_t* w, const uint16_t* wd, long lon
 hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws, const uint16_t* const* wds, const int* rows, float* const* ys,
                              const float* const* biases, int cols, const int8_t* xq, const float* xs, const int* bsums, int ntok, int acc,
                              hipStream_t st, long long ldy = 0);
-// Q4_K and Q6_K (in any mix, up to three matrices), exact, the weights made in the operand registers (kernels_gemm_reg.hip);
+// Q4_K and Q6_K in any mix, or Q2_K or IQ2_XXS (up to three matrices), exact, the weights made in the operand registers (kernels_gemm_reg.hip);
 // hipErrorNotSupported, and nothing launched, where the shapes are not that kernel's
 hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws, const int* rows, float* const* ys, const float* const* biases,
                              int cols, const int8_t* xq, const float* xd, const int* bsums, int ntok, int acc, hipStream_t st, long long ldy = 0);
-// Q2_K, exact, on the pipelined kernel (kernels_gemm_bf16.hip): scale * quant as int8
-hipError_t ilt_k_gemm_i8_planes(const uint8_t* w, long long row_bytes, int rows, int cols, const int8_t* xq, const float* xd,
-                                const int* bsums, int ntok, float* y, const float* bias, int acc, hipStream_t st, long long ldy = 0);
 // The exact product in two passes (Q6_K): the two int8 planes and d per row and super-block once, then the product from them
 hipError_t ilt_k_planes_i8(int fmt, const uint8_t* w, long long row_bytes, int rows, int cols, uint8_t* wh, uint8_t* wl, float* wdf,
                            hipStream_t st);
@@ -187,9 +188,11 @@ hipError_t ilt_k_gemm_i8_pp(const uint8_t* wh, const uint8_t* wl, const float* w
 // Q8_0, exact, on the pipelined kernel (cols a multiple of 64)
 hipError_t ilt_k_gemm_i8_q8(const uint8_t* wq, const uint16_t* wd, int rows, int cols, const int8_t* xq, const float* xs, int ntok,
                             float* y, const float* bias, int acc, hipStream_t st, long long ldy = 0);
-hipError_t ilt_k_gemm_i8_planes_id(int fmt, const uint64_t* ptrs, long long add, const uint32_t* counts, const uint32_t* bases, int ne,
-                                   long long row_bytes, int rows, int cols, const int8_t* xq, const float* xd, const int* bsums,
-                                   long long total_rows, float* y, hipStream_t st);
+// The experts' IQ2_XXS and Q2_K, grouped: expert z's counts[z] rows from bases[z] on; y2 set: a second matrix of each expert at add2
+// as well (bsums: Q2_K only)
+hipError_t ilt_k_gemm_i8_reg_id(int fmt, const uint64_t* ptrs, long long add, long long add2, const uint32_t* counts, const uint32_t* bases, int ne,
+                                int rows, int cols, const int8_t* xq, const float* xd, const int* bsums, long long total_rows, float* y, float* y2,
+                                hipStream_t st);
 hipError_t ilt_k_gemm_i8_id(int fmt, const uint64_t* ptrs, long long add, const uint32_t* counts, const uint32_t* bases,
                             int ne, long long row_bytes, int rows, int cols, const int8_t* xq, const float* xs,
                             const int* bsums, long long total_rows, float* y, hipStream_t st);

@@ -430,20 +430,19 @@ hipError_t ilt_k_gemm_i8(int fmt, const uint8_t* w, const uint16_t* wd, long lon
   if (ntok <= 0 || rows <= 0) return hipSuccess;
   if (ldy == 0) ldy = rows;
   if (ldy < rows) return hipErrorInvalidValue;
-  // The kernels of few tokens and of operands in registers (Q6_K, Q4_K) have rules of their own; Q2_K and Q8_0 with enough
-  // tokens and rows to fill 128 x 128 tiles take pipelined kernels, the same bits.  ILT_I8_PLANES (tests): "0" none of
-  // them, "1" the pipelined ones and the registers' whenever the format allows.
+  // The kernels of few tokens (Q8_0, Q4_K, Q6_K) and of operands in registers (all but Q8_0) have rules of their own; Q2_K and
+  // IQ2_XXS on up to 16 tokens stay here, where a tile is 64 tokens and not 128; Q8_0 with enough tokens and rows to fill
+  // 128 x 128 tiles takes a pipelined kernel, the same bits.  ILT_I8_PLANES (tests): "0" neither the registers' nor the
+  // pipelined one, "1" these whenever the format allows.
   const char* force = getenv("ILT_I8_PLANES");
   const int forced = force ? atoi(force) : -1;
   {
     hipError_t e = ilt_k_gemm_i8_few(1, &fmt, &w, &wd, &rows, &y, &bias, cols, xq, xs, bsums, ntok, acc, st, ldy);
-    if (e == hipErrorNotSupported && forced != 0)
+    if (e == hipErrorNotSupported && forced != 0 && (ntok > 16 || forced == 1 || fmt == ILT_Q4_K || fmt == ILT_Q6_K))
       e = ilt_k_gemm_i8_reg(1, &fmt, &w, &rows, &y, &bias, cols, xq, xs, bsums, ntok, acc, st, ldy);
     if (e != hipErrorNotSupported) return e;
   }
-  const bool fits = rows < (1 << 21) && ldy < (1 << 21) && (long long)rows * row_bytes < 0x7FFFFFFFLL;      // the pipelined kernels' 32-bit offsets
-  if (fits && fmt == ILT_Q2_K && cols % 256 == 0 && forced != 0 && (forced == 1 || (ntok >= 96 && rows >= 128)))
-    return ilt_k_gemm_i8_planes(w, row_bytes, rows, cols, xq, xs, bsums, ntok, y, bias, acc, st, ldy);
+  const bool fits = rows < (1 << 21) && ldy < (1 << 21) && (long long)rows * row_bytes < 0x7FFFFFFFLL;      // the pipelined kernel's 32-bit offsets
   if (fits && fmt == ILT_Q8_0 && cols % 64 == 0 && forced != 0 && (forced == 1 || (ntok >= 96 && rows >= 128)))
     return ilt_k_gemm_i8_q8(w, wd, rows, cols, xq, xs, ntok, y, bias, acc, st, ldy);
   GemmParams p = {};
@@ -457,14 +456,10 @@ hipError_t ilt_k_gemm_i8_id(int fmt, const uint64_t* ptrs, long long add, const 
                             const int* bsums, long long total_rows, float* y, hipStream_t st) {
   if (total_rows <= 0 || rows <= 0 || ne <= 0) return hipSuccess;
   if (ne > 256) return hipErrorInvalidValue;
-  {
-    // the experts' IQ2_XXS and Q2_K (and Q4_K / Q6_K) matrices on the planes kernel when the groups average at least a quarter of a tile of 128 rows
-    const char* force = getenv("ILT_I8_PLANES");
-    const int forced = force ? atoi(force) : -1;
-    if (rows < (1 << 21) && (long long)rows * row_bytes < 0x7FFFFFFFLL &&
-        (fmt == ILT_Q6_K || fmt == ILT_Q4_K || fmt == ILT_Q2_K || fmt == ILT_IQ2_XXS) && cols % 256 == 0 && forced != 0 &&
-        (forced == 1 || (total_rows >= 32LL * ne && rows >= 128)))
-      return ilt_k_gemm_i8_planes_id(fmt, ptrs, add, counts, bases, ne, row_bytes, rows, cols, xq, xs, bsums, total_rows, y, st);
+  const char* force = getenv("ILT_I8_PLANES");       // "0" (tests): the kernel here
+  if (!(force && force[0] == '0')) {
+    const hipError_t e = ilt_k_gemm_i8_reg_id(fmt, ptrs, add, 0, counts, bases, ne, rows, cols, xq, xs, bsums, total_rows, y, nullptr, st);
+    if (e != hipErrorNotSupported) return e;
   }
   GemmParams p = {};
   p.ptrs = ptrs; p.add = add; p.counts = counts; p.bases = bases; p.ne = ne;

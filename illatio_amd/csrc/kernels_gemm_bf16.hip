@@ -28,8 +28,8 @@
 // expert's rows in turn; for the experts' own formats, IQ2_XXS and Q2_K, it has a kernel of
 // its own that dequantizes into the MFMA operands without a detour of the weights through LDS
 // as bf16 (gemm_bf16_regb_kernel).
-// The same pipeline also carries the exact product (gemm_i8p_kernel, further down): scale * quant
-// as int8 planes on v_mfma_i32_32x32x32_i8, the bits of the CPU path's MATMUL!.
+// The same pipeline also carries exact products (further down): Q8_0, and Q6_K from int8 planes made beforehand, on
+// v_mfma_i32_32x32x32_i8, with the bits of the CPU path's MATMUL!.
 #include "ilt_device.h"
 #include "ilt_gemm_tile.h"
 #include "ilt_iq2xxs_tables.h"
@@ -740,177 +740,8 @@ hipError_t launch_regb(const BfParams& p, long long token_tiles, hipStream_t st)
   return hipGetLastError();
 }
 
-// ---- the exact product on the same pipeline: Q6_K and Q4_K as two int8 planes -------------------
-// Bit for bit the CPU path's MATMUL! (and gemm_i8_kernel's) result: per super-block an integer
-// isum = sum over its 256 columns of (scale * quant) * xq, then sum += (d*yd) * float(isum) (and
-// Q4_K's term of the minimums before it), block after block (kquant.lisp:180-236).  Any exact
-// way to the integer will do, so the products P = sc*(q-32) (Q6_K, 13 bits) or sc*q (Q4_K, 10
-// bits) go to the int8 matrix cores as two planes, the bytes of T = P + C0 >= 0 (C0 = 4128 or
-// 0): hi = T >> 8 (0..31) and lo = (T & 255) - 128, so
-//   isum = 256*(hi.xq) + (lo.xq) + (128 - C0)*(sum of the block's xq),
-// the last from the activations' sums of 16.  v_mfma_i32_32x32x32_i8 accumulates both planes
-// over the super-block's four steps of 64 columns; the lanes then combine them once per block.
-// Four weights are made at a time: the even and the odd bytes of a word as two 16-bit fields
-// and one 24-bit multiply(-add) for both fields (each field's total is within 0..65535, so
-// borrows between them cancel).  Q4_K's sum of minimum * (sum of 32 quants) over the eight
-// groups is one more pair of small products per super-block, the sums of 32 split into planes
-// the same way.
 typedef int v4i_ __attribute__((ext_vector_type(4)));
 typedef int v16i_ __attribute__((ext_vector_type(16)));
-typedef int v3i_ __attribute__((ext_vector_type(3)));
-
-template <int FMT> struct I8p;
-
-// Thread (row, q4) makes columns 16*q4.. of its row in every step of 64 columns: part
-// 2*jj + q4/2 of half c (jj = the step within the half), weights 16*(q4 & 1).. of the part.
-template <> struct I8p<ILT_Q6_K> {
-  static constexpr int KCX = 4000;                           // isum = 256*hi + lo - KCX * (sum of xq)
-  static constexpr int PLANES = 2, WL = 4;                   // planes; loads of a raw set
-  struct Raw { int4 ql, qh; int2 sc; u32 d; };               // a half super-block's share
-  static __device__ __forceinline__ void load(Raw& r, __amdgpu_buffer_rsrc_t rw, u32 rowoff, int hb, int q4) {
-    const u32 b = rowoff + (u32)(hb >> 1) * ILT_Q6K_STRIDE;
-    const int c = hb & 1;
-    r.ql = ilt_bld16(rw, b + 64 * c + 16 * q4);              // ql[64c + 32*(part & 1) + l], part & 1 = q4 / 2, l = 16*(q4 & 1)..
-    r.qh = ilt_bld16(rw, b + 128 + 32 * c + 16 * (q4 & 1));
-    r.sc = ilt_bld8(rw, b + 192 + 8 * c);
-    r.d = ilt_bld2(rw, b + 208);
-  }
-  static __device__ __forceinline__ float d_of(const Raw& r) { return ilt_h2f((u16)r.d); }
-  // J: the step within the super-block
-  template <typename SM> static __device__ __forceinline__ void planes(const Raw& r, int J, int q4, int* hi, int* lo, const SM&) {
-    const int jj = J & 1;
-    const int sc = (int)(i8)(((u32)(jj ? r.sc.y : r.sc.x) >> (8 * q4)) & 0xFF);      // scale 8c + 2*part + (q4 & 1)
-    const int cpair = (4128 - 32 * sc) * 0x10001;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const u32 v = ((word_of(r.ql, i) >> (4 * jj)) & 0x0F0F0F0F) | (((word_of(r.qh, i) >> (4 * jj + 2 * (q4 >> 1))) & 0x03030303) << 4);
-      const u32 te = (u32)(__mul24((int)(v & 0x00FF00FF), sc) + cpair), to = (u32)(__mul24((int)((v >> 8) & 0x00FF00FF), sc) + cpair);
-      hi[i] = (int)__builtin_amdgcn_perm(to, te, 0x07030501u);                  // the fields' high bytes, in the weights' order
-      lo[i] = (int)(__builtin_amdgcn_perm(to, te, 0x06020400u) ^ 0x80808080u);   // their low bytes - 128
-    }
-  }
-};
-
-// Q4_K: step J of a super-block is groups 2J (low nibbles) and 2J+1 (high nibbles) of qs[32J..32J+31].
-template <> struct I8p<ILT_Q4_K> {
-  static constexpr int KCX = -128;
-  static constexpr int PLANES = 2, WL = 4;
-  struct Raw { int4 q[2]; v3i_ s; u32 dd; };                 // a half's two steps of quants (the thread's 16 bytes), the block's 12 scale bytes, d and dmin
-  static __device__ __forceinline__ void load(Raw& r, __amdgpu_buffer_rsrc_t rw, u32 rowoff, int hb, int q4) {
-    const u32 b = rowoff + (u32)(hb >> 1) * 144;
-    r.q[0] = ilt_bld16(rw, b + 16 + 64 * (hb & 1) + 16 * (q4 & 1));
-    r.q[1] = ilt_bld16(rw, b + 48 + 64 * (hb & 1) + 16 * (q4 & 1));
-    r.s = __builtin_amdgcn_raw_buffer_load_b96(rw, b + 4, 0, 0);
-    r.dd = ilt_bld4(rw, b);
-  }
-  static __device__ __forceinline__ float d_of(const Raw& r) { return ilt_h2f((u16)(r.dd & 0xFFFF)); }
-  static __device__ __forceinline__ float dmin_of(const Raw& r) { return ilt_h2f((u16)(r.dd >> 16)); }
-  static __device__ __forceinline__ u32 sbyte(const Raw& r, int i) { return ((u32)(i < 4 ? r.s.x : i < 8 ? r.s.y : r.s.z) >> (8 * (i & 3))) & 0xFF; }
-  // scale-min-k4 (kquant.lisp:64-72), g a constant
-  static __device__ __forceinline__ u32 scale_of(const Raw& r, int g) {
-    return g < 4 ? (sbyte(r, g) & 63) : ((sbyte(r, g + 4) & 15) | ((sbyte(r, g - 4) >> 6) << 4));
-  }
-  static __device__ __forceinline__ u32 min_of(const Raw& r, int g) {
-    return g < 4 ? (sbyte(r, g + 4) & 63) : ((sbyte(r, g + 4) >> 4) | ((sbyte(r, g) >> 6) << 4));
-  }
-  template <typename SM> static __device__ __forceinline__ void planes(const Raw& r, int J, int q4, int* hi, int* lo, const SM&) {
-    const int jp = q4 >> 1;                                  // group 2J + jp
-    const int sc = (int)(jp ? scale_of(r, 2 * J + 1) : scale_of(r, 2 * J));
-    const int4& q = r.q[J & 1];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const u32 v = (word_of(q, i) >> (4 * jp)) & 0x0F0F0F0F;
-      const u32 te = (u32)__mul24((int)(v & 0x00FF00FF), sc), to = (u32)__mul24((int)((v >> 8) & 0x00FF00FF), sc);
-      hi[i] = (int)__builtin_amdgcn_perm(to, te, 0x07030501u);
-      lo[i] = (int)(__builtin_amdgcn_perm(to, te, 0x06020400u) ^ 0x80808080u);
-    }
-  }
-};
-
-// Q2_K: sc*q is at most 45, one plane.  Step J of a super-block is parts 2*(J&1) and 2*(J&1)+1 of half J/2, all four
-// parts of a half in the same 32 bytes of quants, two bits each; the minimums' term over the sixteen groups of 16.
-template <> struct I8p<ILT_Q2_K> {
-  static constexpr int KCX = 0;
-  static constexpr int PLANES = 1, WL = 3;
-  struct Raw { int4 q, s; u32 dd; };                         // the thread's 16 bytes of the half's quants, the block's 16 scale bytes, d and dmin
-  static __device__ __forceinline__ void load(Raw& r, __amdgpu_buffer_rsrc_t rw, u32 rowoff, int hb, int q4) {
-    const u32 b = rowoff + (u32)(hb >> 1) * 84;
-    r.q = ilt_bld16(rw, b + 16 + 32 * (hb & 1) + 16 * (q4 & 1));
-    r.s = ilt_bld16(rw, b);
-    r.dd = ilt_bld4(rw, b + 80);
-  }
-  static __device__ __forceinline__ float d_of(const Raw& r) { return ilt_h2f((u16)(r.dd & 0xFFFF)); }
-  static __device__ __forceinline__ float dmin_of(const Raw& r) { return ilt_h2f((u16)(r.dd >> 16)); }
-  template <typename SM> static __device__ __forceinline__ void planes(const Raw& r, int J, int q4, int*, int* lo, const SM&) {
-    const int c = J >> 1, jj = J & 1;
-    const u32 sc = (word_of(r.s, 2 * c + jj) >> (8 * q4)) & 15;             // scale 8c + 2*part + (q4 & 1), part = 2jj + q4/2
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const u32 v = (word_of(r.q, i) >> (4 * jj + 2 * (q4 >> 1))) & 0x03030303;
-      lo[i] = (int)(v * sc);                                  // four products of at most 45: no carries between the bytes
-    }
-  }
-};
-
-template <int TM> struct I8pSmemT {
-  __align__(16) u8 xs[3][128 * 64];       // the tokens' quants, 64 columns a step
-  __align__(16) u8 wh[2][TM * 64];        // the rows' hi plane, the step's and the next step's
-  __align__(16) u8 wl[2][TM * 64];        // lo plane
-  float wd[128], wdm[128];                // of the super-block: d (and Q4_K's dmin) of the rows,
-  float xd[128];                          //   the tokens' scales
-  int cx[128];                            //   and KCX * the sum of their quants
-  union {
-    // Q4_K's minimums: the rows' eight minimums and their sum; the tokens' eight sums of 32 as planes
-    // (U = sum + 4096: U >> 8, and (U & 255) - 128)
-    struct { int2 wmn[128]; int wms[128]; int2 bh[128], bl[128]; };
-    // IQ2_XXS: the codebook, and for each 7-bit sign index (+ parity) 0xFF in the bytes of the negative weights
-    struct { u64 grid[256]; u64 smask[128]; };
-  };
-  u32 scan[256];
-  int tile_z, tile_t0, tile_n;
-};
-typedef I8pSmemT<128> I8pSmem;
-
-// IQ2_XXS: a block's eight groups of 32 weights add (float(sumi) * (0.5 + scale)) alternately to two sums,
-// fa (even groups) and fb (odd), then sum += (d*yd) * (fa + fb) (iquant.lisp:161-215).  Every term is a
-// multiple of 1/2, and with the codebook's entries (byte sums of at most 203) twice a sum of four of them
-// stays below 2^24 (at most 4 * 31 * 4 * 128 * 203 = 12,888,064): none of those float additions rounds, and
-// fa = float(S) * 0.5 for the integer S = sum over the even groups of (2*scale + 1) * sumi.  (Were the
-// last addition to round, it would round the exact sum once, as the conversion of S does.)  So the weights go in as (2*scale + 1) * (signed
-// magnitude), at most 1333 in absolute value, + 1408 as two planes, and a step's first 32 columns (an even
-// group) and second 32 (an odd one) have integer sums of their own.
-template <> struct I8p<ILT_IQ2_XXS> {
-  static constexpr int KCX = 1280;
-  static constexpr int PLANES = 2, WL = 3;
-  struct Raw { int2 g[2]; u32 d; };                          // the thread's group of each of the half's two steps (8 bytes: four codebook indices, signs and scale), d
-  static __device__ __forceinline__ void load(Raw& r, __amdgpu_buffer_rsrc_t rw, u32 rowoff, int hb, int q4) {
-    const u32 b = rowoff + (u32)(hb >> 1) * 66 + 2 + 8 * (4 * (hb & 1) + (q4 >> 1));
-    r.g[0] = ilt_bld8(rw, b);
-    r.g[1] = ilt_bld8(rw, b + 16);
-    r.d = ilt_bld2(rw, rowoff + (u32)(hb >> 1) * 66);
-  }
-  static __device__ __forceinline__ float d_of(const Raw& r) { return ilt_h2f((u16)r.d); }
-  template <typename SM> static __device__ __forceinline__ void planes(const Raw& r, int J, int q4, int* hi, int* lo, const SM& S) {
-    const u32 idx = (u32)r.g[J & 1].x, aux = (u32)r.g[J & 1].y;
-    const int mult = 2 * (int)(aux >> 28) + 1;
-    const u32 c0 = 1408u * 0x10001u;
-#pragma unroll
-    for (int l2 = 0; l2 < 2; l2++) {
-      const int l = 2 * (q4 & 1) + l2;                       // the group's l-th run of 8 weights
-      const int2 mag = ilt_lds_ld8(&S.grid[(idx >> (8 * l)) & 0xFF]);
-      const int2 neg = ilt_lds_ld8(&S.smask[(aux >> (7 * l)) & 127]);
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const u32 m = (u32)(h ? mag.y : mag.x), nb = (u32)(h ? neg.y : neg.x);
-        const u32 pe = (u32)__mul24((int)(m & 0x00FF00FF), mult), po = (u32)__mul24((int)((m >> 8) & 0x00FF00FF), mult);
-        const u32 me = __builtin_amdgcn_perm(nb, nb, 0x02020000u), mo = __builtin_amdgcn_perm(nb, nb, 0x03030101u);   // the fields of the negative weights
-        const u32 te = (pe ^ me) + (c0 - me), to = (po ^ mo) + (c0 - mo);       // 1408 +- the product, in both fields
-        hi[2 * l2 + h] = (int)__builtin_amdgcn_perm(to, te, 0x07030501u);
-        lo[2 * l2 + h] = (int)(__builtin_amdgcn_perm(to, te, 0x06020400u) ^ 0x80808080u);
-      }
-    }
-  }
-};
 
 __device__ __forceinline__ void ilt_lds_st4_untracked(void* p, u32 v) {
   asm volatile("ds_write_b32 %0, %1" :: "v"((u32)(uintptr_t)(ILT_LDS void*)p), "v"(v) : "memory");
@@ -918,331 +749,6 @@ __device__ __forceinline__ void ilt_lds_st4_untracked(void* p, u32 v) {
 __device__ __forceinline__ void ilt_lds_st8_untracked(void* p, u32 a, u32 b) {
   const uint2 v = {a, b};
   asm volatile("ds_write_b64 %0, %1" :: "v"((u32)(uintptr_t)(ILT_LDS void*)p), "v"(v) : "memory");
-}
-
-// 128 rows x 128 tokens a workgroup of eight waves (one workgroup a CU, two waves a SIMD: a
-// wave's two planes of integer sums, its float sums and the raw bytes leave no room for more);
-// wave w: rows 32*(w/2).., tokens 64*(w%2)...  TM 64 (dense): 64 rows x 128 tokens a workgroup of four waves, two or
-// three workgroups a CU -- for products whose 128-row tiles are fewer than the CUs, or leave the last round over them
-// mostly empty (a prompt's chunk on a small model's matrices); the same sums in the same order.
-template <int FMT, bool GROUPED, int TM = 128>
-__global__ __launch_bounds__(4 * TM, TM == 128 ? 1 : 2) void gemm_i8p_kernel(BfParams p) {
-  typedef I8p<FMT> F;
-  typedef typename F::Raw Raw;
-  static_assert(TM == 128 || (TM == 64 && !GROUPED), "the grouped wave layout takes eight waves");
-  constexpr int TN = 128, NA = 2, THREADS = 4 * TM, NI = 512 / THREADS;
-  // Q6_K needs the quants' sum over a block and IQ2_XXS over its even and odd groups (d4_mm_id_iq2_xxs has no argument for
-  // the sums of 16 anyway): both are added up from the slabs in LDS, which saves four 16-byte loads a thread and block.
-  constexpr bool XSLAB = FMT == ILT_IQ2_XXS || FMT == ILT_Q6_K;
-  constexpr int WL = F::WL, XL = XSLAB ? 1 : 5;               // loads of a raw set, of a token's constants
-  constexpr bool TWO = F::PLANES == 2;
-  constexpr bool SPLIT = FMT == ILT_IQ2_XXS;                 // the first and the second 32 columns of a step have sums of their own
-  constexpr int KW = 64;                                     // columns a step
-  __shared__ I8pSmemT<TM> S;
-  // Q2_K has no hi plane: its room holds the minimums' operands (sixteen groups: 16 bytes a row or token; 6 KB of the
-  // hi plane's two slabs, 8 KB at 64 rows)
-  int4* const q2_wmn = (int4*)S.wh[0];
-  int4* const q2_bh = q2_wmn + 128;
-  int4* const q2_bl = q2_bh + 128;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-
-  long tok0; int ntok, rt; const u8* w = p.w;
-  if (!pick_tile<TM, TN>(p, S, tok0, ntok, rt, w)) return;
-  const int r0 = rt * TM;
-  int* const cxo = (int*)S.wdm;                              // IQ2_XXS: cx for the even groups, this for the odd ones
-  if constexpr (FMT == ILT_IQ2_XXS) {
-    if (t < 256) S.grid[t] = bf_grid_dev[t];
-    if (t < 128) {
-      const u32 sb = (u32)t | ((__popc(t) & 1) << 7);
-      u32 m[2] = {0, 0};
-#pragma unroll
-      for (int j = 0; j < 8; j++) m[j >> 2] |= ((sb >> j) & 1) ? 0xFFu << (8 * (j & 3)) : 0u;
-      S.smask[t] = (u64)m[0] | ((u64)m[1] << 32);
-    }
-    __syncthreads();
-  }
-
-  const int wrow = t >> 2, q4 = t & 3;
-  const __amdgpu_buffer_rsrc_t rw = ilt_rsrc(ilt_uniform_ptr(w), (u32)min((long long)p.rows * p.row_bytes, 0xFFFFFFF0LL));
-  const u32 wrowoff = (u32)((long long)min(r0 + wrow, p.rows - 1) * p.row_bytes);
-  const u32 wdst = slab_off(wrow, q4);
-  const u8* xbase = (const u8*)ilt_uniform_ptr((const i8*)p.x + tok0 * (long)p.cols);
-  u32 xoff[NI];                                              // piece (wave * NI + i) * 64 + lane of a slab: token piece / 4, part piece % 4
-#pragma unroll
-  for (int i = 0; i < NI; i++) {
-    const int P = (wave * NI + i) * 64 + lane;
-    xoff[i] = (u32)min(P >> 2, ntok - 1) * (u32)p.cols + 16 * ((P & 3) ^ (int)slab_swz(P >> 2));
-  }
-  const int nk = p.cols / KW, nsb = p.cols / 256;
-  // a token's constants for a super-block, by thread t & 127 (every wave loads, so that all count the same loads)
-  const long ctok = tok0 + min(t & 127, ntok - 1);
-  const float* xdp = p.xd + ctok * nsb;
-  const int4* bsp = (const int4*)(p.bsums + ctok * (p.cols / 16));      // (IQ2_XXS: not read)
-  float c_yd; int4 c_bs[4];
-  auto load_consts = [&](int sb) {
-    c_yd = xdp[sb];
-    if constexpr (!XSLAB) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) c_bs[i] = bsp[4 * sb + i];
-    }
-  };
-  auto store_consts = [&](const Raw& ra) {                   // after a barrier that ends the last block's reads
-    if (t < 128) {
-      int sx = 0;
-      if constexpr (!XSLAB) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) sx += c_bs[i].x + c_bs[i].y + c_bs[i].z + c_bs[i].w;
-      }
-      ilt_lds_st4_untracked(&S.xd[t], __builtin_bit_cast(u32, c_yd));
-      if constexpr (!XSLAB) ilt_lds_st4_untracked(&S.cx[t], (u32)(F::KCX * sx));
-      if constexpr (FMT == ILT_Q4_K) {
-        u32 h[2] = {0, 0}, l[2] = {0, 0};
-#pragma unroll
-        for (int g = 0; g < 8; g++) {                        // the sum of group g's 32 quants
-          const int4& bs = c_bs[g >> 1];
-          const u32 u = (u32)(((g & 1) ? bs.z + bs.w : bs.x + bs.y) + 4096);
-          h[g >> 2] |= (u >> 8) << (8 * (g & 3));
-          l[g >> 2] |= ((u & 255) ^ 128) << (8 * (g & 3));
-        }
-        ilt_lds_st8_untracked(&S.bh[t], h[0], h[1]);
-        ilt_lds_st8_untracked(&S.bl[t], l[0], l[1]);
-      }
-      if constexpr (FMT == ILT_Q2_K) {
-        u32 h[4] = {0, 0, 0, 0}, l[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int g = 0; g < 16; g++) {                       // the sum of group g's 16 quants + 2048, as planes
-          const u32 u = (u32)(word_of(c_bs[g >> 2], g & 3) + 2048);
-          h[g >> 2] |= (u >> 8) << (8 * (g & 3));
-          l[g >> 2] |= ((u & 255) ^ 128) << (8 * (g & 3));
-        }
-        ilt_lds_st16_untracked(&q2_bh[t], (int)h[0], (int)h[1], (int)h[2], (int)h[3]);
-        ilt_lds_st16_untracked(&q2_bl[t], (int)l[0], (int)l[1], (int)l[2], (int)l[3]);
-      }
-    }
-    if (q4 == 0) {
-      ilt_lds_st4_untracked(&S.wd[wrow], __builtin_bit_cast(u32, F::d_of(ra)));
-      if constexpr (FMT == ILT_Q4_K) {
-        ilt_lds_st4_untracked(&S.wdm[wrow], __builtin_bit_cast(u32, F::dmin_of(ra)));
-        u32 m[2] = {0, 0}, ms = 0;
-#pragma unroll
-        for (int g = 0; g < 8; g++) { const u32 mn = F::min_of(ra, g); m[g >> 2] |= mn << (8 * (g & 3)); ms += mn; }
-        ilt_lds_st8_untracked(&S.wmn[wrow], m[0], m[1]);
-        ilt_lds_st4_untracked(&S.wms[wrow], ms);
-      }
-      if constexpr (FMT == ILT_Q2_K) {
-        ilt_lds_st4_untracked(&S.wdm[wrow], __builtin_bit_cast(u32, F::dmin_of(ra)));
-        u32 m[4], ms = 0;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {                        // the minimums: the scale bytes' high nibbles
-          m[i] = (word_of(ra.s, i) >> 4) & 0x0F0F0F0F;
-          ms += (m[i] & 0xFF) + ((m[i] >> 8) & 0xFF) + ((m[i] >> 16) & 0xFF) + (m[i] >> 24);
-        }
-        ilt_lds_st16_untracked(&q2_wmn[wrow], (int)m[0], (int)m[1], (int)m[2], (int)m[3]);
-        ilt_lds_st4_untracked(&S.wms[wrow], ms);
-      }
-    }
-  };
-  auto load_raw = [&](Raw& r, int hb) { F::load(r, rw, wrowoff, hb, q4); };       // half super-block hb of the thread's row
-  auto issue_x = [&](int stage, int ks) {
-#pragma unroll
-    for (int i = 0; i < NI; i++) ilt_g2lds16(xbase + ks * KW + xoff[i], S.xs[stage] + (wave * NI + i) * 1024);
-  };
-  // the thread's 16 weights of step J of a super-block, out of the set that holds its half, into a pair of slabs
-  auto dequant_to = [&](const Raw& r, int J, int slab) {
-    int hi[4], lo[4];
-    F::planes(r, J, q4, hi, lo, S);
-    if constexpr (TWO) ilt_lds_st16_untracked(S.wh[slab] + wdst, hi[0], hi[1], hi[2], hi[3]);
-    ilt_lds_st16_untracked(S.wl[slab] + wdst, lo[0], lo[1], lo[2], lo[3]);
-  };
-
-  v16f sum[NA][1];
-  v16i_ ah[SPLIT ? 2 : 1][NA], al[SPLIT ? 2 : 1][NA];
-  int xsum[NI] = {};                                         // IQ2_XXS, Q6_K: see the step
-#pragma unroll
-  for (int a = 0; a < NA; a++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) sum[a][0][r] = 0.0f;
-
-  // this wave's tokens and rows in the tile.  Grouped: waves 0-3 the first 64 tokens, 4-7 the second, one of each on
-  // every SIMD, and a wave whose tokens the group does not have (a group of up to 64 rows) only makes planes.
-  const int wt0 = GROUPED ? 64 * (wave >> 2) : 64 * (wave & 1), wr0 = GROUPED ? 32 * (wave & 3) : 32 * (wave >> 1);
-  const bool work = !GROUPED || __builtin_amdgcn_readfirstlane(wt0) < ntok;
-  const int l32 = lane & 31, lh = lane >> 5;
-  u32 aoff[NA];                                              // fragment offsets of the step's first 32 columns (piece lh); the second 32 at ^ 32
-#pragma unroll
-  for (int a = 0; a < NA; a++) aoff[a] = slab_off(wt0 + 32 * a + l32, lh);
-  const u32 boff = slab_off(wr0 + l32, lh);
-
-  // Raw set A holds half 0 of a super-block and B half 1, two steps each; step ks multiplies
-  // slab ks while it makes step ks+1's planes, so A is free after step 0 and loaded again (the
-  // next block's) in step 1, B after step 2 and loaded in step 3.  The next block's token
-  // constants are loaded in step 2 and stored in the next step 0.
-  Raw rawa, rawb;
-  load_raw(rawa, 0);
-  load_consts(0);
-  issue_x(0, 0);
-  load_raw(rawb, 1);
-  issue_x(1, 1);
-  int st0 = 0, st1 = 1, st2 = 2;
-  dequant_to(rawa, 0, 0);
-  store_consts(rawa);
-
-  auto step = [&](int ks, auto Jc) {
-    constexpr int J = decltype(Jc)::value;                   // the step's place in its super-block
-    // All loads but the previous step's have landed: this step's x slab has (sent two steps ago).
-    constexpr int prev = NI + ((J == 0 || J == 2) ? WL : J == 3 ? XL : 0);
-    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(prev) : "memory");
-    ilt_barrier_lds();                                       // no fence: later steps' loads stay in flight
-    const int sb = ks >> 2;
-    if (J == 0 && ks > 0) store_consts(rawa);                // (the first block's were stored before the loop)
-    if (J == 1) load_raw(rawa, min(2 * sb + 2, 2 * nsb - 1));
-    if (J == 2) load_consts(min(sb + 1, nsb - 1));
-    if (J == 3) load_raw(rawb, min(2 * sb + 3, 2 * nsb - 1));
-    issue_x(st2, min(ks + 2, nk - 1));
-    __builtin_amdgcn_sched_barrier(0);
-    const u8* xs = S.xs[st0];
-    const u8* whs = S.wh[J & 1];
-    const u8* wls = S.wl[J & 1];
-    const v16i_ zero = {};
-    if constexpr (XSLAB) {
-      // the sums of the tokens' quants over the block (IQ2_XXS: over its even and its odd groups), from the slabs: thread t
-      // adds piece t & 3 of token t / 4 (and of token t / 4 + 64 with four waves); pieces 0 and 1 are the step's even
-      // group, 2 and 3 its odd one
-#pragma unroll
-      for (int i = 0; i < NI; i++) {
-        const int4 xv = ilt_lds_ld16(xs + slab_off((t >> 2) + (THREADS / 4) * i, t & 3));
-        int sp = __builtin_amdgcn_sdot4(xv.x, 0x01010101, 0, false);
-        sp = __builtin_amdgcn_sdot4(xv.y, 0x01010101, sp, false);
-        sp = __builtin_amdgcn_sdot4(xv.z, 0x01010101, sp, false);
-        sp = __builtin_amdgcn_sdot4(xv.w, 0x01010101, sp, false);
-        sp += __shfl_xor(sp, 1);
-        if constexpr (!SPLIT) sp += __shfl_xor(sp, 2);
-        xsum[i] = J == 0 ? sp : xsum[i] + sp;
-      }
-    }
-#pragma unroll
-    for (int kk = 0; kk < 2; kk++) {
-      v4i_ af[NA] = {}, bh = {}, bl = {};
-      if (work) {
-#pragma unroll
-        for (int a = 0; a < NA; a++) af[a] = *(const v4i_*)(xs + (aoff[a] ^ (32 * kk)));
-        if constexpr (TWO) bh = *(const v4i_*)(whs + (boff ^ (32 * kk)));
-        bl = *(const v4i_*)(wls + (boff ^ (32 * kk)));
-      }
-      if (kk == 0) {       // step ks+1's planes: J+1 = 1 from A, 2 and 3 from B, 4 = the next block's 0 from A (past the last step: planes nobody reads)
-        if (J == 0) dequant_to(rawa, 1, 1);
-        if (J == 1) dequant_to(rawb, 2, 0);
-        if (J == 2) dequant_to(rawb, 3, 1);
-        if (J == 3) dequant_to(rawa, 0, 0);
-      }
-      if (work) {
-#pragma unroll
-        for (int a = 0; a < NA; a++) {                       // a super-block's first products start its integer sums
-          constexpr int ps = 0;
-          const int pk = SPLIT ? kk : ps;
-          const bool first = J == 0 && (SPLIT || kk == 0);
-          if constexpr (TWO) ah[pk][a] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[a], bh, first ? zero : ah[pk][a], 0, 0, 0);
-          al[pk][a] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[a], bl, first ? zero : al[pk][a], 0, 0, 0);
-        }
-      }
-    }
-    if constexpr (XSLAB) {
-      if (J == 3) {        // the block's sums of quants, for everyone's terms below
-#pragma unroll
-        for (int i = 0; i < NI; i++) {
-          if ((t & 3) == 0) ilt_lds_st4_untracked(&S.cx[(t >> 2) + (THREADS / 4) * i], (u32)(F::KCX * xsum[i]));
-          if (SPLIT && (t & 3) == 2) ilt_lds_st4_untracked(&cxo[(t >> 2) + (THREADS / 4) * i], (u32)(F::KCX * xsum[i]));
-        }
-        ilt_barrier_lds();
-      }
-    }
-    if (J == 3 && work) {  // the super-block is complete: its terms, as the CPU path adds them
-      const int row = wr0 + l32;
-      const float d = S.wd[row];
-      if constexpr (FMT == ILT_Q4_K) {
-        // im = sum over the groups of minimum * (sum of 32 quants) = 256*(mn.hi) + (mn.lo) - 3968*(sum of mn)
-        const float dm = S.wdm[row];
-        const int ms = 3968 * S.wms[row];
-        const int2 mnb = S.wmn[row];
-        const v4i_ bm = { lh ? 0 : mnb.x, lh ? 0 : mnb.y, 0, 0 };
-#pragma unroll
-        for (int a = 0; a < NA; a++) {
-          const int2 th = S.bh[wt0 + 32 * a + l32], tl = S.bl[wt0 + 32 * a + l32];
-          const v4i_ fh = { lh ? 0 : th.x, lh ? 0 : th.y, 0, 0 }, fl = { lh ? 0 : tl.x, lh ? 0 : tl.y, 0, 0 };
-          const v16i_ mh = __builtin_amdgcn_mfma_i32_32x32x32_i8(fh, bm, zero, 0, 0, 0);
-          const v16i_ ml = __builtin_amdgcn_mfma_i32_32x32x32_i8(fl, bm, zero, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 16; r++) {
-            const int tk = wt0 + 32 * a + 8 * (r >> 2) + 4 * lh + (r & 3);
-            const float yd = S.xd[tk];
-            const int im = 256 * mh[r] + ml[r] - ms;
-            const int isum = 256 * ah[0][a][r] + al[0][a][r] - S.cx[tk];
-            sum[a][0][r] = sum[a][0][r] - (yd * dm) * (float)im;
-            sum[a][0][r] = sum[a][0][r] + (yd * d) * (float)isum;
-          }
-        }
-      } else if constexpr (FMT == ILT_IQ2_XXS) {
-#pragma unroll
-        for (int a = 0; a < NA; a++) {
-#pragma unroll
-          for (int r = 0; r < 16; r++) {
-            const int tk = wt0 + 32 * a + 8 * (r >> 2) + 4 * lh + (r & 3);
-            const float fa = (float)(256 * ah[0][a][r] + al[0][a][r] - S.cx[tk]) * 0.5f;
-            const float fb = (float)(256 * ah[1][a][r] + al[1][a][r] - cxo[tk]) * 0.5f;
-            sum[a][0][r] = sum[a][0][r] + (d * S.xd[tk]) * (fa + fb);
-          }
-        }
-      } else if constexpr (FMT == ILT_Q2_K) {
-        // im = sum over the sixteen groups of minimum * (sum of 16 quants) = 256*(mn.hi) + (mn.lo) - 1920*(sum of mn)
-        const float dm = S.wdm[row];
-        const int ms = 1920 * S.wms[row];
-        const int4 mnb = q2_wmn[row];
-        const v4i_ bm = { lh ? 0 : mnb.x, lh ? 0 : mnb.y, lh ? 0 : mnb.z, lh ? 0 : mnb.w };
-#pragma unroll
-        for (int a = 0; a < NA; a++) {
-          const int4 th = q2_bh[wt0 + 32 * a + l32], tl = q2_bl[wt0 + 32 * a + l32];
-          const v4i_ fh = { lh ? 0 : th.x, lh ? 0 : th.y, lh ? 0 : th.z, lh ? 0 : th.w };
-          const v4i_ fl = { lh ? 0 : tl.x, lh ? 0 : tl.y, lh ? 0 : tl.z, lh ? 0 : tl.w };
-          const v16i_ mh = __builtin_amdgcn_mfma_i32_32x32x32_i8(fh, bm, zero, 0, 0, 0);
-          const v16i_ ml = __builtin_amdgcn_mfma_i32_32x32x32_i8(fl, bm, zero, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 16; r++) {
-            const int tk = wt0 + 32 * a + 8 * (r >> 2) + 4 * lh + (r & 3);
-            const float yd = S.xd[tk];
-            const int im = 256 * mh[r] + ml[r] - ms;
-            sum[a][0][r] = sum[a][0][r] + ((-yd) * dm) * (float)im;
-            sum[a][0][r] = sum[a][0][r] + (yd * d) * (float)al[0][a][r];
-          }
-        }
-      } else {
-#pragma unroll
-        for (int a = 0; a < NA; a++) {
-#pragma unroll
-          for (int r = 0; r < 16; r++) {
-            const int tk = wt0 + 32 * a + 8 * (r >> 2) + 4 * lh + (r & 3);
-            const int isum = 256 * ah[0][a][r] + al[0][a][r] - S.cx[tk];
-            sum[a][0][r] = sum[a][0][r] + (d * S.xd[tk]) * (float)isum;
-          }
-        }
-      }
-    }
-    const int s_ = st0; st0 = st1; st1 = st2; st2 = s_;
-  };
-  for (int ks = 0; ks < nk; ks += 4) {     // one super-block of 256 columns
-    step(ks + 0, std::integral_constant<int, 0>{});
-    step(ks + 1, std::integral_constant<int, 1>{});
-    step(ks + 2, std::integral_constant<int, 2>{});
-    step(ks + 3, std::integral_constant<int, 3>{});
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the tail's redundant loads: nothing may land in LDS after the workgroup ends
-
-  if constexpr (FMT == ILT_IQ2_XXS) {
-#pragma unroll
-    for (int a = 0; a < NA; a++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) sum[a][0][r] = 0.25f * sum[a][0][r];
-  }
-  store_tile<NA, 1>(sum, p, tok0, ntok, r0, wt0, wr0, l32, lh);
 }
 
 // ---- the exact Q8_0 product on the same pipeline -------------------------------------------------
@@ -1343,15 +849,41 @@ __global__ __launch_bounds__(512, 2) void gemm_i8q_kernel(BfParams p) {
 }
 
 // ---- the exact product in two passes: the planes once, then a loop without dequantization -------
-// As for bf16: with thousands of tokens (or a matrix multiplied again and again) the two planes
-// of a Q6_K matrix are worth writing out once -- a byte a weight each, in slabs of 128 rows x 64
-// columns (the row count padded to a multiple of 128), and d per row and super-block as floats -- so that the product's loop holds only direct loads of
-// three slabs, fragment reads, MFMAs and the combine per super-block.  The same integers, the
-// same float expression per block: the same bits as gemm_i8p_kernel and the CPU path.
-template <int FMT>
+// Per super-block the CPU path's MATMUL! forms an integer isum = sum over its 256 columns of (scale * (quant - 32)) * xq, then
+// sum += (d*yd) * float(isum) (kquant.lisp:206-236).  Any exact way to the integer will do, so the products P = sc*(q-32)
+// (13 bits) go to the int8 matrix cores as two planes, the bytes of T = P + 4128 >= 0: hi = T >> 8 (0..31) and
+// lo = (T & 255) - 128, so isum = 256*(hi.xq) + (lo.xq) - 4000*(sum of the block's xq).  As for bf16: with thousands of tokens
+// (or a matrix multiplied again and again) the two planes of a Q6_K matrix are worth writing out once -- a byte a weight each,
+// in slabs of 128 rows x 64 columns (the row count padded to a multiple of 128), and d per row and super-block as floats -- so
+// that the product's loop holds only direct loads of three slabs, fragment reads, MFMAs and the combine per super-block.  The
+// same integers, the same float expression per block: the same bits as gemm_i8r_kernel and the CPU path.
+// Thread (row, q4) makes columns 16*q4.. of its row in every step of 64 columns: part 2*jj + q4/2 of half c (jj = the step
+// within the half), weights 16*(q4 & 1).. of the part.  Four weights are made at a time: the even and the odd bytes of a word
+// as two 16-bit fields and one 24-bit multiply-add for both (each field's total is within 0..65535, so borrows between them
+// cancel).
+struct PlanesRaw { int4 ql, qh; int2 sc; u32 d; };           // a half super-block's share
+__device__ __forceinline__ void planes_load(PlanesRaw& r, __amdgpu_buffer_rsrc_t rw, u32 rowoff, int hb, int q4) {
+  const u32 b = rowoff + (u32)(hb >> 1) * ILT_Q6K_STRIDE;
+  const int c = hb & 1;
+  r.ql = ilt_bld16(rw, b + 64 * c + 16 * q4);                // ql[64c + 32*(part & 1) + l], part & 1 = q4 / 2, l = 16*(q4 & 1)..
+  r.qh = ilt_bld16(rw, b + 128 + 32 * c + 16 * (q4 & 1));
+  r.sc = ilt_bld8(rw, b + 192 + 8 * c);
+  r.d = ilt_bld2(rw, b + 208);
+}
+// jj: the step within the half
+__device__ __forceinline__ void planes_of(const PlanesRaw& r, int jj, int q4, int* hi, int* lo) {
+  const int sc = (int)(i8)(((u32)(jj ? r.sc.y : r.sc.x) >> (8 * q4)) & 0xFF);      // scale 8c + 2*part + (q4 & 1)
+  const int cpair = (4128 - 32 * sc) * 0x10001;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const u32 v = ((word_of(r.ql, i) >> (4 * jj)) & 0x0F0F0F0F) | (((word_of(r.qh, i) >> (4 * jj + 2 * (q4 >> 1))) & 0x03030303) << 4);
+    const u32 te = (u32)(__mul24((int)(v & 0x00FF00FF), sc) + cpair), to = (u32)(__mul24((int)((v >> 8) & 0x00FF00FF), sc) + cpair);
+    hi[i] = (int)__builtin_amdgcn_perm(to, te, 0x07030501u);                  // the fields' high bytes, in the weights' order
+    lo[i] = (int)(__builtin_amdgcn_perm(to, te, 0x06020400u) ^ 0x80808080u);   // their low bytes - 128
+  }
+}
 __global__ __launch_bounds__(256) void planes_i8_kernel(const u8* __restrict__ w, long long row_bytes, int rows, int cols,
                                                         u8* __restrict__ wh, u8* __restrict__ wl, float* __restrict__ wdf) {
-  typedef I8p<FMT> F;
   const int nsb = cols / 256;
   const long long u = (long long)blockIdx.x * 256 + threadIdx.x;       // 16 weights: unit q4 of step J of a super-block of a row
   if (u >= (long long)rows * nsb * 16) return;
@@ -1360,22 +892,17 @@ __global__ __launch_bounds__(256) void planes_i8_kernel(const u8* __restrict__ w
   const int sb = (int)(sr % nsb);
   const long long row = sr / nsb;
   const __amdgpu_buffer_rsrc_t rw = ilt_rsrc(ilt_uniform_ptr(w), (u32)min((long long)rows * row_bytes, 0xFFFFFFF0LL));
-  typename F::Raw r;
-  F::load(r, rw, (u32)(row * row_bytes), 2 * sb + (J >> 1), q4);
+  PlanesRaw r;
+  planes_load(r, rw, (u32)(row * row_bytes), 2 * sb + (J >> 1), q4);
   int hi[4], lo[4];
-  const int dummy = 0;
-  switch (J) {            // (the step is a constant inside planes)
-    case 0: F::planes(r, 0, q4, hi, lo, dummy); break;
-    case 1: F::planes(r, 1, q4, hi, lo, dummy); break;
-    case 2: F::planes(r, 2, q4, hi, lo, dummy); break;
-    default: F::planes(r, 3, q4, hi, lo, dummy); break;
-  }
+  if (J & 1) planes_of(r, 1, q4, hi, lo);            // (the step is a constant inside)
+  else planes_of(r, 0, q4, hi, lo);
   // slab order: the 64 columns of a step for 128 consecutive rows are 8 KB in one piece (row r of the group at 64*r),
   // the groups' slabs for step 0, 1, ... one after another, so that the product's direct loads read whole lines
   const long long o = ((row >> 7) * (cols / 64) + sb * 4 + J) * 8192 + (row & 127) * 64 + 16 * q4;
   *(int4*)(wh + o) = make_int4(hi[0], hi[1], hi[2], hi[3]);
   *(int4*)(wl + o) = make_int4(lo[0], lo[1], lo[2], lo[3]);
-  if (J == 0 && q4 == 0) wdf[row * nsb + sb] = F::d_of(r);
+  if (J == 0 && q4 == 0) wdf[row * nsb + sb] = ilt_h2f((u16)r.d);
 }
 
 // NB row patches a wave: 1 = eight waves of 32 rows x 64 tokens (one workgroup a CU, slabs four steps ahead).
@@ -1950,47 +1477,13 @@ hipError_t ilt_k_gemm_bf16_id_glu(int fmt, const uint64_t* ptrs, long long add_g
   return launch_regb<ILT_IQ2_XXS, true>(p, total_rows / 128 + ne, st);
 }
 
-// 64-row tiles (dense) where the 128-row tiles would leave CUs idle: fewer tiles than one and a half rounds over the
-// 256 CUs, or a last round less than half full.  ILT_I8P_TM (tests): 64 or 128 whatever the shape.
-static int i8p_tile_rows(long long tiles128) {
-  const char* force = getenv("ILT_I8P_TM");
-  if (force && (atoi(force) == 64 || atoi(force) == 128)) return atoi(force);
-  const long long rem = tiles128 % 256;
-  return (tiles128 < 384 || (tiles128 < 1024 && rem != 0 && rem < 128)) ? 64 : 128;
-}
-
-static bool i8p_grid(const BfParams& p, long long token_tiles, int tm, dim3& grid) {
-  if (p.cols % 256 != 0 || (long long)p.rows * 1024 >= 0x7FFFFFFFLL) return false;
-  const long long total = token_tiles * ((p.rows + tm - 1) / tm), per = (total + 7) / 8;
-  if (per * 8 > 0x7FFFFFFFLL) return false;
-  grid = dim3((unsigned)(per * 8));
-  return true;
-}
-
-hipError_t ilt_k_gemm_i8_planes(const uint8_t* w, long long row_bytes, int rows, int cols, const int8_t* xq, const float* xd,
-                                const int* bsums, int ntok, float* y, const float* bias, int acc, hipStream_t st, long long ldy) {
-  if (ntok <= 0 || rows <= 0) return hipSuccess;
-  if (ldy == 0) ldy = rows;
-  if (ldy < rows || ldy * 1024 >= 0x7FFFFFFFLL) return hipErrorInvalidValue;
-  BfParams p = {};
-  p.w = w; p.rows = rows; p.cols = cols; p.row_bytes = row_bytes; p.x = (const u16*)xq; p.xd = xd; p.bsums = bsums;
-  p.y = y; p.bias = bias; p.acc = acc; p.ntok = ntok; p.ldy = ldy;
-  const long long tt = (ntok + 127) / 128;
-  const int tm = i8p_tile_rows(tt * ((rows + 127) / 128));
-  dim3 grid;
-  if (!i8p_grid(p, tt, tm, grid)) return hipErrorInvalidValue;
-  if (tm == 64) hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q2_K, false, 64>), grid, dim3(256), 0, st, p);
-  else hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q2_K, false>), grid, dim3(512), 0, st, p);
-  return hipGetLastError();
-}
-
 hipError_t ilt_k_planes_i8(int fmt, const uint8_t* w, long long row_bytes, int rows, int cols, uint8_t* wh, uint8_t* wl, float* wdf,
                            hipStream_t st) {
   if (rows <= 0) return hipSuccess;
   if (fmt != ILT_Q6_K || cols % 256 != 0 || (long long)rows * row_bytes >= 0xFFFFFFF0LL) return hipErrorInvalidValue;
   const long long units = (long long)rows * (cols / 256) * 16;
   if ((units + 255) / 256 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(planes_i8_kernel<ILT_Q6_K>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, w, row_bytes, rows, cols, wh, wl, wdf);
+  hipLaunchKernelGGL(planes_i8_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, w, row_bytes, rows, cols, wh, wl, wdf);
   return hipGetLastError();
 }
 
@@ -2026,27 +1519,6 @@ hipError_t ilt_k_gemm_i8_q8(const uint8_t* wq, const uint16_t* wd, int rows, int
   const long long total = (long long)((ntok + 127) / 128) * ((rows + 127) / 128), per = (total + 7) / 8;
   if (per * 8 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
   hipLaunchKernelGGL(gemm_i8q_kernel, dim3((unsigned)(per * 8)), dim3(512), 0, st, p);
-  return hipGetLastError();
-}
-
-hipError_t ilt_k_gemm_i8_planes_id(int fmt, const uint64_t* ptrs, long long add, const uint32_t* counts, const uint32_t* bases, int ne,
-                                   long long row_bytes, int rows, int cols, const int8_t* xq, const float* xd, const int* bsums,
-                                   long long total_rows, float* y, hipStream_t st) {
-  if (total_rows <= 0 || rows <= 0 || ne <= 0) return hipSuccess;
-  if (ne > 256) return hipErrorInvalidValue;
-  BfParams p = {};
-  p.ptrs = ptrs; p.add = add; p.counts = counts; p.bases = bases; p.ne = ne;
-  p.rows = rows; p.cols = cols; p.row_bytes = row_bytes; p.x = (const u16*)xq; p.xd = xd; p.bsums = bsums;
-  p.y = y; p.ntok = (int)total_rows; p.ldy = rows;
-  dim3 grid;
-  if (!i8p_grid(p, total_rows / 128 + ne, 128, grid)) return hipErrorInvalidValue;
-  switch (fmt) {
-    case ILT_Q6_K: hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q6_K, true>), grid, dim3(512), 0, st, p); break;
-    case ILT_Q4_K: hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q4_K, true>), grid, dim3(512), 0, st, p); break;
-    case ILT_Q2_K: hipLaunchKernelGGL((gemm_i8p_kernel<ILT_Q2_K, true>), grid, dim3(512), 0, st, p); break;
-    case ILT_IQ2_XXS: hipLaunchKernelGGL((gemm_i8p_kernel<ILT_IQ2_XXS, true>), grid, dim3(512), 0, st, p); break;
-    default: return hipErrorInvalidValue;
-  }
   return hipGetLastError();
 }
 

@@ -8,6 +8,7 @@
 //   Q4_K: a scale is two digits, sc = 8 sh + sl, and q * digit is at most 105: four bytes times a digit is one 16-bit packed
 //         multiply with no carry between them.  isum = 8 * (sh q . xq) + (sl q . xq).
 //   Q6_K: T = sc (q - 32) = 256 hi + lo with lo signed: 16-bit fields, one packed multiply-add for two weights.
+//   Q2_K: sc * q is at most 45, one plane; IQ2_XXS: a group's sums scaled by the lanes (below).
 // The minimums (Q4_K) are one f16 product of the tokens' sums of 32, in two parts of seven bits, with the 6-bit minimums:
 // whole numbers below 2^21, exact in its single-precision sums.
 //
@@ -26,6 +27,7 @@
 // 62 -> 40; 110 -> 79; 1,400 -> 985 (741 TFLOP/s).
 #include "ilt_device.h"
 #include "ilt_gemm_tile.h"
+#include "ilt_iq2xxs_tables.h"
 #include "ilt_kernels.h"
 #include <stdlib.h>
 #include <type_traits>
@@ -54,19 +56,19 @@ template <int FMT> struct RegW;
 template <> struct RegW<ILT_Q4_K> {
   static constexpr int BLOCK = 144;
   static constexpr bool MINS = true;
-  static constexpr int SH = 3;              // isum = (hi sums << SH) + (lo sums)
+  static constexpr int PLANES = 2, SH = 3;  // isum = (hi sums << SH) + (lo sums)
   struct Block { u32 sc[2]; float d, dm; v8h mins; };
   struct Quants { int4 q[2]; };
   // In LDS: the quants of eight rows a kilobyte, piece p of row r at p ^ (r >> 1 & 7); behind them a header a row.
   static constexpr int LOADS = 5, LBYTES = 5120;             // direct loads, bytes of LDS for 32 rows
   struct At { u32 a, b, h; };
-  static __device__ __forceinline__ At place(u32 row_bytes, int lane) {
+  static __device__ __forceinline__ At place(u32 row_bytes, int lane, int, int) {
     const u32 pc = 16 * (u32)((lane & 7) ^ ((lane >> 4) & 3)), rr = (u32)(lane >> 3) * row_bytes + 16;
     return At{rr + pc, rr + (pc ^ 64), (u32)(lane & 31) * row_bytes};
   }
-  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t rw, const At& at, u32 row_bytes, u32 base, u8* dst) {
-    if (i < 4) __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 1024 * i), 16, i & 1 ? at.b : at.a, base + 8 * i * row_bytes, 0, 0);
-    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 4096), 16, at.h, base, 0, 0);
+  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t rw, const u8*, const At& at, u32 row_bytes, u32 row0, u32 block, u8* dst) {
+    if (i < 4) __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 1024 * i), 16, (i & 1 ? at.b : at.a) + (row0 + 8 * i) * row_bytes, block, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 4096), 16, at.h + row0 * row_bytes, block, 0, 0);
   }
   static __device__ __forceinline__ void block(Block& o, const u8* src, int l32, int) {
     const int4 h = ilt_lds_ld16(src + 4096 + 16 * l32);
@@ -88,7 +90,7 @@ template <> struct RegW<ILT_Q4_K> {
     if (g % 2 == 0) o.q[(g >> 1) & 1] = ilt_lds_ld16(src + 128 * l32 + 16 * ((g + lh) ^ ((l32 >> 1) & 7)));
   }
   static __device__ __forceinline__ void quants_now(Quants&, const u8*, int, int, int) {}
-  static __device__ __forceinline__ void group(const Block& b, const Quants& r, int g, int, v4i& hi, v4i& lo) {
+  static __device__ __forceinline__ void group(Block& b, const Quants& r, int g, int, v4i& hi, v4i& lo) {
     const v2u l = splat<0>((b.sc[g >> 2] >> (8 * (g & 3))) & 7), h = splat<0>((b.sc[g >> 2] >> (8 * (g & 3) + 3)) & 7);
 #pragma unroll
     for (int k = 0; k < 4; k++) {
@@ -103,17 +105,17 @@ template <> struct RegW<ILT_Q4_K> {
 template <> struct RegW<ILT_Q6_K> {
   static constexpr int BLOCK = ILT_Q6K_STRIDE;
   static constexpr bool MINS = false;
-  static constexpr int SH = 8;
+  static constexpr int PLANES = 2, SH = 8;
   struct Block { int4 sc; float d, dm; v8h mins; };
   struct Quants { int4 l[2], h; };
   // In LDS: four rows a kilobyte and 64 bytes, piece p of row r at p ^ (r & 3) of its 256; piece 13 the block's last 16 bytes.
   static constexpr int LOADS = 8, LBYTES = 8704;
   struct At { u32 a; };
-  static __device__ __forceinline__ At place(u32 row_bytes, int lane) {
+  static __device__ __forceinline__ At place(u32 row_bytes, int lane, int, int) {
     return At{(u32)(lane >> 4) * row_bytes + min(16u * (u32)((lane & 15) ^ (lane >> 4)), 196u)};
   }
-  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t rw, const At& at, u32 row_bytes, u32 base, u8* dst) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 1088 * i), 16, at.a, base + 4 * i * row_bytes, 0, 0);
+  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t rw, const u8*, const At& at, u32 row_bytes, u32 row0, u32 block, u8* dst) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 1088 * i), 16, at.a + (row0 + 4 * i) * row_bytes, block, 0, 0);
   }
   static __device__ __forceinline__ const u8* row_of(const u8* src, int l32) { return src + (l32 >> 2) * 1088 + (l32 & 3) * 256; }
   static __device__ __forceinline__ void block(Block& o, const u8* src, int l32, int) {
@@ -132,7 +134,7 @@ template <> struct RegW<ILT_Q6_K> {
   static __device__ __forceinline__ void quants_now(Quants& o, const u8* src, int g, int l32, int lh) {
     if (g % 4 == 0) o.h = ilt_lds_ld16(row_of(src, l32) + 16 * ((8 + 2 * (g >> 2) + lh) ^ (l32 & 3)));
   }
-  static __device__ __forceinline__ void group(const Block& b, const Quants& r, int g, int lh, v4i& hi, v4i& lo) {
+  static __device__ __forceinline__ void group(Block& b, const Quants& r, int g, int lh, v4i& hi, v4i& lo) {
     const int j = g & 3;                             // columns 32g + 16lh ..: scale 2g + lh
     const int s = (int)(i8)((wordr(b.sc, g >> 1) >> (8 * lh)) >> (16 * (g & 1)));
     const u32 kk = (u32)(128 - 32 * s);
@@ -148,49 +150,182 @@ template <> struct RegW<ILT_Q6_K> {
   }
 };
 
-template <int TN, int RAW, bool MINS> struct RegSmem {
+// Q2_K: scale * quant is at most 45, one plane.  In LDS: eight rows a kilobyte, piece p of row r at p ^ (r >> 1 & 7); piece 5
+// the block's last 16 bytes.
+template <> struct RegW<ILT_Q2_K> {
+  static constexpr int BLOCK = 84;
+  static constexpr bool MINS = true;
+  static constexpr int PLANES = 1, SH = 0;
+  struct Block { u32 sc[4]; float d, dm; v8h mins; };
+  struct Quants { int4 q[2]; };
+  static constexpr int LOADS = 4, LBYTES = 4096;
+  struct At { u32 a, b; };
+  static __device__ __forceinline__ At place(u32 row_bytes, int lane, int, int) {
+    const u32 pc = (u32)((lane & 7) ^ ((lane >> 4) & 3)), rr = (u32)(lane >> 3) * row_bytes;
+    return At{rr + min(16 * pc, 68u), rr + min(16 * (pc ^ 4), 68u)};
+  }
+  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t rw, const u8*, const At& at, u32 row_bytes, u32 row0, u32 block, u8* dst) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 1024 * i), 16, (i & 1 ? at.b : at.a) + (row0 + 8 * i) * row_bytes, block, 0, 0);
+  }
+  static __device__ __forceinline__ void block(Block& o, const u8* src, int l32, int lh) {
+    const u8* row = src + 128 * l32;
+    const int x = (l32 >> 1) & 7;
+    const int4 s = ilt_lds_ld16(row + 16 * x);
+    const u32 dd = *ILT_LDS_PTR(const u32, row + 16 * (5 ^ x) + 12);
+    o.d = ilt_h2f((u16)(dd & 0xFFFF));
+    o.dm = ilt_h2f((u16)(dd >> 16));
+#pragma unroll
+    for (int i = 0; i < 4; i++) o.sc[i] = wordr(s, i) & 0x0F0F0F0Fu;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {                    // the minimums of groups 8 lh ..
+      const u32 m = ((u32)(lh ? wordr(s, 2 + i) : wordr(s, i)) >> 4) & 0x0F0F0F0Fu;
+      const v2h k = {(_Float16)1024.0f, (_Float16)1024.0f};
+      const v2h m01 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0, m, 0x0C010C00u) | 0x64006400u) - k;
+      const v2h m23 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0, m, 0x0C030C02u) | 0x64006400u) - k;
+      o.mins[4 * i] = m01[0]; o.mins[4 * i + 1] = m01[1]; o.mins[4 * i + 2] = m23[0]; o.mins[4 * i + 3] = m23[1];
+    }
+  }
+  // a half's four groups share 16 bytes, two bits each
+  static __device__ __forceinline__ void quants(Quants& o, const u8* src, int g, int l32, int lh) {
+    if (g % 4 == 0) o.q[g >> 2] = ilt_lds_ld16(src + 128 * l32 + 16 * ((1 + 2 * (g >> 2) + lh) ^ ((l32 >> 1) & 7)));
+  }
+  static __device__ __forceinline__ void quants_now(Quants&, const u8*, int, int, int) {}
+  static __device__ __forceinline__ void group(Block& b, const Quants& r, int g, int lh, v4i&, v4i& lo) {
+    const v2u s = splat<0>((b.sc[g >> 1] >> (8 * lh + 16 * (g & 1))) & 15);       // scale 2g + lh
+#pragma unroll
+    for (int k = 0; k < 4; k++) lo[k] = (int)asw(as2((wordr(r.q[g >> 2], k) >> (2 * (g & 3))) & 0x03030303u) * s);
+  }
+};
+
+// IQ2_XXS: a block's eight groups of 32 weights add (float(sumi) * (0.5 + scale)) alternately to two sums, and the block's term
+// is (d yd) times the two together (iquant.lisp:161-215).  Every partial sum is a multiple of 1/2 whose double stays below 2^24
+// (test_oracle.py asserts it from the codebook), so nothing rounds before the two meet, and their sum is float(isum) / 2 for
+// isum = sum of (2 scale + 1) * sumi.  The signed codebook entries (at most 43) are the operand and a group is one MFMA, whose
+// results are scaled by the lanes (a row's scale is its lane's own): as two planes of scaled weights the entries take three
+// times the arithmetic, which is what groups of a few tokens would wait for.
+// In LDS: a row's 64 bytes of indices and signs, piece p of row r at p ^ (r >> 2 & 3), and behind them 16 bytes with its d.
+__device__ const u64 iq2_grid_reg[256] = { ILT_IQ2XXS_GRID_VALUES };
+__device__ __forceinline__ u64* iq2_tables() {       // the codebook, and the byte masks of the 128 sign patterns
+  __shared__ u64 tab[384];
+  return tab;
+}
+__device__ __forceinline__ void iq2_tables_load(int t, int threads) {       // a barrier follows
+  u64* const tab = iq2_tables();
+  for (int i = t; i < 384; i += threads) {
+    u64 v;
+    if (i < 256) v = iq2_grid_reg[i];
+    else {
+      const u32 s = (u32)(i - 256) | ((u32)(__popc(i - 256) & 1) << 7);
+      u32 m[2] = {0, 0};
+#pragma unroll
+      for (int j = 0; j < 8; j++) m[j >> 2] |= (s >> j) & 1 ? 0xFFu << (8 * (j & 3)) : 0u;
+      v = (u64)m[0] | ((u64)m[1] << 32);
+    }
+    tab[i] = v;
+  }
+}
+template <> struct RegW<ILT_IQ2_XXS> {
+  static constexpr int BLOCK = 66;
+  static constexpr bool MINS = false;
+  static constexpr int PLANES = 0, SH = 0;           // PLANES 0: a group's sums scaled by the lanes
+  struct Block { u32 sc; float d, dm; v8h mins; };   // the groups' scales, four bits each
+  struct Quants { int4 q[2]; int2 mag[2], neg[2]; };
+  static constexpr int LOADS = 3, LBYTES = 3072;
+  struct At { u32 a[2], h; };
+  // (the blocks are two-byte aligned; a row past the matrix's is its last one)
+  static __device__ __forceinline__ At place(u32 row_bytes, int lane, int row0, int rows) {
+    At o;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      o.a[i] = (u32)min(row0 + 16 * i + (lane >> 2), rows - 1) * row_bytes + 2 + 16 * (u32)((lane & 3) ^ ((lane >> 4) & 3));
+    o.h = (u32)min(row0 + (lane & 31), rows - 1) * row_bytes;
+    return o;
+  }
+  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t, const u8* w, const At& at, u32, u32, u32 block, u8* dst) {
+    ilt_g2lds16(w + (size_t)block + (i < 2 ? at.a[i] : at.h), dst + 1024 * i);
+  }
+  static __device__ __forceinline__ void block(Block& o, const u8* src, int l32, int) {
+    o.sc = 0;
+    o.d = ilt_h2f(*ILT_LDS_PTR(const u16, src + 2048 + 16 * l32));
+  }
+  static __device__ __forceinline__ void quants(Quants& o, const u8* src, int g, int l32, int) {
+    if (g % 2 == 0) o.q[(g >> 1) & 1] = ilt_lds_ld16(src + 64 * l32 + 16 * ((g >> 1) ^ ((l32 >> 2) & 3)));
+  }
+  static __device__ __forceinline__ u32 index_word(const Quants& r, int g) { return wordr(r.q[(g >> 1) & 1], 2 * (g & 1)); }
+  static __device__ __forceinline__ u32 sign_word(const Quants& r, int g) { return wordr(r.q[(g >> 1) & 1], 2 * (g & 1) + 1); }
+  // the table entries of the lane's two runs of eight weights
+  static __device__ __forceinline__ void quants_now(Quants& o, const u8*, int g, int, int lh) {
+    const u64* const tab = iq2_tables();
+    const u32 idx = index_word(o, g) >> (16 * lh), sg = sign_word(o, g) >> (14 * lh);
+#pragma unroll
+    for (int l = 0; l < 2; l++) {
+      o.mag[l] = ilt_lds_ld8(tab + ((idx >> (8 * l)) & 0xFF));
+      o.neg[l] = ilt_lds_ld8(tab + 256 + ((sg >> (7 * l)) & 127));
+    }
+  }
+  static __device__ __forceinline__ void group(Block& b, const Quants& r, int g, int, v4i&, v4i& lo) {
+    b.sc |= (sign_word(r, g) >> 28) << (4 * g);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const u32 m = (u32)(k & 1 ? r.neg[k >> 1].y : r.neg[k >> 1].x), v = (u32)(k & 1 ? r.mag[k >> 1].y : r.mag[k >> 1].x);
+      lo[k] = (int)((v ^ m) + (m & 0x01010101u));    // (no entry is zero: no carry between the bytes)
+    }
+  }
+  static __device__ __forceinline__ int scale(const Block& b, int g) { return (int)(2 * ((b.sc >> (4 * g)) & 15) + 1); }
+};
+
+template <int TN, int RAW, bool MINS, int XB = 1> struct RegSmem {
   // the tokens' quants of a super-block: four tokens a kilobyte and 64 bytes, piece p of token t at p ^ (t & 3) of its 256
-  __align__(16) u8 xs[TN / 4 * 1088];
-  __align__(16) u8 ms[3][MINS ? TN * 32 : 16];          // the sums of 32 as halves: eight times 128 * (sum >> 7), eight times sum & 127
+  __align__(16) u8 xs[XB][TN / 4 * 1088];
+  __align__(16) u8 ms[3][MINS ? TN * 32 : 16];          // the sums of 32 as halves: eight times 128 * (sum >> 7), eight times sum & 127 (Q2_K: the sums of 16, exact as they are)
   __align__(16) u8 ws[RAW];                 // the rows' blocks
   float xd[3][TN];
 };
-template <int FMT, int WR, int WT> constexpr int raw_bytes() { return (WT == 1 ? 1 : 2) * WR * RegW<FMT>::LBYTES; }
+template <int FMT, int NP, int WR, int WT> constexpr int raw_bytes() { return (WT == 1 && NP > 1 ? 1 : 2) * WR * RegW<FMT>::LBYTES; }
+template <int FMT, int NP, int WR, int WT> using RegSmemOf = RegSmem<32 * NP * WT, raw_bytes<FMT, NP, WR, WT>(), RegW<FMT>::MINS, NP == 1 ? 2 : 1>;
 
-// Rows r0 .. of one matrix (rows of them, results to y) x tokens tok0 .. tok0 + ntok - 1: WR x WT waves of 32 rows x 32 NP tokens
+// Rows r0 .. of one matrix (p.rows of them, results to p.y) x tokens tok0 .. tok0 + ntok - 1: WR x WT waves of 32 rows x 32 NP
+// tokens.  NP 1: nothing to share out between two halves, so the tokens and the rows' blocks are in two buffers and a block ahead.
 template <int FMT, int NP, int WR, int WT>
 __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0, long tok0, int ntok, unsigned char* smem) {
   using F = RegW<FMT>;
   constexpr int TN = 32 * NP * WT, THREADS = 64 * WR * WT;
-  constexpr int NI = TN / (8 * WR * WT);             // direct loads of a wave a super-block's half of the tokens (four tokens each)
+  constexpr bool DEEP = NP == 1;
+  constexpr int NI = DEEP ? 8 / WR : TN / (8 * WR * WT);       // direct loads of a wave a super-block's half (NP 1: all) of the tokens (four tokens each)
   constexpr int NW = (F::LOADS + WT - 1) / WT;       // and of the rows' blocks
-  static_assert((NP == 2 || NP == 4) && 2 * TN == THREADS, "a thread a half token's sums");
-  using Smem = RegSmem<TN, raw_bytes<FMT, WR, WT>(), F::MINS>;
+  static_assert((NP == 1 ? WT == 1 && 8 % WR == 0 : NP == 2 || NP == 4) && 2 * TN <= THREADS, "a thread a half token's sums");
+  using Smem = RegSmemOf<FMT, NP, WR, WT>;
   Smem& S = *(Smem*)smem;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int nsb = p.cols / 256;
   const int l32 = lane & 31, lh = lane >> 5;
   const int wr0 = 32 * (wave % WR), wt0 = 32 * NP * (wave / WR);
   const __amdgpu_buffer_rsrc_t rw = ilt_rsrc(ilt_uniform_ptr(w), (u32)p.rows * (u32)(nsb * F::BLOCK));
-  const u32 row_bytes = (u32)(nsb * F::BLOCK), wbase = (u32)(r0 + wr0) * row_bytes;      // (past the matrix's rows: zeros)
-  const typename F::At at = F::place(row_bytes, lane);
+  // (past the matrix's rows: zeros.  What may lie past the end goes into the loads' vector offset, which the descriptor's bound
+  // is checked against whatever the scalar one is; the scalar offset is the block's within a row.)
+  const u32 row_bytes = (u32)(nsb * F::BLOCK);
+  const typename F::At at = F::place(row_bytes, lane, r0 + wr0, p.rows);
   const int wg = wave % WR, wq = wave / WR;          // the wave's group of rows, its place among those that share it
   auto issue_w = [&](int sb, int buf) {
-    u8* const dst = S.ws + ((WT == 1 ? 0 : buf) * WR + wg) * F::LBYTES;
+    u8* const dst = S.ws + ((WT == 1 && !DEEP ? 0 : buf) * WR + wg) * F::LBYTES;
+    u32 rb = row_bytes;
+    asm volatile("" : "+s"(rb));                     // (offsets made here each time: kept, they are registers the products want)
 #pragma unroll
     for (int i = 0; i < NW; i++)
-      if (F::LOADS % WT == 0 || wq * NW + i < F::LOADS) F::issue(wq * NW + i, rw, at, row_bytes, wbase + (u32)sb * F::BLOCK, dst);
+      if (F::LOADS % WT == 0 || wq * NW + i < F::LOADS) F::issue(wq * NW + i, rw, w, at, rb, (u32)(r0 + wr0), (u32)sb * F::BLOCK, dst);
   };
   const u8* xbase = (const u8*)ilt_uniform_ptr((const i8*)p.x + tok0 * (long)p.cols);
   // (past the tile's tokens: zeros)
   const __amdgpu_buffer_rsrc_t rx = ilt_rsrc(xbase, (u32)(__builtin_amdgcn_readfirstlane(ntok) * p.cols));
-  const u32 xlane = (u32)(lane >> 4) * (u32)p.cols, xpiece = 16 * (u32)((lane & 15) ^ (lane >> 4));
-  // half H of the tokens: the first or the second NP / 2 patches of every wave's
+  const u32 xlane = (u32)(lane >> 4) * (u32)p.cols + 16 * (u32)((lane & 15) ^ (lane >> 4));
+  // half H of the tokens: the first or the second NP / 2 patches of every wave's (NP 1: all of them, into buffer H)
   auto issue_x = [&](int sb, int h) {
+    u32 cols = (u32)p.cols;
+    asm volatile("" : "+s"(cols));
 #pragma unroll
     for (int i = 0; i < NI; i++) {
-      const int j = wave * NI + i, q = j / (4 * NP), k4 = 8 * NP * q + 4 * NP * h + j % (4 * NP);      // tokens 4 k4 .. + 3
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (ILT_LDS void*)(S.xs + k4 * 1088), 16, xlane + xpiece, k4 * 4 * p.cols + sb * 256, 0, 0);
+      const int j = wave * NI + i, q = j / (4 * NP), k4 = DEEP ? j : 8 * NP * q + 4 * NP * h + j % (4 * NP);      // tokens 4 k4 .. + 3
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (ILT_LDS void*)(S.xs[DEEP ? h : 0] + k4 * 1088), 16, xlane + (u32)(k4 * 4) * cols, sb * 256, 0, 0);
     }
   };
   // the tokens' scales and sums of 32 of a super-block, through registers
@@ -199,6 +334,7 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
   float c_yd; int4 c_bs[2];
   const u32 ctok = (u32)((t >> 1) * nsb);            // (past the tile's tokens: zeros)
   auto load_consts = [&](int sb) {
+    if (2 * TN < THREADS && t >= 2 * TN) return;
     c_yd = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, ctok * 4, sb * 4, 0));
     if constexpr (F::MINS) {
       const u32 o = ctok * 64 + 32 * (t & 1);
@@ -207,8 +343,14 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
     }
   };
   auto store_consts = [&](int buf) {
+    if (2 * TN < THREADS && t >= 2 * TN) return;
     if ((t & 1) == 0) S.xd[buf][t >> 1] = c_yd;
-    if constexpr (F::MINS) {
+    if constexpr (FMT == ILT_Q2_K) {
+      _Float16 hh[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) hh[k] = (_Float16)(float)(k < 4 ? (int)wordr(c_bs[0], k) : (int)wordr(c_bs[1], k - 4));
+      __builtin_memcpy(S.ms[buf] + 32 * (t >> 1) + 16 * (t & 1), hh, 16);
+    } else if constexpr (F::MINS) {
       const int s[4] = { c_bs[0].x + c_bs[0].y, c_bs[0].z + c_bs[0].w, c_bs[1].x + c_bs[1].y, c_bs[1].z + c_bs[1].w };
       _Float16 hh[4], ll[4];
 #pragma unroll
@@ -228,6 +370,7 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
   v4i hi[8], lo[8];
   typename F::Block blk;
   issue_w(0, 0);
+  if (DEEP) issue_w(min(1, nsb - 1), 1);
   issue_x(0, 0);
   load_consts(0);
   store_consts(0);
@@ -240,23 +383,26 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
 #pragma unroll
     for (int g = 0; g < 8; g++) { F::quants(qs, wsrc, g, l32, lh); F::quants_now(qs, wsrc, g, l32, lh); F::group(blk, qs, g, lh, hi[g], lo[g]); }
   }
+  if (DEEP && WT > 1) ilt_barrier_lds();             // (a shared first buffer is written again)
   // integer sums: of the patch being multiplied, and of the one before as they are, or put together where registers are short
-  constexpr bool TIGHT = NP == 4;
-  v16i X[TIGHT ? 1 : 2], Y[TIGHT ? 1 : 2], P;
+  constexpr bool TIGHT = (NP == 4 && F::PLANES == 2) || DEEP;
+  v16i X[TIGHT || F::PLANES < 2 ? 1 : 2], Y[TIGHT ? 1 : 2], P, D[2];      // (D: a group's sums, still without its scale)
 #pragma unroll
-  for (int r = 0; r < 16; r++) { if (TIGHT) P[r] = 0; else { X[1][r] = 0; Y[1][r] = 0; } }
+  for (int r = 0; r < 16; r++) { if (TIGHT) P[r] = 0; else { X[F::PLANES == 2][r] = 0; Y[1][r] = 0; } }
   v16f im = {};                                      // and of the minimums
   float dprev = 0.0f, dmprev = 0.0f;
   int c0 = 0, c1 = 1, c2 = 2;                        // where the tokens' constants of this block, the next and the one before are
   // Patch a of the block: its products, and beside them the terms of the patch before it and, with the last patch, the next
   // block's operands, each group's as soon as this block's have been multiplied.
-  auto patch = [&](auto ac, const u8* wnext) {
+  auto patch = [&](auto ac, const u8* wnext, const u8* xs) {
     constexpr int a = decltype(ac)::value, par = a & 1, pa = (a + NP - 1) % NP;
     constexpr bool last = a == NP - 1;
-    v16i &XC = X[TIGHT ? 0 : par], &YC = Y[TIGHT ? 0 : par], &XP = X[TIGHT ? 0 : par ^ 1], &YP = Y[TIGHT ? 0 : par ^ 1];
+    constexpr int XI = TIGHT || F::PLANES < 2 ? 0 : 1, YI = TIGHT ? 0 : 1;
+    v16i &XC = X[par * XI], &YC = Y[par * YI], &XP = X[(par ^ 1) * XI], &YP = Y[(par ^ 1) * YI];
+
     const float dp = a == 0 ? dprev : blk.d, dmp = a == 0 ? dmprev : blk.dm;
     const float* const xp = S.xd[a == 0 ? c2 : c0] + wt0 + 32 * pa + 4 * lh;
-    auto frag = [&](int g) { return __builtin_bit_cast(v4i, ilt_lds_ld16(S.xs + (g & 1 ? x1 : x0) + 8704 * a + 64 * (g >> 1))); };
+    auto frag = [&](int g) { return __builtin_bit_cast(v4i, ilt_lds_ld16((DEEP ? xs : S.xs[0]) + (g & 1 ? x1 : x0) + 8704 * a + 64 * (g >> 1))); };
     const v16i zi = {};
     typename F::Block nb = {};
     typename F::Quants qs;
@@ -275,13 +421,22 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
       if (g % 2 == 0 && g < 6) yn = lds_f4(xp + 4 * g + 8);
       if (F::MINS && g == 6) sums = __builtin_bit_cast(v8h, ilt_lds_ld16(S.ms[c0] + 32 * (wt0 + 32 * a + l32) + 16 * lh));
       __builtin_amdgcn_sched_barrier(0);
-      XC = __builtin_amdgcn_mfma_i32_32x32x32_i8(f, hi[g], g ? XC : zi, 0, 0, 0);
-      YC = __builtin_amdgcn_mfma_i32_32x32x32_i8(f, lo[g], g ? YC : zi, 0, 0, 0);
+      if constexpr (F::PLANES == 2) XC = __builtin_amdgcn_mfma_i32_32x32x32_i8(f, hi[g], g ? XC : zi, 0, 0, 0);
+      if constexpr (F::PLANES > 0) YC = __builtin_amdgcn_mfma_i32_32x32x32_i8(f, lo[g], g ? YC : zi, 0, 0, 0);
+      else {                                         // the group before's sums by its scale while this one's are made
+        D[g & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f, lo[g], zi, 0, 0, 0);
+        if (g > 0) {
+          const int sc = F::scale(blk, g - 1);
+#pragma unroll
+          for (int r = 0; r < 16; r++) YC[r] = g > 1 ? ilt_mad24(D[(g & 1) ^ 1][r], sc, YC[r]) : ilt_mul24(D[(g & 1) ^ 1][r], sc);
+          asm volatile("" : "+v"(YC));
+        }
+      }
       // two results' terms, step by step side by side (one after the other every instruction waits for the one before it)
       {
         const int r = 2 * g;
         const float y0 = r & 2 ? yp.z : yp.x, y1 = r & 2 ? yp.w : yp.y;
-        const int i0 = TIGHT ? P[r] : (XP[r] << F::SH) + YP[r], i1 = TIGHT ? P[r + 1] : (XP[r + 1] << F::SH) + YP[r + 1];
+        const int i0 = TIGHT ? P[r] : F::PLANES == 2 ? (XP[r] << F::SH) + YP[r] : YP[r], i1 = TIGHT ? P[r + 1] : F::PLANES == 2 ? (XP[r + 1] << F::SH) + YP[r + 1] : YP[r + 1];
         float b0 = y0 * dp, b1 = y1 * dp, f0_ = (float)i0, f1_ = (float)i1, s0 = sum[pa][0][r], s1 = sum[pa][0][r + 1];
         if constexpr (F::MINS) {
           float a0 = y0 * dmp, a1 = y1 * dmp;
@@ -292,6 +447,7 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
           asm volatile("" : "+v"(s0), "+v"(s1));
         } else {
           asm volatile("" : "+v"(b0), "+v"(b1), "+v"(f0_), "+v"(f1_));
+          if constexpr (F::PLANES == 0) { f0_ = f0_ * 0.5f; f1_ = f1_ * 0.5f; }
           b0 = b0 * f0_; b1 = b1 * f1_;
           asm volatile("" : "+v"(b0), "+v"(b1));
         }
@@ -302,9 +458,16 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
       asm volatile("" : "+v"(sum[pa][0]));
       if constexpr (last) {
         F::group(nb, qs, g, lh, hi[g], lo[g]);
-        asm volatile("" : "+v"(hi[g]), "+v"(lo[g]));
+        if constexpr (F::PLANES == 2) asm volatile("" : "+v"(hi[g]), "+v"(lo[g]));
+        else asm volatile("" : "+v"(lo[g]));
       }
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (F::PLANES == 0) {
+      const int sc = F::scale(blk, 7);
+#pragma unroll
+      for (int r = 0; r < 16; r++) YC[r] = ilt_mad24(D[1][r], sc, YC[r]);
+      asm volatile("" : "+v"(YC));
     }
     if constexpr (F::MINS) {
       const v16f zf = {};
@@ -312,7 +475,7 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
     }
     if constexpr (TIGHT) {
 #pragma unroll
-      for (int r = 0; r < 16; r++) P[r] = (XC[r] << F::SH) + YC[r];
+      for (int r = 0; r < 16; r++) P[r] = F::PLANES == 2 ? (XC[r] << F::SH) + YC[r] : YC[r];
       asm volatile("" : "+v"(P));
     }
     if constexpr (last) { dprev = blk.d; dmprev = blk.dm; blk = nb; }
@@ -322,27 +485,35 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
     const int nx = min(sb + 1, nsb - 1), nbuf = (sb + 1) & 1;       // (the last block's again, for nobody)
     using std::integral_constant;
     __builtin_amdgcn_sched_barrier(0);
-    issue_x(sb, 1);                                  // (the block before's second half has been multiplied)
-    issue_w(nx, nbuf);                               // (and this block's operands are made)
+    if constexpr (DEEP) {
+      issue_x(nx, nbuf);
+      issue_w(min(sb + 2, nsb - 1), sb & 1);         // (this block's operands are made)
+    } else {
+      issue_x(sb, 1);                                // (the block before's second half has been multiplied)
+      issue_w(nx, nbuf);                             // (and this block's operands are made)
+    }
     load_consts(nx);
     __builtin_amdgcn_sched_barrier(0);
-    const u8* const wnext = wsrc + (WT == 1 ? 0 : nbuf) * WR * F::LBYTES;
-    patch(integral_constant<int, 0>{}, wnext);
-    if constexpr (NP == 4) patch(integral_constant<int, 1>{}, wnext);
+    const u8* const wnext = wsrc + (WT == 1 && !DEEP ? 0 : nbuf) * WR * F::LBYTES;
+    const u8* const xs = S.xs[DEEP ? sb & 1 : 0];
+    patch(integral_constant<int, 0>{}, wnext, xs);
+    if constexpr (NP == 4) patch(integral_constant<int, 1>{}, wnext, xs);
     store_consts(c1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     ilt_barrier_lds();
-    __builtin_amdgcn_sched_barrier(0);
-    issue_x(nx, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (NP == 4) {
-      patch(integral_constant<int, 2>{}, wnext);
-      patch(integral_constant<int, 3>{}, wnext);
-    } else {
-      patch(integral_constant<int, 1>{}, wnext);
+    if constexpr (!DEEP) {
+      __builtin_amdgcn_sched_barrier(0);
+      issue_x(nx, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (NP == 4) {
+        patch(integral_constant<int, 2>{}, wnext, xs);
+        patch(integral_constant<int, 3>{}, wnext, xs);
+      } else {
+        patch(integral_constant<int, 1>{}, wnext, xs);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      ilt_barrier_lds();
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    ilt_barrier_lds();
     const int c = c2; c2 = c0; c0 = c1; c1 = c;
   }
   {
@@ -350,8 +521,15 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       if constexpr (F::MINS) sum[NP - 1][0][r] = sum[NP - 1][0][r] - (xp[8 * (r >> 2) + (r & 3)] * dmprev) * im[r];
-      sum[NP - 1][0][r] = sum[NP - 1][0][r] + (xp[8 * (r >> 2) + (r & 3)] * dprev) * (float)(TIGHT ? P[r] : (X[TIGHT ? 0 : 1][r] << F::SH) + Y[TIGHT ? 0 : 1][r]);
+      const int is = TIGHT ? P[r] : F::PLANES == 2 ? (X[F::PLANES == 2 && !TIGHT][r] << F::SH) + Y[!TIGHT][r] : Y[!TIGHT][r];
+      sum[NP - 1][0][r] = sum[NP - 1][0][r] + (xp[8 * (r >> 2) + (r & 3)] * dprev) * (F::PLANES == 0 ? (float)is * 0.5f : (float)is);
     }
+  }
+  if constexpr (F::PLANES == 0) {
+#pragma unroll
+    for (int a = 0; a < NP; a++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) sum[a][0][r] = 0.25f * sum[a][0][r];
   }
   store_tile<NP, 1>(sum, p, tok0, ntok, r0, wt0, wr0, l32, lh);
 }
@@ -375,14 +553,14 @@ __global__ __launch_bounds__(64 * WR * WT, 2) void gemm_i8r_kernel(BfParams p) {
   p.bias = m == 0 ? p.mbias[0] : m == 1 ? p.mbias[1] : p.mbias[2];
   if (p.nmulti > 1) p.ldy = p.rows;
   const int fmt = m == 0 ? p.mfmt[0] : m == 1 ? p.mfmt[1] : p.mfmt[2];
+  if constexpr (FSET == ILT_IQ2_XXS) { iq2_tables_load(threadIdx.x, 64 * WR * WT); __syncthreads(); }
   if constexpr (FSET != 0) reg_tile<FSET, NP, WR, WT>(p, w, rt * TM, tok0, ntok, smem);
   else if (fmt == ILT_Q4_K) reg_tile<ILT_Q4_K, NP, WR, WT>(p, w, rt * TM, tok0, ntok, smem);
   else reg_tile<ILT_Q6_K, NP, WR, WT>(p, w, rt * TM, tok0, ntok, smem);
 }
 
 template <int FMT, int NP, int WR, int WT> constexpr size_t reg_smem() {
-  constexpr int TN = 32 * NP * WT;
-  if constexpr (FMT != 0) return sizeof(RegSmem<TN, raw_bytes<FMT, WR, WT>(), RegW<FMT>::MINS>);
+  if constexpr (FMT != 0) return sizeof(RegSmemOf<FMT, NP, WR, WT>);
   else return reg_smem<ILT_Q4_K, NP, WR, WT>() > reg_smem<ILT_Q6_K, NP, WR, WT>() ? reg_smem<ILT_Q4_K, NP, WR, WT>() : reg_smem<ILT_Q6_K, NP, WR, WT>();
 }
 
@@ -408,29 +586,75 @@ hipError_t launch_i8r(BfParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
+struct GroupScan { u32 scan[256]; int tile_z, tile_t0, tile_n; };
+
+// The experts' products: token tiles of every expert's rows in turn, 128 rows of the expert's matrix (of two, one behind the
+// other in the output: gate and up) a workgroup.  A group of up to 32 (64) rows goes as one (two) patches of 32.
+template <int FMT>
+__global__ __launch_bounds__(256, 2) void gemm_i8r_group_kernel(BfParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ GroupScan scan;
+  if constexpr (FMT == ILT_IQ2_XXS) iq2_tables_load(threadIdx.x, 256);
+  long tok0; int ntok, rt; const u8* w;
+  const int rows = p.rows, nr = (rows + 127) / 128;
+  if (p.nmulti > 1) p.rows = 2 * nr * 128;
+  if (!pick_tile<128, 128>(p, scan, tok0, ntok, rt, w)) return;       // (barriers inside)
+  p.rows = rows;
+  if (rt >= nr) { rt -= nr; w += p.up_delta; p.y = p.my[1]; }
+  ntok = __builtin_amdgcn_readfirstlane(ntok);
+  if (ntok <= 32) reg_tile<FMT, 1, 4, 1>(p, w, rt * 128, tok0, ntok, smem);
+  else if (ntok <= 64) reg_tile<FMT, 2, 4, 1>(p, w, rt * 128, tok0, ntok, smem);
+  else reg_tile<FMT, 4, 4, 1>(p, w, rt * 128, tok0, ntok, smem);
+}
+
+template <int FMT>
+hipError_t launch_i8r_group(const BfParams& p, long long total_rows, hipStream_t st) {
+  constexpr size_t a = reg_smem<FMT, 1, 4, 1>(), b = reg_smem<FMT, 2, 4, 1>(), c = reg_smem<FMT, 4, 4, 1>();
+  constexpr size_t smem = a > b ? (a > c ? a : c) : (b > c ? b : c);
+  static_assert(2 * (smem + 5120) <= 160 * 1024, "two workgroups a CU");
+  static bool attr_set[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  if (!attr_set[dev]) {
+    const hipError_t e = hipFuncSetAttribute((const void*)gemm_i8r_group_kernel<FMT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return e;
+    attr_set[dev] = true;
+  }
+  // sum over experts of ceil(count / 128) <= total / 128 + ne
+  const long long total = (total_rows / 128 + p.ne) * ((p.rows + 127) / 128) * p.nmulti, per = (total + 7) / 8;
+  if (per * 8 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(gemm_i8r_group_kernel<FMT>, dim3((unsigned)(per * 8)), dim3(256), smem, st, p);
+  return hipGetLastError();
+}
+
 template <int FSET>
 hipError_t dispatch_i8r(BfParams& p, bool big, hipStream_t st) {
   return big ? launch_i8r<FSET, 4, 4, 1>(p, st) : launch_i8r<FSET, 2, 2, 2>(p, st);
 }
 
+constexpr int block_bytes_of(int fmt) {
+  return fmt == ILT_Q4_K ? RegW<ILT_Q4_K>::BLOCK : fmt == ILT_Q6_K ? RegW<ILT_Q6_K>::BLOCK : fmt == ILT_Q2_K ? RegW<ILT_Q2_K>::BLOCK : RegW<ILT_IQ2_XXS>::BLOCK;
+}
+
 }  // namespace
 
-// Up to three matrices (Q4_K, Q6_K in any mix) on the same tokens in one launch, their row tiles one after another.
+// Up to three matrices (Q4_K, Q6_K in any mix, or all Q2_K, or all IQ2_XXS) on the same tokens in one launch, their row tiles one after another.
 // hipErrorNotSupported, and nothing launched, where the shapes are not this kernel's.  128 rows x 128 tokens a workgroup from
 // 150 such tiles on; fewer leave CUs idle, and 64 x 128 (each weight unpacked twice, for 64 tokens at a time) fills twice
 // as many: Q6_K 2560 x 9728 on 512 tokens, 80 tiles: 79 against 104 us; on 1,024, 160: 124 against 112; Q4_K 2560 x 4096 the
 // same 39 against 49, 54 against 53; 19456 x 2560 on 128, 152: 36.4 against 35.5.  ILT_I8_TM (tests): 64 or 128 rows whatever the shape.
 hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws, const int* rows, float* const* ys, const float* const* biases,
                              int cols, const int8_t* xq, const float* xd, const int* bsums, int ntok, int acc, hipStream_t st, long long ldy) {
-  if (nmat < 1 || nmat > 3 || ntok < 1 || cols < 256 || cols % 256 != 0 || (long long)cols * 128 >= 0x7FFFFFFFLL) return hipErrorNotSupported;
+  if (nmat < 1 || nmat > 3 || ntok < 1 || cols < 256 || cols % 256 != 0 || cols >= (1 << 22)) return hipErrorNotSupported;
   BfParams p = {};
   long long tiles128 = 0;
   int fset = fmts[0];
   for (int m = 0; m < nmat; m++) {
-    if (fmts[m] != ILT_Q4_K && fmts[m] != ILT_Q6_K) return hipErrorNotSupported;
-    if (fmts[m] != fset) fset = 0;
-    const long long bytes = (long long)rows[m] * (cols / 256) * (fmts[m] == ILT_Q4_K ? 144 : ILT_Q6K_STRIDE);
-    if (rows[m] < 1 || bytes >= 0x7FFFFFFFLL || (((uintptr_t)ws[m]) & 3) || rows[m] >= (1 << 21)) return hipErrorNotSupported;      // 32-bit offsets
+    const bool two = fmts[m] == ILT_Q2_K || fmts[m] == ILT_IQ2_XXS;
+    if (fmts[m] != ILT_Q4_K && fmts[m] != ILT_Q6_K && !two) return hipErrorNotSupported;
+    if (fmts[m] != fset) { if (two || fset == ILT_Q2_K || fset == ILT_IQ2_XXS) return hipErrorNotSupported; fset = 0; }
+    const long long bytes = (long long)rows[m] * (cols / 256) * block_bytes_of(fmts[m]);
+    if (rows[m] < 1 || bytes >= 0x7FFFFFFFLL || (((uintptr_t)ws[m]) & (fmts[m] == ILT_IQ2_XXS ? 1 : 3)) || rows[m] >= (1 << 21)) return hipErrorNotSupported;      // 32-bit offsets
     p.mw[m] = ws[m]; p.mrows[m] = rows[m]; p.my[m] = ys[m]; p.mbias[m] = biases ? biases[m] : nullptr; p.mfmt[m] = fmts[m];
     tiles128 += (rows[m] + 127) / 128;
   }
@@ -443,6 +667,24 @@ hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws
   switch (fset) {
     case ILT_Q4_K: return dispatch_i8r<ILT_Q4_K>(p, big, st);
     case ILT_Q6_K: return dispatch_i8r<ILT_Q6_K>(p, big, st);
+    case ILT_Q2_K: return dispatch_i8r<ILT_Q2_K>(p, big, st);
+    case ILT_IQ2_XXS: return dispatch_i8r<ILT_IQ2_XXS>(p, big, st);
     default: return dispatch_i8r<0>(p, big, st);
   }
+}
+
+// The grouped product of the experts' IQ2_XXS and Q2_K matrices: expert z's rows counts[z] from bases[z] on; y2 set: a second
+// matrix at add2 as well, its results there.  hipErrorNotSupported, and nothing launched, where the shapes are not this kernel's.
+hipError_t ilt_k_gemm_i8_reg_id(int fmt, const uint64_t* ptrs, long long add, long long add2, const uint32_t* counts, const uint32_t* bases, int ne,
+                                int rows, int cols, const int8_t* xq, const float* xd, const int* bsums, long long total_rows, float* y, float* y2,
+                                hipStream_t st) {
+  const long long row_bytes = (long long)(cols / 256) * block_bytes_of(fmt), delta = y2 ? add2 - add : 0;
+  if ((fmt != ILT_IQ2_XXS && fmt != ILT_Q2_K) || ne < 1 || ne > 256 || rows < 1 || rows >= (1 << 21) || cols < 256 || cols % 256 || rows * row_bytes >= 0x7FFFFFFFLL ||
+      cols >= (1 << 22) || total_rows < 1 || total_rows >= 0x7FFFFFFFLL || delta < 0 || delta > 0x7FFFFFFFLL || (fmt == ILT_Q2_K && (add & 3)))
+    return hipErrorNotSupported;
+  BfParams p = {};
+  p.ptrs = ptrs; p.add = add; p.up_delta = (unsigned)delta; p.counts = counts; p.bases = bases; p.ne = ne;
+  p.rows = rows; p.cols = cols; p.row_bytes = row_bytes; p.x = (const u16*)xq; p.xd = xd; p.bsums = bsums;
+  p.y = y; p.my[1] = y2; p.nmulti = y2 ? 2 : 1; p.ntok = (int)total_rows; p.ldy = rows;
+  return fmt == ILT_IQ2_XXS ? launch_i8r_group<ILT_IQ2_XXS>(p, total_rows, st) : launch_i8r_group<ILT_Q2_K>(p, total_rows, st);
 }

@@ -57,3 +57,48 @@ def test_operands_in_registers_bit_for_bit(dev, monkeypatch, rows_a_tile, qtype,
         hip.hip_free(b)
     act.free()
     m.free()
+
+
+@pytest.mark.parametrize("rows_a_tile", ["64", "128"])
+@pytest.mark.parametrize("qtype,rows,cols,n", [(synth.Q2_K, 129, 768, 33), (synth.Q2_K, 64, 256, 130), (synth.IQ2_XXS, 129, 256, 65), (synth.IQ2_XXS, 100, 1280, 128)])
+def test_expert_formats_on_a_dense_matrix_bit_for_bit(dev, monkeypatch, rows_a_tile, qtype, rows, cols, n):
+    from illatio_amd import ds4f, hip
+    monkeypatch.setenv("ILT_I8_TM", rows_a_tile)
+    rng = synth.make_rng(rows + cols + n)
+    w, x = synth.weights(qtype, rows, cols, rng), synth.activations((n, cols), rng)
+    x[n // 2] = 1.0
+    wb, xb, y = hip.hip_upload_new(dev, w), hip.hip_upload_new(dev, x), hip.hip_alloc(dev, 4 * n * rows)
+    ds4f.dk_mm(dev, "d4_mm_q2_k" if qtype == synth.Q2_K else "d4_mm_iq2_xxs", wb, None, synth.row_bytes(qtype, cols), rows, cols, xb, y, n)
+    want = orc.matmul(qtype, w, rows, cols, x, nthreads=8).reshape(n, rows)
+    got = hip.hip_floats(y, n * rows).reshape(n, rows)
+    assert np.array_equal(bits(got), bits(want)), np.argwhere(bits(got) != bits(want))[:5]
+    for b in (wb, xb, y):
+        hip.hip_free(b)
+
+
+# groups around patches of 32 and tiles of 128, one without rows
+@pytest.mark.parametrize("qtype,rows,cols", [(synth.Q2_K, 128, 256), (synth.Q2_K, 161, 1280), (synth.IQ2_XXS, 128, 256), (synth.IQ2_XXS, 200, 768)])
+def test_groups_bit_for_bit(dev, qtype, rows, cols):
+    from illatio_amd import ds4f, hip
+    rng = synth.make_rng(rows + cols)
+    counts = np.array([1, 32, 0, 33, 64, 65, 128, 129, 260], np.uint32)
+    ne, total = len(counts), int(counts.sum())
+    bases = (np.cumsum(counts) - counts).astype(np.uint32)
+    rb = synth.row_bytes(qtype, cols)
+    w = synth.weights(qtype, ne * rows, cols, rng).reshape(ne, rows, rb)
+    x = synth.activations((total, cols), rng)
+    wb, xb, y = hip.hip_upload_new(dev, w), hip.hip_upload_new(dev, x), hip.hip_alloc(dev, 4 * total * rows)
+    ptrs = hip.hip_upload_new(dev, np.array([wb.ptr + z * rows * rb for z in range(ne)], np.uint64))
+    cb, bb = hip.hip_upload_new(dev, counts), hip.hip_upload_new(dev, bases)
+    xq, xd, xs = ds4f._q8k(dev, xb, total * cols)
+    hip.launch(dev, "d4_mm_id_q2_k" if qtype == synth.Q2_K else "d4_mm_id_iq2_xxs", (1, 1, ne), 128,
+               [cols, rows, rb, cols, rows, hip.I64(0), ptrs, cb, bb, xq, y, xd, xs, hip.I64(total)])
+    got = hip.hip_floats(y, total * rows).reshape(total, rows)
+    for z in range(ne):
+        if counts[z] == 0:
+            continue
+        at = slice(int(bases[z]), int(bases[z] + counts[z]))
+        want = orc.matmul(qtype, w[z], rows, cols, x[at], nthreads=8).reshape(-1, rows)
+        assert np.array_equal(bits(got[at]), bits(want)), (z, np.argwhere(bits(got[at]) != bits(want))[:5])
+    for b in (wb, xb, y, ptrs, cb, bb, xq, xd, xs):
+        hip.hip_free(b)
