@@ -793,6 +793,33 @@ int ilt_d4_mm_id_iq2_xxs(uint64_t stream, int ncols, int nrows, int row_bytes, i
   return mm_id(stream, ILT_IQ2_XXS, ncols, nrows, row_bytes, add, ptrs, counts, bases, ne, total_rows, xq, xd, nullptr, y);
 }
 
+// gate and up of every expert in one launch where the kernel takes it
+int ilt_d4_mm_id2_iq2_xxs(uint64_t stream, int ncols, int nrows, int row_bytes, int64_t add_gate, int64_t add_up, const uint64_t* ptrs,
+                          const uint32_t* counts, const uint32_t* bases, int ne, int64_t total_rows, const int8_t* xq, const float* xd,
+                          float* gate, float* up) {
+  ILT_REQUIRE(ncols > 0 && ncols % 256 == 0 && nrows >= 0 && ne >= 0 && ne <= 256 && total_rows >= 0 && row_bytes == ncols / 256 * block_bytes(ILT_IQ2_XXS) &&
+              add_gate >= 0 && add_up >= 0 && ((add_gate | add_up) & 1) == 0);
+  if (nrows == 0 || ne == 0 || total_rows == 0) return ILT_OK;
+  ILT_REQUIRE(ptrs && counts && bases && xq && xd && gate && up && ((uintptr_t)xq & 15) == 0);
+  const char* force = getenv("ILT_I8_PLANES");
+  hipError_t e = hipErrorNotSupported;
+  if (!(force && force[0] == '0'))
+    e = ilt_k_gemm_i8_reg_id(ILT_IQ2_XXS, ptrs, add_gate, add_up, counts, bases, ne, nrows, ncols, xq, xd, nullptr, total_rows, gate, up, S(stream));
+  if (e != hipErrorNotSupported) return (int)e;
+  const int r = ilt_d4_mm_id_iq2_xxs(stream, ncols, nrows, row_bytes, add_gate, ptrs, counts, bases, ne, total_rows, xq, xd, gate);
+  return r ? r : ilt_d4_mm_id_iq2_xxs(stream, ncols, nrows, row_bytes, add_up, ptrs, counts, bases, ne, total_rows, xq, xd, up);
+}
+
+int ilt_d4_gather_q8k(uint64_t stream, int d, int nrows, const int8_t* xq, const float* xd, const uint32_t* map, int8_t* oq, float* od) {
+  ILT_REQUIRE(d > 0 && d % 256 == 0 && nrows >= 0 && (nrows == 0 || (xq && xd && map && oq && od)) && (((uintptr_t)xq | (uintptr_t)oq) & 15) == 0);
+  return (int)ilt_k_gather_q8k(d, nrows, xq, xd, map, oq, od, S(stream));
+}
+
+int ilt_d4_swiglu_w_q8k(uint64_t stream, int n, int ff, float clamp, const float* g, const float* u, const float* w, int8_t* xq, float* xd, int32_t* bsums) {
+  ILT_REQUIRE(n >= 0 && ff > 0 && ff % 256 == 0 && (n == 0 || (g && u && w && xq && xd && bsums)) && (((uintptr_t)g | (uintptr_t)u) & 15) == 0);
+  return (int)ilt_k_swiglu_w_quant_q8k(n, ff, clamp, g, u, w, xq, xd, bsums, S(stream));
+}
+
 int ilt_d4_mm_id_q2_k(uint64_t stream, int ncols, int nrows, int row_bytes, int64_t add, const uint64_t* ptrs,
                       const uint32_t* counts, const uint32_t* bases, int ne, int64_t total_rows,
                       const int8_t* xq, const float* xd, const int32_t* bsums, float* y) {
@@ -1398,6 +1425,12 @@ int ilt_launch(const char* kernel, unsigned gx, unsigned gy, unsigned gz, unsign
   K("d4_mm_id_iq2_xxs")
     return ilt_d4_mm_id_iq2_xxs(stream, a.i32(0), a.i32(1), a.i32(2), a.i64(5), a.ptr<const uint64_t*>(6), a.ptr<cu32>(7),
                                 a.ptr<cu32>(8), (int)gz, a.i64(13), a.ptr<ci8>(9), a.ptr<cf>(11), a.ptr<float*>(10));
+  K("d4_mm_id2_iq2_xxs")
+    return ilt_d4_mm_id2_iq2_xxs(stream, a.i32(0), a.i32(1), a.i32(2), a.i64(3), a.i64(4), a.ptr<const uint64_t*>(5), a.ptr<cu32>(6), a.ptr<cu32>(7),
+                                 a.i32(8), a.i64(9), a.ptr<ci8>(10), a.ptr<cf>(11), a.ptr<float*>(12), a.ptr<float*>(13));
+  K("d4_gather_q8k") return ilt_d4_gather_q8k(stream, a.i32(0), a.i32(1), a.ptr<ci8>(2), a.ptr<cf>(3), a.ptr<cu32>(4), a.ptr<int8_t*>(5), a.ptr<float*>(6));
+  K("d4_swiglu_w_q8k") return ilt_d4_swiglu_w_q8k(stream, a.i32(0), a.i32(1), a.f32(2), a.ptr<cf>(3), a.ptr<cf>(4), a.ptr<cf>(5), a.ptr<int8_t*>(6),
+                                                  a.ptr<float*>(7), a.ptr<int32_t*>(8));
   K("d4_mm_id_q2_k")
     return ilt_d4_mm_id_q2_k(stream, a.i32(0), a.i32(1), a.i32(2), a.i64(5), a.ptr<const uint64_t*>(6), a.ptr<cu32>(7),
                              a.ptr<cu32>(8), (int)gz, a.i64(13), a.ptr<ci8>(9), a.ptr<cf>(11), a.ptr<const int32_t*>(12),

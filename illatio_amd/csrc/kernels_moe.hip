@@ -111,6 +111,18 @@ __global__ void gather_rows_kernel(int d, int nrows, const float* __restrict__ s
   *(float4*)(x + gid) = *(const float4*)(src + (long long)map[r] * d + j);
 }
 
+// The rows of a chunk gathered as the blocks they are quantized to (a token is quantized once, not once a row of its): 16 bytes
+// a thread, the scales by the row's first threads.
+__global__ __launch_bounds__(256) void gather_q8k_kernel(int d, long long pieces, const i8* __restrict__ xq, const float* __restrict__ xd,
+                                                         const u32* __restrict__ map, i8* __restrict__ oq, float* __restrict__ od) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= pieces) return;
+  const int per = d / 16, r = (int)(i / per), c = (int)(i - (long long)r * per);
+  const long long t = map[r];
+  *(int4*)(oq + i * 16) = *(const int4*)(xq + t * d + 16 * c);
+  if (c < d / 256) od[(long long)r * (d / 256) + c] = xd[t * (d / 256) + c];
+}
+
 // mid[r][j] = (silu(g) * u) * w[r] (no w: weights of one), g and u clamped first when clamp > 1e-6
 // (d4-routed!, ds4f.lisp:1016-1019); quantized to Q8_0 with a float scale as well when xq
 // is given (the shared expert's down projection takes Q8_0 activations).
@@ -263,6 +275,13 @@ hipError_t ilt_k_gather_rows(int d, int nrows, const float* src, const uint32_t*
   if (d % 4) return hipErrorInvalidValue;
   const long long n4 = (long long)nrows * d / 4;
   hipLaunchKernelGGL(gather_rows_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, d, nrows, src, map, x);
+  return hipGetLastError();
+}
+
+hipError_t ilt_k_gather_q8k(int d, int nrows, const int8_t* xq, const float* xd, const uint32_t* map, int8_t* oq, float* od, hipStream_t st) {
+  const long long pieces = (long long)nrows * (d / 16);
+  if (pieces <= 0) return hipSuccess;
+  hipLaunchKernelGGL(gather_q8k_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st, d, pieces, xq, xd, map, oq, od);
   return hipGetLastError();
 }
 

@@ -41,11 +41,11 @@ __global__ __launch_bounds__(256) void quant_q8_kernel(const float* __restrict__
 // d = 1/iscale; sums of each 16 quants.
 // GLU: the values quantized are swiglu!'s (model.lisp:364-378) of x and up, (x / (1 + e^-x)) * up with the exponential
 // through double -- a prompt chunk's gated activations go straight into the blocks the down product reads, and the
-// floats are neither written nor read again.
-template <bool GLU>
+// floats are neither written nor read again.  GLU 2: d4-routed!'s (ds4f.lisp:1016-1019), clamped, times the row's weight.
+template <int GLU>
 __global__ __launch_bounds__(256) void quant_q8k_kernel(const float* __restrict__ x, const float* __restrict__ up, i8* __restrict__ xq,
                                                         float* __restrict__ xd, int* __restrict__ bsums, long long nblocks,
-                                                        long long bpr, long long x_stride) {
+                                                        long long bpr, long long x_stride, float clamp, const float* __restrict__ wrow) {
   const int lane = threadIdx.x & 63;
   const long long b = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (b >= nblocks) return;
@@ -56,7 +56,12 @@ __global__ __launch_bounds__(256) void quant_q8k_kernel(const float* __restrict_
     const float4 u4 = ((const float4*)(up + b * 256))[lane];
     const float u[4] = {u4.x, u4.y, u4.z, u4.w};
 #pragma unroll
-    for (int k = 0; k < 4; k++) v[k] = (v[k] / (1.0f + ilt_expf_via_double(-v[k]))) * u[k];
+    for (int k = 0; k < 4; k++) {
+      if (GLU == 1) { v[k] = (v[k] / (1.0f + ilt_expf_via_double(-v[k]))) * u[k]; continue; }
+      float g = v[k], uu = u[k];
+      if (clamp > 1e-6f) { g = fminf(g, clamp); uu = fmaxf(-clamp, fminf(uu, clamp)); }
+      v[k] = (ilt_silu(g) * uu) * wrow[b / bpr];
+    }
   }
   // |v|'s bits order as |v| does; the low word prefers the earlier index
   u64 key = 0;
@@ -264,13 +269,22 @@ hipError_t ilt_k_quant_q8(const float* x, int8_t* xq, float* xs, int* xsum, long
 
 hipError_t ilt_k_quant_q8k(const float* x, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st) {
   if (nblocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(quant_q8k_kernel<false>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, x, (const float*)nullptr, xq, xd, bsums, nblocks, 0LL, 0LL);
+  hipLaunchKernelGGL(quant_q8k_kernel<0>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, x, (const float*)nullptr, xq, xd, bsums, nblocks, 0LL, 0LL, 0.0f, (const float*)nullptr);
   return hipGetLastError();
 }
 
 hipError_t ilt_k_swiglu_quant_q8k(const float* gate, const float* up, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st) {
   if (nblocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(quant_q8k_kernel<true>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, gate, up, xq, xd, bsums, nblocks, 0LL, 0LL);
+  hipLaunchKernelGGL(quant_q8k_kernel<1>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, gate, up, xq, xd, bsums, nblocks, 0LL, 0LL, 0.0f, (const float*)nullptr);
+  return hipGetLastError();
+}
+
+hipError_t ilt_k_swiglu_w_quant_q8k(int nrows, int ff, float clamp, const float* gate, const float* up, const float* wrow, int8_t* xq, float* xd, int* bsums,
+                                    hipStream_t st) {
+  const long long nblocks = (long long)nrows * (ff / 256);
+  if (nblocks <= 0) return hipSuccess;
+  hipLaunchKernelGGL(quant_q8k_kernel<2>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, gate, up, xq, xd, bsums, nblocks, (long long)(ff / 256),
+                     (long long)ff, clamp, wrow);
   return hipGetLastError();
 }
 
@@ -280,7 +294,7 @@ hipError_t ilt_k_quant_rows(int k, const float* x, int8_t* xq, float* xs, int* b
   if (ntok <= 0) return hipSuccess;
   if (cols <= 0 || cols % bw != 0 || x_stride < cols || (k && x_stride % 4 != 0)) return hipErrorInvalidValue;
   const long long bpr = cols / bw, nblocks = ntok * bpr;
-  if (k) hipLaunchKernelGGL(quant_q8k_kernel<false>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, x, (const float*)nullptr, xq, xs, bsums, nblocks, bpr, x_stride);
+  if (k) hipLaunchKernelGGL(quant_q8k_kernel<0>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, x, (const float*)nullptr, xq, xs, bsums, nblocks, bpr, x_stride, 0.0f, (const float*)nullptr);
   else hipLaunchKernelGGL(quant_q8_kernel, dim3((unsigned)((nblocks * 32 + 255) / 256)), dim3(256), 0, st, x, xq, xs, (int*)nullptr, nblocks,
                           f16_scale, bpr, x_stride);
   return hipGetLastError();

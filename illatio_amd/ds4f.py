@@ -453,9 +453,9 @@ def ffn_routed_chunk_bf16(dev, pool, logits, norm2, sout, n, ne, nu, scale, clam
 
 def ffn_routed_chunk(dev, pool, logits, norm2, sout, n, ne, nu, scale, clamp, bias=None, keep=None, ws=None):
     """A chunk of N tokens past the router (DK-FFN-ROUTED-CHUNK): each token's experts and
-    weights (d4_route), the (token, slot) rows grouped by expert, the rows gathered and
-    quantized, every expert's gate, up and down as one grouped product each over its rows
-    (d4_mm_id_*), the gated activation between, then each token's rows summed in slot order
+    weights (d4_route), the (token, slot) rows grouped by expert, the tokens quantized and their
+    blocks gathered, every expert's gate and up, and its down, as one grouped product over its rows
+    (d4_mm_id_*), the gated activation quantized between, then each token's rows summed in slot order
     with the shared expert's SOUT.  LOGITS (N x NE), NORM2 (N x D) and SOUT (N x D) are
     DBufs; returns MOE (N x D).  With a Workspace WS nothing is allocated, freed or waited for."""
     d, ff = pool.d, pool.ff
@@ -465,22 +465,18 @@ def ffn_routed_chunk(dev, pool, logits, norm2, sout, n, ne, nu, scale, clamp, bi
     sel, w = route(dev, logits, n, ne, nu, scale, bias, A)
     g = group_rows(dev, sel, w, n, ne, nu, A)
     ptrs = pool.ptrs
-    x = A(dev, 4 * rows * d)
-    hip.launch(dev, "d4_gather_rows", (rows * d + 255) // 256, 256, [d, rows, norm2, g["rmap"], x])
-    xq, xd, xs = _q8k(dev, x, rows * d, A)
-    gg, gu, mid = (A(dev, 4 * rows * ff) for _ in range(3))
+    # a token is quantized once and its blocks gathered into each of its rows
+    tq, td, ts = _q8k(dev, norm2, n * d, A)
+    xq, xd = A(dev, rows * d), A(dev, 4 * rows * d // 256)
+    hip.launch(dev, "d4_gather_q8k", (rows * d + 4095) // 4096, 256, [d, rows, tq, td, g["rmap"], xq, xd])
+    gg, gu = (A(dev, 4 * rows * ff) for _ in range(2))
     down, moe = A(dev, 4 * rows * d), A(dev, 4 * n * d)
-
-    def mm_id(kernel, ncols, nrows, rb, add, xin, yout):
-        hip.launch(dev, kernel, ((n + 63) // 64, (nrows + 63) // 64, ne), 128,
-                   [ncols, nrows, rb, ncols, nrows, hip.I64(add), ptrs, g["counts"], g["bases"], xin[0], yout,
-                    xin[1], xin[2], hip.I64(rows)])
-
-    mm_id("d4_mm_id_iq2_xxs", d, ff, pool.grb, 0, (xq, xd, None), gg)
-    mm_id("d4_mm_id_iq2_xxs", d, ff, pool.grb, gb, (xq, xd, None), gu)
-    hip.launch(dev, "d4_swiglu_w", (rows * ff + 255) // 256, 256, [rows, ff, float(clamp), gg, gu, g["wrow"], mid, None, None])
-    mq, md, ms = _q8k(dev, mid, rows * ff, A)
-    mm_id("d4_mm_id_q2_k", ff, d, pool.drb, 2 * gb, (mq, md, ms), down)
+    hip.launch(dev, "d4_mm_id2_iq2_xxs", ((n + 63) // 64, (ff + 63) // 64, ne), 128,
+               [d, ff, pool.grb, hip.I64(0), hip.I64(gb), ptrs, g["counts"], g["bases"], ne, hip.I64(rows), xq, xd, gg, gu])
+    mq, md, ms = A(dev, rows * ff), A(dev, 4 * rows * ff // 256), A(dev, 4 * rows * ff // 16)
+    hip.launch(dev, "d4_swiglu_w_q8k", (rows * ff // 256 + 3) // 4, 256, [rows, ff, float(clamp), gg, gu, g["wrow"], mq, md, ms])
+    hip.launch(dev, "d4_mm_id_q2_k", ((n + 63) // 64, (d + 63) // 64, ne), 128,
+               [ff, d, pool.drb, ff, d, hip.I64(2 * gb), ptrs, g["counts"], g["bases"], mq, down, md, ms, hip.I64(rows)])
     hip.launch(dev, "d4_moe_sum_rows", (n * d + 255) // 256, 256, [d, nu, n, down, g["smap"], sout, moe])
     if ws:
         return moe
@@ -489,6 +485,6 @@ def ffn_routed_chunk(dev, pool, logits, norm2, sout, n, ne, nu, scale, clamp, bi
         keep["sel"] = hip.hip_download(sel, np.uint32, rows).reshape(n, nu)
         keep["w"] = hip.hip_floats(w, rows).reshape(n, nu)
         keep["counts"] = hip.hip_download(g["counts"], np.uint32, ne)
-    for b in [sel, w, x, xq, xd, xs, gg, gu, mid, mq, md, ms, down] + list(g.values()):
+    for b in [sel, w, tq, td, ts, xq, xd, gg, gu, mq, md, ms, down] + list(g.values()):
         hip.hip_free(b)
     return moe

@@ -488,6 +488,14 @@ int ilt_mm_q8_mma2(uint64_t stream, const int8_t* w0, const uint16_t* d0, float*
 int ilt_d4_mm_id_iq2_xxs(uint64_t stream, int ncols, int nrows, int row_bytes, int64_t add, const uint64_t* ptrs,
                          const uint32_t* counts, const uint32_t* bases, int ne, int64_t total_rows,
                          const int8_t* xq, const float* xd, float* y);
+/* Not in the reference: gate and up of every expert in one launch (the numbers of two d4_mm_id_iq2_xxs); rows of Q8_K quants (and
+   their block scales) gathered through map; d4_swiglu_w and quantize-q8k! of its n rows of ff in one launch. */
+int ilt_d4_mm_id2_iq2_xxs(uint64_t stream, int ncols, int nrows, int row_bytes, int64_t add_gate, int64_t add_up, const uint64_t* ptrs,
+                          const uint32_t* counts, const uint32_t* bases, int ne, int64_t total_rows, const int8_t* xq, const float* xd,
+                          float* gate, float* up);
+int ilt_d4_gather_q8k(uint64_t stream, int d, int nrows, const int8_t* xq, const float* xd, const uint32_t* map, int8_t* oq, float* od);
+int ilt_d4_swiglu_w_q8k(uint64_t stream, int n, int ff, float clamp, const float* g, const float* u, const float* w, int8_t* xq, float* xd,
+                        int32_t* bsums);
 int ilt_d4_mm_id_q2_k(uint64_t stream, int ncols, int nrows, int row_bytes, int64_t add, const uint64_t* ptrs,
                       const uint32_t* counts, const uint32_t* bases, int ne, int64_t total_rows,
                       const int8_t* xq, const float* xd, const int32_t* bsums, float* y);
