@@ -683,7 +683,7 @@ int ilt_d4_ffn_small(uint64_t stream, void* wsp, uint64_t ws_bytes, int n, int n
   ILT_TRY(ilt_k_quant_q8(x, xq, xs, nullptr, (long long)n * d / 32, 0, S(stream)));
   if ((e = ilt_mm_q8_mma2(stream, wt->sgate_q, wt->sgate_d, sg, nullptr, ff, wt->sup_q, wt->sup_d, su, nullptr, ff, nullptr, nullptr, nullptr, nullptr, 0,
                           xq, xs, d, n, 0))) return e;
-  ILT_TRY(ilt_k_swiglu_w(n, ff, clamp, sg, su, nullptr, nullptr, mq, ms, S(stream)));
+  ILT_TRY(ilt_k_swiglu_w_quant_q8(n, ff, clamp, sg, su, nullptr, mq, ms, S(stream)));
   if ((e = ilt_mm_q8(stream, wt->sdown_q, wt->sdown_d, mq, ms, sout, nullptr, d, ff, n, 0))) return e;
   // the routed experts, a slot a (token, slot) row, an expert's rows one after another
   if ((e = gemv_experts(stream, ILT_IQ2_XXS, d, ff, grb, 0, wt->gate_bytes, d, ff, wt->slots, rows, nullptr, nullptr, nullptr, x, wrow, clamp, bm, rexp,
@@ -813,6 +813,11 @@ int ilt_d4_mm_id2_iq2_xxs(uint64_t stream, int ncols, int nrows, int row_bytes, 
 int ilt_d4_gather_q8k(uint64_t stream, int d, int nrows, const int8_t* xq, const float* xd, const uint32_t* map, int8_t* oq, float* od) {
   ILT_REQUIRE(d > 0 && d % 256 == 0 && nrows >= 0 && (nrows == 0 || (xq && xd && map && oq && od)) && (((uintptr_t)xq | (uintptr_t)oq) & 15) == 0);
   return (int)ilt_k_gather_q8k(d, nrows, xq, xd, map, oq, od, S(stream));
+}
+
+int ilt_d4_swiglu_q8(uint64_t stream, int n, int ff, float clamp, const float* g, const float* u, int8_t* xq, float* xs) {
+  ILT_REQUIRE(n >= 0 && ff > 0 && ff % 32 == 0 && (n == 0 || (g && u && xq && xs)));
+  return (int)ilt_k_swiglu_w_quant_q8(n, ff, clamp, g, u, nullptr, xq, xs, S(stream));
 }
 
 int ilt_d4_swiglu_w_q8k(uint64_t stream, int n, int ff, float clamp, const float* g, const float* u, const float* w, int8_t* xq, float* xd, int32_t* bsums) {
@@ -1281,6 +1286,8 @@ int ilt_dense_chunk(const ilt_dense_model* m, int nparts, const ilt_dense_work* 
       const ilt_dense_act& f = W.act[2];
       if (f.kq && !f.xq) {
         if ((e = ilt_swiglu_quant_q8k(W.stream, W.fa, W.fb, f.kq, f.kd, f.ksum, (int64_t)n * m->ffn / 256))) return e;
+      } else if (f.xq && !f.kq) {
+        ILT_TRY(ilt_k_swiglu_quant_q8(W.fa, W.fb, f.xq, f.xs, (long long)n * m->ffn / 32, 1, S(W.stream)));
       } else {
         if ((e = ilt_swiglu(W.stream, W.fa, W.fb, (int64_t)n * m->ffn))) return e;
         if ((e = chunk_quant(W.stream, W.fa, nullptr, f, m->ffn, 0.0f, n))) return e;
@@ -1429,6 +1436,7 @@ int ilt_launch(const char* kernel, unsigned gx, unsigned gy, unsigned gz, unsign
     return ilt_d4_mm_id2_iq2_xxs(stream, a.i32(0), a.i32(1), a.i32(2), a.i64(3), a.i64(4), a.ptr<const uint64_t*>(5), a.ptr<cu32>(6), a.ptr<cu32>(7),
                                  a.i32(8), a.i64(9), a.ptr<ci8>(10), a.ptr<cf>(11), a.ptr<float*>(12), a.ptr<float*>(13));
   K("d4_gather_q8k") return ilt_d4_gather_q8k(stream, a.i32(0), a.i32(1), a.ptr<ci8>(2), a.ptr<cf>(3), a.ptr<cu32>(4), a.ptr<int8_t*>(5), a.ptr<float*>(6));
+  K("d4_swiglu_q8") return ilt_d4_swiglu_q8(stream, a.i32(0), a.i32(1), a.f32(2), a.ptr<cf>(3), a.ptr<cf>(4), a.ptr<int8_t*>(5), a.ptr<float*>(6));
   K("d4_swiglu_w_q8k") return ilt_d4_swiglu_w_q8k(stream, a.i32(0), a.i32(1), a.f32(2), a.ptr<cf>(3), a.ptr<cf>(4), a.ptr<cf>(5), a.ptr<int8_t*>(6),
                                                   a.ptr<float*>(7), a.ptr<int32_t*>(8));
   K("d4_mm_id_q2_k")

@@ -28,8 +28,6 @@ struct BfParams {
   unsigned up_delta; const float* wrow; float clamp; u16* mid;
   // the exact products (gemm_i8r_kernel): x = the tokens' Q8_K quants (a byte a column), with their block scales and sums of 16
   const float* xd; const int* bsums;
-  // Q8_0 (gemm_i8q_kernel): w = the quants (a byte a weight, rows of cols bytes), wdq their f16 scales, xd the tokens' scales (one per 32)
-  const u16* wdq;
   // the planes made beforehand (gemm_i8pp_kernel): w = the hi plane, wlo the lo plane (a byte a weight, rows of cols bytes), wdf = d per row and super-block
   const u8* wlo; const float* wdf;
   // the columns split over workgroups (gemm_bf16_kernel, dense): workgroups from split_from on take the tiles from

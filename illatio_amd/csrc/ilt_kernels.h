@@ -123,8 +123,10 @@ unsigned long long ilt_k_streamed_launches();      // decode products launched a
 
 hipError_t ilt_k_quant_q8(const float* x, int8_t* xq, float* xs, int* xsum, long long nblocks, int f16_scale, hipStream_t st);
 hipError_t ilt_k_quant_q8k(const float* x, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st);
+hipError_t ilt_k_swiglu_quant_q8(const float* gate, const float* up, int8_t* xq, float* xs, long long nblocks, int f16_scale, hipStream_t st);
 hipError_t ilt_k_swiglu_quant_q8k(const float* gate, const float* up, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st);
 // d4_swiglu_w and quantize-q8k! of its rows in one
+hipError_t ilt_k_swiglu_w_quant_q8(int nrows, int ff, float clamp, const float* gate, const float* up, const float* wrow, int8_t* xq, float* xs, hipStream_t st);
 hipError_t ilt_k_swiglu_w_quant_q8k(int nrows, int ff, float clamp, const float* gate, const float* up, const float* wrow, int8_t* xq, float* xd, int* bsums,
                                     hipStream_t st);
 // ntok rows of cols floats, x_stride floats apart, quantized into packed rows: quantize-q8! (k 0) or quantize-q8k! (k 1)
@@ -185,9 +187,9 @@ hipError_t ilt_k_planes_i8(int fmt, const uint8_t* w, long long row_bytes, int r
                            hipStream_t st);
 hipError_t ilt_k_gemm_i8_pp(const uint8_t* wh, const uint8_t* wl, const float* wdf, int rows, int cols, const int8_t* xq, const float* xd,
                             int ntok, float* y, const float* bias, int acc, hipStream_t st);
-// Q8_0, exact, on the pipelined kernel (cols a multiple of 64)
-hipError_t ilt_k_gemm_i8_q8(const uint8_t* wq, const uint16_t* wd, int rows, int cols, const int8_t* xq, const float* xs, int ntok,
-                            float* y, const float* bias, int acc, hipStream_t st, long long ldy = 0);
+// Up to four Q8_0 matrices on the same tokens, exact (cols a multiple of 64)
+hipError_t ilt_k_gemm_q8(int nmat, const uint8_t* const* ws, const uint16_t* const* wds, const int* rows, float* const* ys, const float* const* biases,
+                         int cols, const int8_t* xq, const float* xs, int ntok, int acc, hipStream_t st, long long ldy = 0);
 // The experts' IQ2_XXS and Q2_K, grouped: expert z's counts[z] rows from bases[z] on; y2 set: a second matrix of each expert at add2
 // as well (bsums: Q2_K only)
 hipError_t ilt_k_gemm_i8_reg_id(int fmt, const uint64_t* ptrs, long long add, long long add2, const uint32_t* counts, const uint32_t* bases, int ne,

@@ -442,9 +442,10 @@ hipError_t ilt_k_gemm_i8(int fmt, const uint8_t* w, const uint16_t* wd, long lon
       e = ilt_k_gemm_i8_reg(1, &fmt, &w, &rows, &y, &bias, cols, xq, xs, bsums, ntok, acc, st, ldy);
     if (e != hipErrorNotSupported) return e;
   }
-  const bool fits = rows < (1 << 21) && ldy < (1 << 21) && (long long)rows * row_bytes < 0x7FFFFFFFLL;      // the pipelined kernel's 32-bit offsets
-  if (fits && fmt == ILT_Q8_0 && cols % 64 == 0 && forced != 0 && (forced == 1 || (ntok >= 96 && rows >= 128)))
-    return ilt_k_gemm_i8_q8(w, wd, rows, cols, xq, xs, ntok, y, bias, acc, st, ldy);
+  if (fmt == ILT_Q8_0 && forced != 0) {
+    const hipError_t e = ilt_k_gemm_q8(1, &w, &wd, &rows, &y, &bias, cols, xq, xs, ntok, acc, st, ldy);
+    if (e != hipErrorNotSupported) return e;
+  }
   GemmParams p = {};
   p.w = w; p.wdq = wd; p.rows = rows; p.cols = cols; p.row_bytes = row_bytes;
   p.xq = xq; p.xs = xs; p.bsums = bsums; p.y = y; p.bias = bias; p.acc = acc; p.ntok = ntok; p.ldy = (long)ldy;

@@ -431,8 +431,10 @@ hipError_t few_dispatch(FewParams& p, int forced, hipStream_t st) {
 // lies at the number of 32 x 32 tiles that take as long (Q4_K: 2560 x 4096 on 192 tokens, 480 tiles: 25 against 33 us, on 256,
 // 640: 38 against 33; 19456 x 2560 on 24, 608: 22 against 32, on 48, 1,216: 37 against 33; Q6_K: 2560 x 9728 on 192, 480: 63
 // against 75, on 256: 91 against 75; 9728 x 2560 on 24, 304: 21 against 23, on 48: 32 against 23).  With up to 32 tokens the
-// other kernel does four times the work for nothing, with up to 16 eight times.  Q8_0 against the pipelined kernel of its own,
-// which wants 96 tokens and 128 rows: 640 tiles (4864 x 896 on 128 tokens 16.8 against 18.6, on 256 25 against 20).
+// other kernel does four times the work for nothing, with up to 16 eight times.  Q8_0 against its own kernel (kernels_gemm_q8.hip),
+// whose waves make a tile's terms and sums in registers: up to 16 tokens here, unless the tiles of 16 rows fill the chip (896 x 4864
+// on 16 tokens 12.7 us against 16.1, on 24 17.1 against 16.1; 4096 x 2048 on 16, 256 tiles: 8.1 against 8.3; 9728 x 896, 608:
+// 7.7 against 5.8); where its smallest tile does not go (cols no multiple of 128) from 640 tiles of 32 x 32 and 96 tokens on.
 // ILT_I8_FEW (tests): "0" never, "1" always, "2", "4", "8" always, that cut.
 hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws, const uint16_t* const* wds, const int* rows, float* const* ys,
                              const float* const* biases, int cols, const int8_t* xq, const float* xs, const int* bsums, int ntok, int acc,
@@ -456,12 +458,17 @@ hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws
     m.row_bytes = fm == ILT_Q8_0 ? cols : (long long)(cols / 256) * (fm == ILT_Q4_K ? 144 : ILT_Q6K_STRIDE);
     if (m.ldy < rows[i] || (long long)rows[i] * m.row_bytes >= 0x7FFFFFFFLL || (((uintptr_t)ws[i]) & 15)) return hipErrorNotSupported;   // 32-bit offsets
     tiles32 += (rows[i] + 31) / 32;
-    small |= rows[i] < 128 || (fm == ILT_Q8_0 && cols % 64 != 0);
+    small |= rows[i] < 128;
   }
   tiles32 *= (ntok + 31) / 32;
   if (tiles32 > 0x3FFFFFFF) return hipErrorNotSupported;
   const long long line = ntok <= 32 ? 1250 : fset == ILT_Q4_K ? 620 : fset == ILT_Q6_K ? 480 : 550;
-  if (forced < 0 && !small && (fset == ILT_Q8_0 ? ntok >= 96 && tiles32 > 640 : ntok > 16 && tiles32 > line)) return hipErrorNotSupported;
+  if (forced < 0 && fset == ILT_Q8_0) {
+    if (cols % 128 == 0 ? ntok > 16 || tiles32 > 128 : ntok >= 96 && tiles32 > 640) {
+      const hipError_t e = ilt_k_gemm_q8(nmat, ws, wds, rows, ys, biases, cols, xq, xs, ntok, acc, st, ldy);
+      if (e != hipErrorNotSupported) return e;
+    }
+  } else if (forced < 0 && !small && ntok > 16 && tiles32 > line) return hipErrorNotSupported;
   switch (fset) {
     case ILT_Q8_0: return few_dispatch<ILT_Q8_0>(p, forced, st);
     case ILT_Q4_K: return few_dispatch<ILT_Q4_K>(p, forced, st);

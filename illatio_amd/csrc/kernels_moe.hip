@@ -123,7 +123,7 @@ __global__ __launch_bounds__(256) void gather_q8k_kernel(int d, long long pieces
   if (c < d / 256) od[(long long)r * (d / 256) + c] = xd[t * (d / 256) + c];
 }
 
-// mid[r][j] = (silu(g) * u) * w[r] (no w: weights of one), g and u clamped first when clamp > 1e-6
+// mid[r][j] = (silu(g) * u) * w[r], g and u clamped first when clamp > 1e-6
 // (d4-routed!, ds4f.lisp:1016-1019); quantized to Q8_0 with a float scale as well when xq
 // is given (the shared expert's down projection takes Q8_0 activations).
 __global__ __launch_bounds__(256) void swiglu_w_kernel(long long total, int ff, float clamp, const float* __restrict__ g,
@@ -135,9 +135,8 @@ __global__ __launch_bounds__(256) void swiglu_w_kernel(long long total, int ff, 
   if (live) {
     float gv = g[i], uv = u[i];
     if (clamp > 1e-6f) { gv = fminf(gv, clamp); uv = fmaxf(-clamp, fminf(uv, clamp)); }
-    v = ilt_silu(gv) * uv;
-    if (w) v = v * w[i / ff];
-    if (mid) mid[i] = v;
+    v = (ilt_silu(gv) * uv) * w[i / ff];
+    mid[i] = v;
   }
   if (xq) {
     float amax = ilt_max16(fabsf(v));

@@ -9,59 +9,81 @@ namespace {
 
 __device__ const u64 q_grid_dev[256] = { ILT_IQ2XXS_GRID_VALUES };
 
-// Q8_0 activations (quantize-q8!): a block of 32 per half wave.  d = amax/127; the
-// stored scale is d through fp16 when f16_scale; q = round-half-even(x * (1/d)) with the
-// unrounded d.  xsum (optional) gets the block's integer sum.
-__global__ __launch_bounds__(256) void quant_q8_kernel(const float* __restrict__ x, i8* __restrict__ xq,
-                                                       float* __restrict__ xs, int* __restrict__ xsum,
-                                                       long long nblocks, int f16_scale, long long bpr, long long x_stride) {
+// The value that is quantized.  GLU 1: swiglu!'s (model.lisp:364-378) of g and u, (g / (1 + e^-g)) * u with the exponential
+// through double; GLU 2: d4-routed!'s (ds4f.lisp:1016-1019), clamped, times the row's weight (null: one).  A prompt chunk's gated
+// activations go straight into the blocks the down product reads, and the floats are neither written nor read again.
+template <int GLU>
+__device__ __forceinline__ float glu_of(float g, float u, float clamp, const float* __restrict__ wrow, u32 row) {
+  if (GLU == 0) return g;
+  if (GLU == 1) return (g / (1.0f + ilt_expf_via_double(-g))) * u;
+  if (clamp > 1e-6f) { g = fminf(g, clamp); u = fmaxf(-clamp, fminf(u, clamp)); }
+  const float v = ilt_silu(g) * u;
+  return wrow ? v * wrow[row] : v;
+}
+
+// Q8_0 activations (quantize-q8!): a block of 32 by eight lanes, four values each (a 16-byte load, a 4-byte store; a value a
+// lane moved 4 bytes a lane and instruction: 4,096 x 1,000 values in 14.3 us).  d = amax/127; the stored scale is d through
+// fp16 when f16_scale; q = round-half-even(x * (1/d)) with the unrounded d.  xsum (optional) gets the block's integer sum.
+// bpr: blocks in a row (rows x_stride floats apart); 0: all in one.
+template <int GLU>
+__global__ __launch_bounds__(256) void quant_q8_kernel(const float* __restrict__ x, const float* __restrict__ up, i8* __restrict__ xq,
+                                                       float* __restrict__ xs, int* __restrict__ xsum, u32 nblocks, int f16_scale, u32 bpr,
+                                                       long long x_stride, float clamp, const float* __restrict__ wrow) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  const long long b = i >> 5;
-  const bool live = b < nblocks;
-  // bpr > 0: rows of bpr blocks, x_stride floats from one row's start to the next's (the output stays packed)
-  const float v = live ? x[bpr > 0 ? (b / bpr) * x_stride + (b % bpr) * 32 + (i & 31) : i] : 0.0f;
-  float amax = ilt_max16(fabsf(v));
-  amax = fmaxf(amax, __shfl_xor(amax, 16));
+  const u32 b = (u32)(i >> 3);
+  const bool live = (i >> 3) < nblocks;
+  const u32 row = bpr ? b / bpr : 0;
+  float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (live) {
+    const long long at = bpr ? row * x_stride + (long long)(b - row * bpr) * 32 + 4 * (i & 7) : 4 * i;
+    const int4 g4 = ilt_ld16((const u8*)(x + at));
+    const float g[4] = {__int_as_float(g4.x), __int_as_float(g4.y), __int_as_float(g4.z), __int_as_float(g4.w)};
+    int4 u4 = {};
+    if (GLU) u4 = ilt_ld16((const u8*)(up + at));
+    const float u[4] = {__int_as_float(u4.x), __int_as_float(u4.y), __int_as_float(u4.z), __int_as_float(u4.w)};
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = glu_of<GLU>(g[k], u[k], clamp, wrow, row);
+  }
+  float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+  amax = fmaxf(amax, ilt_dppf<ILT_DPP_XOR1>(amax));
+  amax = fmaxf(amax, ilt_dppf<ILT_DPP_XOR2>(amax));
+  amax = fmaxf(amax, ilt_dppf<ILT_DPP_HALF_MIRROR>(amax));
   const float d = amax / 127.0f;
   const float id = d == 0.0f ? 0.0f : 1.0f / d;
-  const int q = (int)rintf(v * id);
-  int sum = ilt_sum16(q);
-  sum += __shfl_xor(sum, 16);
-  if (!live) return;
-  xq[i] = (i8)q;
-  if ((threadIdx.x & 31) == 0) {
-    xs[b] = f16_scale ? __half2float(__float2half_rn(d)) : d;
-    if (xsum) xsum[b] = sum;
+  int q[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) q[k] = (int)rintf(v[k] * id);
+  if (xsum) {
+    const int sum = ilt_sum8((q[0] + q[1]) + (q[2] + q[3]));
+    if (live && (threadIdx.x & 7) == 0) xsum[b] = sum;
   }
+  if (!live) return;
+  const u32 packed = (u32)(q[0] & 0xFF) | ((u32)(q[1] & 0xFF) << 8) | ((u32)(q[2] & 0xFF) << 16) | ((u32)(q[3] & 0xFF) << 24);
+  __builtin_memcpy(xq + 4 * i, &packed, 4);
+  if ((threadIdx.x & 7) == 0) xs[b] = f16_scale ? __half2float(__float2half_rn(d)) : d;
 }
 
 // Q8_K activations (quantize-q8k!): a block of 256 per wave, four consecutive values a lane
 // (a 16-byte load, a 4-byte store; no LDS, no barrier).  The largest-magnitude value, the
 // first of equals, sets iscale = -127/max; q = min(127, round-half-even(iscale*x));
 // d = 1/iscale; sums of each 16 quants.
-// GLU: the values quantized are swiglu!'s (model.lisp:364-378) of x and up, (x / (1 + e^-x)) * up with the exponential
-// through double -- a prompt chunk's gated activations go straight into the blocks the down product reads, and the
-// floats are neither written nor read again.  GLU 2: d4-routed!'s (ds4f.lisp:1016-1019), clamped, times the row's weight.
 template <int GLU>
 __global__ __launch_bounds__(256) void quant_q8k_kernel(const float* __restrict__ x, const float* __restrict__ up, i8* __restrict__ xq,
-                                                        float* __restrict__ xd, int* __restrict__ bsums, long long nblocks,
-                                                        long long bpr, long long x_stride, float clamp, const float* __restrict__ wrow) {
+                                                        float* __restrict__ xd, int* __restrict__ bsums, u32 nblocks,
+                                                        u32 bpr, long long x_stride, float clamp, const float* __restrict__ wrow) {
   const int lane = threadIdx.x & 63;
-  const long long b = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (b >= nblocks) return;
+  const u32 bw = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (bw >= nblocks) return;
   // bpr > 0: rows of bpr blocks, x_stride floats (a multiple of 4) from one row's start to the next's
-  const float4 v4 = ((const float4*)(x + (bpr > 0 ? (b / bpr) * x_stride + (b % bpr) * 256 : b * 256)))[lane];
+  const u32 row = bpr ? bw / bpr : 0;
+  const long long b = bw;
+  const float4 v4 = ((const float4*)(x + (bpr ? row * x_stride + (long long)(bw - row * bpr) * 256 : b * 256)))[lane];
   float v[4] = {v4.x, v4.y, v4.z, v4.w};
   if (GLU) {
     const float4 u4 = ((const float4*)(up + b * 256))[lane];
     const float u[4] = {u4.x, u4.y, u4.z, u4.w};
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      if (GLU == 1) { v[k] = (v[k] / (1.0f + ilt_expf_via_double(-v[k]))) * u[k]; continue; }
-      float g = v[k], uu = u[k];
-      if (clamp > 1e-6f) { g = fminf(g, clamp); uu = fmaxf(-clamp, fminf(uu, clamp)); }
-      v[k] = (ilt_silu(g) * uu) * wrow[b / bpr];
-    }
+    for (int k = 0; k < 4; k++) v[k] = glu_of<GLU>(v[k], u[k], clamp, wrow, row);
   }
   // |v|'s bits order as |v| does; the low word prefers the earlier index
   u64 key = 0;
@@ -260,32 +282,51 @@ __global__ __launch_bounds__(256) void mm_f16_dot16_kernel(int ncols, int nrows,
 
 }  // namespace
 
-hipError_t ilt_k_quant_q8(const float* x, int8_t* xq, float* xs, int* xsum, long long nblocks, int f16_scale, hipStream_t st) {
+namespace {
+// up: GLU's other half; bpr blocks a row (0: no rows), x_stride floats from one row's start to the next's
+template <int GLU>
+hipError_t launch_q8(const float* x, const float* up, int8_t* xq, float* xs, int* xsum, long long nblocks, int f16_scale, long long bpr, long long x_stride,
+                     float clamp, const float* wrow, hipStream_t st) {
   if (nblocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(quant_q8_kernel, dim3((unsigned)((nblocks * 32 + 255) / 256)), dim3(256), 0, st, x, xq, xs, xsum, nblocks, f16_scale,
-                     0LL, 0LL);
+  if (nblocks > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(quant_q8_kernel<GLU>, dim3((unsigned)((nblocks + 31) / 32)), dim3(256), 0, st, x, up, xq, xs, xsum, (u32)nblocks, f16_scale, (u32)bpr,
+                     x_stride, clamp, wrow);
   return hipGetLastError();
+}
+template <int GLU>
+hipError_t launch_q8k(const float* x, const float* up, int8_t* xq, float* xd, int* bsums, long long nblocks, long long bpr, long long x_stride, float clamp,
+                      const float* wrow, hipStream_t st) {
+  if (nblocks <= 0) return hipSuccess;
+  if (nblocks > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(quant_q8k_kernel<GLU>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, x, up, xq, xd, bsums, (u32)nblocks, (u32)bpr, x_stride,
+                     clamp, wrow);
+  return hipGetLastError();
+}
+}  // namespace
+
+hipError_t ilt_k_quant_q8(const float* x, int8_t* xq, float* xs, int* xsum, long long nblocks, int f16_scale, hipStream_t st) {
+  return launch_q8<0>(x, nullptr, xq, xs, xsum, nblocks, f16_scale, 0, 0, 0.0f, nullptr, st);
 }
 
 hipError_t ilt_k_quant_q8k(const float* x, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st) {
-  if (nblocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(quant_q8k_kernel<0>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, x, (const float*)nullptr, xq, xd, bsums, nblocks, 0LL, 0LL, 0.0f, (const float*)nullptr);
-  return hipGetLastError();
+  return launch_q8k<0>(x, nullptr, xq, xd, bsums, nblocks, 0, 0, 0.0f, nullptr, st);
 }
 
 hipError_t ilt_k_swiglu_quant_q8k(const float* gate, const float* up, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st) {
-  if (nblocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(quant_q8k_kernel<1>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, gate, up, xq, xd, bsums, nblocks, 0LL, 0LL, 0.0f, (const float*)nullptr);
-  return hipGetLastError();
+  return launch_q8k<1>(gate, up, xq, xd, bsums, nblocks, 0, 0, 0.0f, nullptr, st);
+}
+
+hipError_t ilt_k_swiglu_quant_q8(const float* gate, const float* up, int8_t* xq, float* xs, long long nblocks, int f16_scale, hipStream_t st) {
+  return launch_q8<1>(gate, up, xq, xs, nullptr, nblocks, f16_scale, 0, 0, 0.0f, nullptr, st);
+}
+
+hipError_t ilt_k_swiglu_w_quant_q8(int nrows, int ff, float clamp, const float* gate, const float* up, const float* wrow, int8_t* xq, float* xs, hipStream_t st) {
+  return launch_q8<2>(gate, up, xq, xs, nullptr, (long long)nrows * (ff / 32), 0, ff / 32, ff, clamp, wrow, st);
 }
 
 hipError_t ilt_k_swiglu_w_quant_q8k(int nrows, int ff, float clamp, const float* gate, const float* up, const float* wrow, int8_t* xq, float* xd, int* bsums,
                                     hipStream_t st) {
-  const long long nblocks = (long long)nrows * (ff / 256);
-  if (nblocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(quant_q8k_kernel<2>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, gate, up, xq, xd, bsums, nblocks, (long long)(ff / 256),
-                     (long long)ff, clamp, wrow);
-  return hipGetLastError();
+  return launch_q8k<2>(gate, up, xq, xd, bsums, (long long)nrows * (ff / 256), ff / 256, ff, clamp, wrow, st);
 }
 
 hipError_t ilt_k_quant_rows(int k, const float* x, int8_t* xq, float* xs, int* bsums, long long ntok, int cols, long long x_stride,
@@ -294,10 +335,8 @@ hipError_t ilt_k_quant_rows(int k, const float* x, int8_t* xq, float* xs, int* b
   if (ntok <= 0) return hipSuccess;
   if (cols <= 0 || cols % bw != 0 || x_stride < cols || (k && x_stride % 4 != 0)) return hipErrorInvalidValue;
   const long long bpr = cols / bw, nblocks = ntok * bpr;
-  if (k) hipLaunchKernelGGL(quant_q8k_kernel<0>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, x, (const float*)nullptr, xq, xs, bsums, nblocks, bpr, x_stride, 0.0f, (const float*)nullptr);
-  else hipLaunchKernelGGL(quant_q8_kernel, dim3((unsigned)((nblocks * 32 + 255) / 256)), dim3(256), 0, st, x, xq, xs, (int*)nullptr, nblocks,
-                          f16_scale, bpr, x_stride);
-  return hipGetLastError();
+  if (k) return launch_q8k<0>(x, nullptr, xq, xs, bsums, nblocks, bpr, x_stride, 0.0f, nullptr, st);
+  return launch_q8<0>(x, nullptr, xq, xs, nullptr, nblocks, f16_scale, bpr, x_stride, 0.0f, nullptr, st);
 }
 
 hipError_t ilt_k_repack_q8(const uint8_t* raw, int8_t* qs, uint16_t* d, long long nblocks, hipStream_t st) {

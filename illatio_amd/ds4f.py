@@ -147,21 +147,22 @@ def dk_mm(dev, kernel, w, wd, rbytes, rows, cols, x, y, n, x_stride=None, y_stri
 
 def ffn_shared_chunk(dev, sh, norm2, n, clamp, ws=None):
     """The shared expert of a chunk of N tokens (DK-FFN-HEAD-CHUNK's second half, cuda-ds4f-prefill.lisp:294-298):
-    gate and up through D4_MM_Q8_0 on the float rows, the gated activation, down through D4_MM_Q8_0.  Each token's
-    row has d4-shared!'s bits.  Returns SOUT (N x d)."""
+    D4_MM_Q8_0's products, the rows quantized once for gate and up (one launch) and the gated activation where it
+    is made.  Each token's row has d4-shared!'s bits.  Returns SOUT (N x d)."""
     d, ff = sh.d, sh.ff
     A = ws.alloc if ws else hip.hip_alloc
-    sg, su, smid, sout = A(dev, 4 * n * ff), A(dev, 4 * n * ff), A(dev, 4 * n * ff), A(dev, 4 * n * d)
-    if getattr(sh, "ones", None) is None or sh.ones.bytes < 4 * n:
-        sh.ones = hip.hip_upload_new(dev, np.ones(n, np.float32))
-    dk_mm(dev, "d4_mm_q8_0", sh.gate.qs, sh.gate.d, 0, ff, d, norm2, sg, n)
-    dk_mm(dev, "d4_mm_q8_0", sh.up.qs, sh.up.d, 0, ff, d, norm2, su, n)
-    hip.launch(dev, "d4_swiglu_w", (n * ff + 255) // 256, 256, [n, ff, float(clamp), sg, su, sh.ones, smid, None, None])
-    dk_mm(dev, "d4_mm_q8_0", sh.down.qs, sh.down.d, 0, d, ff, smid, sout, n)
+    nq, ns = A(dev, n * d), A(dev, n * d // 8)
+    sg, su, sout = A(dev, 4 * n * ff), A(dev, 4 * n * ff), A(dev, 4 * n * d)
+    mq, ms = A(dev, n * ff), A(dev, n * ff // 8)
+    hip.launch(dev, "d4_quant", (n * d + 255) // 256, 256, [norm2, nq, ns, n * d // 32])
+    hip.launch(dev, "mm_q8_mma2", ((n + 63) // 64, (2 * ff + 63) // 64), 256,
+               [sh.gate.qs, sh.gate.d, sg, None, ff, sh.up.qs, sh.up.d, su, None, ff, None, None, None, None, 0, nq, ns, d, n, 0])
+    hip.launch(dev, "d4_swiglu_q8", (n * ff + 1023) // 1024, 256, [n, ff, float(clamp), sg, su, mq, ms])
+    hip.launch(dev, "mm_q8", ((n + 63) // 64, (d + 63) // 64), 256, [sh.down.qs, sh.down.d, mq, ms, sout, None, d, ff, n, 0])
     if ws:
         return sout
     hip.hip_sync(dev)
-    for b in (sg, su, smid):
+    for b in (nq, ns, sg, su, mq, ms):
         hip.hip_free(b)
     return sout
 
