@@ -392,61 +392,68 @@ __global__ __launch_bounds__(256, 2) void attn_scores_quad_kernel(const float* _
   }
 }
 
-// One token's qk_rope and scores in one launch: every workgroup of a query head norms and turns that head
-// itself (wave 0; a sixteenth of a microsecond of arithmetic against a launch), the workgroup whose 256
-// positions hold the token's own does the same for its KV head's key (wave 1) and takes that key from LDS,
-// and the group's first query head there writes the key and the value into the caches, for the launch with
-// the values.  q and k are left as they came.
+constexpr int kStepHeads = 8, kStepPositions = 128;      // a workgroup of one token's score kernel: query heads, positions
+// One token's qk_rope and scores in one launch.  A workgroup takes PB positions of a KV head for all (up to GH) of its query heads:
+// the keys, which are most of what the launch reads, come from memory once and lie in registers while one query head after another
+// is multiplied with them (a workgroup a query head read them once a head, and on different dies: 14.3 us at 4,117 positions of the
+// Qwen3-4B shape, 17 MB of keys).  Waves 0 .. GH - 1 norm and turn the query heads, the next one the KV head's key where the
+// workgroup's positions hold the token's own; that workgroup takes the key from LDS and writes key and value into the caches, for
+// the launch with the values.  q and k are left as they came.
 template <int NJ>      // hd / 16 as a constant, or 0: read at run time (heads up to 256)
-__global__ __launch_bounds__(1024) void attn_step_scores_kernel(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+__global__ __launch_bounds__(1024, 8) void attn_step_scores_kernel(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
                                                                 const float* __restrict__ qn, const float* __restrict__ kn,
                                                                 const float* __restrict__ rope, float* __restrict__ kc, float* __restrict__ vc,
                                                                 float* __restrict__ raw, int nh, int nkv, int hd, int rd, int pos, float eps,
                                                                 int neox, float scale, int spitch) {
-  __shared__ float qsh[256], ksh[256];
-  __shared__ double scs[2];
-  const int h = blockIdx.x, tid = threadIdx.x, npos = pos + 1, pbase = blockIdx.y * 256;
-  if (pbase >= npos) return;
-  const int group = nh / nkv, kvd = nkv * hd, kh = h / group, ko = kh * hd;
+  constexpr int GH = kStepHeads, NU = kStepPositions / 64;
+  __shared__ float qsh[GH][256], ksh[256];
+  __shared__ double scs[GH + 1];
+  const int kh = blockIdx.x, tid = threadIdx.x, npos = pos + 1, pbase = blockIdx.y * kStepPositions;
+  const int group = nh / nkv, kvd = nkv * hd, ko = kh * hd, h0 = kh * group + blockIdx.z * GH, heads = min(GH, group - (int)blockIdx.z * GH);
   constexpr int NJM = NJ ? NJ : 16;
   const int l = tid & 15, pg = tid >> 4, nj = NJ ? NJ : hd >> 4, wave = tid >> 6;
-  const bool own = pos < pbase + 256;              // this workgroup's positions hold the token's own
-  // the head's own loads first (waves 0 and 1), the keys' after: the norms and the turn wait for the first alone
+  const bool own = pos < pbase + kStepPositions;   // this workgroup's positions hold the token's own
+  // the heads' own loads first, the keys' after: the norms and the turns wait for the first alone
   const float* cs = rope + (long long)pos * rd;
   RopeIn<4> rin;
-  const bool turns = wave == 0 || (wave == 1 && own);
-  if (turns) rope_head_load(rin, wave == 0 ? q + h * hd : k + ko, wave == 0 ? qn : kn, cs, hd, rd, tid & 63);
-  float kv[4][NJM];
+  const bool isk = wave == GH, turns = wave < heads || (isk && own);
+  if (turns) rope_head_load(rin, isk ? k + ko : q + (h0 + wave) * hd, isk ? kn : qn, cs, hd, rd, tid & 63);
+  float kv[NU][NJM];
 #pragma unroll
-  for (int u = 0; u < 4; u++) {
+  for (int u = 0; u < NU; u++) {
     const float* kr = kc + (long long)min(pbase + 64 * u + pg, max(pos - 1, 0)) * kvd + ko;      // rows before the token's own
 #pragma unroll
     for (int j = 0; j < NJM; j++) kv[u][j] = (NJ || j < nj) ? kr[l + 16 * j] : 0.0f;
   }
-  if (turns) rope_head_turn(rin, (wave == 0 ? qn : kn) != nullptr, wave == 0 ? qsh : ksh, &scs[wave], hd, rd, eps, neox, tid & 63);
+  if (turns) rope_head_turn(rin, (isk ? kn : qn) != nullptr, isk ? ksh : qsh[wave], &scs[wave], hd, rd, eps, neox, tid & 63);
   __syncthreads();
-  if (own && h == kh * group && tid < hd) {
+  if (own && blockIdx.z == 0 && tid < hd) {
     kc[(long long)pos * kvd + ko + tid] = ksh[tid];
     vc[(long long)pos * kvd + ko + tid] = v[ko + tid];
   }
-  float qv[NJM];
 #pragma unroll
-  for (int j = 0; j < NJM; j++) qv[j] = (NJ || j < nj) ? qsh[l + 16 * j] : 0.0f;
-#pragma unroll
-  for (int u = 0; u < 4; u++) {
-    const int p = pbase + 64 * u + pg;
-    if (p == pos) {
+  for (int u = 0; u < NU; u++)
+    if (pbase + 64 * u + pg == pos) {
 #pragma unroll
       for (int j = 0; j < NJM; j++) kv[u][j] = (NJ || j < nj) ? ksh[l + 16 * j] : 0.0f;
     }
-    float sacc = 0.0f;
+#pragma unroll 1
+  for (int h = 0; h < heads; h++) {
+    float qv[NJM];
 #pragma unroll
-    for (int j = 0; j < NJM; j++) if (NJ || j < nj) sacc = sacc + kv[u][j] * qv[j];
-    sacc = sacc + ilt_dppf<ILT_DPP_SHL(4)>(sacc);
-    sacc = sacc + ilt_dppf<ILT_DPP_SHL(8)>(sacc);
-    sacc = sacc + ilt_dppf<ILT_DPP_SHL(1)>(sacc);
-    sacc = sacc + ilt_dppf<ILT_DPP_SHL(2)>(sacc);
-    if (l == 0 && p < npos) raw[(long long)h * spitch + p] = sacc * scale;
+    for (int j = 0; j < NJM; j++) qv[j] = (NJ || j < nj) ? qsh[h][l + 16 * j] : 0.0f;
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      const int p = pbase + 64 * u + pg;
+      float sacc = 0.0f;
+#pragma unroll
+      for (int j = 0; j < NJM; j++) if (NJ || j < nj) sacc = sacc + kv[u][j] * qv[j];
+      sacc = sacc + ilt_dppf<ILT_DPP_SHL(4)>(sacc);
+      sacc = sacc + ilt_dppf<ILT_DPP_SHL(8)>(sacc);
+      sacc = sacc + ilt_dppf<ILT_DPP_SHL(1)>(sacc);
+      sacc = sacc + ilt_dppf<ILT_DPP_SHL(2)>(sacc);
+      if (l == 0 && p < npos) raw[(long long)(h0 + h) * spitch + p] = sacc * scale;
+    }
   }
 }
 
@@ -1018,6 +1025,7 @@ __global__ __launch_bounds__(256) void attn_values_tiled_kernel(const float* __r
 // scores and stored into the buffer tile t-1 has left while tile t is being added, and tile t+2's loads are on their way
 // from then on.  All sixteen waves take the softmax first (the scores come from attn_step_scores_kernel, raw).  The
 // numbers are attn_values_tiled_kernel<1>'s: every product and every sum the same, in the same order.
+constexpr int kStreamMost = 8192;                  // positions: the scores' room ends there
 constexpr int kStreamTile = 480, kStreamPitch = kStreamTile + 36;      // (a row: 32 floats of room past a tile for the reads ahead; 4 mod 64)
 __global__ __launch_bounds__(1024) void attn_values_stream_kernel(const float* __restrict__ raw, const float* __restrict__ vc, float* __restrict__ out,
                                                                   int nh, int nkv, int hd, int pos, int spitch) {
@@ -1053,41 +1061,61 @@ __global__ __launch_bounds__(1024) void attn_values_stream_kernel(const float* _
       }
     }
   };
+  // The scores' loads go first and stay in registers through the softmax; the values', which come from memory, after them: loads
+  // return in the order they were asked for.  From here on the barriers wait for LDS alone (__syncthreads would wait for the
+  // tiles in flight at every one).
+  float e[kStreamMost / 1024];
+#pragma unroll
+  for (int u = 0; u < kStreamMost / 1024; u++) {
+    e[u] = -3.402823466e38f;
+    if (1024 * u < npos) e[u] = rw[min(tid + 1024 * u, npos - 1)];       // (the last position again, where there is none: the maximum is the same)
+  }
   float4 ra[2], rb[2];
   if (wave > 0) {
     load_tile(0, ra);
     if (ntiles > 1) load_tile(1, rb);
   }
   // softmax (attn_softmax's steps over sixteen waves)
-  float mx = -3.402823466e38f;
-  for (int p = tid; p < npos; p += 1024) { const float sv = rw[p]; sc[p] = sv; mx = fmaxf(mx, sv); }
+  float mx = e[0];
+#pragma unroll
+  for (int u = 1; u < kStreamMost / 1024; u++) mx = fmaxf(mx, e[u]);
   mx = wave_max_float(mx);
   if (lane == 0) redf[wave] = mx;
-  __syncthreads();
+  ilt_barrier_lds();
   mx = redf[0];
 #pragma unroll
   for (int w = 1; w < 16; w++) mx = fmaxf(mx, redf[w]);
   double part = 0.0;
-  for (int p = tid; p < npos; p += 1024) { const float e = ilt_expf_via_double(sc[p] - mx); sc[p] = e; part += (double)e; }
+#pragma unroll
+  for (int u = 0; u < kStreamMost / 1024; u++)
+    if (1024 * u < npos) {
+      const int p = tid + 1024 * u;
+      e[u] = p < npos ? ilt_expf_via_double(e[u] - mx) : 0.0f;
+      part += (double)e[u];
+    }
   part = wave_sum_double(part);
   if (lane == 0) redd[wave] = part;
-  __syncthreads();
+  ilt_barrier_lds();
   double sum = redd[0];
 #pragma unroll
   for (int w = 1; w < 16; w++) sum += redd[w];
   float inv;
   if (!recip_settled(sum, npos, &inv)) {           // the same in every thread
+#pragma unroll
+    for (int u = 0; u < kStreamMost / 1024; u++) if (tid + 1024 * u < npos) sc[tid + 1024 * u] = e[u];
+    ilt_barrier_lds();
     if (tid == 0) { double s2 = 0.0; for (int p = 0; p < npos; p++) s2 += (double)sc[p]; redd[16] = s2; }
-    __syncthreads();
+    ilt_barrier_lds();
     inv = (float)(1.0 / redd[16]);
   }
-  for (int p = tid; p < npos; p += 1024) sc[p] = sc[p] * inv;
-  __syncthreads();                                 // every position's scaled score, for the products
+#pragma unroll
+  for (int u = 0; u < kStreamMost / 1024; u++) if (tid + 1024 * u < npos) sc[tid + 1024 * u] = e[u] * inv;
+  ilt_barrier_lds();                               // every position's scaled score, for the products
   if (wave > 0) store_tile(0, ra);
   float o = 0.0f;
   const float* col = vt + lane * kStreamPitch;     // (lanes 0 .. 15 of wave 0)
   auto step = [&](int t, float4 (&next)[2], float4 (&after)[2]) {      // next holds tile t+1; after: free, takes tile t+2
-    __syncthreads();                               // tile t is in place, and tile t-1's chains are through with the other buffer
+    ilt_barrier_lds();                               // tile t is in place, and tile t-1's chains are through with the other buffer
     if (wave == 0) {
       if (lane < 16) o = chain_add_from(o, col + (t & 1) * (16 * kStreamPitch), min(kStreamTile, npos - t * kStreamTile), kStreamPitch - 36);
     } else {
@@ -1587,7 +1615,8 @@ hipError_t ilt_k_attn_step(const float* q, const float* k, const float* v, const
     return hipGetLastError();
   }
   {
-    const dim3 gs(nh, (ctx + 255) / 256);
+    const int group = nh / nkv;
+    const dim3 gs(nkv, (ctx + kStepPositions - 1) / kStepPositions, (group + kStepHeads - 1) / kStepHeads);
     if (hd == 128)
       hipLaunchKernelGGL(attn_step_scores_kernel<8>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax);
     else if (hd == 64)
