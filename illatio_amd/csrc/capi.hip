@@ -360,7 +360,7 @@ static int gemv_experts(uint64_t stream, int fmt, int ncols, int nrows, int row_
   }
   p.ptrs = ptrs; p.sel = sel; p.cols = ncols;
   p.xq = xq; p.xs = xd; p.bsums = bsums; p.xf = xf; p.x_stride = x_stride; p.y_stride = y_stride;
-  p.counts = counts; p.bases = bases; p.xrow = xrow;
+  p.counts = counts; p.bases = counts ? bases : xrow;
   return (int)ilt_gemv_launch(p, nz, S(stream));
 }
 

@@ -105,10 +105,10 @@ struct IltGemvParams {
   IltRowsAhead rows_ahead;
   // grid y's expert on several rows of activations (the looping variant only): rows bases[y] .. bases[y] + counts[y] - 1
   // of the activations and of the output, x_stride / y_stride apart, its matrix read from memory once and from the
-  // cache for the rows after the first (the counts / bases of the reference's d4_mv_*, ds4f.cu:762-772); null = row y
+  // cache for the rows after the first (the counts / bases of the reference's d4_mv_*, ds4f.cu:762-772); null = row y.
+  // Bases without counts (the looping variant too): grid y works on the activations' row bases[y] and gives row y.
   const uint32_t* counts;
   const uint32_t* bases;
-  const uint32_t* xrow;      // grid y works on row xrow[y] of the activations (the looping variant only); null = row y
 };
 
 // The kernel is chosen by the matrices' formats (mat[i].fmt): one format, or Q4_K and Q6_K mixed.

@@ -701,7 +701,7 @@ __device__ __forceinline__ void gemv_body(const IltGemvParams& p, const int z, c
 
   // Float activations to quantize here: their first loads go out before any weight load, since
   // loads return in order and these (hot in L2) are needed first.
-  const long xoff = (p.xrow ? (long)p.xrow[xy] : xy) * p.x_stride + (long)group * p.cols;
+  const long xoff = (p.bases && !p.counts ? (long)p.bases[xy] : xy) * p.x_stride + (long)group * p.cols;
   float4 xfirst[4], nfirst[4];
   if (!q8 && p.xf) load_q8k_pass(p.xf + xoff, S, 0, xfirst);
   // ... and when they are normalized first: the norm's weights likewise, and now the squares
@@ -1578,7 +1578,7 @@ hipError_t ilt_gemv_launch(IltGemvParams& p, int nz, hipStream_t st) {
     if (!p.bases || !p.ptrs || p.sel || !p.xf || p.glu || p.acc || p.norm_w || p.group_rows || p.nmat != 1 || p.mat[0].bias ||
         !(fset == ILT_IQ2_XXS || fset == ILT_Q2_K))
       return hipErrorNotSupported;
-  } else if (!p.xrow) {
+  } else if (!p.bases) {
     const hipError_t e = gemv_stream_launch(p, fset, nz, st);
     if (e != hipErrorNotSupported || p.sum.rows) return e;
   }
