@@ -10,6 +10,7 @@ kernels between them add in the CPU's order.
 synth_model makes the random-init model the benchmark and the tests run (there are no model files here):
 Q4_K for most matrices, Q6_K for V, down and the tied embedding / output head, as Q4_K_M files have them.
 """
+import copy
 import ctypes as C
 
 import numpy as np
@@ -89,8 +90,7 @@ def _mat(w):
     return _Mat(w.type, w.rows, w.cols, w.qs.ptr, w.d.ptr if w.d else 0)
 
 
-PARTS_WORK = 1e10
-PARTS_FROM, PARTS_UPTO = 256, 4096      # eval_tokens: chunks of so many tokens as parts side by side on streams of their own (0, -1: never)
+PARTS_FROM, PARTS_UPTO = 193, 4096      # eval_tokens: pieces of a prompt of so many tokens as parts side by side on streams of their own (0, -1: never)
 
 
 class _Work:
@@ -324,15 +324,21 @@ class DenseModel:
         most of its launches with fewer workgroups than the GPU has room for (at 512 tokens V is 64 workgroups, wo and
         down 160, of 512 that fit), and while one part is in its attention (vector ALU) another is in its products
         (matrix cores): the parts' launches fill each other's gaps.  Every token's results are forward_n's."""
-        n, dev = len(tokens), self.dev
+        n, dev = len(tokens), self.dev      # (up to K chunks' tokens: a part is at most a chunk)
         per = ((n + k - 1) // k + 127) // 128 * 128
-        if k < 2 or per * (k - 1) >= n or n > self.chunk or self.pos + n > self.nctx or self.pos + n > 8192:
+        if k < 2 or per * (k - 1) >= n or per > self.chunk or self.pos + n > self.nctx or self.pos + n > 8192:
             return self.forward_n(tokens, logits)
-        while len(self.more_work) < k - 1:
-            import copy
-            dev2 = copy.copy(dev)
-            dev2.stream, dev2.second = hip.hip_stream_create(dev), None
-            self.more_work.append(self._work_set(dev2, ((self.chunk + 1) // 2 + 127) // 128 * 128))      # (a part: up to half a chunk, rounded up to whole tiles of 128 tokens)
+        for j in range(k - 1):
+            # (room for half a chunk from the start, for more once a longer part comes)
+            room = max(per, ((self.chunk + 1) // 2 + 127) // 128 * 128)
+            if j == len(self.more_work):
+                dev2 = copy.copy(dev)
+                dev2.stream, dev2.second = hip.hip_stream_create(dev), None
+                self.more_work.append(self._work_set(dev2, room))
+            elif self.more_work[j].n < per:
+                hip.hip_sync(dev)                       # (parts end before what this stream does next)
+                self._free_work(self.more_work[j])
+                self.more_work[j] = self._work_set(self.more_work[j].dev, room)
         works = [self.work] + self.more_work[:k - 1]
         parts = [tokens[j * per:(j + 1) * per] for j in range(k)]
         # (the events of a chunk of k parts: one a part but the last and layer, then one a part)
@@ -367,36 +373,45 @@ class DenseModel:
         return self.logits
 
     def eval_tokens(self, tokens, logits=True):
-        """The prompt in chunks (CUDA-EVAL, cuda-dense.lisp:295-305); the logits of the last token only.  A chunk of
-        PARTS_FROM to PARTS_UPTO tokens goes as two or four parts side by side where that was measured to gain
-        (forward_parts)."""
+        """The prompt in chunks (CUDA-EVAL, cuda-dense.lisp:295-305); the logits of the last token only.  Up to two chunks'
+        tokens go as two halves side by side where that was measured to gain (forward_parts)."""
         tokens = list(tokens)
-        for i in range(0, len(tokens), self.chunk):
-            part = tokens[i:i + self.chunk]
-            want = logits and i + len(part) >= len(tokens)
-            npart = len(part)
-            # Parts, measured on the Qwen3-4B shape (whole -> parts): 256 tokens 14.6 -> 14.0 ms, 512 18.7 -> 17.9 as halves;
-            # 900 31.7 -> 28.0, 1,024 33.0 -> 30.2, 1,100 37.6 -> 33.8, 1,280 42.9 -> 40.8, 1,536 53.3 -> 50.4, 1,800 68.2 -> 64.0 as
-            # halves (thirds and quarters of those lose); 2,048 78.8 -> 76.7 as halves, 72.1 as quarters.  Between 256 and 900
-            # tokens only the powers of two gain (384 +8 %, but 448 -2 %, 640 0, 768 -1 to -6 %).  A chunk of 512 tokens far
-            # into a long prompt is mostly attention, and its halves gain nothing (4,096 tokens in chunks of 512: 256.5 ->
-            # 258-266 ms).  The bf16 products from the quantized matrices: two halves from 1,024 tokens on (1,024 tokens
-            # 29.5 -> 26.1 ms, 2,048 66.7 -> 62.7; quarters lose, and so do halves of a 512-token chunk; their sums' order
-            # depends on a launch's token count with or without parts); from resident copies 28.4 -> 27.2 and 62.7 -> 62.1:
-            # left whole.  And a small model's launches are over before the next is queued, so twice as many of them only
-            # cost (the Qwen2.5-0.5B shape's 512-token prompt 7.7 -> 10.6 ms as halves): a part must bring PARTS_WORK products
-            # of a weight and a token to a layer (the Qwen3-4B shape's halves of 128 tokens bring 1.3e10, the 0.5B shape's
-            # halves of 256 tokens 3.8e9).
-            exact = self.prefill == "exact"
-            k = 4 if exact and npart >= 2048 else 2
-            c = self.c
-            layer_weights = c["d"] * (2 * self.qd + 2 * self.kvd + 3 * c["ffn"])
-            fits = npart >= 896 or (npart & (npart - 1) == 0 and self.pos < 1024)
-            if ((exact and fits) or (self.prefill == "bf16" and npart >= 1024)) and PARTS_FROM <= npart <= PARTS_UPTO \
-                    and (npart // k) * layer_weights >= PARTS_WORK:
-                self.forward_parts(part, logits=want, k=k)
-            else:
-                self.forward_n(part, logits=want)
+        i = 0
+        while i < len(tokens):
+            left = len(tokens) - i
+            n = min(left, 2 * self.chunk)
+            halves = self._gains_as_halves(n)
+            if not halves:
+                n = min(left, self.chunk)
+                halves = self._gains_as_halves(n)
+            want = logits and n == left
+            (self.forward_parts if halves else self.forward_n)(tokens[i:i + n], logits=want)
+            i += n
+
+    def _gains_as_halves(self, n):
+        """Whether the next N tokens of a prompt take less time as two halves side by side than whole (or, past a chunk, than
+        one after another)."""
+        half = ((n + 1) // 2 + 127) // 128 * 128
+        if not PARTS_FROM <= n <= PARTS_UPTO or half > self.chunk or self.pos + n > min(self.nctx, 8192):
+            return False
+        work = n // 2 * self.c["d"] * (2 * self.qd + 2 * self.kvd + 3 * self.c["ffn"])
+        if self.prefill != "exact":
+            # The bf16 products from the quantized matrices: from 1,024 tokens on (1,024 tokens 29.5 -> 26.1 ms, 2,048 66.7 ->
+            # 62.7; halves of a 512-token chunk lose; their sums' order depends on a launch's token count with or without
+            # parts); from resident copies 28.4 -> 27.2 and 62.7 -> 62.1: left whole.
+            return self.prefill == "bf16" and 1024 <= n <= self.chunk and work >= 1e10
+        # The exact ones, the Qwen3-4B shape (whole -> halves, ms; thirds and quarters always lose to halves): 640 tokens 15.6 ->
+        # 15.2, 832 21.0 -> 18.8, 1,024 24.5 -> 23.7, 2,048 60.2 -> 58.9; of two chunks 2,100 69.0 (2,048 and then 52) -> 62.4,
+        # 2,500 87.2 -> 81.7, 4,096 183.4 -> 179.4.  Below 640 the halves, whole tiles of 128 tokens but for the last, gain
+        # where they leave little of a tile empty: 224 tokens 10.1 -> 9.1, 256 10.4 -> 9.7..10.2, 448 13.0 -> 12.7, 512 14.0 ->
+        # 13.6; 288, 320, 416 and 576 lose up to 10 %.  Far into a conversation a few hundred tokens are mostly attention, whose
+        # launches fill the GPU whole: 448 at 1,500 positions 23.4 -> 24.7.
+        if not (n >= 640 or 448 <= n <= 512 and self.pos < 1024 or n <= 256):
+            return False
+        # A small model's launches are over before the next is queued, so twice as many of them only cost (the Qwen2.5-0.5B
+        # shape: 384 tokens 2.8 -> 3.0 ms, 512 3.28 -> 3.15, 1,024 6.7 -> 5.7; at 1,500 positions 1,536 tokens 16.8 -> 18.4,
+        # 2,048 even): a half must bring so many products of a weight and a token to a layer.
+        return work >= (3.5e9 if self.pos < 1024 else 1.2e10)
 
     def argmax(self):
         """The greedy token of self.logits (ARGMAX, model.lisp:464-468: the first of equal ones)."""

@@ -433,6 +433,31 @@ def test_a_chunk_as_parts_side_by_side(dev):
             assert np.array_equal(bits(a), bits(b)), (nprompt, chunk)
 
 
+@pytest.mark.parametrize("nprompt,first", [(257, 0), (300, 0), (512, 0), (400, 130)])
+def test_two_chunks_as_halves(dev, nprompt, first):
+    """Halves of more than one chunk together (chunks of 256; the second set of buffers grows after a shorter prompt's)."""
+    from illatio_amd import hip, model
+    host = model.synth_model(12, d=512, ffn=1024, nh=8, nkv=2, hd=64, nl=2, vocab=700)
+    c = host["config"]
+    prompt = synth.make_rng(78).integers(0, c["vocab"], first + nprompt).tolist()
+    res = []
+    for halves in (True, False):
+        m = model.DenseModel(dev, host, nctx=first + nprompt, chunk=256)
+        if first:
+            m.forward_parts(prompt[:first]) if halves else m.forward_n(prompt[:first])
+        if halves:
+            m.forward_parts(prompt[first:])
+        else:
+            m.forward_n(prompt[first:first + 256], logits=False)
+            m.forward_n(prompt[first + 256:])
+        hip.hip_sync(dev)
+        assert m.pos == first + nprompt
+        res.append([hip.hip_floats(m.logits, c["vocab"])] + [hip.hip_floats(m.layers[1][nm], m.pos * c["nkv"] * c["hd"]) for nm in ("kc", "vc")])
+        m.free()
+    for a, b in zip(*res):
+        assert np.array_equal(bits(a), bits(b))
+
+
 def test_bf16_chunk_as_halves_stays_within_the_bf16_roundings(dev):
     """The bf16 prefill through forward_parts: the halves' products are other launches (other token counts, so the
     split over the columns may fall otherwise), not other numbers -- the first layer's caches within a few bf16 roundings of the whole
