@@ -392,24 +392,26 @@ __global__ __launch_bounds__(256, 2) void attn_scores_quad_kernel(const float* _
   }
 }
 
-constexpr int kStepHeads = 8, kStepPositions = 128;      // a workgroup of one token's score kernel: query heads, positions
-// One token's qk_rope and scores in one launch.  A workgroup takes PB positions of a KV head for all (up to GH) of its query heads:
-// the keys, which are most of what the launch reads, come from memory once and lie in registers while one query head after another
-// is multiplied with them (a workgroup a query head read them once a head, and on different dies: 14.3 us at 4,117 positions of the
-// Qwen3-4B shape, 17 MB of keys).  Waves 0 .. GH - 1 norm and turn the query heads, the next one the KV head's key where the
-// workgroup's positions hold the token's own; that workgroup takes the key from LDS and writes key and value into the caches, for
-// the launch with the values.  q and k are left as they came.
+constexpr int kStepHeads = 8, kStepPositions = 128;      // a workgroup of one token's score kernel: query heads at most, positions
+// One token's qk_rope and scores in one launch.  A workgroup takes kStepPositions positions of a KV head for GH of its query heads
+// (blockIdx.z: which; the host says how many): the keys, which are most of what the launch reads, come from memory once and lie in
+// registers while one query head after another is multiplied with them (a workgroup a query head read them once a head, and on
+// different dies: 14.3 us at 4,117 positions of the Qwen3-4B shape, 17 MB of keys; now 7.5).  Waves 0 .. GH - 1 norm and turn the
+// query heads, wave kStepHeads the KV head's key where the workgroup's positions hold the token's own; that workgroup takes the key
+// from LDS, and the group's first writes key and value into the caches, for the launch with the values.  q and k are left as they came.
+// Registers: two workgroups a CU where the width is a constant; read at run time the keys have room for heads of 256, which in 64
+// registers spilled (14 heads of 48, 501 positions: 17.4 us a call in 64, 15.1 in 128).
 template <int NJ>      // hd / 16 as a constant, or 0: read at run time (heads up to 256)
-__global__ __launch_bounds__(1024, 8) void attn_step_scores_kernel(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+__global__ __launch_bounds__(1024, NJ ? 8 : 4) void attn_step_scores_kernel(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
                                                                 const float* __restrict__ qn, const float* __restrict__ kn,
                                                                 const float* __restrict__ rope, float* __restrict__ kc, float* __restrict__ vc,
                                                                 float* __restrict__ raw, int nh, int nkv, int hd, int rd, int pos, float eps,
-                                                                int neox, float scale, int spitch) {
+                                                                int neox, float scale, int spitch, int gh) {
   constexpr int GH = kStepHeads, NU = kStepPositions / 64;
   __shared__ float qsh[GH][256], ksh[256];
   __shared__ double scs[GH + 1];
   const int kh = blockIdx.x, tid = threadIdx.x, npos = pos + 1, pbase = blockIdx.y * kStepPositions;
-  const int group = nh / nkv, kvd = nkv * hd, ko = kh * hd, h0 = kh * group + blockIdx.z * GH, heads = min(GH, group - (int)blockIdx.z * GH);
+  const int group = nh / nkv, kvd = nkv * hd, ko = kh * hd, h0 = kh * group + blockIdx.z * gh, heads = min(gh, group - (int)blockIdx.z * gh);
   constexpr int NJM = NJ ? NJ : 16;
   const int l = tid & 15, pg = tid >> 4, nj = NJ ? NJ : hd >> 4, wave = tid >> 6;
   const bool own = pos < pbase + kStepPositions;   // this workgroup's positions hold the token's own
@@ -1616,13 +1618,20 @@ hipError_t ilt_k_attn_step(const float* q, const float* k, const float* v, const
   }
   {
     const int group = nh / nkv;
-    const dim3 gs(nkv, (ctx + kStepPositions - 1) / kStepPositions, (group + kStepHeads - 1) / kStepHeads);
+    // Query heads a workgroup: the fewest that leave no more workgroups than CUs.  A workgroup takes its heads one after another,
+    // with few of them on the chip that is a chain (us a call, two launches: 14 heads of 48 on 2 KV heads, 501 positions, 8
+    // workgroups of seven 15.1, 56 of one 11.2; 32 heads of 128 on 8, 1,101 positions, 72 of four 13.3, 144 of two 12.6), and past
+    // the CUs the keys are only read again (the latter at 4,117, 264 of four 25.3, 528 of two 25.8, 1,056 of one 27.1).
+    const int blocks = (ctx + kStepPositions - 1) / kStepPositions;
+    int gh = 1;
+    while (gh < group && gh < kStepHeads && (long long)nkv * blocks * ((group + gh - 1) / gh) > 256) gh++;
+    const dim3 gs(nkv, blocks, (group + gh - 1) / gh);
     if (hd == 128)
-      hipLaunchKernelGGL(attn_step_scores_kernel<8>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax);
+      hipLaunchKernelGGL(attn_step_scores_kernel<8>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax, gh);
     else if (hd == 64)
-      hipLaunchKernelGGL(attn_step_scores_kernel<4>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax);
+      hipLaunchKernelGGL(attn_step_scores_kernel<4>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax, gh);
     else
-      hipLaunchKernelGGL(attn_step_scores_kernel<0>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax);
+      hipLaunchKernelGGL(attn_step_scores_kernel<0>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax, gh);
   }
   // past the one-launch kernel's 1,024 positions the values come in tiles while the chains run (at 1,536 positions 523
   // tok/s at the Qwen3-4B shape against 493 with the whole slice brought into LDS first, at 1,990 500 against 464);

@@ -121,6 +121,42 @@ def test_attn_step_is_qk_rope_then_attn_rows(dev, norms, nh, nkv, hd):
         hip.hip_free(b)
 
 
+# query heads a KV head: more than a workgroup takes (9 and 16: a second workgroup with the rest), a number that its share does not
+# divide (5 by 3), one; positions on and beside a block's edge
+@pytest.mark.parametrize("nh,nkv,hd,pos", [(72, 8, 32, 4095), (16, 1, 32, 384), (40, 8, 48, 1300), (40, 8, 64, 1100), (72, 8, 128, 2304), (8, 8, 80, 127)])
+def test_attn_step_shares_out_its_query_heads(dev, nh, nkv, hd, pos):
+    """One token's attention as two launches against qk_rope and attn_rows, bit for bit, however the query heads of a KV head
+    fall on the score kernel's workgroups."""
+    import ctypes as C
+    from illatio_amd import hip
+    nctx, eps = (pos + 4) // 4 * 4, 1e-6
+    rng = synth.make_rng(nh + pos)
+    f = lambda *sh: (rng.standard_normal(sh) * 1.5).astype(np.float32)
+    up = lambda a: hip.hip_upload_new(dev, a)
+    P = lambda b: C.c_uint64(b.ptr if b is not None else 0)
+    S = C.c_uint64(0)
+    table = np.zeros((nctx, hd), np.float32)
+    assert hip.lib().ilt_rope_table(C.c_int(hd), C.c_int(0), C.c_int(nctx), C.c_float(1e6), table.ctypes.data_as(C.c_void_p)) == 0
+    kc0, vc0, q, k, v = f(nctx, nkv * hd), f(nctx, nkv * hd), f(nh * hd), f(nkv * hd), f(nkv * hd)
+    rope, qn, kn, scratch, dq, dk, dv = (up(a) for a in (table, f(hd), f(hd), np.zeros(nh * nctx, np.float32), q, k, v))
+    ints = (C.c_int(nh), C.c_int(nkv), C.c_int(hd), C.c_int(hd), C.c_int(pos), C.c_float(eps), C.c_int(1))
+    res = []
+    for step in (True, False):
+        kc, vc, out = up(kc0), up(vc0), hip.hip_alloc(dev, 4 * nh * hd)
+        if step:
+            hip.call("ilt_attn_step", S, P(dq), P(dk), P(dv), P(qn), P(kn), P(rope), P(kc), P(vc), P(out), *ints, P(scratch), C.c_int(nctx))
+        else:
+            hip.call("ilt_qk_rope", S, P(dq), P(dk), P(dv), P(qn), P(kn), P(rope), P(kc), P(vc), *ints, C.c_int(1))
+            hip.call("ilt_attn_rows", S, P(dq), P(kc), P(vc), P(out), C.c_int(nh), C.c_int(nkv), C.c_int(hd), C.c_int(pos), C.c_int(1), P(None))
+        res.append([hip.hip_floats(b, n) for b, n in ((out, nh * hd), (kc, nctx * nkv * hd), (vc, nctx * nkv * hd))])
+        for b in (kc, vc, out):
+            hip.hip_free(b)
+    for a, b, what in zip(res[0], res[1], ("out", "kc", "vc")):
+        assert np.array_equal(bits(a), bits(b)), what
+    for b in (rope, qn, kn, scratch, dq, dk, dv):
+        hip.hip_free(b)
+
+
 def test_the_reference_attention_names_launch(dev):
     """attn_decode + attn_merge and attn_prefill / attn_prefill2 by the reference's names and argument lists
     (cuda-dense.lisp:341-364): the heads they leave are attn_rows' -- the CPU's float order -- and attn_merge's
