@@ -371,9 +371,11 @@ __device__ __forceinline__ void few_tile(const FewParams& p, const FewMat& m, in
   }
 }
 
-// FSET: the matrices' format, or 0 where Q4_K and Q6_K meet in a launch
+// FSET: the matrices' format, or 0 where Q4_K and Q6_K meet in a launch.  Registers: a Q6_K tile of two patches, alone or beside
+// Q4_K, spills in the 168 that three workgroups a CU leave (a mixed launch of 1024 + 512 + 512 rows x 1024 on 17 tokens 7.1 us
+// with twelve spilled, 6.3 with two workgroups; 2048 + 512 + 512 x 2560 10.2 and 9.5).
 template <int FSET, int NT, int RT, int NW>
-__global__ __launch_bounds__(64 * NW, (NW == 8 ? (NT == 1 ? 2 : 1) : RT * NT == 1 ? 4 : RT * NT == 2 && FSET != ILT_Q6_K ? 3 : 2)) void gemm_i8_few_kernel(FewParams p) {
+__global__ __launch_bounds__(64 * NW, (NW == 8 ? (NT == 1 ? 2 : 1) : RT * NT == 1 ? 4 : RT * NT == 2 && FSET != ILT_Q6_K && FSET != 0 ? 3 : 2)) void gemm_i8_few_kernel(FewParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   // the token tiles of a row tile next to one another on a die, so that its blocks come into that die's L2 once
   const int ntile = gridDim.x / p.ttiles, per = (ntile + 7) >> 3;
