@@ -710,12 +710,12 @@ int ilt_mm_q8_mma2(uint64_t stream, const int8_t* w0, const uint16_t* d0, float*
   const uint8_t* fw[3]; const uint16_t* fd[3]; float* fy[3]; const float* fb[3]; int fr[3], fm[3], nm = 0;
   for (int i = 0; i < 3; i++) {
     ILT_REQUIRE(rows[i] >= 0);
-    if (rows[i] == 0 || !ws[i]) continue;
+    if (rows[i] == 0 || !ws[i] || n == 0) continue;       // (no tokens: nothing is read or written, whatever the pointers)
     ILT_REQUIRE(ds[i] && ys[i] && ((uintptr_t)ws[i] & 15) == 0);
     fw[nm] = (const uint8_t*)ws[i]; fd[nm] = ds[i]; fy[nm] = ys[i]; fb[nm] = bs[i]; fr[nm] = rows[i]; fm[nm] = ILT_Q8_0; nm++;
   }
-  if (nm > 1 && n > 0) {
-    ILT_REQUIRE(xq && xs && ((uintptr_t)xq & 15) == 0 && cols > 0 && cols % 32 == 0);
+  if (nm > 1) {
+    ILT_REQUIRE(n > 0 && xq && xs && ((uintptr_t)xq & 15) == 0 && cols > 0 && cols % 32 == 0);
     const hipError_t e = ilt_k_gemm_i8_few(nm, fm, fw, fd, fr, fy, fb, cols, xq, xs, nullptr, n, acc, S(stream));
     if (e != hipErrorNotSupported) return (int)e;
   }

@@ -32,6 +32,17 @@ def test_error_string_and_unknown_kernel_need_no_gpu():
     assert hip.lib().ilt_error_string(1)          # some text for an invalid-value error
 
 
+@pytest.mark.parametrize("n,cols,code", [(0, 64, 0), (0, 48, 1), (-1, 64, 1), (3, 64, 1)])
+def test_products_of_no_tokens_look_at_no_pointer(n, cols, code):
+    """ilt_mm_q8_mma2 on no tokens is done whatever stands where the results and scales would (what it always refused stays
+    refused: columns that are no whole number of blocks, a negative number of tokens, no results for three)."""
+    from illatio_amd import hip
+    w = C.c_uint64(0x1002)                            # on no 16-byte boundary: not read
+    none, f = C.c_uint64(0), hip.lib().ilt_mm_q8_mma2
+    mat = [w, none, none, none, C.c_int(32)]
+    assert f(none, *mat, *mat, none, none, none, none, C.c_int(0), none, none, C.c_int(cols), C.c_int(n), C.c_int(0)) == code
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     from illatio_amd import hip
     monkeypatch.setattr(hip, "_lib", None)
