@@ -197,6 +197,22 @@ template <> struct RegW<ILT_Q2_K> {
   }
 };
 
+// The same for a matrix on a two-byte boundary (an expert's slot may lie on one; buffer loads of dwords want four): the blocks by
+// loads through pointers, as IQ2_XXS's, a row past the matrix's its last one.
+struct RegWQ2KHalf : RegW<ILT_Q2_K> {
+  struct At { u32 a[4]; };
+  static __device__ __forceinline__ At place(u32 row_bytes, int lane, int row0, int rows) {
+    At o;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      o.a[i] = (u32)min(row0 + 8 * i + (lane >> 3), rows - 1) * row_bytes + min(16 * (u32)((lane & 7) ^ ((lane >> 4) & 3) ^ (i & 1 ? 4 : 0)), 68u);
+    return o;
+  }
+  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t, const u8* w, const At& at, u32, u32, u32 block, u8* dst) {
+    ilt_g2lds16(w + (size_t)block + at.a[i], dst + 1024 * i);
+  }
+};
+
 // IQ2_XXS: a block's eight groups of 32 weights add (float(sumi) * (0.5 + scale)) alternately to two sums, and the block's term
 // is (d yd) times the two together (iquant.lisp:161-215).  Every partial sum is a multiple of 1/2 whose double stays below 2^24
 // (test_oracle.py asserts it from the codebook), so nothing rounds before the two meet, and their sum is float(isum) / 2 for
@@ -286,9 +302,8 @@ template <int FMT, int NP, int WR, int WT> using RegSmemOf = RegSmem<32 * NP * W
 
 // Rows r0 .. of one matrix (p.rows of them, results to p.y) x tokens tok0 .. tok0 + ntok - 1: WR x WT waves of 32 rows x 32 NP
 // tokens.  NP 1: nothing to share out between two halves, so the tokens and the rows' blocks are in two buffers and a block ahead.
-template <int FMT, int NP, int WR, int WT>
+template <int FMT, int NP, int WR, int WT, class F = RegW<FMT>>
 __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0, long tok0, int ntok, unsigned char* smem) {
-  using F = RegW<FMT>;
   constexpr int TN = 32 * NP * WT, THREADS = 64 * WR * WT;
   constexpr bool DEEP = NP == 1;
   constexpr int NI = DEEP ? 8 / WR : TN / (8 * WR * WT);       // direct loads of a wave a super-block's half (NP 1: all) of the tokens (four tokens each)
@@ -602,6 +617,9 @@ __global__ __launch_bounds__(256, 2) void gemm_i8r_group_kernel(BfParams p) {
   p.rows = rows;
   if (rt >= nr) { rt -= nr; w += p.up_delta; p.y = p.my[1]; }
   ntok = __builtin_amdgcn_readfirstlane(ntok);
+  if constexpr (FMT == ILT_Q2_K) {
+    if ((u32)(uintptr_t)ilt_uniform_ptr(w) & 3) { reg_tile<FMT, 4, 4, 1, RegWQ2KHalf>(p, w, rt * 128, tok0, ntok, smem); return; }
+  }
   if (ntok <= 32) reg_tile<FMT, 1, 4, 1>(p, w, rt * 128, tok0, ntok, smem);
   else if (ntok <= 64) reg_tile<FMT, 2, 4, 1>(p, w, rt * 128, tok0, ntok, smem);
   else reg_tile<FMT, 4, 4, 1>(p, w, rt * 128, tok0, ntok, smem);
@@ -674,13 +692,13 @@ hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws
 }
 
 // The grouped product of the experts' IQ2_XXS and Q2_K matrices: expert z's rows counts[z] from bases[z] on; y2 set: a second
-// matrix at add2 as well, its results there.  hipErrorNotSupported, and nothing launched, where the shapes are not this kernel's.
+// matrix at add2 as well, its results there.  Slots on two-byte boundaries.  hipErrorNotSupported, and nothing launched, where the shapes are not this kernel's.
 hipError_t ilt_k_gemm_i8_reg_id(int fmt, const uint64_t* ptrs, long long add, long long add2, const uint32_t* counts, const uint32_t* bases, int ne,
                                 int rows, int cols, const int8_t* xq, const float* xd, const int* bsums, long long total_rows, float* y, float* y2,
                                 hipStream_t st) {
   const long long row_bytes = (long long)(cols / 256) * block_bytes_of(fmt), delta = y2 ? add2 - add : 0;
   if ((fmt != ILT_IQ2_XXS && fmt != ILT_Q2_K) || ne < 1 || ne > 256 || rows < 1 || rows >= (1 << 21) || cols < 256 || cols % 256 || rows * row_bytes >= 0x7FFFFFFFLL ||
-      cols >= (1 << 22) || total_rows < 1 || total_rows >= 0x7FFFFFFFLL || delta < 0 || delta > 0x7FFFFFFFLL || (fmt == ILT_Q2_K && (add & 3)))
+      cols >= (1 << 22) || total_rows < 1 || total_rows >= 0x7FFFFFFFLL || delta < 0 || delta > 0x7FFFFFFFLL)
     return hipErrorNotSupported;
   BfParams p = {};
   p.ptrs = ptrs; p.add = add; p.up_delta = (unsigned)delta; p.counts = counts; p.bases = bases; p.ne = ne;

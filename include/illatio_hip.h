@@ -433,7 +433,7 @@ int ilt_swiglu_quant_q8k(uint64_t stream, const float* gate, const float* up, in
    mm_k (kquant.cu:223, 458-466 mm_k / mm_q4k_mma / mm_q6k_mma): type 0 Q4_K, 2 Q6_K;
      activations from ilt_quant_q8k.
    d4_mm_id_* (ds4f_mm.cu:256-257): the grouped expert product.  Expert z's matrix is at
-     ptrs[z] + add; it multiplies rows bases[z] .. bases[z]+counts[z]-1 of the gathered,
+     ptrs[z] + add (an even address; a multiple of 4 is faster for Q2_K); it multiplies rows bases[z] .. bases[z]+counts[z]-1 of the gathered,
      Q8_K-quantized activations (xq/xd/bsums, ncols apart) into the same rows of y (nrows
      apart).  ne experts (at most 256), total_rows = the sum of counts. */
 int ilt_mm_q8(uint64_t stream, const int8_t* wq, const uint16_t* wd, const int8_t* xq, const float* xs, float* y,

@@ -102,3 +102,35 @@ def test_groups_bit_for_bit(dev, qtype, rows, cols):
         assert np.array_equal(bits(got[at]), bits(want)), (z, np.argwhere(bits(got[at]) != bits(want))[:5])
     for b in (wb, xb, y, ptrs, cb, bb, xq, xd, xs):
         hip.hip_free(b)
+
+
+# experts' matrices on two-byte boundaries: by the slot's address, by the offset into it, and both (together a multiple of four)
+@pytest.mark.parametrize("rows,cols", [(128, 256), (161, 1280)])
+@pytest.mark.parametrize("at,add", [(2, 0), (0, 2), (2, 2), (6, 8)])
+def test_groups_of_q2_k_on_even_addresses_bit_for_bit(dev, rows, cols, at, add):
+    from illatio_amd import ds4f, hip
+    rng = synth.make_rng(rows + cols + at + add)
+    counts = np.array([1, 0, 33, 64, 65, 129], np.uint32)
+    ne, total = len(counts), int(counts.sum())
+    bases = (np.cumsum(counts) - counts).astype(np.uint32)
+    rb = synth.row_bytes(synth.Q2_K, cols)
+    w = synth.weights(synth.Q2_K, ne * rows, cols, rng).reshape(ne, rows, rb)
+    x = synth.activations((total, cols), rng)
+    step = rows * rb + 16                             # (a slot ends 16 bytes before the next one: a multiple of four)
+    host = np.zeros(at + add + ne * step, np.uint8)
+    for z in range(ne):
+        host[at + add + z * step:][:rows * rb] = w[z].ravel()
+    wb, xb, y = hip.hip_upload_new(dev, host), hip.hip_upload_new(dev, x), hip.hip_alloc(dev, 4 * total * rows)
+    ptrs = hip.hip_upload_new(dev, np.array([wb.ptr + at + z * step for z in range(ne)], np.uint64))
+    cb, bb = hip.hip_upload_new(dev, counts), hip.hip_upload_new(dev, bases)
+    xq, xd, xs = ds4f._q8k(dev, xb, total * cols)
+    hip.launch(dev, "d4_mm_id_q2_k", (1, 1, ne), 128, [cols, rows, rb, cols, rows, hip.I64(add), ptrs, cb, bb, xq, y, xd, xs, hip.I64(total)])
+    got = hip.hip_floats(y, total * rows).reshape(total, rows)
+    for z in range(ne):
+        if counts[z] == 0:
+            continue
+        part = slice(int(bases[z]), int(bases[z] + counts[z]))
+        want = orc.matmul(synth.Q2_K, w[z], rows, cols, x[part], nthreads=8).reshape(-1, rows)
+        assert np.array_equal(bits(got[part]), bits(want)), (z, np.argwhere(bits(got[part]) != bits(want))[:5])
+    for b in (wb, xb, y, ptrs, cb, bb, xq, xd, xs):
+        hip.hip_free(b)
