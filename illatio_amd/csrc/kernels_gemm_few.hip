@@ -400,9 +400,18 @@ hipError_t few_launch(FewParams& p, hipStream_t st) {
   constexpr int terms = FSET == ILT_Q6_K ? 1 : 2, scales = FSET == ILT_Q8_0 ? 2 : 1, ucols = FSET == ILT_Q8_0 ? 64 : 256;
   constexpr int per = terms * 1024 * RT * NT + scales * 64 * NT;
   const int units = (p.cols + ucols - 1) / ucols;
-  const int most = (76 * 1024) / per / (2 * NW) * (2 * NW);      // two workgroups a CU at least
+  constexpr int room = 76 * 1024;                                // two workgroups a CU at least
+  const int most = room / per / (2 * NW) * (2 * NW);
   p.uround = units <= most ? units : most;
-  static_assert((76 * 1024) / per >= 2 * NW, "a round is whole turns of the four waves' two register sets");
+  static bool attr_set[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  if (!attr_set[dev]) {            // more dynamic LDS than the default 64 KB (Q6_K on 9,728 columns: 68): asked for once per device
+    const hipError_t e = hipFuncSetAttribute((const void*)gemm_i8_few_kernel<FSET, NT, RT, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, room);
+    if (e != hipSuccess) return e;
+    attr_set[dev] = true;
+  }
+  static_assert(room / per >= 2 * NW, "a round is whole turns of the four waves' two register sets");
   hipLaunchKernelGGL((gemm_i8_few_kernel<FSET, NT, RT, NW>), dim3(tiles * p.ttiles), dim3(64 * NW), (size_t)p.uround * per, st, p);
   return hipGetLastError();
 }

@@ -1,0 +1,81 @@
+"""Every launch with more dynamic LDS than the 64 KB that a kernel gets by itself asks for it first (hipFuncSetAttribute).  The
+library's host code runs here on a stand-in for the HIP runtime that notes what it is asked for and launches nothing (no GPU)."""
+import os
+import subprocess
+import sys
+
+RUNTIME = r"""
+#include <stdio.h>
+#include <string.h>
+typedef struct { unsigned x, y, z; } dim3_;
+static struct { const void* f; const char* name; long asked; } k[2048];
+static int nk;
+static __thread struct { dim3_ g, b; size_t lds; void* st; } cfg;
+void** __hipRegisterFatBinary(const void* d) { static void* h; return &h; }
+void __hipUnregisterFatBinary(void** h) {}
+void __hipRegisterVar(void** m, void* v, char* n, char* d, int e, size_t s, int c, int g) {}
+void __hipRegisterFunction(void** m, const void* f, char* n, const char* d, unsigned t, void* a, void* b, void* c, void* e, int* w) {
+  if (nk < 2048) { k[nk].f = f; k[nk].name = d; k[nk].asked = 65536; nk++; }
+}
+int __hipPushCallConfiguration(dim3_ g, dim3_ b, size_t lds, void* st) { cfg.g = g; cfg.b = b; cfg.lds = lds; cfg.st = st; return 0; }
+int __hipPopCallConfiguration(dim3_* g, dim3_* b, size_t* lds, void** st) { *g = cfg.g; *b = cfg.b; *lds = cfg.lds; *st = cfg.st; return 0; }
+int hipGetDevice(int* d) { *d = 0; return 0; }
+int hipGetLastError(void) { return 0; }
+int hipFuncSetAttribute(const void* f, int attr, int v) {
+  for (int i = 0; i < nk; i++) if (k[i].f == f && attr == 8 && v > k[i].asked) k[i].asked = v;
+  return 0;
+}
+int hipLaunchKernel(const void* f, dim3_ g, dim3_ b, void** args, size_t lds, void* st) {
+  for (int i = 0; i < nk; i++) if (k[i].f == f) printf("%s %s %zu of %ld\n", (long)lds > k[i].asked ? "UNASKED" : "ok", k[i].name, lds, k[i].asked);
+  return 0;
+}
+"""
+
+CALLS = r"""
+import ctypes as C, os, sys
+C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+L = C.CDLL(sys.argv[2])
+P, Z, I, S = C.c_uint64(1 << 40), C.c_uint64(0), C.c_int, C.c_uint64(0)
+def ok(e, *what):
+    assert e == 0, (e,) + what
+for cols in (256, 2560, 4096, 9728, 16384):
+    for rows in (32, 2560, 19456):
+        for n in (2, 16, 17, 40, 130, 512, 2048):
+            for t in (0, 2):
+                ok(L.ilt_mm_k(S, I(t), P, P, P, P, P, Z, I(rows), I(cols), I(n), I(0)), "mm_k", t, rows, cols, n)
+            ok(L.ilt_mm_k_n(S, I(2), P, P, Z, I(rows), P, P, Z, I(rows), Z, Z, Z, I(0), P, P, P, I(cols), I(n), I(0)), "mm_k_n", rows, cols, n)
+            ok(L.ilt_mm_q8(S, P, P, P, P, P, Z, I(rows), I(cols), I(n), I(0)), "mm_q8", rows, cols, n)
+            ok(L.ilt_mm_q8_mma2(S, P, P, P, Z, I(rows), P, P, P, Z, I(rows), Z, Z, Z, Z, I(0), P, P, I(cols), I(n), I(0)), "mm_q8_mma2", rows, cols, n)
+            ok(L.ilt_cvt_bf16(S, P, P, C.c_int64(n * cols)), "cvt")
+            for t in (12, 14):
+                ok(L.ilt_mm_k_bf16(S, I(t), P, P, P, Z, I(rows), I(cols), I(n), I(0)), "mm_k_bf16", t, rows, cols, n)
+            if rows % 256 == 0:
+                ok(L.ilt_mm_bf16(S, P, P, P, Z, I(rows), I(cols), I(n), I(0)), "mm_bf16", rows, cols, n)
+for total in (8, 300, 24576):
+    for d, ff in ((512, 256), (4096, 2048)):
+        grb, drb = d // 256 * 66, ff // 256 * 84
+        add, T = C.c_int64, C.c_int64(total)
+        ok(L.ilt_d4_mm_id2_iq2_xxs(S, I(d), I(ff), I(grb), add(0), add(ff * grb), P, P, P, I(64), T, P, P, P, P), "id2")
+        ok(L.ilt_d4_mm_id_q2_k(S, I(ff), I(d), I(drb), add(2 * ff * grb), P, P, P, I(64), T, P, P, P, P), "id")
+        ok(L.ilt_d4_mm_id_bf16(S, I(10), I(ff), I(d), I(drb), add(2 * ff * grb), P, P, P, I(64), T, P, Z, P), "id_bf16")
+        ok(L.ilt_d4_mm_id_glu_bf16(S, I(16), I(d), I(ff), I(grb), add(0), add(ff * grb), P, P, P, I(64), T, P, P, C.c_float(0), P, P), "id_glu_bf16")
+for nh, nkv, hd in ((32, 8, 128), (14, 2, 64), (32, 8, 96)):
+    for pos in (0, 500, 1000, 1500, 4000, 8000):
+        ok(L.ilt_attn_step(S, P, P, P, Z, Z, P, P, P, P, I(nh), I(nkv), I(hd), I(hd), I(pos), C.c_float(1e-6), I(1), P, I(8192)), "attn_step", hd, pos)
+        for n in (1, 33, 130):
+            for scratch in (P, Z):
+                ok(L.ilt_attn_rows(S, P, P, P, P, I(nh), I(nkv), I(hd), I(pos), I(n), scratch), "attn_rows", hd, pos, n)
+"""
+
+
+def test_no_launch_takes_more_lds_than_it_asked_for(tmp_path):
+    from illatio_amd import hip
+    (tmp_path / "runtime.c").write_text(RUNTIME)
+    so = str(tmp_path / "runtime.so")
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-w", "-o", so, str(tmp_path / "runtime.c")])
+    r = subprocess.run([sys.executable, "-c", CALLS, so, hip.LIB_PATH], env={**os.environ, "ILT_ATTN_SPLIT": "0"}, capture_output=True, text=True)
+    lines = r.stdout.splitlines()
+    assert r.returncode == 0, (r.stderr[-2000:], lines[-3:])
+    assert len(lines) > 500 and sum("gemm_i8_few" in x for x in lines) > 50
+    assert any(int(x.split()[-3]) > 65536 for x in lines)
+    assert not sorted({x for x in lines if x.startswith("UNASKED")})
