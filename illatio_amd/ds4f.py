@@ -322,15 +322,23 @@ def ffn_small(dev, pool, sh, logits, norm2, n, ne, nu, scale, clamp, bias=None, 
         return _ffn_small_counts(dev, pool, sh, logits, norm2, n, ne, nu, scale, clamp, bias)
     f = hip.lib().ilt_d4_ffn_small_workspace
     f.restype = C.c_uint64
-    moe, ws = hip.hip_alloc(dev, 4 * n * pool.d, zero=False), pool.lend(int(f(C.c_int(n), C.c_int(nu), C.c_int(pool.d), C.c_int(pool.ff))))
     wt = step_weights(pool, sh)
+    ws, moe = pool.lend(int(f(C.c_int(n), C.c_int(nu), C.c_int(pool.d), C.c_int(pool.ff)))), None
     try:
+        moe = hip.hip_alloc(dev, 4 * n * pool.d, zero=False)
         hip.call("ilt_d4_ffn_small", C.c_uint64(dev.stream), C.c_uint64(ws.ptr), C.c_uint64(ws.bytes), C.c_int(n), C.c_int(ne), C.c_int(nu),
                  C.c_int(pool.d), C.c_int(pool.ff), C.c_float(scale), C.c_float(clamp), C.byref(wt), C.c_uint64(logits.ptr),
                  C.c_uint64(bias.ptr if bias is not None else 0), C.c_uint64(norm2.ptr), C.c_uint64(moe.ptr))
         hip.hip_sync(dev)
-    finally:
-        pool.give_back(ws)
+    except BaseException:
+        try:
+            hip.hip_sync(dev)                          # launches queued before the failure use both
+        except hip.HipError:
+            pass                                       # (the first error is the one to report)
+        hip.hip_free(ws)
+        hip.hip_free(moe)
+        raise
+    pool.give_back(ws)
     return moe
 
 
