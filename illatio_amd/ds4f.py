@@ -76,8 +76,10 @@ class ExpertPool:
         hip.hip_sync(self.dev)
         hip.hip_free(self.pool)
         hip.hip_free(self.ptrs)
-        while self._spare:
-            hip.hip_free(self._spare.pop())
+        with self._lock:
+            spare, self._spare = self._spare, []
+        for b in spare:
+            hip.hip_free(b)
         if self.host_buf:
             hip.hip_host_free(self.host_buf)
             self.host_buf = 0

@@ -1,5 +1,5 @@
 """The host side of a short pass through a MoE layer on a library that notes its calls (no GPU): what happens to its buffers when
-a call fails."""
+a call fails, and how the pool lets its workspaces go."""
 import ctypes as C
 import threading
 
@@ -84,3 +84,16 @@ def test_a_failed_allocation_leaves_no_buffer(setting):
     with pytest.raises(hip.HipError):
         call()
     assert lib.held == {b.ptr for b in pool._spare}
+
+
+def test_free_takes_the_pools_lock(setting):
+    lib, pool, call = setting()
+    call()
+    taken = []
+
+    class Lock:
+        def __enter__(self): taken.append(len(pool._spare))
+        def __exit__(self, *a): pass
+    pool._lock = Lock()
+    pool.free()
+    assert taken == [1] and not pool._spare
