@@ -115,7 +115,7 @@ __device__ __forceinline__ int ubyte(int v, int i) { return (u32)(v << (24 - 8 *
 // One unit's float terms of 16 RT rows x 16 NT tokens: t[k][rp][np], k < TERMS; yd: the activation scales of the unit,
 // tokens 4q .. 4q+3 of each patch.  The expressions are the CPU kernels' (kquant.lisp:180-236, tensor.lisp:329-336).
 template <int NT, int RT>
-__device__ __forceinline__ void few_unit(const FewW<ILT_Q4_K> (&w)[RT], FewX<ILT_Q4_K, NT>& x, const float* yd, int q, int, v4f (&t)[2][RT][NT]) {
+__device__ __forceinline__ void few_unit(const FewW<ILT_Q4_K> (&w)[RT], FewX<ILT_Q4_K, NT>& x, const float* yd, int q, v4f (&t)[2][RT][NT]) {
   v4i isum[RT][NT];
 #pragma unroll
   for (int rp = 0; rp < RT; rp++)
@@ -181,7 +181,7 @@ __device__ __forceinline__ void few_unit(const FewW<ILT_Q4_K> (&w)[RT], FewX<ILT
 }
 
 template <int NT, int RT>
-__device__ __forceinline__ void few_unit(const FewW<ILT_Q6_K> (&w)[RT], FewX<ILT_Q6_K, NT>& x, const float* yd, int q, int, v4f (&t)[1][RT][NT]) {
+__device__ __forceinline__ void few_unit(const FewW<ILT_Q6_K> (&w)[RT], FewX<ILT_Q6_K, NT>& x, const float* yd, int q, v4f (&t)[1][RT][NT]) {
   v4i isum[RT][NT];
   // -32 * sum of scale * (sum of 16 quants): the quants' offset
 #pragma unroll
@@ -252,8 +252,7 @@ __device__ __forceinline__ void few_unit(const FewW<ILT_Q6_K> (&w)[RT], FewX<ILT
 }
 
 template <int NT, int RT>
-__device__ __forceinline__ void few_unit(const FewW<ILT_Q8_0> (&w)[RT], FewX<ILT_Q8_0, NT>& x, const float* yd, int q, int blocks, v4f (&t)[2][RT][NT]) {
-  (void)blocks;
+__device__ __forceinline__ void few_unit(const FewW<ILT_Q8_0> (&w)[RT], FewX<ILT_Q8_0, NT>& x, const float* yd, int q, v4f (&t)[2][RT][NT]) {
 #pragma unroll
   for (int np = 0; np < NT; np++) deal(x.x[np][0]);
 #pragma unroll
@@ -322,7 +321,7 @@ __device__ __forceinline__ void few_tile(const FewParams& p, const FewMat& m, in
     __syncthreads();
     auto unit = [&](const FewW<FMT> (&w)[RT], FewX<FMT, NT>& x, int u) {
       v4f t[F::TERMS][RT][NT];
-      few_unit<NT, RT>(w, x, xls + (u - u0) * F::SCALES * TW, q, 0, t);
+      few_unit<NT, RT>(w, x, xls + (u - u0) * F::SCALES * TW, q, t);
 #pragma unroll
       for (int k = 0; k < F::TERMS; k++)
 #pragma unroll
@@ -428,9 +427,12 @@ hipError_t few_dispatch(FewParams& p, int forced, hipStream_t st) {
   long tiles = 0;
   for (int i = 0; i < p.nmat; i++) tiles += (p.mat[i].rows + 15) / 16;
   tiles *= p.ttiles;
-  const bool wide = tiles > (FSET == ILT_Q8_0 || nt == 1 ? 600 : 256), deep = tiles <= 256 && p.cols >= (FSET == ILT_Q8_0 ? 2048 : nt == 2 ? 8192 : 1 << 30);
+  const bool wide = tiles > (FSET == ILT_Q8_0 || nt == 1 ? 600 : 256), deep = tiles <= 256 && p.cols >= (FSET == ILT_Q8_0 ? 2048 : 8192);
   const int v = forced > 1 ? forced : wide ? 2 : deep ? 8 : 4;
-  if (nt == 1) return v == 2 ? few_launch<FSET, 1, 2, 4>(p, st) : v == 8 ? few_launch<FSET, 1, 1, 8>(p, st) : few_launch<FSET, 1, 1, 4>(p, st);
+  if (nt == 1) {
+    if constexpr (FSET == ILT_Q8_0) { if (v == 8) return few_launch<FSET, 1, 1, 8>(p, st); }      // (K-quants on up to 16 tokens: four waves)
+    return v == 2 ? few_launch<FSET, 1, 2, 4>(p, st) : few_launch<FSET, 1, 1, 4>(p, st);
+  }
   return v == 2 ? few_launch<FSET, 2, 2, 4>(p, st) : v == 8 ? few_launch<FSET, 2, 1, 8>(p, st) : few_launch<FSET, 2, 1, 4>(p, st);
 }
 
