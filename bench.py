@@ -625,6 +625,19 @@ def workload_c4(args, dev):
                       "launch_mode": args.mode}, "roofline": roof, "cpu": cpu}
 
 
+def chunk_work(kernel, a, rows):
+    """The operations of one launch of a routed chunk of ROWS (token, slot) rows, from its name and arguments."""
+    if kernel == "d4_mm_id_bf16":
+        return 2.0 * rows * a[1] * a[2]
+    if kernel == "d4_mm_id_glu_bf16":                # gate and up
+        return 2 * 2.0 * rows * a[1] * a[2]
+    if kernel == "d4_mm_id2_iq2_xxs":                # gate and up
+        return 2 * 2.0 * rows * a[0] * a[1]
+    if kernel == "d4_mm_id_q2_k":
+        return 2.0 * rows * a[0] * a[1]
+    return 0
+
+
 def workload_c5(args, dev):
     from illatio_amd import ds4f, hip, synth
     rng = synth.make_rng(55)
@@ -646,16 +659,7 @@ def workload_c5(args, dev):
         ws.reset()
         fn(dev, pool, lb, nb, sb, n, ne, nu, 1.5, 0.0, ws=ws)
 
-    def work_of(kernel, a):
-        if kernel == "d4_mm_id_bf16":
-            return 2.0 * rows * a[1] * a[2]
-        if kernel == "d4_mm_id_glu_bf16":            # gate and up
-            return 2 * 2.0 * rows * a[1] * a[2]
-        if kernel in ("d4_mm_id_iq2_xxs", "d4_mm_id_q2_k"):
-            return 2.0 * rows * a[0] * a[1]
-        return 0
-
-    ms, dev_ms, per = tm.run(step, args.steps, args.warmup, probe_steps=2, work_of=work_of)
+    ms, dev_ms, per = tm.run(step, args.steps, args.warmup, probe_steps=2, work_of=lambda kernel, a: chunk_work(kernel, a, rows))
     # the grouped products: gate + up (IQ2_XXS; one launch with the gated activation on the bf16 path) and down (Q2_K)
     mm = [k for k in per if per[k][1]]
     allmm = [sum(per[k][0] for k in mm), sum(per[k][1] for k in mm), sum(per[k][2] for k in mm)]
