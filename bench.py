@@ -453,8 +453,9 @@ def workload_c3(args, dev):
         def step(_):
             tm.launch("quant", 0, lambda: dense.quantize_act(dev, xf, act))
             tm.launch("mm", flops, lambda: dense.cmat_mul(dev, m, act, y, n=T))
-        names = {"mm": "gemm_i8p_kernel (scale * quant as two int8 planes in LDS, v_mfma_i32_32x32x32_i8, one float combine per super-block: "
-                       "bit-exact with the CPU path)"}
+        names = {"mm": "gemm_q8_kernel (Q8_0 blocks, v_mfma_i32_16x16x32_i8 a block: bit-exact with the CPU path)" if qt == synth.Q8_0 else
+                       "gemm_i8r_kernel (scale * quant as two int8 planes made in the operand registers, v_mfma_i32_32x32x32_i8, one float "
+                       "combine per super-block: bit-exact with the CPU path)"}
     ms, dev_ms, per = tm.run(step, args.steps, args.warmup)
     roof = roofline_of({k: v for k, v in per.items() if k == "mm"}, "mfma", MFMA_PEAK_TFLOPS[args.path], "TFLOP/s" if bf16_path else "TOP/s", names)
     roof["unit"] = "TFLOP/s"
@@ -665,7 +666,8 @@ def workload_c5(args, dev):
     allmm = [sum(per[k][0] for k in mm), sum(per[k][1] for k in mm), sum(per[k][2] for k in mm)]
     roof = roofline_of({"mm_id": allmm}, "mfma", MFMA_PEAK_TFLOPS[args.path], "TFLOP/s",
                        {"mm_id": "gemm_bf16_regb_kernel<16, true> (d4_mm_id_glu_bf16: gate, up, activation) + <10, false> (d4_mm_id_bf16: down)" if args.path == "bf16"
-                        else "gemm_i8p_kernel<16> (d4_mm_id_iq2_xxs x2) + <10> (d4_mm_id_q2_k): scale * quant as int8 planes, grouped, bit-exact with the CPU path"})
+                        else "gemm_i8r_group_kernel<16> (d4_mm_id2_iq2_xxs: gate and up) + <10> (d4_mm_id_q2_k: down): operands made in registers, "
+                             "v_mfma_i32_32x32x32_i8, bit-exact with the CPU path"})
     roof["launch_us_all"] = {k: round(v[0] / v[2] * 1e3, 2) for k, v in per.items()}
     if args.path == "bf16" and n == 4096:
         t5 = TRAFFIC.get("c5", {})

@@ -22,3 +22,12 @@ def test_a_chunks_launches_add_up_to_its_products(monkeypatch, path):
     x = buf(dev, 4 * n * d)
     routed(dev, pool, x, x, x, n, ne, nu, 1.5, 0.0, ws=types.SimpleNamespace(alloc=buf))
     assert sum(bench.chunk_work(kernel, args, n * nu) for kernel, args in seen) == 2.0 * n * nu * 3 * ff * d
+
+
+def test_every_kernel_it_names_is_in_the_sources():
+    src = os.path.join(ROOT, "illatio_amd", "csrc")
+    text = "".join(open(os.path.join(src, f)).read() for f in sorted(os.listdir(src)) if f.endswith(".hip"))
+    here = set(re.findall(r"__global__[^;{]*?\b([a-z0-9_]+_kernel)\(", text))
+    named = set(re.findall(r"\b([a-z0-9_]+_kernel)\b", open(os.path.join(ROOT, "bench.py")).read()))
+    assert len(here) > 30 and len(named) > 5
+    assert not named - here
