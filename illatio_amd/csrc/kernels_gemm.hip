@@ -431,9 +431,10 @@ hipError_t ilt_k_gemm_i8(int fmt, const uint8_t* w, const uint16_t* wd, long lon
   if (ldy == 0) ldy = rows;
   if (ldy < rows) return hipErrorInvalidValue;
   // The kernels of few tokens (Q8_0, Q4_K, Q6_K) and of operands in registers (all but Q8_0) have rules of their own; Q2_K and
-  // IQ2_XXS on up to 16 tokens stay here, where a tile is 64 tokens and not 128; Q8_0 with enough tokens and rows to fill
-  // 128 x 128 tiles takes a pipelined kernel, the same bits.  ILT_I8_PLANES (tests): "0" neither the registers' nor the
-  // pipelined one, "1" these whenever the format allows.
+  // IQ2_XXS on up to 16 tokens stay here, where a tile is 64 tokens and not 128; Q8_0 past the few tokens takes its own kernel
+  // (kernels_gemm_q8.hip) in the tile that it picks, all of them the same bits.  What is left for the kernel here: those few
+  // rows of Q2_K and IQ2_XXS, and shapes and addresses that the others refuse.  ILT_I8_PLANES (tests): "0" the kernel here
+  // always, "1" the kernels of many tokens whenever the format allows.
   const char* force = getenv("ILT_I8_PLANES");
   const int forced = force ? atoi(force) : -1;
   {

@@ -444,7 +444,8 @@ hipError_t few_dispatch(FewParams& p, int forced, hipStream_t st) {
 // lies at the number of 32 x 32 tiles that take as long (Q4_K: 2560 x 4096 on 192 tokens, 480 tiles: 25 against 33 us, on 256,
 // 640: 38 against 33; 19456 x 2560 on 24, 608: 22 against 32, on 48, 1,216: 37 against 33; Q6_K: 2560 x 9728 on 192, 480: 63
 // against 75, on 256: 91 against 75; 9728 x 2560 on 24, 304: 21 against 23, on 48: 32 against 23).  With up to 32 tokens the
-// other kernel does four times the work for nothing, with up to 16 eight times.  Q8_0 against its own kernel (kernels_gemm_q8.hip),
+// other kernel does four times the work for nothing, with up to 16 eight times.  (These
+// four shapes are what the lines were drawn from; a mixed launch's lies between the two formats'.)  Q8_0 against its own kernel (kernels_gemm_q8.hip),
 // whose waves make a tile's terms and sums in registers: up to 16 tokens here, unless the tiles of 16 rows fill the chip (896 x 4864
 // on 16 tokens 12.7 us against 16.1, on 24 17.1 against 16.1; 4096 x 2048 on 16, 256 tiles: 8.1 against 8.3; 9728 x 896, 608:
 // 7.7 against 5.8); where its smallest tile does not go (cols no multiple of 128) from 640 tiles of 32 x 32 and 96 tokens on.
@@ -459,7 +460,7 @@ hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws
   p.nmat = nmat; p.cols = cols; p.ntok = ntok; p.acc = acc; p.xq = xq; p.xs = xs; p.bsums = bsums;
   int fset = fmts[0];
   long long tiles32 = 0;
-  bool small = false;                       // a matrix the pipelined kernels do not take
+  bool small = false;                       // a matrix of less than a tile of the registers' kernel
   for (int i = 0; i < nmat; i++) {
     const int fm = fmts[i];
     if (fm != ILT_Q4_K && fm != ILT_Q6_K && fm != ILT_Q8_0) return hipErrorNotSupported;

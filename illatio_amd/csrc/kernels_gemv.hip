@@ -530,9 +530,6 @@ __device__ __forceinline__ void stage_q8k_from_f32(const float* __restrict__ x, 
 
 // Q8_0 (quantize-q8!, tensor.lisp:245-262): 8 lanes a block of 32.  XSUM: each block's sum of
 // quants as well.  NW, NSCALE, H as for the Q8_K staging.
-// NP passes of the workgroup's first 256 threads over the blocks' float4s from c0 on: every pass's loads are asked for
-// before the first is quantized (a pass a trip to memory otherwise), without a branch around any of them (past the
-// end: the last float4 again; nothing is stored for it).
 // One float4 of a block, number C of N8, weighted already: its block's scale by the block's eight lanes, and its four quants.
 __device__ __forceinline__ void q8_store(const float4& w, int c, int n8, int f16_scale, i8* lxq, float* lxs, int* xsum) {
   float amax = fmaxf(fmaxf(fabsf(w.x), fabsf(w.y)), fmaxf(fabsf(w.z), fabsf(w.w)));
@@ -554,6 +551,9 @@ __device__ __forceinline__ void q8_store(const float4& w, int c, int n8, int f16
 __device__ __forceinline__ float4 norm_weighted(const float4& x, float nscale, const float4& n) {
   return make_float4((x.x * nscale) * n.x, (x.y * nscale) * n.y, (x.z * nscale) * n.z, (x.w * nscale) * n.w);
 }
+// NP passes of the workgroup's first 256 threads over the blocks' float4s from c0 on: every pass's loads are asked for
+// before the first is quantized (a pass a trip to memory otherwise), without a branch around any of them (past the
+// end: the last float4 again; nothing is stored for it).
 template <int NP>
 __device__ __forceinline__ void stage_q8_passes(const float* __restrict__ x, int n8, int c0, int f16_scale, i8* lxq, float* lxs, int* xsum,
                                                 const float* __restrict__ nw, float nscale, float* __restrict__ h, int tid, int nthreads) {

@@ -405,7 +405,8 @@ class DenseModel:
         # 2,500 87.2 -> 81.7, 4,096 183.4 -> 179.4.  Below 640 the halves, whole tiles of 128 tokens but for the last, gain
         # where they leave little of a tile empty: 224 tokens 10.1 -> 9.1, 256 10.4 -> 9.7..10.2, 448 13.0 -> 12.7, 512 14.0 ->
         # 13.6; 288, 320, 416 and 576 lose up to 10 %.  Far into a conversation a few hundred tokens are mostly attention, whose
-        # launches fill the GPU whole: 448 at 1,500 positions 23.4 -> 24.7.
+        # launches fill the GPU whole: 448 at 1,500 positions 23.4 -> 24.7.  (Other shapes take these lines and the next as they
+        # are: two shapes are what they were drawn from.)
         if not (n >= 640 or 448 <= n <= 512 and self.pos < 1024 or n <= 256):
             return False
         # A small model's launches are over before the next is queued, so twice as many of them only cost (the Qwen2.5-0.5B

@@ -37,15 +37,14 @@ CASES = [
 ]
 
 
-# ILT_I8_PLANES: "0" = the 64 x 64 kernel always, "1" = always the pipelined kernels (Q6_K and Q4_K as two int8 planes, Q8_0
-# a block per MFMA), else only with enough tokens and rows to fill their 128 x 128 tiles.  The planes' kernel takes 64-row
-# tiles where 128-row tiles would leave most CUs idle -- every shape here -- and ILT_I8P_TM=128 holds it to the large tile
-# ("1/128").
+# ILT_I8_PLANES: "0" = the 64 x 64 kernel always, "1" = always the kernels of many tokens (Q6_K and Q4_K with their operands in
+# registers, Q8_0 in register tiles), else whichever the shape is for.  The former takes tiles of 64 rows where tiles of 128
+# would leave most CUs idle -- every shape here -- and ILT_I8_TM=128 holds it to the large tile ("1/128").
 @pytest.mark.parametrize("planes", [None, "0", "1", "1/128"])
 @pytest.mark.parametrize("qtype,rows,cols,n", CASES)
 def test_dense_prefill_equals_cpu_matmul_bit_for_bit(dev, monkeypatch, qtype, rows, cols, n, planes):
     from illatio_amd import dense, hip
-    monkeypatch.delenv("ILT_I8P_TM", raising=False)
+    monkeypatch.delenv("ILT_I8_TM", raising=False)
     if planes is None:
         monkeypatch.delenv("ILT_I8_PLANES", raising=False)
     elif cols % 64 or (planes == "1/128" and qtype == synth.Q8_0):
@@ -53,7 +52,7 @@ def test_dense_prefill_equals_cpu_matmul_bit_for_bit(dev, monkeypatch, qtype, ro
     else:
         monkeypatch.setenv("ILT_I8_PLANES", planes[0])
         if planes == "1/128":
-            monkeypatch.setenv("ILT_I8P_TM", "128")
+            monkeypatch.setenv("ILT_I8_TM", "128")
     rng = synth.make_rng(qtype * 31 + rows + n)
     w = synth.weights(qtype, rows, cols, rng)
     x = synth.activations((n, cols), rng)
@@ -230,7 +229,7 @@ def test_products_of_no_tokens_write_nothing(dev):
 
 @pytest.mark.parametrize("ne,d,ff,nu,n,clamp", [(8, 512, 256, 3, 37, 0.0), (16, 1024, 512, 4, 150, 0.6),
                                                  (12, 4096, 2048, 6, 96, 0.0)])
-@pytest.mark.parametrize("planes", [None, "0", "1"])        # the down product (Q2_K) on the 64 x 64 kernel / on the planes kernel
+@pytest.mark.parametrize("planes", [None, "0", "1"])        # the grouped products as the shape says / on the 64 x 64 kernel / on the registers' kernel
 def test_moe_prefill_chunk_bit_exact(dev, monkeypatch, ne, d, ff, nu, n, clamp, planes):
     """the benchmark's config 5's sequence (route -> group -> gather -> grouped gate, up -> gated
     activation -> grouped down -> slot-ordered sum + shared) at reduced expert and token
