@@ -394,7 +394,7 @@ __global__ __launch_bounds__(256, 2) void attn_scores_quad_kernel(const float* _
 
 constexpr int kStepHeads = 8, kStepPositions = 128;      // a workgroup of one token's score kernel: query heads at most, positions
 // One token's qk_rope and scores in one launch.  A workgroup takes kStepPositions positions of a KV head for GH of its query heads
-// (blockIdx.z: which; the host says how many): the keys, which are most of what the launch reads, come from memory once and lie in
+// (blockIdx.z: which; gridDim.z: how many shares): the keys, which are most of what the launch reads, come from memory once and lie in
 // registers while one query head after another is multiplied with them (a workgroup a query head read them once a head, and on
 // different dies: 14.3 us at 4,117 positions of the Qwen3-4B shape, 17 MB of keys; now 7.5).  Waves 0 .. GH - 1 norm and turn the
 // query heads, wave kStepHeads the KV head's key where the workgroup's positions hold the token's own; that workgroup takes the key
@@ -406,12 +406,13 @@ __global__ __launch_bounds__(1024, NJ ? 8 : 4) void attn_step_scores_kernel(cons
                                                                 const float* __restrict__ qn, const float* __restrict__ kn,
                                                                 const float* __restrict__ rope, float* __restrict__ kc, float* __restrict__ vc,
                                                                 float* __restrict__ raw, int nh, int nkv, int hd, int rd, int pos, float eps,
-                                                                int neox, float scale, int spitch, int gh) {
+                                                                int neox, float scale, int spitch) {
   constexpr int GH = kStepHeads, NU = kStepPositions / 64;
   __shared__ float qsh[GH][256], ksh[256];
   __shared__ double scs[GH + 1];
   const int kh = blockIdx.x, tid = threadIdx.x, npos = pos + 1, pbase = blockIdx.y * kStepPositions;
-  const int group = nh / nkv, kvd = nkv * hd, ko = kh * hd, h0 = kh * group + blockIdx.z * gh, heads = min(gh, group - (int)blockIdx.z * gh);
+  const int group = nh / nkv, gh = (group + (int)gridDim.z - 1) / (int)gridDim.z;      // (gridDim.z = ceil(group / a share): no workgroup is without heads)
+  const int kvd = nkv * hd, ko = kh * hd, h0 = kh * group + blockIdx.z * gh, heads = min(gh, group - (int)blockIdx.z * gh);
   constexpr int NJM = NJ ? NJ : 16;
   const int l = tid & 15, pg = tid >> 4, nj = NJ ? NJ : hd >> 4, wave = tid >> 6;
   const bool own = pos < pbase + kStepPositions;   // this workgroup's positions hold the token's own
@@ -1627,11 +1628,11 @@ hipError_t ilt_k_attn_step(const float* q, const float* k, const float* v, const
     while (gh < group && gh < kStepHeads && (long long)nkv * blocks * ((group + gh - 1) / gh) > 256) gh++;
     const dim3 gs(nkv, blocks, (group + gh - 1) / gh);
     if (hd == 128)
-      hipLaunchKernelGGL(attn_step_scores_kernel<8>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax, gh);
+      hipLaunchKernelGGL(attn_step_scores_kernel<8>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax);
     else if (hd == 64)
-      hipLaunchKernelGGL(attn_step_scores_kernel<4>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax, gh);
+      hipLaunchKernelGGL(attn_step_scores_kernel<4>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax);
     else
-      hipLaunchKernelGGL(attn_step_scores_kernel<0>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax, gh);
+      hipLaunchKernelGGL(attn_step_scores_kernel<0>, gs, dim3(1024), 0, st, q, k, v, qn, kn, rope, kc, vc, scratch, nh, nkv, hd, rd, pos, eps, neox, scale, smax);
   }
   // past the one-launch kernel's 1,024 positions the values come in tiles while the chains run (at 1,536 positions 523
   // tok/s at the Qwen3-4B shape against 493 with the whole slice brought into LDS first, at 1,990 500 against 464);
