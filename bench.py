@@ -669,8 +669,8 @@ def workload_c5(args, dev):
                         else "gemm_i8r_group_kernel<16> (d4_mm_id2_iq2_xxs: gate and up) + <10> (d4_mm_id_q2_k: down): operands made in registers, "
                              "v_mfma_i32_32x32x32_i8, bit-exact with the CPU path"})
     roof["launch_us_all"] = {k: round(v[0] / v[2] * 1e3, 2) for k, v in per.items()}
-    if args.path == "bf16" and n == 4096:
-        t5 = TRAFFIC.get("c5", {})
+    if n == 4096:
+        t5 = TRAFFIC.get("c5" if args.path == "bf16" else "c5_exact", {})
         roof["traffic"] = int(sum(t5.values()) / len(t5)) if t5 else None       # per launch, over the step's two grouped launches
     tf = flops / (ms * 1e-3) / 1e12
 
