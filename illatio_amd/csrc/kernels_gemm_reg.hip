@@ -1,5 +1,5 @@
 // The exact prefill product of many tokens, the weights made in the matrix cores' operand registers: Y[t][r] = W[r].x_t, W in
-// GGUF Q4_K / Q6_K blocks, every result with the CPU path's bits (MATMUL!: kquant.lisp:180-236, batch.lisp:128).
+// GGUF Q4_K / Q6_K / Q2_K / IQ2_XXS blocks, every result with the CPU path's bits (MATMUL!: kquant.lisp:180-236, batch.lisp:128).
 //
 // What bounds it: the vector ALU and the matrix cores together (gfx950 issues a multiply or an add of two waves in the time a
 // third of an MFMA takes, and an MFMA hides permutes and 16-bit arithmetic but only half of the plain float work beside it),
