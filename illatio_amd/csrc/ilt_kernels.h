@@ -232,6 +232,11 @@ hipError_t ilt_k_attn_step(const float* q, const float* k, const float* v, const
 hipError_t ilt_k_attn_giveups(unsigned long long* out);
 hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok,
                            float* scratch, hipStream_t st);
+// A chunk's scores and values with the matrix cores' products (kernels_attn_mm.hip)
+bool ilt_k_attn_mm_takes(const float* q, const float* kc, const float* scratch, const float* out, int nh, int nkv, int hd, int ctx);
+hipError_t ilt_k_attn_scores_mm(const float* q, const float* kc, float* raw, int nh, int nkv, int hd, int pos0, int ntok, float scale, int spitch,
+                                hipStream_t st);
+hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, int spitch, hipStream_t st);
 hipError_t ilt_k_swiglu_rows(float* a, const float* b, long long n, hipStream_t st);
 
 #endif  // ILT_KERNELS_H

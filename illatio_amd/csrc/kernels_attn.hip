@@ -281,117 +281,6 @@ __global__ __launch_bounds__(1024) void attn_scores_kernel(const float* __restri
   }
 }
 
-// A prompt chunk's scores, sixteen of them a thread: a workgroup of 256 threads takes 64 tokens x 64 positions of a
-// query head, thread (tq, pq) the tokens tq + 16a and the positions pq + 16b.  F32-DOT16 keeps sixteen running sums,
-// sum l over the columns l, l + 16, ..., and adds them as ((s_l + s_l+4) + (s_l+8 + s_l+12)) = X_l for l = 0..3, then
-// (X_0 + X_1) + (X_2 + X_3).  The kernel above gives a score to sixteen lanes, a running sum each, and every lane
-// then goes through the four adds of the tree and the scaling for the sake of lane 0; here one thread keeps a score's
-// four sums l = e, e+4, e+8, e+12 for e = 0, 1, 2, 3 in turn, so that nothing is added that the score does not need, and
-// a 16-byte read of a token's or a position's row serves four scores.  For that the rows lie in LDS with every sixteen
-// columns transposed as 4 x 4 (place 4e + m holds column 4m + e): a thread that brings a row's sixteen columns in
-// stores them as four pieces of 16 bytes.  Row pitch HD + 4 floats: sixteen lanes' 16-byte reads of sixteen
-// consecutive rows fall on different banks.  The numbers are those of the kernel above.
-template <int NJ>      // HD / 16
-__global__ __launch_bounds__(256, 2) void attn_scores_quad_kernel(const float* __restrict__ q, const float* __restrict__ kc, float* __restrict__ raw,
-                                                               int nh, int nkv, int pos0, int ntok, float scale, int spitch) {
-  constexpr int HD = 16 * NJ, RP = HD + 4;
-  extern __shared__ __align__(16) float dyn[];     // 2 * 64 * RP floats
-  float* const qs = dyn;
-  float* const ks = dyn + 64 * RP;
-  const int h = blockIdx.x, p0 = blockIdx.y * 64, t0 = blockIdx.z * 64, tid = threadIdx.x;
-  const int tn = min(64, ntok - t0), nposmax = pos0 + t0 + tn;
-  if (p0 >= nposmax) return;                       // the same in every thread
-  const int group = nh / nkv, kvd = nkv * HD, ko = (h / group) * HD;
-  // rows 0..63: the tokens' q, 64..127: the positions' keys; 128 * NJ groups of sixteen columns, NJ / 2 a thread
-#pragma unroll
-  for (int u = 0; u < NJ / 2; u++) {
-    const int g = tid + 256 * u, row = g / NJ, j = g - row * NJ;
-    const float* src = row < 64 ? q + ((long long)(t0 + min(row, tn - 1)) * nh + h) * HD + 16 * j
-                                : kc + (long long)min(p0 + row - 64, nposmax - 1) * kvd + ko + 16 * j;
-    const float4 m0 = *(const float4*)src, m1 = *(const float4*)(src + 4), m2 = *(const float4*)(src + 8), m3 = *(const float4*)(src + 12);
-    float* dst = (row < 64 ? qs + row * RP : ks + (row - 64) * RP) + 16 * j;
-    *(float4*)dst = make_float4(m0.x, m1.x, m2.x, m3.x);
-    *(float4*)(dst + 4) = make_float4(m0.y, m1.y, m2.y, m3.y);
-    *(float4*)(dst + 8) = make_float4(m0.z, m1.z, m2.z, m3.z);
-    *(float4*)(dst + 12) = make_float4(m0.w, m1.w, m2.w, m3.w);
-  }
-  __syncthreads();
-  const int tq = tid >> 4, pq = tid & 15;
-  // none of the thread's positions is any of its tokens' to see (its first position, its last token)
-  if (p0 + pq >= pos0 + t0 + tq + 48 + 1) return;
-  const float* Q = qs + tq * RP;
-  const float* K = ks + pq * RP;
-  float y[4][4], z[4][4];
-  auto read_step = [&](float4 (&qr)[4], float4 (&kr)[4], const float* Qe, const float* Ke) {
-#pragma unroll
-    for (int a = 0; a < 4; a++) qr[a] = *(const float4*)(Qe + 16 * a * RP);
-#pragma unroll
-    for (int b = 0; b < 4; b++) kr[b] = *(const float4*)(Ke + 16 * b * RP);
-  };
-  // sums e, e+4, e+8, e+12 of the sixteen scores: two steps of sixteen columns a turn of the loop, each step's reads sent
-  // off before the step before it is multiplied (left to itself the compiler reads every step's rows first and spills)
-  auto sums = [&](auto Ec) {
-    constexpr int e = decltype(Ec)::value;
-    float4 acc[4][4], qa[4], ka[4], qb[4], kb[4];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-      for (int b = 0; b < 4; b++) acc[a][b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    auto mac = [&](const float4 (&qr)[4], const float4 (&kr)[4]) {
-#pragma unroll
-      for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-          acc[a][b].x = acc[a][b].x + kr[b].x * qr[a].x;
-          acc[a][b].y = acc[a][b].y + kr[b].y * qr[a].y;
-          acc[a][b].z = acc[a][b].z + kr[b].z * qr[a].z;
-          acc[a][b].w = acc[a][b].w + kr[b].w * qr[a].w;
-        }
-    };
-    const float* Qe = Q + 4 * e;
-    const float* Ke = K + 4 * e;
-    read_step(qa, ka, Qe, Ke);
-#pragma unroll 1
-    for (int j = 0; j < NJ; j += 2) {
-      read_step(qb, kb, Qe + 16 * (j + 1), Ke + 16 * (j + 1));
-      mac(qa, ka);
-      asm volatile("" ::: "memory");
-      const int jn = min(j + 2, NJ - 2);           // (after the last step: rows read again, for nobody)
-      read_step(qa, ka, Qe + 16 * jn, Ke + 16 * jn);
-      mac(qb, kb);
-      asm volatile("" ::: "memory");
-    }
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-      for (int b = 0; b < 4; b++) {
-        float x = (acc[a][b].x + acc[a][b].y) + (acc[a][b].z + acc[a][b].w);      // X_e
-        asm volatile("" : "+v"(x));                // (added here, not where the score is stored: the four sums are not kept till then)
-        if (e == 0) y[a][b] = x;
-        if (e == 1) y[a][b] = y[a][b] + x;
-        if (e == 2) z[a][b] = x;
-        if (e == 3) z[a][b] = z[a][b] + x;
-      }
-    __builtin_amdgcn_sched_barrier(0);             // (one set of sums in registers at a time)
-  };
-  sums(std::integral_constant<int, 0>{});
-  sums(std::integral_constant<int, 1>{});
-  sums(std::integral_constant<int, 2>{});
-  sums(std::integral_constant<int, 3>{});
-#pragma unroll
-  for (int a = 0; a < 4; a++) {
-    const int tt = tq + 16 * a, npos = pos0 + t0 + tt + 1;
-    if (tt < tn) {
-      float* dst = raw + ((long long)(t0 + tt) * nh + h) * spitch;
-#pragma unroll
-      for (int b = 0; b < 4; b++) {
-        const int p = p0 + pq + 16 * b;
-        if (p < npos) dst[p] = (y[a][b] + z[a][b]) * scale;
-      }
-    }
-  }
-}
-
 constexpr int kStepHeads = 8, kStepPositions = 128;      // a workgroup of one token's score kernel: query heads at most, positions
 // One token's qk_rope and scores in one launch.  A workgroup takes kStepPositions positions of a KV head for GH of its query heads
 // (blockIdx.z: which; gridDim.z: how many shares): the keys, which are most of what the launch reads, come from memory once and lie in
@@ -1192,135 +1081,6 @@ __global__ __launch_bounds__(1024) void attn_values_chunk_kernel(const float* __
   if (tt < tn) out[((long long)(t0 + tt) * nh + h) * hd + 32 * cs + c] = o;
 }
 
-// The same values with sixteen chains a thread, four tokens by four columns: a workgroup of 256 threads takes a query
-// head's HD columns for 4096 / HD tokens (32 at HD = 128).  The kernel above reads LDS eight times (16 bytes each) per
-// chain and 16 positions, which is what it waits for; here the four scores of a token (16 bytes along the positions)
-// serve four columns and a position's four values (16 bytes along the columns, as the cache holds them: no transpose)
-// four tokens -- half a read per chain and 4 positions -- and what is left is the multiplies and adds.  Tiles of 32
-// positions, in two LDS buffers, loaded into registers a tile ahead of their store.  A tile that lies wholly below all
-// of a wave's tokens goes without a test; the one or two at the tokens' own positions leave a chain alone from its
-// token's last position on.  Every chain: the same products and sums in the
-// same order as above.
-template <int HD>
-__global__ __launch_bounds__(256) void attn_values_quad_kernel(const float* __restrict__ raw, const float* __restrict__ vc, float* __restrict__ out,
-                                                               int nh, int nkv, int pos0, int ntok, int spitch) {
-  constexpr int CQ = HD / 4, TQ = 256 / CQ, NTOK = 4 * TQ, P = 32, SP = P + 4;
-  constexpr int NV = P * CQ / 256;                 // 16-byte pieces of a tile a thread brings in: of the values,
-  constexpr int NS = NTOK * (P / 4) / 256;         // of the scores
-  static_assert((NV == 2 || NV == 4) && (NS == 1 || NS == 2) && 256 % CQ == 0, "HD 64 or 128");
-  __shared__ __align__(16) float scs[2][NTOK * SP];      // a row a token
-  __shared__ __align__(16) float vts[2][P * HD];         // a row a position
-  const int gx = gridDim.x, h = (gx & 7) ? (int)blockIdx.x : (int)(blockIdx.x & 7) * (gx >> 3) + (int)(blockIdx.x >> 3);
-  // (token tiles: the first half of the launch takes them from the last -- the longest -- downwards, the second half
-  // from the first upwards: workgroups half a launch apart tend to share a CU, and so a long one meets a short one)
-  const int ny = gridDim.y, yh = ny >> 1, by = blockIdx.y;
-  const int t0 = (by < yh ? ny - 1 - by : by - yh) * NTOK, tid = threadIdx.x;
-  const int tn = min(NTOK, ntok - t0), nposmax = pos0 + t0 + tn;
-  const int group = nh / nkv, kvd = nkv * HD, ko = (h / group) * HD;
-  const float* rbase = raw + ((long long)t0 * nh + h) * spitch;
-  const int tq = tid / CQ, cq = tid - tq * CQ;     // tokens t0 + 4 tq .. + 3, columns 4 cq .. + 3
-  const int wtq = (tid >> 6) * (64 / CQ);          // the wave's first tq
-  const int ntiles = (nposmax + P - 1) / P;
-  // (named registers: arrays indexed in these loops were left in private memory)
-  float4 rs0 = {}, rs1 = {}, rv0 = {}, rv1 = {}, rv2 = {}, rv3 = {};
-  // (past a token's own positions, past the rows' end and past the chunk's last token: a piece that exists, never used)
-  auto load_s = [&](int p0, int u) {
-    const int i = tid + 256 * u, rt = min(i >> 3, tn - 1), pc = min((p0 >> 2) + (i & 7), (spitch >> 2) - 1);
-    return *(const float4*)(rbase + (long long)rt * nh * spitch + 4 * pc);
-  };
-  auto load_v = [&](int p0, int u) {
-    const int k = tid + 256 * u, p = min(p0 + k / CQ, nposmax - 1);
-    return *(const float4*)(vc + (long long)p * kvd + ko + 4 * (k % CQ));
-  };
-  auto load_tile = [&](int tile) {
-    const int p0 = tile * P;
-    rs0 = load_s(p0, 0);
-    if (NS > 1) rs1 = load_s(p0, 1);
-    rv0 = load_v(p0, 0);
-    if (NV > 1) rv1 = load_v(p0, 1);
-    if (NV > 2) { rv2 = load_v(p0, 2); rv3 = load_v(p0, 3); }
-  };
-  auto store_s = [&](int buf, int u, const float4& r) {
-    const int i = tid + 256 * u;
-    *(float4*)(scs[buf] + (i >> 3) * SP + 4 * (i & 7)) = r;
-  };
-  auto store_tile = [&](int buf) {
-    store_s(buf, 0, rs0);
-    if (NS > 1) store_s(buf, 1, rs1);
-    *(float4*)(vts[buf] + 4 * tid) = rv0;
-    if (NV > 1) *(float4*)(vts[buf] + 4 * (tid + 256)) = rv1;
-    if (NV > 2) { *(float4*)(vts[buf] + 4 * (tid + 512)) = rv2; *(float4*)(vts[buf] + 4 * (tid + 768)) = rv3; }
-  };
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int k = 0; k < 4; k++) acc[i][k] = 0.0f;
-  load_tile(0);
-  store_tile(0);
-  if (ntiles > 1) load_tile(1);
-  __syncthreads();
-  for (int t = 0; t < ntiles; t++) {
-    // tile t is in buffer t & 1; the registers hold tile t+1, and the other buffer's readers passed the last barrier
-    if (t + 1 < ntiles) store_tile((t + 1) & 1);
-    if (t + 2 < ntiles) load_tile(t + 2);
-    const float* S = scs[t & 1] + 4 * tq * SP;
-    const float* V = vts[t & 1] + 4 * cq;
-    // of the tile's positions, token 4 tq + i has the first np + i (all of them from 32 on, none up to 0)
-    const int np = pos0 + t0 + 4 * tq + 1 - t * P;
-    const int npw = pos0 + t0 + 4 * wtq + 1 - t * P;       // the wave's first tokens': its least
-    if (npw >= P) {
-#pragma unroll
-      for (int q = 0; q < P / 4; q++) {
-        float4 s[4], v[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) s[i] = *(const float4*)(S + i * SP + 4 * q);
-#pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = *(const float4*)(V + (4 * q + j) * HD);
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            const float sv = j == 0 ? s[i].x : j == 1 ? s[i].y : j == 2 ? s[i].z : s[i].w;
-            acc[i][0] = acc[i][0] + sv * v[j].x;
-            acc[i][1] = acc[i][1] + sv * v[j].y;
-            acc[i][2] = acc[i][2] + sv * v[j].z;
-            acc[i][3] = acc[i][3] + sv * v[j].w;
-          }
-      }
-    } else if (npw + 4 * (64 / CQ) - 1 > 0) {              // some lane of the wave has positions here
-#pragma unroll 1
-      for (int q = 0; q < P / 4; q++) {
-        if (4 * q >= np + 3) break;
-        float4 s[4], v[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) s[i] = *(const float4*)(S + i * SP + 4 * q);
-#pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = *(const float4*)(V + (4 * q + j) * HD);
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            const float sv = j == 0 ? s[i].x : j == 1 ? s[i].y : j == 2 ? s[i].z : s[i].w;
-            const bool own = 4 * q + j < np + i;
-            const float a0 = acc[i][0] + sv * v[j].x, a1 = acc[i][1] + sv * v[j].y;
-            const float a2 = acc[i][2] + sv * v[j].z, a3 = acc[i][3] + sv * v[j].w;
-            acc[i][0] = own ? a0 : acc[i][0];
-            acc[i][1] = own ? a1 : acc[i][1];
-            acc[i][2] = own ? a2 : acc[i][2];
-            acc[i][3] = own ? a3 : acc[i][3];
-          }
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int tk = t0 + 4 * tq + i;
-    if (tk < ntok) *(float4*)(out + ((long long)tk * nh + h) * HD + 4 * cq) = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
-  }
-}
-
 // ARGMAX (model.lisp:464-468): best = 0; an element replaces the best when it is greater -- so the first of equal
 // maxima, a NaN never (and if v[0] is a NaN nothing replaces it).  Two steps: each workgroup the best of its
 // stretch (every thread's own elements first, eight 16-byte loads in flight, then the threads', a smaller index
@@ -1419,56 +1179,27 @@ hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, flo
   static bool attr_set[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  // A chunk: scores, softmax, then 32 tokens x 32 columns a workgroup.  "ILT_ATTN_CHUNK=0": the kernels of 16 tokens x 16
-  // columns below instead (tests).
+  // A chunk: scores, softmax, then the values.  Heads of 64 and 128 columns: the matrix cores' products (kernels_attn_mm.hip;
+  // "ILT_ATTN_QUAD=0", tests: not those); others, and what lies on addresses that 16-byte accesses do not take: sixteen lanes
+  // a score and 32 tokens x 32 columns a workgroup.  "ILT_ATTN_CHUNK=0": the kernels of 16 tokens x 16 columns below instead (tests).
   if (scratch && ntok > 1 && pos0 + ntok <= 8192 && hd % 32 == 0) {
-    const char* off = getenv("ILT_ATTN_CHUNK");
+    const char *off = getenv("ILT_ATTN_CHUNK"), *quad = getenv("ILT_ATTN_QUAD");
     if (!(off && off[0] == '0')) {
+      const int ctx = pos0 + ntok;
+      const bool mm = !(quad && quad[0] == '0') && ilt_k_attn_mm_takes(q, kc, scratch, out, nh, nkv, hd, ctx);
       static bool set[64] = {};
       const size_t smem = sizeof(float) * 2 * 32 * (size_t)kChunkPitch;
-      if (!set[dev]) {
+      if (!mm && !set[dev]) {
         const hipError_t e = hipFuncSetAttribute((const void*)attn_values_chunk_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         if (e != hipSuccess) return e;
         set[dev] = true;
       }
-      const int ctx = pos0 + ntok;
-      // sixteen scores a thread for heads of 64 or 128 columns (16-byte loads of q and kc); "ILT_ATTN_QUAD=0" or "=v": the
-      // kernel of sixteen lanes a score (tests)
-      const char* quad = getenv("ILT_ATTN_QUAD");
-      const bool qaligned = ((((uintptr_t)q) | ((uintptr_t)kc)) & 15) == 0;
-      // (either kernel where it fills the GPU: 14 heads of 64 on 512 tokens are 112 workgroups of the values kernel,
-      // and the kernel of a chain a thread, 448 workgroups, takes 59 us for the chunk's attention where this one took 78;
-      // "ILT_ATTN_QUAD=1": whatever the shape)
-      const bool forced = quad && quad[0] == '1';
-      const long long swgs = (long long)nh * ((ctx + 63) / 64) * ((ntok + 63) / 64);
-      const long long vwgs = (long long)nh * ((ntok + (hd == 128 ? 31 : 63)) / (hd == 128 ? 32 : 64));
-      if ((hd == 128 || hd == 64) && qaligned && !(quad && (quad[0] == '0' || quad[0] == 'v')) && (forced || swgs >= 256)) {
-        static bool qset[64] = {};
-        const size_t qsmem = sizeof(float) * 2 * 64 * (size_t)(hd + 4);
-        if (!qset[dev]) {
-          hipError_t e = hipFuncSetAttribute((const void*)attn_scores_quad_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(float) * 2 * 64 * 132));
-          if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)attn_scores_quad_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(float) * 2 * 64 * 68));
-          if (e != hipSuccess) return e;
-          qset[dev] = true;
-        }
-        const dim3 gq(nh, (ctx + 63) / 64, (ntok + 63) / 64);
-        if (hd == 128) hipLaunchKernelGGL(attn_scores_quad_kernel<8>, gq, dim3(256), qsmem, st, q, kc, scratch, nh, nkv, pos0, ntok, scale, smax);
-        else hipLaunchKernelGGL(attn_scores_quad_kernel<4>, gq, dim3(256), qsmem, st, q, kc, scratch, nh, nkv, pos0, ntok, scale, smax);
-      } else {
-        launch_scores<16>(dim3(nh, (ctx + 255) / 256, (ntok + 15) / 16), st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);
-      }
+      if (mm) {
+        const hipError_t e = ilt_k_attn_scores_mm(q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax, st);
+        if (e != hipSuccess) return e;
+      } else launch_scores<16>(dim3(nh, (ctx + 255) / 256, (ntok + 15) / 16), st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);
       hipLaunchKernelGGL(attn_softmax_kernel, dim3(nh, ntok), dim3(256), sizeof(float) * smax, st, scratch, nh, pos0, smax);
-      // sixteen chains a thread for heads of 64 or 128 columns (16-byte loads and stores: of scratch, vc and out);
-      // "ILT_ATTN_QUAD=0": the kernel of one chain a thread (tests)
-      const bool aligned = ((((uintptr_t)scratch) | ((uintptr_t)vc) | ((uintptr_t)out)) & 15) == 0;
-      if ((hd == 128 || hd == 64) && aligned && !(quad && quad[0] == '0') && (forced || vwgs >= 192)) {
-        if (hd == 128)
-          hipLaunchKernelGGL(attn_values_quad_kernel<128>, dim3(nh, (ntok + 31) / 32), dim3(256), 0, st, scratch, vc, out, nh, nkv, pos0, ntok, smax);
-        else
-          hipLaunchKernelGGL(attn_values_quad_kernel<64>, dim3(nh, (ntok + 63) / 64), dim3(256), 0, st, scratch, vc, out, nh, nkv, pos0, ntok, smax);
-        return hipGetLastError();
-      }
+      if (mm) return ilt_k_attn_values_mm(scratch, vc, out, nh, nkv, hd, pos0, ntok, smax, st);
       hipLaunchKernelGGL(attn_values_chunk_kernel, dim3(nh * (hd / 32), (ntok + 31) / 32), dim3(1024), smem, st, scratch, vc, out, nh, nkv, hd, pos0,
                          ntok, smax);
       return hipGetLastError();

@@ -1,0 +1,232 @@
+// A prompt chunk's attention with its products made by the matrix cores (heads of 64 and 128 columns), every number the CPU
+// path's (attend-head!, model.lisp:298-334; F32-DOT16, tensor.lisp:370-378).
+//
+// Both halves of it are products rounded to single and then added in a fixed order, so no fused multiply-add and no sum
+// inside the matrix cores will do.  But v_mfma_f32_16x16x1_4b_f32 has one product a result, and with zeros to add to, each
+// result is that product rounded once (denormals and all: compared with v_mul_f32 over 26 million pairs; a product that
+// rounds to -0 stays -0, where 0 + -0 would be +0: no sum here shows it).  A thousand products are one instruction that
+// takes the time of sixteen adds, and its operands are sixteen rows and sixteen columns in one register each, straight from
+// memory: nothing passes through LDS.  The adds are the vector ALU's, a register of sixty-four sums an instruction.  (The
+// two do not run at the same time on gfx950: an instruction with 16 results and 16 adds beside it take 33-36 ns a SIMD, 15
+// and 17 apart; as mul and add they take 32.  What the matrix cores save is the operands' way: sixteen chains a thread
+// read LDS once a chain and four products.)
+//
+// The query heads of a KV head see the same keys and values, so a KV head's rows -- token t, head g of its group: row
+// t * group + g -- go through in tiles of 16 (or 4), whatever heads they are of.
+#include "ilt_device.h"
+#include "ilt_kernels.h"
+#include <type_traits>
+
+namespace {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ float part(const float4& v, int e) { return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w; }
+
+// raw[(t * nh + h) * spitch + p] = F32-DOT16(K[p], q) * scale.  A wave takes 16 rows and, one after another, npt tiles of 16
+// positions.  Block m of the instruction has columns 4m + e of every sixteen, so its results are the running sums e, 4 + e,
+// 8 + e and 12 + e of 256 scores, and a lane's four 16-byte pieces of a row (or a key) are its operands for e = 0 .. 3.
+// Positions are the results' rows: a lane stores four scores of one row.
+template <int NJ>      // hd / 16
+__global__ __launch_bounds__(256, 3) void attn_scores_mm_kernel(const float* __restrict__ q, const float* __restrict__ kc, float* __restrict__ raw,
+                                                                int nh, int group, int kvd, int pos0, int ntok, float scale, int spitch, int npt) {
+  constexpr int HD = 16 * NJ;
+  const int kvh = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = lane & 15, m = lane >> 4, rows = ntok * group;
+  // (the four waves: row tiles on the same positions, whose keys then come from the CU's own cache)
+  const int r0 = (blockIdx.z * 4 + wave) * 16, p0 = blockIdx.y * npt * 16;
+  if (r0 >= rows) return;
+  const int nposmax = pos0 + (min(r0 + 15, rows - 1)) / group + 1, pend = min(p0 + 16 * npt, nposmax);
+  if (p0 >= pend) return;
+  const int row = min(r0 + i, rows - 1), t = row / group, h = kvh * group + row - t * group;
+  const float* const qr = q + ((long long)t * nh + h) * HD + 4 * m;
+  float4 qa[NJ], ka[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; j++) qa[j] = *(const float4*)(qr + 16 * j);
+  float* const dst = raw + ((long long)t * nh + h) * spitch + 4 * m;
+  const float* const kbase = kc + (long long)kvh * HD + 4 * m;
+  auto load = [&](int p) {
+    const float* kr = kbase + (long long)min(p + i, nposmax - 1) * kvd;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) ka[j] = *(const float4*)(kr + 16 * j);
+  };
+  for (int p = p0; p < pend; p += 16) {
+    load(p);
+    v4f y, z;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const v16f zero = {};
+      v16f s = __builtin_amdgcn_mfma_f32_16x16x1f32(part(ka[0], e), part(qa[0], e), zero, 0, 0, 0);
+      v16f d = __builtin_amdgcn_mfma_f32_16x16x1f32(part(ka[1], e), part(qa[1], e), zero, 0, 0, 0);
+#pragma unroll
+      for (int j = 2; j <= NJ; j++) {
+        v16f dn = {};
+        if (j < NJ) dn = __builtin_amdgcn_mfma_f32_16x16x1f32(part(ka[j], e), part(qa[j], e), zero, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[r] = s[r] + d[r];
+        asm volatile("" : "+v"(s));
+        d = dn;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const float x = (s[r] + s[4 + r]) + (s[8 + r] + s[12 + r]);
+        if (e == 0) y[r] = x;
+        if (e == 1) y[r] = y[r] + x;
+        if (e == 2) z[r] = x;
+        if (e == 3) z[r] = z[r] + x;
+      }
+    }
+    if (r0 + i < rows && p + 4 * m < spitch) {       // (what lies past the row's own positions is never read)
+      v4f o;
+#pragma unroll
+      for (int r = 0; r < 4; r++) o[r] = (y[r] + z[r]) * scale;
+      *(v4f*)(dst + p) = o;
+    }
+  }
+}
+
+// out = the values' rows times the scaled scores (attn_softmax_kernel's), position after position.  A wave takes R rows
+// (16, or 4: v_mfma_f32_4x4x1_16b_f32) and 64 columns; an instruction is one position, its operands the position's values in
+// the wave's columns and its scores in the wave's rows.
+// R 16: the values are the product's rows and four scores a 16-byte load of a row's lane the columns, the same in all four
+// blocks.  R 4: a register holds the four rows' scores of sixteen positions, a block each, and the instruction broadcasts one
+// block to all (16-byte loads there, sixteen lanes with the same address, were the launch's time: 321 positions 11.2 -> 8 us).
+template <int R> struct ValMM;
+template <> struct ValMM<16> {
+  typedef v16f V;
+  static constexpr int P = 8, AHEAD = 2, NS = 8;     // positions a set of registers, sets, registers of scores in one
+  template <int K> static __device__ __forceinline__ V mul(const float (&s)[NS], float v) { const V z = {}; return __builtin_amdgcn_mfma_f32_16x16x1f32(v, s[K], z, 0, 0, 0); }
+};
+template <> struct ValMM<4> {
+  typedef v4f V;
+  static constexpr int P = 16, AHEAD = 3, NS = 1;
+  template <int K> static __device__ __forceinline__ V mul(const float (&s)[NS], float v) { const V z = {}; return __builtin_amdgcn_mfma_f32_4x4x1f32(s[0], v, z, 4, K, 0); }
+};
+
+template <int R, int HD>
+__global__ __launch_bounds__(256, R == 16 ? 4 : 2) void attn_values_mm_kernel(const float* __restrict__ prob, const float* __restrict__ vc, float* __restrict__ out,
+                                                                int nh, int group, int kvd, int pos0, int ntok, int spitch) {
+  using M = ValMM<R>;
+  using V = typename M::V;
+  constexpr int CG = HD / 64, WR = 4 / CG;           // column groups and row tiles of a workgroup's four waves
+  constexpr int P = M::P, AHEAD = M::AHEAD;
+  const int kvh = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rows = ntok * group, cg = wave % CG;
+  // (the last rows, which see the most positions, first: the launch ends with the short ones)
+  const int r0 = ((gridDim.y - 1 - blockIdx.y) * WR + wave / CG) * R;
+  if (r0 >= rows) return;
+  const int t0 = r0 / group, t1 = min(r0 + R - 1, rows - 1) / group;
+  const int npos0 = pos0 + t0 + 1, nposmax = pos0 + t1 + 1;
+  // (through buffer loads: a set's values are one vector offset and scalar ones that never change; what lies past the last
+  // position or in the next row is never added)
+  const __amdgpu_buffer_rsrc_t rs = ilt_rsrc(ilt_uniform_ptr(prob + ((long long)t0 * nh + kvh * group) * spitch), (u32)((t1 - t0) * nh + group) * (u32)spitch * 4u);
+  const __amdgpu_buffer_rsrc_t rv = ilt_rsrc(ilt_uniform_ptr(vc), (u32)nposmax * (u32)kvd * 4u);
+  const int srow = min(r0 + (lane & (R - 1)), rows - 1), st = srow / group;
+  const u32 so = ((u32)((st - t0) * nh + srow - st * group) * (u32)spitch + (R == 4 ? (u32)(lane >> 2) : 0u)) * 4u, vo = (u32)(kvh * HD + 64 * cg + lane) * 4u;
+  struct Set { float s[M::NS], v[P]; };
+  auto load = [&](Set& x, int p) {
+#pragma unroll
+    for (int k = 0; k < M::NS; k += 4) {
+      if constexpr (R == 4) x.s[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, so + 4u * (u32)p, 0, 0));
+      else {
+        const float4 f = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, so + 4u * (u32)p + 4u * k, 0, 0));
+        x.s[k] = f.x; x.s[k + 1] = f.y; x.s[k + 2] = f.z; x.s[k + 3] = f.w;
+      }
+    }
+    const u32 pv = vo + (u32)p * (u32)kvd * 4u;
+#pragma unroll
+    for (int k = 0; k < P; k++) x.v[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, pv, k * kvd * 4, 0));
+  };
+  V acc = {};
+  int npos[R == 4 ? 4 : 1];                          // R 16: a lane's results are one row's; R 4: its column's in four rows
+#pragma unroll
+  for (int r = 0; r < (R == 4 ? 4 : 1); r++) npos[r] = pos0 + (R == 4 ? min(r0 + r, rows - 1) / group : st) + 1;
+  auto set = [&](const Set& x, int p, auto ownc) {   // OWN: rows may end inside these positions
+    constexpr bool OWN = decltype(ownc)::value;
+    auto mul = [&](auto kc) { constexpr int k = decltype(kc)::value; return M::template mul<k>(x.s, x.v[k]); };
+    auto add = [&](const V& d, int k) {
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const float a = acc[r] + d[r];
+        acc[r] = !OWN || p + k < npos[R == 4 ? r : 0] ? a : acc[r];
+      }
+      asm volatile("" : "+v"(acc));
+    };
+    using std::integral_constant;
+    V d0 = mul(integral_constant<int, 0>{}), d1;
+    auto two = [&](auto kc) {                        // a product ahead of the sums
+      constexpr int k = decltype(kc)::value;
+      d1 = mul(integral_constant<int, k + 1>{});
+      add(d0, k);
+      if constexpr (k + 2 < P) d0 = mul(integral_constant<int, k + 2>{});
+      add(d1, k + 1);
+    };
+    two(integral_constant<int, 0>{}); two(integral_constant<int, 2>{}); two(integral_constant<int, 4>{}); two(integral_constant<int, 6>{});
+    if constexpr (P == 16) { two(integral_constant<int, 8>{}); two(integral_constant<int, 10>{}); two(integral_constant<int, 12>{}); two(integral_constant<int, 14>{}); }
+  };
+  Set x[AHEAD];
+#pragma unroll
+  for (int u = 0; u < AHEAD; u++) load(x[u], P * u);
+  int p = 0;
+  for (; p + P * AHEAD <= npos0; p += P * AHEAD) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++) {
+      set(x[u], p + P * u, std::false_type{});
+      load(x[u], p + P * u + P * AHEAD);
+    }
+  }
+  for (; p < nposmax; p += P * AHEAD) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++) {
+      const int pu = p + P * u;
+      if (pu + P <= npos0) set(x[u], pu, std::false_type{});
+      else if (pu < nposmax) set(x[u], pu, std::true_type{});
+      if (pu + P * AHEAD < nposmax) load(x[u], pu + P * AHEAD);
+    }
+  }
+  auto row_out = [&](int row) { return out + ((long long)(row / group) * nh + kvh * group + row % group) * HD + 64 * cg; };
+  if constexpr (R == 4) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) if (r0 + r < rows) row_out(r0 + r)[lane] = acc[r];
+  } else if (r0 + (lane & 15) < rows) {
+    float* const o = row_out(srow) + 4 * (lane >> 4);
+#pragma unroll
+    for (int b = 0; b < 4; b++) *(v4f*)(o + 16 * b) = v4f{acc[4 * b], acc[4 * b + 1], acc[4 * b + 2], acc[4 * b + 3]};
+  }
+}
+
+}  // namespace
+
+bool ilt_k_attn_mm_takes(const float* q, const float* kc, const float* scratch, const float* out, int nh, int nkv, int hd, int ctx) {
+  return (hd == 64 || hd == 128) && ((((uintptr_t)q) | ((uintptr_t)kc) | ((uintptr_t)scratch) | ((uintptr_t)out)) & 15) == 0 &&      // 16-byte loads and stores of them
+         (long long)ctx * nkv * hd < (1LL << 30) && 17LL * nh * (ctx + 3) < (1LL << 30);                         // 32-bit offsets: the values, a tile's rows
+}
+
+// A wave's position tiles: four, its rows' loads and the launch's waves shared among them, where the launch has more than twice
+// what the chip holds (512 tokens at none before 95 us for the chunk's attention with four, 99 with one; 1,250 at 1,250 917 and
+// 1,083); one below (21 tokens at 300: 23 us against 27).
+hipError_t ilt_k_attn_scores_mm(const float* q, const float* kc, float* raw, int nh, int nkv, int hd, int pos0, int ntok, float scale, int spitch,
+                                hipStream_t st) {
+  const int group = nh / nkv, rtiles = (ntok * group + 15) / 16, ptiles = (pos0 + ntok + 15) / 16;
+  const int npt = (long long)rtiles * nkv * ptiles < 8192 ? 1 : 4;
+  const dim3 grid(nkv, (ptiles + npt - 1) / npt, (rtiles + 3) / 4);
+  if (hd == 128) hipLaunchKernelGGL(attn_scores_mm_kernel<8>, grid, dim3(256), 0, st, q, kc, raw, nh, group, nkv * hd, pos0, ntok, scale, spitch, npt);
+  else hipLaunchKernelGGL(attn_scores_mm_kernel<4>, grid, dim3(256), 0, st, q, kc, raw, nh, group, nkv * hd, pos0, ntok, scale, spitch, npt);
+  return hipGetLastError();
+}
+
+// Sixteen rows a wave once that leaves about six waves a CU (32 heads of 128 over 8 on 512 tokens, 2,048 waves: 95.7 us for the
+// chunk's attention against 97.6 with four; 1,250 at 1,250 893 against 1,102), else four: a wave's chain of positions, an
+// instruction every few cycles, is the launch's time (256 tokens 41 us against 43, 64 tokens 13.9 against 15.5, 14 heads of 64
+// over 2 on 1,250 121 against 137, 3 tokens at 2,000 55 against 115).
+hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, int spitch, hipStream_t st) {
+  const int group = nh / nkv, rows = ntok * group, cg = hd / 64, wr = 4 / cg;
+  const int r = (long long)((rows + 15) / 16) * nkv * cg >= 1600 ? 16 : 4;
+  const dim3 grid(nkv, ((rows + r - 1) / r + wr - 1) / wr);
+#define ILT_VALUES(R, HD) hipLaunchKernelGGL((attn_values_mm_kernel<R, HD>), grid, dim3(256), 0, st, prob, vc, out, nh, group, nkv * hd, pos0, ntok, spitch)
+  if (r == 16) { if (hd == 128) ILT_VALUES(16, 128); else ILT_VALUES(16, 64); }
+  else { if (hd == 128) ILT_VALUES(4, 128); else ILT_VALUES(4, 64); }
+#undef ILT_VALUES
+  return hipGetLastError();
+}

@@ -440,6 +440,41 @@ def test_chunk_attention_with_sixteen_scores_and_chains_a_thread(dev, monkeypatc
         hip.hip_free(b)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,pos0,ntok,what", [(3, 3, 64, 0, 2, ""), (7, 1, 64, 47, 5, ""), (14, 2, 64, 15, 33, "nan"), (8, 2, 128, 16, 17, "denormal"),
+                                                      (32, 8, 128, 301, 21, "nan"), (6, 2, 128, 1000, 63, "odd"), (16, 16, 128, 5, 801, "nan"),
+                                                      (15, 3, 64, 1, 1900, "denormal")])
+def test_chunk_attention_with_the_matrix_cores_products(dev, nh, nkv, hd, pos0, ntok, what):
+    """A chunk's attention with its products from the matrix cores against attn_rows' one launch, bit for bit: groups of 1, 2, 3,
+    4, 5 and 7 query heads, rows that end inside a tile of 16 and of 4, tiles of 16 (the last two) and of 4 rows; values of the
+    last position and the key before it that are NaN and infinite, which only the last tokens may see; values so small that
+    products are denormal; a query on an address that 16-byte loads do not take, which the other kernels get."""
+    import ctypes as C
+    from illatio_amd import hip
+    rng = synth.make_rng(2000 + nh + hd + pos0 + ntok)
+    f = lambda *sh: (rng.standard_normal(sh) * 1.5).astype(np.float32)
+    nctx = pos0 + ntok
+    qh, kh, vh = f(ntok * nh * hd + 1), f(nctx, nkv * hd), f(nctx, nkv * hd)
+    if what == "nan":
+        vh[-1, ::2], vh[-1, 1::2], kh[-1, 0] = np.nan, np.inf, np.nan
+    if what == "denormal":
+        vh *= np.float32(1e-38)
+    q, kc, vc = (hip.hip_upload_new(dev, a) for a in (qh, kh, vh))
+    scratch = hip.hip_alloc(dev, 4 * ntok * nh * ((nctx + 3) & ~3))
+    P = lambda b, at=0: C.c_uint64(b.ptr + at if b is not None else 0)
+    ints = (C.c_int(nh), C.c_int(nkv), C.c_int(hd), C.c_int(pos0), C.c_int(ntok))
+    outs = []
+    for scr in (None, scratch):
+        out = hip.hip_upload_new(dev, np.full(ntok * nh * hd, 7.0, np.float32))
+        hip.call("ilt_attn_rows", C.c_uint64(0), P(q, 4 if what == "odd" else 0), P(kc), P(vc), P(out), *ints, P(scr))
+        outs.append(hip.hip_floats(out, ntok * nh * hd).reshape(ntok, -1))
+        hip.hip_free(out)
+    n = ntok - 1 if what == "nan" else ntok
+    assert np.isfinite(outs[0][:n]).all() and np.array_equal(outs[1], outs[0], equal_nan=True)      # (which NaN is nobody's promise)
+    assert np.array_equal(bits(outs[1][:n]), bits(outs[0][:n])), np.abs(outs[1][:n] - outs[0][:n]).max()
+    for b in (q, kc, vc, scratch):
+        hip.hip_free(b)
+
+
 def test_a_chunk_as_parts_side_by_side(dev):
     """forward_parts -- a chunk's halves or quarters on streams of their own, a part's attention waiting for the earlier
     parts' keys layer by layer -- leaves forward_n's logits and caches, bit for bit: halves of 128 + 128, of 256 + 44 (the
