@@ -21,13 +21,14 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The softmax's 1/sum as the CPU rounds it to a single, from a sum of n exps added in another order than the CPU's
-// (within sum * (n + 8) * 2^-51 of the CPU's): one division, then whether every sum that near has the same single for
-// its reciprocal -- the reciprocals of all of them lie within inv * (1 -+ d), d a little more than twice that slack
-// plus the division's own rounding, and rounding to single keeps their order.  False: the caller adds the exps again
-// in the CPU's order.
+// The softmax's 1/sum as the CPU rounds it to a single, from a sum of n exps added in another order than the CPU's: one
+// division, then whether every sum that the CPU's could be has the same single for its reciprocal.  No term is negative, so
+// the CPU's n - 1 adds one after another leave a double within (n - 1) 2^-53 of the exact sum, relatively, and a sum whose
+// terms go through at most 64 adds each (here: a thread's own, at most 32, a wave's six, the waves') one within 64 * 2^-53;
+// the two divisions, d's own arithmetic and the bounds' second order are the rest of d, and rounding to single keeps the
+// reciprocals' order.  False: the caller adds the exps again in the CPU's order.
 __device__ __forceinline__ bool recip_settled(double sum, int n, float* inv) {
-  const double r = 1.0 / sum, d = (double)(n + 8) * 0x1p-50 + 0x1p-50;
+  const double r = 1.0 / sum, d = (double)(n + 128) * 0x1p-53;
   *inv = (float)r;
   return (float)(r - r * d) == (float)(r + r * d);
 }
@@ -482,23 +483,116 @@ __device__ __forceinline__ void attn_softmax(const float* __restrict__ rw, const
   for (int p = me; p < npos; p += NT) sc[p] = sc[p] * inv;
 }
 
+// A prompt chunk's softmax, once a (head, token): the raw scores of row (t, h) become the scaled scores, in place.  NT threads a
+// row -- a wave, so that nobody waits for other waves; the workgroup where rows are few and long -- hold it in registers, NV
+// pieces of four positions each: a pass over the scores and back, 20 double operations an exponential beside it.
+typedef float ilt_f4u __attribute__((ext_vector_type(4), aligned(4)));
+template <int NT, int NV>
+__global__ __launch_bounds__(256) void attn_softmax_kernel(float* __restrict__ raw, int nh, int rows, int pos0, int spitch) {
+  __shared__ float redf[4];
+  __shared__ double redd[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, me = NT == 64 ? lane : threadIdx.x;
+  const int row = NT == 64 ? __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wave) : blockIdx.x;
+  if (row >= rows) return;                           // (NT 64: no barrier follows)
+  const int npos = pos0 + row / nh + 1, n4 = (npos + 3) >> 2;
+  float* const rw = raw + (long long)row * spitch;
+  ilt_f4u v[NV];
+  float mx = -3.402823466e38f;
+#pragma unroll
+  for (int u = 0; u < NV; u++) {
+    if (NT * u >= n4) break;
+    v[u] = *(const ilt_f4u*)(rw + 4 * min(me + NT * u, n4 - 1));
+  }
+#pragma unroll
+  for (int u = 0; u < NV; u++) {
+    if (NT * u >= n4) break;
+#pragma unroll
+    for (int k = 0; k < 4; k++) if (4 * (me + NT * u) + k < npos) mx = fmaxf(mx, v[u][k]);
+  }
+  mx = wave_max_float(mx);
+  if (NT > 64) {
+    if (lane == 0) redf[wave] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
+  }
+  double sum = 0.0;
+#pragma unroll
+  for (int u = 0; u < NV; u++) {
+    if (NT * u >= n4) break;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      v[u][k] = ilt_expf_via_double(v[u][k] - mx);
+      if (4 * (me + NT * u) + k < npos) sum += (double)v[u][k];
+    }
+  }
+  sum = wave_sum_double(sum);
+  if (NT > 64) {
+    if (lane == 0) redd[wave] = sum;
+    __syncthreads();
+    sum = (redd[0] + redd[1]) + (redd[2] + redd[3]);
+  }
+  // the CPU adds the terms one after another: its sum where the order could show in the rounded reciprocal (a row in 10^5 at
+  // 2,500 positions)
+  float inv;
+  if (!recip_settled(sum, npos, &inv)) {             // the same in all NT threads
+    sum = 0.0;
+    if constexpr (NT == 64) {
+#pragma unroll
+      for (int u = 0; u < NV; u++) {
+        if (NT * u >= n4) break;
+        for (int l = 0; l < min(64, n4 - 64 * u); l++)
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            if (4 * (l + 64 * u) + k < npos) sum += (double)__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[u][k]), l));
+      }
+    } else {
+      extern __shared__ __align__(16) float dyn[];   // spitch floats
+#pragma unroll
+      for (int u = 0; u < NV; u++) {
+        if (NT * u >= n4) break;
+        if (me + NT * u < n4)
+#pragma unroll
+          for (int k = 0; k < 4; k++) dyn[4 * (me + NT * u) + k] = v[u][k];
+      }
+      __syncthreads();
+      int p = 0;
+      for (; p + 16 <= npos; p += 16) {
+        float4 f[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) f[k] = *(const float4*)(dyn + p + 4 * k);
+#pragma unroll
+        for (int k = 0; k < 4; k++) { sum += (double)f[k].x; sum += (double)f[k].y; sum += (double)f[k].z; sum += (double)f[k].w; }
+      }
+      for (; p < npos; p++) sum += (double)dyn[p];
+    }
+    inv = (float)(1.0 / sum);
+  }
+#pragma unroll
+  for (int u = 0; u < NV; u++) {
+    if (NT * u >= n4) break;
+    if (me + NT * u < n4) *(ilt_f4u*)(rw + 4 * (me + NT * u)) = v[u] * inv;       // (past the row's positions: within its pitch, never read)
+  }
+}
+// A wave a row up to 4,096 positions (32 heads, 1,250 tokens: 44-48 us at none before, 95 at 1,250 before, where the workgroup takes 74
+// and 117); past that it is no faster (512 tokens at 7,000: a chunk's attention 1,337 us against 1,334), and the workgroup takes a
+// row where they are so few that waves are left.
+hipError_t launch_softmax(float* raw, int nh, int pos0, int ntok, int spitch, hipStream_t st) {
+  if (pos0 + ntok > 8192 || (long long)nh * ntok > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+  const int rows = nh * ntok, ctx = pos0 + ntok;
+#define ILT_SOFTMAX(NT, NV) \
+  hipLaunchKernelGGL((attn_softmax_kernel<NT, NV>), dim3(NT == 64 ? (rows + 3) / 4 : rows), dim3(256), NT == 64 ? 0 : sizeof(float) * spitch, st, raw, nh, rows, pos0, spitch)
+  if (ctx <= 1024) ILT_SOFTMAX(64, 4);
+  else if (ctx <= 2048 && rows >= 1024) ILT_SOFTMAX(64, 8);
+  else if (ctx <= 4096 && rows >= 1024) ILT_SOFTMAX(64, 16);
+  else ILT_SOFTMAX(256, 8);
+#undef ILT_SOFTMAX
+  return hipGetLastError();
+}
+
 // grid x = head * (hd/16) + column slice; grid y = token group.  LDS: TG rows of spitch scores, then the value
 // slice with the positions along a row, vt[c * vpitch + p] (vpitch = 4 mod 64: sixteen threads' 16-byte reads
 // of sixteen rows fall on different banks).  NB: the slice is at most NB * 2048 16-byte pieces (512 NB positions).
 // With one token a workgroup the slice is stored times that token's scores, by all threads, and the chains add.
-// A prompt chunk's softmax, once a (head, token) instead of once in each of the head's hd/16 workgroups of
-// attn_values_kernel (the exps go through double: eight times over they were most of that kernel): the raw scores of
-// row (t, h) become the scaled scores, in place.
-__global__ __launch_bounds__(256) void attn_softmax_kernel(float* __restrict__ raw, int nh, int pos0, int spitch) {
-  extern __shared__ __align__(16) float dyn[];
-  __shared__ float redf[4];
-  __shared__ double redd[8];
-  const int h = blockIdx.x, t = blockIdx.y, npos = pos0 + t + 1;
-  float* rw = raw + ((long long)t * nh + h) * spitch;
-  attn_softmax<256, false>(rw, nullptr, dyn, npos, threadIdx.x, redf, redd);
-  for (int p = threadIdx.x; p < npos; p += 256) rw[p] = dyn[p];       // (each thread the entries it scaled itself)
-}
-
 // PROB: raw holds the scaled scores already (attn_softmax_kernel ran).
 template <int TG, int NB, bool PROB = false>
 __global__ __launch_bounds__(256) void attn_values_kernel(const float* __restrict__ raw, const float* __restrict__ vc, float* __restrict__ out,
@@ -1198,7 +1292,8 @@ hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, flo
         const hipError_t e = ilt_k_attn_scores_mm(q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax, st);
         if (e != hipSuccess) return e;
       } else launch_scores<16>(dim3(nh, (ctx + 255) / 256, (ntok + 15) / 16), st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);
-      hipLaunchKernelGGL(attn_softmax_kernel, dim3(nh, ntok), dim3(256), sizeof(float) * smax, st, scratch, nh, pos0, smax);
+      const hipError_t es = launch_softmax(scratch, nh, pos0, ntok, smax, st);
+      if (es != hipSuccess) return es;
       if (mm) return ilt_k_attn_values_mm(scratch, vc, out, nh, nkv, hd, pos0, ntok, smax, st);
       hipLaunchKernelGGL(attn_values_chunk_kernel, dim3(nh * (hd / 32), (ntok + 31) / 32), dim3(1024), smem, st, scratch, vc, out, nh, nkv, hd, pos0,
                          ntok, smax);
@@ -1226,7 +1321,8 @@ hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, flo
     if (e == hipSuccess) {                                                                                                                     \
       set[dev] = true;                                                                                                                         \
       launch_scores<TG>(gs, st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);                                                         \
-      if (TG > 1) hipLaunchKernelGGL(attn_softmax_kernel, dim3(nh, ntok), dim3(256), sizeof(float) * smax, st, scratch, nh, pos0, smax);        \
+      if (TG > 1) e = launch_softmax(scratch, nh, pos0, ntok, smax, st);                                                                       \
+      if (e != hipSuccess) return e;                                                                                                           \
       hipLaunchKernelGGL((attn_values_kernel<TG, NB, (TG > 1)>), gv, dim3(256), bytes(TG), st, scratch, vc, out, nh, nkv, hd, pos0, ntok,      \
                          smax, vpitch);                                                                                                        \
       e = hipGetLastError();                                                                                                                   \
@@ -1251,7 +1347,8 @@ hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, flo
     }
     if (tg == 16) {
       launch_scores<16>(gs, st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);
-      hipLaunchKernelGGL(attn_softmax_kernel, dim3(nh, ntok), dim3(256), sizeof(float) * smax, st, scratch, nh, pos0, smax);
+      const hipError_t es = launch_softmax(scratch, nh, pos0, ntok, smax, st);
+      if (es != hipSuccess) return es;
       hipLaunchKernelGGL(attn_values_tiled_kernel<16>, gv, dim3(256), smem, st, scratch, vc, out, nh, nkv, hd, pos0, ntok, smax);
     } else {
       launch_scores<1>(gs, st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);

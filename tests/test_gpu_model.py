@@ -475,6 +475,42 @@ def test_chunk_attention_with_the_matrix_cores_products(dev, nh, nkv, hd, pos0, 
         hip.hip_free(b)
 
 
+@pytest.mark.parametrize("nh,pos0,ntok", [(2, 60, 3), (2, 1020, 4), (8, 1100, 130), (8, 2100, 130), (2, 2100, 5), (1, 8000, 192)])
+def test_chunk_softmax_where_the_order_of_the_sum_shows(dev, nh, pos0, ntok):
+    """A chunk whose exponentials' sum lies on the edge between two singles for its reciprocal, so that the softmax kernels (a wave
+    a row up to 1,024, 2,048 and 4,096 positions, a workgroup a row) take the CPU's order of adds: against attn_rows' one launch, bit
+    for bit.  One position's score is 0, the last one's is chosen so that 1 / sum is within the kernels' doubt of 1 - 2^-25."""
+    import ctypes as C
+    from illatio_amd import hip
+    hd, nctx = 64, pos0 + ntok                           # scale 1/8: a score is its key's first column over 8, exactly
+    rng = synth.make_rng(3000 + nctx)
+    sc = np.float32(-45.0 - rng.random(nctx, dtype=np.float32))
+    sc[0] = 0.0
+    ex = lambda v: np.exp(v.astype(np.float64)).astype(np.float32).astype(np.float64)
+    tie = 1.0 / (1.0 - 2.0 ** -25)
+    for i, room in ((nctx - 2, 2e-13), (nctx - 1, 0.0)):      # what is left to the edge: most of it by one, the rest by the other
+        sc[i] = -200.0
+        sc[i] = np.log(tie - room - np.cumsum(ex(sc))[-1])
+    total = np.cumsum(ex(sc))[-1]
+    doubt = (1.0 / total) * (nctx + 128) * 2.0 ** -53
+    assert np.float32(1.0 / total - doubt) != np.float32(1.0 / total + doubt)
+    qh, kh = np.zeros((ntok, nh * hd), np.float32), np.zeros((nctx, hd), np.float32)
+    qh[:, ::hd] = 1.0
+    kh[:, 0] = 8.0 * sc
+    q, kc, vc = (hip.hip_upload_new(dev, a) for a in (qh, kh, rng.standard_normal((nctx, hd)).astype(np.float32)))
+    scratch = hip.hip_alloc(dev, 4 * ntok * nh * ((nctx + 3) & ~3))
+    P = lambda b: C.c_uint64(b.ptr if b is not None else 0)
+    outs = []
+    for scr in (None, scratch):
+        out = hip.hip_upload_new(dev, np.full(ntok * nh * hd, np.nan, np.float32))
+        hip.call("ilt_attn_rows", C.c_uint64(0), P(q), P(kc), P(vc), P(out), C.c_int(nh), C.c_int(1), C.c_int(hd), C.c_int(pos0), C.c_int(ntok), P(scr))
+        outs.append(hip.hip_floats(out, ntok * nh * hd))
+        hip.hip_free(out)
+    assert np.isfinite(outs[0]).all() and np.array_equal(bits(outs[1]), bits(outs[0]))
+    for b in (q, kc, vc, scratch):
+        hip.hip_free(b)
+
+
 def test_a_chunk_as_parts_side_by_side(dev):
     """forward_parts -- a chunk's halves or quarters on streams of their own, a part's attention waiting for the earlier
     parts' keys layer by layer -- leaves forward_n's logits and caches, bit for bit: halves of 128 + 128, of 256 + 44 (the
