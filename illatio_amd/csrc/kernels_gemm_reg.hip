@@ -308,7 +308,8 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
   constexpr bool DEEP = NP == 1;
   constexpr int NI = DEEP ? 8 / WR : TN / (8 * WR * WT);       // direct loads of a wave a super-block's half (NP 1: all) of the tokens (four tokens each)
   constexpr int NW = (F::LOADS + WT - 1) / WT;       // and of the rows' blocks
-  static_assert((NP == 1 ? WT == 1 && 8 % WR == 0 : NP == 2 || NP == 4) && 2 * TN <= THREADS, "a thread a half token's sums");
+  constexpr int NC = (2 * TN + THREADS - 1) / THREADS;         // half tokens' sums a thread brings
+  static_assert(NP == 1 ? WT == 1 && 8 % WR == 0 : NP == 2 || NP == 4, "patches a wave");
   using Smem = RegSmemOf<FMT, NP, WR, WT>;
   Smem& S = *(Smem*)smem;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -346,33 +347,42 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
   // the tokens' scales and sums of 32 of a super-block, through registers
   const __amdgpu_buffer_rsrc_t rd = ilt_rsrc(ilt_uniform_ptr(p.xd + tok0 * nsb), (u32)(__builtin_amdgcn_readfirstlane(ntok) * nsb) * 4);
   const __amdgpu_buffer_rsrc_t rb = ilt_rsrc(ilt_uniform_ptr(p.bsums + (F::MINS ? tok0 * (p.cols >> 4) : 0)), F::MINS ? (u32)(__builtin_amdgcn_readfirstlane(ntok) * (p.cols >> 4)) * 4 : 0);
-  float c_yd; int4 c_bs[2];
-  const u32 ctok = (u32)((t >> 1) * nsb);            // (past the tile's tokens: zeros)
+  float c_yd[NC]; int4 c_bs[NC][2];                  // (past the tile's tokens: zeros)
   auto load_consts = [&](int sb) {
-    if (2 * TN < THREADS && t >= 2 * TN) return;
-    c_yd = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, ctok * 4, sb * 4, 0));
-    if constexpr (F::MINS) {
-      const u32 o = ctok * 64 + 32 * (t & 1);
-      const ilt_v4i a = __builtin_amdgcn_raw_buffer_load_b128(rb, o, sb * 64, 0), b = __builtin_amdgcn_raw_buffer_load_b128(rb, o + 16, sb * 64, 0);
-      c_bs[0] = make_int4(a.x, a.y, a.z, a.w); c_bs[1] = make_int4(b.x, b.y, b.z, b.w);
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+      const int h = t + i * THREADS;
+      if (2 * TN < THREADS && h >= 2 * TN) return;
+      const u32 ctok = (u32)((h >> 1) * nsb);
+      c_yd[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, ctok * 4, sb * 4, 0));
+      if constexpr (F::MINS) {
+        const u32 o = ctok * 64 + 32 * (h & 1);
+        const ilt_v4i a = __builtin_amdgcn_raw_buffer_load_b128(rb, o, sb * 64, 0), b = __builtin_amdgcn_raw_buffer_load_b128(rb, o + 16, sb * 64, 0);
+        c_bs[i][0] = make_int4(a.x, a.y, a.z, a.w); c_bs[i][1] = make_int4(b.x, b.y, b.z, b.w);
+      }
     }
   };
   auto store_consts = [&](int buf) {
-    if (2 * TN < THREADS && t >= 2 * TN) return;
-    if ((t & 1) == 0) S.xd[buf][t >> 1] = c_yd;
-    if constexpr (FMT == ILT_Q2_K) {
-      _Float16 hh[8];
 #pragma unroll
-      for (int k = 0; k < 8; k++) hh[k] = (_Float16)(float)(k < 4 ? (int)wordr(c_bs[0], k) : (int)wordr(c_bs[1], k - 4));
-      __builtin_memcpy(S.ms[buf] + 32 * (t >> 1) + 16 * (t & 1), hh, 16);
-    } else if constexpr (F::MINS) {
-      const int s[4] = { c_bs[0].x + c_bs[0].y, c_bs[0].z + c_bs[0].w, c_bs[1].x + c_bs[1].y, c_bs[1].z + c_bs[1].w };
-      _Float16 hh[4], ll[4];
+    for (int i = 0; i < NC; i++) {
+      const int h = t + i * THREADS;
+      if (2 * TN < THREADS && h >= 2 * TN) return;
+      if ((h & 1) == 0) S.xd[buf][h >> 1] = c_yd[i];
+      const int4 &b0 = c_bs[i][0], &b1 = c_bs[i][1];
+      if constexpr (FMT == ILT_Q2_K) {
+        _Float16 hh[8];
 #pragma unroll
-      for (int k = 0; k < 4; k++) { hh[k] = (_Float16)(float)(s[k] & ~127); ll[k] = (_Float16)(float)(s[k] & 127); }
-      _Float16* const dst = (_Float16*)(S.ms[buf] + 32 * (t >> 1)) + 4 * (t & 1);
-      __builtin_memcpy(dst, hh, 8);
-      __builtin_memcpy(dst + 8, ll, 8);
+        for (int k = 0; k < 8; k++) hh[k] = (_Float16)(float)(k < 4 ? (int)wordr(b0, k) : (int)wordr(b1, k - 4));
+        __builtin_memcpy(S.ms[buf] + 32 * (h >> 1) + 16 * (h & 1), hh, 16);
+      } else if constexpr (F::MINS) {
+        const int s[4] = { b0.x + b0.y, b0.z + b0.w, b1.x + b1.y, b1.z + b1.w };
+        _Float16 hh[4], ll[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) { hh[k] = (_Float16)(float)(s[k] & ~127); ll[k] = (_Float16)(float)(s[k] & 127); }
+        _Float16* const dst = (_Float16*)(S.ms[buf] + 32 * (h >> 1)) + 4 * (h & 1);
+        __builtin_memcpy(dst, hh, 8);
+        __builtin_memcpy(dst + 8, ll, 8);
+      }
     }
   };
   v16f sum[NP][1];
@@ -389,7 +399,7 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
   issue_x(0, 0);
   load_consts(0);
   store_consts(0);
-  if (t < TN) S.xd[2][t] = 0.0f;                     // (the block before the first: nothing)
+  for (int i = t; i < TN; i += THREADS) S.xd[2][i] = 0.0f;       // (the block before the first: nothing)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the direct loads have landed
   ilt_barrier_lds();
   F::block(blk, wsrc, l32, lh);
@@ -553,7 +563,7 @@ struct NoScan { u32 scan[1]; int tile_z, tile_t0, tile_n; };      // (tiles of g
 
 // FSET: the matrices' format, or 0 where Q4_K and Q6_K meet in a launch
 template <int FSET, int NP, int WR, int WT>
-__global__ __launch_bounds__(64 * WR * WT, 2) void gemm_i8r_kernel(BfParams p) {
+__global__ __launch_bounds__(64 * WR * WT, WR * WT == 1 ? 1 : 2) void gemm_i8r_kernel(BfParams p) {
   constexpr int TM = 32 * WR, TN = 32 * NP * WT;
   extern __shared__ __align__(16) unsigned char smem[];
   long tok0; int ntok, rt; const u8* w = p.w;
@@ -645,9 +655,54 @@ hipError_t launch_i8r_group(const BfParams& p, long long total_rows, hipStream_t
   return hipGetLastError();
 }
 
+// The tiles a launch may be cut into.  What a workgroup of each takes for a super-block, microseconds, with 1, 2, ... of them on
+// a CU, as many as fit (Q4_K; Q6_K), measured on 1,024 to 19,456 rows and 17 to 768 tokens: a wave alone on its SIMD issues an
+// instruction in 2.1 ns, two in 1.05 each, so tiles of one wave are the fastest way through the columns while there are fewer
+// of them than SIMDs, and large tiles, which unpack a weight for more tokens, once there are more.  (Workgroups of two waves come
+// to lie on the same two SIMDs of a CU: 1.4, then 2.35.)
+struct RegTile { int rows, tokens, fit; float us[2][5]; };
+constexpr RegTile kRegTiles[] = {
+  {32, 32, 5, {{1.1f, 1.18f, 1.3f, 1.35f, 2.0f}, {1.4f, 1.5f, 1.65f, 2.05f, 4.0f}}},       // (Q6_K: four fit, a fifth is a second round)
+  {32, 64, 4, {{1.75f, 1.95f, 2.05f, 2.4f}, {1.75f, 1.9f, 2.1f, 2.4f}}},
+  {64, 64, 4, {{1.4f, 2.35f, 2.6f, 3.05f}, {1.6f, 2.65f, 2.85f, 3.3f}}},
+  {64, 128, 2, {{1.7f, 2.8f}, {1.75f, 2.9f}}},
+  {128, 128, 2, {{2.6f, 4.4f}, {2.55f, 4.4f}}},
+};
+// Which of them, by the rounds that the chip takes the launch's workgroups in.  (Shapes, us for the tiles taken and for 64 or 128
+// rows x 128 tokens: Q6_K 2560 x 9728 on 256 tokens 57-64 and 89, on 512 81 and 90; Q4_K 2560 x 4096 on 256 25 and 33; 19456 x 2560 on 32
+// 17.6 and 31, on 192 35 and 48; 9728 x 2560 on 64 17.2 and 22.)
 template <int FSET>
-hipError_t dispatch_i8r(BfParams& p, bool big, hipStream_t st) {
-  return big ? launch_i8r<FSET, 4, 4, 1>(p, st) : launch_i8r<FSET, 2, 2, 2>(p, st);
+int reg_tile_of(const BfParams& p) {
+  int best = 0;
+  float least = 0.0f;
+  for (int v = 0; v < 5; v++) {
+    const RegTile& c = kRegTiles[v];
+    const int f = FSET == ILT_Q4_K ? 0 : 1, fit = v == 0 && f ? 4 : c.fit;
+    long long n = 0;
+    for (int m = 0; m < p.nmulti; m++) n += (p.mrows[m] + c.rows - 1) / c.rows;
+    n *= (p.ntok + c.tokens - 1) / c.tokens;
+    const long long round = 256LL * fit, rest = n % round;
+    const float us = (float)(n / round) * c.us[f][fit - 1] + (rest ? c.us[f][(rest + 255) / 256 - 1] : 0.0f);
+    if (v == 0 || us < least) { best = v; least = us; }
+  }
+  return best;
+}
+
+template <int FSET>
+hipError_t dispatch_i8r(BfParams& p, int forced, hipStream_t st) {
+  if constexpr (FSET == ILT_Q2_K || FSET == ILT_IQ2_XXS) {
+    // 128 rows x 128 tokens from 150 such tiles on; fewer leave CUs idle, and 64 x 128 fills twice as many
+    const bool big = forced ? forced == 128 : (long long)((p.mrows[0] + 127) / 128) * ((p.ntok + 127) / 128) >= 150;
+    return big ? launch_i8r<FSET, 4, 4, 1>(p, st) : launch_i8r<FSET, 2, 2, 2>(p, st);
+  } else {
+    switch (forced == 128 ? 4 : forced == 64 ? 3 : forced >= 1 && forced <= 5 ? forced - 1 : reg_tile_of<FSET>(p)) {
+      case 0: return launch_i8r<FSET, 1, 1, 1>(p, st);
+      case 1: return launch_i8r<FSET, 2, 1, 1>(p, st);
+      case 2: return launch_i8r<FSET, 2, 2, 1>(p, st);
+      case 3: return launch_i8r<FSET, 2, 2, 2>(p, st);
+      default: return launch_i8r<FSET, 4, 4, 1>(p, st);
+    }
+  }
 }
 
 constexpr int block_bytes_of(int fmt) {
@@ -657,10 +712,8 @@ constexpr int block_bytes_of(int fmt) {
 }  // namespace
 
 // Up to three matrices (Q4_K, Q6_K in any mix, or all Q2_K, or all IQ2_XXS) on the same tokens in one launch, their row tiles one after another.
-// hipErrorNotSupported, and nothing launched, where the shapes are not this kernel's.  128 rows x 128 tokens a workgroup from
-// 150 such tiles on; fewer leave CUs idle, and 64 x 128 (each weight unpacked twice, for 64 tokens at a time) fills twice
-// as many: Q6_K 2560 x 9728 on 512 tokens, 80 tiles: 79 against 104 us; on 1,024, 160: 124 against 112; Q4_K 2560 x 4096 the
-// same 39 against 49, 54 against 53; 19456 x 2560 on 128, 152: 36.4 against 35.5.  ILT_I8_TM (tests): 64 or 128 rows whatever the shape.
+// hipErrorNotSupported, and nothing launched, where the shapes are not this kernel's.  ILT_I8_TM (tests): 64 or 128 rows by 128 tokens
+// whatever the shape, 1 to 5 the tiles in kRegTiles' order.
 hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws, const int* rows, float* const* ys, const float* const* biases,
                              int cols, const int8_t* xq, const float* xd, const int* bsums, int ntok, int acc, hipStream_t st, long long ldy) {
   if (nmat < 1 || nmat > 3 || ntok < 1 || cols < 256 || cols % 256 != 0 || cols >= (1 << 22)) return hipErrorNotSupported;
@@ -681,13 +734,12 @@ hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws
   p.nmulti = nmat; p.cols = cols; p.x = (const u16*)xq; p.xd = xd; p.bsums = bsums; p.acc = acc; p.ntok = ntok;
   const char* force = getenv("ILT_I8_TM");
   const int forced = force ? atoi(force) : 0;
-  const bool big = forced ? forced == 128 : tiles128 * ((ntok + 127) / 128) >= 150;
   switch (fset) {
-    case ILT_Q4_K: return dispatch_i8r<ILT_Q4_K>(p, big, st);
-    case ILT_Q6_K: return dispatch_i8r<ILT_Q6_K>(p, big, st);
-    case ILT_Q2_K: return dispatch_i8r<ILT_Q2_K>(p, big, st);
-    case ILT_IQ2_XXS: return dispatch_i8r<ILT_IQ2_XXS>(p, big, st);
-    default: return dispatch_i8r<0>(p, big, st);
+    case ILT_Q4_K: return dispatch_i8r<ILT_Q4_K>(p, forced, st);
+    case ILT_Q6_K: return dispatch_i8r<ILT_Q6_K>(p, forced, st);
+    case ILT_Q2_K: return dispatch_i8r<ILT_Q2_K>(p, forced, st);
+    case ILT_IQ2_XXS: return dispatch_i8r<ILT_IQ2_XXS>(p, forced, st);
+    default: return dispatch_i8r<0>(p, forced, st);
   }
 }
 

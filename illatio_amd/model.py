@@ -400,14 +400,14 @@ class DenseModel:
             # 62.7; halves of a 512-token chunk lose; their sums' order depends on a launch's token count with or without
             # parts); from resident copies 28.4 -> 27.2 and 62.7 -> 62.1: left whole.
             return self.prefill == "bf16" and 1024 <= n <= self.chunk and work >= 1e10
-        # The exact ones, the Qwen3-4B shape (whole -> halves, ms; thirds and quarters always lose to halves): 640 tokens 15.6 ->
-        # 15.2, 832 21.0 -> 18.8, 1,024 24.5 -> 23.7, 2,048 60.2 -> 58.9; of two chunks 2,100 69.0 (2,048 and then 52) -> 62.4,
-        # 2,500 87.2 -> 81.7, 4,096 183.4 -> 179.4.  Below 640 the halves, whole tiles of 128 tokens but for the last, gain
-        # where they leave little of a tile empty: 224 tokens 10.1 -> 9.1, 256 10.4 -> 9.7..10.2, 448 13.0 -> 12.7, 512 14.0 ->
-        # 13.6; 288, 320, 416 and 576 lose up to 10 %.  Far into a conversation a few hundred tokens are mostly attention, whose
-        # launches fill the GPU whole: 448 at 1,500 positions 23.4 -> 24.7.  (Other shapes take these lines and the next as they
+        # The exact ones, the Qwen3-4B shape (whole -> halves, ms; thirds and quarters always lose to halves): 832 tokens 19.3 ->
+        # 18.0, 1,024 22.7 -> 21.2, 1,536 35.7 -> 34.3, 2,048 53.0 -> 51.1; 576, 640 and 768 lose up to 5 %.  Below that the halves,
+        # whole tiles of 128 tokens but for the last, gain where they leave little of a tile empty: 224 tokens 8.4 -> 7.8, 416
+        # 11.5 -> 10.7, 448 12.2 -> 11.0, 512 13.1 -> 12.3; 160, 192, 288, 320 and 384 lose up to 14 %.  Far into a conversation a few
+        # hundred tokens are mostly attention, whose launches fill the GPU whole: 512 at 1,500 positions 22.1 -> 23.8, 768 31.1 ->
+        # 34.9; 224 14.1 -> 13.0, 1,024 and more as whole or up to 2 % better.  (Other shapes take these lines and the next as they
         # are: two shapes are what they were drawn from.)
-        if not (n >= 640 or 448 <= n <= 512 and self.pos < 1024 or n <= 256):
+        if not (n <= 256 or n >= 1024 or self.pos < 1024 and (n >= 800 or 416 <= n <= 512)):
             return False
         # A small model's launches are over before the next is queued, so twice as many of them only cost (the Qwen2.5-0.5B
         # shape: 384 tokens 2.8 -> 3.0 ms, 512 3.28 -> 3.15, 1,024 6.7 -> 5.7; at 1,500 positions 1,536 tokens 16.8 -> 18.4,

@@ -19,7 +19,7 @@ def dev():
 
 
 # rows around tiles of 32, 64 and 128, tokens around patches of 32 and tiles of 128, one super-block, two, an odd number
-@pytest.mark.parametrize("rows_a_tile", ["64", "128"])
+@pytest.mark.parametrize("rows_a_tile", ["64", "128", "1", "2", "3"])
 @pytest.mark.parametrize("qtype,rows,cols,n", [
     (synth.Q4_K, 1, 256, 17), (synth.Q4_K, 127, 512, 33), (synth.Q4_K, 129, 768, 128), (synth.Q4_K, 300, 2560, 130),
     (synth.Q6_K, 31, 256, 64), (synth.Q6_K, 128, 512, 127), (synth.Q6_K, 65, 1280, 129), (synth.Q6_K, 257, 2816, 250)])
