@@ -293,6 +293,7 @@ int ilt_mv_multi_ahead(uint64_t stream, int nmat, const ilt_mv_desc* descs, int 
   if (e != ILT_OK || live == 0) return e;
   // (the next product's activations do not matter to its plan: this call's stand in for them)
   static const bool rows_on = []{ const char* f = getenv("ILT_ROWS_AHEAD"); return !(f && f[0] == '0'); }();      // ("0": never, for tests)
+  p.once = next_nmat > 0;                            // (a chain of products: this one's rows are not the next call's)
   if (rows_on && next_nmat && build(pn, &live_n, next_nmat, next_descs, next_cols, xf, nullptr, 0, next_glu) == ILT_OK && live_n &&
       ilt_gemv_plan(p, 1) == hipSuccess && ilt_gemv_plan(pn, 1) == hipSuccess)
     ilt_gemv_rows_of(pn, p.rows_ahead);
@@ -361,6 +362,7 @@ static int gemv_experts(uint64_t stream, int fmt, int ncols, int nrows, int row_
   p.ptrs = ptrs; p.sel = sel; p.cols = ncols;
   p.xq = xq; p.xs = xd; p.bsums = bsums; p.xf = xf; p.x_stride = x_stride; p.y_stride = y_stride;
   p.counts = counts; p.bases = counts ? bases : xrow;
+  p.once = 1;                                        // (which experts a token takes: not the last one's)
   return (int)ilt_gemv_launch(p, nz, S(stream));
 }
 
@@ -430,7 +432,7 @@ static int mvq8_glu(uint64_t stream, int rows, int cols, const int8_t* gq, const
     p.mat[i].rows = rows; p.mat[i].fmt = ILT_Q8_0; p.mat[i].row_bytes = cols;
   }
   p.cols = cols; p.xf = x; p.f16_scale = 0; p.glu = 2; p.clamp = clamp;
-  if (route) { p.route = *route; p.route.done = 0; }
+  if (route) { p.route = *route; p.route.done = 0; p.once = 1; }      // (a step's launch)
   const int e = (int)ilt_gemv_launch(p, 1, S(stream));
   if (route) route->done = e == ILT_OK ? p.route.done : 0;
   return e;
@@ -546,6 +548,7 @@ int shared_down_sum(uint64_t stream, int d, int ff, const int8_t* wq, const uint
   if (e != ILT_OK) return e;
   if (live == 0) return (int)hipErrorNotSupported;
   p.sum = {bd, (long long)d, nu};
+  p.once = 1;
   return (int)ilt_gemv_launch(p, 1, S(stream));
 }
 // A caller's events around the step's launches (ilt_d4_ffn_step_events): event i recorded on the stream before launch
@@ -1087,6 +1090,7 @@ static int dec_build(DecLaunch& L, int nmat, const ilt_mv_desc* descs, int cols,
   ILT_REQUIRE(xf && (norm || !glu));
   const int e = gemv_multi_build(L.p, &L.live, nmat, fmts, ws, wds, ys, bs, rows, cols, nullptr, nullptr, nullptr, xf, 1, acc, glu, 0, norm, eps, 0);
   if (e != ILT_OK) return e;
+  L.p.once = 1;
   L.planned = L.live > 0 && ilt_gemv_plan(L.p, 1) == hipSuccess;
   return ILT_OK;
 }

@@ -72,6 +72,7 @@ struct IltSumAlong {
 struct IltGemvParams {
   IltGemvMat mat[4];         // up to four matrices sharing the activations
   int nmat;
+  int once;                  // streamed variant: the rows are not wanted again soon (a launch of a token's chain; experts'): they leave L2 first
   const uint64_t* ptrs;      // experts: grid y's matrices are at ptrs[y] + mat[i].add,
   const uint32_t* sel;       //   or at ptrs[sel[y]] + mat[i].add when sel is given (ptrs = all the slots)
   int cols;

@@ -884,20 +884,23 @@ __device__ __forceinline__ int stream_scales(const u8* src_, int nbytes, u8* lds
   return nfull + (tail ? 1 : 0);
 }
 
-// Returns the number of load instructions issued (the same in every lane).
+// Returns the number of load instructions issued (the same in every lane).  ONCE: ilt_g2lds16_once's loads.
 template <int FMT>
-__device__ __forceinline__ int stream_run(const u8* w, long row0, int nrows, int S, long row_bytes, u8* lds_run, int lane) {
+__device__ __forceinline__ int stream_run(const u8* w, long row0, int nrows, int S, long row_bytes, u8* lds_run, int lane, int once) {
   using B = LdsBlk<FMT>;
   const u8* src = (const u8*)ilt_uniform_ptr(w + row0 * row_bytes);
   const int npieces = __builtin_amdgcn_readfirstlane(nrows * S * B::PPB);
   const int nfull = npieces >> 6, tail = npieces & 63;
   // this lane's piece of the first instruction; each further instruction is 64 pieces on
   u32 blk = (u32)lane / B::PPB, pc = (u32)lane % B::PPB;
-  for (int i = 0; i < nfull; i++) {
-    ilt_g2lds16(src + blk * B::BB + B::goff(pc), lds_run + i * 1024);
+  auto next = [&]() {
     blk += 64 / B::PPB; pc += 64 % B::PPB;
     if (pc >= B::PPB) { pc -= B::PPB; blk += 1; }
-  }
+  };
+  if (once)
+    for (int i = 0; i < nfull; i++) { ilt_g2lds16_once(src + blk * B::BB + B::goff(pc), lds_run + i * 1024); next(); }
+  else
+    for (int i = 0; i < nfull; i++) { ilt_g2lds16(src + blk * B::BB + B::goff(pc), lds_run + i * 1024); next(); }
   if (tail && lane < tail) ilt_g2lds16(src + blk * B::BB + B::goff(pc), lds_run + nfull * 1024);   // the lanes past the end load nothing
   return nfull + (tail ? 1 : 0);
 }
@@ -1231,7 +1234,7 @@ __global__ __launch_bounds__(kStreamThreads) void gemv_stream_kernel(IltGemvPara
   // What a row wave must know before its first loads, read from the arguments in two goes -- the launch's numbers and
   // the matrices' first batches; then this wave's matrix, whole.  (Argument loads left where the values are used
   // come one after another, each behind a branch on the one before: a dozen round trips to the scalar cache.)
-  const int a_nbatches = p.nbatches, a_nmat = p.nmat, a_glu = p.glu, a_batch = p.batch, a_region = p.region, a_cols = p.cols;
+  const int a_nbatches = p.nbatches, a_nmat = p.nmat, a_once = p.once, a_glu = p.glu, a_batch = p.batch, a_region = p.region, a_cols = p.cols;
   const int b1 = p.mat[1].batch0, b2 = p.mat[2].batch0, b3 = p.mat[3].batch0;
   const uint64_t* const a_ptrs = p.ptrs;
   const uint32_t* const a_sel = p.sel;
@@ -1240,7 +1243,7 @@ __global__ __launch_bounds__(kStreamThreads) void gemv_stream_kernel(IltGemvPara
   const long long u_row_bytes = p.mat[1].row_bytes, u_add = p.mat[1].add;
   const int u_fmt = p.mat[1].fmt;
   IltGemvMat m = p.mat[0];          // (the first matrix with them: the only one of most launches, no second go for those)
-  asm volatile("" ::"s"(a_nbatches), "s"(a_nmat), "s"(a_glu), "s"(a_batch), "s"(a_region), "s"(a_cols), "s"(b1), "s"(b2), "s"(b3), "s"(a_ptrs),
+  asm volatile("" ::"s"(a_nbatches), "s"(a_nmat), "s"(a_once), "s"(a_glu), "s"(a_batch), "s"(a_region), "s"(a_cols), "s"(b1), "s"(b2), "s"(b3), "s"(a_ptrs),
                "s"(a_sel), "s"(u_w), "s"(u_wd), "s"(u_row_bytes), "s"(u_add), "s"(u_fmt), "s"(m.w), "s"(m.wd), "s"(m.y), "s"(m.bias),
                "s"(m.row_bytes), "s"(m.add), "s"(m.rows), "s"(m.fmt), "s"(m.batch0), "s"(m.nbat), "s"(m.rq), "s"(m.rr));
   float* tw = terms + (long)rw * a_batch * tpr * nglu;
@@ -1286,10 +1289,10 @@ __global__ __launch_bounds__(kStreamThreads) void gemv_stream_kernel(IltGemvPara
   }
   int nup = 0;              // load instructions of the up matrix's rows: the last ones issued
   if (live) {
-    with_format<FSET>(fmt, [&](auto F) { stream_run<decltype(F)::value>(wg, row0, nrows, S, m.row_bytes, region, lane); });
+    with_format<FSET>(fmt, [&](auto F) { stream_run<decltype(F)::value>(wg, row0, nrows, S, m.row_bytes, region, lane, a_once); });
     if (q8) stream_scales((const u8*)(m.wd + row0 * S), nrows * S * 2, (u8*)scales, lane);
     if (a_glu) {
-      with_format<FSET>(ufmt, [&](auto F) { nup = stream_run<decltype(F)::value>(wu, row0, nrows, S, u_row_bytes, region_up, lane); });
+      with_format<FSET>(ufmt, [&](auto F) { nup = stream_run<decltype(F)::value>(wu, row0, nrows, S, u_row_bytes, region_up, lane, a_once); });
       if (q8) nup += stream_scales((const u8*)(u_wd + row0 * S), nrows * S * 2, (u8*)scales_up, lane);
     }
   }
