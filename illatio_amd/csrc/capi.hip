@@ -649,7 +649,7 @@ int ilt_d4_ffn_step_noalloc(uint64_t stream, int ne, int nu, int d, int ff, floa
 }
 
 namespace {
-struct SmallLayout { uint64_t rexp, xrow, wrow, smap, xq, xs, sg, su, mq, ms, sout, bm, bd, total; };
+struct SmallLayout { uint64_t rexp, xrow, wrow, smap, xq, xs, sg, su, mq, ms, sout, bm, bd, kq, kd, ks, total; };
 SmallLayout small_layout(int n, int nu, int d, int ff) {
   const uint64_t rows = (uint64_t)n * nu;
   SmallLayout l; uint64_t o = 0;
@@ -659,6 +659,8 @@ SmallLayout small_layout(int n, int nu, int d, int ff) {
   l.sg = take(4ull * n * ff); l.su = take(4ull * n * ff);
   l.mq = take((uint64_t)n * ff); l.ms = take((uint64_t)n * ff / 8);
   l.sout = take(4ull * n * d); l.bm = take(4 * rows * ff); l.bd = take(4 * rows * d);
+  const uint64_t k = std::max((uint64_t)n * d, rows * ff);                   // the tokens in Q8_K, then the gated activations
+  l.kq = take(k); l.kd = take(k / 64); l.ks = take(k / 4);
   l.total = o;
   return l;
 }
@@ -681,17 +683,30 @@ int ilt_d4_ffn_small(uint64_t stream, void* wsp, uint64_t ws_bytes, int n, int n
   int8_t *xq = (int8_t*)(ws + l.xq), *mq = (int8_t*)(ws + l.mq);
   const int rows = n * nu, grb = d / 256 * 66, drb = ff / 256 * 84;
   int e;
-  ILT_TRY(ilt_k_small_route(ne, nu, scale, logits, bias, n, rexp, xrow, wrow, smap, S(stream)));
+  // an expert's blocks decoded once for all its rows, or a row at a time (past 4096 columns a step is no whole row)
+  const bool share = ilt_k_share_takes(d, ff);
+  int8_t* const kq = (int8_t*)(ws + l.kq); float* const kd = (float*)(ws + l.kd); int* const ks = (int*)(ws + l.ks);
+  if (share) {
+    ILT_TRY(ilt_k_share_open(ne, nu, scale, logits, bias, n, rexp, xrow, wrow, smap, x, d, xq, xs, kq, kd, ks, S(stream)));
+  } else {
+    ILT_TRY(ilt_k_small_route(ne, nu, scale, logits, bias, n, rexp, xrow, wrow, smap, S(stream)));
+    ILT_TRY(ilt_k_quant_q8(x, xq, xs, nullptr, (long long)n * d / 32, 0, S(stream)));
+  }
   // the shared expert: its matrices once for all the tokens
-  ILT_TRY(ilt_k_quant_q8(x, xq, xs, nullptr, (long long)n * d / 32, 0, S(stream)));
   if ((e = ilt_mm_q8_mma2(stream, wt->sgate_q, wt->sgate_d, sg, nullptr, ff, wt->sup_q, wt->sup_d, su, nullptr, ff, nullptr, nullptr, nullptr, nullptr, 0,
                           xq, xs, d, n, 0))) return e;
-  ILT_TRY(ilt_k_swiglu_w_quant_q8(n, ff, clamp, sg, su, nullptr, mq, ms, S(stream)));
-  if ((e = ilt_mm_q8(stream, wt->sdown_q, wt->sdown_d, mq, ms, sout, nullptr, d, ff, n, 0))) return e;
   // the routed experts, a slot a (token, slot) row, an expert's rows one after another
-  if ((e = gemv_experts(stream, ILT_IQ2_XXS, d, ff, grb, 0, wt->gate_bytes, d, ff, wt->slots, rows, nullptr, nullptr, nullptr, x, wrow, clamp, bm, rexp,
-                        nullptr, nullptr, xrow))) return e;
-  if ((e = gemv_experts(stream, ILT_Q2_K, ff, d, drb, 2 * wt->gate_bytes, -1, ff, d, wt->slots, rows, nullptr, nullptr, nullptr, bm, nullptr, 0.0f, bd, rexp))) return e;
+  if (share) {
+    ILT_TRY(ilt_k_share_gate_up(wt->slots, 0, wt->gate_bytes, d, ff, rows, rexp, xrow, kq, kd, wrow, clamp, bm, S(stream)));
+    ILT_TRY(ilt_k_share_mid(n, rows, ff, clamp, sg, su, mq, ms, bm, kq, kd, ks, S(stream)));
+    ILT_TRY(ilt_k_share_down(wt->slots, 2 * wt->gate_bytes, ff, d, rows, rexp, kq, kd, ks, bd, S(stream)));
+  } else {
+    ILT_TRY(ilt_k_swiglu_w_quant_q8(n, ff, clamp, sg, su, nullptr, mq, ms, S(stream)));
+    if ((e = gemv_experts(stream, ILT_IQ2_XXS, d, ff, grb, 0, wt->gate_bytes, d, ff, wt->slots, rows, nullptr, nullptr, nullptr, x, wrow, clamp, bm, rexp,
+                          nullptr, nullptr, xrow))) return e;
+    if ((e = gemv_experts(stream, ILT_Q2_K, ff, d, drb, 2 * wt->gate_bytes, -1, ff, d, wt->slots, rows, nullptr, nullptr, nullptr, bm, nullptr, 0.0f, bd, rexp))) return e;
+  }
+  if ((e = ilt_mm_q8(stream, wt->sdown_q, wt->sdown_d, mq, ms, sout, nullptr, d, ff, n, 0))) return e;
   return (int)ilt_k_moe_sum_rows(d, nu, n, bd, smap, sout, moe, S(stream));
 }
 

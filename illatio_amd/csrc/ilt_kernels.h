@@ -122,6 +122,20 @@ void ilt_gemv_rows_of(const IltGemvParams& p, IltRowsAhead& out);
 
 unsigned long long ilt_k_streamed_launches();      // decode products launched as the streamed variant so far (diagnostic)
 
+// A short pass's routed experts, an expert's blocks decoded once for up to four of its rows (kernels_gemv_share.hip): rows i of the
+// n grouped ones work on expert rexp[i], equal ones side by side.  Whether the widths are the kernels'; ilt_k_small_route and the
+// tokens in both roundings (Q8_0's and Q8_K) in one launch; gate and up with the gated activation (ff floats a row);
+// ilt_k_swiglu_w_quant_q8 of the shared expert's gate and up and quantize-q8k! of those rows in one; the down product.
+int ilt_k_share_takes(int d, int ff);
+hipError_t ilt_k_share_open(int ne, int nu, float scale, const float* logits, const float* bias, int ntok, uint32_t* rexp, uint32_t* xrow, float* wrow,
+                            uint32_t* smap, const float* x, int d, int8_t* xq, float* xs, int8_t* kq, float* kd, int* bsums, hipStream_t st);
+hipError_t ilt_k_share_mid(int ntok, int rows, int ff, float clamp, const float* g, const float* u, int8_t* mq, float* ms, const float* x, int8_t* kq,
+                           float* kd, int* bsums, hipStream_t st);
+hipError_t ilt_k_share_gate_up(const uint64_t* ptrs, long long gate, long long up, int d, int ff, int n, const uint32_t* rexp, const uint32_t* xrow,
+                               const int8_t* kq, const float* kd, const float* wts, float clamp, float* y, hipStream_t st);
+hipError_t ilt_k_share_down(const uint64_t* ptrs, long long add, int ff, int d, int n, const uint32_t* rexp, const int8_t* kq, const float* kd,
+                            const int* bsums, float* y, hipStream_t st);
+
 hipError_t ilt_k_quant_q8(const float* x, int8_t* xq, float* xs, int* xsum, long long nblocks, int f16_scale, hipStream_t st);
 hipError_t ilt_k_quant_q8k(const float* x, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st);
 hipError_t ilt_k_swiglu_quant_q8(const float* gate, const float* up, int8_t* xq, float* xs, long long nblocks, int f16_scale, hipStream_t st);

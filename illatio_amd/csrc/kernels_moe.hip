@@ -23,28 +23,11 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_kernel(int ntok, int n
                  hash == 1 ? tid2eid + (long long)tokens[t] * nu : nullptr, sel + (long long)t * nu, wout + (long long)t * nu, s_idx[wv], s_sc[wv]);
 }
 
-// A short pass's routing and grouping, one workgroup: wave t routes token t into LDS, then thread r finds its (token, slot)
-// row's place among all of them ordered by expert (at most a hundred rows in earnest: counting the smaller ones is a few
-// microseconds less than the counters, the scan and the scatter as launches of their own, 7 + 15 us of a pass's launches).
 template <int K>
 __global__ __launch_bounds__(1024) void small_route_kernel(int ntok, int ne, int nu, float scale, const float* __restrict__ logits,
                                                            const float* __restrict__ bias, u32* __restrict__ rexp, u32* __restrict__ xrow,
                                                            float* __restrict__ wrow, u32* __restrict__ smap) {
-  __shared__ u32 s_idx[16][64];
-  __shared__ float s_sc[16][64];
-  __shared__ u32 sel[1024];
-  __shared__ float w[1024];
-  const int lane = threadIdx.x & 63, t = threadIdx.x >> 6;
-  if (t < ntok)
-    route_token<K>(lane, ne, nu, scale, logits + (long long)t * ne, bias, nullptr, sel + t * nu, w + t * nu, s_idx[t], s_sc[t]);
-  __syncthreads();
-  const int n = ntok * nu;
-  for (int r = threadIdx.x; r < n; r += blockDim.x) {
-    const u32 e = sel[r];
-    int at = 0;
-    for (int i = 0; i < n; i++) at += sel[i] < e || (sel[i] == e && i < r);
-    rexp[at] = e; xrow[at] = (u32)(r / nu); wrow[at] = w[r]; smap[r] = (u32)at;
-  }
+  small_route<K>(ntok, ne, nu, scale, logits, bias, rexp, xrow, wrow, smap);
 }
 
 __global__ void group_zero_kernel(int ne, u32* counts) {

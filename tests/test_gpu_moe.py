@@ -349,6 +349,34 @@ def test_moe_short_pass_of_a_few_tokens_bit_exact(dev, ne, d, ff, nu, n, clamp):
     pool.free(); sh.free()
 
 
+# an expert's rows from one to nine (groups of three and of two of them, whole and broken), more than 64 rows in all, every
+# width that the shared decoding takes at its ends, steps with lanes left over, fewer weight rows than a workgroup's, and widths
+# past it that take a row at a time, more experts than one launch routes beside the rounding
+@pytest.mark.parametrize("ne,d,ff,nu,n", [(3, 256, 1024, 3, 9), (16, 512, 512, 8, 9), (70, 1024, 256, 1, 9), (8, 256, 256, 2, 1),
+                                          (9, 4096, 256, 4, 5), (5, 256, 4096, 4, 7), (8, 768, 2816, 2, 4), (6, 2304, 1536, 3, 4),
+                                          (4, 4352, 256, 2, 3), (4, 256, 4352, 2, 3), (600, 256, 256, 3, 2)])
+def test_moe_short_pass_over_groups_and_widths(dev, ne, d, ff, nu, n):
+    from illatio_amd import ds4f, hip
+    rng = synth.make_rng(ne * 131 + d + ff + n)
+    gate, up, down, sg, su, sd = _moe_weights(rng, ne, d, ff)
+    pool = ds4f.ExpertPool(dev, ne, d, ff, gate, up, down)
+    sh = ds4f.SharedExpert(dev, d, ff, sg, su, sd)
+    norm = synth.activations((n, d), rng)
+    norm[0, 3::64] = 0.0
+    norm[-1, 17], norm[-1, 40] = 50.0, -50.0            # a block's largest magnitude with both signs
+    if n > 2:
+        norm[1] = 0.0
+    logits = synth.activations((n, ne), rng)
+    lb, nb = hip.hip_upload_new(dev, logits), hip.hip_upload_new(dev, norm)
+    moe = ds4f.ffn_small(dev, pool, sh, lb, nb, n, ne, nu, 1.5, 0.0)
+    got = hip.hip_floats(moe, n * d).reshape(n, d)
+    for t in range(n):
+        want, _, _ = orc.moe_token(gate, up, down, sg, su, sd, d, ff, ne, nu, 1.5, 0.0, logits[t], norm[t])
+        assert np.array_equal(bits(got[t]), bits(want)), (t, np.abs(got[t] - want).max())
+    for b in (lb, nb, moe):
+        hip.hip_free(b)
+    pool.free(); sh.free()
+
 
 @pytest.mark.parametrize("d,ff,n,clamp", [(512, 256, 37, 0.05), (4096, 2048, 130, 0.0)])
 def test_shared_expert_over_a_chunk_bit_exact(dev, d, ff, n, clamp):
