@@ -345,7 +345,7 @@ static int gemv_experts(uint64_t stream, int fmt, int ncols, int nrows, int row_
                         int x_stride, int y_stride, const uint64_t* ptrs, int nz, const int8_t* xq, const float* xd,
                         const int32_t* bsums, const float* xf, const float* wts, float clamp, float* dst,
                         const uint32_t* sel = nullptr, const uint32_t* counts = nullptr, const uint32_t* bases = nullptr,
-                        const uint32_t* xrow = nullptr) {
+                        const uint32_t* xrow = nullptr, int once = 0) {
   ILT_REQUIRE(nrows >= 0 && nz >= 0 && ncols > 0 && ncols % 256 == 0 && row_bytes == ncols / 256 * block_bytes(fmt));
   if (nrows == 0 || nz == 0) return ILT_OK;
   ILT_REQUIRE(ptrs && dst && add >= 0 && (add & 1) == 0 && (add_up < 0 || (add_up & 1) == 0) && x_stride % 256 == 0 && x_stride >= 0);
@@ -362,7 +362,7 @@ static int gemv_experts(uint64_t stream, int fmt, int ncols, int nrows, int row_
   p.ptrs = ptrs; p.sel = sel; p.cols = ncols;
   p.xq = xq; p.xs = xd; p.bsums = bsums; p.xf = xf; p.x_stride = x_stride; p.y_stride = y_stride;
   p.counts = counts; p.bases = counts ? bases : xrow;
-  p.once = 1;                                        // (which experts a token takes: not the last one's)
+  p.once = once;
   return (int)ilt_gemv_launch(p, nz, S(stream));
 }
 
@@ -421,7 +421,7 @@ int ilt_d4_mv_q2_k_f32(uint64_t stream, int ncols, int nrows, int row_bytes, int
 
 // route: a token's routing for the launch to carry along, or null; its done says whether the launch did
 static int mvq8_glu(uint64_t stream, int rows, int cols, const int8_t* gq, const uint16_t* gd, const int8_t* uq,
-                    const uint16_t* ud, const float* x, float clamp, float* mid, IltRouteAlong* route) {
+                    const uint16_t* ud, const float* x, float clamp, float* mid, IltRouteAlong* route, int once = 0) {
   ILT_REQUIRE(rows >= 0 && cols > 0 && cols % 32 == 0);
   if (rows == 0) return ILT_OK;
   ILT_REQUIRE(gq && gd && uq && ud && x && mid && ((uintptr_t)gq & 15) == 0 && ((uintptr_t)uq & 15) == 0 && ((uintptr_t)x & 15) == 0);
@@ -432,7 +432,8 @@ static int mvq8_glu(uint64_t stream, int rows, int cols, const int8_t* gq, const
     p.mat[i].rows = rows; p.mat[i].fmt = ILT_Q8_0; p.mat[i].row_bytes = cols;
   }
   p.cols = cols; p.xf = x; p.f16_scale = 0; p.glu = 2; p.clamp = clamp;
-  if (route) { p.route = *route; p.route.done = 0; p.once = 1; }      // (a step's launch)
+  if (route) { p.route = *route; p.route.done = 0; }
+  p.once = once;
   const int e = (int)ilt_gemv_launch(p, 1, S(stream));
   if (route) route->done = e == ILT_OK ? p.route.done : 0;
   return e;
@@ -540,7 +541,7 @@ int step_args_ok(int ne, int nu, int d, int ff, const ilt_ffn_step_weights* wt, 
 // The shared expert's down product as the step's last launch, the step's sum carried along (IltSumAlong): MOE gets
 // ((0 + bd[0]) + ... + bd[nu-1]) + W.smid.  hipErrorNotSupported (nothing launched) where the launch cannot take it.
 int shared_down_sum(uint64_t stream, int d, int ff, const int8_t* wq, const uint16_t* wd, const float* smid, const float* bd, int nu,
-                    float* moe) {
+                    float* moe, int once) {
   IltGemvParams p;
   int live = 0, fmt = ILT_Q8_0, rows = d;
   const void* w = wq; const float* nobias = nullptr;
@@ -548,7 +549,7 @@ int shared_down_sum(uint64_t stream, int d, int ff, const int8_t* wq, const uint
   if (e != ILT_OK) return e;
   if (live == 0) return (int)hipErrorNotSupported;
   p.sum = {bd, (long long)d, nu};
-  p.once = 1;
+  p.once = once;
   return (int)ilt_gemv_launch(p, 1, S(stream));
 }
 // A caller's events around the step's launches (ilt_d4_ffn_step_events): event i recorded on the stream before launch
@@ -567,21 +568,27 @@ int step_run(uint64_t stream, uint8_t* ws, int ne, int nu, int d, int ff, float 
   float *w = (float*)(ws + l.w), *smid = (float*)(ws + l.smid), *sout = (float*)(ws + l.sout);
   float *bm = (float*)(ws + l.bm), *bd = (float*)(ws + l.bd);
   const int grb = d / 256 * 66, drb = ff / 256 * 84;
+  // A step whose matrices are more than the dies' L2s hold (32 MB) finds none of them there the next time, so they leave L2 first
+  // (ilt_g2lds16_once): 6 of 256 experts, 4,096 x 2,048 (80 MB) 40.4 -> 38.6 us.  A smaller one may: 3 of 32, 2,048 x 2,048
+  // (24 MB), the same step again: 23.9 us, and 24.9 if they left.
+  const int once = (long long)nu * (2 * wt->gate_bytes + (long long)d * drb) + 3LL * d * ff * 17 / 16 > (32LL << 20);
   // the routing rides along with the shared expert's gate/up launch (one of its waves routes while the rows stream
   // in); where that launch cannot take it, a launch of its own
   IltRouteAlong route = {logits, bias, sel, w, ne, nu, scale, 0};
   g_step_marked = 0;
   ILT_TRY((hipError_t)step_mark(stream));
-  ILT_TRY((hipError_t)mvq8_glu(stream, ff, d, wt->sgate_q, wt->sgate_d, wt->sup_q, wt->sup_d, x, clamp, smid, &route));
+  ILT_TRY((hipError_t)mvq8_glu(stream, ff, d, wt->sgate_q, wt->sgate_d, wt->sup_q, wt->sup_d, x, clamp, smid, &route, once));
   if (!route.done) ILT_TRY((hipError_t)ilt_d4_route(stream, ne, nu, 0, scale, bias ? 1 : 0, logits, bias, nullptr, nullptr, sel, w, 1));
   ILT_TRY((hipError_t)step_mark(stream));
-  ILT_TRY((hipError_t)ilt_d4_mv_glu_iq2_xxs(stream, d, ff, grb, 0, wt->gate_bytes, 0, ff, wt->slots, sel, nu, x, w, clamp, bm));
+  ILT_TRY((hipError_t)gemv_experts(stream, ILT_IQ2_XXS, d, ff, grb, 0, wt->gate_bytes, 0, ff, wt->slots, nu, nullptr, nullptr, nullptr, x, w, clamp, bm, sel,
+                                   nullptr, nullptr, nullptr, once));
   ILT_TRY((hipError_t)step_mark(stream));
-  ILT_TRY((hipError_t)ilt_d4_mv_q2_k_f32(stream, ff, d, drb, 2 * wt->gate_bytes, ff, d, wt->slots, sel, nu, bm, bd));
+  ILT_TRY((hipError_t)gemv_experts(stream, ILT_Q2_K, ff, d, drb, 2 * wt->gate_bytes, -1, ff, d, wt->slots, nu, nullptr, nullptr, nullptr, bm, nullptr, 0.0f, bd,
+                                   sel, nullptr, nullptr, nullptr, once));
   ILT_TRY((hipError_t)step_mark(stream));
   // the shared expert's down product last, adding the routed experts' rows and its own as it stores them; where
   // that launch cannot (more than eight slots, a matrix too small for the streamed variant): the product, then the sum
-  int e = shared_down_sum(stream, d, ff, wt->sdown_q, wt->sdown_d, smid, bd, nu, moe);
+  int e = shared_down_sum(stream, d, ff, wt->sdown_q, wt->sdown_d, smid, bd, nu, moe, once);
   if (e == (int)hipErrorNotSupported) {
     ilt_mv_desc down = {ILT_Q8_0, d, wt->sdown_q, wt->sdown_d, sout, nullptr};
     ILT_TRY((hipError_t)ilt_mv_multi(stream, 1, &down, ff, nullptr, nullptr, nullptr, smid, 0, 0, 0));
