@@ -53,6 +53,14 @@ __device__ __forceinline__ float4 lds_f4(const float* p) {
 
 template <int FMT> struct RegW;
 
+// ilt_g2lds16 as the compiler does not see it: behind the one that it does see it waits for every load in flight before it reads
+// LDS again, and the kernel waits for its loads itself.  (Not so behind the buffer loads, which want addresses of whole dwords.)
+__device__ __forceinline__ void g2lds16_untracked(const void* src, void* dst) {
+  u32 m0;                                            // (the compiler's, put back)
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+               : "=&s"(m0) : "v"(src), "s"(__builtin_amdgcn_readfirstlane((u32)(uintptr_t)(ILT_LDS void*)dst)) : "memory");
+}
+
 template <> struct RegW<ILT_Q4_K> {
   static constexpr int BLOCK = 144;
   static constexpr bool MINS = true;
@@ -221,21 +229,24 @@ struct RegWQ2KHalf : RegW<ILT_Q2_K> {
 // times the arithmetic, which is what groups of a few tokens would wait for.
 // In LDS: a row's 64 bytes of indices and signs, piece p of row r at p ^ (r >> 2 & 3), and behind them 16 bytes with its d.
 __device__ const u64 iq2_grid_reg[256] = { ILT_IQ2XXS_GRID_VALUES };
-__device__ __forceinline__ u64* iq2_tables() {       // the codebook, and the byte masks of the 128 sign patterns
-  __shared__ u64 tab[384];
+// Four bytes an entry: a nibble a weight (weight k < 4 in byte k's low one, 4 + k in its high one), of the codebook which of the
+// three magnitudes it is, of the 128 sign patterns 4 where it is negative; together the selector of a byte permutation.
+__device__ __forceinline__ u32* iq2_tables() {
+  __shared__ u32 tab[384];
   return tab;
 }
 __device__ __forceinline__ void iq2_tables_load(int t, int threads) {       // a barrier follows
-  u64* const tab = iq2_tables();
+  u32* const tab = iq2_tables();
   for (int i = t; i < 384; i += threads) {
-    u64 v;
-    if (i < 256) v = iq2_grid_reg[i];
-    else {
+    u32 v;
+    if (i < 256) {
+      const u64 g = iq2_grid_reg[i];
+      v = ((u32)(g >> 4) & 0x03030303u) | ((u32)(g >> 32) & 0x30303030u);
+    } else {
       const u32 s = (u32)(i - 256) | ((u32)(__popc(i - 256) & 1) << 7);
-      u32 m[2] = {0, 0};
+      v = 0;
 #pragma unroll
-      for (int j = 0; j < 8; j++) m[j >> 2] |= (s >> j) & 1 ? 0xFFu << (8 * (j & 3)) : 0u;
-      v = (u64)m[0] | ((u64)m[1] << 32);
+      for (int j = 0; j < 4; j++) v |= (((s >> j) & 1) << (8 * j + 2)) | (((s >> (4 + j)) & 1) << (8 * j + 6));
     }
     tab[i] = v;
   }
@@ -244,24 +255,20 @@ template <> struct RegW<ILT_IQ2_XXS> {
   static constexpr int BLOCK = 66;
   static constexpr bool MINS = false;
   static constexpr int PLANES = 0, SH = 0;           // PLANES 0: a group's sums scaled by the lanes
-  struct Block { u32 sc; float d, dm; v8h mins; };   // the groups' scales, four bits each
-  struct Quants { int4 q[2]; int2 mag[2], neg[2]; };
+  struct Block { int k[8]; float d, dm; v8h mins; };  // the groups' scales
+  struct Quants { int4 q[2]; u32 sel[2]; };
   static constexpr int LOADS = 3, LBYTES = 3072;
-  struct At { u32 a[2], h; };
-  // (the blocks are two-byte aligned; a row past the matrix's is its last one)
-  static __device__ __forceinline__ At place(u32 row_bytes, int lane, int row0, int rows) {
-    At o;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-      o.a[i] = (u32)min(row0 + 16 * i + (lane >> 2), rows - 1) * row_bytes + 2 + 16 * (u32)((lane & 3) ^ ((lane >> 4) & 3));
-    o.h = (u32)min(row0 + (lane & 31), rows - 1) * row_bytes;
-    return o;
-  }
-  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t, const u8* w, const At& at, u32, u32, u32 block, u8* dst) {
-    ilt_g2lds16(w + (size_t)block + (i < 2 ? at.a[i] : at.h), dst + 1024 * i);
+  struct At { int lane, row0, rows; };
+  static __device__ __forceinline__ At place(u32, int lane, int row0, int rows) { return At{lane, row0, rows}; }
+  // (the blocks are two-byte aligned; a row past the matrix's is its last one; the offsets made each time: kept, they are in
+  // scratch memory, whose reads wait for the loads before them)
+  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t, const u8* w, const At& at, u32 row_bytes, u32, u32 block, u8* dst) {
+    u32 lane = (u32)at.lane;
+    asm volatile("" : "+v"(lane));
+    const u32 r = i < 2 ? 16 * i + (lane >> 2) : lane & 31, o = i < 2 ? 2 + 16 * ((lane & 3) ^ ((lane >> 4) & 3)) : 0;
+    g2lds16_untracked(w + (size_t)block + (u32)min(at.row0 + (int)r, at.rows - 1) * row_bytes + o, dst + 1024 * i);
   }
   static __device__ __forceinline__ void block(Block& o, const u8* src, int l32, int) {
-    o.sc = 0;
     o.d = ilt_h2f(*ILT_LDS_PTR(const u16, src + 2048 + 16 * l32));
   }
   static __device__ __forceinline__ void quants(Quants& o, const u8* src, int g, int l32, int) {
@@ -271,23 +278,18 @@ template <> struct RegW<ILT_IQ2_XXS> {
   static __device__ __forceinline__ u32 sign_word(const Quants& r, int g) { return wordr(r.q[(g >> 1) & 1], 2 * (g & 1) + 1); }
   // the table entries of the lane's two runs of eight weights
   static __device__ __forceinline__ void quants_now(Quants& o, const u8*, int g, int, int lh) {
-    const u64* const tab = iq2_tables();
+    const u32* const tab = iq2_tables();
     const u32 idx = index_word(o, g) >> (16 * lh), sg = sign_word(o, g) >> (14 * lh);
 #pragma unroll
-    for (int l = 0; l < 2; l++) {
-      o.mag[l] = ilt_lds_ld8(tab + ((idx >> (8 * l)) & 0xFF));
-      o.neg[l] = ilt_lds_ld8(tab + 256 + ((sg >> (7 * l)) & 127));
-    }
+    for (int l = 0; l < 2; l++) o.sel[l] = *ILT_LDS_PTR(const u32, tab + ((idx >> (8 * l)) & 0xFF)) | *ILT_LDS_PTR(const u32, tab + 256 + ((sg >> (7 * l)) & 127));
   }
   static __device__ __forceinline__ void group(Block& b, const Quants& r, int g, int, v4i&, v4i& lo) {
-    b.sc |= (sign_word(r, g) >> 28) << (4 * g);
+    b.k[g] = (int)((sign_word(r, g) >> 27) | 1);
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const u32 m = (u32)(k & 1 ? r.neg[k >> 1].y : r.neg[k >> 1].x), v = (u32)(k & 1 ? r.mag[k >> 1].y : r.mag[k >> 1].x);
-      lo[k] = (int)((v ^ m) + (m & 0x01010101u));    // (no entry is zero: no carry between the bytes)
-    }
+    for (int k = 0; k < 4; k++)                      // 8, 25, 43 and what they are negated
+      lo[k] = (int)__builtin_amdgcn_perm(0x00D5E7F8u, 0x002B1908u, (k & 1 ? r.sel[k >> 1] >> 4 : r.sel[k >> 1]) & 0x07070707u);
   }
-  static __device__ __forceinline__ int scale(const Block& b, int g) { return (int)(2 * ((b.sc >> (4 * g)) & 15) + 1); }
+  static __device__ __forceinline__ int scale(const Block& b, int g) { return b.k[g]; }
 };
 
 template <int TN, int RAW, bool MINS, int XB = 1> struct RegSmem {
