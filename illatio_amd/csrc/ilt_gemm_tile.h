@@ -91,7 +91,7 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[NA][NB], const BfPa
 // Which tile a workgroup takes: row tile rt, tokens tok0 .. tok0+ntok-1 (of expert z's group,
 // with w its matrix, when grouped).  Tiles are numbered so that the eight XCDs' workgroups (the
 // hardware deals them round-robin) each walk a contiguous run, GR row tiles of one token tile
-// after another.  False: none (the grid is rounded up).  S: scan[256], tile_z, tile_t0, tile_n.
+// after another.  False: none (the grid is rounded up).
 // (dense) tile number s of the NT x NR: its row tile and its first token
 __device__ __forceinline__ void tile_place(int s, int NT, int NR, int& rt, int& tt) {
   const int rg = s / (GR * NT), rem = s - rg * GR * NT, nr = min(GR, NR - rg * GR);
@@ -99,22 +99,34 @@ __device__ __forceinline__ void tile_place(int s, int NT, int NR, int& rt, int& 
   rt = rg * GR + (rem - tt * nr);
 }
 
-// LIMIT >= 0: only the tiles before it are dealt out (a multiple of 8; the workgroups from it on take parts of the rest)
-template <int TM, int TN, typename SM>
-__device__ __forceinline__ bool pick_tile(const BfParams& p, SM& S, long& tok0, int& ntok, int& rt, const u8*& w, int limit = -1) {
-  const int t = threadIdx.x;
-  const int NR = (p.rows + TM - 1) / TM;
+// lane i: the sum of lanes 0 .. i
+__device__ __forceinline__ u32 wave_sums_upto(u32 v) {
+  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);      // row_shr 1, 2, 4, 8
+  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);
+  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);
+  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);
+  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);      // row_bcast 15 to rows 1 and 3
+  return v + (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);      // row_bcast 31 to rows 2 and 3
+}
+
+// LIMIT >= 0: only the tiles before it are dealt out (a multiple of 8; the workgroups from it on take parts of the rest).
+// Grouped: every wave adds up the groups' tiles by itself, four groups a lane (up to 256), without LDS or a barrier: the scan
+// through LDS took 17 barriers, some 2 us of every workgroup's time, those with no tile (two of three) included (24 tokens, 6 of
+// 256 experts, 4,096 x 2,048: Q2_K's down product 44.5 -> 31.3 us, IQ2_XXS's gate and up 87 -> 78).
+template <int TM, int TN>
+__device__ __forceinline__ bool pick_tile(const BfParams& p, long& tok0, int& ntok, int& rt, const u8*& w, int limit = -1) {
+  const int NR = (p.rows + TM - 1) / TM, lane = threadIdx.x & 63;
   int NT;
+  u32 n[4], upto = 0;                                  // grouped: the lane's four counts; the tiles of its groups and those before
   if (p.ptrs) {
-    if (t < 256) S.scan[t] = t < p.ne ? (p.counts[t] + TN - 1) / TN : 0;
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-      const u32 v = (t < 256 && t >= off) ? S.scan[t - off] : 0;
-      __syncthreads();
-      if (t < 256) S.scan[t] += v;
-      __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int z = 4 * lane + k;
+      n[k] = z < p.ne ? p.counts[z] : 0;
+      upto += (n[k] + TN - 1) / TN;
     }
-    NT = (int)S.scan[255];
+    upto = wave_sums_upto(upto);
+    NT = (int)__builtin_amdgcn_readlane(upto, 63);
   } else {
     NT = (p.ntok + TN - 1) / TN;
   }
@@ -125,17 +137,21 @@ __device__ __forceinline__ bool pick_tile(const BfParams& p, SM& S, long& tok0, 
   int tt;
   tile_place(s, NT, NR, rt, tt);
   if (p.ptrs) {
-    if (t < p.ne) {
-      const u32 incl = S.scan[t], tiles = (p.counts[t] + TN - 1) / TN, excl = incl - tiles;
-      if ((u32)tt >= excl && (u32)tt < incl) {
-        S.tile_z = t;
-        S.tile_t0 = (int)(p.bases[t] + ((u32)tt - excl) * TN);
-        S.tile_n = (int)min((u32)TN, p.counts[t] - ((u32)tt - excl) * TN);
+    // the lane whose groups the tile is among, then which of the four
+    const int l = __builtin_ctzll(__ballot(upto > (u32)tt));
+    u32 z = 4 * l, c = 0, first = l ? (u32)__builtin_amdgcn_readlane(upto, l - 1) : 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const u32 ck = (u32)__builtin_amdgcn_readlane(n[k], l), tiles = (ck + TN - 1) / TN;
+      if (c == 0) {                                    // (not found yet)
+        if ((u32)tt < first + tiles) { z = 4 * l + k; c = ck; }
+        else first += tiles;
       }
     }
-    __syncthreads();
-    tok0 = S.tile_t0; ntok = S.tile_n;
-    w = (const u8*)(p.ptrs[S.tile_z] + p.add);
+    const u32 skip = ((u32)tt - first) * TN;
+    tok0 = (long)(p.bases[z] + skip);
+    ntok = (int)min((u32)TN, c - skip);
+    w = (const u8*)(p.ptrs[z] + p.add);
   } else {
     tok0 = (long)tt * TN;
     ntok = min(TN, p.ntok - (int)tok0);

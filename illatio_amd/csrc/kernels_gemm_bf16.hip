@@ -35,6 +35,7 @@
 #include "ilt_iq2xxs_tables.h"
 #include "ilt_kernels.h"
 #include <stdlib.h>
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -194,8 +195,6 @@ template <int TM, int TN, int NXS, int NWS> struct Smem {
   __align__(16) u8 xs[NXS][TN * KS * 2];
   __align__(16) u8 ws[NWS][TM * KS * 2];
   Iq2Tables iq2;
-  u32 scan[256];
-  int tile_z, tile_t0, tile_n;
 };
 
 // Piece p (16 bytes) of row r of a slab.  Rows are 64 bytes, so 8 consecutive rows span 128
@@ -233,7 +232,7 @@ __global__ __launch_bounds__((bf16_threads<TM, NB>()), (TM * TN == 65536 ? 1 : T
     ntok = min(TN, p.ntok - (int)tok0);
     sb0 = (int)((long)ky * sb1 / p.ksplit);
     sb1 = (int)((long)(ky + 1) * sb1 / p.ksplit);
-  } else if (!pick_tile<TM, TN>(p, S, tok0, ntok, rt, w, p.ksplit > 1 ? p.split_from : -1)) return;
+  } else if (!pick_tile<TM, TN>(p, tok0, ntok, rt, w, p.ksplit > 1 ? p.split_from : -1)) return;
   const int r0 = rt * TM;
   if (FMT == ILT_IQ2_XXS) {
     if (t < 256) iq2_tables_fill(S.iq2, t);
@@ -484,11 +483,10 @@ template <> struct RegB<ILT_Q2_K> {
   }
 };
 
-struct TileSel { u32 scan[256]; int tile_z, tile_t0, tile_n, pad; };
 
-// dynamic LDS: the x ring, the two buffers of blocks, the tile choice's scratch, IQ2_XXS's tables
+// dynamic LDS: the x ring, the two buffers of blocks, IQ2_XXS's tables
 template <int FMT> constexpr size_t regb_smem() {
-  return 3 * 128 * KS * 2 + 2 * 256 * RegB<FMT>::LB + sizeof(TileSel) + (FMT == ILT_IQ2_XXS ? sizeof(Iq2Tables) : 0);
+  return 3 * 128 * KS * 2 + 2 * 256 * RegB<FMT>::LB + (FMT == ILT_IQ2_XXS ? sizeof(Iq2Tables) : 0);
 }
 
 // GLU: the tile's 256 rows are 128 rows of the gate matrix and the same 128 of the up matrix,
@@ -507,12 +505,11 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_regb_kernel(BfParams p) {
   extern __shared__ __align__(16) u8 regb_lds[];
   u8* const xsl = regb_lds;                                  // [3][XS]
   u8* const wsl = regb_lds + 3 * XS;                         // [2][WS]
-  TileSel& S = *(TileSel*)(regb_lds + 3 * XS + 2 * WS);
-  const Iq2Tables* T = (const Iq2Tables*)(regb_lds + 3 * XS + 2 * WS + sizeof(TileSel));
+  const Iq2Tables* T = (const Iq2Tables*)(regb_lds + 3 * XS + 2 * WS);
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
 
   long tok0; int ntok, rt; const u8* w = p.w;
-  if (!pick_tile<TR, TN>(p, S, tok0, ntok, rt, w)) return;
+  if (!pick_tile<TR, TN>(p, tok0, ntok, rt, w)) return;
   const int r0 = rt * TR;
   if (FMT == ILT_IQ2_XXS) iq2_tables_fill(*(Iq2Tables*)T, t);     // (a barrier follows, before the first operands are made)
 
@@ -820,8 +817,6 @@ template <int NB> struct I8ppSmem {
   __align__(16) u8 wl[RING][128 * 64];
   float wd[128], xd[128];                 // of the super-block: d of the rows, the tokens' scales
   int cx[128];                            //   and 4000 * the sum of their quants
-  u32 scan[256];
-  int tile_z, tile_t0, tile_n, pad;
 };
 
 template <int NB>
@@ -834,7 +829,7 @@ __global__ __launch_bounds__(512 / NB, 2) void gemm_i8pp_kernel(BfParams p) {
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
 
   long tok0; int ntok, rt; const u8* w = p.w;
-  if (!pick_tile<TM, TN>(p, S, tok0, ntok, rt, w)) return;
+  if (!pick_tile<TM, TN>(p, tok0, ntok, rt, w)) return;
   const int r0 = rt * TM;
   const int nk = p.cols / KW, nsb = p.cols / 256;
 
@@ -1357,13 +1352,13 @@ hipError_t ilt_k_gemm_bf16_id(int fmt, const uint64_t* ptrs, long long add, cons
   const int forced = force ? atoi(force) : 0;
   if (rows % 256 == 0 && forced == 0 && (fmt == ILT_IQ2_XXS || fmt == ILT_Q2_K)) {      // weights straight into MFMA operands
     if ((long long)rows * row_bytes >= 0x7FFFFFFFLL || row_bytes >= (1 << 24)) return hipErrorInvalidValue;      // the kernel's 32- and 24-bit address arithmetic
-    return fmt == ILT_IQ2_XXS ? launch_regb<ILT_IQ2_XXS, false>(p, total_rows / 128 + ne, st) : launch_regb<ILT_Q2_K, false>(p, total_rows / 128 + ne, st);
+    return fmt == ILT_IQ2_XXS ? launch_regb<ILT_IQ2_XXS, false>(p, total_rows / 128 + std::min<long long>(ne, total_rows), st) : launch_regb<ILT_Q2_K, false>(p, total_rows / 128 + std::min<long long>(ne, total_rows), st);
   }
   if (rows % 256 == 0 && forced != 1) {      // the expert formats (Q4_K / Q6_K raw sets would not fit the registers)
-    if (fmt == ILT_IQ2_XXS) return launch_bf16<ILT_IQ2_XXS, 256, 128, 4>(p, total_rows / 128 + ne, st);
-    if (fmt == ILT_Q2_K) return launch_bf16<ILT_Q2_K, 256, 128, 4>(p, total_rows / 128 + ne, st);
+    if (fmt == ILT_IQ2_XXS) return launch_bf16<ILT_IQ2_XXS, 256, 128, 4>(p, total_rows / 128 + std::min<long long>(ne, total_rows), st);
+    if (fmt == ILT_Q2_K) return launch_bf16<ILT_Q2_K, 256, 128, 4>(p, total_rows / 128 + std::min<long long>(ne, total_rows), st);
   }
-  return dispatch_bf16<128, 128, 2>(fmt, p, total_rows / 128 + ne, st);
+  return dispatch_bf16<128, 128, 2>(fmt, p, total_rows / 128 + std::min<long long>(ne, total_rows), st);
 }
 
 hipError_t ilt_k_gemm_bf16_id_glu(int fmt, const uint64_t* ptrs, long long add_gate, long long add_up, const uint32_t* counts,
@@ -1379,7 +1374,7 @@ hipError_t ilt_k_gemm_bf16_id_glu(int fmt, const uint64_t* ptrs, long long add_g
   p.ptrs = ptrs; p.add = add_gate; p.up_delta = (unsigned)(add_up - add_gate); p.counts = counts; p.bases = bases; p.ne = ne;
   p.rows = rows; p.cols = cols; p.row_bytes = row_bytes; p.x = xb; p.rmap = rmap; p.ntok = (int)total_rows;
   p.wrow = wrow; p.clamp = clamp; p.mid = mid;
-  return launch_regb<ILT_IQ2_XXS, true>(p, total_rows / 128 + ne, st);
+  return launch_regb<ILT_IQ2_XXS, true>(p, total_rows / 128 + std::min<long long>(ne, total_rows), st);
 }
 
 hipError_t ilt_k_planes_i8(int fmt, const uint8_t* w, long long row_bytes, int rows, int cols, uint8_t* wh, uint8_t* wl, float* wdf,

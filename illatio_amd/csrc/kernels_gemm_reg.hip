@@ -30,6 +30,7 @@
 #include "ilt_iq2xxs_tables.h"
 #include "ilt_kernels.h"
 #include <stdlib.h>
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -561,15 +562,13 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
   store_tile<NP, 1>(sum, p, tok0, ntok, r0, wt0, wr0, l32, lh);
 }
 
-struct NoScan { u32 scan[1]; int tile_z, tile_t0, tile_n; };      // (tiles of groups only)
-
 // FSET: the matrices' format, or 0 where Q4_K and Q6_K meet in a launch
 template <int FSET, int NP, int WR, int WT>
 __global__ __launch_bounds__(64 * WR * WT, WR * WT == 1 ? 1 : 2) void gemm_i8r_kernel(BfParams p) {
   constexpr int TM = 32 * WR, TN = 32 * NP * WT;
   extern __shared__ __align__(16) unsigned char smem[];
   long tok0; int ntok, rt; const u8* w = p.w;
-  if (!pick_tile<TM, TN>(p, *(NoScan*)smem, tok0, ntok, rt, w)) return;
+  if (!pick_tile<TM, TN>(p, tok0, ntok, rt, w)) return;
   // which of the launch's matrices the row tile belongs to
   const int n0 = (p.mrows[0] + TM - 1) / TM, n1 = n0 + (p.mrows[1] + TM - 1) / TM;
   const int m = rt < n0 ? 0 : rt < n1 ? 1 : 2;
@@ -613,19 +612,16 @@ hipError_t launch_i8r(BfParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
-struct GroupScan { u32 scan[256]; int tile_z, tile_t0, tile_n; };
-
 // The experts' products: token tiles of every expert's rows in turn, 128 rows of the expert's matrix (of two, one behind the
 // other in the output: gate and up) a workgroup.  A group of up to 32 (64) rows goes as one (two) patches of 32.
 template <int FMT>
 __global__ __launch_bounds__(256, 2) void gemm_i8r_group_kernel(BfParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ GroupScan scan;
-  if constexpr (FMT == ILT_IQ2_XXS) iq2_tables_load(threadIdx.x, 256);
   long tok0; int ntok, rt; const u8* w;
   const int rows = p.rows, nr = (rows + 127) / 128;
   if (p.nmulti > 1) p.rows = 2 * nr * 128;
-  if (!pick_tile<128, 128>(p, scan, tok0, ntok, rt, w)) return;       // (barriers inside)
+  if (!pick_tile<128, 128>(p, tok0, ntok, rt, w)) return;
+  if constexpr (FMT == ILT_IQ2_XXS) { iq2_tables_load(threadIdx.x, 256); __syncthreads(); }
   p.rows = rows;
   if (rt >= nr) { rt -= nr; w += p.up_delta; p.y = p.my[1]; }
   ntok = __builtin_amdgcn_readfirstlane(ntok);
@@ -650,8 +646,8 @@ hipError_t launch_i8r_group(const BfParams& p, long long total_rows, hipStream_t
     if (e != hipSuccess) return e;
     attr_set[dev] = true;
   }
-  // sum over experts of ceil(count / 128) <= total / 128 + ne
-  const long long total = (total_rows / 128 + p.ne) * ((p.rows + 127) / 128) * p.nmulti, per = (total + 7) / 8;
+  // sum over experts of ceil(count / 128) <= total / 128 + those with a row
+  const long long total = (total_rows / 128 + std::min<long long>(p.ne, total_rows)) * ((p.rows + 127) / 128) * p.nmulti, per = (total + 7) / 8;
   if (per * 8 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
   hipLaunchKernelGGL(gemm_i8r_group_kernel<FMT>, dim3((unsigned)(per * 8)), dim3(256), smem, st, p);
   return hipGetLastError();

@@ -104,6 +104,34 @@ def test_groups_bit_for_bit(dev, qtype, rows, cols):
         hip.hip_free(b)
 
 
+# which expert and which of its rows a workgroup takes: as many experts as a launch has and a number that is no multiple of four,
+# most without rows, the first and the last with some, whole tiles and a row more
+@pytest.mark.parametrize("ne,some", [(256, [0, 3, 4, 63, 64, 127, 200, 255]), (253, [2, 7, 128, 252]), (5, [4]), (3, [0])])
+def test_groups_far_apart_bit_for_bit(dev, ne, some):
+    from illatio_amd import hip, ds4f
+    rng = synth.make_rng(ne)
+    rows, cols = 128, 256
+    counts = np.zeros(ne, np.uint32)
+    counts[some] = [(1, 129, 128, 257)[i % 4] for i in range(len(some))]
+    total = int(counts.sum())
+    bases = (np.cumsum(counts) - counts).astype(np.uint32)
+    rb = synth.row_bytes(synth.Q2_K, cols)
+    w = synth.weights(synth.Q2_K, 3 * rows, cols, rng).reshape(3, rows, rb)
+    x = synth.activations((total, cols), rng)
+    wb, xb, y = hip.hip_upload_new(dev, w), hip.hip_upload_new(dev, x), hip.hip_alloc(dev, 4 * total * rows)
+    ptrs = hip.hip_upload_new(dev, np.array([wb.ptr + z % 3 * rows * rb for z in range(ne)], np.uint64))
+    cb, bb = hip.hip_upload_new(dev, counts), hip.hip_upload_new(dev, bases)
+    xq, xd, xs = ds4f._q8k(dev, xb, total * cols)
+    hip.launch(dev, "d4_mm_id_q2_k", (1, 1, ne), 128, [cols, rows, rb, cols, rows, hip.I64(0), ptrs, cb, bb, xq, y, xd, xs, hip.I64(total)])
+    got = hip.hip_floats(y, total * rows).reshape(total, rows)
+    for z in some:
+        at = slice(int(bases[z]), int(bases[z] + counts[z]))
+        want = orc.matmul(synth.Q2_K, w[z % 3], rows, cols, x[at], nthreads=8).reshape(-1, rows)
+        assert np.array_equal(bits(got[at]), bits(want)), (z, np.argwhere(bits(got[at]) != bits(want))[:5])
+    for b in (wb, xb, y, ptrs, cb, bb, xq, xd, xs):
+        hip.hip_free(b)
+
+
 # experts' matrices on two-byte boundaries: by the slot's address, by the offset into it, and both (together a multiple of four)
 @pytest.mark.parametrize("rows,cols", [(128, 256), (161, 1280)])
 @pytest.mark.parametrize("at,add", [(2, 0), (0, 2), (2, 2), (6, 8)])
