@@ -154,22 +154,55 @@ __global__ __launch_bounds__(64 * WR * WT, OCC) void gemm_q8_kernel(Q8Params p) 
         dx[4 * g] = __int_as_float(d4.x); dx[4 * g + 1] = __int_as_float(d4.y); dx[4 * g + 2] = __int_as_float(d4.z); dx[4 * g + 3] = __int_as_float(d4.w);
       }
     };
+    if constexpr (RP * TP == 1) {                    // one patch a wave: a block's operands as they are wanted (all of them first: 3 % slower)
 #pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      O wv[RP];
-#pragma unroll
-      for (int b = 0; b < RP; b++) wv[b] = Q8Acc<MS>::load(cur + roff[b][kk]);
-#pragma unroll
-      for (int a = 0; a < TP; a++) {
-        const O xv = Q8Acc<MS>::load(cur + toff[a][kk]);
+      for (int kk = 0; kk < KB; kk++) {
+        const O wv = Q8Acc<MS>::load(cur + roff[0][kk]), xv = Q8Acc<MS>::load(cur + toff[0][kk]);
         float dx[NR];
-        load_dx(a, kk, dx);
+        load_dx(0, kk, dx);
+        const vi d = Q8Acc<MS>::mul(xv, wv, magic);
 #pragma unroll
-        for (int b = 0; b < RP; b++) {
-          const vi d = Q8Acc<MS>::mul(xv, wv[b], magic);
+        for (int i = 0; i < NR; i++) sum[0][0][i] = sum[0][0][i] + (__int_as_float(d[i]) - 12582912.0f) * (dw[0][kk] * dx[i]);
+      }
+    } else {
+      // a patch's products are made while the one before it is scaled and added, four results side by side: one after another every
+      // instruction waited for the one before it (4096 x 4096 on 1,000 tokens: tiles of 64 x 64 90.8 -> 84.4 us, on 100, where a CU has
+      // one of them, 44.4 -> 33.2; of 128 x 128 98 -> 90)
+      constexpr int N = KB * TP * RP;
+      O wv[KB][RP], xv[KB][TP];
 #pragma unroll
-          for (int i = 0; i < NR; i++) sum[a][b][i] = sum[a][b][i] + (__int_as_float(d[i]) - 12582912.0f) * (dw[b][kk] * dx[i]);
+      for (int kk = 0; kk < KB; kk++) {
+#pragma unroll
+        for (int b = 0; b < RP; b++) wv[kk][b] = Q8Acc<MS>::load(cur + roff[b][kk]);
+#pragma unroll
+        for (int a = 0; a < TP; a++) xv[kk][a] = Q8Acc<MS>::load(cur + toff[a][kk]);
+      }
+      float dx[2][NR];
+      load_dx(0, 0, dx[0]);
+      vi d[2];
+      d[0] = Q8Acc<MS>::mul(xv[0][0], wv[0][0], magic);
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        const int kk = k / (TP * RP), a = k / RP % TP, b = k % RP, n = k + 1;
+        if (n < N) {
+          if (n % RP == 0) load_dx(n / RP % TP, n / (TP * RP), dx[n / RP & 1]);
+          d[n & 1] = Q8Acc<MS>::mul(xv[n / (TP * RP)][n / RP % TP], wv[n / (TP * RP)][n % RP], magic);
         }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < NR; i += 4) {
+          float u[4], m[4];
+#pragma unroll
+          for (int j = 0; j < 4; j++) { u[j] = __int_as_float(d[k & 1][i + j]) - 12582912.0f; m[j] = dw[b][kk] * dx[k / RP & 1][i + j]; }
+          asm volatile("" : "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]), "+v"(m[0]), "+v"(m[1]), "+v"(m[2]), "+v"(m[3]));
+#pragma unroll
+          for (int j = 0; j < 4; j++) u[j] = u[j] * m[j];
+          asm volatile("" : "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]));
+#pragma unroll
+          for (int j = 0; j < 4; j++) sum[a][b][i + j] = sum[a][b][i + j] + u[j];
+        }
+        asm volatile("" : "+v"(sum[a][b]));
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
     fill = cur;
@@ -214,6 +247,27 @@ hipError_t q8_launch(Q8Params& p, hipStream_t st) {
   return hipGetLastError();
 }
 
+// What a workgroup of each kind of tile takes for 4,096 columns, microseconds, with 1, 2, ... of them on a CU (4,096 rows on 64 to
+// 2,304 tokens): a small tile is the shortest chain of steps, a large one reads LDS less a result.  Workgroups past those that fit
+// take over the places that come free, all but the largest's, which start and end together.  (4096 x 4096 on 1,000 tokens: 128 x 64 68.9
+// us, 64 x 64 84.4; 9728 x 896 on 301 20.2 and 18.7; 4096 x 4096 on 4,096 261, 312, and 230 for 128 x 128.)
+struct Q8Kind { int rows, tokens, fit; float us[5]; };
+constexpr Q8Kind kQ8Tiles[] = {
+  {32, 32, 4, {15.2f, 19.0f, 26.0f, 33.2f}},
+  {64, 64, 5, {33.0f, 43.8f, 65.8f, 84.6f, 102.0f}},
+  {128, 64, 3, {54.5f, 69.2f, 102.0f}},
+  {128, 128, 2, {90.0f, 116.8f}},
+};
+float q8_time(const Q8Kind& c, const Q8Params& p) {
+  long long n = 0;
+  for (int i = 0; i < p.nmat; i++) n += (p.mat[i].rows + c.rows - 1) / c.rows;
+  n *= (p.ntok + c.tokens - 1) / c.tokens;
+  const long long full = 256LL * c.fit, rest = n % full;
+  if (n <= full) return c.us[(n + 255) / 256 - 1];
+  if (c.rows * c.tokens < 128 * 128) return c.us[c.fit - 1] * (float)n / (float)full;
+  return (float)(n / full) * c.us[c.fit - 1] + (rest ? c.us[(rest + 255) / 256 - 1] : 0.0f);
+}
+
 }  // namespace
 
 hipError_t ilt_k_gemm_q8(int nmat, const uint8_t* const* ws, const uint16_t* const* wds, const int* rows, float* const* ys, const float* const* biases,
@@ -221,24 +275,21 @@ hipError_t ilt_k_gemm_q8(int nmat, const uint8_t* const* ws, const uint16_t* con
   if (nmat < 1 || nmat > 4 || ntok < 1 || cols < 64 || cols % 64 || (long long)128 * cols >= 0x7FFFFFFFLL || ((uintptr_t)xq & 15) || ((uintptr_t)xs & 3)) return hipErrorNotSupported;
   Q8Params p = {};
   p.nmat = nmat; p.cols = cols; p.ntok = ntok; p.acc = acc; p.xq = xq; p.xs = xs;
-  long long tiles = 0;
   for (int i = 0; i < nmat; i++) {
     Q8Mat& m = p.mat[i];
     m.w = ws[i]; m.wd = wds[i]; m.y = ys[i]; m.bias = biases ? biases[i] : nullptr; m.rows = rows[i]; m.ldy = ldy ? ldy : rows[i];
     if (rows[i] < 1 || m.ldy < rows[i] || m.ldy * 1024 >= 0x7FFFFFFFLL || ((uintptr_t)ws[i] & 15) || ((uintptr_t)wds[i] & 3)) return hipErrorNotSupported;
-    tiles += (rows[i] + 31) / 32;
   }
-  tiles *= (ntok + 31) / 32;
-  // Which tile, T = the number of 32 x 32 tiles.  Up to 1,300 the time is a wave's chain of steps, shortest with one patch a wave
-  // (steps of 128 columns: half the barriers); past that the chip is full and larger tiles read LDS less a result: a wave of
-  // 32 x 32 up to 5,500, of 64 x 32 from there, and of 64 x 64 where the workgroups fill the places (two a CU, 8,192 tiles a
-  // turn: a turn takes 1.85 us a step of 64 columns against 0.26 us a thousand tiles of the kind before it).
-  // 896 x 4864 on 512 tokens (T = 448) 19.9 us with the smallest, 51.6 with the next; 9728 x 896 on 512 (4,864) 34 / 25.7 / 26.8;
-  // on 1,024 (9,728) 47 / 41 / 56; 4096 x 4096 on 4,096 (16,384) 325 / 269 / 239.
   // ILT_Q8_TILE (tests): 1 to 4, that one.
   const char* const f = getenv("ILT_Q8_TILE");
-  const long long turns = (tiles + 8191) / 8192;
-  int v = f ? atoi(f) : tiles <= 1300 ? 1 : tiles <= 5500 ? 2 : 1850 * turns + 150 < tiles * 26 / 100 ? 4 : 3;
+  int v = f ? atoi(f) : 0;
+  if (v < 1 || v > 4) {
+    float least = 0.0f;
+    for (int k = cols % 128 ? 1 : 0; k < 4; k++) {
+      const float us = q8_time(kQ8Tiles[k], p);
+      if (!v || us < least) { v = k + 1; least = us; }
+    }
+  }
   if (v == 1 && cols % 128) v = 2;
   switch (v) {
     case 1: return q8_launch<16, 1, 1, 2, 2, 4, 4, 4>(p, st);
