@@ -269,9 +269,10 @@ uint64_t ilt_d4_ffn_step_workspace(int nu, int d, int ff);
 int ilt_d4_ffn_step(uint64_t stream, void* ws, uint64_t ws_bytes, int ne, int nu, int d, int ff, float scale, float clamp,
                     const ilt_ffn_step_weights* wt, const float* logits, const float* bias, const float* x, float* moe);
 /* The same for a short pass's n <= 9 tokens (DK-FFN-SMALL, cuda-ds4f-spec.lisp:30-100: a speculative step's verification):
-   logits n x ne, x n x d, moe n x d, every token with ilt_d4_ffn_step's bits.  Eight launches on stream: the routing and the
-   rows' order by expert, the shared expert's quantizer, gate and up, gated activation and down (its matrices read once for
-   all the tokens), the routed experts' gate/up/activation and down over the n * nu (token, slot) rows, the sums.  Nothing is
+   logits n x ne, x n x d, moe n x d, every token with ilt_d4_ffn_step's bits.  Seven launches on stream: the routing, the
+   rows' order by expert and the tokens quantized, the shared expert's gate and up and its down (its matrices read once for all
+   the tokens), the routed experts' gate/up/activation and down over the n * nu (token, slot) rows (an expert's blocks decoded
+   once for up to three), the gated activations quantized, the sums; nine where d or ff is past 4096.  Nothing is
    allocated, freed or waited for; ws as above, ilt_d4_ffn_small_workspace bytes. */
 uint64_t ilt_d4_ffn_small_workspace(int n, int nu, int d, int ff);
 int ilt_d4_ffn_small(uint64_t stream, void* ws, uint64_t ws_bytes, int n, int ne, int nu, int d, int ff, float scale, float clamp,
