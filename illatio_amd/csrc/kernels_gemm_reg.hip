@@ -55,8 +55,8 @@ __device__ __forceinline__ float4 lds_f4(const float* p) {
 template <int FMT> struct RegW;
 
 // ilt_g2lds16 as the compiler does not see it: behind the one that it does see it waits for every load in flight before it reads
-// LDS again, and the kernel waits for its loads itself (6 of 256 experts, 1,000 tokens: IQ2_XXS's gate and up 550 -> 505 us, 475 with
-// the tables of 4 bytes an entry).  Not so behind the buffer loads, which want addresses of whole dwords.
+// LDS again, and the kernel waits for its loads itself (6 of 256 experts, 1,000 tokens: IQ2_XXS's gate and up 550 -> 475 us, the
+// tables of 4 bytes an entry included).  Not so behind the buffer loads, which want addresses of whole dwords.
 __device__ __forceinline__ void g2lds16_untracked(const void* src, void* dst) {
   u32 m0;                                            // (the compiler's, put back)
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
