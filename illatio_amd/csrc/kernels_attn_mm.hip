@@ -15,6 +15,7 @@
 // t * group + g -- go through in tiles of 16 (or 4), whatever heads they are of.
 #include "ilt_device.h"
 #include "ilt_kernels.h"
+#include "ilt_value_sets.h"
 #include <type_traits>
 
 namespace {
@@ -118,38 +119,48 @@ __global__ __launch_bounds__(256, R == 16 ? 4 : 2) void attn_values_mm_kernel(co
   if (r0 >= rows) return;
   const int t0 = r0 / group, t1 = min(r0 + R - 1, rows - 1) / group;
   const int npos0 = pos0 + t0 + 1, nposmax = pos0 + t1 + 1;
-  // (through buffer loads: a set's values are one vector offset and scalar ones that never change; what lies past the last
-  // position or in the next row is never added)
+  // (through buffer loads: a set's values are one vector offset and scalar ones that never change, all of them within the cache
+  // -- ilt_value_sets.h --, since how a buffer load's range check counts a scalar offset the public descriptions do not agree on.
+  // The scores' whole offset is in the vector part: what lies past the tile's last row is zero, what lies past a row's last
+  // position or in the next row is never added.)
   const __amdgpu_buffer_rsrc_t rs = ilt_rsrc(ilt_uniform_ptr(prob + ((long long)t0 * nh + kvh * group) * spitch), (u32)((t1 - t0) * nh + group) * (u32)spitch * 4u);
   const __amdgpu_buffer_rsrc_t rv = ilt_rsrc(ilt_uniform_ptr(vc), (u32)nposmax * (u32)kvd * 4u);
   const int srow = min(r0 + (lane & (R - 1)), rows - 1), st = srow / group;
   const u32 so = ((u32)((st - t0) * nh + srow - st * group) * (u32)spitch + (R == 4 ? (u32)(lane >> 2) : 0u)) * 4u, vo = (u32)(kvh * HD + 64 * cg + lane) * 4u;
   struct Set { float s[M::NS], v[P]; };
+  int ko[P];
+#pragma unroll
+  for (int k = 0; k < P; k++) ko[k] = ilt_set_at(k, nposmax) * kvd * 4;
   auto load = [&](Set& x, int p) {
+    const u32 base = (u32)ilt_set_base(p, P, nposmax);
 #pragma unroll
     for (int k = 0; k < M::NS; k += 4) {
-      if constexpr (R == 4) x.s[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, so + 4u * (u32)p, 0, 0));
+      if constexpr (R == 4) x.s[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, so + 4u * base, 0, 0));
       else {
-        const float4 f = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, so + 4u * (u32)p + 4u * k, 0, 0));
+        const float4 f = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, so + 4u * base + 4u * k, 0, 0));
         x.s[k] = f.x; x.s[k + 1] = f.y; x.s[k + 2] = f.z; x.s[k + 3] = f.w;
       }
     }
-    const u32 pv = vo + (u32)p * (u32)kvd * 4u;
+    const u32 pv = vo + base * (u32)kvd * 4u;
 #pragma unroll
-    for (int k = 0; k < P; k++) x.v[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, pv, k * kvd * 4, 0));
+    for (int k = 0; k < P; k++) x.v[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, pv, ko[k], 0));
   };
   V acc = {};
   int npos[R == 4 ? 4 : 1];                          // R 16: a lane's results are one row's; R 4: its column's in four rows
 #pragma unroll
   for (int r = 0; r < (R == 4 ? 4 : 1); r++) npos[r] = pos0 + (R == 4 ? min(r0 + r, rows - 1) / group : st) + 1;
-  auto set = [&](const Set& x, int p, auto ownc) {   // OWN: rows may end inside these positions
+  auto set = [&](const Set& x, int p, auto ownc) {   // OWN: rows may end inside these positions, and they may lie further down
     constexpr bool OWN = decltype(ownc)::value;
+    const int base = ilt_set_base(p, P, nposmax);
+    u32 left[R == 4 ? 4 : 1];
+#pragma unroll
+    for (int r = 0; r < (R == 4 ? 4 : 1); r++) left[r] = ilt_set_left(p, npos[r]);
     auto mul = [&](auto kc) { constexpr int k = decltype(kc)::value; return M::template mul<k>(x.s, x.v[k]); };
     auto add = [&](const V& d, int k) {
 #pragma unroll
       for (int r = 0; r < R; r++) {
         const float a = acc[r] + d[r];
-        acc[r] = !OWN || p + k < npos[R == 4 ? r : 0] ? a : acc[r];
+        acc[r] = !OWN || ilt_set_from(p, base, k) < left[R == 4 ? r : 0] ? a : acc[r];
       }
       asm volatile("" : "+v"(acc));
     };
@@ -166,25 +177,8 @@ __global__ __launch_bounds__(256, R == 16 ? 4 : 2) void attn_values_mm_kernel(co
     if constexpr (P == 16) { two(integral_constant<int, 8>{}); two(integral_constant<int, 10>{}); two(integral_constant<int, 12>{}); two(integral_constant<int, 14>{}); }
   };
   Set x[AHEAD];
-#pragma unroll
-  for (int u = 0; u < AHEAD; u++) load(x[u], P * u);
-  int p = 0;
-  for (; p + P * AHEAD <= npos0; p += P * AHEAD) {
-#pragma unroll
-    for (int u = 0; u < AHEAD; u++) {
-      set(x[u], p + P * u, std::false_type{});
-      load(x[u], p + P * u + P * AHEAD);
-    }
-  }
-  for (; p < nposmax; p += P * AHEAD) {
-#pragma unroll
-    for (int u = 0; u < AHEAD; u++) {
-      const int pu = p + P * u;
-      if (pu + P <= npos0) set(x[u], pu, std::false_type{});
-      else if (pu < nposmax) set(x[u], pu, std::true_type{});
-      if (pu + P * AHEAD < nposmax) load(x[u], pu + P * AHEAD);
-    }
-  }
+  ilt_value_sets<P, AHEAD>(x, npos0, nposmax, load, [&](const Set& x, int p) { set(x, p, std::false_type{}); },
+                           [&](const Set& x, int p) { set(x, p, std::true_type{}); });
   auto row_out = [&](int row) { return out + ((long long)(row / group) * nh + kvh * group + row % group) * HD + 64 * cg; };
   if constexpr (R == 4) {
 #pragma unroll
