@@ -447,43 +447,32 @@ __device__ __forceinline__ float chain_muladd_from(float o, const float* sc, con
   return o;
 }
 
-// softmax of one token's raw scores into sc (LDS) by the NT threads that call it (me = 0..NT-1): NT = 64, one
-// wave, or the whole workgroup of 256 with red/redd for the waves to meet.  PRE: the thread's raw scores
-// (positions me, me + NT, ..) are in pre already, at most eight of them.
-template <int NT, bool PRE>
-__device__ __forceinline__ void attn_softmax(const float* __restrict__ rw, const float* pre, float* sc, int npos, int me, float* redf, double* redd) {
+// softmax of one token's raw scores into sc (LDS) by a workgroup of 256 threads, red/redd for its waves to meet.  The thread's raw
+// scores (positions me, me + 256, ..) are in pre already, at most eight of them.
+__device__ __forceinline__ void attn_softmax(const float* pre, float* sc, int npos, int me, float* redf, double* redd) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float mx = -3.402823466e38f;
-  if (PRE) {
 #pragma unroll
-    for (int u = 0; u < 8; u++) if (me + NT * u < npos) { sc[me + NT * u] = pre[u]; mx = fmaxf(mx, pre[u]); }
-  } else {
-    for (int p = me; p < npos; p += NT) { const float sv = rw[p]; sc[p] = sv; mx = fmaxf(mx, sv); }
-  }
+  for (int u = 0; u < 8; u++) if (me + 256 * u < npos) { sc[me + 256 * u] = pre[u]; mx = fmaxf(mx, pre[u]); }
   mx = wave_max_float(mx);
-  if (NT > 64) {
-    if (lane == 0) redf[wave] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
-  }
+  if (lane == 0) redf[wave] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
   double part = 0.0;
-  for (int p = me; p < npos; p += NT) { const float e = ilt_expf_via_double(sc[p] - mx); sc[p] = e; part += (double)e; }
+  for (int p = me; p < npos; p += 256) { const float e = ilt_expf_via_double(sc[p] - mx); sc[p] = e; part += (double)e; }
   part = wave_sum_double(part);
-  double sum = part;
-  if (NT > 64) {
-    if (lane == 0) redd[wave] = part;
-    __syncthreads();
-    sum = (redd[0] + redd[1]) + (redd[2] + redd[3]);
-  }
+  if (lane == 0) redd[wave] = part;
+  __syncthreads();
+  const double sum = (redd[0] + redd[1]) + (redd[2] + redd[3]);
   // the CPU adds the terms one after another: take its sum where the order could show in the rounded reciprocal
   float inv;
-  if (!recip_settled(sum, npos, &inv)) {           // the same in all NT threads
-    if (NT > 64) __syncthreads();
-    if (me == 0) { double s2 = 0.0; for (int p = 0; p < npos; p++) s2 += (double)sc[p]; redd[NT > 64 ? 0 : 4 + wave] = s2; }
-    if (NT > 64) __syncthreads();
-    inv = (float)(1.0 / redd[NT > 64 ? 0 : 4 + wave]);
+  if (!recip_settled(sum, npos, &inv)) {           // the same in all threads
+    __syncthreads();
+    if (me == 0) { double s2 = 0.0; for (int p = 0; p < npos; p++) s2 += (double)sc[p]; redd[0] = s2; }
+    __syncthreads();
+    inv = (float)(1.0 / redd[0]);
   }
-  for (int p = me; p < npos; p += NT) sc[p] = sc[p] * inv;
+  for (int p = me; p < npos; p += 256) sc[p] = sc[p] * inv;
 }
 
 // A prompt chunk's softmax, once a (head, token): the raw scores of row (t, h) become the scaled scores, in place.  NT threads a
@@ -596,8 +585,8 @@ hipError_t launch_softmax(float* raw, int nh, int pos0, int ntok, int spitch, hi
 // slice with the positions along a row, vt[c * vpitch + p] (vpitch = 4 mod 64: sixteen threads' 16-byte reads
 // of sixteen rows fall on different banks).  NB: the slice is at most NB * 2048 16-byte pieces (512 NB positions).
 // With one token a workgroup the slice is stored times that token's scores, by all threads, and the chains add.
-// PROB: raw holds the scaled scores already (attn_softmax_kernel ran).
-template <int TG, int NB, bool PROB = false>
+// With more, raw holds the scaled scores (attn_softmax_kernel ran).
+template <int TG, int NB>
 __global__ __launch_bounds__(256) void attn_values_kernel(const float* __restrict__ raw, const float* __restrict__ vc, float* __restrict__ out,
                                                           int nh, int nkv, int hd, int pos0, int ntok, int spitch, int vpitch) {
   extern __shared__ __align__(16) float dyn[];
@@ -605,7 +594,7 @@ __global__ __launch_bounds__(256) void attn_values_kernel(const float* __restric
   __shared__ double redd[8];
   // (a head's hd/16 workgroups on one die, as in attn_step_fused_kernel: the head's score rows come into one L2)
   const int gx = gridDim.x, bx = (gx & 7) ? (int)blockIdx.x : (int)(blockIdx.x & 7) * (gx >> 3) + (int)(blockIdx.x >> 3);
-  const int ns = hd >> 4, h = bx / ns, cs = bx - h * ns, t0 = blockIdx.y * TG, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int ns = hd >> 4, h = bx / ns, cs = bx - h * ns, t0 = blockIdx.y * TG, tid = threadIdx.x;
   const int tn = min(TG, ntok - t0), nposmax = pos0 + t0 + tn;
   const int group = nh / nkv, kvd = nkv * hd, ko = (h / group) * hd + 16 * cs;
   float* scores = dyn;
@@ -631,9 +620,9 @@ __global__ __launch_bounds__(256) void attn_values_kernel(const float* __restric
   if (TG == 1) {
 #pragma unroll
     for (int u = 2 * NB; u < 8; u++) pre[u] = 0.0f;
-    attn_softmax<256, true>(nullptr, pre, scores, nposmax, tid, redf, redd);
+    attn_softmax(pre, scores, nposmax, tid, redf, redd);
     __syncthreads();                               // every thread's scaled scores, for the products below
-  } else if (PROB) {
+  } else {
     // the group's rows of scaled scores, 16 bytes a thread, eight loads in flight before the first is stored (a load
     // and its store one pair after another would be a trip to memory each); what lies past a token's own positions in
     // its row is carried along and never read
@@ -652,9 +641,6 @@ __global__ __launch_bounds__(256) void attn_values_kernel(const float* __restric
         if (i < totalq) *(float4*)(scores + tt * lp + 4 * j) = tmp[u];
       }
     }
-  } else {
-    for (int tt = wave; tt < tn; tt += 4)
-      attn_softmax<64, false>(raw + ((long long)(t0 + tt) * nh + h) * spitch, nullptr, scores + tt * lp, pos0 + t0 + tt + 1, lane, redf, redd);
   }
 #pragma unroll
   for (int u = 0; u < 8 * NB; u++) {
@@ -916,23 +902,19 @@ __global__ __launch_bounds__(1024) void attn_step_fused_kernel(const float* __re
 
 // The same for contexts whose value slice no longer fits LDS (2,049 to 8,192 positions): the slice comes through
 // LDS in tiles of kValTile positions, and a chain carries its sum from tile to tile -- position after position all
-// the same.  TG 1: the token's scores are taken and scaled here and stay in LDS.  TG 16 (a prompt's chunk): the
-// scores come scaled from attn_softmax_kernel and go through LDS tile by tile like the values.
-constexpr int kValTile = 1024, kValPitch = kValTile + 4;
-template <int TG>
+// the same.  TG tokens of a prompt's chunk; their scores come scaled from attn_softmax_kernel and go through LDS tile by
+// tile like the values.
+constexpr int kValTile = 1024, kValPitch = kValTile + 4, kValTokens = 16;
 __global__ __launch_bounds__(256) void attn_values_tiled_kernel(const float* __restrict__ raw, const float* __restrict__ vc, float* __restrict__ out,
                                                                 int nh, int nkv, int hd, int pos0, int ntok, int spitch) {
   extern __shared__ __align__(16) float dyn[];
-  __shared__ float redf[4];
-  __shared__ double redd[8];
+  constexpr int TG = kValTokens, lp = kValPitch;     // lp: a token's scores of the tile
   const int ns = hd >> 4, h = blockIdx.x / ns, cs = blockIdx.x - h * ns, t0 = blockIdx.y * TG, tid = threadIdx.x;
   const int tn = min(TG, ntok - t0), nposmax = pos0 + t0 + tn;
   const int group = nh / nkv, kvd = nkv * hd, ko = (h / group) * hd + 16 * cs;
-  const int lp = TG > 1 ? kValPitch : spitch;        // TG > 1: a token's scores of the tile; TG 1: all of the token's
   float* scores = dyn;
   float* vt = dyn + TG * lp;
   const float* rbase = raw + ((long long)t0 * nh + h) * spitch;
-  if (TG == 1) attn_softmax<256, false>(rbase, nullptr, scores, nposmax, tid, redf, redd);
   const int tt = tid >> 4, c = tid & 15, npos = pos0 + t0 + tt + 1;       // a chain's token and column (tid < tn * 16)
   const float* sc = scores + tt * lp;
   const float* col = vt + c * kValPitch;
@@ -945,23 +927,21 @@ __global__ __launch_bounds__(256) void attn_values_tiled_kernel(const float* __r
       const int i = min(tid + 256 * u, total - 1);
       r[u] = *(const float4*)(vc + (long long)(p0 + (i >> 2)) * kvd + ko + 4 * (i & 3));
     }
-    __syncthreads();                                 // the scores are there (TG 1, first tile); the chains are through with the tile before
-    if (TG > 1) {
-      // the group's scores of the tile's positions: 256 pieces a row at most (what lies past a token's own positions is
-      // carried along and never read; past the row's end nothing is loaded)
-      const int q4 = (npt + 3) >> 2, totalq = tn * q4;
-      for (int base = 0; base < totalq; base += 256 * 8) {
-        float4 tmp[8];
+    __syncthreads();                                 // the chains are through with the tile before
+    // the group's scores of the tile's positions: 256 pieces a row at most (what lies past a token's own positions is
+    // carried along and never read; past the row's end nothing is loaded)
+    const int q4 = (npt + 3) >> 2, totalq = tn * q4;
+    for (int base = 0; base < totalq; base += 256 * 8) {
+      float4 tmp[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int i = min(base + tid + 256 * u, totalq - 1), rt = i / q4, j = i - rt * q4;
-          tmp[u] = *(const float4*)(rbase + (long long)rt * nh * spitch + p0 + 4 * j);
-        }
+      for (int u = 0; u < 8; u++) {
+        const int i = min(base + tid + 256 * u, totalq - 1), rt = i / q4, j = i - rt * q4;
+        tmp[u] = *(const float4*)(rbase + (long long)rt * nh * spitch + p0 + 4 * j);
+      }
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int i = base + tid + 256 * u, rt = i / q4, j = i - rt * q4;
-          if (i < totalq) *(float4*)(scores + rt * lp + 4 * j) = tmp[u];
-        }
+      for (int u = 0; u < 8; u++) {
+        const int i = base + tid + 256 * u, rt = i / q4, j = i - rt * q4;
+        if (i < totalq) *(float4*)(scores + rt * lp + 4 * j) = tmp[u];
       }
     }
 #pragma unroll
@@ -969,40 +949,24 @@ __global__ __launch_bounds__(256) void attn_values_tiled_kernel(const float* __r
       const int i = tid + 256 * u;
       if (i < total) {
         float* dst = vt + (4 * (i & 3)) * kValPitch + (i >> 2);
-        if (TG == 1) {
-          const float sp = scores[p0 + (i >> 2)];
-          dst[0] = sp * r[u].x; dst[kValPitch] = sp * r[u].y; dst[2 * kValPitch] = sp * r[u].z; dst[3 * kValPitch] = sp * r[u].w;
-        } else {
-          dst[0] = r[u].x; dst[kValPitch] = r[u].y; dst[2 * kValPitch] = r[u].z; dst[3 * kValPitch] = r[u].w;
-        }
+        dst[0] = r[u].x; dst[kValPitch] = r[u].y; dst[2 * kValPitch] = r[u].z; dst[3 * kValPitch] = r[u].w;
       }
     }
     __syncthreads();
     if (tid < tn * 16) {
       const int np = min(kValTile, npos - p0);       // of the tile's positions, the token's own (may be none)
       int p = 0;
-      if (TG == 1) {
-        for (; p + 32 <= np; p += 32) {
-          float4 v4[8];
+      for (; p + 16 <= np; p += 16) {
+        float4 s4[4], v4[4];
 #pragma unroll
-          for (int u = 0; u < 8; u++) v4[u] = *(const float4*)(col + p + 4 * u);
+        for (int u = 0; u < 4; u++) { s4[u] = *(const float4*)(sc + p + 4 * u); v4[u] = *(const float4*)(col + p + 4 * u); }
 #pragma unroll
-          for (int u = 0; u < 8; u++) { o = o + v4[u].x; o = o + v4[u].y; o = o + v4[u].z; o = o + v4[u].w; }
+        for (int u = 0; u < 4; u++) {
+          const float a0 = s4[u].x * v4[u].x, a1 = s4[u].y * v4[u].y, a2 = s4[u].z * v4[u].z, a3 = s4[u].w * v4[u].w;
+          o = o + a0; o = o + a1; o = o + a2; o = o + a3;
         }
-        for (; p < np; p++) o = o + col[p];
-      } else {
-        for (; p + 16 <= np; p += 16) {
-          float4 s4[4], v4[4];
-#pragma unroll
-          for (int u = 0; u < 4; u++) { s4[u] = *(const float4*)(sc + p + 4 * u); v4[u] = *(const float4*)(col + p + 4 * u); }
-#pragma unroll
-          for (int u = 0; u < 4; u++) {
-            const float a0 = s4[u].x * v4[u].x, a1 = s4[u].y * v4[u].y, a2 = s4[u].z * v4[u].z, a3 = s4[u].w * v4[u].w;
-            o = o + a0; o = o + a1; o = o + a2; o = o + a3;
-          }
-        }
-        for (; p < np; p++) o = o + sc[p] * col[p];
       }
+      for (; p < np; p++) o = o + sc[p] * col[p];
     }
   }
   if (tid < tn * 16) out[((long long)(t0 + tt) * nh + h) * hd + 16 * cs + c] = o;
@@ -1013,7 +977,7 @@ __global__ __launch_bounds__(256) void attn_values_tiled_kernel(const float* __r
 // each, tile after tile -- and the other fifteen waves bring the tiles in: tile t+1 is multiplied by its positions'
 // scores and stored into the buffer tile t-1 has left while tile t is being added, and tile t+2's loads are on their way
 // from then on.  All sixteen waves take the softmax first (the scores come from attn_step_scores_kernel, raw).  The
-// numbers are attn_values_tiled_kernel<1>'s: every product and every sum the same, in the same order.
+// numbers are attn_values_kernel<1>'s: every product and every sum the same, in the same order.
 constexpr int kStreamMost = 8192;                  // positions: the scores' room ends there
 constexpr int kStreamTile = 480, kStreamPitch = kStreamTile + 36;      // (a row: 32 floats of room past a tile for the reads ahead; 4 mod 64)
 __global__ __launch_bounds__(1024) void attn_values_stream_kernel(const float* __restrict__ raw, const float* __restrict__ vc, float* __restrict__ out,
@@ -1122,7 +1086,7 @@ __global__ __launch_bounds__(1024) void attn_values_stream_kernel(const float* _
 // A prompt chunk's values, 32 tokens x 32 columns of a query head a workgroup of 1,024 threads, a chain each: the scaled
 // scores (attn_softmax_kernel's) and the value slice come through LDS in tiles of 256 positions, each tile's loads on
 // their way while the tile before it is multiplied and added.  A tile of scores serves 32 columns and a tile of values
-// 32 tokens -- attn_values_kernel<16> and attn_values_tiled_kernel<16> bring a tile in for 16 of each, and what those
+// 32 tokens -- attn_values_kernel<16> and attn_values_tiled_kernel bring a tile in for 16 of each, and what those
 // kernels wait for is the tiles, not the chains.  The numbers are theirs: the same products and sums in the same order.
 constexpr int kChunkTile = 256, kChunkPitch = kChunkTile + 4;      // (4 mod 64: sixteen rows' 16-byte reads on different banks)
 __global__ __launch_bounds__(1024) void attn_values_chunk_kernel(const float* __restrict__ raw, const float* __restrict__ vc, float* __restrict__ out,
@@ -1277,13 +1241,13 @@ hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, flo
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
   // A chunk: scores, softmax, then the values.  Heads of 64 and 128 columns: the matrix cores' products (kernels_attn_mm.hip;
-  // "ILT_ATTN_QUAD=0", tests: not those); others, and what lies on addresses that 16-byte accesses do not take: sixteen lanes
+  // "ILT_ATTN_MM=0", tests: not those); others, and what lies on addresses that 16-byte accesses do not take: sixteen lanes
   // a score and 32 tokens x 32 columns a workgroup.  "ILT_ATTN_CHUNK=0": the kernels of 16 tokens x 16 columns below instead (tests).
   if (scratch && ntok > 1 && pos0 + ntok <= 8192 && hd % 32 == 0) {
-    const char *off = getenv("ILT_ATTN_CHUNK"), *quad = getenv("ILT_ATTN_QUAD");
+    const char *off = getenv("ILT_ATTN_CHUNK"), *with_mm = getenv("ILT_ATTN_MM");
     if (!(off && off[0] == '0')) {
       const int ctx = pos0 + ntok;
-      const bool mm = !(quad && quad[0] == '0') && ilt_k_attn_mm_takes(q, kc, scratch, out, nh, nkv, hd, ctx);
+      const bool mm = !(with_mm && with_mm[0] == '0') && ilt_k_attn_mm_takes(q, kc, scratch, out, nh, nkv, hd, ctx);
       static bool set[64] = {};
       const size_t smem = sizeof(float) * 2 * 32 * (size_t)kChunkPitch;
       if (!mm && !set[dev]) {
@@ -1319,14 +1283,14 @@ hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, flo
   if (tg == TG && nb == NB) {                                                                                                                  \
     static bool set[64] = {};                                                                                                                  \
     e = set[dev] ? hipSuccess                                                                                                                  \
-                 : hipFuncSetAttribute((const void*)attn_values_kernel<TG, NB, (TG > 1)>, hipFuncAttributeMaxDynamicSharedMemorySize,          \
+                 : hipFuncSetAttribute((const void*)attn_values_kernel<TG, NB>, hipFuncAttributeMaxDynamicSharedMemorySize,                    \
                                        152 * 1024);                                                                                            \
     if (e == hipSuccess) {                                                                                                                     \
       set[dev] = true;                                                                                                                         \
       launch_scores<TG>(gs, st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);                                                         \
       if (TG > 1) e = launch_softmax(scratch, nh, pos0, ntok, smax, st);                                                                       \
       if (e != hipSuccess) return e;                                                                                                           \
-      hipLaunchKernelGGL((attn_values_kernel<TG, NB, (TG > 1)>), gv, dim3(256), bytes(TG), st, scratch, vc, out, nh, nkv, hd, pos0, ntok,      \
+      hipLaunchKernelGGL((attn_values_kernel<TG, NB>), gv, dim3(256), bytes(TG), st, scratch, vc, out, nh, nkv, hd, pos0, ntok,                \
                          smax, vpitch);                                                                                                        \
       e = hipGetLastError();                                                                                                                   \
     }                                                                                                                                          \
@@ -1338,26 +1302,23 @@ hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, flo
     }
   }
   if (scratch && pos0 + ntok <= 8192) {              // the value slice through LDS in tiles
-    const int ctx = pos0 + ntok, tg = ntok > 1 ? 16 : 1;
-    const size_t smem = sizeof(float) * ((tg > 1 ? (size_t)tg * kValPitch : (size_t)smax) + 16 * (size_t)kValPitch);
-    const dim3 gs(nh, (ctx + 255) / 256, (ntok + tg - 1) / tg), gv(nh * (hd / 16), (ntok + tg - 1) / tg);
+    const int ctx = pos0 + ntok;
+    if (ntok == 1) {
+      launch_scores<1>(dim3(nh, (ctx + 255) / 256), st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);
+      return launch_values_stream(dev, scratch, vc, out, nh, nkv, hd, pos0, smax, st);
+    }
+    const int groups = (ntok + kValTokens - 1) / kValTokens;
+    const size_t smem = sizeof(float) * (kValTokens + 16) * (size_t)kValPitch;
     static bool set[64] = {};
     if (!set[dev]) {
-      hipError_t e = hipFuncSetAttribute((const void*)attn_values_tiled_kernel<1>, hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024);
-      if (e == hipSuccess) e = hipFuncSetAttribute((const void*)attn_values_tiled_kernel<16>, hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024);
+      const hipError_t e = hipFuncSetAttribute((const void*)attn_values_tiled_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024);
       if (e != hipSuccess) return e;
       set[dev] = true;
     }
-    if (tg == 16) {
-      launch_scores<16>(gs, st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);
-      const hipError_t es = launch_softmax(scratch, nh, pos0, ntok, smax, st);
-      if (es != hipSuccess) return es;
-      hipLaunchKernelGGL(attn_values_tiled_kernel<16>, gv, dim3(256), smem, st, scratch, vc, out, nh, nkv, hd, pos0, ntok, smax);
-    } else {
-      launch_scores<1>(gs, st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);
-      const hipError_t e = launch_values_stream(dev, scratch, vc, out, nh, nkv, hd, pos0, smax, st);
-      if (e != hipSuccess) return e;
-    }
+    launch_scores<kValTokens>(dim3(nh, (ctx + 255) / 256, groups), st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);
+    const hipError_t es = launch_softmax(scratch, nh, pos0, ntok, smax, st);
+    if (es != hipSuccess) return es;
+    hipLaunchKernelGGL(attn_values_tiled_kernel, dim3(nh * (hd / 16), groups), dim3(256), smem, st, scratch, vc, out, nh, nkv, hd, pos0, ntok, smax);
     return hipGetLastError();
   }
   if (!attr_set[dev]) {

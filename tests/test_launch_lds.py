@@ -1,5 +1,6 @@
-"""Every launch with more dynamic LDS than the 64 KB that a kernel gets by itself asks for it first (hipFuncSetAttribute).  The
-library's host code runs here on a stand-in for the HIP runtime that notes what it is asked for and launches nothing (no GPU)."""
+"""Every launch with more dynamic LDS than the 64 KB that a kernel gets by itself asks for it first (hipFuncSetAttribute), and which
+kernels a chunk's attention takes.  The library's host code runs here on a stand-in for the HIP runtime that notes what it is
+asked for and launches nothing (no GPU)."""
 import os
 import subprocess
 import sys
@@ -68,14 +69,41 @@ for nh, nkv, hd in ((32, 8, 128), (14, 2, 64), (32, 8, 96)):
 """
 
 
-def test_no_launch_takes_more_lds_than_it_asked_for(tmp_path):
+def launched(tmp_path, calls, **env):
+    """The lines that the stand-in printed for CALLS: a launch each."""
     from illatio_amd import hip
     (tmp_path / "runtime.c").write_text(RUNTIME)
     so = str(tmp_path / "runtime.so")
     subprocess.check_call(["gcc", "-shared", "-fPIC", "-w", "-o", so, str(tmp_path / "runtime.c")])
-    r = subprocess.run([sys.executable, "-c", CALLS, so, hip.LIB_PATH], env={**os.environ, "ILT_ATTN_SPLIT": "0"}, capture_output=True, text=True)
+    r = subprocess.run([sys.executable, "-c", calls, so, hip.LIB_PATH], env={**os.environ, **env}, capture_output=True, text=True)
     lines = r.stdout.splitlines()
     assert r.returncode == 0, (r.stderr[-2000:], lines[-3:])
+    return lines
+
+
+def test_no_launch_takes_more_lds_than_it_asked_for(tmp_path):
+    lines = launched(tmp_path, CALLS, ILT_ATTN_SPLIT="0")
     assert len(lines) > 500 and sum("gemm_i8_few" in x for x in lines) > 50
     assert any(int(x.split()[-3]) > 65536 for x in lines)
     assert not sorted({x for x in lines if x.startswith("UNASKED")})
+
+
+CHUNKS = r"""
+import ctypes as C, sys
+C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+L = C.CDLL(sys.argv[2])
+I = C.c_int
+at = lambda off=0: C.c_uint64((1 << 40) + off)
+for hd in (64, 128):
+    for ctx in (100, 1000, 3000):
+        assert L.ilt_attn_rows(C.c_uint64(0), at(QUERY), at(), at(), at(), I(16), I(4), I(hd), I(ctx - 40), I(40), at()) == 0
+"""
+
+
+def test_which_kernels_a_chunks_attention_takes(tmp_path):
+    names = lambda lines: {n for n in ("attn_scores_mm", "attn_values_mm", "attn_scores_kernel", "attn_values_chunk", "attn_values_kernel", "attn_values_tiled")
+                           for x in lines if n in x}
+    assert names(launched(tmp_path, "QUERY = 0" + CHUNKS, ILT_ATTN_MM="1")) == {"attn_scores_mm", "attn_values_mm"}
+    assert names(launched(tmp_path, "QUERY = 0" + CHUNKS, ILT_ATTN_MM="0")) == {"attn_scores_kernel", "attn_values_chunk"}
+    assert names(launched(tmp_path, "QUERY = 4" + CHUNKS)) == {"attn_scores_kernel", "attn_values_chunk"}
+    assert names(launched(tmp_path, "QUERY = 0" + CHUNKS, ILT_ATTN_CHUNK="0")) == {"attn_scores_kernel", "attn_values_kernel", "attn_values_tiled"}
