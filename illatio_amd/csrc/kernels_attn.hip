@@ -24,14 +24,20 @@ __device__ __forceinline__ void wave_lds_sync() {
 // The softmax's 1/sum as the CPU rounds it to a single, from a sum of n exps added in another order than the CPU's: one
 // division, then whether every sum that the CPU's could be has the same single for its reciprocal.  No term is negative, so
 // the CPU's n - 1 adds one after another leave a double within (n - 1) 2^-53 of the exact sum, relatively, and a sum whose
-// terms go through at most 64 adds each (here: a thread's own, at most 32, a wave's six, the waves') one within 64 * 2^-53;
-// the two divisions, d's own arithmetic and the bounds' second order are the rest of d, and rounding to single keeps the
-// reciprocals' order.  False: the caller adds the exps again in the CPU's order.
+// terms go through at most ADDS adds each one within ADDS 2^-53; each of the two divisions and the bounds' own subtraction
+// and addition round once more, and what is of second order is under 2^-53 in all for fewer than 2^26 terms.  That is
+// n + ADDS + 3 of the n + 128 taken, and rounding to single keeps the reciprocals' order.  False: the caller adds the exps
+// again in the CPU's order.
+template <int ADDS>
 __device__ __forceinline__ bool recip_settled(double sum, int n, float* inv) {
+  static_assert(ADDS + 3 <= 128, "more adds than the bound counts");
   const double r = 1.0 / sum, d = (double)(n + 128) * 0x1p-53;
   *inv = (float)r;
   return (float)(r - r * d) == (float)(r + r * d);
 }
+// The adds that a term goes through in a sum by threads: a thread's own TERMS one after another (the first to nothing), a
+// wave's six (wave_sum_double), and what the waves' sums take.
+constexpr int sum_adds(int terms, int waves) { return terms - 1 + 6 + waves; }
 
 // One head by one wave: x (hd floats) into xs (LDS): rmsnorm! of the head when its weights are given
 // (model.lisp:205-216: the squares, rounded to floats, added in double one after another), then rope-head!
@@ -134,6 +140,8 @@ __global__ __launch_bounds__(64) void qk_rope_kernel(float* __restrict__ q, floa
 // chain, so a column is one thread's; the value rows come through LDS in tiles of 64 positions that all sixteen
 // waves load (two tiles in flight), so the chain never waits for memory.
 constexpr int kAttnThreads = 1024, kAttnTile = 64;
+constexpr int kRowsLds = 150 * 1024;               // the scores and two tiles of values fit it
+constexpr int kRowsMost = kRowsLds / 4 - 2 * kAttnTile * 16;      // positions, at the narrowest head
 __global__ __launch_bounds__(kAttnThreads) void attn_rows_kernel(const float* __restrict__ q, const float* __restrict__ kc,
                                                                  const float* __restrict__ vc, float* __restrict__ out, int nh, int nkv, int hd,
                                                                  int pos0, float scale, int smax) {
@@ -188,7 +196,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_rows_kernel(const float* __
 #pragma unroll
   for (int w = 0; w < 16; w++) sum += redd[w];
   float inv;
-  if (!recip_settled(sum, npos, &inv)) {           // the same in every thread
+  if (!recip_settled<sum_adds((kRowsMost + kAttnThreads - 1) / kAttnThreads, 15)>(sum, npos, &inv)) {      // the same in every thread
     __syncthreads();
     if (tid == 0) { double s2 = 0.0; for (int p = 0; p < npos; p++) s2 += (double)scores[p]; redd[0] = s2; }
     __syncthreads();
@@ -466,7 +474,7 @@ __device__ __forceinline__ void attn_softmax(const float* pre, float* sc, int np
   const double sum = (redd[0] + redd[1]) + (redd[2] + redd[3]);
   // the CPU adds the terms one after another: take its sum where the order could show in the rounded reciprocal
   float inv;
-  if (!recip_settled(sum, npos, &inv)) {           // the same in all threads
+  if (!recip_settled<sum_adds(8, 2)>(sum, npos, &inv)) {      // the same in all threads
     __syncthreads();
     if (me == 0) { double s2 = 0.0; for (int p = 0; p < npos; p++) s2 += (double)sc[p]; redd[0] = s2; }
     __syncthreads();
@@ -526,7 +534,7 @@ __global__ __launch_bounds__(256) void attn_softmax_kernel(float* __restrict__ r
   // the CPU adds the terms one after another: its sum where the order could show in the rounded reciprocal (a row in 10^5 at
   // 2,500 positions)
   float inv;
-  if (!recip_settled(sum, npos, &inv)) {             // the same in all NT threads
+  if (!recip_settled<sum_adds(4 * NV, NT > 64 ? 2 : 0)>(sum, npos, &inv)) {      // the same in all NT threads
     sum = 0.0;
     if constexpr (NT == 64) {
 #pragma unroll
@@ -873,7 +881,7 @@ __global__ __launch_bounds__(1024) void attn_step_fused_kernel(const float* __re
   for (int w = 1; w < 16; w++) sum += redd[w];
   // the CPU adds the terms one after another: take its sum where the order could show in the rounded reciprocal
   float inv;
-  if (!recip_settled(sum, npos, &inv)) {           // the same in every thread
+  if (!recip_settled<sum_adds(1, 15)>(sum, npos, &inv)) {      // the same in every thread
     if (tid == 0) { double s2 = 0.0; for (int p = 0; p < npos; p++) s2 += (double)sc[p]; redd[16] = s2; }
     ilt_barrier_lds();
     inv = (float)(1.0 / redd[16]);
@@ -1053,7 +1061,7 @@ __global__ __launch_bounds__(1024) void attn_values_stream_kernel(const float* _
 #pragma unroll
   for (int w = 1; w < 16; w++) sum += redd[w];
   float inv;
-  if (!recip_settled(sum, npos, &inv)) {           // the same in every thread
+  if (!recip_settled<sum_adds(kStreamMost / 1024, 15)>(sum, npos, &inv)) {      // the same in every thread
 #pragma unroll
     for (int u = 0; u < kStreamMost / 1024; u++) if (tid + 1024 * u < npos) sc[tid + 1024 * u] = e[u];
     ilt_barrier_lds();
@@ -1327,7 +1335,7 @@ hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, flo
     attr_set[dev] = true;
   }
   const size_t smem = sizeof(float) * ((size_t)smax + 2 * (size_t)kAttnTile * hd);
-  if (smem > 150 * 1024) return hipErrorInvalidValue;      // a query's scores sit in LDS: about 20,000 positions at hd 128
+  if (smem > kRowsLds) return hipErrorInvalidValue;        // a query's scores sit in LDS: about 20,000 positions at hd 128
   hipLaunchKernelGGL(attn_rows_kernel, dim3(nh, ntok), dim3(kAttnThreads), smem, st, q, kc, vc, out, nh, nkv, hd, pos0, scale, smax);
   return hipGetLastError();
 }
