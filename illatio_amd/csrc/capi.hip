@@ -293,7 +293,9 @@ int ilt_mv_multi_ahead(uint64_t stream, int nmat, const ilt_mv_desc* descs, int 
   if (e != ILT_OK || live == 0) return e;
   // (the next product's activations do not matter to its plan: this call's stand in for them)
   static const bool rows_on = []{ const char* f = getenv("ILT_ROWS_AHEAD"); return !(f && f[0] == '0'); }();      // ("0": never, for tests)
-  p.once = next_nmat > 0;                            // (a chain of products: this one's rows are not the next call's)
+  // A chain of products: this one's rows are not the next call's.  (Also where all of the chain's matrices fit the dies' L2s: gate, up and
+  // down of 3,072 x 1,024, 6 MB and 24 MB in all, 11.9-13.1 us a set against 12.6-13.1 with rows that stay.)
+  p.once = next_nmat > 0;
   if (rows_on && next_nmat && build(pn, &live_n, next_nmat, next_descs, next_cols, xf, nullptr, 0, next_glu) == ILT_OK && live_n &&
       ilt_gemv_plan(p, 1) == hipSuccess && ilt_gemv_plan(pn, 1) == hipSuccess)
     ilt_gemv_rows_of(pn, p.rows_ahead);
@@ -569,8 +571,10 @@ int step_run(uint64_t stream, uint8_t* ws, int ne, int nu, int d, int ff, float 
   float *bm = (float*)(ws + l.bm), *bd = (float*)(ws + l.bd);
   const int grb = d / 256 * 66, drb = ff / 256 * 84;
   // A step whose matrices are more than the dies' L2s hold (32 MB) finds none of them there the next time, so they leave L2 first
-  // (ilt_g2lds16_once): 6 of 256 experts, 4,096 x 2,048 (80 MB) 40.4 -> 38.6 us.  A smaller one may: 3 of 32, 2,048 x 2,048
-  // (24 MB), the same step again: 23.9 us, and 24.9 if they left.
+  // (ilt_g2lds16_once).  A smaller one may.  Rows that stay and rows that leave, us, the same token again and other tokens: 3 of 32
+  // experts, 2,048 x 2,048 (23 MB) 24.9 and 25.5, 25.0 and 26.1; 8 of 128, 2,048 x 1,536 (30 MB) 30.4 and 30.3, 30.7 and 30.6; 8 of 256,
+  // 2,048 x 2,048 (40 MB) 36.3 and 35.0, 37.9 and 35.5; 6 of 256, 4,096 x 2,048 (66 MB) 39.8 and 38.2, 41.4 and 38.4; 8 of 256 (80
+  // MB) 49.3 and 48.7, 50.4 and 50.3.
   const int once = (long long)nu * (2 * wt->gate_bytes + (long long)d * drb) + 3LL * d * ff * 17 / 16 > (32LL << 20);
   // the routing rides along with the shared expert's gate/up launch (one of its waves routes while the rows stream
   // in); where that launch cannot take it, a launch of its own
@@ -1112,6 +1116,8 @@ static int dec_build(DecLaunch& L, int nmat, const ilt_mv_desc* descs, int cols,
   ILT_REQUIRE(xf && (norm || !glu));
   const int e = gemv_multi_build(L.p, &L.live, nmat, fmts, ws, wds, ys, bs, rows, cols, nullptr, nullptr, nullptr, xf, 1, acc, glu, 0, norm, eps, 0);
   if (e != ILT_OK) return e;
+  // (whatever the model's size: decoders of 9, 17, 25, 32, 40, 63 and 94 MB in all 40.7, 67.6, 94.2, 121.7, 148.2, 229.8 and 337.1 us a
+  // token, and 40.5, 67.1, 94.7, 122.0, 148.6, 229.3 and 336.8 with rows that stay; one layer of 62 MB 52.9 and 54.5)
   L.p.once = 1;
   L.planned = L.live > 0 && ilt_gemv_plan(L.p, 1) == hipSuccess;
   return ILT_OK;

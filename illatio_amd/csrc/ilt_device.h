@@ -163,8 +163,8 @@ __device__ __forceinline__ void ilt_g2lds16(const void* src, void* lds_base) {
 
 // The same for bytes that nobody reads again before megabytes of others have gone by: they leave the die's L2 first.  What a
 // token's next launch wants of L2 -- its code above all, which each launch's CUs fetch afresh and which otherwise comes from
-// beyond L2 a jump at a time, the vectors, the rows read ahead -- then outlives the rows of this one (a token of the Qwen3-4B
-// shape at 600 positions: 27.7 -> 26.6 ms for 17).
+// beyond L2 a jump at a time, the vectors, the rows read ahead -- then outlives the rows of this one (the Qwen3-4B shape at
+// 600 positions: 27.3 -> 26.6 ms for 17 tokens).
 __device__ __forceinline__ void ilt_g2lds16_once(const void* src, void* lds_base) {
   __builtin_amdgcn_global_load_lds((const ILT_GLOBAL void*)src, (ILT_LDS void*)lds_base, 16, 0, 2);
 }

@@ -250,7 +250,8 @@ hipError_t q8_launch(Q8Params& p, hipStream_t st) {
 // What a workgroup of each kind of tile takes for 4,096 columns, microseconds, with 1, 2, ... of them on a CU (4,096 rows on 64 to
 // 2,304 tokens): a small tile is the shortest chain of steps, a large one reads LDS less a result.  Workgroups past those that fit
 // take over the places that come free, all but the largest's, which start and end together.  (4096 x 4096 on 1,000 tokens: 128 x 64 68.9
-// us, 64 x 64 84.4; 9728 x 896 on 301 20.2 and 18.7; 4096 x 4096 on 4,096 261, 312, and 230 for 128 x 128.)
+// us, 64 x 64 84.4; 9728 x 896 on 301 20.2 and 18.7; 4096 x 4096 on 4,096 261, 312, and 230 for 128 x 128.)  Other widths are chosen for by
+// the same figures: what grows with the columns and what a launch costs by itself are not apart in them.
 struct Q8Kind { int rows, tokens, fit; float us[5]; };
 constexpr Q8Kind kQ8Tiles[] = {
   {32, 32, 4, {15.2f, 19.0f, 26.0f, 33.2f}},

@@ -658,7 +658,9 @@ hipError_t launch_i8r_group(const BfParams& p, long long total_rows, hipStream_t
 // a CU, as many as fit (Q4_K; Q6_K), measured on 1,024 to 19,456 rows and 17 to 768 tokens: a wave alone on its SIMD issues an
 // instruction in 2.1 ns, two in 1.05 each, so tiles of one wave are the fastest way through the columns while there are fewer
 // of them than SIMDs, and large tiles, which unpack a weight for more tokens, once there are more.  (Workgroups of two waves come
-// to lie on the same two SIMDs of a CU: 1.4, then 2.35.)
+// to lie on the same two SIMDs of a CU: 1.4, then 2.35.)  The chip is taken to be empty: where another stream's launches run beside
+// (the halves of a prompt) a launch takes longer than this says -- down at the Qwen3-4B shape on 256 tokens 61 us here, 57-64 alone,
+// 87 beside the other half -- and the choice is the one for a launch alone.
 struct RegTile { int rows, tokens, fit; float us[2][5]; };
 constexpr RegTile kRegTiles[] = {
   {32, 32, 5, {{1.1f, 1.18f, 1.3f, 1.35f, 2.0f}, {1.4f, 1.5f, 1.65f, 2.05f, 4.0f}}},       // (Q6_K: four fit, a fifth is a second round)
