@@ -439,12 +439,11 @@ hipError_t few_dispatch(FewParams& p, int forced, hipStream_t st) {
 }  // namespace
 
 // Up to four matrices (all Q8_0, or Q4_K and Q6_K in any mix) on the same quantized tokens in one launch.
-// hipErrorNotSupported (nothing launched) where the shapes are not this kernel's.  Against the kernel with the weights in
-// operand registers (kernels_gemm_reg.hip), whose smallest tiles are 32 rows x 32 tokens a wave, the line lies at the number of
-// those that take as long, whatever the tokens (Q4_K: 9728 x 2560 on 32 tokens, 304 tiles: 15.7 against 16.0 us, 6144 x 2560 on 64, 384:
-// 16.0 against 16.3, 2560 x 4096 on 128, 320: 24.3 against 22.8, 19456 x 2560 on 32, 608: 24 against 17.6; Q6_K: 6144 x 2560 on
-// 32, 192: 15.7 against 18.5, 2560 x 9728 on 96, 240: 43 against 57, 4096 x 1024 on 64, 256: 10.0 both, 9728 x 2560 on 32, 304: 21.8
-// against 19.1).  Up to 16 tokens half of those tiles is for nothing.  (A mixed launch's line lies between the two formats'.)  Q8_0 against its own kernel (kernels_gemm_q8.hip),
+// hipErrorNotSupported (nothing launched) where the shapes are not this kernel's.  Against the kernels with the weights in
+// operand registers (kernels_gemm_reg.hip), whose smallest tiles are 32 rows x 32 tokens, the line lies at 128 of those, whatever the
+// tokens (us here and there: Q4_K 4096 x 2560 on 32 tokens, 128 tiles: 9.2 and 10.8, 6144 x 2560 on 21, 192: 12.1 and 11.5, 2560 x 4096 on
+// 40, 160: 16.6 and 12.5; Q6_K: 2560 x 9728 on 32, 80: 25.5 both, on 40, 160: 41 and 25.6, 1024 x 2560 on 128, 128: 10.8 and 11.0).  Up to 16 tokens
+// half of those tiles is for nothing.  Q8_0 against its own kernel (kernels_gemm_q8.hip),
 // whose waves make a tile's terms and sums in registers: up to 16 tokens here, unless the tiles of 16 rows fill the chip (896 x 4864
 // on 16 tokens 12.7 us against 16.1, on 24 17.1 against 16.1; 4096 x 2048 on 16, 256 tiles: 8.1 against 8.3; 9728 x 896, 608:
 // 7.7 against 5.8); where its smallest tile does not go (cols no multiple of 128) from 640 tiles of 32 x 32 and 96 tokens on.
@@ -475,13 +474,12 @@ hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws
   }
   tiles32 *= (ntok + 31) / 32;
   if (tiles32 > 0x3FFFFFFF) return hipErrorNotSupported;
-  const long long line = fset == ILT_Q4_K ? 320 : fset == ILT_Q6_K ? 250 : 285;
   if (forced < 0 && fset == ILT_Q8_0) {
     if (cols % 128 == 0 ? ntok > 16 || tiles32 > 128 : ntok >= 96 && tiles32 > 640) {
       const hipError_t e = ilt_k_gemm_q8(nmat, ws, wds, rows, ys, biases, cols, xq, xs, ntok, acc, st, ldy);
       if (e != hipErrorNotSupported) return e;
     }
-  } else if (forced < 0 && !small && ntok > 16 && tiles32 > line) return hipErrorNotSupported;
+  } else if (forced < 0 && !small && ntok > 16 && tiles32 > 128) return hipErrorNotSupported;
   switch (fset) {
     case ILT_Q8_0: return few_dispatch<ILT_Q8_0>(p, forced, st);
     case ILT_Q4_K: return few_dispatch<ILT_Q4_K>(p, forced, st);

@@ -37,6 +37,7 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef unsigned short v2u __attribute__((ext_vector_type(2)));
@@ -511,6 +512,7 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
   };
 #pragma unroll 1
   for (int sb = 0; sb < nsb; sb++) {
+
     const int nx = min(sb + 1, nsb - 1), nbuf = (sb + 1) & 1;       // (the last block's again, for nobody)
     using std::integral_constant;
     __builtin_amdgcn_sched_barrier(0);
@@ -563,6 +565,208 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
   store_tile<NP, 1>(sum, p, tok0, ntok, r0, wt0, wr0, l32, lh);
 }
 
+// Rows r0 .. x tokens tok0 .. tok0 + ntok - 1 where the launch has few tiles: a tile of 32 rows x 32 tokens is KS waves', super-block
+// u wave u mod KS's, 4 / KS tiles of rows a workgroup.  What bounds such a launch is the chain of a row's blocks: a wave alone on
+// its SIMD issues an instruction in 5 cycles, 1.4 us a block, whatever the rest of the chip could do meanwhile.  A block's
+// integers and float terms depend on nothing before them, only the sums' order does, so every wave makes its blocks' terms as
+// reg_tile does (its own loads, operands and products, a block ahead: nothing shared), leaves them in LDS, and once a round -- KS
+// blocks -- each adds the terms of its own 4 / KS quarters of the tile in the CPU's order.  A round takes 1.95 us (four waves of a CU
+// share its LDS and the loads' way: 1.6 without the loads).  us before and now, matrices from memory: Q6_K 2560 x 9728 on 33 to 96
+// tokens 41-43 -> 26-27, on 160 62 -> 43; 4096 x 4096 on 64 28 -> 15; Q4_K 2560 x 4096 on 40 16.7 -> 12.8, on 128 24 -> 20.
+template <int FMT, int KS> struct SplitSmem {
+  RegSmem<32, 2 * RegW<FMT>::LBYTES, RegW<FMT>::MINS, 2> w[4];
+  __align__(16) float ex[4 / KS][4][KS][RegW<FMT>::MINS ? 2 : 1][256];       // terms [rows' tile][quarter][wave][a term][lane's four]
+};
+template <int FMT, int KS>
+__device__ __forceinline__ void reg_split(const BfParams& p, const u8* w, int r0, long tok0, int ntok, unsigned char* smem) {
+  using F = RegW<FMT>;
+  constexpr int OWN = 4 / KS, TERMS = F::MINS ? 2 : 1;
+  static_assert(F::PLANES == 2 && (KS == 2 || KS == 4), "");
+  SplitSmem<FMT, KS>& W = *(SplitSmem<FMT, KS>*)smem;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ks = wave % KS, wr = wave / KS;
+  auto& S = W.w[wave];
+  const int nsb = p.cols / 256, rounds = (nsb + KS - 1) / KS;
+  const int l32 = lane & 31, lh = lane >> 5, wr0 = 32 * wr;
+  const u32 row_bytes = (u32)(nsb * F::BLOCK);
+  const __amdgpu_buffer_rsrc_t rw = ilt_rsrc(ilt_uniform_ptr(w), (u32)p.rows * row_bytes);      // (past the matrix's rows: zeros)
+  const typename F::At at = F::place(row_bytes, lane, r0 + wr0, p.rows);
+  auto issue_w = [&](int sb, int buf) {
+#pragma unroll
+    for (int i = 0; i < F::LOADS; i++) F::issue(i, rw, w, at, row_bytes, (u32)(r0 + wr0), (u32)sb * F::BLOCK, S.ws + buf * F::LBYTES);
+  };
+  ntok = __builtin_amdgcn_readfirstlane(ntok);
+  const __amdgpu_buffer_rsrc_t rx = ilt_rsrc(ilt_uniform_ptr((const i8*)p.x + tok0 * (long)p.cols), (u32)(ntok * p.cols));      // (past the tile's tokens: zeros)
+  const u32 xlane = (u32)(lane >> 4) * (u32)p.cols + 16 * (u32)((lane & 15) ^ (lane >> 4));
+  auto issue_x = [&](int sb, int buf) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (ILT_LDS void*)(S.xs[buf] + i * 1088), 16, xlane + (u32)(i * 4) * (u32)p.cols, sb * 256, 0, 0);
+  };
+  const __amdgpu_buffer_rsrc_t rd = ilt_rsrc(ilt_uniform_ptr(p.xd + tok0 * nsb), (u32)(ntok * nsb) * 4);
+  const __amdgpu_buffer_rsrc_t rb = ilt_rsrc(ilt_uniform_ptr(p.bsums + (F::MINS ? tok0 * (p.cols >> 4) : 0)), F::MINS ? (u32)(ntok * (p.cols >> 4)) * 4 : 0);
+  float c_yd; int4 c_bs[2];
+  auto load_consts = [&](int sb) {                   // half a token's sums of 16 a lane
+    const u32 ctok = (u32)((lane >> 1) * nsb);
+    c_yd = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, ctok * 4, sb * 4, 0));
+    if constexpr (F::MINS) {
+      const u32 o = ctok * 64 + 32 * (lane & 1);
+      const ilt_v4i a = __builtin_amdgcn_raw_buffer_load_b128(rb, o, sb * 64, 0), b = __builtin_amdgcn_raw_buffer_load_b128(rb, o + 16, sb * 64, 0);
+      c_bs[0] = make_int4(a.x, a.y, a.z, a.w); c_bs[1] = make_int4(b.x, b.y, b.z, b.w);
+    }
+  };
+  auto store_consts = [&](int buf) {
+    if ((lane & 1) == 0) S.xd[buf][lane >> 1] = c_yd;
+    if constexpr (F::MINS) {
+      const int4 &b0 = c_bs[0], &b1 = c_bs[1];
+      const int s[4] = { b0.x + b0.y, b0.z + b0.w, b1.x + b1.y, b1.z + b1.w };
+      _Float16 hh[4], ll[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) { hh[k] = (_Float16)(float)(s[k] & ~127); ll[k] = (_Float16)(float)(s[k] & 127); }
+      _Float16* const dst = (_Float16*)(S.ms[buf] + 32 * (lane >> 1)) + 4 * (lane & 1);
+      __builtin_memcpy(dst, hh, 8);
+      __builtin_memcpy(dst + 8, ll, 8);
+    }
+  };
+  const u32 x0 = (u32)(l32 >> 2) * 1088 + (u32)(l32 & 3) * 256 + 16 * (u32)(lh ^ (l32 & 3)), x1 = x0 ^ 32;
+  v4f sum[OWN];
+#pragma unroll
+  for (int o = 0; o < OWN; o++) sum[o] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  v4i hi[8], lo[8];
+  typename F::Block blk;
+  auto mine = [&](int i) { return min(i * KS + ks, nsb - 1); };      // the wave's block of round i (past the last: the last again, for nobody)
+  issue_w(mine(0), 0);
+  issue_x(mine(0), 0);
+  load_consts(mine(0));
+  issue_w(mine(1), 1);
+  store_consts(0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  F::block(blk, S.ws, l32, lh);
+  {
+    typename F::Quants qs;
+#pragma unroll
+    for (int g = 0; g < 8; g++) { F::quants(qs, S.ws, g, l32, lh); F::quants_now(qs, S.ws, g, l32, lh); F::group(blk, qs, g, lh, hi[g], lo[g]); }
+  }
+  v16i X, Y, P;
+  v16f im = {};
+  float dprev = 0.0f, dmprev = 0.0f;
+#pragma unroll
+  for (int r = 0; r < 16; r++) P[r] = 0;
+  float* const ex = (float*)W.ex[wr];
+  // four results' terms, of the round before, to their quarter's place
+  auto term = [&](int j, const float4& y) {
+    float a[4], b[4], f[4];
+    const float yv[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) { b[i] = yv[i] * dprev; f[i] = (float)P[4 * j + i]; if constexpr (F::MINS) a[i] = yv[i] * dmprev; }
+#pragma unroll
+    for (int i = 0; i < 4; i++) { b[i] = b[i] * f[i]; if constexpr (F::MINS) a[i] = a[i] * im[4 * j + i]; }
+    float* const o = ex + ((j * KS + ks) * TERMS) * 256 + 4 * lane;
+    if constexpr (F::MINS) *ILT_LDS_PTR(v4f, o) = v4f{a[0], a[1], a[2], a[3]};
+    *ILT_LDS_PTR(v4f, o + (TERMS - 1) * 256) = v4f{b[0], b[1], b[2], b[3]};
+  };
+  // the wave's quarters: the terms of round i's blocks in order
+  auto add = [&](int i) {
+#pragma unroll
+    for (int o = 0; o < OWN; o++) {
+      v4f t[KS][TERMS];
+#pragma unroll
+      for (int s = 0; s < KS; s++)
+#pragma unroll
+        for (int k = 0; k < TERMS; k++) t[s][k] = *ILT_LDS_PTR(const v4f, ex + (((ks * OWN + o) * KS + s) * TERMS + k) * 256 + 4 * lane);
+#pragma unroll
+      for (int s = 0; s < KS; s++)
+        if (i * KS + s < nsb) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            if constexpr (F::MINS) sum[o][r] = sum[o][r] - t[s][0][r];
+            sum[o][r] = sum[o][r] + t[s][TERMS - 1][r];
+          }
+        }
+      asm volatile("" : "+v"(sum[o]));               // (the reads have come back before the wave meets the next barrier)
+    }
+  };
+  int c0 = 0, c1 = 1, c2 = 2;
+#pragma unroll 1
+  for (int i = 0; i < rounds; i++) {
+    const int nbuf = (i + 1) & 1;
+    __builtin_amdgcn_sched_barrier(0);
+    issue_x(mine(i + 1), nbuf);
+    load_consts(mine(i + 1));
+    issue_w(mine(i + 2), i & 1);                     // (this block's operands are made)
+    __builtin_amdgcn_sched_barrier(0);
+    const u8 *const wnext = S.ws + nbuf * F::LBYTES, *const xs = S.xs[i & 1];
+    const float* const xp = S.xd[c2] + 4 * lh;
+    auto frag = [&](int g) { return __builtin_bit_cast(v4i, ilt_lds_ld16(xs + (g & 1 ? x1 : x0) + 64 * (g >> 1))); };
+    const v16i zi = {};
+    typename F::Block nb = {};
+    typename F::Quants qs;
+    v4i f0 = frag(0), f1 = frag(1);
+    float4 y = lds_f4(xp);
+    v8h sums;
+    F::block(nb, wnext, l32, lh); F::quants(qs, wnext, 0, l32, lh);
+#pragma unroll
+    for (int g = 0; g < 8; g++) {
+      const v4i f = f0;
+      f0 = f1;
+      if (g < 6) f1 = frag(g + 2);
+      F::quants_now(qs, wnext, g, l32, lh);
+      if (g < 7) F::quants(qs, wnext, g + 1, l32, lh);
+      if (F::MINS && g == 6) sums = __builtin_bit_cast(v8h, ilt_lds_ld16(S.ms[c0] + 32 * l32 + 16 * lh));
+      __builtin_amdgcn_sched_barrier(0);
+      X = __builtin_amdgcn_mfma_i32_32x32x32_i8(f, hi[g], g ? X : zi, 0, 0, 0);
+      Y = __builtin_amdgcn_mfma_i32_32x32x32_i8(f, lo[g], g ? Y : zi, 0, 0, 0);
+      if (g == 0) asm volatile("s_barrier" ::: "memory");      // (the round before's terms have been added)
+      if (g % 2 == 1) {
+        term(g >> 1, y);
+        if (g < 7) y = lds_f4(xp + 8 * (g >> 1) + 8);
+      }
+      F::group(nb, qs, g, lh, hi[g], lo[g]);
+      asm volatile("" : "+v"(hi[g]), "+v"(lo[g]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (F::MINS) {
+      const v16f zf = {};
+      im = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, blk.mins, zf, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) P[r] = (X[r] << F::SH) + Y[r];
+    dprev = blk.d; dmprev = blk.dm; blk = nb;
+    store_consts(c1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    ilt_barrier_lds();
+    if (i > 0) add(i - 1);
+    const int c = c2; c2 = c0; c0 = c1; c1 = c;
+  }
+  ilt_barrier_lds();
+  {
+    const float* const xp = S.xd[c2] + 4 * lh;
+#pragma unroll
+    for (int j = 0; j < 4; j++) term(j, lds_f4(xp + 8 * j));
+  }
+  ilt_barrier_lds();
+  add(rounds - 1);
+  // results: tokens 8 j + 4 lh .. of the row
+  const int row = r0 + wr0 + l32;
+  const bool ok = row < p.rows;
+  const __amdgpu_buffer_rsrc_t ry = ilt_rsrc(ilt_uniform_ptr(p.y + tok0 * p.ldy), ((u32)(ntok - 1) * (u32)p.ldy + (u32)p.rows) * 4);
+  const u32 rows4 = (u32)p.ldy * 4, base = ok ? (u32)((8 * OWN * ks + 4 * lh) * (int)p.ldy + row) * 4 : 0x80000000u;
+  const float bv = p.bias && ok ? p.bias[row] : 0.0f;
+#pragma unroll
+  for (int o = 0; o < OWN; o++) {
+    float old[4];
+    if (p.acc) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) old[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ry, base + (u32)(8 * o + r) * rows4, 0, 0));
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      float v = sum[o][r];
+      if (p.bias) v = v + bv;
+      if (p.acc) v = old[r] + v;
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, v), ry, base + (u32)(8 * o + r) * rows4, 0, 0);
+    }
+  }
+}
+
 // FSET: the matrices' format, or 0 where Q4_K and Q6_K meet in a launch
 template <int FSET, int NP, int WR, int WT>
 __global__ __launch_bounds__(64 * WR * WT, WR * WT == 1 ? 1 : 2) void gemm_i8r_kernel(BfParams p) {
@@ -584,6 +788,27 @@ __global__ __launch_bounds__(64 * WR * WT, WR * WT == 1 ? 1 : 2) void gemm_i8r_k
   if constexpr (FSET != 0) reg_tile<FSET, NP, WR, WT>(p, w, rt * TM, tok0, ntok, smem);
   else if (fmt == ILT_Q4_K) reg_tile<ILT_Q4_K, NP, WR, WT>(p, w, rt * TM, tok0, ntok, smem);
   else reg_tile<ILT_Q6_K, NP, WR, WT>(p, w, rt * TM, tok0, ntok, smem);
+}
+
+template <int FSET, int KS>
+__global__ __launch_bounds__(256, 1) void gemm_i8s_kernel(BfParams p) {
+  constexpr int TM = 32 * (4 / KS);
+  extern __shared__ __align__(16) unsigned char smem[];
+  long tok0; int ntok, rt; const u8* w = p.w;
+  if (!pick_tile<TM, 32>(p, tok0, ntok, rt, w)) return;
+  // which of the launch's matrices the row tile belongs to
+  const int n0 = (p.mrows[0] + TM - 1) / TM, n1 = n0 + (p.mrows[1] + TM - 1) / TM;
+  const int m = rt < n0 ? 0 : rt < n1 ? 1 : 2;
+  rt -= m == 0 ? 0 : m == 1 ? n0 : n1;
+  w = m == 0 ? p.mw[0] : m == 1 ? p.mw[1] : p.mw[2];
+  p.rows = m == 0 ? p.mrows[0] : m == 1 ? p.mrows[1] : p.mrows[2];
+  p.y = m == 0 ? p.my[0] : m == 1 ? p.my[1] : p.my[2];
+  p.bias = m == 0 ? p.mbias[0] : m == 1 ? p.mbias[1] : p.mbias[2];
+  if (p.nmulti > 1) p.ldy = p.rows;
+  const int fmt = m == 0 ? p.mfmt[0] : m == 1 ? p.mfmt[1] : p.mfmt[2];
+  if constexpr (FSET != 0) reg_split<FSET, KS>(p, w, rt * TM, tok0, ntok, smem);
+  else if (fmt == ILT_Q4_K) reg_split<ILT_Q4_K, KS>(p, w, rt * TM, tok0, ntok, smem);
+  else reg_split<ILT_Q6_K, KS>(p, w, rt * TM, tok0, ntok, smem);
 }
 
 template <int FMT, int NP, int WR, int WT> constexpr size_t reg_smem() {
@@ -610,6 +835,29 @@ hipError_t launch_i8r(BfParams& p, hipStream_t st) {
   const long long total = (long long)((p.ntok + TN - 1) / TN) * tiles, per = (total + 7) / 8;
   if (per * 8 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
   hipLaunchKernelGGL((gemm_i8r_kernel<FSET, NP, WR, WT>), dim3((unsigned)(per * 8)), dim3(64 * WR * WT), smem, st, p);
+  return hipGetLastError();
+}
+
+template <int FSET, int KS>
+hipError_t launch_i8s(BfParams& p, hipStream_t st) {
+  constexpr int TM = 32 * (4 / KS);
+  constexpr size_t s4 = sizeof(SplitSmem<ILT_Q4_K, KS>), s6 = sizeof(SplitSmem<ILT_Q6_K, KS>);
+  constexpr size_t smem = FSET == ILT_Q4_K ? s4 : FSET == ILT_Q6_K ? s6 : s4 > s6 ? s4 : s6;
+  static_assert(smem <= 160 * 1024, "a workgroup's LDS");
+  static bool attr_set[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  if (!attr_set[dev]) {
+    const hipError_t e = hipFuncSetAttribute((const void*)gemm_i8s_kernel<FSET, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return e;
+    attr_set[dev] = true;
+  }
+  long long tiles = 0;
+  for (int m = 0; m < p.nmulti; m++) tiles += (p.mrows[m] + TM - 1) / TM;
+  p.rows = (int)(tiles * TM);
+  const long long total = (long long)((p.ntok + 31) / 32) * tiles, per = (total + 7) / 8;
+  if (per * 8 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((gemm_i8s_kernel<FSET, KS>), dim3((unsigned)(per * 8)), dim3(256), smem, st, p);
   return hipGetLastError();
 }
 
@@ -669,22 +917,34 @@ constexpr RegTile kRegTiles[] = {
   {64, 128, 2, {{1.7f, 2.8f}, {1.75f, 2.9f}}},
   {128, 128, 2, {{2.6f, 4.4f}, {2.55f, 4.4f}}},
 };
+// The same for tiles whose super-blocks are shared out (reg_split): a workgroup of four waves takes what a CU's LDS holds, and 1.95
+// us for a round of KS blocks whatever the format (a wave alone on its SIMD, 571 instructions for Q6_K); besides, microseconds, a
+// tile's start and end, and the launch's, which tiles of the other kinds have once.
+constexpr float kRegStart = 4.0f, kSplitStart = 2.8f, kSplitTile = 2.2f, kSplitRound = 1.95f;
 // Which of them, by the rounds that the chip takes the launch's workgroups in.  (Shapes, us for the tiles taken and for 64 or 128
 // rows x 128 tokens: Q6_K 2560 x 9728 on 256 tokens 57-64 and 89, on 512 81 and 90; Q4_K 2560 x 4096 on 256 25 and 33; 19456 x 2560 on 32
 // 17.6 and 31, on 192 35 and 48; 9728 x 2560 on 64 17.2 and 22.)
 template <int FSET>
 int reg_tile_of(const BfParams& p) {
+  const int f = FSET == ILT_Q4_K ? 0 : 1, nsb = p.cols / 256;
+  auto workgroups = [&](int rows, int tokens) {
+    long long n = 0;
+    for (int m = 0; m < p.nmulti; m++) n += (p.mrows[m] + rows - 1) / rows;
+    return n * ((p.ntok + tokens - 1) / tokens);
+  };
   int best = 0;
   float least = 0.0f;
   for (int v = 0; v < 5; v++) {
     const RegTile& c = kRegTiles[v];
-    const int f = FSET == ILT_Q4_K ? 0 : 1, fit = v == 0 && f ? 4 : c.fit;
-    long long n = 0;
-    for (int m = 0; m < p.nmulti; m++) n += (p.mrows[m] + c.rows - 1) / c.rows;
-    n *= (p.ntok + c.tokens - 1) / c.tokens;
-    const long long round = 256LL * fit, rest = n % round;
-    const float us = (float)(n / round) * c.us[f][fit - 1] + (rest ? c.us[f][(rest + 255) / 256 - 1] : 0.0f);
+    const int fit = v == 0 && f ? 4 : c.fit;
+    const long long n = workgroups(c.rows, c.tokens), round = 256LL * fit, rest = n % round;
+    const float us = kRegStart + (float)nsb * ((float)(n / round) * c.us[f][fit - 1] + (rest ? c.us[f][(rest + 255) / 256 - 1] : 0.0f));
     if (v == 0 || us < least) { best = v; least = us; }
+  }
+  for (int v = 5; v < 7; v++) {                      // KS 2 and 4, a workgroup a CU
+    const int ks = v == 5 ? 2 : 4;
+    const float us = kSplitStart + (float)((workgroups(128 / ks, 32) + 255) / 256) * (kSplitTile + kSplitRound * (float)((nsb + ks - 1) / ks));
+    if (us < least) { best = v; least = us; }
   }
   return best;
 }
@@ -696,11 +956,13 @@ hipError_t dispatch_i8r(BfParams& p, int forced, hipStream_t st) {
     const bool big = forced ? forced == 128 : (long long)((p.mrows[0] + 127) / 128) * ((p.ntok + 127) / 128) >= 150;
     return big ? launch_i8r<FSET, 4, 4, 1>(p, st) : launch_i8r<FSET, 2, 2, 2>(p, st);
   } else {
-    switch (forced == 128 ? 4 : forced == 64 ? 3 : forced >= 1 && forced <= 5 ? forced - 1 : reg_tile_of<FSET>(p)) {
+    switch (forced == 128 ? 4 : forced == 64 ? 3 : forced >= 1 && forced <= 7 ? forced - 1 : reg_tile_of<FSET>(p)) {
       case 0: return launch_i8r<FSET, 1, 1, 1>(p, st);
       case 1: return launch_i8r<FSET, 2, 1, 1>(p, st);
       case 2: return launch_i8r<FSET, 2, 2, 1>(p, st);
       case 3: return launch_i8r<FSET, 2, 2, 2>(p, st);
+      case 5: return launch_i8s<FSET, 2>(p, st);
+      case 6: return launch_i8s<FSET, 4>(p, st);
       default: return launch_i8r<FSET, 4, 4, 1>(p, st);
     }
   }

@@ -59,6 +59,35 @@ def test_operands_in_registers_bit_for_bit(dev, monkeypatch, rows_a_tile, qtype,
     m.free()
 
 
+# the super-blocks shared out over two and four waves: fewer of them than waves, a last round that is not whole, whole rounds; rows and
+# tokens around tiles of 32 and 64
+@pytest.mark.parametrize("tile", ["6", "7"])
+@pytest.mark.parametrize("qtype,rows,cols,n", [
+    (synth.Q4_K, 1, 256, 17), (synth.Q4_K, 33, 512, 33), (synth.Q4_K, 64, 1024, 32), (synth.Q4_K, 95, 1280, 65), (synth.Q4_K, 300, 2560, 40),
+    (synth.Q6_K, 31, 256, 64), (synth.Q6_K, 32, 768, 31), (synth.Q6_K, 65, 1024, 97), (synth.Q6_K, 128, 9728, 21), (synth.Q6_K, 257, 2816, 50)])
+def test_super_blocks_shared_out_bit_for_bit(dev, monkeypatch, tile, qtype, rows, cols, n):
+    test_operands_in_registers_bit_for_bit(dev, monkeypatch, tile, qtype, rows, cols, n)
+
+
+# Q, K and V of mixed formats in one launch of such tiles, against the products for few tokens
+@pytest.mark.parametrize("tile", ["6", "7"])
+def test_mixed_formats_with_super_blocks_shared_out(dev, monkeypatch, tile):
+    from illatio_amd import hip, model
+    host = model.synth_model(12, d=768, ffn=1024, nh=12, nkv=4, hd=64, nl=2, vocab=700)
+    c = host["config"]
+    prompt = synth.make_rng(91).integers(0, c["vocab"], 37).tolist()
+    res = []
+    for one in (True, False):
+        monkeypatch.setenv("ILT_I8_FEW", "0" if one else "1")
+        monkeypatch.setenv("ILT_I8_TM", tile)
+        m = model.DenseModel(dev, host, nctx=40)
+        m.forward_n(prompt)
+        res.append([hip.hip_floats(m.logits, c["vocab"])] + [hip.hip_floats(m.layers[1][k], 37 * c["nkv"] * c["hd"]) for k in ("kc", "vc")])
+        m.free()
+    for a, b in zip(*res):
+        assert np.isfinite(a).all() and np.array_equal(bits(a), bits(b))
+
+
 @pytest.mark.parametrize("rows_a_tile", ["64", "128"])
 @pytest.mark.parametrize("qtype,rows,cols,n", [(synth.Q2_K, 129, 768, 33), (synth.Q2_K, 64, 256, 130), (synth.IQ2_XXS, 129, 256, 65), (synth.IQ2_XXS, 100, 1280, 128)])
 def test_expert_formats_on_a_dense_matrix_bit_for_bit(dev, monkeypatch, rows_a_tile, qtype, rows, cols, n):
