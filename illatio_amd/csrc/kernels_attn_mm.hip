@@ -190,6 +190,78 @@ __global__ __launch_bounds__(256, R == 16 ? 4 : 2) void attn_values_mm_kernel(co
   }
 }
 
+// Four registers of the four groups of 16 lanes, register and group exchanged.
+__device__ __forceinline__ void across(float* v) {
+  auto swap32 = [](float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(a), __float_as_int(b), false, false);
+    const int x = r[0], y = r[1];
+    a = __int_as_float(x); b = __int_as_float(y);
+  };
+  auto swap16 = [](float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_int(a), __float_as_int(b), false, false);
+    const int x = r[0], y = r[1];
+    a = __int_as_float(x); b = __int_as_float(y);
+  };
+  swap32(v[0], v[2]); swap32(v[1], v[3]);
+  swap16(v[0], v[1]); swap16(v[2], v[3]);
+}
+
+// The same for few rows: a wave takes one row and 64 columns.  What bounds a launch of few waves is a wave's chain of positions, and
+// what a position costs is instructions (a wave alone on its SIMD issues one in 5 cycles): four rows a wave are an instruction of
+// the matrix cores, four adds and a load, one row a multiplication by a score broadcast within its row of lanes, an addition
+// and, the values as 16-byte loads of four positions a wave, a quarter of a load and an exchange between lanes.
+// us for scores, softmax and values: 32 heads of 128 over 8, 8 tokens at 300 positions 16.4 -> 13.4, 21 18.6 -> 17.6, 3 at 2,000
+// 50 -> 36; 14 of 64 over 2, 48 at 300 17.4 -> 15.2, 21 at 2,000 52 -> 37.
+template <int K> __device__ __forceinline__ float times_score(float s, float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x150 + K, 0xF, 0xF, true)) * v;      // row_newbcast:K
+}
+template <int HD, int AHEAD>
+__global__ __launch_bounds__(256) void attn_values_row_kernel(const float* __restrict__ prob, const float* __restrict__ vc, float* __restrict__ out,
+                                                              int nh, int group, int kvd, int pos0, int ntok, int spitch) {
+  constexpr int CG = HD / 64, P = 16;
+  const int kvh = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int id = ((int)gridDim.y - 1 - (int)blockIdx.y) * 4 + wave, row = id / CG, cg = id % CG;
+  if (row >= ntok * group) return;
+  const int t = row / group, h = kvh * group + row - t * group, npos = pos0 + t + 1;
+  const __amdgpu_buffer_rsrc_t rs = ilt_rsrc(ilt_uniform_ptr(prob + ((long long)t * nh + h) * spitch), (u32)npos * 4u);
+  const __amdgpu_buffer_rsrc_t rv = ilt_rsrc(ilt_uniform_ptr(vc), (u32)npos * (u32)kvd * 4u);
+  const int col = 64 * cg + 4 * (lane & 15);
+  u32 vo[P / 4];                                     // the lane's position of each four
+#pragma unroll
+  for (int k = 0; k < P / 4; k++) vo[k] = (u32)(ilt_set_at(4 * k + (lane >> 4), npos) * kvd + kvh * HD + col) * 4u;
+  struct Set { float s, v[P]; };
+  auto load = [&](Set& x, int p) {
+    const u32 base = (u32)ilt_set_base(p, P, npos), bv = base * (u32)kvd * 4u;
+    x.s = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, 4u * (base + (u32)(lane & 15)), 0, 0));
+#pragma unroll
+    for (int k = 0; k < P; k += 4) {
+      const float4 f = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rv, vo[k / 4] + bv, 0, 0));
+      x.v[k] = f.x; x.v[k + 1] = f.y; x.v[k + 2] = f.z; x.v[k + 3] = f.w;
+    }
+  };
+  float acc = 0.0f;
+  auto set = [&](Set& x, int p, auto ownc) {
+    constexpr bool OWN = decltype(ownc)::value;
+    const int base = ilt_set_base(p, P, npos);
+    const u32 left = ilt_set_left(p, npos);
+    auto four = [&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      across(x.v + k);
+      const float d[4] = {times_score<k>(x.s, x.v[k]), times_score<k + 1>(x.s, x.v[k + 1]), times_score<k + 2>(x.s, x.v[k + 2]), times_score<k + 3>(x.s, x.v[k + 3])};
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float a = acc + d[i];
+        acc = !OWN || ilt_set_from(p, base, k + i) < left ? a : acc;
+      }
+    };
+    using std::integral_constant;
+    four(integral_constant<int, 0>{}); four(integral_constant<int, 4>{}); four(integral_constant<int, 8>{}); four(integral_constant<int, 12>{});
+  };
+  Set x[AHEAD];
+  ilt_value_sets<P, AHEAD>(x, npos, npos, load, [&](Set& x, int p) { set(x, p, std::false_type{}); }, [&](Set& x, int p) { set(x, p, std::true_type{}); });
+  out[((long long)t * nh + h) * HD + col + (lane >> 4)] = acc;      // (the exchange leaves column 4 c + g of sixteen c in lane 16 g + c)
+}
+
 }  // namespace
 
 bool ilt_k_attn_mm_takes(const float* q, const float* kc, const float* scratch, const float* out, int nh, int nkv, int hd, int ctx) {
@@ -213,9 +285,19 @@ hipError_t ilt_k_attn_scores_mm(const float* q, const float* kc, float* raw, int
 // Sixteen rows a wave once that leaves about six waves a CU (32 heads of 128 over 8 on 512 tokens, 2,048 waves: 95.7 us for the
 // chunk's attention against 97.6 with four; 1,250 at 1,250 893 against 1,102), else four: a wave's chain of positions, an
 // instruction every few cycles, is the launch's time (256 tokens 41 us against 43, 64 tokens 13.9 against 15.5, 14 heads of 64
-// over 2 on 1,250 121 against 137, 3 tokens at 2,000 55 against 115).
+// over 2 on 1,250 121 against 137).  One row a wave up to 1,400 waves, a little more than the SIMDs (32 heads of 128 over 8 at 300
+// positions, 1,344 waves 17.6 us against 18.6, 2,112 21.1 against 19.3; 14 of 64 over 2, 1,400 19.8 against 20.9, 2,800 30.5 against
+// 29.1); its values three sets ahead up to 512 positions, four past them (3 tokens at 2,000: 35.5 against 39.7).
 hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, int spitch, hipStream_t st) {
   const int group = nh / nkv, rows = ntok * group, cg = hd / 64, wr = 4 / cg;
+  if ((long long)rows * nkv * cg <= 1400) {
+    const dim3 grid(nkv, (rows * cg + 3) / 4);
+#define ILT_VALUES(HD, AHEAD) hipLaunchKernelGGL((attn_values_row_kernel<HD, AHEAD>), grid, dim3(256), 0, st, prob, vc, out, nh, group, nkv * hd, pos0, ntok, spitch)
+    if (pos0 + ntok <= 512) { if (hd == 128) ILT_VALUES(128, 3); else ILT_VALUES(64, 3); }
+    else { if (hd == 128) ILT_VALUES(128, 4); else ILT_VALUES(64, 4); }
+#undef ILT_VALUES
+    return hipGetLastError();
+  }
   const int r = (long long)((rows + 15) / 16) * nkv * cg >= 1600 ? 16 : 4;
   const dim3 grid(nkv, ((rows + r - 1) / r + wr - 1) / wr);
 #define ILT_VALUES(R, HD) hipLaunchKernelGGL((attn_values_mm_kernel<R, HD>), grid, dim3(256), 0, st, prob, vc, out, nh, group, nkv * hd, pos0, ntok, spitch)

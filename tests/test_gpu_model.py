@@ -473,6 +473,14 @@ def test_chunk_attention_with_the_matrix_cores_products(dev, nh, nkv, hd, pos0, 
         hip.hip_free(b)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,pos0,ntok,what", [(32, 8, 128, 301, 33, "nan"), (14, 2, 64, 2, 130, "denormal"), (4, 4, 128, 3, 177, "odd"),      # four rows a wave
+                                                      (2, 1, 128, 0, 2, "nan"), (4, 4, 64, 14, 2, ""), (8, 2, 64, 15, 175, "denormal"),        # one row, 1,400 waves
+                                                      (10, 2, 128, 506, 6, "nan"), (10, 2, 128, 507, 6, "nan"), (6, 6, 64, 2047, 3, "odd")])      # up to and past 512 positions
+def test_chunk_attention_of_one_and_of_four_rows_a_wave(dev, nh, nkv, hd, pos0, ntok, what):
+    """The same where the values take four rows a wave, and one: from two positions on, and around the sixteen of a set."""
+    test_chunk_attention_with_the_matrix_cores_products(dev, nh, nkv, hd, pos0, ntok, what)
+
+
 @pytest.mark.parametrize("nh,pos0,ntok", [(2, 60, 3), (2, 1020, 4), (8, 1100, 130), (8, 2100, 130), (2, 2100, 5), (1, 8000, 192)])
 def test_chunk_softmax_where_the_order_of_the_sum_shows(dev, nh, pos0, ntok):
     """A chunk whose exponentials' sum lies on the edge between two singles for its reciprocal, so that the softmax kernels (a wave
