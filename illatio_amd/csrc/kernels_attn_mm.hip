@@ -206,7 +206,7 @@ __device__ __forceinline__ void across(float* v) {
   swap16(v[0], v[1]); swap16(v[2], v[3]);
 }
 
-// The same for few rows: a wave takes one row and 64 columns.  What bounds a launch of few waves is a wave's chain of positions, and
+// The same for few rows, by the vector ALU alone: a wave takes one row and 64 columns.  What bounds a launch of few waves is a wave's chain of positions, and
 // what a position costs is instructions (a wave alone on its SIMD issues one in 5 cycles): four rows a wave are an instruction of
 // the matrix cores, four adds and a load, one row a multiplication by a score broadcast within its row of lanes, an addition
 // and, the values as 16-byte loads of four positions a wave, a quarter of a load and an exchange between lanes.
@@ -216,7 +216,7 @@ template <int K> __device__ __forceinline__ float times_score(float s, float v) 
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x150 + K, 0xF, 0xF, true)) * v;      // row_newbcast:K
 }
 template <int HD, int AHEAD>
-__global__ __launch_bounds__(256) void attn_values_row_kernel(const float* __restrict__ prob, const float* __restrict__ vc, float* __restrict__ out,
+__global__ __launch_bounds__(256) void attn_values_mm_row_kernel(const float* __restrict__ prob, const float* __restrict__ vc, float* __restrict__ out,
                                                               int nh, int group, int kvd, int pos0, int ntok, int spitch) {
   constexpr int CG = HD / 64, P = 16;
   const int kvh = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -292,7 +292,7 @@ hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, 
   const int group = nh / nkv, rows = ntok * group, cg = hd / 64, wr = 4 / cg;
   if ((long long)rows * nkv * cg <= 1400) {
     const dim3 grid(nkv, (rows * cg + 3) / 4);
-#define ILT_VALUES(HD, AHEAD) hipLaunchKernelGGL((attn_values_row_kernel<HD, AHEAD>), grid, dim3(256), 0, st, prob, vc, out, nh, group, nkv * hd, pos0, ntok, spitch)
+#define ILT_VALUES(HD, AHEAD) hipLaunchKernelGGL((attn_values_mm_row_kernel<HD, AHEAD>), grid, dim3(256), 0, st, prob, vc, out, nh, group, nkv * hd, pos0, ntok, spitch)
     if (pos0 + ntok <= 512) { if (hd == 128) ILT_VALUES(128, 3); else ILT_VALUES(64, 3); }
     else { if (hd == 128) ILT_VALUES(128, 4); else ILT_VALUES(64, 4); }
 #undef ILT_VALUES
