@@ -489,6 +489,11 @@ int ilt_d4_group_scatter(uint64_t stream, int n, int ne, int nu, const uint32_t*
   ILT_REQUIRE(n >= 0 && nu > 0 && (n == 0 || (sel && rank && bases && w && rmap && smap && wrow)));
   return (int)ilt_k_group_scatter(n, ne, nu, sel, rank, bases, w, rmap, smap, wrow, S(stream));
 }
+int ilt_d4_group_rows(uint64_t stream, int n, int ne, int nu, const uint32_t* sel, const float* w, uint32_t* counts, uint32_t* bases, uint32_t* rank,
+                      uint32_t* rmap, uint32_t* smap, float* wrow) {
+  ILT_REQUIRE(n >= 0 && ne > 0 && nu > 0 && counts && bases && (n == 0 || (sel && w && rank && rmap && smap && wrow)));
+  return (int)ilt_k_group_rows(n, ne, nu, sel, w, counts, bases, rank, rmap, smap, wrow, S(stream));
+}
 int ilt_d4_rows_expert(uint64_t stream, int n, const uint32_t* sel, const uint32_t* smap, uint32_t* rexp) {
   ILT_REQUIRE(n >= 0 && (n == 0 || (sel && smap && rexp)));
   return (int)ilt_k_rows_expert(n, sel, smap, rexp, S(stream));
@@ -842,6 +847,11 @@ int ilt_d4_mm_id2_iq2_xxs(uint64_t stream, int ncols, int nrows, int row_bytes, 
 int ilt_d4_gather_q8k(uint64_t stream, int d, int nrows, const int8_t* xq, const float* xd, const uint32_t* map, int8_t* oq, float* od) {
   ILT_REQUIRE(d > 0 && d % 256 == 0 && nrows >= 0 && (nrows == 0 || (xq && xd && map && oq && od)) && (((uintptr_t)xq | (uintptr_t)oq) & 15) == 0);
   return (int)ilt_k_gather_q8k(d, nrows, xq, xd, map, oq, od, S(stream));
+}
+
+int ilt_d4_quant_q8k_rows(uint64_t stream, int d, int ntok, int nu, const float* x, const uint32_t* smap, int8_t* xq, float* xd) {
+  ILT_REQUIRE(d > 0 && d % 256 == 0 && ntok >= 0 && nu >= 1 && nu <= 64 && (ntok == 0 || (x && smap && xq && xd)) && ((uintptr_t)xq & 3) == 0);
+  return (int)ilt_k_quant_q8k_rows(x, smap, ntok, nu, d, xq, xd, S(stream));
 }
 
 int ilt_d4_swiglu_q8(uint64_t stream, int n, int ff, float clamp, const float* g, const float* u, int8_t* xq, float* xs) {
@@ -1467,6 +1477,7 @@ int ilt_launch(const char* kernel, unsigned gx, unsigned gy, unsigned gz, unsign
   K("d4_mm_id2_iq2_xxs")
     return ilt_d4_mm_id2_iq2_xxs(stream, a.i32(0), a.i32(1), a.i32(2), a.i64(3), a.i64(4), a.ptr<const uint64_t*>(5), a.ptr<cu32>(6), a.ptr<cu32>(7),
                                  a.i32(8), a.i64(9), a.ptr<ci8>(10), a.ptr<cf>(11), a.ptr<float*>(12), a.ptr<float*>(13));
+  K("d4_quant_q8k_rows") return ilt_d4_quant_q8k_rows(stream, a.i32(0), a.i32(1), a.i32(2), a.ptr<cf>(3), a.ptr<cu32>(4), a.ptr<int8_t*>(5), a.ptr<float*>(6));
   K("d4_gather_q8k") return ilt_d4_gather_q8k(stream, a.i32(0), a.i32(1), a.ptr<ci8>(2), a.ptr<cf>(3), a.ptr<cu32>(4), a.ptr<int8_t*>(5), a.ptr<float*>(6));
   K("d4_swiglu_q8") return ilt_d4_swiglu_q8(stream, a.i32(0), a.i32(1), a.f32(2), a.ptr<cf>(3), a.ptr<cf>(4), a.ptr<int8_t*>(5), a.ptr<float*>(6));
   K("d4_swiglu_w_q8k") return ilt_d4_swiglu_w_q8k(stream, a.i32(0), a.i32(1), a.f32(2), a.ptr<cf>(3), a.ptr<cf>(4), a.ptr<cf>(5), a.ptr<int8_t*>(6),
@@ -1507,6 +1518,8 @@ int ilt_launch(const char* kernel, unsigned gx, unsigned gy, unsigned gz, unsign
   K("embed_k") return ilt_embed_k(stream, a.i32(0), a.ptr<const void*>(1), a.ptr<const int32_t*>(2), a.ptr<float*>(3), a.i32(4), (int)gx);
   K("d4_route") return ilt_d4_route(stream, a.i32(0), a.i32(1), a.i32(2), a.f32(3), a.i32(4), a.ptr<cf>(5), a.ptr<cf>(6),
                                     a.ptr<const int32_t*>(7), a.ptr<cu32>(8), a.ptr<uint32_t*>(9), a.ptr<float*>(10), (int)gx);
+  K("d4_group_rows") return ilt_d4_group_rows(stream, a.i32(0), a.i32(1), a.i32(2), a.ptr<cu32>(3), a.ptr<cf>(4), a.ptr<uint32_t*>(5), a.ptr<uint32_t*>(6),
+                                              a.ptr<uint32_t*>(7), a.ptr<uint32_t*>(8), a.ptr<uint32_t*>(9), a.ptr<float*>(10));
   K("d4_group_zero") return ilt_d4_group_zero(stream, a.i32(0), a.ptr<uint32_t*>(1));
   K("d4_group_count") return ilt_d4_group_count(stream, a.i32(0), a.i32(1), a.i32(2), a.ptr<cu32>(3), a.ptr<uint32_t*>(4), a.ptr<uint32_t*>(5));
   K("d4_group_scan") return ilt_d4_group_scan(stream, a.i32(0), a.i32(1), a.i32(2), a.ptr<cu32>(3), a.ptr<uint32_t*>(4));

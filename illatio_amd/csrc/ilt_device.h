@@ -199,6 +199,16 @@ __device__ __forceinline__ void ilt_kernarg_warm7() {
 }
 __device__ __forceinline__ void ilt_barrier_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// lane i: the sum of lanes 0 .. i
+__device__ __forceinline__ u32 wave_sums_upto(u32 v) {
+  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);      // row_shr 1, 2, 4, 8
+  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);
+  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);
+  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);
+  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);      // row_bcast 15 to rows 1 and 3
+  return v + (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);      // row_bcast 31 to rows 2 and 3
+}
+
 // SBCL evaluates single-float exp and log by widening to double, calling libm and
 // rounding back (the CPU path's silu, softplus); the kernels do the same.
 __device__ __forceinline__ float ilt_expf_via_double(float x) { return (float)exp((double)x); }

@@ -99,16 +99,6 @@ __device__ __forceinline__ void tile_place(int s, int NT, int NR, int& rt, int& 
   rt = rg * GR + (rem - tt * nr);
 }
 
-// lane i: the sum of lanes 0 .. i
-__device__ __forceinline__ u32 wave_sums_upto(u32 v) {
-  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);      // row_shr 1, 2, 4, 8
-  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);
-  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);
-  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);
-  v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);      // row_bcast 15 to rows 1 and 3
-  return v + (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);      // row_bcast 31 to rows 2 and 3
-}
-
 // LIMIT >= 0: only the tiles before it are dealt out (a multiple of 8; the workgroups from it on take parts of the rest).
 // Grouped: every wave adds up the groups' tiles by itself, four groups a lane (up to 256), without LDS or a barrier: the scan
 // through LDS took 17 barriers, some 2 us of every workgroup's time, those with no tile (two of three) included (24 tokens, 6 of

@@ -170,6 +170,8 @@ hipError_t ilt_k_route(int ne, int nu, int hash, float scale, int has_bias, cons
 // experts, row i on expert rexp[i] of token xrow[i] with weight wrow[i]; smap[token * nu + slot] = the row
 hipError_t ilt_k_small_route(int ne, int nu, float scale, const float* logits, const float* bias, int ntok, uint32_t* rexp, uint32_t* xrow,
                              float* wrow, uint32_t* smap, hipStream_t st);
+hipError_t ilt_k_group_rows(int n, int ne, int nu, const uint32_t* sel, const float* w, uint32_t* counts, uint32_t* bases, uint32_t* rank, uint32_t* rmap,
+                            uint32_t* smap, float* wrow, hipStream_t st);
 hipError_t ilt_k_group_zero(int ne, uint32_t* counts, hipStream_t st);
 hipError_t ilt_k_group_count(int n, int ne, int nu, const uint32_t* sel, uint32_t* counts, uint32_t* rank, hipStream_t st);
 hipError_t ilt_k_group_scan(int n, int ne, int nu, const uint32_t* counts, uint32_t* bases, hipStream_t st);
@@ -177,6 +179,7 @@ hipError_t ilt_k_group_scatter(int n, int ne, int nu, const uint32_t* sel, const
                                const float* w, uint32_t* rmap, uint32_t* smap, float* wrow, hipStream_t st);
 hipError_t ilt_k_rows_expert(int n, const uint32_t* sel, const uint32_t* smap, uint32_t* rexp, hipStream_t st);
 hipError_t ilt_k_gather_rows(int d, int nrows, const float* src, const uint32_t* map, float* x, hipStream_t st);
+hipError_t ilt_k_quant_q8k_rows(const float* x, const uint32_t* smap, int ntok, int nu, int d, int8_t* xq, float* xd, hipStream_t st);
 hipError_t ilt_k_gather_q8k(int d, int nrows, const int8_t* xq, const float* xd, const uint32_t* map, int8_t* oq, float* od, hipStream_t st);
 hipError_t ilt_k_swiglu_w(int n, int ff, float clamp, const float* g, const float* u, const float* w, float* mid,
                           int8_t* xq, float* xs, hipStream_t st);

@@ -67,6 +67,32 @@ __global__ __launch_bounds__(256) void quant_q8_kernel(const float* __restrict__
 // (a 16-byte load, a 4-byte store; no LDS, no barrier).  The largest-magnitude value, the
 // first of equals, sets iscale = -127/max; q = min(127, round-half-even(iscale*x));
 // d = 1/iscale; sums of each 16 quants.
+// A wave's block, four values a lane: its quants and d.
+__device__ __forceinline__ float q8k_block(const float (&v)[4], int lane, int (&q)[4]) {
+  // |v|'s bits order as |v| does; the low word prefers the earlier index
+  u64 key = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const u64 kk = ((u64)__float_as_uint(fabsf(v[k])) << 32) | (u32)(255 - (4 * lane + k));
+    key = kk > key ? kk : key;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const u32 hi = __shfl_xor((u32)(key >> 32), off), lo = __shfl_xor((u32)key, off);
+    const u64 o = ((u64)hi << 32) | lo;
+    key = o > key ? o : key;
+  }
+  const int idx = 255 - (int)(key & 0xFFFFFFFFu);             // the same in every lane
+  const int ik = idx & 3;
+  const float mine = ik == 0 ? v[0] : ik == 1 ? v[1] : ik == 2 ? v[2] : v[3];
+  const float mx = __shfl(mine, idx >> 2);
+  const bool any = (key >> 32) != 0;
+  const float iscale = any ? -127.0f / mx : 0.0f;
+#pragma unroll
+  for (int k = 0; k < 4; k++) q[k] = any ? min(127, (int)rintf(iscale * v[k])) : 0;
+  return any ? 1.0f / iscale : 0.0f;
+}
+__device__ __forceinline__ u32 q8k_pack(const int (&q)[4]) { return (u32)(q[0] & 0xFF) | ((u32)(q[1] & 0xFF) << 8) | ((u32)(q[2] & 0xFF) << 16) | ((u32)(q[3] & 0xFF) << 24); }
 template <int GLU>
 __global__ __launch_bounds__(256) void quant_q8k_kernel(const float* __restrict__ x, const float* __restrict__ up, i8* __restrict__ xq,
                                                         float* __restrict__ xd, int* __restrict__ bsums, u32 nblocks,
@@ -85,37 +111,34 @@ __global__ __launch_bounds__(256) void quant_q8k_kernel(const float* __restrict_
 #pragma unroll
     for (int k = 0; k < 4; k++) v[k] = glu_of<GLU>(v[k], u[k], clamp, wrow, row);
   }
-  // |v|'s bits order as |v| does; the low word prefers the earlier index
-  u64 key = 0;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const u64 kk = ((u64)__float_as_uint(fabsf(v[k])) << 32) | (u32)(255 - (4 * lane + k));
-    key = kk > key ? kk : key;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const u32 hi = __shfl_xor((u32)(key >> 32), off), lo = __shfl_xor((u32)key, off);
-    const u64 o = ((u64)hi << 32) | lo;
-    key = o > key ? o : key;
-  }
-  const int idx = 255 - (int)(key & 0xFFFFFFFFu);             // the same in every lane
-  const int ik = idx & 3;
-  const float mine = ik == 0 ? v[0] : ik == 1 ? v[1] : ik == 2 ? v[2] : v[3];
-  const float mx = __shfl(mine, idx >> 2);
-  int q[4] = {0, 0, 0, 0};
-  float iscale = 0.0f;
-  const bool any = (key >> 32) != 0;
-  if (any) {
-    iscale = -127.0f / mx;
-#pragma unroll
-    for (int k = 0; k < 4; k++) q[k] = min(127, (int)rintf(iscale * v[k]));
-  }
-  ((u32*)(xq + b * 256))[lane] = (u32)(q[0] & 0xFF) | ((u32)(q[1] & 0xFF) << 8) | ((u32)(q[2] & 0xFF) << 16) | ((u32)(q[3] & 0xFF) << 24);
+  int q[4];
+  const float d = q8k_block(v, lane, q);
+  ((u32*)(xq + b * 256))[lane] = q8k_pack(q);
   int s = (q[0] + q[1]) + (q[2] + q[3]);
   s += __shfl_xor(s, 1);
   s += __shfl_xor(s, 2);
   if ((lane & 3) == 0) bsums[b * 16 + (lane >> 2)] = s;
-  if (lane == 0) xd[b] = any ? 1.0f / iscale : 0.0f;
+  if (lane == 0) xd[b] = d;
+}
+
+// The tokens' blocks straight into each of a token's nu rows of a grouping (token t's slot s is row smap[t nu + s]), without the sums.
+__global__ __launch_bounds__(256) void quant_q8k_rows_kernel(const float* __restrict__ x, const u32* __restrict__ smap, int nu, i8* __restrict__ xq,
+                                                             float* __restrict__ xd, u32 nblocks, u32 bpr) {
+  const int lane = threadIdx.x & 63;
+  const u32 b = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (b >= nblocks) return;
+  const u32 tok = b / bpr, at = b - tok * bpr;
+  const float4 v4 = ((const float4*)(x + (long long)b * 256))[lane];
+  const u32 mine = lane < nu ? smap[(long long)tok * nu + lane] : 0u;      // (at most 64 slots)
+  const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+  int q[4];
+  const float d = q8k_block(v, lane, q);
+  const u32 pack = q8k_pack(q);
+  for (int s = 0; s < nu; s++) {
+    const long long o = (long long)(u32)__builtin_amdgcn_readlane(mine, s) * bpr + at;
+    ((u32*)(xq + o * 256))[lane] = pack;
+    if (lane == 0) xd[o] = d;
+  }
 }
 
 // GGUF Q8_0 blocks (f16 d, 32 int8) split into an int8 array and an f16 scale array.
@@ -310,6 +333,14 @@ hipError_t ilt_k_quant_q8(const float* x, int8_t* xq, float* xs, int* xsum, long
 
 hipError_t ilt_k_quant_q8k(const float* x, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st) {
   return launch_q8k<0>(x, nullptr, xq, xd, bsums, nblocks, 0, 0, 0.0f, nullptr, st);
+}
+
+hipError_t ilt_k_quant_q8k_rows(const float* x, const uint32_t* smap, int ntok, int nu, int d, int8_t* xq, float* xd, hipStream_t st) {
+  const long long nblocks = (long long)ntok * (d / 256);
+  if (nblocks <= 0) return hipSuccess;
+  if (d % 256 || nu < 1 || nu > 64 || nblocks > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(quant_q8k_rows_kernel, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, st, x, smap, nu, xq, xd, (u32)nblocks, (u32)(d / 256));
+  return hipGetLastError();
 }
 
 hipError_t ilt_k_swiglu_quant_q8k(const float* gate, const float* up, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st) {

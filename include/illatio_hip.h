@@ -315,6 +315,9 @@ int ilt_d4_group_count(uint64_t stream, int n, int ne, int nu, const uint32_t* s
 int ilt_d4_group_scan(uint64_t stream, int n, int ne, int nu, const uint32_t* counts, uint32_t* bases);
 int ilt_d4_group_scatter(uint64_t stream, int n, int ne, int nu, const uint32_t* sel, const uint32_t* rank,
                          const uint32_t* bases, const float* w, uint32_t* rmap, uint32_t* smap, float* wrow);
+/* Not in the reference: the four d4_group_* launches as one (n rows of nu a token, ne experts). */
+int ilt_d4_group_rows(uint64_t stream, int n, int ne, int nu, const uint32_t* sel, const float* w, uint32_t* counts, uint32_t* bases,
+                      uint32_t* rank, uint32_t* rmap, uint32_t* smap, float* wrow);
 int ilt_d4_gather_rows(uint64_t stream, int d, int nrows, const float* src, const uint32_t* map, float* x);
 /* The expert of every grouped row: rexp[smap[i]] = sel[i] for the n (token, slot) pairs.  With it the indexed
    expert kernels (sel = rexp over the table of all slots, one launch slot a grouped row) take an expert's rows
@@ -495,6 +498,8 @@ int ilt_d4_mm_id2_iq2_xxs(uint64_t stream, int ncols, int nrows, int row_bytes, 
                           const uint32_t* counts, const uint32_t* bases, int ne, int64_t total_rows, const int8_t* xq, const float* xd,
                           float* gate, float* up);
 int ilt_d4_gather_q8k(uint64_t stream, int d, int nrows, const int8_t* xq, const float* xd, const uint32_t* map, int8_t* oq, float* od);
+/* the two before in one: ntok rows of d floats quantized straight into each of their nu grouped rows */
+int ilt_d4_quant_q8k_rows(uint64_t stream, int d, int ntok, int nu, const float* x, const uint32_t* smap, int8_t* xq, float* xd);
 int ilt_d4_swiglu_q8(uint64_t stream, int n, int ff, float clamp, const float* g, const float* u, int8_t* xq, float* xs);   /* Q8_0, a float scale, weights of one */
 int ilt_d4_swiglu_w_q8k(uint64_t stream, int n, int ff, float clamp, const float* g, const float* u, const float* w, int8_t* xq, float* xd,
                         int32_t* bsums);

@@ -147,6 +147,33 @@ def test_route_with_nan_and_masked_scores(dev):
             hip.hip_free(x)
 
 
+@pytest.mark.parametrize("n,ne,nu", [(1, 1, 1), (1, 1024, 64), (16, 64, 64), (341, 5, 3), (1025, 256, 1), (1366, 1000, 3), (8192, 2, 8), (8193, 256, 8)])
+def test_rows_grouped_and_quantized_into_their_places(dev, n, ne, nu):
+    """The grouping's one launch (the last size takes the four: as many rows more than 65,536), around a workgroup's 1,024 rows, with
+    experts that nobody chose; and the tokens' blocks in each of their rows against quant_q8k's, gathered."""
+    from illatio_amd import ds4f, hip
+    rng = synth.make_rng(n + ne + nu)
+    rows, d = n * nu, 512
+    sh = np.sort(rng.integers(0, max(1, ne * 3 // 4), rows)).astype(np.uint32) if n == 341 else (rng.random(rows) ** 3 * ne).astype(np.uint32)
+    wh, xh = rng.standard_normal(rows).astype(np.float32), synth.activations((n, d), rng)
+    xh[0, :256] = 0.0
+    sel, w, x = hip.hip_upload_new(dev, sh), hip.hip_upload_new(dev, wh), hip.hip_upload_new(dev, xh)
+    g = ds4f.group_rows(dev, sel, w, n, ne, nu)
+    get = lambda k, c: hip.hip_download(g[k], np.uint32, c)
+    counts, bases, rmap, smap = get("counts", ne), get("bases", ne), get("rmap", rows), get("smap", rows)
+    assert np.array_equal(counts, np.bincount(sh, minlength=ne)) and np.array_equal(bases, np.cumsum(counts) - counts)
+    assert np.array_equal(np.sort(smap), np.arange(rows)) and np.array_equal(rmap[smap], np.arange(rows) // nu)
+    assert np.array_equal(smap, bases[sh] + get("rank", rows)) and ((smap >= bases[sh]) & (smap < bases[sh] + counts[sh])).all()
+    assert np.array_equal(hip.hip_floats(g["wrow"], rows)[smap], wh)
+    xq, xd, xs = ds4f._q8k(dev, x, n * d)
+    oq, od = hip.hip_alloc(dev, rows * d), hip.hip_alloc(dev, 4 * rows * d // 256)
+    hip.launch(dev, "d4_quant_q8k_rows", (n * d // 256 + 3) // 4, 256, [d, n, nu, x, g["smap"], oq, od])
+    assert np.array_equal(hip.hip_download(oq, np.int8, rows * d).reshape(rows, d), hip.hip_download(xq, np.int8, n * d).reshape(n, d)[rmap])
+    assert np.array_equal(hip.hip_floats(od, rows * d // 256).reshape(rows, -1), hip.hip_floats(xd, n * d // 256).reshape(n, -1)[rmap])
+    for b in [sel, w, x, xq, xd, xs, oq, od] + list(g.values()):
+        hip.hip_free(b)
+
+
 def test_group_rows_invariants_and_gather(dev):
     from illatio_amd import ds4f, hip
     rng = synth.make_rng(5)
