@@ -708,21 +708,24 @@ int ilt_d4_ffn_small(uint64_t stream, void* wsp, uint64_t ws_bytes, int n, int n
     ILT_TRY(ilt_k_small_route(ne, nu, scale, logits, bias, n, rexp, xrow, wrow, smap, S(stream)));
     ILT_TRY(ilt_k_quant_q8(x, xq, xs, nullptr, (long long)n * d / 32, 0, S(stream)));
   }
-  // the shared expert: its matrices once for all the tokens
-  if ((e = ilt_mm_q8_mma2(stream, wt->sgate_q, wt->sgate_d, sg, nullptr, ff, wt->sup_q, wt->sup_d, su, nullptr, ff, nullptr, nullptr, nullptr, nullptr, 0,
-                          xq, xs, d, n, 0))) return e;
-  // the routed experts, a slot a (token, slot) row, an expert's rows one after another
+  // the routed experts, a slot a (token, slot) row, an expert's rows one after another; the shared expert's matrices once for all
+  // the tokens, beside them
   if (share) {
-    ILT_TRY(ilt_k_share_gate_up(wt->slots, 0, wt->gate_bytes, d, ff, rows, rexp, xrow, kq, kd, wrow, clamp, bm, S(stream)));
+    ILT_REQUIRE((((uintptr_t)wt->sgate_q | (uintptr_t)wt->sup_q | (uintptr_t)wt->sdown_q) & 15) == 0);
+    const IltShareBeside gu = {{wt->sgate_q, wt->sup_q}, {wt->sgate_d, wt->sup_d}, {sg, su}, 2, ff, d, n, xq, xs};
+    const IltShareBeside dn = {{wt->sdown_q, nullptr}, {wt->sdown_d, nullptr}, {sout, nullptr}, 1, d, ff, n, mq, ms};
+    ILT_TRY(ilt_k_share_gate_up(wt->slots, 0, wt->gate_bytes, d, ff, rows, rexp, xrow, kq, kd, wrow, clamp, bm, &gu, S(stream)));
     ILT_TRY(ilt_k_share_mid(n, rows, ff, clamp, sg, su, mq, ms, bm, kq, kd, ks, S(stream)));
-    ILT_TRY(ilt_k_share_down(wt->slots, 2 * wt->gate_bytes, ff, d, rows, rexp, kq, kd, ks, bd, S(stream)));
+    ILT_TRY(ilt_k_share_down(wt->slots, 2 * wt->gate_bytes, ff, d, rows, rexp, kq, kd, ks, bd, &dn, S(stream)));
   } else {
+    if ((e = ilt_mm_q8_mma2(stream, wt->sgate_q, wt->sgate_d, sg, nullptr, ff, wt->sup_q, wt->sup_d, su, nullptr, ff, nullptr, nullptr, nullptr, nullptr, 0,
+                            xq, xs, d, n, 0))) return e;
     ILT_TRY(ilt_k_swiglu_w_quant_q8(n, ff, clamp, sg, su, nullptr, mq, ms, S(stream)));
     if ((e = gemv_experts(stream, ILT_IQ2_XXS, d, ff, grb, 0, wt->gate_bytes, d, ff, wt->slots, rows, nullptr, nullptr, nullptr, x, wrow, clamp, bm, rexp,
                           nullptr, nullptr, xrow))) return e;
     if ((e = gemv_experts(stream, ILT_Q2_K, ff, d, drb, 2 * wt->gate_bytes, -1, ff, d, wt->slots, rows, nullptr, nullptr, nullptr, bm, nullptr, 0.0f, bd, rexp))) return e;
+    if ((e = ilt_mm_q8(stream, wt->sdown_q, wt->sdown_d, mq, ms, sout, nullptr, d, ff, n, 0))) return e;
   }
-  if ((e = ilt_mm_q8(stream, wt->sdown_q, wt->sdown_d, mq, ms, sout, nullptr, d, ff, n, 0))) return e;
   return (int)ilt_k_moe_sum_rows(d, nu, n, bd, smap, sout, moe, S(stream));
 }
 

@@ -131,10 +131,13 @@ hipError_t ilt_k_share_open(int ne, int nu, float scale, const float* logits, co
                             uint32_t* smap, const float* x, int d, int8_t* xq, float* xs, int8_t* kq, float* kd, int* bsums, hipStream_t st);
 hipError_t ilt_k_share_mid(int ntok, int rows, int ff, float clamp, const float* g, const float* u, int8_t* mq, float* ms, const float* x, int8_t* kq,
                            float* kd, int* bsums, hipStream_t st);
+// A product of the shared expert that rides along: up to two Q8_0 matrices (rows of cols int8, f16 scales) on ntok <= 9 tokens'
+// quants, results a token a row
+struct IltShareBeside { const int8_t* w[2]; const uint16_t* wd[2]; float* y[2]; int nmat, rows, cols, ntok; const int8_t* xq; const float* xs; };
 hipError_t ilt_k_share_gate_up(const uint64_t* ptrs, long long gate, long long up, int d, int ff, int n, const uint32_t* rexp, const uint32_t* xrow,
-                               const int8_t* kq, const float* kd, const float* wts, float clamp, float* y, hipStream_t st);
+                               const int8_t* kq, const float* kd, const float* wts, float clamp, float* y, const IltShareBeside* beside, hipStream_t st);
 hipError_t ilt_k_share_down(const uint64_t* ptrs, long long add, int ff, int d, int n, const uint32_t* rexp, const int8_t* kq, const float* kd,
-                            const int* bsums, float* y, hipStream_t st);
+                            const int* bsums, float* y, const IltShareBeside* beside, hipStream_t st);
 
 hipError_t ilt_k_quant_q8(const float* x, int8_t* xq, float* xs, int* xsum, long long nblocks, int f16_scale, hipStream_t st);
 hipError_t ilt_k_quant_q8k(const float* x, int8_t* xq, float* xd, int* bsums, long long nblocks, hipStream_t st);

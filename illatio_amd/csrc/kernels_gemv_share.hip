@@ -4,6 +4,7 @@
 #include "ilt_kernels.h"
 #include "ilt_iq2xxs_tables.h"
 #include "ilt_route.h"
+#include <algorithm>
 
 namespace {
 
@@ -18,6 +19,7 @@ struct ShareArgs {
   const float* wts; float clamp;
   float* y;                    // n rows of `rows` results
   int rows, row_bytes, S, n;
+  IltShareBeside beside; int by;        // the shared expert's product in the same launch: the grid's first by rows of workgroups
 };
 
 constexpr int kAhead = 2;      // steps loaded ahead
@@ -145,6 +147,65 @@ __device__ __forceinline__ float share_sum(const float* t, int n) {        // ((
   return o;
 }
 
+// The shared expert's Q8_0 rows on the pass's tokens: a wave takes one row of a matrix (two up to six tokens), 32 blocks a step, two
+// lanes a block; the blocks' float terms in LDS, then a lane a row and token adds them in order.
+// Why here: as launches of their own these products wait for memory, 13 and 8 us of five tokens', and the routed experts' for their
+// instructions, 26 and 14, one after the other; as the first workgroups of the same launch they are over before it (the pass 97 -> 84 us, waiting for it
+// included).
+constexpr int kBesideTokens = 9;
+__device__ __forceinline__ void share_beside(const IltShareBeside& q, int at, u8* smem) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 1;
+  const int nb = q.cols >> 5, rw = q.ntok <= 6 ? 2 : 1, r0 = (at * 4 + wave) * rw;
+  if (r0 >= q.nmat * q.rows) return;                   // (whole waves; no barrier below)
+  const int m = r0 >= q.rows ? 1 : 0, row = r0 - m * q.rows;       // (an even number of rows a matrix)
+  const i8* const w = (const i8*)ilt_uniform_ptr(m ? q.w[1] : q.w[0]) + (long)row * q.cols;
+  const u16* const wd = (const u16*)ilt_uniform_ptr(m ? q.wd[1] : q.wd[0]) + (long)row * nb;
+  const int pitch = nb + 1;                            // (a float between rows: the sums' lanes on different banks)
+  float* const terms = (float*)smem + (long)wave * rw * q.ntok * pitch;
+  const int steps = (q.cols + 1023) >> 10;             // at most four
+  int4 wv[2][4]; u16 dv[2][4];
+#pragma unroll
+  for (int r = 0; r < 2; r++)
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+      if (r < rw && s < steps) {
+        const int c = min(1024 * s + 16 * lane, q.cols - 16);
+        wv[r][s] = *(const int4*)(w + (long)r * q.cols + c);
+        dv[r][s] = wd[(long)r * nb + (c >> 5)];
+      }
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+    if (s < steps) {
+      const int c = min(1024 * s + 16 * lane, q.cols - 16), b = c >> 5;
+      const bool live = 1024 * s + 16 * lane < q.cols;
+      const float d0 = ilt_h2f(dv[0][s]), d1 = ilt_h2f(dv[1][s]);
+#pragma unroll
+      for (int t0 = 0; t0 < kBesideTokens; t0 += 2)
+        if (t0 < q.ntok) {
+          int4 x[2]; float dx[2];
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+            const int tk = min(t0 + t, q.ntok - 1);
+            x[t] = *(const int4*)(q.xq + (long)tk * q.cols + c);
+            dx[t] = q.xs[(long)tk * nb + b];
+          }
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+            const int i0 = ilt_sum2(ilt_dot16(wv[0][s], x[t], 0)), i1 = rw > 1 ? ilt_sum2(ilt_dot16(wv[1][s], x[t], 0)) : 0;
+            const float v = (float)(j ? i1 : i0) * ((j ? d1 : d0) * dx[t]);      // lane 0 of a block the first row's term, lane 1 the second's
+            if (live && j < rw && t0 + t < q.ntok) ilt_lds_stf(terms + (j * q.ntok + t0 + t) * pitch + b, v);
+          }
+        }
+    }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (lane < rw * q.ntok) {
+    const int r = lane / q.ntok, t = lane - r * q.ntok;
+    (m ? q.y[1] : q.y[0])[(long)t * q.rows + row + r] = share_sum(terms + lane * pitch, nb);
+  }
+}
+
 // Grid y: up to R rows of an expert (as many workgroups as rows: those past the last group end at once).  A wave: STEPS steps of
 // whole rows of up to 16 blocks (four lanes a block) of each matrix.  A step's blocks lie at the same place in their rows in every
 // step, so a lane's share of the R rows of activations stays in registers.
@@ -160,6 +221,8 @@ __global__ __launch_bounds__(256, 5) void share_kernel(ShareArgs p) {
   using F = ShareFmt<FMT>;
   constexpr int R = F::R;
   extern __shared__ __align__(16) unsigned char smem[];
+  if ((int)blockIdx.y < p.by) { share_beside(p.beside, blockIdx.y * gridDim.x + blockIdx.x, smem); return; }
+  const int group = (int)blockIdx.y - p.by;
   u32* const tab = (u32*)smem;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 3;
   int y0 = -1;
@@ -168,7 +231,7 @@ __global__ __launch_bounds__(256, 5) void share_kernel(ShareArgs p) {
     const u32 v = p.rexp[min(i, p.n - 1)], pv = p.rexp[max(min(i, p.n - 1) - 1, 0)];
     const u64 upto = ~0ull >> (63 - lane), starts = __ballot(i < p.n && (i == 0 || v != pv)), mine = starts & upto;
     const bool first = i < p.n && (i - (mine ? c + 63 - __builtin_clzll(mine) : run)) % R == 0;
-    const u64 firsts = __ballot(first), hit = __ballot(first && groups + __builtin_popcountll(firsts & upto) - 1 == (int)blockIdx.y);
+    const u64 firsts = __ballot(first), hit = __ballot(first && groups + __builtin_popcountll(firsts & upto) - 1 == group);
     if (hit) { y0 = c + __builtin_ctzll(hit); break; }
     groups += __builtin_popcountll(firsts);
     if (starts) run = c + 63 - __builtin_clzll(starts);
@@ -179,6 +242,7 @@ __global__ __launch_bounds__(256, 5) void share_kernel(ShareArgs p) {
   int nr = 1;
 #pragma unroll
   for (int r = 1; r < R; r++) nr += p.rexp[min(y0 + r, p.n - 1)] == e && y0 + r < p.n;      // (an expert's rows lie side by side)
+  nr = __builtin_amdgcn_readfirstlane(nr);
 
   const int S = p.S, rps = 16 / S, rb = F::STEPS * rps;      // rows a step, rows a wave
   // this lane's block of a step (lanes past the last whole row: block 0 once more, and no terms), its row of the step, its place there
@@ -332,11 +396,19 @@ __global__ __launch_bounds__(256) void share_mid_kernel(u32 nshared, const float
 }
 
 template <int FMT>
-hipError_t launch_share(const ShareArgs& p, hipStream_t st) {
+hipError_t launch_share(ShareArgs& p, const IltShareBeside* beside, hipStream_t st) {
   using F = ShareFmt<FMT>;
-  const int S = p.S, rb = F::STEPS * (16 / S);
-  const size_t lds = (FMT == ILT_IQ2_XXS ? 384 * 4 : 0) + 4ull * F::R * F::MATS * rb * (S * F::TERMS + 1) * 4;
-  hipLaunchKernelGGL(share_kernel<FMT>, dim3((p.rows + 4 * rb - 1) / (4 * rb), p.n), dim3(256), lds, st, p);
+  const int S = p.S, rb = F::STEPS * (16 / S), gx = (p.rows + 4 * rb - 1) / (4 * rb);
+  size_t lds = (FMT == ILT_IQ2_XXS ? 384 * 4 : 0) + 4ull * F::R * F::MATS * rb * (S * F::TERMS + 1) * 4;
+  if (beside) {
+    const IltShareBeside& q = *beside;
+    if (q.ntok < 1 || q.ntok > kBesideTokens || q.cols < 256 || q.cols > 4096 || q.cols % 256 || q.rows < 2 || q.rows % 2 || q.nmat < 1 || q.nmat > 2) return hipErrorInvalidValue;
+    const int rw = q.ntok <= 6 ? 2 : 1, tiles = (q.nmat * q.rows + 4 * rw - 1) / (4 * rw);
+    p.beside = q; p.by = (tiles + gx - 1) / gx;
+    lds = std::max(lds, (size_t)16 * rw * q.ntok * (q.cols / 32 + 1));      // (25 KB at most)
+  }
+  if (p.n + p.by > 65535) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(share_kernel<FMT>, dim3(gx, p.n + p.by), dim3(256), lds, st, p);
   return hipGetLastError();
 }
 
@@ -375,19 +447,19 @@ hipError_t ilt_k_share_mid(int ntok, int rows, int ff, float clamp, const float*
 }
 
 hipError_t ilt_k_share_gate_up(const uint64_t* ptrs, long long gate, long long up, int d, int ff, int n, const uint32_t* rexp, const uint32_t* xrow,
-                               const int8_t* kq, const float* kd, const float* wts, float clamp, float* y, hipStream_t st) {
+                               const int8_t* kq, const float* kd, const float* wts, float clamp, float* y, const IltShareBeside* beside, hipStream_t st) {
   if (n < 1 || n > 65535) return hipErrorInvalidValue;
   ShareArgs p = {};
   p.ptrs = (const u64*)ptrs; p.rexp = rexp; p.xrow = xrow; p.xq = kq; p.xd = kd; p.add = gate; p.add2 = up; p.wts = wts; p.clamp = clamp; p.y = y;
   p.rows = ff; p.row_bytes = d / 256 * 66; p.S = d / 256; p.n = n;
-  return launch_share<ILT_IQ2_XXS>(p, st);
+  return launch_share<ILT_IQ2_XXS>(p, beside, st);
 }
 
 hipError_t ilt_k_share_down(const uint64_t* ptrs, long long add, int ff, int d, int n, const uint32_t* rexp, const int8_t* kq, const float* kd,
-                            const int* bsums, float* y, hipStream_t st) {
+                            const int* bsums, float* y, const IltShareBeside* beside, hipStream_t st) {
   if (n < 1 || n > 65535) return hipErrorInvalidValue;
   ShareArgs p = {};
   p.ptrs = (const u64*)ptrs; p.rexp = rexp; p.xq = kq; p.xd = kd; p.bsums = bsums; p.add = add; p.y = y;
   p.rows = d; p.row_bytes = ff / 256 * 84; p.S = ff / 256; p.n = n;
-  return launch_share<ILT_Q2_K>(p, st);
+  return launch_share<ILT_Q2_K>(p, beside, st);
 }

@@ -313,9 +313,9 @@ def ffn_small(dev, pool, sh, logits, norm2, n, ne, nu, scale, clamp, bias=None, 
     """The FFN past the router for a short pass's N <= 9 tokens (DK-FFN-SMALL,
     cuda-ds4f-spec.lisp:30-100: a speculative step's verification), every token with decode's
     bits.  The reference routes on the CPU and hands each expert its tokens' rows through
-    counts/bases; here one call (ilt_d4_ffn_small) queues seven launches: the routing leaves the
+    counts/bases; here one call (ilt_d4_ffn_small) queues five launches: the routing leaves the
     (token, slot) rows on the device in the order of their experts, and the expert kernels decode an
-    expert's blocks once for up to three of its rows.  Returns
+    expert's blocks once for up to three of its rows, the shared expert's products beside them.  Returns
     MOE (N x d), a new DBuf, when it is there.  GROUPED "counts": DK-FFN-SMALL's own launches with its argument lists
     (cuda-ds4f-spec.lisp:82-88) -- d4_gather_rows, d4_mv_iq2_xxs for the gates and again for the ups,
     d4_swiglu_w, d4_mv_q2_k, each expert kernel over all NE slots with the counts and bases that

@@ -405,6 +405,13 @@ def test_moe_short_pass_over_groups_and_widths(dev, ne, d, ff, nu, n):
     pool.free(); sh.free()
 
 
+# the shared expert's rows beside the routed experts': two rows a wave at their last number of tokens, one at its first, a last step
+# of columns that is a quarter and three quarters of one
+@pytest.mark.parametrize("ne,d,ff,nu,n", [(4, 1280, 512, 2, 6), (5, 512, 1792, 2, 6), (4, 1280, 768, 3, 7), (3, 3840, 256, 1, 2)])
+def test_moe_short_pass_with_the_shared_expert_beside(dev, ne, d, ff, nu, n):
+    test_moe_short_pass_over_groups_and_widths(dev, ne, d, ff, nu, n)
+
+
 @pytest.mark.parametrize("d,ff,n,clamp", [(512, 256, 37, 0.05), (4096, 2048, 130, 0.0)])
 def test_shared_expert_over_a_chunk_bit_exact(dev, d, ff, n, clamp):
     """The shared expert of a chunk through d4_mm_q8_0 (DK-FFN-HEAD-CHUNK, cuda-ds4f-prefill.lisp:294-298): every
