@@ -29,8 +29,9 @@ __device__ __forceinline__ float part(const float4& v, int e) { return e == 0 ? 
 // positions.  Block m of the instruction has columns 4m + e of every sixteen, so its results are the running sums e, 4 + e,
 // 8 + e and 12 + e of 256 scores, and a lane's four 16-byte pieces of a row (or a key) are its operands for e = 0 .. 3.
 // Positions are the results' rows: a lane stores four scores of one row.
-template <int NJ>      // hd / 16
-__global__ __launch_bounds__(256, 3) void attn_scores_mm_kernel(const float* __restrict__ q, const float* __restrict__ kc, float* __restrict__ raw,
+// QL: the rows' operands in LDS, a read an instruction, and four waves a SIMD instead of three.
+template <int NJ, bool QL>      // hd / 16
+__global__ __launch_bounds__(256, QL ? 4 : 3) void attn_scores_mm_kernel(const float* __restrict__ q, const float* __restrict__ kc, float* __restrict__ raw,
                                                                 int nh, int group, int kvd, int pos0, int ntok, float scale, int spitch, int npt) {
   constexpr int HD = 16 * NJ;
   const int kvh = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -42,9 +43,17 @@ __global__ __launch_bounds__(256, 3) void attn_scores_mm_kernel(const float* __r
   if (p0 >= pend) return;
   const int row = min(r0 + i, rows - 1), t = row / group, h = kvh * group + row - t * group;
   const float* const qr = q + ((long long)t * nh + h) * HD + 4 * m;
+  __shared__ float qs[QL ? 4 : 1][QL ? 4 * NJ : 1][64];       // (a wave's own: no barrier)
   float4 qa[NJ], ka[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; j++) qa[j] = *(const float4*)(qr + 16 * j);
+  if constexpr (QL) {
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) qs[wave][4 * j + e][lane] = part(qa[j], e);
+  }
+  auto qpart = [&](int j, int e) { if constexpr (QL) return qs[wave][4 * j + e][lane]; else return part(qa[j], e); };
   float* const dst = raw + ((long long)t * nh + h) * spitch + 4 * m;
   const float* const kbase = kc + (long long)kvh * HD + 4 * m;
   auto load = [&](int p) {
@@ -58,12 +67,12 @@ __global__ __launch_bounds__(256, 3) void attn_scores_mm_kernel(const float* __r
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       const v16f zero = {};
-      v16f s = __builtin_amdgcn_mfma_f32_16x16x1f32(part(ka[0], e), part(qa[0], e), zero, 0, 0, 0);
-      v16f d = __builtin_amdgcn_mfma_f32_16x16x1f32(part(ka[1], e), part(qa[1], e), zero, 0, 0, 0);
+      v16f s = __builtin_amdgcn_mfma_f32_16x16x1f32(part(ka[0], e), qpart(0, e), zero, 0, 0, 0);
+      v16f d = __builtin_amdgcn_mfma_f32_16x16x1f32(part(ka[1], e), qpart(1, e), zero, 0, 0, 0);
 #pragma unroll
       for (int j = 2; j <= NJ; j++) {
         v16f dn = {};
-        if (j < NJ) dn = __builtin_amdgcn_mfma_f32_16x16x1f32(part(ka[j], e), part(qa[j], e), zero, 0, 0, 0);
+        if (j < NJ) dn = __builtin_amdgcn_mfma_f32_16x16x1f32(part(ka[j], e), qpart(j, e), zero, 0, 0, 0);
 #pragma unroll
         for (int r = 0; r < 16; r++) s[r] = s[r] + d[r];
         asm volatile("" : "+v"(s));
@@ -269,16 +278,21 @@ bool ilt_k_attn_mm_takes(const float* q, const float* kc, const float* scratch, 
          (long long)ctx * nkv * hd < (1LL << 30) && 17LL * nh * (ctx + 3) < (1LL << 30);                         // 32-bit offsets: the values, a tile's rows
 }
 
-// A wave's position tiles: four, its rows' loads and the launch's waves shared among them, where the launch has more than twice
-// what the chip holds (512 tokens at none before 95 us for the chunk's attention with four, 99 with one; 1,250 at 1,250 917 and
-// 1,083); one below (21 tokens at 300: 23 us against 27).
+// A wave's position tiles, its rows' loads and the launch's waves shared among them: one where the launch has no more than twice what
+// the chip holds (21 tokens at 300: 23 us against 27 for the chunk's attention), four from there on (512 tokens at none before 95 against
+// 99), sixteen from 100,000 tiles on (scores of 1,250 tokens at 1,250, 32 heads of 128 over 8: four 439 us, eight 431, sixteen 414; 14
+// of 64 over 2 109, 105, 104; 512 at none, 33,000 tiles, 39, 47, 49).  The rows' operands in LDS past 16,384 tiles (454 -> 439; 512 at
+// none 40.5 -> 39.1; 256 at none, 8,192, 15.3 against 16.0).
 hipError_t ilt_k_attn_scores_mm(const float* q, const float* kc, float* raw, int nh, int nkv, int hd, int pos0, int ntok, float scale, int spitch,
                                 hipStream_t st) {
   const int group = nh / nkv, rtiles = (ntok * group + 15) / 16, ptiles = (pos0 + ntok + 15) / 16;
-  const int npt = (long long)rtiles * nkv * ptiles < 8192 ? 1 : 4;
+  const long long tiles = (long long)rtiles * nkv * ptiles;
+  const int npt = tiles < 8192 ? 1 : tiles < 100000 ? 4 : 16;
   const dim3 grid(nkv, (ptiles + npt - 1) / npt, (rtiles + 3) / 4);
-  if (hd == 128) hipLaunchKernelGGL(attn_scores_mm_kernel<8>, grid, dim3(256), 0, st, q, kc, raw, nh, group, nkv * hd, pos0, ntok, scale, spitch, npt);
-  else hipLaunchKernelGGL(attn_scores_mm_kernel<4>, grid, dim3(256), 0, st, q, kc, raw, nh, group, nkv * hd, pos0, ntok, scale, spitch, npt);
+#define ILT_SCORES(NJ, QL) hipLaunchKernelGGL((attn_scores_mm_kernel<NJ, QL>), grid, dim3(256), 0, st, q, kc, raw, nh, group, nkv * hd, pos0, ntok, scale, spitch, npt)
+  if (tiles > 16384) { if (hd == 128) ILT_SCORES(8, true); else ILT_SCORES(4, true); }
+  else { if (hd == 128) ILT_SCORES(8, false); else ILT_SCORES(4, false); }
+#undef ILT_SCORES
   return hipGetLastError();
 }
 
