@@ -565,34 +565,55 @@ __device__ __forceinline__ void reg_tile(const BfParams& p, const u8* w, int r0,
   store_tile<NP, 1>(sum, p, tok0, ntok, r0, wt0, wr0, l32, lh);
 }
 
-// Rows r0 .. x tokens tok0 .. tok0 + ntok - 1 where the launch has few tiles: a tile of 32 rows x 32 tokens is KS waves', super-block
-// u wave u mod KS's, 4 / KS tiles of rows a workgroup.  What bounds such a launch is the chain of a row's blocks: a wave alone on
-// its SIMD issues an instruction in 5 cycles, 1.4 us a block, whatever the rest of the chip could do meanwhile.  A block's
-// integers and float terms depend on nothing before them, only the sums' order does, so every wave makes its blocks' terms as
-// reg_tile does (its own loads, operands and products, a block ahead: nothing shared), leaves them in LDS, and once a round -- KS
-// blocks -- each adds the terms of its own 4 / KS quarters of the tile in the CPU's order.  A round takes 1.95 us (four waves of a CU
-// share its LDS and the loads' way: 1.6 without the loads).  us before and now, matrices from memory: Q6_K 2560 x 9728 on 33 to 96
-// tokens 41-43 -> 26-27, on 160 62 -> 43; 4096 x 4096 on 64 28 -> 15; Q4_K 2560 x 4096 on 40 16.7 -> 12.8, on 128 24 -> 20.
-template <int FMT, int KS> struct SplitSmem {
-  RegSmem<32, 2 * RegW<FMT>::LBYTES, RegW<FMT>::MINS, 2> w[4];
-  __align__(16) float ex[4 / KS][4][KS][RegW<FMT>::MINS ? 2 : 1][256];       // terms [rows' tile][quarter][wave][a term][lane's four]
+// A quarter of a tile's results to y: tokens t0 .. t0 + 3 of the row
+__device__ __forceinline__ void split_store(const BfParams& p, const v4f& sum, long tok0, int ntok, int row, int t0) {
+  const bool ok = row < p.rows;
+  const __amdgpu_buffer_rsrc_t ry = ilt_rsrc(ilt_uniform_ptr(p.y + tok0 * p.ldy), ((u32)(ntok - 1) * (u32)p.ldy + (u32)p.rows) * 4);
+  const u32 rows4 = (u32)p.ldy * 4, base = ok ? (u32)(t0 * (int)p.ldy + row) * 4 : 0x80000000u;
+  const float bv = p.bias && ok ? p.bias[row] : 0.0f;
+  float old[4];
+  if (p.acc) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) old[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ry, base + (u32)r * rows4, 0, 0));
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    float v = sum[r];
+    if (p.bias) v = v + bv;
+    if (p.acc) v = old[r] + v;
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, v), ry, base + (u32)r * rows4, 0, 0);
+  }
+}
+
+// Rows r0 .. x tokens tok0 .. tok0 + ntok - 1 where the launch has few tiles: a tile of 32 rows x 32 tokens is a workgroup's, its
+// super-block u wave u mod 4's.  What bounds such a launch is the chain of a row's blocks: a wave alone on its SIMD issues an
+// instruction in 5 cycles, 1.4 us a block, whatever the rest of the chip could do meanwhile.  A block's integers and float terms
+// depend on nothing before them, only the sums' order does, so every wave makes its blocks' terms as reg_tile does (its own loads,
+// operands and products, a block ahead: nothing shared), leaves them in LDS, and once a round -- four blocks -- each adds the terms of
+// its own quarter of the tile in the CPU's order.  A round takes 1.95 us (four waves of a CU share its LDS and the loads' way: 1.6
+// without the loads).  us before and now, matrices from memory: Q6_K 2560 x 9728 on 33 to 96 tokens 41-43 -> 26-27; 4096 x 4096 on 64
+// 28 -> 15; Q4_K 2560 x 4096 on 40 16.7 -> 12.8.  (Two waves a tile and two tiles of rows a workgroup: on 160 tokens 43.)
+constexpr int KS = 4;                  // waves of a workgroup, and super-blocks of a round
+template <int FMT> struct SplitSmem {
+  RegSmem<32, 2 * RegW<FMT>::LBYTES, RegW<FMT>::MINS, 2> w[KS];
+  __align__(16) float ex[KS][KS][RegW<FMT>::MINS ? 2 : 1][256];       // terms [quarter][wave][a term][lane's four]
 };
-template <int FMT, int KS>
+template <int FMT>
 __device__ __forceinline__ void reg_split(const BfParams& p, const u8* w, int r0, long tok0, int ntok, unsigned char* smem) {
   using F = RegW<FMT>;
-  constexpr int OWN = 4 / KS, TERMS = F::MINS ? 2 : 1;
-  static_assert(F::PLANES == 2 && (KS == 2 || KS == 4), "");
-  SplitSmem<FMT, KS>& W = *(SplitSmem<FMT, KS>*)smem;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ks = wave % KS, wr = wave / KS;
-  auto& S = W.w[wave];
+  constexpr int TERMS = F::MINS ? 2 : 1;
+  static_assert(F::PLANES == 2, "a result's integer is two planes");
+  SplitSmem<FMT>& W = *(SplitSmem<FMT>*)smem;
+  const int lane = threadIdx.x & 63, ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto& S = W.w[ks];
   const int nsb = p.cols / 256, rounds = (nsb + KS - 1) / KS;
-  const int l32 = lane & 31, lh = lane >> 5, wr0 = 32 * wr;
+  const int l32 = lane & 31, lh = lane >> 5;
   const u32 row_bytes = (u32)(nsb * F::BLOCK);
   const __amdgpu_buffer_rsrc_t rw = ilt_rsrc(ilt_uniform_ptr(w), (u32)p.rows * row_bytes);      // (past the matrix's rows: zeros)
-  const typename F::At at = F::place(row_bytes, lane, r0 + wr0, p.rows);
+  const typename F::At at = F::place(row_bytes, lane, r0, p.rows);
   auto issue_w = [&](int sb, int buf) {
 #pragma unroll
-    for (int i = 0; i < F::LOADS; i++) F::issue(i, rw, w, at, row_bytes, (u32)(r0 + wr0), (u32)sb * F::BLOCK, S.ws + buf * F::LBYTES);
+    for (int i = 0; i < F::LOADS; i++) F::issue(i, rw, w, at, row_bytes, (u32)r0, (u32)sb * F::BLOCK, S.ws + buf * F::LBYTES);
   };
   ntok = __builtin_amdgcn_readfirstlane(ntok);
   const __amdgpu_buffer_rsrc_t rx = ilt_rsrc(ilt_uniform_ptr((const i8*)p.x + tok0 * (long)p.cols), (u32)(ntok * p.cols));      // (past the tile's tokens: zeros)
@@ -627,9 +648,7 @@ __device__ __forceinline__ void reg_split(const BfParams& p, const u8* w, int r0
     }
   };
   const u32 x0 = (u32)(l32 >> 2) * 1088 + (u32)(l32 & 3) * 256 + 16 * (u32)(lh ^ (l32 & 3)), x1 = x0 ^ 32;
-  v4f sum[OWN];
-#pragma unroll
-  for (int o = 0; o < OWN; o++) sum[o] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
   v4i hi[8], lo[8];
   typename F::Block blk;
   auto mine = [&](int i) { return min(i * KS + ks, nsb - 1); };      // the wave's block of round i (past the last: the last again, for nobody)
@@ -650,7 +669,7 @@ __device__ __forceinline__ void reg_split(const BfParams& p, const u8* w, int r0
   float dprev = 0.0f, dmprev = 0.0f;
 #pragma unroll
   for (int r = 0; r < 16; r++) P[r] = 0;
-  float* const ex = (float*)W.ex[wr];
+  float* const ex = (float*)W.ex;
   // four results' terms, of the round before, to their quarter's place
   auto term = [&](int j, const float4& y) {
     float a[4], b[4], f[4];
@@ -663,26 +682,23 @@ __device__ __forceinline__ void reg_split(const BfParams& p, const u8* w, int r0
     if constexpr (F::MINS) *ILT_LDS_PTR(v4f, o) = v4f{a[0], a[1], a[2], a[3]};
     *ILT_LDS_PTR(v4f, o + (TERMS - 1) * 256) = v4f{b[0], b[1], b[2], b[3]};
   };
-  // the wave's quarters: the terms of round i's blocks in order
+  // the wave's quarter: the terms of round i's blocks in order
   auto add = [&](int i) {
+    v4f t[KS][TERMS];
 #pragma unroll
-    for (int o = 0; o < OWN; o++) {
-      v4f t[KS][TERMS];
+    for (int s = 0; s < KS; s++)
 #pragma unroll
-      for (int s = 0; s < KS; s++)
+      for (int k = 0; k < TERMS; k++) t[s][k] = *ILT_LDS_PTR(const v4f, ex + ((ks * KS + s) * TERMS + k) * 256 + 4 * lane);
 #pragma unroll
-        for (int k = 0; k < TERMS; k++) t[s][k] = *ILT_LDS_PTR(const v4f, ex + (((ks * OWN + o) * KS + s) * TERMS + k) * 256 + 4 * lane);
+    for (int s = 0; s < KS; s++)
+      if (i * KS + s < nsb) {
 #pragma unroll
-      for (int s = 0; s < KS; s++)
-        if (i * KS + s < nsb) {
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            if constexpr (F::MINS) sum[o][r] = sum[o][r] - t[s][0][r];
-            sum[o][r] = sum[o][r] + t[s][TERMS - 1][r];
-          }
+        for (int r = 0; r < 4; r++) {
+          if constexpr (F::MINS) sum[r] = sum[r] - t[s][0][r];
+          sum[r] = sum[r] + t[s][TERMS - 1][r];
         }
-      asm volatile("" : "+v"(sum[o]));               // (the reads have come back before the wave meets the next barrier)
-    }
+      }
+    asm volatile("" : "+v"(sum));                    // (the reads have come back before the wave meets the next barrier)
   };
   int c0 = 0, c1 = 1, c2 = 2;
 #pragma unroll 1
@@ -744,27 +760,183 @@ __device__ __forceinline__ void reg_split(const BfParams& p, const u8* w, int r0
   }
   ilt_barrier_lds();
   add(rounds - 1);
-  // results: tokens 8 j + 4 lh .. of the row
-  const int row = r0 + wr0 + l32;
-  const bool ok = row < p.rows;
-  const __amdgpu_buffer_rsrc_t ry = ilt_rsrc(ilt_uniform_ptr(p.y + tok0 * p.ldy), ((u32)(ntok - 1) * (u32)p.ldy + (u32)p.rows) * 4);
-  const u32 rows4 = (u32)p.ldy * 4, base = ok ? (u32)((8 * OWN * ks + 4 * lh) * (int)p.ldy + row) * 4 : 0x80000000u;
-  const float bv = p.bias && ok ? p.bias[row] : 0.0f;
+  split_store(p, sum, tok0, ntok, r0 + l32, 8 * ks + 4 * lh);
+}
+
+// The same with two workgroups a CU, where there are more tiles than CUs: one buffer for the tokens and one for the rows' blocks, asked
+// for anew as soon as a block is through, so that a wave waits for them while the other workgroup's waves work; the tokens' sums in
+// registers; and of a block's terms only those in LDS that another wave adds: 77 to 79 KB.  Alone on a CU it takes 2.25 us
+// a round for reg_split's 1.95, two of them 3.15.  us with whole tiles and now, matrices from memory: Q6_K 2560 x 9728 on 160 tokens
+// 62 -> 37, on 256 62 -> 54; 4096 x 4096 on 128 28 -> 20; Q4_K 2560 x 4096 on 128 24 -> 18.
+template <int FMT> struct SplitSmem2 {
+  struct { __align__(16) u8 xs[8192]; __align__(16) u8 ws[RegW<FMT>::LBYTES]; float xd[2][32]; } w[KS];
+  __align__(16) float ex[KS][KS - 1][RegW<FMT>::MINS ? 2 : 1][256];       // terms [quarter][the other waves in turn][a term][lane's four]
+};
+template <int FMT>
+__device__ __forceinline__ void reg_split2(const BfParams& p, const u8* w, int r0, long tok0, int ntok, unsigned char* smem) {
+  using F = RegW<FMT>;
+  constexpr int TERMS = F::MINS ? 2 : 1;
+  static_assert(F::PLANES == 2, "a result's integer is two planes");
+  SplitSmem2<FMT>& W = *(SplitSmem2<FMT>*)smem;
+  const int lane = threadIdx.x & 63, ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto& S = W.w[ks];
+  const int nsb = p.cols / 256, rounds = (nsb + KS - 1) / KS;
+  const int l32 = lane & 31, lh = lane >> 5;
+  const u32 row_bytes = (u32)(nsb * F::BLOCK);
+  const __amdgpu_buffer_rsrc_t rw = ilt_rsrc(ilt_uniform_ptr(w), (u32)p.rows * row_bytes);      // (past the matrix's rows: zeros)
+  const typename F::At at = F::place(row_bytes, lane, r0, p.rows);
+  ntok = __builtin_amdgcn_readfirstlane(ntok);
+  const __amdgpu_buffer_rsrc_t rx = ilt_rsrc(ilt_uniform_ptr((const i8*)p.x + tok0 * (long)p.cols), (u32)(ntok * p.cols));      // (past the tile's tokens: zeros)
+  // the tokens' quants: a kilobyte the half of a super-block of eight tokens, piece q of token t at q ^ (t >> 1 & 7) of its eight
+  const u32 xpc = 16 * (u32)((lane & 7) ^ ((lane >> 4) & 3)), xrow = (u32)(lane >> 3) * (u32)p.cols;
+  const __amdgpu_buffer_rsrc_t rd = ilt_rsrc(ilt_uniform_ptr(p.xd + tok0 * nsb), (u32)(ntok * nsb) * 4);
+  const __amdgpu_buffer_rsrc_t rb = ilt_rsrc(ilt_uniform_ptr(p.bsums + (F::MINS ? tok0 * (p.cols >> 4) : 0)), F::MINS ? (u32)(ntok * (p.cols >> 4)) * 4 : 0);
+  float c_yd; int4 c_bs[4];
+  auto mine = [&](int i) { return min(i * KS + ks, nsb - 1); };      // the wave's block of round i (past the last: the last again, for nobody)
+  auto issue_w = [&](int sb) {
 #pragma unroll
-  for (int o = 0; o < OWN; o++) {
-    float old[4];
-    if (p.acc) {
+    for (int i = 0; i < F::LOADS; i++) F::issue(i, rw, w, at, row_bytes, (u32)r0, (u32)sb * F::BLOCK, S.ws);
+  };
+  auto issue_x = [&](int sb) {                       // and the token's scale and sums of 16, a token two lanes
 #pragma unroll
-      for (int r = 0; r < 4; r++) old[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ry, base + (u32)(8 * o + r) * rows4, 0, 0));
+    for (int i = 0; i < 8; i++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (ILT_LDS void*)(S.xs + i * 1024), 16, xrow + (i & 1 ? xpc ^ 64 : xpc) + (u32)(8 * (i & 3)) * (u32)p.cols + 128 * (i >> 2), sb * 256, 0, 0);
+    const u32 ctok = (u32)(l32 * nsb);
+    c_yd = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, ctok * 4, sb * 4, 0));
+    if constexpr (F::MINS) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const ilt_v4i a = __builtin_amdgcn_raw_buffer_load_b128(rb, ctok * 64 + 16 * k, sb * 64, 0);
+        c_bs[k] = make_int4(a.x, a.y, a.z, a.w);
+      }
     }
+  };
+  const u8* const xb = S.xs + 128 * l32;
+  const int xsw = (l32 >> 1) & 7;
+  auto frag = [&](int g) { return __builtin_bit_cast(v4i, ilt_lds_ld16(xb + 4096 * (g >> 2) + 16 * ((2 * (g & 3) + lh) ^ xsw))); };
+  v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
+  v4i hi[8], lo[8];
+  typename F::Block blk;
+  issue_w(mine(0));
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  F::block(blk, S.ws, l32, lh);
+  {
+    typename F::Quants qs;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      float v = sum[o][r];
-      if (p.bias) v = v + bv;
-      if (p.acc) v = old[r] + v;
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, v), ry, base + (u32)(8 * o + r) * rows4, 0, 0);
-    }
+    for (int g = 0; g < 8; g++) { F::quants(qs, S.ws, g, l32, lh); F::quants_now(qs, S.ws, g, l32, lh); F::group(blk, qs, g, lh, hi[g], lo[g]); }
   }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the blocks' place is written again)
+  issue_x(mine(0));
+  issue_w(mine(1));
+  v16i X, Y, P;
+  v16f im = {};
+  float dprev = 0.0f, dmprev = 0.0f;
+#pragma unroll
+  for (int r = 0; r < 16; r++) P[r] = 0;
+  float* const ex = (float*)W.ex;
+  auto place = [&](int j, int s) { return ex + ((j * (KS - 1) + s) * TERMS) * 256 + 4 * lane; };      // (s: the source's number without the owner's)
+  v4f own[TERMS];
+  // four results' terms, of the round before
+  auto term = [&](int j, const float4& y) {
+    v4f a = {}, b;
+    const float yv[4] = {y.x, y.y, y.z, y.w};
+    float f[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) { b[i] = yv[i] * dprev; f[i] = (float)P[4 * j + i]; if constexpr (F::MINS) a[i] = yv[i] * dmprev; }
+#pragma unroll
+    for (int i = 0; i < 4; i++) { b[i] = b[i] * f[i]; if constexpr (F::MINS) a[i] = a[i] * im[4 * j + i]; }
+    if (j == ks) {
+      if constexpr (F::MINS) own[0] = a;
+      own[TERMS - 1] = b;
+    } else {
+      float* const o = place(j, ks - (ks > j ? 1 : 0));
+      if constexpr (F::MINS) *ILT_LDS_PTR(v4f, o) = a;
+      *ILT_LDS_PTR(v4f, o + (TERMS - 1) * 256) = b;
+    }
+  };
+  // the wave's quarter: the terms of round i's blocks in order, its own among the others'
+  auto add = [&](int i) {
+    v4f t[KS][TERMS];
+#pragma unroll
+    for (int s = 0; s < KS - 1; s++)
+#pragma unroll
+      for (int k = 0; k < TERMS; k++) t[s][k] = *ILT_LDS_PTR(const v4f, place(ks, s) + k * 256);
+#pragma unroll
+    for (int s = KS - 1; s >= 0; s--)                // (moved up from the wave's place on)
+#pragma unroll
+      for (int k = 0; k < TERMS; k++) t[s][k] = s == ks ? own[k] : s > ks ? t[s - (s > 0)][k] : t[s][k];
+#pragma unroll
+    for (int s = 0; s < KS; s++)
+      if (i * KS + s < nsb) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          if constexpr (F::MINS) sum[r] = sum[r] - t[s][0][r];
+          sum[r] = sum[r] + t[s][TERMS - 1][r];
+        }
+      }
+    asm volatile("" : "+v"(sum));                    // (the reads have come back before the wave meets the next barrier)
+  };
+#pragma unroll 1
+  for (int i = 0; i < rounds; i++) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const float* const xp = S.xd[(i & 1) ^ 1] + 4 * lh;
+    const v16i zi = {};
+    typename F::Block nb = {};
+    typename F::Quants qs;
+    v4i f0 = frag(0), f1 = frag(1);
+    float4 y = lds_f4(xp);
+    F::block(nb, S.ws, l32, lh); F::quants(qs, S.ws, 0, l32, lh);
+    if (lh == 0) S.xd[i & 1][l32] = c_yd;
+    v8h sums;
+    if constexpr (F::MINS) {                         // the sums of 32, eight times 128 * (sum >> 7) or eight times sum & 127
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const int v = k & 1 ? wordr(c_bs[k >> 1], 2) + wordr(c_bs[k >> 1], 3) : wordr(c_bs[k >> 1], 0) + wordr(c_bs[k >> 1], 1);
+        sums[k] = (_Float16)(float)(v & (lh ? 127 : ~127));
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < 8; g++) {
+      const v4i f = f0;
+      f0 = f1;
+      if (g < 6) f1 = frag(g + 2);
+      F::quants_now(qs, S.ws, g, l32, lh);
+      if (g < 7) F::quants(qs, S.ws, g + 1, l32, lh);
+      __builtin_amdgcn_sched_barrier(0);
+      X = __builtin_amdgcn_mfma_i32_32x32x32_i8(f, hi[g], g ? X : zi, 0, 0, 0);
+      Y = __builtin_amdgcn_mfma_i32_32x32x32_i8(f, lo[g], g ? Y : zi, 0, 0, 0);
+      if (g == 0) asm volatile("s_barrier" ::: "memory");      // (the round before's terms have been added)
+      if (g % 2 == 1) {
+        term(g >> 1, y);
+        if (g < 7) y = lds_f4(xp + 8 * (g >> 1) + 8);
+      }
+      F::group(nb, qs, g, lh, hi[g], lo[g]);
+      asm volatile("" : "+v"(hi[g]), "+v"(lo[g]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (F::MINS) {
+      const v16f zf = {};
+      im = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, blk.mins, zf, 0, 0, 0);
+    }
+    dprev = blk.d; dmprev = blk.dm; blk = nb;
+    asm volatile("" : "+v"(blk.d));
+    ilt_barrier_lds();                               // the terms are in, and this wave has read its tokens and blocks
+    issue_x(mine(i + 1));
+    issue_w(mine(i + 2));
+    if (i > 0) add(i - 1);
+#pragma unroll
+    for (int r = 0; r < 16; r++) P[r] = (X[r] << F::SH) + Y[r];
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the last round's loads, for nobody: nothing may land in LDS after the workgroup ends)
+  ilt_barrier_lds();
+  {
+    const float* const xp = S.xd[(rounds & 1) ^ 1] + 4 * lh;
+#pragma unroll
+    for (int j = 0; j < 4; j++) term(j, lds_f4(xp + 8 * j));
+  }
+  ilt_barrier_lds();
+  add(rounds - 1);
+  split_store(p, sum, tok0, ntok, r0 + l32, 8 * ks + 4 * lh);
 }
 
 // FSET: the matrices' format, or 0 where Q4_K and Q6_K meet in a launch
@@ -790,9 +962,10 @@ __global__ __launch_bounds__(64 * WR * WT, WR * WT == 1 ? 1 : 2) void gemm_i8r_k
   else reg_tile<ILT_Q6_K, NP, WR, WT>(p, w, rt * TM, tok0, ntok, smem);
 }
 
-template <int FSET, int KS>
-__global__ __launch_bounds__(256, 1) void gemm_i8s_kernel(BfParams p) {
-  constexpr int TM = 32 * (4 / KS);
+// TWO: reg_split2, two workgroups a CU
+template <int FSET, bool TWO>
+__global__ __launch_bounds__(256, TWO ? 2 : 1) void gemm_i8s_kernel(BfParams p) {
+  constexpr int TM = 32;
   extern __shared__ __align__(16) unsigned char smem[];
   long tok0; int ntok, rt; const u8* w = p.w;
   if (!pick_tile<TM, 32>(p, tok0, ntok, rt, w)) return;
@@ -806,9 +979,15 @@ __global__ __launch_bounds__(256, 1) void gemm_i8s_kernel(BfParams p) {
   p.bias = m == 0 ? p.mbias[0] : m == 1 ? p.mbias[1] : p.mbias[2];
   if (p.nmulti > 1) p.ldy = p.rows;
   const int fmt = m == 0 ? p.mfmt[0] : m == 1 ? p.mfmt[1] : p.mfmt[2];
-  if constexpr (FSET != 0) reg_split<FSET, KS>(p, w, rt * TM, tok0, ntok, smem);
-  else if (fmt == ILT_Q4_K) reg_split<ILT_Q4_K, KS>(p, w, rt * TM, tok0, ntok, smem);
-  else reg_split<ILT_Q6_K, KS>(p, w, rt * TM, tok0, ntok, smem);
+  if constexpr (TWO) {
+    if constexpr (FSET != 0) reg_split2<FSET>(p, w, rt * TM, tok0, ntok, smem);
+    else if (fmt == ILT_Q4_K) reg_split2<ILT_Q4_K>(p, w, rt * TM, tok0, ntok, smem);
+    else reg_split2<ILT_Q6_K>(p, w, rt * TM, tok0, ntok, smem);
+  } else {
+    if constexpr (FSET != 0) reg_split<FSET>(p, w, rt * TM, tok0, ntok, smem);
+    else if (fmt == ILT_Q4_K) reg_split<ILT_Q4_K>(p, w, rt * TM, tok0, ntok, smem);
+    else reg_split<ILT_Q6_K>(p, w, rt * TM, tok0, ntok, smem);
+  }
 }
 
 template <int FMT, int NP, int WR, int WT> constexpr size_t reg_smem() {
@@ -838,26 +1017,25 @@ hipError_t launch_i8r(BfParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <int FSET, int KS>
+template <int FSET, bool TWO>
 hipError_t launch_i8s(BfParams& p, hipStream_t st) {
-  constexpr int TM = 32 * (4 / KS);
-  constexpr size_t s4 = sizeof(SplitSmem<ILT_Q4_K, KS>), s6 = sizeof(SplitSmem<ILT_Q6_K, KS>);
+  constexpr size_t s4 = TWO ? sizeof(SplitSmem2<ILT_Q4_K>) : sizeof(SplitSmem<ILT_Q4_K>), s6 = TWO ? sizeof(SplitSmem2<ILT_Q6_K>) : sizeof(SplitSmem<ILT_Q6_K>);
   constexpr size_t smem = FSET == ILT_Q4_K ? s4 : FSET == ILT_Q6_K ? s6 : s4 > s6 ? s4 : s6;
-  static_assert(smem <= 160 * 1024, "a workgroup's LDS");
+  static_assert((TWO ? 2 : 1) * smem <= 160 * 1024, "one workgroup's LDS, or two's");
   static bool attr_set[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
   if (!attr_set[dev]) {
-    const hipError_t e = hipFuncSetAttribute((const void*)gemm_i8s_kernel<FSET, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    const hipError_t e = hipFuncSetAttribute((const void*)gemm_i8s_kernel<FSET, TWO>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) return e;
     attr_set[dev] = true;
   }
   long long tiles = 0;
-  for (int m = 0; m < p.nmulti; m++) tiles += (p.mrows[m] + TM - 1) / TM;
-  p.rows = (int)(tiles * TM);
+  for (int m = 0; m < p.nmulti; m++) tiles += (p.mrows[m] + 31) / 32;
+  p.rows = (int)(tiles * 32);
   const long long total = (long long)((p.ntok + 31) / 32) * tiles, per = (total + 7) / 8;
   if (per * 8 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((gemm_i8s_kernel<FSET, KS>), dim3((unsigned)(per * 8)), dim3(256), smem, st, p);
+  hipLaunchKernelGGL((gemm_i8s_kernel<FSET, TWO>), dim3((unsigned)(per * 8)), dim3(256), smem, st, p);
   return hipGetLastError();
 }
 
@@ -917,12 +1095,12 @@ constexpr RegTile kRegTiles[] = {
   {64, 128, 2, {{1.7f, 2.8f}, {1.75f, 2.9f}}},
   {128, 128, 2, {{2.6f, 4.4f}, {2.55f, 4.4f}}},
 };
-// The same for tiles whose super-blocks are shared out (reg_split): a workgroup of four waves takes what a CU's LDS holds, and 1.95
-// us for a round of KS blocks whatever the format (a wave alone on its SIMD, 571 instructions for Q6_K); besides, microseconds, a
-// tile's start and end, and the launch's, which tiles of the other kinds have once.
-constexpr float kRegStart = 4.0f, kSplitStart = 2.8f, kSplitTile = 2.2f, kSplitRound = 1.95f;
+// The same for tiles whose super-blocks are shared out, where a round is KS of them, whatever the format: a workgroup a CU (reg_split)
+// 1.95 us a round, one of two (reg_split2) 2.25, two 3.15; besides, microseconds, a tile's start and end, and the launch's, which tiles
+// of the other kinds have once.  Workgroups past those that fit start as the first ones end: 0.7 of what they take alone.
+constexpr float kRegStart = 4.0f, kSplitStart = 2.8f, kSplitTile = 2.2f, kSplitRound = 1.95f, kSplitRound2[2] = {2.25f, 3.15f};
 // Which of them, by the rounds that the chip takes the launch's workgroups in.  (Shapes, us for the tiles taken and for 64 or 128
-// rows x 128 tokens: Q6_K 2560 x 9728 on 256 tokens 57-64 and 89, on 512 81 and 90; Q4_K 2560 x 4096 on 256 25 and 33; 19456 x 2560 on 32
+// rows x 128 tokens: Q6_K 2560 x 9728 on 256 tokens 54 and 89, on 512 81 and 90; Q4_K 2560 x 4096 on 256 25 and 33; 19456 x 2560 on 32
 // 17.6 and 31, on 192 35 and 48; 9728 x 2560 on 64 17.2 and 22.)
 template <int FSET>
 int reg_tile_of(const BfParams& p) {
@@ -941,11 +1119,11 @@ int reg_tile_of(const BfParams& p) {
     const float us = kRegStart + (float)nsb * ((float)(n / round) * c.us[f][fit - 1] + (rest ? c.us[f][(rest + 255) / 256 - 1] : 0.0f));
     if (v == 0 || us < least) { best = v; least = us; }
   }
-  for (int v = 5; v < 7; v++) {                      // KS 2 and 4, a workgroup a CU
-    const int ks = v == 5 ? 2 : 4;
-    const float us = kSplitStart + (float)((workgroups(128 / ks, 32) + 255) / 256) * (kSplitTile + kSplitRound * (float)((nsb + ks - 1) / ks));
-    if (us < least) { best = v; least = us; }
-  }
+  const long long n = workgroups(32, 32), rest = n % 512;
+  const float rounds = (float)((nsb + KS - 1) / KS);
+  if (n <= 256 && kSplitStart + kSplitTile + kSplitRound * rounds < least) return 5;
+  const float part = rest ? kSplitTile + kSplitRound2[(rest - 1) / 256] * rounds : 0.0f;
+  if (kSplitStart + (float)(n / 512) * (kSplitTile + kSplitRound2[1] * rounds) + (n > 512 ? 0.7f : 1.0f) * part < least) return 6;
   return best;
 }
 
@@ -961,8 +1139,8 @@ hipError_t dispatch_i8r(BfParams& p, int forced, hipStream_t st) {
       case 1: return launch_i8r<FSET, 2, 1, 1>(p, st);
       case 2: return launch_i8r<FSET, 2, 2, 1>(p, st);
       case 3: return launch_i8r<FSET, 2, 2, 2>(p, st);
-      case 5: return launch_i8s<FSET, 2>(p, st);
-      case 6: return launch_i8s<FSET, 4>(p, st);
+      case 5: return launch_i8s<FSET, false>(p, st);
+      case 6: return launch_i8s<FSET, true>(p, st);
       default: return launch_i8r<FSET, 4, 4, 1>(p, st);
     }
   }
@@ -976,7 +1154,7 @@ constexpr int block_bytes_of(int fmt) {
 
 // Up to three matrices (Q4_K, Q6_K in any mix, or all Q2_K, or all IQ2_XXS) on the same tokens in one launch, their row tiles one after another.
 // hipErrorNotSupported, and nothing launched, where the shapes are not this kernel's.  ILT_I8_TM (tests): 64 or 128 rows by 128 tokens
-// whatever the shape, 1 to 5 the tiles in kRegTiles' order.
+// whatever the shape, 1 to 5 the tiles in kRegTiles' order, 6 and 7 the two kernels for few tiles.
 hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws, const int* rows, float* const* ys, const float* const* biases,
                              int cols, const int8_t* xq, const float* xd, const int* bsums, int ntok, int acc, hipStream_t st, long long ldy) {
   if (nmat < 1 || nmat > 3 || ntok < 1 || cols < 256 || cols % 256 != 0 || cols >= (1 << 22)) return hipErrorNotSupported;
