@@ -30,14 +30,30 @@ __device__ __forceinline__ float part(const float4& v, int e) { return e == 0 ? 
 // 8 + e and 12 + e of 256 scores, and a lane's four 16-byte pieces of a row (or a key) are its operands for e = 0 .. 3.
 // Positions are the results' rows: a lane stores four scores of one row.
 // QL: the rows' operands in LDS, a read an instruction, and four waves a SIMD instead of three.
+// The grid's columns are pairs of row tiles' sets, one from the start and one from the end: a set for a column left as many workgroups without
+// a position as with one, and a wave needed sixteen tiles where the pairs are quickest with eight (us: 2,048 tokens at none, 32 heads
+// of 128 over 8, 407 -> 369, 1,000 115 -> 104, 1,250 at 1,250 419 -> 403; 14 of 64 over 2, 2,048 at none 118 -> 88).
+// The waves, npt position tiles each, that the positions of row tiles 4 set .. 4 set + 3 take
+__host__ __device__ __forceinline__ int score_waves(int set, int pos0, int rows, int group, int npt) {
+  const int last = 64 * set + 63 < rows ? 64 * set + 63 : rows - 1;
+  return (pos0 + last / group + 16 * npt) / (16 * npt);
+}
 template <int NJ, bool QL>      // hd / 16
 __global__ __launch_bounds__(256, QL ? 4 : 3) void attn_scores_mm_kernel(const float* __restrict__ q, const float* __restrict__ kc, float* __restrict__ raw,
                                                                 int nh, int group, int kvd, int pos0, int ntok, float scale, int spitch, int npt) {
   constexpr int HD = 16 * NJ;
   const int kvh = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 15, m = lane >> 4, rows = ntok * group;
-  // (the four waves: row tiles on the same positions, whose keys then come from the CU's own cache)
-  const int r0 = (blockIdx.z * 4 + wave) * 16, p0 = blockIdx.y * npt * 16;
+  // (the four waves: row tiles on the same positions, whose keys then come from the CU's own cache; a column of the grid's is the
+  // positions of a set of row tiles and then those of the set as far from the last, so that every one has as many)
+  const int sets = (rows + 63) / 64;
+  int set = blockIdx.z, pw = blockIdx.y;
+  if (const int nw = score_waves(set, pos0, rows, group, npt); pw >= nw) {
+    pw -= nw;
+    if (set == sets - 1 - set) return;
+    set = sets - 1 - set;
+  }
+  const int r0 = (set * 4 + wave) * 16, p0 = pw * npt * 16;
   if (r0 >= rows) return;
   const int nposmax = pos0 + (min(r0 + 15, rows - 1)) / group + 1, pend = min(p0 + 16 * npt, nposmax);
   if (p0 >= pend) return;
@@ -278,17 +294,20 @@ bool ilt_k_attn_mm_takes(const float* q, const float* kc, const float* scratch, 
          (long long)ctx * nkv * hd < (1LL << 30) && 17LL * nh * (ctx + 3) < (1LL << 30);                         // 32-bit offsets: the values, a tile's rows
 }
 
-// A wave's position tiles, its rows' loads and the launch's waves shared among them: one where the launch has no more than twice what
-// the chip holds (21 tokens at 300: 23 us against 27 for the chunk's attention), four from there on (512 tokens at none before 95 against
-// 99), sixteen from 100,000 tiles on (scores of 1,250 tokens at 1,250, 32 heads of 128 over 8: four 439 us, eight 431, sixteen 414; 14
-// of 64 over 2 109, 105, 104; 512 at none, 33,000 tiles, 39, 47, 49).  The rows' operands in LDS past 16,384 tiles (454 -> 439; 512 at
-// none 40.5 -> 39.1; 256 at none, 8,192, 15.3 against 16.0).
+// A wave's position tiles, its rows' loads and the launch's waves shared among them, by all the launch's tiles (us of the scores for one,
+// two, four and eight of them): 2,944 tiles 10.0, 10.5, 11.3, 17.5; 6,912 17.3, 14.5, 16.3, 18.2; 14,336 15.4, 14.8, 15.8, 18.7; 32,768 39.8, 35.5, 36.1,
+// 38.8; 45,600 52.6, 45.6, 44.2, 49.0; 75,000 four 107, eight 104, sixteen 119; 205,000 155, 150, 158;
+// 393,000 421, 403, 404 (and 2,500 tokens as two halves 68.6, 68.7 and 68.3 ms).  The rows' operands in LDS past 16,384
+// tiles (512 tokens at none 40.5 -> 39.1; 256 at none, 8,192, 15.3 against 16.0).
 hipError_t ilt_k_attn_scores_mm(const float* q, const float* kc, float* raw, int nh, int nkv, int hd, int pos0, int ntok, float scale, int spitch,
                                 hipStream_t st) {
   const int group = nh / nkv, rtiles = (ntok * group + 15) / 16, ptiles = (pos0 + ntok + 15) / 16;
   const long long tiles = (long long)rtiles * nkv * ptiles;
-  const int npt = tiles < 8192 ? 1 : tiles < 100000 ? 4 : 16;
-  const dim3 grid(nkv, (ptiles + npt - 1) / npt, (rtiles + 3) / 4);
+  const int npt = tiles < 6000 ? 1 : tiles <= 16384 ? 2 : tiles < 70000 ? 4 : tiles < 300000 ? 8 : 16;
+  const int rows = ntok * group, sets = (rows + 63) / 64;
+  // (a column's positions: no pair of sets has more than this)
+  const int waves = sets == 1 ? score_waves(0, pos0, rows, group, npt) : (2 * pos0 + (64 * sets + 62) / group + 32 * npt) / (16 * npt);
+  const dim3 grid(nkv, waves, (sets + 1) / 2);
 #define ILT_SCORES(NJ, QL) hipLaunchKernelGGL((attn_scores_mm_kernel<NJ, QL>), grid, dim3(256), 0, st, q, kc, raw, nh, group, nkv * hd, pos0, ntok, scale, spitch, npt)
   if (tiles > 16384) { if (hd == 128) ILT_SCORES(8, true); else ILT_SCORES(4, true); }
   else { if (hd == 128) ILT_SCORES(8, false); else ILT_SCORES(4, false); }
@@ -299,7 +318,12 @@ hipError_t ilt_k_attn_scores_mm(const float* q, const float* kc, float* raw, int
 // Sixteen rows a wave once that leaves about six waves a CU (32 heads of 128 over 8 on 512 tokens, 2,048 waves: 95.7 us for the
 // chunk's attention against 97.6 with four; 1,250 at 1,250 893 against 1,102), else four: a wave's chain of positions, an
 // instruction every few cycles, is the launch's time (256 tokens 41 us against 43, 64 tokens 13.9 against 15.5, 14 heads of 64
-// over 2 on 1,250 121 against 137).  One row a wave up to 1,400 waves, a little more than the SIMDs (32 heads of 128 over 8 at 300
+// over 2 on 1,250 121 against 137).  Further into a conversation than the chunk is long, where it also has the GPU to itself, sixteen as soon
+// as their chain, 53 ns a position, is over before the four times as many waves of four rows, 19 ns a position each, are through: by how
+// many waves they are and how much of the longest chain their average is (values, us, four and sixteen; 32 heads of 128 over 8: 128
+// tokens at 1,900, 502 by this count, 76 and 107; 200 at 1,200, 743, 90 and 78; 300 at 1,700, 1,110, 161 and 139; 380 at 600 87 and 69; 14 of
+// 64 over 2, 700 at 3,000, 556, 173 and 192).  Beside a chunk's other half four rows are better (256 at 256, 768 by this count: the prompt of
+// 512 11.6 ms against 12.1).  One row a wave up to 1,400 waves, a little more than the SIMDs (32 heads of 128 over 8 at 300
 // positions, 1,344 waves 17.6 us against 18.6, 2,112 21.1 against 19.3; 14 of 64 over 2, 1,400 19.8 against 20.9, 2,800 30.5 against
 // 29.1); its values three sets ahead up to 512 positions, four past them (3 tokens at 2,000: 35.5 against 39.7).
 hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, int spitch, hipStream_t st) {
@@ -312,7 +336,8 @@ hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, 
 #undef ILT_VALUES
     return hipGetLastError();
   }
-  const int r = (long long)((rows + 15) / 16) * nkv * cg >= 1600 ? 16 : 4;
+  const long long w16 = (long long)((rows + 15) / 16) * nkv * cg;
+  const int r = w16 >= 1600 || (pos0 > ntok && w16 * (2LL * pos0 + ntok) >= 1440LL * (pos0 + ntok)) ? 16 : 4;
   const dim3 grid(nkv, ((rows + r - 1) / r + wr - 1) / wr);
 #define ILT_VALUES(R, HD) hipLaunchKernelGGL((attn_values_mm_kernel<R, HD>), grid, dim3(256), 0, st, prob, vc, out, nh, group, nkv * hd, pos0, ntok, spitch)
   if (r == 16) { if (hd == 128) ILT_VALUES(16, 128); else ILT_VALUES(16, 64); }

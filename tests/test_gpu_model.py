@@ -481,6 +481,13 @@ def test_chunk_attention_of_one_and_of_four_rows_a_wave(dev, nh, nkv, hd, pos0, 
     test_chunk_attention_with_the_matrix_cores_products(dev, nh, nkv, hd, pos0, ntok, what)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,pos0,ntok,what", [(4, 4, 128, 0, 65, "nan"), (5, 5, 64, 33, 129, ""), (9, 3, 64, 14, 43, "denormal"),      # a tile of positions a wave; two, three and three sets
+                                                      (4, 4, 128, 37, 705, "nan"), (16, 16, 64, 3, 831, "odd"), (32, 32, 64, 62, 960, "nan")])      # two, four and eight tiles
+def test_chunk_attention_whose_scores_pair_row_tiles(dev, nh, nkv, hd, pos0, ntok, what):
+    """The same for the scores' sets of row tiles, one from the start and one from the end a column of the grid: even and odd numbers of sets."""
+    test_chunk_attention_with_the_matrix_cores_products(dev, nh, nkv, hd, pos0, ntok, what)
+
+
 @pytest.mark.parametrize("nh,pos0,ntok", [(2, 60, 3), (2, 1020, 4), (8, 1100, 130), (8, 2100, 130), (2, 2100, 5), (1, 8000, 192)])
 def test_chunk_softmax_where_the_order_of_the_sum_shows(dev, nh, pos0, ntok):
     """A chunk whose exponentials' sum lies on the edge between two singles for its reciprocal, so that the softmax kernels (a wave
