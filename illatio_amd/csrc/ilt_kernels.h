@@ -251,13 +251,19 @@ hipError_t ilt_k_argmax(const float* v, int n, int* out, void* scratch, hipStrea
 hipError_t ilt_k_attn_step(const float* q, const float* k, const float* v, const float* qn, const float* kn, const float* rope, float* kc,
                            float* vc, float* out, int nh, int nkv, int hd, int rd, int pos, float eps, int neox, float* scratch, hipStream_t st);
 hipError_t ilt_k_attn_giveups(unsigned long long* out);
+// Where a chunk's attention leaves its rows quantized instead (Q8_0, scales through halves; Q8_K), if what it takes for the shapes
+// can: done says so, and out is then not written.
+enum { ILT_ROWS_Q8 = 1, ILT_ROWS_Q8K = 2 };
+struct IltRowsQuant { int8_t* q; float* d; int* sums; int kind; bool done; };
 hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok,
-                           float* scratch, hipStream_t st);
+                           float* scratch, hipStream_t st, IltRowsQuant* to = nullptr);
 // A chunk's scores and values with the matrix cores' products (kernels_attn_mm.hip)
 bool ilt_k_attn_mm_takes(const float* q, const float* kc, const float* scratch, const float* out, int nh, int nkv, int hd, int ctx);
 hipError_t ilt_k_attn_scores_mm(const float* q, const float* kc, float* raw, int nh, int nkv, int hd, int pos0, int ntok, float scale, int spitch,
                                 hipStream_t st);
-hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, int spitch, hipStream_t st);
+bool ilt_k_attn_mm_quantizes(int kind, int nh, int nkv, int hd);
+hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, int spitch, const IltRowsQuant* to,
+                                hipStream_t st);
 hipError_t ilt_k_swiglu_rows(float* a, const float* b, long long n, hipStream_t st);
 
 #endif  // ILT_KERNELS_H

@@ -1240,7 +1240,7 @@ hipError_t ilt_k_qk_rope(float* q, float* k, const float* v, const float* qn, co
 // scratch: ntok * nh * ((pos0 + ntok + 3) & ~3) floats for the variants of two or three launches (contexts up to 8192
 // positions), or null: one launch
 hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok,
-                           float* scratch, hipStream_t st) {
+                           float* scratch, hipStream_t st, IltRowsQuant* to) {
   if (ntok <= 0) return hipSuccess;
   if (hd % 16 || hd > 256 || nh % nkv || pos0 < 0) return hipErrorInvalidValue;
   const int smax = (pos0 + ntok + 3) & ~3;
@@ -1269,7 +1269,12 @@ hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, flo
       } else launch_scores<16>(dim3(nh, (ctx + 255) / 256, (ntok + 15) / 16), st, q, kc, scratch, nh, nkv, hd, pos0, ntok, scale, smax);
       const hipError_t es = launch_softmax(scratch, nh, pos0, ntok, smax, st);
       if (es != hipSuccess) return es;
-      if (mm) return ilt_k_attn_values_mm(scratch, vc, out, nh, nkv, hd, pos0, ntok, smax, st);
+      if (mm) {
+        if (to && !ilt_k_attn_mm_quantizes(to->kind, nh, nkv, hd)) to = nullptr;
+        const hipError_t e = ilt_k_attn_values_mm(scratch, vc, out, nh, nkv, hd, pos0, ntok, smax, to, st);
+        if (to) to->done = e == hipSuccess;
+        return e;
+      }
       hipLaunchKernelGGL(attn_values_chunk_kernel, dim3(nh * (hd / 32), (ntok + 31) / 32), dim3(1024), smem, st, scratch, vc, out, nh, nkv, hd, pos0,
                          ntok, smax);
       return hipGetLastError();

@@ -13,6 +13,7 @@
 //
 // The query heads of a KV head see the same keys and values, so a KV head's rows -- token t, head g of its group: row
 // t * group + g -- go through in tiles of 16 (or 4), whatever heads they are of.
+#include "ilt_act_blocks.h"
 #include "ilt_device.h"
 #include "ilt_kernels.h"
 #include "ilt_value_sets.h"
@@ -112,6 +113,33 @@ __global__ __launch_bounds__(256, QL ? 4 : 3) void attn_scores_mm_kernel(const f
   }
 }
 
+// A workgroup's ROWS x HD results, rows from rb on, in LDS (HD + 4 floats a row) to the blocks of the output product's activations: a
+// launch and the results' way to memory and back less, 2.5 us a layer of 97 at 21 tokens of the Qwen3-4B shape, 4 of 440 at 700.
+struct RowsQuant { i8* q; float* d; int* sums; int kind; };      // kind: ILT_ROWS_Q8 or ILT_ROWS_Q8K
+template <int HD, int ROWS>
+__device__ __forceinline__ void rows_to_blocks(const float* tile, const RowsQuant& o, int rb, int rows, int nh, int group, int kvh, int wave, int lane) {
+  __syncthreads();
+  for (int c = wave; c < ROWS * HD / 256; c += 4) {
+    const int at = 256 * c + 4 * lane, r = at / HD, row = rb + r, t = row / group;
+    const float4 f = *(const float4*)(tile + r * (HD + 4) + at % HD);
+    const float v[4] = {f.x, f.y, f.z, f.w};
+    const long long p = ((long long)t * nh + kvh * group + row - t * group) * HD + at % HD;
+    const bool live = row < rows;
+    int q[4];
+    if (o.kind == ILT_ROWS_Q8K) {
+      const float d = q8k_block(v, lane, q);
+      if (live) q8k_store(q, d, lane, o.q, o.d, o.sums, p >> 8);      // (a block's rows are all there or none is)
+    } else {
+      const float d = q8_block(v, q);
+      if (live) {
+        const u32 packed = act_pack(q);
+        __builtin_memcpy(o.q + p, &packed, 4);
+        if ((lane & 7) == 0) o.d[p >> 5] = __half2float(__float2half_rn(d));
+      }
+    }
+  }
+}
+
 // out = the values' rows times the scaled scores (attn_softmax_kernel's), position after position.  A wave takes R rows
 // (16, or 4: v_mfma_f32_4x4x1_16b_f32) and 64 columns; an instruction is one position, its operands the position's values in
 // the wave's columns and its scores in the wave's rows.
@@ -130,9 +158,9 @@ template <> struct ValMM<4> {
   template <int K> static __device__ __forceinline__ V mul(const float (&s)[NS], float v) { const V z = {}; return __builtin_amdgcn_mfma_f32_4x4x1f32(s[0], v, z, 4, K, 0); }
 };
 
-template <int R, int HD>
+template <int R, int HD, bool QUANT>
 __global__ __launch_bounds__(256, R == 16 ? 4 : 2) void attn_values_mm_kernel(const float* __restrict__ prob, const float* __restrict__ vc, float* __restrict__ out,
-                                                                int nh, int group, int kvd, int pos0, int ntok, int spitch) {
+                                                                int nh, int group, int kvd, int pos0, int ntok, int spitch, RowsQuant quant) {
   using M = ValMM<R>;
   using V = typename M::V;
   constexpr int CG = HD / 64, WR = 4 / CG;           // column groups and row tiles of a workgroup's four waves
@@ -140,8 +168,12 @@ __global__ __launch_bounds__(256, R == 16 ? 4 : 2) void attn_values_mm_kernel(co
   const int kvh = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rows = ntok * group, cg = wave % CG;
   // (the last rows, which see the most positions, first: the launch ends with the short ones)
-  const int r0 = ((gridDim.y - 1 - blockIdx.y) * WR + wave / CG) * R;
-  if (r0 >= rows) return;
+  const int rb = (int)(gridDim.y - 1 - blockIdx.y) * WR * R;
+  int r0 = rb + wave / CG * R;
+  if (r0 >= rows) {
+    if constexpr (!QUANT) return;
+    r0 = rows - 1;                                   // (the last row again, for nobody)
+  }
   const int t0 = r0 / group, t1 = min(r0 + R - 1, rows - 1) / group;
   const int npos0 = pos0 + t0 + 1, nposmax = pos0 + t1 + 1;
   // (through buffer loads: a set's values are one vector offset and scalar ones that never change, all of them within the cache
@@ -204,6 +236,19 @@ __global__ __launch_bounds__(256, R == 16 ? 4 : 2) void attn_values_mm_kernel(co
   Set x[AHEAD];
   ilt_value_sets<P, AHEAD>(x, npos0, nposmax, load, [&](const Set& x, int p) { set(x, p, std::false_type{}); },
                            [&](const Set& x, int p) { set(x, p, std::true_type{}); });
+  if constexpr (QUANT) {
+    __shared__ __align__(16) float tile[WR * R * (HD + 4)];
+    float* const mine = tile + wave / CG * R * (HD + 4) + 64 * cg;
+    if constexpr (R == 4) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) mine[r * (HD + 4) + lane] = acc[r];
+    } else {
+#pragma unroll
+      for (int b = 0; b < 4; b++) *(v4f*)(mine + (lane & 15) * (HD + 4) + 16 * b + 4 * (lane >> 4)) = v4f{acc[4 * b], acc[4 * b + 1], acc[4 * b + 2], acc[4 * b + 3]};
+    }
+    rows_to_blocks<HD, WR * R>(tile, quant, rb, rows, nh, group, kvh, wave, lane);
+    return;
+  }
   auto row_out = [&](int row) { return out + ((long long)(row / group) * nh + kvh * group + row % group) * HD + 64 * cg; };
   if constexpr (R == 4) {
 #pragma unroll
@@ -240,13 +285,17 @@ __device__ __forceinline__ void across(float* v) {
 template <int K> __device__ __forceinline__ float times_score(float s, float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x150 + K, 0xF, 0xF, true)) * v;      // row_newbcast:K
 }
-template <int HD, int AHEAD>
+template <int HD, int AHEAD, bool QUANT>
 __global__ __launch_bounds__(256) void attn_values_mm_row_kernel(const float* __restrict__ prob, const float* __restrict__ vc, float* __restrict__ out,
-                                                              int nh, int group, int kvd, int pos0, int ntok, int spitch) {
+                                                              int nh, int group, int kvd, int pos0, int ntok, int spitch, RowsQuant quant) {
   constexpr int CG = HD / 64, P = 16;
   const int kvh = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int id = ((int)gridDim.y - 1 - (int)blockIdx.y) * 4 + wave, row = id / CG, cg = id % CG;
-  if (row >= ntok * group) return;
+  const int rb = ((int)gridDim.y - 1 - (int)blockIdx.y) * (4 / CG), cg = wave % CG;
+  int row = rb + wave / CG;
+  if (row >= ntok * group) {
+    if constexpr (!QUANT) return;
+    row = ntok * group - 1;                          // (again, for nobody)
+  }
   const int t = row / group, h = kvh * group + row - t * group, npos = pos0 + t + 1;
   const __amdgpu_buffer_rsrc_t rs = ilt_rsrc(ilt_uniform_ptr(prob + ((long long)t * nh + h) * spitch), (u32)npos * 4u);
   const __amdgpu_buffer_rsrc_t rv = ilt_rsrc(ilt_uniform_ptr(vc), (u32)npos * (u32)kvd * 4u);
@@ -284,6 +333,12 @@ __global__ __launch_bounds__(256) void attn_values_mm_row_kernel(const float* __
   };
   Set x[AHEAD];
   ilt_value_sets<P, AHEAD>(x, npos, npos, load, [&](Set& x, int p) { set(x, p, std::false_type{}); }, [&](Set& x, int p) { set(x, p, std::true_type{}); });
+  if constexpr (QUANT) {
+    __shared__ __align__(16) float tile[4 / CG * (HD + 4)];
+    tile[wave / CG * (HD + 4) + col + (lane >> 4)] = acc;
+    rows_to_blocks<HD, 4 / CG>(tile, quant, rb, ntok * group, nh, group, kvh, wave, lane);
+    return;
+  }
   out[((long long)t * nh + h) * HD + col + (lane >> 4)] = acc;      // (the exchange leaves column 4 c + g of sixteen c in lane 16 g + c)
 }
 
@@ -293,6 +348,9 @@ bool ilt_k_attn_mm_takes(const float* q, const float* kc, const float* scratch, 
   return (hd == 64 || hd == 128) && ((((uintptr_t)q) | ((uintptr_t)kc) | ((uintptr_t)scratch) | ((uintptr_t)out)) & 15) == 0 &&      // 16-byte loads and stores of them
          (long long)ctx * nkv * hd < (1LL << 30) && 17LL * nh * (ctx + 3) < (1LL << 30);                         // 32-bit offsets: the values, a tile's rows
 }
+
+// Blocks of 32 lie within a row; blocks of 256 are rows of one token and start where a tile's rows do where a group's columns are whole blocks.
+bool ilt_k_attn_mm_quantizes(int kind, int nh, int nkv, int hd) { return kind == ILT_ROWS_Q8 || (kind == ILT_ROWS_Q8K && nh / nkv * hd % 256 == 0); }
 
 // A wave's position tiles, its rows' loads and the launch's waves shared among them, by all the launch's tiles (us of the scores for one,
 // two, four and eight of them): 2,944 tiles 10.0, 10.5, 11.3, 17.5; 6,912 17.3, 14.5, 16.3, 18.2; 14,336 15.4, 14.8, 15.8, 18.7; 32,768 39.8, 35.5, 36.1,
@@ -326,22 +384,28 @@ hipError_t ilt_k_attn_scores_mm(const float* q, const float* kc, float* raw, int
 // 512 11.6 ms against 12.1).  One row a wave up to 1,400 waves, a little more than the SIMDs (32 heads of 128 over 8 at 300
 // positions, 1,344 waves 17.6 us against 18.6, 2,112 21.1 against 19.3; 14 of 64 over 2, 1,400 19.8 against 20.9, 2,800 30.5 against
 // 29.1); its values three sets ahead up to 512 positions, four past them (3 tokens at 2,000: 35.5 against 39.7).
-hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, int spitch, hipStream_t st) {
+hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, int spitch, const IltRowsQuant* to,
+                                hipStream_t st) {
   const int group = nh / nkv, rows = ntok * group, cg = hd / 64, wr = 4 / cg;
+  const RowsQuant quant = to ? RowsQuant{to->q, to->d, to->sums, to->kind} : RowsQuant{};
   if ((long long)rows * nkv * cg <= 1400) {
     const dim3 grid(nkv, (rows * cg + 3) / 4);
-#define ILT_VALUES(HD, AHEAD) hipLaunchKernelGGL((attn_values_mm_row_kernel<HD, AHEAD>), grid, dim3(256), 0, st, prob, vc, out, nh, group, nkv * hd, pos0, ntok, spitch)
-    if (pos0 + ntok <= 512) { if (hd == 128) ILT_VALUES(128, 3); else ILT_VALUES(64, 3); }
-    else { if (hd == 128) ILT_VALUES(128, 4); else ILT_VALUES(64, 4); }
+#define ILT_VALUES(HD, AHEAD, QUANT) hipLaunchKernelGGL((attn_values_mm_row_kernel<HD, AHEAD, QUANT>), grid, dim3(256), 0, st, prob, vc, out, nh, group, nkv * hd, pos0, ntok, spitch, quant)
+#define ILT_VALUES_OF(AHEAD, QUANT) do { if (hd == 128) ILT_VALUES(128, AHEAD, QUANT); else ILT_VALUES(64, AHEAD, QUANT); } while (0)
+    if (pos0 + ntok <= 512) { if (to) ILT_VALUES_OF(3, true); else ILT_VALUES_OF(3, false); }
+    else { if (to) ILT_VALUES_OF(4, true); else ILT_VALUES_OF(4, false); }
+#undef ILT_VALUES_OF
 #undef ILT_VALUES
     return hipGetLastError();
   }
   const long long w16 = (long long)((rows + 15) / 16) * nkv * cg;
   const int r = w16 >= 1600 || (pos0 > ntok && w16 * (2LL * pos0 + ntok) >= 1440LL * (pos0 + ntok)) ? 16 : 4;
   const dim3 grid(nkv, ((rows + r - 1) / r + wr - 1) / wr);
-#define ILT_VALUES(R, HD) hipLaunchKernelGGL((attn_values_mm_kernel<R, HD>), grid, dim3(256), 0, st, prob, vc, out, nh, group, nkv * hd, pos0, ntok, spitch)
-  if (r == 16) { if (hd == 128) ILT_VALUES(16, 128); else ILT_VALUES(16, 64); }
-  else { if (hd == 128) ILT_VALUES(4, 128); else ILT_VALUES(4, 64); }
+#define ILT_VALUES(R, HD, QUANT) hipLaunchKernelGGL((attn_values_mm_kernel<R, HD, QUANT>), grid, dim3(256), 0, st, prob, vc, out, nh, group, nkv * hd, pos0, ntok, spitch, quant)
+#define ILT_VALUES_OF(R, QUANT) do { if (hd == 128) ILT_VALUES(R, 128, QUANT); else ILT_VALUES(R, 64, QUANT); } while (0)
+  if (r == 16) { if (to) ILT_VALUES_OF(16, true); else ILT_VALUES_OF(16, false); }
+  else { if (to) ILT_VALUES_OF(4, true); else ILT_VALUES_OF(4, false); }
+#undef ILT_VALUES_OF
 #undef ILT_VALUES
   return hipGetLastError();
 }

@@ -1,6 +1,7 @@
 // Activation quantizers, the Q8_0 upload repack, and row dequantizers for gfx950.
 // Every result is bit-for-bit what the reference's CPU path stores
 // (tensor.lisp:245-262, kquant.lisp:130-167, 466-497, iquant.lisp:161-230).
+#include "ilt_act_blocks.h"
 #include "ilt_device.h"
 #include "ilt_iq2xxs_tables.h"
 #include "ilt_kernels.h"
@@ -44,21 +45,14 @@ __global__ __launch_bounds__(256) void quant_q8_kernel(const float* __restrict__
 #pragma unroll
     for (int k = 0; k < 4; k++) v[k] = glu_of<GLU>(g[k], u[k], clamp, wrow, row);
   }
-  float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-  amax = fmaxf(amax, ilt_dppf<ILT_DPP_XOR1>(amax));
-  amax = fmaxf(amax, ilt_dppf<ILT_DPP_XOR2>(amax));
-  amax = fmaxf(amax, ilt_dppf<ILT_DPP_HALF_MIRROR>(amax));
-  const float d = amax / 127.0f;
-  const float id = d == 0.0f ? 0.0f : 1.0f / d;
   int q[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) q[k] = (int)rintf(v[k] * id);
+  const float d = q8_block(v, q);
   if (xsum) {
     const int sum = ilt_sum8((q[0] + q[1]) + (q[2] + q[3]));
     if (live && (threadIdx.x & 7) == 0) xsum[b] = sum;
   }
   if (!live) return;
-  const u32 packed = (u32)(q[0] & 0xFF) | ((u32)(q[1] & 0xFF) << 8) | ((u32)(q[2] & 0xFF) << 16) | ((u32)(q[3] & 0xFF) << 24);
+  const u32 packed = act_pack(q);
   __builtin_memcpy(xq + 4 * i, &packed, 4);
   if ((threadIdx.x & 7) == 0) xs[b] = f16_scale ? __half2float(__float2half_rn(d)) : d;
 }
@@ -67,32 +61,6 @@ __global__ __launch_bounds__(256) void quant_q8_kernel(const float* __restrict__
 // (a 16-byte load, a 4-byte store; no LDS, no barrier).  The largest-magnitude value, the
 // first of equals, sets iscale = -127/max; q = min(127, round-half-even(iscale*x));
 // d = 1/iscale; sums of each 16 quants.
-// A wave's block, four values a lane: its quants and d.
-__device__ __forceinline__ float q8k_block(const float (&v)[4], int lane, int (&q)[4]) {
-  // |v|'s bits order as |v| does; the low word prefers the earlier index
-  u64 key = 0;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const u64 kk = ((u64)__float_as_uint(fabsf(v[k])) << 32) | (u32)(255 - (4 * lane + k));
-    key = kk > key ? kk : key;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const u32 hi = __shfl_xor((u32)(key >> 32), off), lo = __shfl_xor((u32)key, off);
-    const u64 o = ((u64)hi << 32) | lo;
-    key = o > key ? o : key;
-  }
-  const int idx = 255 - (int)(key & 0xFFFFFFFFu);             // the same in every lane
-  const int ik = idx & 3;
-  const float mine = ik == 0 ? v[0] : ik == 1 ? v[1] : ik == 2 ? v[2] : v[3];
-  const float mx = __shfl(mine, idx >> 2);
-  const bool any = (key >> 32) != 0;
-  const float iscale = any ? -127.0f / mx : 0.0f;
-#pragma unroll
-  for (int k = 0; k < 4; k++) q[k] = any ? min(127, (int)rintf(iscale * v[k])) : 0;
-  return any ? 1.0f / iscale : 0.0f;
-}
-__device__ __forceinline__ u32 q8k_pack(const int (&q)[4]) { return (u32)(q[0] & 0xFF) | ((u32)(q[1] & 0xFF) << 8) | ((u32)(q[2] & 0xFF) << 16) | ((u32)(q[3] & 0xFF) << 24); }
 template <int GLU>
 __global__ __launch_bounds__(256) void quant_q8k_kernel(const float* __restrict__ x, const float* __restrict__ up, i8* __restrict__ xq,
                                                         float* __restrict__ xd, int* __restrict__ bsums, u32 nblocks,
@@ -113,12 +81,7 @@ __global__ __launch_bounds__(256) void quant_q8k_kernel(const float* __restrict_
   }
   int q[4];
   const float d = q8k_block(v, lane, q);
-  ((u32*)(xq + b * 256))[lane] = q8k_pack(q);
-  int s = (q[0] + q[1]) + (q[2] + q[3]);
-  s += __shfl_xor(s, 1);
-  s += __shfl_xor(s, 2);
-  if ((lane & 3) == 0) bsums[b * 16 + (lane >> 2)] = s;
-  if (lane == 0) xd[b] = d;
+  q8k_store(q, d, lane, xq, xd, bsums, b);
 }
 
 // The tokens' blocks straight into each of a token's nu rows of a grouping (token t's slot s is row smap[t nu + s]), without the sums.
@@ -133,7 +96,7 @@ __global__ __launch_bounds__(256) void quant_q8k_rows_kernel(const float* __rest
   const float v[4] = {v4.x, v4.y, v4.z, v4.w};
   int q[4];
   const float d = q8k_block(v, lane, q);
-  const u32 pack = q8k_pack(q);
+  const u32 pack = act_pack(q);
   for (int s = 0; s < nu; s++) {
     const long long o = (long long)(u32)__builtin_amdgcn_readlane(mine, s) * bpr + at;
     ((u32*)(xq + o * 256))[lane] = pack;

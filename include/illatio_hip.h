@@ -413,7 +413,7 @@ int ilt_dense_decode(uint64_t stream, const ilt_dense_model* m, const int32_t* t
    second, forked, joined: a stream beside the work's own and two events, for products that share their activations and
    do not fill the GPU one by one, or zeros (all on the one stream).  act[0] holds the quantized activations of width d,
    act[1] of nh * hd, act[2] of ffn, in the formats their matrices take (Q8_0's xq and xs, the K-quants' kq, kd and ksum;
-   a format nobody takes: nulls).  scores: ntok * nh * ((pos + ntok + 3) & ~3) floats for contexts of up to 8192
+   a format nobody takes: nulls); what att holds afterwards is not defined.  scores: ntok * nh * ((pos + ntok + 3) & ~3) floats for contexts of up to 8192
    positions, not read past that.  No counterpart in the reference, whose host queues the launches one by one. */
 typedef struct ilt_dense_act { int8_t* xq; float* xs; int8_t* kq; float* kd; int32_t* ksum; } ilt_dense_act;
 typedef struct ilt_dense_work {

@@ -524,6 +524,28 @@ def test_chunk_softmax_where_the_order_of_the_sum_shows(dev, nh, pos0, ntok):
         hip.hip_free(b)
 
 
+@pytest.mark.parametrize("q8,nh,nkv,hd,n", [(False, 8, 2, 128, 2), (False, 8, 2, 128, 85), (False, 6, 3, 128, 177), (False, 8, 2, 64, 351), (False, 16, 8, 128, 819),      # whole blocks: a row a wave, the last of its kind, four rows, sixteen
+                                            (False, 6, 2, 128, 9), (False, 4, 2, 64, 5),                                                   # groups of one and a half blocks and of half a block
+                                            (True, 14, 2, 64, 3), (True, 3, 1, 128, 234), (True, 14, 2, 64, 201), (True, 14, 14, 64, 1833)])
+def test_chunk_attention_leaves_its_rows_quantized(dev, monkeypatch, q8, nh, nkv, hd, n):
+    """A chunk whose attention leaves the output product's activations in blocks, against the other attention kernels and the
+    quantizing launch behind them: logits, and the next layer's keys and values of every token, bit for bit."""
+    from illatio_amd import hip, model
+    host = (model.synth_model_q8 if q8 else model.synth_model)(31, d=256, ffn=512, nh=nh, nkv=nkv, hd=hd, nl=2, vocab=300)
+    prompt = synth.make_rng(79).integers(0, 300, n).tolist()
+    res = []
+    for mm in ("1", "0"):
+        monkeypatch.setenv("ILT_ATTN_MM", mm)
+        m = model.DenseModel(dev, host, nctx=n, chunk=n)
+        m.forward_n(prompt)
+        hip.hip_sync(dev)
+        res.append([hip.hip_floats(m.logits, 300)] + [hip.hip_floats(m.layers[1][nm], n * nkv * hd) for nm in ("kc", "vc")])
+        m.free()
+    assert np.isfinite(res[0][0]).all()
+    for a, b in zip(*res):
+        assert np.array_equal(bits(a), bits(b))
+
+
 def test_a_chunk_as_parts_side_by_side(dev):
     """forward_parts -- a chunk's halves or quarters on streams of their own, a part's attention waiting for the earlier
     parts' keys layer by layer -- leaves forward_n's logits and caches, bit for bit: halves of 128 + 128, of 256 + 44 (the
