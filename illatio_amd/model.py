@@ -325,12 +325,12 @@ class DenseModel:
         down 160, of 512 that fit), and while one part is in its attention (vector ALU) another is in its products
         (matrix cores): the parts' launches fill each other's gaps.  Every token's results are forward_n's."""
         n, dev = len(tokens), self.dev      # (up to K chunks' tokens: a part is at most a chunk)
-        per = ((n + k - 1) // k + 127) // 128 * 128
+        per = self._part(n, k)
         if k < 2 or per * (k - 1) >= n or per > self.chunk or self.pos + n > self.nctx or self.pos + n > 8192:
             return self.forward_n(tokens, logits)
         for j in range(k - 1):
             # (room for half a chunk from the start, for more once a longer part comes)
-            room = max(per, ((self.chunk + 1) // 2 + 127) // 128 * 128)
+            room = max(per, self._part(self.chunk, 2))
             if j == len(self.more_work):
                 dev2 = copy.copy(dev)
                 dev2.stream, dev2.second = hip.hip_stream_create(dev), None
@@ -388,10 +388,16 @@ class DenseModel:
             (self.forward_parts if halves else self.forward_n)(tokens[i:i + n], logits=want)
             i += n
 
+    def _part(self, n, k):
+        """The tokens of one of K parts of N: whole tiles of 128; of 64 for a few hundred through the exact products, whose tiles are
+        also of 32 and 64 tokens (280 tokens 8.5 -> 8.0 ms, 300 9.0 -> 8.1, 350 9.4 -> 9.1, 384 9.46 -> 9.59; 850 18.2 and 18.7)."""
+        g = 64 if self.prefill == "exact" and n <= 512 else 128
+        return ((n + k - 1) // k + g - 1) // g * g
+
     def _gains_as_halves(self, n):
         """Whether the next N tokens of a prompt take less time as two halves side by side than whole (or, past a chunk, than
         one after another)."""
-        half = ((n + 1) // 2 + 127) // 128 * 128
+        half = self._part(n, 2)
         if not PARTS_FROM <= n <= PARTS_UPTO or half > self.chunk or self.pos + n > min(self.nctx, 8192):
             return False
         work = n // 2 * self.c["d"] * (2 * self.qd + 2 * self.kvd + 3 * self.c["ffn"])
@@ -400,9 +406,9 @@ class DenseModel:
             # 62.7; halves of a 512-token chunk lose; their sums' order depends on a launch's token count with or without
             # parts); from resident copies 28.4 -> 27.2 and 62.7 -> 62.1: left whole.
             return self.prefill == "bf16" and 1024 <= n <= self.chunk and work >= 1e10
-        # The exact ones, the Qwen3-4B shape (whole -> halves, ms): 200 tokens 7.5 -> 7.0, 256 8.0 -> 7.1, 300 9.1 -> 8.1, 350 9.7 ->
-        # 9.0, 420 11.8 -> 10.3, 512 13.1 -> 11.9, 832 19.4 -> 18.7, 1,000 22.1 -> 20.7, 2,500 76 -> 68; 576 to 768 lose up to 9 %, 140 to
-        # 192 up to 11 %, thirds and quarters always lose to halves.  Far into a conversation a few hundred tokens are mostly
+        # The exact ones, the Qwen3-4B shape (whole -> halves, ms): 194 tokens 7.3 -> 7.0, 256 7.7 -> 7.1, 300 8.9 -> 8.1, 350 9.5 ->
+        # 9.1, 384 9.9 -> 9.6, 420 11.8 -> 11.1, 512 13.1 -> 11.8, 850 19.7 -> 18.2, 1,000 21.8 -> 21.0, 2,500 76 -> 68; 576 to 768 lose up to
+        # 9 %, 140 to 192 up to 11 %, thirds and quarters always lose to halves.  Far into a conversation a few hundred tokens are mostly
         # attention, whose launches fill the GPU whole: 512 at 1,500 positions 22.1 -> 23.8, 768 31.1 -> 34.9; 224 14.1 -> 13.0,
         # 1,024 and more as whole or up to 2 % better.  (Other shapes take these lines and the next as they are: two shapes are
         # what they were drawn from.)

@@ -548,9 +548,8 @@ def test_chunk_attention_leaves_its_rows_quantized(dev, monkeypatch, q8, nh, nkv
 
 def test_a_chunk_as_parts_side_by_side(dev):
     """forward_parts -- a chunk's halves or quarters on streams of their own, a part's attention waiting for the earlier
-    parts' keys layer by layer -- leaves forward_n's logits and caches, bit for bit: halves of 128 + 128, of 256 + 44 (the
-    second half on the products for few tokens), a second chunk whose halves see the first chunk's positions, and
-    quarters of 128."""
+    parts' keys layer by layer -- leaves forward_n's logits and caches, bit for bit: halves of 128 + 128, of 192 + 108,
+    a second chunk whose halves see the first chunk's positions, and quarters of 128."""
     from illatio_amd import hip, model
     host = model.synth_model(12, d=512, ffn=1024, nh=8, nkv=2, hd=64, nl=3, vocab=700)
     c = host["config"]
