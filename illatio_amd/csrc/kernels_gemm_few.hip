@@ -405,7 +405,7 @@ hipError_t few_launch(FewParams& p, hipStream_t st) {
   static bool attr_set[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  if (!attr_set[dev]) {            // more dynamic LDS than the default 64 KB (Q6_K on 9,728 columns: 68): asked for once per device
+  if (!attr_set[dev]) {            // more dynamic LDS than the default 64 KB: asked for once per device
     const hipError_t e = hipFuncSetAttribute((const void*)gemm_i8_few_kernel<FSET, NT, RT, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, room);
     if (e != hipSuccess) return e;
     attr_set[dev] = true;
@@ -415,9 +415,8 @@ hipError_t few_launch(FewParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
-// How a launch is cut: 32 tokens a tile from 17 on; tiles of 16 rows with the columns shared out over four waves, or over
-// eight where a row is long and the launch has no more tiles than CUs (Q6_K 2560 x 9728 on 21 tokens 25.9 -> 22.2 us, Q8_0
-// 896 x 4864 20.6 -> 16.4); tiles of 32 rows, which read the tokens half as often, once tiles of 16 are more than the CUs
+// How a launch is cut: 32 tokens a tile from 17 on; tiles of 16 rows with the columns shared out over four waves, or (Q8_0) over
+// eight where a row is long and the launch has no more tiles than CUs (896 x 4864 on 21 tokens 20.6 -> 16.4 us); tiles of 32 rows, which read the tokens half as often, once tiles of 16 are more than the CUs
 // take at a time (Q4_K 2560 x 4096 on 48 tokens, 320 tiles: 17.8 -> 14.2 us; on 32 tokens, 160: 10.5 against 14.1; Q8_0,
 // whose units are short, from 600 tiles on: 4864 x 896 on 32 tokens, 304: 7.5 against 8.5, on 48, 608: 11.6 -> 10.5).
 template <int FSET>
@@ -427,23 +426,30 @@ hipError_t few_dispatch(FewParams& p, int forced, hipStream_t st) {
   long tiles = 0;
   for (int i = 0; i < p.nmat; i++) tiles += (p.mat[i].rows + 15) / 16;
   tiles *= p.ttiles;
-  const bool wide = tiles > (FSET == ILT_Q8_0 || nt == 1 ? 600 : 256), deep = tiles <= 256 && p.cols >= (FSET == ILT_Q8_0 ? 2048 : 8192);
+  const bool wide = tiles > (FSET == ILT_Q8_0 || nt == 1 ? 600 : 256), deep = tiles <= 256 && p.cols >= 2048;
   const int v = forced > 1 ? forced : wide ? 2 : deep ? 8 : 4;
-  if (nt == 1) {
-    if constexpr (FSET == ILT_Q8_0) { if (v == 8) return few_launch<FSET, 1, 1, 8>(p, st); }      // (K-quants on up to 16 tokens: four waves)
-    return v == 2 ? few_launch<FSET, 1, 2, 4>(p, st) : few_launch<FSET, 1, 1, 4>(p, st);
-  }
-  return v == 2 ? few_launch<FSET, 2, 2, 4>(p, st) : v == 8 ? few_launch<FSET, 2, 1, 8>(p, st) : few_launch<FSET, 2, 1, 4>(p, st);
+  if constexpr (FSET == ILT_Q8_0) { if (v == 8) return nt == 1 ? few_launch<FSET, 1, 1, 8>(p, st) : few_launch<FSET, 2, 1, 8>(p, st); }      // (K-quants: four waves)
+  if (nt == 1) return v == 2 ? few_launch<FSET, 1, 2, 4>(p, st) : few_launch<FSET, 1, 1, 4>(p, st);
+  return v == 2 ? few_launch<FSET, 2, 2, 4>(p, st) : few_launch<FSET, 2, 1, 4>(p, st);
+}
+
+// Whether kernels_gemm_reg.hip's tiles of 16 rows are the better ones (rows16: tiles of 16 rows; nsb: super-blocks of a row)
+bool halves_take(bool q4, long long rows16, int ntok, int nsb) {
+  const long long t16 = rows16 * ((ntok + 15) / 16), t32 = rows16 * ((ntok + 31) / 32);
+  if (ntok <= 16) return t16 <= 512 && nsb >= (q4 ? 14 : 4);
+  return t16 <= 256 ? !q4 || nsb >= 4 : t32 <= 256 && (!q4 || nsb >= 12);
 }
 
 }  // namespace
 
 // Up to four matrices (all Q8_0, or Q4_K and Q6_K in any mix) on the same quantized tokens in one launch.
-// hipErrorNotSupported (nothing launched) where the shapes are not this kernel's.  Against the kernels with the weights in
-// operand registers (kernels_gemm_reg.hip), whose smallest tiles are 32 rows x 32 tokens, the line lies at 128 of those, whatever the
-// tokens (us here and there: Q4_K 4096 x 2560 on 32 tokens, 128 tiles: 9.2 and 10.8, 6144 x 2560 on 21, 192: 12.1 and 11.5, 2560 x 4096 on
-// 40, 160: 16.6 and 12.5; Q6_K: 2560 x 9728 on 32, 80: 25.5 both, on 40, 160: 41 and 25.6, 1024 x 2560 on 128, 128: 10.8 and 11.0).  Up to 16 tokens
-// half of those tiles is for nothing.  Q8_0 against its own kernel (kernels_gemm_q8.hip),
+// hipErrorNotSupported (nothing launched) where the shapes are not this kernel's.  K-quants against the kernels with the weights in
+// operand registers (kernels_gemm_reg.hip): those from 17 tokens on where the launch is more than 128 tiles of 32 x 32 (us here and there: Q4_K
+// 6144 x 2560 on 21, 192 tiles: 12.1 and 11.5, 2560 x 4096 on 40, 160: 16.6 and 12.5), and their tiles of 16 rows, eight waves' each, where those fit the
+// chip and their rounds of eight super-blocks have enough to do.  Up to 16 tokens (512 tiles of 16 tokens): Q4_K from fourteen on (2560 x 3072, twelve, on
+// 16 6.6 and 6.8, x 3584 7.3 and 6.7; 8192 x 4096 13.0 and 11.8), else four (2560 x 512 5.0 and 5.1, x 1024 5.8 and 5.2; 8192 x 2560 11.0 and 10.6).  More
+// tokens, 256 tiles of 16: Q4_K from four on (1024 x 512 on 24 5.2 and 5.0, x 1024 5.6 and 5.2), Q6_K always (1024 x 256 5.4 and 4.9); 256 tiles of 32:
+// Q4_K from twelve (4096 x 2560, ten, on 21 8.2 and 8.6; 2560 x 3072 on 24 8.8 and 8.3), Q6_K always (2560 x 512 6.3 and 5.6).  Q8_0 against its own kernel (kernels_gemm_q8.hip),
 // whose waves make a tile's terms and sums in registers: up to 16 tokens here, unless the tiles of 16 rows fill the chip (896 x 4864
 // on 16 tokens 12.7 us against 16.1, on 24 17.1 against 16.1; 4096 x 2048 on 16, 256 tiles: 8.1 against 8.3; 9728 x 896, 608:
 // 7.7 against 5.8); where its smallest tile does not go (cols no multiple of 128) from 640 tiles of 32 x 32 and 96 tokens on.
@@ -457,7 +463,7 @@ hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws
   FewParams p = {};
   p.nmat = nmat; p.cols = cols; p.ntok = ntok; p.acc = acc; p.xq = xq; p.xs = xs; p.bsums = bsums;
   int fset = fmts[0];
-  long long tiles32 = 0;
+  long long tiles32 = 0, tiles16 = 0;
   bool small = false;                       // a matrix of less than a tile of the registers' kernel
   for (int i = 0; i < nmat; i++) {
     const int fm = fmts[i];
@@ -470,6 +476,7 @@ hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws
     m.row_bytes = fm == ILT_Q8_0 ? cols : (long long)(cols / 256) * (fm == ILT_Q4_K ? 144 : ILT_Q6K_STRIDE);
     if (m.ldy < rows[i] || (long long)rows[i] * m.row_bytes >= 0x7FFFFFFFLL || (((uintptr_t)ws[i]) & 15)) return hipErrorNotSupported;   // 32-bit offsets
     tiles32 += (rows[i] + 31) / 32;
+    tiles16 += (rows[i] + 15) / 16;
     small |= rows[i] < 128;
   }
   tiles32 *= (ntok + 31) / 32;
@@ -479,7 +486,8 @@ hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws
       const hipError_t e = ilt_k_gemm_q8(nmat, ws, wds, rows, ys, biases, cols, xq, xs, ntok, acc, st, ldy);
       if (e != hipErrorNotSupported) return e;
     }
-  } else if (forced < 0 && !small && ntok > 16 && tiles32 > 128) return hipErrorNotSupported;
+  } else if (forced < 0 && ((!small && ntok > 16 && tiles32 > 128) || (nmat <= 3 && (nmat == 1 || !ldy) && halves_take(fset != ILT_Q6_K, tiles16, ntok, cols / 256))))
+    return hipErrorNotSupported;
   switch (fset) {
     case ILT_Q8_0: return few_dispatch<ILT_Q8_0>(p, forced, st);
     case ILT_Q4_K: return few_dispatch<ILT_Q4_K>(p, forced, st);

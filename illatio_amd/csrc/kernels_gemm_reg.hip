@@ -39,6 +39,7 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef unsigned short v2u __attribute__((ext_vector_type(2)));
 
@@ -939,6 +940,182 @@ __device__ __forceinline__ void reg_split2(const BfParams& p, const u8* w, int r
   split_store(p, sum, tok0, ntok, r0 + l32, 8 * ks + 4 * lh);
 }
 
+// Rows r0 .. + 15 x tokens tok0 .. tok0 + ntok - 1 (16 NT at most): a super-block in eight a wave's, two waves a SIMD.  A launch of some
+// twenty tokens has 80 tiles of 32 x 32 and a chain of 38 blocks (2560 x 9728), on 4 waves each: most of the chip idle.  Tiles of half the
+// rows are twice as many CUs', eight waves' chains are five blocks, and a block of 16 rows is half the operands and terms: a round takes 1.5 us
+// (NT 1) or 2 (NT 2), a fifth of it the wait for the next blocks, which are asked for as soon as a block is in registers.  The terms go through LDS a
+// float a lane: the wave that adds a result of the lanes reads the eight blocks' in the CPU's order.  NT 2: two places for a round's terms, one
+// barrier a round; NT 1: one, so that two workgroups are a CU's (480 tiles 22 -> 18 us).  us before (four or eight waves with 16-byte loads straight
+// into the operands, or reg_split) and now, matrices from memory: Q6_K 2560 x 9728 on 8 tokens 13.6 -> 11.6, 16 14.9 -> 12.4, 21 23.6 -> 14.7, 32 25.4 ->
+// 15.5, 48 26.2 -> 18.2; 1024 x 2560 on 32 10.5 -> 6.4; Q4_K 2560 x 4096 on 8 7.8 -> 6.4, 21 11.0 -> 8.3, 48 12.6 -> 11.1.
+constexpr int HS = 8;                  // waves of a workgroup, and super-blocks of a round
+template <int FMT> struct HalfW;
+template <> struct HalfW<ILT_Q4_K> {
+  using F = RegW<ILT_Q4_K>;
+  static constexpr int LOADS = 3, LBYTES = 3072;     // RegW's places for 16 rows, the headers behind them
+  struct At { u32 a, b, h; };
+  static __device__ __forceinline__ At place(u32 row_bytes, int lane) {
+    const F::At at = F::place(row_bytes, lane, 0, 0);
+    return At{at.a, at.b, (u32)(lane & 15) * row_bytes};
+  }
+  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t rw, const At& at, u32 row_bytes, u32 row0, u32 block, u8* dst) {
+    if (i < 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 1024 * i), 16, (i ? at.b : at.a) + (row0 + 8 * i) * row_bytes, block, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (ILT_LDS void*)(dst + 2048), 16, at.h + row0 * row_bytes, block, 0, 0);
+  }
+  // a lane's half of the columns (HQ): what its four groups need
+  static __device__ __forceinline__ void read(F::Block& b, F::Quants& q, const u8* ws, int l16, int lh, int hq) {
+    F::quants(q, ws, 0, l16, lh + 4 * hq); F::quants(q, ws, 2, l16, lh + 4 * hq);
+    F::block(b, ws - 2048, l16, lh);
+    b.sc[0] = hq ? b.sc[1] : b.sc[0];
+  }
+};
+template <> struct HalfW<ILT_Q6_K> {
+  using F = RegW<ILT_Q6_K>;
+  static constexpr int LOADS = 4, LBYTES = 4352;
+  using At = F::At;
+  static __device__ __forceinline__ At place(u32 row_bytes, int lane) { return F::place(row_bytes, lane, 0, 0); }
+  static __device__ __forceinline__ void issue(int i, __amdgpu_buffer_rsrc_t rw, const At& at, u32 row_bytes, u32 row0, u32 block, u8* dst) {
+    F::issue(i, rw, nullptr, at, row_bytes, row0, block, dst);
+  }
+  static __device__ __forceinline__ void read(F::Block& b, F::Quants& q, const u8* ws, int l16, int lh, int hq) {
+    F::quants(q, ws, 0, l16, lh + 4 * hq); F::quants(q, ws, 1, l16, lh + 4 * hq);
+    F::quants_now(q, ws, 0, l16, lh + 2 * hq);
+    F::block(b, ws, l16, lh);
+    b.sc.x = hq ? b.sc.z : b.sc.x; b.sc.y = hq ? b.sc.w : b.sc.y;
+  }
+};
+template <int FMT, int NT> struct HalfSmem {
+  struct { __align__(16) u8 xs[4096 * NT]; __align__(16) u8 ws[HalfW<FMT>::LBYTES]; __align__(16) float xd[16 * NT]; } w[HS];
+  float ex[NT][4 * NT][HS][RegW<FMT>::MINS ? 2 : 1][64];       // a round's terms [result of a lane][wave][a term][lane]
+};
+template <int FMT, int NT>
+__device__ __forceinline__ void reg_half(const BfParams& p, const u8* w, int r0, long tok0, int ntok, unsigned char* smem) {
+  using F = RegW<FMT>;
+  using H = HalfW<FMT>;
+  constexpr int TERMS = F::MINS ? 2 : 1;
+  static_assert(NT == 1 || NT == 2, "a wave adds one of a lane's results");
+  HalfSmem<FMT, NT>& W = *(HalfSmem<FMT, NT>*)smem;
+  const int lane = threadIdx.x & 63, ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto& S = W.w[ks];
+  const int nsb = p.cols / 256, rounds = (nsb + HS - 1) / HS;
+  // lane (l16, lh, hq): row (and token) l16, columns 128 hq + 32 s + 16 lh .. of step s
+  const int l16 = lane & 15, lq = lane >> 4, lh = lq & 1, hq = lq >> 1;
+  const u32 row_bytes = (u32)(nsb * F::BLOCK);
+  const __amdgpu_buffer_rsrc_t rw = ilt_rsrc(ilt_uniform_ptr(w), (u32)p.rows * row_bytes);      // (past the matrix's rows: zeros)
+  const typename H::At at = H::place(row_bytes, lane);
+  ntok = __builtin_amdgcn_readfirstlane(ntok);
+  const __amdgpu_buffer_rsrc_t rx = ilt_rsrc(ilt_uniform_ptr((const i8*)p.x + tok0 * (long)p.cols), (u32)(ntok * p.cols));      // (past the tile's tokens: zeros)
+  // the tokens' quants: a kilobyte the half of a super-block of eight tokens, piece q of token t at q ^ (t >> 1 & 7) of its eight
+  const u32 xpc = 16 * (u32)((lane & 7) ^ ((lane >> 4) & 3)), xrow = (u32)(lane >> 3) * (u32)p.cols;
+  const __amdgpu_buffer_rsrc_t rd = ilt_rsrc(ilt_uniform_ptr(p.xd + tok0 * nsb), (u32)(ntok * nsb) * 4);
+  const __amdgpu_buffer_rsrc_t rb = ilt_rsrc(ilt_uniform_ptr(p.bsums + (F::MINS ? tok0 * (p.cols >> 4) : 0)), F::MINS ? (u32)(ntok * (p.cols >> 4)) * 4 : 0);
+  float c_yd; int4 c_bs[NT][2];
+  auto issue = [&](int i) {
+    const int sb = min(i * HS + ks, nsb - 1);        // the wave's block of round i (past the last: the last again, for nobody)
+#pragma unroll
+    for (int k = 0; k < H::LOADS; k++) H::issue(k, rw, at, row_bytes, (u32)r0, (u32)sb * F::BLOCK, S.ws);
+#pragma unroll
+    for (int k = 0; k < 4 * NT; k++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (ILT_LDS void*)(S.xs + k * 1024), 16, xrow + (k & 1 ? xpc ^ 64 : xpc) + (u32)(8 * (k % (2 * NT))) * (u32)p.cols + 128 * (k / (2 * NT)), sb * 256, 0, 0);
+    c_yd = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, (u32)((lane & (16 * NT - 1)) * nsb) * 4, sb * 4, 0));
+    if constexpr (F::MINS) {
+#pragma unroll
+      for (int h = 0; h < NT; h++)
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+          const ilt_v4i a = __builtin_amdgcn_raw_buffer_load_b128(rb, (u32)((l16 + 16 * h) * nsb) * 64 + 32 * lh + 16 * k, sb * 64, 0);
+          c_bs[h][k] = make_int4(a.x, a.y, a.z, a.w);
+        }
+    }
+  };
+  const int xsw = (l16 >> 1) & 7;
+  float sum = 0.0f;
+  issue(0);
+#pragma unroll 1
+  for (int i = 0; i < rounds; i++) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (lane < 16 * NT) S.xd[lane] = c_yd;
+    typename F::Block blk = {};
+    typename F::Quants qs;
+    H::read(blk, qs, S.ws, l16, lh, hq);
+    v4i x[NT][4]; float4 y[NT]; v4h sums[NT];
+#pragma unroll
+    for (int h = 0; h < NT; h++) {
+#pragma unroll
+      for (int s = 0; s < 4; s++) x[h][s] = __builtin_bit_cast(v4i, ilt_lds_ld16(S.xs + 2048 * NT * hq + 128 * (l16 + 16 * h) + 16 * ((2 * s + lh) ^ xsw)));
+      y[h] = lds_f4(S.xd + 16 * h + 4 * lq);
+      if constexpr (F::MINS) {                       // sums of 32: eight times 128 * (sum >> 7) (the lower half's lanes) or eight times sum & 127
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const int4& b = c_bs[h][k >> 1];
+          const int v = k & 1 ? b.z + b.w : b.x + b.y;
+          sums[h][k] = (_Float16)(float)(v & (hq ? 127 : ~127));
+        }
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (their places are written again)
+    __builtin_amdgcn_sched_barrier(0);
+    issue(i + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    v4i X[NT], Y[NT];
+    const v4i zi = {};
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      v4i hi, lo;
+      F::group(blk, qs, s, lh, hi, lo);
+#pragma unroll
+      for (int h = 0; h < NT; h++) {
+        X[h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[h][s], hi, s ? X[h] : zi, 0, 0, 0);
+        Y[h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[h][s], lo, s ? Y[h] : zi, 0, 0, 0);
+      }
+    }
+    if (NT == 1 && i > 0) asm volatile("s_barrier" ::: "memory");      // (the round before's terms have been added)
+    float* const ex = &W.ex[i & (NT - 1)][0][ks][0][lane];
+#pragma unroll
+    for (int h = 0; h < NT; h++) {
+      v4f im = {};
+      if constexpr (F::MINS) {
+        v4h m;
+#pragma unroll
+        for (int k = 0; k < 4; k++) m[k] = lh ? blk.mins[4 + k] : blk.mins[k];
+        im = __builtin_amdgcn_mfma_f32_16x16x16f16(sums[h], m, im, 0, 0, 0);
+      }
+      const float yv[4] = {y[h].x, y[h].y, y[h].z, y[h].w};
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        float* const o = ex + (4 * h + r) * (HS * TERMS * 64);
+        if constexpr (F::MINS) *ILT_LDS_PTR(float, o) = (yv[r] * blk.dm) * im[r];
+        *ILT_LDS_PTR(float, o + (TERMS - 1) * 64) = (yv[r] * blk.d) * (float)((X[h][r] << F::SH) + Y[h][r]);
+      }
+    }
+    ilt_barrier_lds();                               // (and the reads of the round before have come back)
+    if (ks < 4 * NT) {
+      const float* const o = &W.ex[i & (NT - 1)][ks][0][0][lane];
+      float t[HS][TERMS];
+#pragma unroll
+      for (int s = 0; s < HS; s++)
+#pragma unroll
+        for (int k = 0; k < TERMS; k++) t[s][k] = *ILT_LDS_PTR(const float, o + (s * TERMS + k) * 64);
+#pragma unroll
+      for (int s = 0; s < HS; s++)
+        if (i * HS + s < nsb) {
+          if constexpr (F::MINS) sum = sum - t[s][0];
+          sum = sum + t[s][TERMS - 1];
+        }
+      asm volatile("" : "+v"(sum));                  // (the reads have come back before the wave meets the next barrier)
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the last round's loads, for nobody: nothing may land in LDS after the workgroup ends)
+  const int tok = 16 * (ks >> 2) + 4 * lq + (ks & 3), row = r0 + l16;
+  if (ks < 4 * NT && tok < ntok && row < p.rows) {
+    float* const o = p.y + (tok0 + tok) * p.ldy + row;
+    float v = sum;
+    if (p.bias) v = v + p.bias[row];
+    if (p.acc) v = *o + v;
+    *o = v;
+  }
+}
+
 // FSET: the matrices' format, or 0 where Q4_K and Q6_K meet in a launch
 template <int FSET, int NP, int WR, int WT>
 __global__ __launch_bounds__(64 * WR * WT, WR * WT == 1 ? 1 : 2) void gemm_i8r_kernel(BfParams p) {
@@ -990,6 +1167,27 @@ __global__ __launch_bounds__(256, TWO ? 2 : 1) void gemm_i8s_kernel(BfParams p) 
   }
 }
 
+template <int FSET, int NT>
+__global__ __launch_bounds__(64 * HS, NT == 1 ? 2 : 1) void gemm_i8h_kernel(BfParams p) {
+  constexpr int TM = 16;
+  extern __shared__ __align__(16) unsigned char smem[];
+  long tok0; int ntok, rt; const u8* w = p.w;
+  if (!pick_tile<TM, 16 * NT>(p, tok0, ntok, rt, w)) return;
+  // which of the launch's matrices the row tile belongs to
+  const int n0 = (p.mrows[0] + TM - 1) / TM, n1 = n0 + (p.mrows[1] + TM - 1) / TM;
+  const int m = rt < n0 ? 0 : rt < n1 ? 1 : 2;
+  rt -= m == 0 ? 0 : m == 1 ? n0 : n1;
+  w = m == 0 ? p.mw[0] : m == 1 ? p.mw[1] : p.mw[2];
+  p.rows = m == 0 ? p.mrows[0] : m == 1 ? p.mrows[1] : p.mrows[2];
+  p.y = m == 0 ? p.my[0] : m == 1 ? p.my[1] : p.my[2];
+  p.bias = m == 0 ? p.mbias[0] : m == 1 ? p.mbias[1] : p.mbias[2];
+  if (p.nmulti > 1) p.ldy = p.rows;
+  const int fmt = m == 0 ? p.mfmt[0] : m == 1 ? p.mfmt[1] : p.mfmt[2];
+  if constexpr (FSET != 0) reg_half<FSET, NT>(p, w, rt * TM, tok0, ntok, smem);
+  else if (fmt == ILT_Q4_K) reg_half<ILT_Q4_K, NT>(p, w, rt * TM, tok0, ntok, smem);
+  else reg_half<ILT_Q6_K, NT>(p, w, rt * TM, tok0, ntok, smem);
+}
+
 template <int FMT, int NP, int WR, int WT> constexpr size_t reg_smem() {
   if constexpr (FMT != 0) return sizeof(RegSmemOf<FMT, NP, WR, WT>);
   else return reg_smem<ILT_Q4_K, NP, WR, WT>() > reg_smem<ILT_Q6_K, NP, WR, WT>() ? reg_smem<ILT_Q4_K, NP, WR, WT>() : reg_smem<ILT_Q6_K, NP, WR, WT>();
@@ -1036,6 +1234,27 @@ hipError_t launch_i8s(BfParams& p, hipStream_t st) {
   const long long total = (long long)((p.ntok + 31) / 32) * tiles, per = (total + 7) / 8;
   if (per * 8 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
   hipLaunchKernelGGL((gemm_i8s_kernel<FSET, TWO>), dim3((unsigned)(per * 8)), dim3(256), smem, st, p);
+  return hipGetLastError();
+}
+template <int FSET, int NT>
+hipError_t launch_i8h(BfParams& p, hipStream_t st) {
+  constexpr size_t s4 = sizeof(HalfSmem<ILT_Q4_K, NT>), s6 = sizeof(HalfSmem<ILT_Q6_K, NT>);
+  constexpr size_t smem = FSET == ILT_Q4_K ? s4 : FSET == ILT_Q6_K ? s6 : s4 > s6 ? s4 : s6;
+  static_assert((NT == 1 ? 2 : 1) * smem <= 160 * 1024, "two workgroups' LDS, or one's");
+  static bool attr_set[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  if (!attr_set[dev]) {
+    const hipError_t e = hipFuncSetAttribute((const void*)gemm_i8h_kernel<FSET, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return e;
+    attr_set[dev] = true;
+  }
+  long long tiles = 0;
+  for (int m = 0; m < p.nmulti; m++) tiles += (p.mrows[m] + 15) / 16;
+  p.rows = (int)(tiles * 16);
+  const long long total = (long long)((p.ntok + 16 * NT - 1) / (16 * NT)) * tiles, per = (total + 7) / 8;
+  if (per * 8 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((gemm_i8h_kernel<FSET, NT>), dim3((unsigned)(per * 8)), dim3(64 * HS), smem, st, p);
   return hipGetLastError();
 }
 
@@ -1099,6 +1318,8 @@ constexpr RegTile kRegTiles[] = {
 // 1.95 us a round, one of two (reg_split2) 2.25, two 3.15; besides, microseconds, a tile's start and end, and the launch's, which tiles
 // of the other kinds have once.  Workgroups past those that fit start as the first ones end: 0.7 of what they take alone.
 constexpr float kRegStart = 4.0f, kSplitStart = 2.8f, kSplitTile = 2.2f, kSplitRound = 1.95f, kSplitRound2[2] = {2.25f, 3.15f};
+// And for tiles of 16 rows (reg_half), a round eight super-blocks: of 32 tokens 2.1 us, 256 tiles at a time; of 16 tokens 1.75 a workgroup a CU, 2.6 two.
+constexpr float kHalfStart2 = 3.8f, kHalfStart1 = 3.2f, kHalfTile = 1.6f, kHalfRound2 = 2.1f, kHalfRound1[2] = {1.75f, 2.6f};
 // Which of them, by the rounds that the chip takes the launch's workgroups in.  (Shapes, us for the tiles taken and for 64 or 128
 // rows x 128 tokens: Q6_K 2560 x 9728 on 256 tokens 54 and 89, on 512 81 and 90; Q4_K 2560 x 4096 on 256 25 and 33; 19456 x 2560 on 32
 // 17.6 and 31, on 192 35 and 48; 9728 x 2560 on 64 17.2 and 22.)
@@ -1121,9 +1342,17 @@ int reg_tile_of(const BfParams& p) {
   }
   const long long n = workgroups(32, 32), rest = n % 512;
   const float rounds = (float)((nsb + KS - 1) / KS);
-  if (n <= 256 && kSplitStart + kSplitTile + kSplitRound * rounds < least) return 5;
-  const float part = rest ? kSplitTile + kSplitRound2[(rest - 1) / 256] * rounds : 0.0f;
-  if (kSplitStart + (float)(n / 512) * (kSplitTile + kSplitRound2[1] * rounds) + (n > 512 ? 0.7f : 1.0f) * part < least) return 6;
+  auto take = [&](int v, float us) { if (us < least) { best = v; least = us; } };
+  if (n <= 256) take(5, kSplitStart + kSplitTile + kSplitRound * rounds);
+  else {
+    const float part = rest ? kSplitTile + kSplitRound2[(rest - 1) / 256] * rounds : 0.0f;
+    take(6, kSplitStart + (float)(n / 512) * (kSplitTile + kSplitRound2[1] * rounds) + (n > 512 ? 0.7f : 1.0f) * part);
+  }
+  const float rounds8 = (float)((nsb + HS - 1) / HS);
+  const long long n2 = workgroups(16, 32), n1 = workgroups(16, 16), rest1 = n1 % 512;
+  take(7, kHalfStart2 + (float)((n2 + 255) / 256) * (kHalfRound2 * rounds8 + kHalfTile) - kHalfTile);
+  const float part1 = rest1 == 0 ? 0.0f : rest1 <= 256 ? kHalfRound1[0] * rounds8 : kHalfTile + kHalfRound1[1] * rounds8;
+  take(8, kHalfStart1 + (float)(n1 / 512) * (kHalfTile + kHalfRound1[1] * rounds8) + part1);
   return best;
 }
 
@@ -1134,13 +1363,15 @@ hipError_t dispatch_i8r(BfParams& p, int forced, hipStream_t st) {
     const bool big = forced ? forced == 128 : (long long)((p.mrows[0] + 127) / 128) * ((p.ntok + 127) / 128) >= 150;
     return big ? launch_i8r<FSET, 4, 4, 1>(p, st) : launch_i8r<FSET, 2, 2, 2>(p, st);
   } else {
-    switch (forced == 128 ? 4 : forced == 64 ? 3 : forced >= 1 && forced <= 7 ? forced - 1 : reg_tile_of<FSET>(p)) {
+    switch (forced == 128 ? 4 : forced == 64 ? 3 : forced >= 1 && forced <= 9 ? forced - 1 : reg_tile_of<FSET>(p)) {
       case 0: return launch_i8r<FSET, 1, 1, 1>(p, st);
       case 1: return launch_i8r<FSET, 2, 1, 1>(p, st);
       case 2: return launch_i8r<FSET, 2, 2, 1>(p, st);
       case 3: return launch_i8r<FSET, 2, 2, 2>(p, st);
       case 5: return launch_i8s<FSET, false>(p, st);
       case 6: return launch_i8s<FSET, true>(p, st);
+      case 7: return launch_i8h<FSET, 2>(p, st);
+      case 8: return launch_i8h<FSET, 1>(p, st);
       default: return launch_i8r<FSET, 4, 4, 1>(p, st);
     }
   }
@@ -1154,7 +1385,7 @@ constexpr int block_bytes_of(int fmt) {
 
 // Up to three matrices (Q4_K, Q6_K in any mix, or all Q2_K, or all IQ2_XXS) on the same tokens in one launch, their row tiles one after another.
 // hipErrorNotSupported, and nothing launched, where the shapes are not this kernel's.  ILT_I8_TM (tests): 64 or 128 rows by 128 tokens
-// whatever the shape, 1 to 5 the tiles in kRegTiles' order, 6 and 7 the two kernels for few tiles.
+// whatever the shape, 1 to 5 the tiles in kRegTiles' order, 6 and 7 the two kernels for few tiles, 8 and 9 the tiles of 16 rows, 32 and 16 tokens.
 hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws, const int* rows, float* const* ys, const float* const* biases,
                              int cols, const int8_t* xq, const float* xd, const int* bsums, int ntok, int acc, hipStream_t st, long long ldy) {
   if (nmat < 1 || nmat > 3 || ntok < 1 || cols < 256 || cols % 256 != 0 || cols >= (1 << 22)) return hipErrorNotSupported;

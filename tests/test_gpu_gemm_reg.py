@@ -69,8 +69,17 @@ def test_super_blocks_shared_out_bit_for_bit(dev, monkeypatch, tile, qtype, rows
     test_operands_in_registers_bit_for_bit(dev, monkeypatch, tile, qtype, rows, cols, n)
 
 
+# the same over eight waves, tiles of 16 rows and of 32 and 16 tokens
+@pytest.mark.parametrize("tile", ["8", "9"])
+@pytest.mark.parametrize("qtype,rows,cols,n", [
+    (synth.Q4_K, 1, 256, 2), (synth.Q4_K, 17, 2048, 33), (synth.Q4_K, 33, 2304, 16), (synth.Q4_K, 300, 4096, 21),
+    (synth.Q6_K, 15, 256, 31), (synth.Q6_K, 16, 1792, 17), (synth.Q6_K, 47, 4352, 9), (synth.Q6_K, 128, 9728, 64)])
+def test_super_blocks_shared_out_over_eight_waves_bit_for_bit(dev, monkeypatch, tile, qtype, rows, cols, n):
+    test_operands_in_registers_bit_for_bit(dev, monkeypatch, tile, qtype, rows, cols, n)
+
+
 # Q, K and V of mixed formats in one launch of such tiles, against the products for few tokens
-@pytest.mark.parametrize("tile", ["6", "7"])
+@pytest.mark.parametrize("tile", ["6", "7", "8", "9"])
 def test_mixed_formats_with_super_blocks_shared_out(dev, monkeypatch, tile):
     from illatio_amd import hip, model
     host = model.synth_model(12, d=768, ffn=1024, nh=12, nkv=4, hd=64, nl=2, vocab=700)
