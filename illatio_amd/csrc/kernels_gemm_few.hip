@@ -433,10 +433,10 @@ hipError_t few_dispatch(FewParams& p, int forced, hipStream_t st) {
   return v == 2 ? few_launch<FSET, 2, 2, 4>(p, st) : few_launch<FSET, 2, 1, 4>(p, st);
 }
 
-// Whether kernels_gemm_reg.hip's tiles of 16 rows are the better ones (rows16: tiles of 16 rows; nsb: super-blocks of a row)
+// Whether kernels_gemm_reg.hip's waves of 16 rows are the better ones (rows16: tiles of 16 rows; nsb: super-blocks of a row)
 bool halves_take(bool q4, long long rows16, int ntok, int nsb) {
   const long long t16 = rows16 * ((ntok + 15) / 16), t32 = rows16 * ((ntok + 31) / 32);
-  if (ntok <= 16) return t16 <= 512 && nsb >= (q4 ? 14 : 4);
+  if (ntok <= 16) return t16 <= 512 ? nsb >= (q4 ? 14 : 4) : q4 ? ntok >= 12 && t16 >= 1024 : nsb >= 4;
   return t16 <= 256 ? !q4 || nsb >= 4 : t32 <= 256 && (!q4 || nsb >= 12);
 }
 
@@ -447,7 +447,8 @@ bool halves_take(bool q4, long long rows16, int ntok, int nsb) {
 // operand registers (kernels_gemm_reg.hip): those from 17 tokens on where the launch is more than 128 tiles of 32 x 32 (us here and there: Q4_K
 // 6144 x 2560 on 21, 192 tiles: 12.1 and 11.5, 2560 x 4096 on 40, 160: 16.6 and 12.5), and their tiles of 16 rows, eight waves' each, where those fit the
 // chip and their rounds of eight super-blocks have enough to do.  Up to 16 tokens (512 tiles of 16 tokens): Q4_K from fourteen on (2560 x 3072, twelve, on
-// 16 6.6 and 6.8, x 3584 7.3 and 6.7; 8192 x 4096 13.0 and 11.8), else four (2560 x 512 5.0 and 5.1, x 1024 5.8 and 5.2; 8192 x 2560 11.0 and 10.6).  More
+// 16 6.6 and 6.8, x 3584 7.3 and 6.7; 8192 x 4096 13.0 and 11.8), else four (2560 x 512 5.0 and 5.1, x 1024 5.8 and 5.2; 8192 x 2560 11.0 and 10.6); past those tiles
+// Q6_K as before (12288 x 4096 on 8 20.8 and 16.3), Q4_K from 1,024 tiles and twelve tokens on (19456 x 2560 on 4 13.2 and 13.6, 16 15.5 and 14.4).  More
 // tokens, 256 tiles of 16: Q4_K from four on (1024 x 512 on 24 5.2 and 5.0, x 1024 5.6 and 5.2), Q6_K always (1024 x 256 5.4 and 4.9); 256 tiles of 32:
 // Q4_K from twelve (4096 x 2560, ten, on 21 8.2 and 8.6; 2560 x 3072 on 24 8.8 and 8.3), Q6_K always (2560 x 512 6.3 and 5.6).  Q8_0 against its own kernel (kernels_gemm_q8.hip),
 // whose waves make a tile's terms and sums in registers: up to 16 tokens here, unless the tiles of 16 rows fill the chip (896 x 4864

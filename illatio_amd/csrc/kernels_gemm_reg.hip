@@ -767,7 +767,7 @@ __device__ __forceinline__ void reg_split(const BfParams& p, const u8* w, int r0
 // The same with two workgroups a CU, where there are more tiles than CUs: one buffer for the tokens and one for the rows' blocks, asked
 // for anew as soon as a block is through, so that a wave waits for them while the other workgroup's waves work; the tokens' sums in
 // registers; and of a block's terms only those in LDS that another wave adds: 77 to 79 KB.  Alone on a CU it takes 2.25 us
-// a round for reg_split's 1.95, two of them 3.15.  us with whole tiles and now, matrices from memory: Q6_K 2560 x 9728 on 160 tokens
+// a round for reg_split's 1.95, two of them 3.25.  us with whole tiles and now, matrices from memory: Q6_K 2560 x 9728 on 160 tokens
 // 62 -> 37, on 256 62 -> 54; 4096 x 4096 on 128 28 -> 20; Q4_K 2560 x 4096 on 128 24 -> 18.
 template <int FMT> struct SplitSmem2 {
   struct { __align__(16) u8 xs[8192]; __align__(16) u8 ws[RegW<FMT>::LBYTES]; float xd[2][32]; } w[KS];
@@ -1116,6 +1116,144 @@ __device__ __forceinline__ void reg_half(const BfParams& p, const u8* w, int r0,
   }
 }
 
+// Rows r0 .. + 63 x tokens tok0 .. tok0 + ntok - 1 (16 NT at most): four waves of 16 rows, each through all the blocks, on the same tokens in LDS;
+// a barrier a block.  For matrices of many rows on few tokens, where a tile of 32 rows is one wave's, of which there are not enough for the
+// SIMDs, and its block twice the instructions: 0.55, 0.75 and 1.15 us a block for NT 1, 2 and 4 a workgroup a CU, what their 190 to 380
+// instructions take at a wave a SIMD; two workgroups 1.0, 1.25 and 1.75.  (The loads a block further ahead, six or eight waves a workgroup: within 5 %.)
+// us with the tiles before and now, matrices from memory: Q4_K 19456 x 2560 on 21 tokens 17.4 -> 16.6, 48 24.4 -> 22, 64 25.2 -> 23; 6144 x 2560 on 64
+// 14.4 -> 11.9, 128 17.0 -> 15.6, 256 23.4 -> 21.5; 24576 x 4096 on 16 26.7 -> 21.1, 64 39.9 -> 33; Q6_K 12288 x 4096 on 16 20.5 -> 16.3, 21 20.9 -> 18.0,
+// 64 30.7 -> 24.1, 128 41 -> 33.4.
+template <int FMT, int NT> struct RowsSmem {
+  static constexpr int XB = NT > 2 ? 2 : 3;          // buffers of a block's tokens and rows
+  __align__(16) u8 xs[XB][4096 * NT];
+  __align__(16) u8 ws[4][XB][HalfW<FMT>::LBYTES];
+  __align__(16) u8 ms[2][RegW<FMT>::MINS ? 512 * NT : 16];       // the tokens' sums of 32 as halves (RegSmem's)
+  __align__(16) float xd[2][16 * NT];
+};
+template <int FMT, int NT>
+__device__ __forceinline__ void reg_rows(const BfParams& p, const u8* w, int r0, long tok0, int ntok, unsigned char* smem) {
+  using F = RegW<FMT>;
+  using H = HalfW<FMT>;
+  using Smem = RowsSmem<FMT, NT>;
+  constexpr int XB = Smem::XB, AHEAD = XB - 1;
+  static_assert(NT <= 8, "half a token a thread");
+  Smem& S = *(Smem*)smem;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int nsb = p.cols / 256;
+  const int l16 = lane & 15, lq = lane >> 4, lh = lq & 1, hq = lq >> 1;      // (reg_half's)
+  const u32 row_bytes = (u32)(nsb * F::BLOCK);
+  const __amdgpu_buffer_rsrc_t rw = ilt_rsrc(ilt_uniform_ptr(w), (u32)p.rows * row_bytes);      // (past the matrix's rows: zeros)
+  const typename H::At at = H::place(row_bytes, lane);
+  ntok = __builtin_amdgcn_readfirstlane(ntok);
+  const __amdgpu_buffer_rsrc_t rx = ilt_rsrc(ilt_uniform_ptr((const i8*)p.x + tok0 * (long)p.cols), (u32)(ntok * p.cols));      // (past the tile's tokens: zeros)
+  const u32 xpc = 16 * (u32)((lane & 7) ^ ((lane >> 4) & 3)), xrow = (u32)(lane >> 3) * (u32)p.cols;
+  const __amdgpu_buffer_rsrc_t rd = ilt_rsrc(ilt_uniform_ptr(p.xd + tok0 * nsb), (u32)(ntok * nsb) * 4);
+  const __amdgpu_buffer_rsrc_t rb = ilt_rsrc(ilt_uniform_ptr(p.bsums + (F::MINS ? tok0 * (p.cols >> 4) : 0)), F::MINS ? (u32)(ntok * (p.cols >> 4)) * 4 : 0);
+  auto issue = [&](int sb) {
+    const int b = sb % XB, at_sb = min(sb, nsb - 1);      // (past the last: the last again, for nobody)
+#pragma unroll
+    for (int k = 0; k < H::LOADS; k++) H::issue(k, rw, at, row_bytes, (u32)(r0 + 16 * wave), (u32)at_sb * F::BLOCK, S.ws[wave][b]);
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+      const int k = wave * NT + j;                   // a kilobyte: half k / 2 NT of the block, eight tokens
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (ILT_LDS void*)(S.xs[b] + k * 1024), 16, xrow + (k & 1 ? xpc ^ 64 : xpc) + (u32)(8 * (k % (2 * NT))) * (u32)p.cols + 128 * (k / (2 * NT)),
+                                               at_sb * 256, 0, 0);
+    }
+  };
+  // the tokens' scales and sums of 32, half a token a thread
+  float c_yd; int4 c_bs[2];
+  auto load_consts = [&](int sb) {
+    if (t >= 32 * NT) return;
+    const u32 ctok = (u32)((t >> 1) * nsb);
+    c_yd = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, ctok * 4, min(sb, nsb - 1) * 4, 0));
+    if constexpr (F::MINS) {
+      const u32 o = ctok * 64 + 32 * (t & 1);
+      const ilt_v4i a = __builtin_amdgcn_raw_buffer_load_b128(rb, o, min(sb, nsb - 1) * 64, 0), b = __builtin_amdgcn_raw_buffer_load_b128(rb, o + 16, min(sb, nsb - 1) * 64, 0);
+      c_bs[0] = make_int4(a.x, a.y, a.z, a.w); c_bs[1] = make_int4(b.x, b.y, b.z, b.w);
+    }
+  };
+  auto store_consts = [&](int buf) {
+    if (t >= 32 * NT) return;
+    if ((t & 1) == 0) S.xd[buf][t >> 1] = c_yd;
+    if constexpr (F::MINS) {
+      const int4 &b0 = c_bs[0], &b1 = c_bs[1];
+      const int s[4] = { b0.x + b0.y, b0.z + b0.w, b1.x + b1.y, b1.z + b1.w };
+      _Float16 hh[4], ll[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) { hh[k] = (_Float16)(float)(s[k] & ~127); ll[k] = (_Float16)(float)(s[k] & 127); }
+      _Float16* const dst = (_Float16*)(S.ms[buf] + 32 * (t >> 1)) + 4 * (t & 1);
+      __builtin_memcpy(dst, hh, 8);
+      __builtin_memcpy(dst + 8, ll, 8);
+    }
+  };
+  const int xsw = (l16 >> 1) & 7;
+  v4f sum[NT];
+#pragma unroll
+  for (int h = 0; h < NT; h++) sum[h] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  if (AHEAD == 2) { issue(0); __builtin_amdgcn_sched_barrier(0); }
+  load_consts(0);
+  __builtin_amdgcn_sched_barrier(0);
+  issue(AHEAD - 1);
+#pragma unroll 1
+  for (int sb = 0; sb < nsb; sb++) {
+    // this block's loads and its constants' have landed; with three buffers the next block's are still on their way
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"((AHEAD - 1) * (H::LOADS + NT)) : "memory");
+    store_consts(sb & 1);
+    ilt_barrier_lds();
+    __builtin_amdgcn_sched_barrier(0);
+    const int b = sb % XB;
+    typename F::Block blk = {};
+    typename F::Quants qs;
+    v4i x[NT][4]; float4 y[NT]; v4h sums[NT];
+    H::read(blk, qs, S.ws[wave][b], l16, lh, hq);
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int h = 0; h < NT; h++) x[h][s] = __builtin_bit_cast(v4i, ilt_lds_ld16(S.xs[b] + 2048 * NT * hq + 128 * (l16 + 16 * h) + 16 * ((2 * s + lh) ^ xsw)));
+#pragma unroll
+    for (int h = 0; h < NT; h++) {
+      if constexpr (F::MINS) __builtin_memcpy(&sums[h], S.ms[sb & 1] + 32 * (l16 + 16 * h) + 8 * lq, 8);
+      y[h] = lds_f4(S.xd[sb & 1] + 16 * h + 4 * lq);
+    }
+    __builtin_amdgcn_sched_barrier(6);               // (the reads first; what is made of them may wait)
+    load_consts(sb + 1);
+    __builtin_amdgcn_sched_barrier(6);
+    issue(sb + AHEAD);
+    __builtin_amdgcn_sched_barrier(6);
+    v4i X[NT], Y[NT];
+    const v4i zi = {};
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      v4i hi, lo;
+      F::group(blk, qs, s, lh, hi, lo);
+#pragma unroll
+      for (int h = 0; h < NT; h++) {
+        X[h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[h][s], hi, s ? X[h] : zi, 0, 0, 0);
+        Y[h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[h][s], lo, s ? Y[h] : zi, 0, 0, 0);
+      }
+    }
+    v4h m = {};
+    if constexpr (F::MINS) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) m[k] = lh ? blk.mins[4 + k] : blk.mins[k];
+    }
+#pragma unroll
+    for (int h = 0; h < NT; h++) {
+      v4f im = {};
+      if constexpr (F::MINS) im = __builtin_amdgcn_mfma_f32_16x16x16f16(sums[h], m, im, 0, 0, 0);
+      const float yv[4] = {y[h].x, y[h].y, y[h].z, y[h].w};
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        if constexpr (F::MINS) sum[h][r] = sum[h][r] - (yv[r] * blk.dm) * im[r];
+        sum[h][r] = sum[h][r] + (yv[r] * blk.d) * (float)((X[h][r] << F::SH) + Y[h][r]);
+      }
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the last loads, for nobody: nothing may land in LDS after the workgroup ends)
+#pragma unroll
+  for (int h = 0; h < NT; h++) split_store(p, sum[h], tok0, ntok, r0 + 16 * wave + l16, 16 * h + 4 * lq);
+}
+
 // FSET: the matrices' format, or 0 where Q4_K and Q6_K meet in a launch
 template <int FSET, int NP, int WR, int WT>
 __global__ __launch_bounds__(64 * WR * WT, WR * WT == 1 ? 1 : 2) void gemm_i8r_kernel(BfParams p) {
@@ -1188,6 +1326,27 @@ __global__ __launch_bounds__(64 * HS, NT == 1 ? 2 : 1) void gemm_i8h_kernel(BfPa
   else reg_half<ILT_Q6_K, NT>(p, w, rt * TM, tok0, ntok, smem);
 }
 
+template <int FSET, int NT>
+__global__ __launch_bounds__(256, 2) void gemm_i8w_kernel(BfParams p) {
+  constexpr int TM = 64;
+  extern __shared__ __align__(16) unsigned char smem[];
+  long tok0; int ntok, rt; const u8* w = p.w;
+  if (!pick_tile<TM, 16 * NT>(p, tok0, ntok, rt, w)) return;
+  // which of the launch's matrices the row tile belongs to
+  const int n0 = (p.mrows[0] + TM - 1) / TM, n1 = n0 + (p.mrows[1] + TM - 1) / TM;
+  const int m = rt < n0 ? 0 : rt < n1 ? 1 : 2;
+  rt -= m == 0 ? 0 : m == 1 ? n0 : n1;
+  w = m == 0 ? p.mw[0] : m == 1 ? p.mw[1] : p.mw[2];
+  p.rows = m == 0 ? p.mrows[0] : m == 1 ? p.mrows[1] : p.mrows[2];
+  p.y = m == 0 ? p.my[0] : m == 1 ? p.my[1] : p.my[2];
+  p.bias = m == 0 ? p.mbias[0] : m == 1 ? p.mbias[1] : p.mbias[2];
+  if (p.nmulti > 1) p.ldy = p.rows;
+  const int fmt = m == 0 ? p.mfmt[0] : m == 1 ? p.mfmt[1] : p.mfmt[2];
+  if constexpr (FSET != 0) reg_rows<FSET, NT>(p, w, rt * TM, tok0, ntok, smem);
+  else if (fmt == ILT_Q4_K) reg_rows<ILT_Q4_K, NT>(p, w, rt * TM, tok0, ntok, smem);
+  else reg_rows<ILT_Q6_K, NT>(p, w, rt * TM, tok0, ntok, smem);
+}
+
 template <int FMT, int NP, int WR, int WT> constexpr size_t reg_smem() {
   if constexpr (FMT != 0) return sizeof(RegSmemOf<FMT, NP, WR, WT>);
   else return reg_smem<ILT_Q4_K, NP, WR, WT>() > reg_smem<ILT_Q6_K, NP, WR, WT>() ? reg_smem<ILT_Q4_K, NP, WR, WT>() : reg_smem<ILT_Q6_K, NP, WR, WT>();
@@ -1258,6 +1417,28 @@ hipError_t launch_i8h(BfParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
+template <int FSET, int NT>
+hipError_t launch_i8w(BfParams& p, hipStream_t st) {
+  constexpr size_t s4 = sizeof(RowsSmem<ILT_Q4_K, NT>), s6 = sizeof(RowsSmem<ILT_Q6_K, NT>);
+  constexpr size_t smem = FSET == ILT_Q4_K ? s4 : FSET == ILT_Q6_K ? s6 : s4 > s6 ? s4 : s6;
+  static_assert(2 * smem <= 160 * 1024, "two workgroups' LDS");
+  static bool attr_set[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  if (!attr_set[dev]) {
+    const hipError_t e = hipFuncSetAttribute((const void*)gemm_i8w_kernel<FSET, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return e;
+    attr_set[dev] = true;
+  }
+  long long tiles = 0;
+  for (int m = 0; m < p.nmulti; m++) tiles += (p.mrows[m] + 63) / 64;
+  p.rows = (int)(tiles * 64);
+  const long long total = (long long)((p.ntok + 16 * NT - 1) / (16 * NT)) * tiles, per = (total + 7) / 8;
+  if (per * 8 > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((gemm_i8w_kernel<FSET, NT>), dim3((unsigned)(per * 8)), dim3(256), smem, st, p);
+  return hipGetLastError();
+}
+
 // The experts' products: token tiles of every expert's rows in turn, 128 rows of the expert's matrix (of two, one behind the
 // other in the output: gate and up) a workgroup.  A group of up to 32 (64) rows goes as one (two) patches of 32.
 template <int FMT>
@@ -1300,29 +1481,34 @@ hipError_t launch_i8r_group(const BfParams& p, long long total_rows, hipStream_t
 }
 
 // The tiles a launch may be cut into.  What a workgroup of each takes for a super-block, microseconds, with 1, 2, ... of them on
-// a CU, as many as fit (Q4_K; Q6_K), measured on 1,024 to 19,456 rows and 17 to 768 tokens: a wave alone on its SIMD issues an
+// a CU, as many as fit (Q4_K; Q6_K), measured on 1,024 to 19,456 rows and 17 to 1,280 tokens, the matrices from memory: a wave alone on its SIMD issues an
 // instruction in 2.1 ns, two in 1.05 each, so tiles of one wave are the fastest way through the columns while there are fewer
 // of them than SIMDs, and large tiles, which unpack a weight for more tokens, once there are more.  (Workgroups of two waves come
 // to lie on the same two SIMDs of a CU: 1.4, then 2.35.)  The chip is taken to be empty: where another stream's launches run beside
-// (the halves of a prompt) a launch takes longer than this says -- down at the Qwen3-4B shape on 256 tokens 61 us here, 57-64 alone,
-// 87 beside the other half -- and the choice is the one for a launch alone.
+// (the halves of a prompt) a launch takes longer than this says -- down at the Qwen3-4B shape on 256 tokens 49 us here and alone, 60-70 beside the
+// other half -- and the choice is the one for a launch alone, but for the largest tiles, which do the most for an instruction: two on a CU take
+// 5.45 and 5.0 alone, and with those figures here 512 tokens as halves took 11.3 ms instead of 10.6, 2,000 50.1 instead of 48.5.
 struct RegTile { int rows, tokens, fit; float us[2][5]; };
 constexpr RegTile kRegTiles[] = {
-  {32, 32, 5, {{1.1f, 1.18f, 1.3f, 1.35f, 2.0f}, {1.4f, 1.5f, 1.65f, 2.05f, 4.0f}}},       // (Q6_K: four fit, a fifth is a second round)
-  {32, 64, 4, {{1.75f, 1.95f, 2.05f, 2.4f}, {1.75f, 1.9f, 2.1f, 2.4f}}},
-  {64, 64, 4, {{1.4f, 2.35f, 2.6f, 3.05f}, {1.6f, 2.65f, 2.85f, 3.3f}}},
-  {64, 128, 2, {{1.7f, 2.8f}, {1.75f, 2.9f}}},
-  {128, 128, 2, {{2.6f, 4.4f}, {2.55f, 4.4f}}},
+  {32, 32, 5, {{1.1f, 1.18f, 1.3f, 1.35f, 2.0f}, {1.4f, 1.5f, 1.65f, 1.8f, 4.0f}}},       // (Q6_K: four fit, a fifth is a second round)
+  {32, 64, 4, {{1.75f, 1.95f, 2.1f, 2.55f}, {1.95f, 2.05f, 2.15f, 2.35f}}},
+  {64, 64, 4, {{1.55f, 2.5f, 2.8f, 3.3f}, {2.0f, 2.7f, 2.9f, 3.3f}}},
+  {64, 128, 2, {{2.0f, 3.1f}, {2.25f, 3.1f}}},
+  {128, 128, 2, {{3.0f, 4.4f}, {2.85f, 4.4f}}},
+  {64, 16, 2, {{0.57f, 1.04f}, {0.77f, 1.16f}}},     // reg_rows from here on
+  {64, 32, 2, {{0.8f, 1.23f}, {0.86f, 1.38f}}},
+  {64, 64, 2, {{1.2f, 1.88f}, {1.2f, 1.8f}}},
 };
+constexpr int kTileOf[] = {0, 1, 2, 3, 4, 9, 10, 11};      // their numbers in dispatch_i8r
 // The same for tiles whose super-blocks are shared out, where a round is KS of them, whatever the format: a workgroup a CU (reg_split)
-// 1.95 us a round, one of two (reg_split2) 2.25, two 3.15; besides, microseconds, a tile's start and end, and the launch's, which tiles
+// 1.95 us a round, one of two (reg_split2) 2.25, two 3.25; besides, microseconds, a tile's start and end, and the launch's, which tiles
 // of the other kinds have once.  Workgroups past those that fit start as the first ones end: 0.7 of what they take alone.
-constexpr float kRegStart = 4.0f, kSplitStart = 2.8f, kSplitTile = 2.2f, kSplitRound = 1.95f, kSplitRound2[2] = {2.25f, 3.15f};
+constexpr float kRegStart = 4.0f, kSplitStart = 2.8f, kSplitTile = 2.2f, kSplitRound = 1.95f, kSplitRound2[2] = {2.25f, 3.25f};
 // And for tiles of 16 rows (reg_half), a round eight super-blocks: of 32 tokens 2.1 us, 256 tiles at a time; of 16 tokens 1.75 a workgroup a CU, 2.6 two.
 constexpr float kHalfStart2 = 3.8f, kHalfStart1 = 3.2f, kHalfTile = 1.6f, kHalfRound2 = 2.1f, kHalfRound1[2] = {1.75f, 2.6f};
 // Which of them, by the rounds that the chip takes the launch's workgroups in.  (Shapes, us for the tiles taken and for 64 or 128
-// rows x 128 tokens: Q6_K 2560 x 9728 on 256 tokens 54 and 89, on 512 81 and 90; Q4_K 2560 x 4096 on 256 25 and 33; 19456 x 2560 on 32
-// 17.6 and 31, on 192 35 and 48; 9728 x 2560 on 64 17.2 and 22.)
+// rows x 128 tokens: Q6_K 2560 x 9728 on 256 tokens 48 and 89, on 512 71 and 90; Q4_K 2560 x 4096 on 256 22 and 33; 19456 x 2560 on 32
+// 16.8 and 31, on 192 37 and 48.)
 template <int FSET>
 int reg_tile_of(const BfParams& p) {
   const int f = FSET == ILT_Q4_K ? 0 : 1, nsb = p.cols / 256;
@@ -1333,12 +1519,12 @@ int reg_tile_of(const BfParams& p) {
   };
   int best = 0;
   float least = 0.0f;
-  for (int v = 0; v < 5; v++) {
+  for (int v = 0; v < 8; v++) {
     const RegTile& c = kRegTiles[v];
     const int fit = v == 0 && f ? 4 : c.fit;
     const long long n = workgroups(c.rows, c.tokens), round = 256LL * fit, rest = n % round;
     const float us = kRegStart + (float)nsb * ((float)(n / round) * c.us[f][fit - 1] + (rest ? c.us[f][(rest + 255) / 256 - 1] : 0.0f));
-    if (v == 0 || us < least) { best = v; least = us; }
+    if (v == 0 || us < least) { best = kTileOf[v]; least = us; }
   }
   const long long n = workgroups(32, 32), rest = n % 512;
   const float rounds = (float)((nsb + KS - 1) / KS);
@@ -1363,7 +1549,7 @@ hipError_t dispatch_i8r(BfParams& p, int forced, hipStream_t st) {
     const bool big = forced ? forced == 128 : (long long)((p.mrows[0] + 127) / 128) * ((p.ntok + 127) / 128) >= 150;
     return big ? launch_i8r<FSET, 4, 4, 1>(p, st) : launch_i8r<FSET, 2, 2, 2>(p, st);
   } else {
-    switch (forced == 128 ? 4 : forced == 64 ? 3 : forced >= 1 && forced <= 9 ? forced - 1 : reg_tile_of<FSET>(p)) {
+    switch (forced == 128 ? 4 : forced == 64 ? 3 : forced >= 1 && forced <= 12 ? forced - 1 : reg_tile_of<FSET>(p)) {
       case 0: return launch_i8r<FSET, 1, 1, 1>(p, st);
       case 1: return launch_i8r<FSET, 2, 1, 1>(p, st);
       case 2: return launch_i8r<FSET, 2, 2, 1>(p, st);
@@ -1372,6 +1558,9 @@ hipError_t dispatch_i8r(BfParams& p, int forced, hipStream_t st) {
       case 6: return launch_i8s<FSET, true>(p, st);
       case 7: return launch_i8h<FSET, 2>(p, st);
       case 8: return launch_i8h<FSET, 1>(p, st);
+      case 9: return launch_i8w<FSET, 1>(p, st);
+      case 10: return launch_i8w<FSET, 2>(p, st);
+      case 11: return launch_i8w<FSET, 4>(p, st);
       default: return launch_i8r<FSET, 4, 4, 1>(p, st);
     }
   }
@@ -1385,7 +1574,8 @@ constexpr int block_bytes_of(int fmt) {
 
 // Up to three matrices (Q4_K, Q6_K in any mix, or all Q2_K, or all IQ2_XXS) on the same tokens in one launch, their row tiles one after another.
 // hipErrorNotSupported, and nothing launched, where the shapes are not this kernel's.  ILT_I8_TM (tests): 64 or 128 rows by 128 tokens
-// whatever the shape, 1 to 5 the tiles in kRegTiles' order, 6 and 7 the two kernels for few tiles, 8 and 9 the tiles of 16 rows, 32 and 16 tokens.
+// whatever the shape, 1 to 5 the tiles in kRegTiles' order, 6 and 7 the two kernels for few tiles, 8 and 9 the tiles of 16 rows, 32 and 16
+// tokens, 10 to 12 those of four waves of 16 rows.
 hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws, const int* rows, float* const* ys, const float* const* biases,
                              int cols, const int8_t* xq, const float* xd, const int* bsums, int ntok, int acc, hipStream_t st, long long ldy) {
   if (nmat < 1 || nmat > 3 || ntok < 1 || cols < 256 || cols % 256 != 0 || cols >= (1 << 22)) return hipErrorNotSupported;

@@ -78,8 +78,17 @@ def test_super_blocks_shared_out_over_eight_waves_bit_for_bit(dev, monkeypatch, 
     test_operands_in_registers_bit_for_bit(dev, monkeypatch, tile, qtype, rows, cols, n)
 
 
+# four waves of 16 rows on the same tokens, 16, 32 and 64 of them: fewer blocks than buffers, rows and tokens around the tiles
+@pytest.mark.parametrize("tile", ["10", "11", "12"])
+@pytest.mark.parametrize("qtype,rows,cols,n", [
+    (synth.Q4_K, 1, 256, 2), (synth.Q4_K, 63, 512, 33), (synth.Q4_K, 65, 768, 16), (synth.Q4_K, 300, 2560, 65),
+    (synth.Q6_K, 15, 256, 31), (synth.Q6_K, 64, 512, 17), (synth.Q6_K, 129, 1024, 64), (synth.Q6_K, 200, 2816, 130)])
+def test_sixteen_rows_a_wave_bit_for_bit(dev, monkeypatch, tile, qtype, rows, cols, n):
+    test_operands_in_registers_bit_for_bit(dev, monkeypatch, tile, qtype, rows, cols, n)
+
+
 # Q, K and V of mixed formats in one launch of such tiles, against the products for few tokens
-@pytest.mark.parametrize("tile", ["6", "7", "8", "9"])
+@pytest.mark.parametrize("tile", ["6", "7", "8", "9", "10", "11", "12"])
 def test_mixed_formats_with_super_blocks_shared_out(dev, monkeypatch, tile):
     from illatio_amd import hip, model
     host = model.synth_model(12, d=768, ffn=1024, nh=12, nkv=4, hd=64, nl=2, vocab=700)
