@@ -261,6 +261,8 @@ hipError_t ilt_k_attn_rows(const float* q, const float* kc, const float* vc, flo
 bool ilt_k_attn_mm_takes(const float* q, const float* kc, const float* scratch, const float* out, int nh, int nkv, int hd, int ctx);
 hipError_t ilt_k_attn_scores_mm(const float* q, const float* kc, float* raw, int nh, int nkv, int hd, int pos0, int ntok, float scale, int spitch,
                                 hipStream_t st);
+hipError_t ilt_k_attn_short_mm(const float* q, const float* kc, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, float scale,
+                               const IltRowsQuant* to, hipStream_t st);
 bool ilt_k_attn_mm_quantizes(int kind, int nh, int nkv, int hd);
 hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, int spitch, const IltRowsQuant* to,
                                 hipStream_t st);

@@ -16,6 +16,7 @@
 #include "ilt_act_blocks.h"
 #include "ilt_device.h"
 #include "ilt_kernels.h"
+#include "ilt_softmax.h"
 #include "ilt_value_sets.h"
 #include <type_traits>
 
@@ -25,6 +26,8 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ float part(const float4& v, int e) { return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w; }
+
+constexpr int kShortMost = 448;        // positions of attn_short_mm_kernel
 
 // raw[(t * nh + h) * spitch + p] = F32-DOT16(K[p], q) * scale.  A wave takes 16 rows and, one after another, npt tiles of 16
 // positions.  Block m of the instruction has columns 4m + e of every sixteen, so its results are the running sums e, 4 + e,
@@ -113,18 +116,18 @@ __global__ __launch_bounds__(256, QL ? 4 : 3) void attn_scores_mm_kernel(const f
   }
 }
 
-// A workgroup's ROWS x HD results, rows from rb on, in LDS (HD + 4 floats a row) to the blocks of the output product's activations: a
+// A workgroup's NTILE x HD results, rows from rb on, in LDS (HD + 4 floats a row) to the blocks of the output product's activations: a
 // launch and the results' way to memory and back less, 2.5 us a layer of 97 at 21 tokens of the Qwen3-4B shape, 4 of 440 at 700.
 struct RowsQuant { i8* q; float* d; int* sums; int kind; };      // kind: ILT_ROWS_Q8 or ILT_ROWS_Q8K
-template <int HD, int ROWS>
-__device__ __forceinline__ void rows_to_blocks(const float* tile, const RowsQuant& o, int rb, int rows, int nh, int group, int kvh, int wave, int lane) {
+template <int HD, int NW>      // (NW: the workgroup's waves)
+__device__ __forceinline__ void rows_to_blocks(const float* tile, int ntile, const RowsQuant& o, int rb, int rows, int nh, int group, int kvh, int wave, int lane) {
   __syncthreads();
-  for (int c = wave; c < ROWS * HD / 256; c += 4) {
+  for (int c = wave; c < (ntile * HD + 255) / 256; c += NW) {
     const int at = 256 * c + 4 * lane, r = at / HD, row = rb + r, t = row / group;
-    const float4 f = *(const float4*)(tile + r * (HD + 4) + at % HD);
+    const float4 f = *(const float4*)(tile + min(r, ntile - 1) * (HD + 4) + at % HD);
     const float v[4] = {f.x, f.y, f.z, f.w};
     const long long p = ((long long)t * nh + kvh * group + row - t * group) * HD + at % HD;
-    const bool live = row < rows;
+    const bool live = r < ntile && row < rows;
     int q[4];
     if (o.kind == ILT_ROWS_Q8K) {
       const float d = q8k_block(v, lane, q);
@@ -246,7 +249,7 @@ __global__ __launch_bounds__(256, R == 16 ? 4 : 2) void attn_values_mm_kernel(co
 #pragma unroll
       for (int b = 0; b < 4; b++) *(v4f*)(mine + (lane & 15) * (HD + 4) + 16 * b + 4 * (lane >> 4)) = v4f{acc[4 * b], acc[4 * b + 1], acc[4 * b + 2], acc[4 * b + 3]};
     }
-    rows_to_blocks<HD, WR * R>(tile, quant, rb, rows, nh, group, kvh, wave, lane);
+    rows_to_blocks<HD, 4>(tile, WR * R, quant, rb, rows, nh, group, kvh, wave, lane);
     return;
   }
   auto row_out = [&](int row) { return out + ((long long)(row / group) * nh + kvh * group + row % group) * HD + 64 * cg; };
@@ -285,19 +288,10 @@ __device__ __forceinline__ void across(float* v) {
 template <int K> __device__ __forceinline__ float times_score(float s, float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x150 + K, 0xF, 0xF, true)) * v;      // row_newbcast:K
 }
-template <int HD, int AHEAD, bool QUANT>
-__global__ __launch_bounds__(256) void attn_values_mm_row_kernel(const float* __restrict__ prob, const float* __restrict__ vc, float* __restrict__ out,
-                                                              int nh, int group, int kvd, int pos0, int ntok, int spitch, RowsQuant quant) {
-  constexpr int CG = HD / 64, P = 16;
-  const int kvh = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int rb = ((int)gridDim.y - 1 - (int)blockIdx.y) * (4 / CG), cg = wave % CG;
-  int row = rb + wave / CG;
-  if (row >= ntok * group) {
-    if constexpr (!QUANT) return;
-    row = ntok * group - 1;                          // (again, for nobody)
-  }
-  const int t = row / group, h = kvh * group + row - t * group, npos = pos0 + t + 1;
-  const __amdgpu_buffer_rsrc_t rs = ilt_rsrc(ilt_uniform_ptr(prob + ((long long)t * nh + h) * spitch), (u32)npos * 4u);
+// columns 64 cg + 4 (lane & 15) + (lane >> 4) of a row that sees npos positions; scores(base): those of positions base + (lane & 15)
+template <int HD, int AHEAD, class Scores>
+__device__ __forceinline__ float row_values(Scores scores, const float* vc, int kvd, int kvh, int cg, int npos, int lane) {
+  constexpr int P = 16;
   const __amdgpu_buffer_rsrc_t rv = ilt_rsrc(ilt_uniform_ptr(vc), (u32)npos * (u32)kvd * 4u);
   const int col = 64 * cg + 4 * (lane & 15);
   u32 vo[P / 4];                                     // the lane's position of each four
@@ -306,7 +300,7 @@ __global__ __launch_bounds__(256) void attn_values_mm_row_kernel(const float* __
   struct Set { float s, v[P]; };
   auto load = [&](Set& x, int p) {
     const u32 base = (u32)ilt_set_base(p, P, npos), bv = base * (u32)kvd * 4u;
-    x.s = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, 4u * (base + (u32)(lane & 15)), 0, 0));
+    x.s = scores(base);
 #pragma unroll
     for (int k = 0; k < P; k += 4) {
       const float4 f = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rv, vo[k / 4] + bv, 0, 0));
@@ -333,13 +327,111 @@ __global__ __launch_bounds__(256) void attn_values_mm_row_kernel(const float* __
   };
   Set x[AHEAD];
   ilt_value_sets<P, AHEAD>(x, npos, npos, load, [&](Set& x, int p) { set(x, p, std::false_type{}); }, [&](Set& x, int p) { set(x, p, std::true_type{}); });
+  return acc;                                        // (the exchange leaves column 4 c + g of sixteen c in lane 16 g + c)
+}
+template <int HD, int AHEAD, bool QUANT>
+__global__ __launch_bounds__(256) void attn_values_mm_row_kernel(const float* __restrict__ prob, const float* __restrict__ vc, float* __restrict__ out,
+                                                              int nh, int group, int kvd, int pos0, int ntok, int spitch, RowsQuant quant) {
+  constexpr int CG = HD / 64;
+  const int kvh = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rb = ((int)gridDim.y - 1 - (int)blockIdx.y) * (4 / CG), cg = wave % CG;
+  int row = rb + wave / CG;
+  if (row >= ntok * group) {
+    if constexpr (!QUANT) return;
+    row = ntok * group - 1;                          // (again, for nobody)
+  }
+  const int t = row / group, h = kvh * group + row - t * group, npos = pos0 + t + 1;
+  const __amdgpu_buffer_rsrc_t rs = ilt_rsrc(ilt_uniform_ptr(prob + ((long long)t * nh + h) * spitch), (u32)npos * 4u);
+  const int col = 64 * cg + 4 * (lane & 15) + (lane >> 4);
+  const float acc = row_values<HD, AHEAD>([&](u32 base) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, 4u * (base + (u32)(lane & 15)), 0, 0)); },
+                                          vc, kvd, kvh, cg, npos, lane);
   if constexpr (QUANT) {
     __shared__ __align__(16) float tile[4 / CG * (HD + 4)];
-    tile[wave / CG * (HD + 4) + col + (lane >> 4)] = acc;
-    rows_to_blocks<HD, 4 / CG>(tile, quant, rb, ntok * group, nh, group, kvh, wave, lane);
+    tile[wave / CG * (HD + 4) + col] = acc;
+    rows_to_blocks<HD, 4>(tile, 4 / CG, quant, rb, ntok * group, nh, group, kvh, wave, lane);
     return;
   }
-  out[((long long)t * nh + h) * HD + col + (lane >> 4)] = acc;      // (the exchange leaves column 4 c + g of sixteen c in lane 16 g + c)
+  out[((long long)t * nh + h) * HD + col] = acc;
+}
+
+// All of it in one launch where a chunk is short: a workgroup a KV head and token, its rows the heads of the group.  Scores with four
+// lanes a position (sums 4 m + e of F32-DOT16 in lane m), 16 positions a wave at a time, into LDS; a wave a row's softmax; the values a row
+// and 64 columns a wave as above.  Three launches of few workgroups are mostly their own starts and ends, 3 us each; what is left is 10 us
+// for scores and values of 300 positions on eight waves, instructions for the most part (keys or values through LDS, the next keys asked
+// for first, two rows a wave, two waves a row's softmax: none changed it by 5 %).  us for the three and for this: 21 tokens at none 11.3 and 5.6, at
+// 300 19.6 and 15.5, at 900 36.6 and 32.4, 8 at 900 25.4 and 30.4 (32 heads of 128 over 8); 14 of 64 over 2, 48 at none 10.3 and 6.4.
+template <int HD, bool QUANT>
+__global__ __launch_bounds__(512) void attn_short_mm_kernel(const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc, float* __restrict__ out,
+                                                         int nh, int group, int kvd, int pos0, int ntok, float scale, int pitch, RowsQuant quant) {
+  constexpr int CG = HD / 64, NJ = HD / 16, NW = 8;
+  extern __shared__ __align__(16) float sc[];        // group rows of pitch scores, then of HD + 4 results
+  const int kvh = blockIdx.x, t = (int)gridDim.y - 1 - (int)blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int npos = pos0 + t + 1, m = lane & 3, pl = lane >> 2;
+  const float* const kb = kc + (long long)kvh * HD + 4 * m;
+  for (int rb = 0; rb < group; rb += 4) {
+    float4 qa[4][NJ];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float* const qr = q + ((long long)t * nh + kvh * group + min(rb + i, group - 1)) * HD + 4 * m;
+#pragma unroll
+      for (int j = 0; j < NJ; j++) qa[i][j] = *(const float4*)(qr + 16 * j);
+    }
+    for (int p0 = 16 * wave; p0 < npos; p0 += 16 * NW) {
+      const float* const kr = kb + (long long)min(p0 + pl, npos - 1) * kvd;
+      float4 ka[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; j++) ka[j] = *(const float4*)(kr + 16 * j);
+      float x[4][4];
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float d = part(qa[i][j], e) * part(ka[j], e);
+            x[i][e] = j ? x[i][e] + d : d;
+          }
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          x[i][e] = x[i][e] + ilt_dppf<ILT_DPP_XOR1>(x[i][e]);
+          x[i][e] = x[i][e] + ilt_dppf<ILT_DPP_XOR2>(x[i][e]);
+        }
+        const float v = ((x[i][0] + x[i][1]) + (x[i][2] + x[i][3])) * scale;
+        if (m == 0 && rb + i < group && p0 + pl < npos) sc[(rb + i) * pitch + p0 + pl] = v;
+      }
+    }
+  }
+  __syncthreads();
+  for (int row = wave; row < group; row += NW) {     // (a wave's own row: nobody else's until the barrier)
+    float* const w = sc + row * pitch;
+    float mx = -3.402823466e38f;
+    for (int p = lane; p < npos; p += 64) mx = fmaxf(mx, w[p]);
+    mx = wave_max_float(mx);
+    double sum = 0.0;
+    for (int p = lane; p < npos; p += 64) { const float e = ilt_expf_via_double(w[p] - mx); w[p] = e; sum += (double)e; }
+    sum = wave_sum_double(sum);
+    float inv;
+    if (!recip_settled<sum_adds(kShortMost / 64, 0)>(sum, npos, &inv)) {      // the same in every lane
+      wave_lds_sync();
+      sum = 0.0;
+      for (int p = 0; p < npos; p++) sum += (double)w[p];
+      inv = (float)(1.0 / sum);
+    }
+    wave_lds_sync();
+    for (int p = lane; p < npos; p += 64) w[p] = w[p] * inv;
+  }
+  __syncthreads();
+  float* const tile = sc + group * pitch;
+  for (int pr = wave; pr < group * CG; pr += NW) {
+    const int row = pr / CG, cg = pr % CG, col = 64 * cg + 4 * (lane & 15) + (lane >> 4);
+    const float* const pw = sc + row * pitch + (lane & 15);
+    const float acc = row_values<HD, 3>([&](u32 base) { return pw[base]; }, vc, kvd, kvh, cg, npos, lane);
+    if constexpr (QUANT) tile[row * (HD + 4) + col] = acc;
+    else out[((long long)t * nh + kvh * group + row) * HD + col] = acc;
+  }
+  if constexpr (QUANT) rows_to_blocks<HD, NW>(tile, group, quant, t * group, ntok * group, nh, group, kvh, wave, lane);
 }
 
 }  // namespace
@@ -347,6 +439,25 @@ __global__ __launch_bounds__(256) void attn_values_mm_row_kernel(const float* __
 bool ilt_k_attn_mm_takes(const float* q, const float* kc, const float* scratch, const float* out, int nh, int nkv, int hd, int ctx) {
   return (hd == 64 || hd == 128) && ((((uintptr_t)q) | ((uintptr_t)kc) | ((uintptr_t)scratch) | ((uintptr_t)out)) & 15) == 0 &&      // 16-byte loads and stores of them
          (long long)ctx * nkv * hd < (1LL << 30) && 17LL * nh * (ctx + 3) < (1LL << 30);                         // 32-bit offsets: the values, a tile's rows
+}
+
+// hipErrorNotSupported, and nothing launched, where three launches are better: more workgroups than CUs, positions that a few workgroups are
+// long over (whole prompts, one launch's gain: the Qwen3-4B shape, 2 tokens at 16 positions 6.5 %, at 128 2.6, at 300 -0.2; 21 at 300 4.0, at 400 2.1; 40
+// at 128, 320 workgroups, -3.5; the Qwen2.5-0.5B one, 8 at 64 6.5, at 200 1.9; 128 at 200 4.0), groups of fewer than three heads (scores are made
+// for four at a time).
+hipError_t ilt_k_attn_short_mm(const float* q, const float* kc, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, float scale,
+                               const IltRowsQuant* to, hipStream_t st) {
+  const int group = nh / nkv, ctx = pos0 + ntok, pitch = (ctx + 15) & ~15;
+  const long long wgs = (long long)ntok * nkv;
+  if (group < 3 || group > 8 || wgs > 256 || ctx > (wgs >= 128 ? kShortMost : 256)) return hipErrorNotSupported;
+  const RowsQuant quant = to ? RowsQuant{to->q, to->d, to->sums, to->kind} : RowsQuant{};
+  const dim3 grid(nkv, ntok);
+  const size_t smem = sizeof(float) * group * (pitch + hd + 4);
+#define ILT_SHORT(HD, QUANT) hipLaunchKernelGGL((attn_short_mm_kernel<HD, QUANT>), grid, dim3(512), smem, st, q, kc, vc, out, nh, group, nkv * hd, pos0, ntok, scale, pitch, quant)
+  if (hd == 128) { if (to) ILT_SHORT(128, true); else ILT_SHORT(128, false); }
+  else { if (to) ILT_SHORT(64, true); else ILT_SHORT(64, false); }
+#undef ILT_SHORT
+  return hipGetLastError();
 }
 
 // Blocks of 32 lie within a row; blocks of 256 are rows of one token and start where a tile's rows do where a group's columns are whole blocks.

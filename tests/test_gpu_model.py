@@ -488,6 +488,13 @@ def test_chunk_attention_whose_scores_pair_row_tiles(dev, nh, nkv, hd, pos0, nto
     test_chunk_attention_with_the_matrix_cores_products(dev, nh, nkv, hd, pos0, ntok, what)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,pos0,ntok,what", [(3, 1, 64, 0, 2, "nan"), (12, 4, 128, 61, 3, "denormal"), (40, 5, 128, 15, 49, "nan"), (15, 3, 64, 63, 2, "odd"),
+                                                      (24, 4, 64, 412, 36, "nan"), (7, 1, 128, 192, 64, ""), (8, 2, 128, 239, 18, "denormal")])      # the last: one past what one launch takes
+def test_chunk_attention_in_one_launch(dev, nh, nkv, hd, pos0, ntok, what):
+    """The same for a chunk's attention in one launch: groups of 3 to 8 heads, positions around the 16 of a wave and the 128 of a workgroup."""
+    test_chunk_attention_with_the_matrix_cores_products(dev, nh, nkv, hd, pos0, ntok, what)
+
+
 @pytest.mark.parametrize("nh,pos0,ntok", [(2, 60, 3), (2, 1020, 4), (8, 1100, 130), (8, 2100, 130), (2, 2100, 5), (1, 8000, 192)])
 def test_chunk_softmax_where_the_order_of_the_sum_shows(dev, nh, pos0, ntok):
     """A chunk whose exponentials' sum lies on the edge between two singles for its reciprocal, so that the softmax kernels (a wave
@@ -524,9 +531,10 @@ def test_chunk_softmax_where_the_order_of_the_sum_shows(dev, nh, pos0, ntok):
         hip.hip_free(b)
 
 
-@pytest.mark.parametrize("q8,nh,nkv,hd,n", [(False, 8, 2, 128, 2), (False, 8, 2, 128, 85), (False, 6, 3, 128, 177), (False, 8, 2, 64, 351), (False, 16, 8, 128, 819),      # whole blocks: a row a wave, the last of its kind, four rows, sixteen
-                                            (False, 6, 2, 128, 9), (False, 4, 2, 64, 5),                                                   # groups of one and a half blocks and of half a block
-                                            (True, 14, 2, 64, 3), (True, 3, 1, 128, 234), (True, 14, 2, 64, 201), (True, 14, 14, 64, 1833)])
+@pytest.mark.parametrize("q8,nh,nkv,hd,n", [(False, 8, 2, 128, 2), (False, 8, 2, 128, 85), (False, 16, 2, 64, 61),             # one launch
+                                            (False, 4, 2, 128, 97), (False, 6, 3, 128, 177), (False, 8, 2, 64, 351), (False, 16, 8, 128, 819),      # a row a wave, four rows, sixteen
+                                            (False, 6, 2, 128, 9), (False, 4, 2, 64, 5),                                    # groups of one and a half blocks and of half a block
+                                            (True, 14, 2, 64, 3), (True, 3, 1, 128, 234), (True, 2, 1, 64, 77), (True, 14, 2, 64, 201), (True, 14, 14, 64, 1833)])
 def test_chunk_attention_leaves_its_rows_quantized(dev, monkeypatch, q8, nh, nkv, hd, n):
     """A chunk whose attention leaves the output product's activations in blocks, against the other attention kernels and the
     quantizing launch behind them: logits, and the next layer's keys and values of every token, bit for bit."""
