@@ -59,7 +59,7 @@ def test_operands_in_registers_bit_for_bit(dev, monkeypatch, rows_a_tile, qtype,
     m.free()
 
 
-# the super-blocks shared out over two and four waves: fewer of them than waves, a last round that is not whole, whole rounds; rows and
+# the super-blocks shared out over four waves, a workgroup and two a CU: fewer of them than waves, a last round that is not whole, whole rounds; rows and
 # tokens around tiles of 32 and 64
 @pytest.mark.parametrize("tile", ["6", "7"])
 @pytest.mark.parametrize("qtype,rows,cols,n", [
