@@ -444,12 +444,15 @@ bool ilt_k_attn_mm_takes(const float* q, const float* kc, const float* scratch, 
 // hipErrorNotSupported, and nothing launched, where three launches are better: more workgroups than CUs, positions that a few workgroups are
 // long over (whole prompts, one launch's gain: the Qwen3-4B shape, 2 tokens at 16 positions 6.5 %, at 128 2.6, at 300 -0.2; 21 at 300 4.0, at 400 2.1; 40
 // at 128, 320 workgroups, -3.5; the Qwen2.5-0.5B one, 8 at 64 6.5, at 200 1.9; 128 at 200 4.0), groups of fewer than three heads (scores are made
-// for four at a time).
+// for four at a time).  Five heads of 128 and more are two rounds of the eight waves' values and of the scores, and over after a third of those
+// positions (us for one launch and for three, on 8 workgroups: five heads at 96 positions 10.2 and 10.3, at 104 12.2 and 10.4, at 200 16.0 and 11.8; eight at
+// 64 10.0 and 10.3, at 72 11.1 and 10.3, at 200 18.4 and 11.8; on 128 eight heads at 94 11.9 and 12.8, at 102 13.8 and 13.3; on 240 at 108 13.7 and 13.8).
 hipError_t ilt_k_attn_short_mm(const float* q, const float* kc, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, float scale,
                                const IltRowsQuant* to, hipStream_t st) {
   const int group = nh / nkv, ctx = pos0 + ntok, pitch = (ctx + 15) & ~15;
   const long long wgs = (long long)ntok * nkv;
-  if (group < 3 || group > 8 || wgs > 256 || ctx > (wgs >= 128 ? kShortMost : 256)) return hipErrorNotSupported;
+  const int most = group * hd > 8 * 64 ? (wgs >= 128 || group <= 6 ? 96 : 64) : wgs >= 128 ? kShortMost : 256;
+  if (group < 3 || group > 8 || wgs > 256 || ctx > most) return hipErrorNotSupported;
   const RowsQuant quant = to ? RowsQuant{to->q, to->d, to->sums, to->kind} : RowsQuant{};
   const dim3 grid(nkv, ntok);
   const size_t smem = sizeof(float) * group * (pitch + hd + 4);

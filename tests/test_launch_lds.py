@@ -107,3 +107,23 @@ def test_which_kernels_a_chunks_attention_takes(tmp_path):
     assert names(launched(tmp_path, "QUERY = 0" + CHUNKS, ILT_ATTN_MM="0")) == {"attn_scores_kernel", "attn_values_chunk"}
     assert names(launched(tmp_path, "QUERY = 4" + CHUNKS)) == {"attn_scores_kernel", "attn_values_chunk"}
     assert names(launched(tmp_path, "QUERY = 0" + CHUNKS, ILT_ATTN_CHUNK="0")) == {"attn_scores_kernel", "attn_values_kernel", "attn_values_tiled"}
+
+
+SHORT = r"""
+import ctypes as C, sys
+C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+L = C.CDLL(sys.argv[2])
+P, I = C.c_uint64(1 << 40), C.c_int
+for nh, nkv, hd, pos, n in %s:
+    print("at", nh, nkv, hd, pos, n, flush=True)
+    assert L.ilt_attn_rows(C.c_uint64(0), P, P, P, P, I(nh), I(nkv), I(hd), I(pos), I(n), P) == 0
+"""
+
+
+def test_one_launch_of_two_rounds_of_values_only_for_few_positions(tmp_path):
+    """Groups of more heads than a round of attn_short_mm_kernel's waves takes the values of: one launch up to 96 or 64 positions."""
+    one = [(20, 4, 128, 94, 2), (24, 4, 128, 88, 8), (28, 4, 128, 62, 2), (32, 4, 128, 48, 16), (28, 4, 128, 64, 32), (64, 8, 128, 64, 32), (16, 4, 128, 254, 2), (32, 4, 64, 254, 2)]
+    three = [(20, 4, 128, 95, 2), (24, 4, 128, 200, 8), (28, 4, 128, 63, 2), (32, 4, 128, 49, 16), (28, 4, 128, 65, 32), (64, 8, 128, 65, 32), (16, 4, 128, 255, 2), (32, 4, 64, 255, 2)]
+    lines = launched(tmp_path, SHORT % (one + three))
+    taken = " ".join("1" if "attn_short_mm" in x else "0" if "attn_scores_mm" in x else "" for x in lines).split()
+    assert taken == ["1"] * len(one) + ["0"] * len(three)
