@@ -200,7 +200,10 @@ hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws
                              const float* const* biases, int cols, const int8_t* xq, const float* xs, const int* bsums, int ntok, int acc,
                              hipStream_t st, long long ldy = 0);
 // Q4_K and Q6_K in any mix, or Q2_K or IQ2_XXS (up to three matrices), exact, the weights made in the operand registers (kernels_gemm_reg.hip);
-// hipErrorNotSupported, and nothing launched, where the shapes are not that kernel's
+// hipErrorNotSupported, and nothing launched, where the shapes are not that kernel's: rows and a result's pitch from ILT_REG_ROWS on,
+// columns from ILT_REG_COLS on among them (32-bit offsets)
+#define ILT_REG_ROWS (1 << 21)
+#define ILT_REG_COLS (1 << 22)
 hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws, const int* rows, float* const* ys, const float* const* biases,
                              int cols, const int8_t* xq, const float* xd, const int* bsums, int ntok, int acc, hipStream_t st, long long ldy = 0);
 // The exact product in two passes (Q6_K): the two int8 planes and d per row and super-block once, then the product from them

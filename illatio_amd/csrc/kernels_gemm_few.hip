@@ -466,6 +466,7 @@ hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws
   int fset = fmts[0];
   long long tiles32 = 0, tiles16 = 0;
   bool small = false;                       // a matrix of less than a tile of the registers' kernel
+  bool reg = nmat <= 3 && (nmat == 1 || !ldy) && cols < ILT_REG_COLS;      // what that kernel takes at all
   for (int i = 0; i < nmat; i++) {
     const int fm = fmts[i];
     if (fm != ILT_Q4_K && fm != ILT_Q6_K && fm != ILT_Q8_0) return hipErrorNotSupported;
@@ -479,6 +480,7 @@ hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws
     tiles32 += (rows[i] + 31) / 32;
     tiles16 += (rows[i] + 15) / 16;
     small |= rows[i] < 128;
+    reg &= rows[i] < ILT_REG_ROWS && m.ldy < ILT_REG_ROWS;
   }
   tiles32 *= (ntok + 31) / 32;
   if (tiles32 > 0x3FFFFFFF) return hipErrorNotSupported;
@@ -487,7 +489,7 @@ hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws
       const hipError_t e = ilt_k_gemm_q8(nmat, ws, wds, rows, ys, biases, cols, xq, xs, ntok, acc, st, ldy);
       if (e != hipErrorNotSupported) return e;
     }
-  } else if (forced < 0 && ((!small && ntok > 16 && tiles32 > 128) || (nmat <= 3 && (nmat == 1 || !ldy) && halves_take(fset != ILT_Q6_K, tiles16, ntok, cols / 256))))
+  } else if (forced < 0 && ((!small && ntok > 16 && tiles32 > 128) || (reg && halves_take(fset != ILT_Q6_K, tiles16, ntok, cols / 256))))
     return hipErrorNotSupported;
   switch (fset) {
     case ILT_Q8_0: return few_dispatch<ILT_Q8_0>(p, forced, st);

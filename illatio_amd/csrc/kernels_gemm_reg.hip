@@ -1578,7 +1578,7 @@ constexpr int block_bytes_of(int fmt) {
 // tokens, 10 to 12 those of four waves of 16 rows.
 hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws, const int* rows, float* const* ys, const float* const* biases,
                              int cols, const int8_t* xq, const float* xd, const int* bsums, int ntok, int acc, hipStream_t st, long long ldy) {
-  if (nmat < 1 || nmat > 3 || ntok < 1 || cols < 256 || cols % 256 != 0 || cols >= (1 << 22)) return hipErrorNotSupported;
+  if (nmat < 1 || nmat > 3 || ntok < 1 || cols < 256 || cols % 256 != 0 || cols >= ILT_REG_COLS) return hipErrorNotSupported;
   BfParams p = {};
   long long tiles128 = 0;
   int fset = fmts[0];
@@ -1587,12 +1587,12 @@ hipError_t ilt_k_gemm_i8_reg(int nmat, const int* fmts, const uint8_t* const* ws
     if (fmts[m] != ILT_Q4_K && fmts[m] != ILT_Q6_K && !two) return hipErrorNotSupported;
     if (fmts[m] != fset) { if (two || fset == ILT_Q2_K || fset == ILT_IQ2_XXS) return hipErrorNotSupported; fset = 0; }
     const long long bytes = (long long)rows[m] * (cols / 256) * block_bytes_of(fmts[m]);
-    if (rows[m] < 1 || bytes >= 0x7FFFFFFFLL || (((uintptr_t)ws[m]) & (fmts[m] == ILT_IQ2_XXS ? 1 : 3)) || rows[m] >= (1 << 21)) return hipErrorNotSupported;      // 32-bit offsets
+    if (rows[m] < 1 || bytes >= 0x7FFFFFFFLL || (((uintptr_t)ws[m]) & (fmts[m] == ILT_IQ2_XXS ? 1 : 3)) || rows[m] >= ILT_REG_ROWS) return hipErrorNotSupported;
     p.mw[m] = ws[m]; p.mrows[m] = rows[m]; p.my[m] = ys[m]; p.mbias[m] = biases ? biases[m] : nullptr; p.mfmt[m] = fmts[m];
     tiles128 += (rows[m] + 127) / 128;
   }
   p.ldy = nmat > 1 || ldy == 0 ? rows[0] : ldy;
-  if (p.ldy < rows[0] || p.ldy >= (1 << 21) || tiles128 * 128 >= (1 << 30)) return hipErrorNotSupported;
+  if (p.ldy < rows[0] || p.ldy >= ILT_REG_ROWS || tiles128 * 128 >= (1 << 30)) return hipErrorNotSupported;
   p.nmulti = nmat; p.cols = cols; p.x = (const u16*)xq; p.xd = xd; p.bsums = bsums; p.acc = acc; p.ntok = ntok;
   const char* force = getenv("ILT_I8_TM");
   const int forced = force ? atoi(force) : 0;

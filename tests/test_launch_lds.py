@@ -127,3 +127,20 @@ def test_one_launch_of_two_rounds_of_values_only_for_few_positions(tmp_path):
     lines = launched(tmp_path, SHORT % (one + three))
     taken = " ".join("1" if "attn_short_mm" in x else "0" if "attn_scores_mm" in x else "" for x in lines).split()
     assert taken == ["1"] * len(one) + ["0"] * len(three)
+
+
+MANY_ROWS = r"""
+import ctypes as C, sys
+C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+L = C.CDLL(sys.argv[2])
+P, Z, I = C.c_uint64(1 << 40), C.c_uint64(0), C.c_int
+for t, rows, cols, n in %s:
+    assert L.ilt_mm_k(C.c_uint64(0), I(t), P, P, P, P, P, Z, I(rows), I(cols), I(n), I(0)) == 0
+"""
+
+
+def test_few_tokens_stay_where_the_other_kernel_takes_not_so_many_rows(tmp_path):
+    """Up to 16 tokens of Q6_K (2) and Q4_K (0) on 2^21 rows, which the kernel with operands in registers refuses, and on one less."""
+    shapes = [(t, (1 << 21) - less, cols, n) for t, cols, n in ((2, 1024, 2), (2, 1024, 16), (0, 256, 12), (0, 1536, 16)) for less in (0, 1)]
+    lines = launched(tmp_path, MANY_ROWS % shapes)
+    assert ["few" if "gemm_i8_few" in x else "reg" if any(k in x for k in ("gemm_i8h", "gemm_i8w", "gemm_i8s", "gemm_i8r")) else x for x in lines] == ["few", "reg"] * 4
