@@ -853,7 +853,8 @@ int ilt_d4_gather_q8k(uint64_t stream, int d, int nrows, const int8_t* xq, const
 }
 
 int ilt_d4_quant_q8k_rows(uint64_t stream, int d, int ntok, int nu, const float* x, const uint32_t* smap, int8_t* xq, float* xd) {
-  ILT_REQUIRE(d > 0 && d % 256 == 0 && ntok >= 0 && nu >= 1 && nu <= 64 && (ntok == 0 || (x && smap && xq && xd)) && ((uintptr_t)xq & 3) == 0);
+  ILT_REQUIRE(d > 0 && d % 256 == 0 && ntok >= 0 && nu >= 1 && nu <= 64 && (ntok == 0 || (x && smap && xq && xd)));
+  ILT_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)xq & 3) == 0);      // 16-byte loads, 4-byte stores
   return (int)ilt_k_quant_q8k_rows(x, smap, ntok, nu, d, xq, xd, S(stream));
 }
 

@@ -144,3 +144,22 @@ def test_few_tokens_stay_where_the_other_kernel_takes_not_so_many_rows(tmp_path)
     shapes = [(t, (1 << 21) - less, cols, n) for t, cols, n in ((2, 1024, 2), (2, 1024, 16), (0, 256, 12), (0, 1536, 16)) for less in (0, 1)]
     lines = launched(tmp_path, MANY_ROWS % shapes)
     assert ["few" if "gemm_i8_few" in x else "reg" if any(k in x for k in ("gemm_i8h", "gemm_i8w", "gemm_i8s", "gemm_i8r")) else x for x in lines] == ["few", "reg"] * 4
+
+
+QUANT_ROWS = r"""
+import ctypes as C, sys
+C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+L = C.CDLL(sys.argv[2])
+P, I = C.c_uint64(1 << 40), C.c_int
+for x, xq in ((0, 0), (4, 0), (8, 0), (12, 0), (0, 1), (0, 2), (16, 4)):
+    at = lambda off: C.c_uint64((1 << 40) + off)
+    print(x, xq, L.ilt_d4_quant_q8k_rows(C.c_uint64(0), I(512), I(3), I(2), at(x), P, at(xq), P))
+"""
+
+
+def test_quantizing_into_rows_wants_the_addresses_that_its_loads_and_stores_do(tmp_path):
+    """ilt_d4_quant_q8k_rows on floats off 16 bytes or quants off 4: an error and no launch, as ilt_quant_q8k."""
+    lines = launched(tmp_path, QUANT_ROWS)
+    assert sum("quant_q8k_rows" in x for x in lines) == 2
+    codes = [int(x.split()[2]) for x in lines if "quant_q8k_rows" not in x]
+    assert [c == 0 for c in codes] == [True, False, False, False, False, False, True]
