@@ -454,7 +454,7 @@ bool halves_take(bool q4, long long rows16, int ntok, int nsb) {
 // whose waves make a tile's terms and sums in registers: up to 16 tokens here, unless the tiles of 16 rows fill the chip (896 x 4864
 // on 16 tokens 12.7 us against 16.1, on 24 17.1 against 16.1; 4096 x 2048 on 16, 256 tiles: 8.1 against 8.3; 9728 x 896, 608:
 // 7.7 against 5.8); where its smallest tile does not go (cols no multiple of 128) from 640 tiles of 32 x 32 and 96 tokens on.
-// ILT_I8_FEW (tests): "0" never, "1" always, "2", "4", "8" always, that cut.
+// ILT_I8_FEW (tests): "0" never, "1" always, "2", "4" always, that cut, "8" Q8_0's over eight waves (K-quants: "4").
 hipError_t ilt_k_gemm_i8_few(int nmat, const int* fmts, const uint8_t* const* ws, const uint16_t* const* wds, const int* rows, float* const* ys,
                              const float* const* biases, int cols, const int8_t* xq, const float* xs, const int* bsums, int ntok, int acc,
                              hipStream_t st, long long ldy) {

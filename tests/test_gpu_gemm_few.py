@@ -20,11 +20,14 @@ def dev():
 
 # rows around tiles of 16 and 32, tokens around tiles of 16 and 32, columns of fewer units than waves, of a whole and of a
 # broken number of rounds (a round: what LDS holds the terms of), Q8_0 rows that end in half a unit
-@pytest.mark.parametrize("cut", ["2", "4", "8"])
-@pytest.mark.parametrize("qtype,rows,cols,n", [
+SHAPES = [
     (synth.Q4_K, 1, 256, 2), (synth.Q4_K, 33, 2560, 16), (synth.Q4_K, 48, 4608, 17), (synth.Q4_K, 130, 1024, 95),
     (synth.Q6_K, 17, 256, 1), (synth.Q6_K, 32, 2816, 33), (synth.Q6_K, 47, 9728, 32), (synth.Q6_K, 160, 512, 130),
-    (synth.Q8_0, 15, 32, 3), (synth.Q8_0, 64, 896, 31), (synth.Q8_0, 31, 1888, 40), (synth.Q8_0, 16, 4864, 15)])
+    (synth.Q8_0, 15, 32, 3), (synth.Q8_0, 64, 896, 31), (synth.Q8_0, 31, 1888, 40), (synth.Q8_0, 16, 4864, 15)]
+
+
+# (the cut over eight waves: Q8_0's alone)
+@pytest.mark.parametrize("cut,qtype,rows,cols,n", [(cut,) + s for cut in ("2", "4", "8") for s in SHAPES if cut != "8" or s[0] == synth.Q8_0])
 def test_few_tokens_bit_for_bit(dev, monkeypatch, cut, qtype, rows, cols, n):
     from illatio_amd import dense, hip
     monkeypatch.setenv("ILT_I8_FEW", cut)
