@@ -6,7 +6,7 @@
 // result is that product rounded once (denormals and all: compared with v_mul_f32 over 26 million pairs; a product that
 // rounds to -0 stays -0, where 0 + -0 would be +0: no sum here shows it).  A thousand products are one instruction that
 // takes the time of sixteen adds, and its operands are sixteen rows and sixteen columns in one register each, straight from
-// memory: nothing passes through LDS.  The adds are the vector ALU's, a register of sixty-four sums an instruction.  (The
+// memory (the query rows of a long chunk's scores by way of LDS, a read an instruction).  The adds are the vector ALU's, a register of sixty-four sums an instruction.  (The
 // two do not run at the same time on gfx950: an instruction with 16 results and 16 adds beside it take 33-36 ns a SIMD, 15
 // and 17 apart; as mul and add they take 32.  What the matrix cores save is the operands' way: sixteen chains a thread
 // read LDS once a chain and four products.)
@@ -436,6 +436,7 @@ __global__ __launch_bounds__(512) void attn_short_mm_kernel(const float* __restr
 
 }  // namespace
 
+// (The values may lie on any dword: they are read by buffer loads, which want no more, also of 16 bytes.)
 bool ilt_k_attn_mm_takes(const float* q, const float* kc, const float* scratch, const float* out, int nh, int nkv, int hd, int ctx) {
   return (hd == 64 || hd == 128) && ((((uintptr_t)q) | ((uintptr_t)kc) | ((uintptr_t)scratch) | ((uintptr_t)out)) & 15) == 0 &&      // 16-byte loads and stores of them
          (long long)ctx * nkv * hd < (1LL << 30) && 17LL * nh * (ctx + 3) < (1LL << 30);                         // 32-bit offsets: the values, a tile's rows

@@ -482,23 +482,55 @@ def test_chunk_attention_of_one_and_of_four_rows_a_wave(dev, nh, nkv, hd, pos0, 
 
 
 @pytest.mark.parametrize("nh,nkv,hd,pos0,ntok,what", [(4, 4, 128, 0, 65, "nan"), (5, 5, 64, 33, 129, ""), (9, 3, 64, 14, 43, "denormal"),      # a tile of positions a wave; two, three and three sets
-                                                      (4, 4, 128, 37, 705, "nan"), (16, 16, 64, 3, 831, "odd"), (32, 32, 64, 62, 960, "nan")])      # two, four and eight tiles
+                                                      (4, 4, 128, 37, 705, "nan"), (16, 16, 64, 3, 831, "odd"), (32, 32, 64, 62, 960, "nan"),      # two, four and eight tiles
+                                                      (32, 32, 64, 1201, 1201, "")])      # sixteen, from 300,000 tiles on: 367,232 of them, 19 sets
 def test_chunk_attention_whose_scores_pair_row_tiles(dev, nh, nkv, hd, pos0, ntok, what):
     """The same for the scores' sets of row tiles, one from the start and one from the end a column of the grid: even and odd numbers of sets."""
     test_chunk_attention_with_the_matrix_cores_products(dev, nh, nkv, hd, pos0, ntok, what)
 
 
 @pytest.mark.parametrize("nh,nkv,hd,pos0,ntok,what", [(3, 1, 64, 0, 2, "nan"), (12, 4, 128, 61, 3, "denormal"), (40, 5, 128, 15, 49, "nan"), (15, 3, 64, 63, 2, "odd"),
-                                                      (24, 4, 64, 412, 36, "nan"), (7, 1, 128, 192, 64, ""), (8, 2, 128, 239, 18, "denormal")])      # the last: one past what one launch takes
+                                                      (24, 4, 64, 412, 36, "nan"), (7, 1, 128, 0, 64, ""), (24, 3, 128, 40, 44, "nan"), (10, 2, 128, 80, 16, ""),
+                                                      (7, 1, 128, 192, 64, ""), (8, 2, 128, 239, 18, "denormal")])      # the last two: more than one launch takes
 def test_chunk_attention_in_one_launch(dev, nh, nkv, hd, pos0, ntok, what):
-    """The same for a chunk's attention in one launch: groups of 3 to 8 heads, positions around the 16 of a wave and the 128 of a workgroup."""
+    """The same for a chunk's attention in one launch: groups of 3 to 8 heads, positions around the 16 of a wave and the 128 of a workgroup.  (Which
+    shapes take it: tests/test_launch_lds.py.)"""
     test_chunk_attention_with_the_matrix_cores_products(dev, nh, nkv, hd, pos0, ntok, what)
 
 
-@pytest.mark.parametrize("nh,pos0,ntok", [(2, 60, 3), (2, 1020, 4), (8, 1100, 130), (8, 2100, 130), (2, 2100, 5), (1, 8000, 192)])
+# in one launch; values of a row, of four rows and of sixteen a wave; a row a wave on a set of positions that is not whole
+@pytest.mark.parametrize("nh,nkv,hd,pos0,ntok", [(8, 2, 128, 20, 5), (8, 2, 64, 301, 21), (32, 8, 128, 301, 33), (16, 16, 128, 5, 801), (4, 4, 128, 14, 3)])
+def test_chunk_attention_on_values_off_16_bytes(dev, nh, nkv, hd, pos0, ntok):
+    """Cached values on an address that is a multiple of 4 only (their loads are buffer loads, which want whole dwords), against attn_rows' one
+    launch on a copy that lies on 16 bytes, bit for bit."""
+    import ctypes as C
+    from illatio_amd import hip
+    rng = synth.make_rng(2500 + nh + hd + pos0 + ntok)
+    f = lambda n: (rng.standard_normal(n) * 1.5).astype(np.float32)
+    nctx = pos0 + ntok
+    q, kc = hip.hip_upload_new(dev, f(ntok * nh * hd)), hip.hip_upload_new(dev, f(nctx * nkv * hd))
+    vh = f(nctx * nkv * hd)
+    scratch = hip.hip_alloc(dev, 4 * ntok * nh * ((nctx + 3) & ~3))
+    outs = []
+    for off, scr in ((0, 0), (1, scratch.ptr), (3, scratch.ptr)):
+        vc = hip.hip_upload_new(dev, np.concatenate([np.full(off, np.nan, np.float32), vh]))
+        out = hip.hip_upload_new(dev, np.full(ntok * nh * hd, np.nan, np.float32))
+        hip.call("ilt_attn_rows", C.c_uint64(0), C.c_uint64(q.ptr), C.c_uint64(kc.ptr), C.c_uint64(vc.ptr + 4 * off), C.c_uint64(out.ptr), C.c_int(nh), C.c_int(nkv),
+                 C.c_int(hd), C.c_int(pos0), C.c_int(ntok), C.c_uint64(scr))
+        outs.append(hip.hip_floats(out, ntok * nh * hd))
+        hip.hip_free(out)
+        hip.hip_free(vc)
+    assert np.isfinite(outs[0]).all()
+    assert np.array_equal(bits(outs[1]), bits(outs[0])) and np.array_equal(bits(outs[2]), bits(outs[0]))
+    for b in (q, kc, scratch):
+        hip.hip_free(b)
+
+
+@pytest.mark.parametrize("nh,pos0,ntok", [(2, 60, 3), (2, 1020, 4), (8, 1100, 130), (8, 2100, 130), (2, 2100, 5), (1, 8000, 192),
+                                            (3, 60, 3), (8, 200, 50), (4, 300, 130)])      # the softmax of a chunk's attention in one launch
 def test_chunk_softmax_where_the_order_of_the_sum_shows(dev, nh, pos0, ntok):
     """A chunk whose exponentials' sum lies on the edge between two singles for its reciprocal, so that the softmax kernels (a wave
-    a row up to 1,024, 2,048 and 4,096 positions, a workgroup a row) take the CPU's order of adds: against attn_rows' one launch, bit
+    a row up to 1,024, 2,048 and 4,096 positions, a workgroup a row; a wave a row in LDS) take the CPU's order of adds: against attn_rows' one launch, bit
     for bit.  One position's score is 0, the last one's is chosen so that 1 / sum is within the kernels' doubt of 1 - 2^-25."""
     import ctypes as C
     from illatio_amd import hip
@@ -556,14 +588,14 @@ def test_chunk_attention_leaves_its_rows_quantized(dev, monkeypatch, q8, nh, nkv
 
 def test_a_chunk_as_parts_side_by_side(dev):
     """forward_parts -- a chunk's halves or quarters on streams of their own, a part's attention waiting for the earlier
-    parts' keys layer by layer -- leaves forward_n's logits and caches, bit for bit: halves of 128 + 128, of 192 + 108,
-    a second chunk whose halves see the first chunk's positions, and quarters of 128."""
+    parts' keys layer by layer -- leaves forward_n's logits and caches, bit for bit: halves of 128 + 128, of 192 + 108, of
+    128 + 44 and 128 + 12 (the second half on the products for few tokens), a second chunk whose halves see the first chunk's positions, and quarters of 128."""
     from illatio_amd import hip, model
     host = model.synth_model(12, d=512, ffn=1024, nh=8, nkv=2, hd=64, nl=3, vocab=700)
     c = host["config"]
     rng = synth.make_rng(77)
     kvd = c["nkv"] * c["hd"]
-    for nprompt, chunk, k in ((256, 256, 2), (300, 300, 2), (600, 300, 2), (512, 512, 4), (1000, 500, 4), (1000, 1000, 2)):
+    for nprompt, chunk, k in ((256, 256, 2), (300, 300, 2), (172, 172, 2), (140, 140, 2), (600, 300, 2), (512, 512, 4), (1000, 500, 4), (1000, 1000, 2)):
         prompt = rng.integers(0, c["vocab"], nprompt).tolist()
         res = []
         for halves in (True, False):

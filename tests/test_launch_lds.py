@@ -2,6 +2,7 @@
 kernels a chunk's attention takes.  The library's host code runs here on a stand-in for the HIP runtime that notes what it is
 asked for and launches nothing (no GPU)."""
 import os
+import re
 import subprocess
 import sys
 
@@ -100,13 +101,19 @@ for hd in (64, 128):
 """
 
 
+def kernels(lines):
+    """The attention kernels of the launches, and in brackets the template's first number and whether it leaves quantized rows."""
+    found = (re.search(r"\d(attn_[a-z_]+?)_kernel(?:I((?:L[ib]\d+E)+))?", x) for x in lines)
+    return [(m.group(1), m.group(2) or "") for m in found if m]
+
+
 def test_which_kernels_a_chunks_attention_takes(tmp_path):
-    names = lambda lines: {n for n in ("attn_scores_mm", "attn_values_mm", "attn_scores_kernel", "attn_values_chunk", "attn_values_kernel", "attn_values_tiled")
-                           for x in lines if n in x}
-    assert names(launched(tmp_path, "QUERY = 0" + CHUNKS, ILT_ATTN_MM="1")) == {"attn_scores_mm", "attn_values_mm"}
-    assert names(launched(tmp_path, "QUERY = 0" + CHUNKS, ILT_ATTN_MM="0")) == {"attn_scores_kernel", "attn_values_chunk"}
-    assert names(launched(tmp_path, "QUERY = 4" + CHUNKS)) == {"attn_scores_kernel", "attn_values_chunk"}
-    assert names(launched(tmp_path, "QUERY = 0" + CHUNKS, ILT_ATTN_CHUNK="0")) == {"attn_scores_kernel", "attn_values_kernel", "attn_values_tiled"}
+    names = lambda lines: {n for n, _ in kernels(lines)} - {"attn_softmax"}
+    mm = {"attn_short_mm", "attn_scores_mm", "attn_values_mm_row"}
+    assert names(launched(tmp_path, "QUERY = 0" + CHUNKS, ILT_ATTN_MM="1")) == mm
+    assert names(launched(tmp_path, "QUERY = 0" + CHUNKS, ILT_ATTN_MM="0")) == {"attn_scores", "attn_values_chunk"}
+    assert names(launched(tmp_path, "QUERY = 4" + CHUNKS)) == {"attn_scores", "attn_values_chunk"}
+    assert names(launched(tmp_path, "QUERY = 0" + CHUNKS, ILT_ATTN_CHUNK="0")) == {"attn_scores", "attn_values", "attn_values_tiled"}
 
 
 SHORT = r"""
@@ -117,6 +124,7 @@ P, I = C.c_uint64(1 << 40), C.c_int
 for nh, nkv, hd, pos, n in %s:
     print("at", nh, nkv, hd, pos, n, flush=True)
     assert L.ilt_attn_rows(C.c_uint64(0), P, P, P, P, I(nh), I(nkv), I(hd), I(pos), I(n), P) == 0
+    C.CDLL(None).fflush(None)
 """
 
 
@@ -124,9 +132,39 @@ def test_one_launch_of_two_rounds_of_values_only_for_few_positions(tmp_path):
     """Groups of more heads than a round of attn_short_mm_kernel's waves takes the values of: one launch up to 96 or 64 positions."""
     one = [(20, 4, 128, 94, 2), (24, 4, 128, 88, 8), (28, 4, 128, 62, 2), (32, 4, 128, 48, 16), (28, 4, 128, 64, 32), (64, 8, 128, 64, 32), (16, 4, 128, 254, 2), (32, 4, 64, 254, 2)]
     three = [(20, 4, 128, 95, 2), (24, 4, 128, 200, 8), (28, 4, 128, 63, 2), (32, 4, 128, 49, 16), (28, 4, 128, 65, 32), (64, 8, 128, 65, 32), (16, 4, 128, 255, 2), (32, 4, 64, 255, 2)]
-    lines = launched(tmp_path, SHORT % (one + three))
-    taken = " ".join("1" if "attn_short_mm" in x else "0" if "attn_scores_mm" in x else "" for x in lines).split()
-    assert taken == ["1"] * len(one) + ["0"] * len(three)
+    assert [k[0] for k in chunk_kernels(tmp_path, one + three)] == ["attn_short_mm"] * len(one) + ["attn_scores_mm"] * len(three)
+
+
+def chunk_kernels(tmp_path, shapes):
+    """A shape's attention kernels, one after another."""
+    calls = []
+    for x in launched(tmp_path, SHORT % (shapes,)):
+        if x.startswith("at "):
+            calls.append([])
+        else:
+            calls[-1].append(kernels([x])[0])
+    return [[n + (re.match(r"Li(\d+)E", t).group(1) if n == "attn_values_mm" else "") for n, t in c] for c in calls]
+
+
+def test_a_chunks_attention_on_each_side_of_its_lines(tmp_path):
+    """One launch: groups of 3 to 8 heads, up to 256 workgroups (KV heads x tokens), 256 positions, 448 from 128 workgroups on.  Three: values of
+    a row a wave up to 1,400 waves (rows x KV heads x 64-column parts), of sixteen rows from 1,600 waves on, or fewer where the chunk
+    lies further in than it is long; else of four.  (nh, nkv, hd, first position, tokens.)"""
+    short = ["attn_short_mm"]
+    three = lambda values: ["attn_scores_mm", "attn_softmax", values]
+    row, r4, r16 = three("attn_values_mm_row"), three("attn_values_mm4"), three("attn_values_mm16")
+    for shape, want in {
+            (3, 1, 64, 0, 2): short, (2, 1, 64, 0, 2): row, (8, 1, 64, 0, 2): short, (9, 1, 64, 0, 2): row,
+            (32, 8, 128, 0, 32): short, (32, 8, 128, 0, 33): r4, (12, 4, 128, 0, 64): short, (12, 4, 128, 0, 65): r4,
+            (8, 2, 128, 239, 17): short, (8, 2, 128, 239, 18): row, (14, 2, 64, 193, 63): short, (14, 2, 64, 193, 64): short, (14, 2, 64, 194, 63): row,
+            (32, 8, 128, 432, 16): short, (32, 8, 128, 433, 16): row, (32, 8, 128, 433, 15): row, (16, 4, 128, 416, 32): short, (16, 4, 128, 417, 32): row,
+            # the shapes of test_gpu_model's runs in one launch, and of those with a row and with four rows a wave
+            (12, 4, 128, 61, 3): short, (40, 5, 128, 15, 49): short, (15, 3, 64, 63, 2): short, (24, 4, 64, 412, 36): short, (7, 1, 128, 0, 64): short,
+            (24, 3, 128, 40, 44): short, (10, 2, 128, 80, 16): short, (4, 4, 64, 14, 2): row, (8, 2, 64, 15, 175): row, (8, 2, 64, 15, 176): r4,
+            (10, 2, 128, 507, 6): row, (6, 6, 64, 2047, 3): row, (32, 8, 128, 301, 33): r4, (4, 4, 128, 3, 177): r4, (14, 2, 64, 2, 130): r4,
+            (16, 16, 128, 0, 799): r16, (8, 8, 128, 0, 1584): r4, (8, 8, 128, 0, 1585): r16,
+            (32, 8, 128, 600, 256): r16, (32, 8, 128, 256, 256): r4, (32, 8, 128, 600, 128): r4}.items():
+        assert chunk_kernels(tmp_path, [shape])[0] == want, shape
 
 
 MANY_ROWS = r"""
