@@ -390,7 +390,8 @@ class DenseModel:
 
     def _part(self, n, k):
         """The tokens of one of K parts of N: whole tiles of 128; of 64 for a few hundred through the exact products, whose tiles are
-        also of 32 and 64 tokens (280 tokens 8.5 -> 8.0 ms, 300 9.0 -> 8.1, 350 9.4 -> 9.1, 384 9.46 -> 9.59; 850 18.2 and 18.7)."""
+        also of 32 and 64 tokens (halves of whole tiles of 128 and of 64, the Qwen3-4B shape: 280 tokens 8.6 and 8.3 ms, 300 8.5 and 7.8, 320 8.8 and
+        7.9, 350 8.7 and 8.6, 384 9.0 and 9.4, 400 to 512 the same)."""
         g = 64 if self.prefill == "exact" and n <= 512 else 128
         return ((n + k - 1) // k + g - 1) // g * g
 
@@ -406,17 +407,17 @@ class DenseModel:
             # 62.7; halves of a 512-token chunk lose; their sums' order depends on a launch's token count with or without
             # parts); from resident copies 28.4 -> 27.2 and 62.7 -> 62.1: left whole.
             return self.prefill == "bf16" and 1024 <= n <= self.chunk and work >= 1e10
-        # The exact ones, the Qwen3-4B shape (whole -> halves, ms): 194 tokens 7.3 -> 7.0, 256 7.7 -> 7.1, 300 8.9 -> 8.1, 350 9.5 ->
-        # 9.1, 384 9.9 -> 9.6, 420 11.8 -> 11.1, 512 13.1 -> 11.8, 850 19.7 -> 18.2, 1,000 21.8 -> 21.0, 2,500 76 -> 68; 576 to 768 lose up to
-        # 9 %, 140 to 192 up to 11 %, thirds and quarters always lose to halves.  Far into a conversation a few hundred tokens are mostly
-        # attention, whose launches fill the GPU whole: 512 at 1,500 positions 22.1 -> 23.8, 768 31.1 -> 34.9; 224 14.1 -> 13.0,
-        # 1,024 and more as whole or up to 2 % better.  (Other shapes take these lines and the next as they are: two shapes are
-        # what they were drawn from.)
+        # The exact ones, the Qwen3-4B shape (whole -> halves, ms): 140 tokens 5.4 -> 5.8, 192 5.8 -> 6.2, 194 and 224 as whole, 256 7.4 -> 7.0, 300 7.9 ->
+        # 7.6, 350 8.7 -> 8.4, 420 11.1 -> 9.5, 512 12.0 -> 10.6, 850 19.7 -> 17.2, 1,000 21.8 -> 20.1, 2,500 74 -> 67.5; thirds and quarters always
+        # lose to halves.  Halves of 257 to 288 tokens (280 7.6 -> 7.9) and of 384 (9.0 -> 9.3) lose 3 to 4 %, and 576 to 768 would gain 2 to 5 (700
+        # 15.2 -> 14.5): the lines are older than the products they were drawn with.  Far into a conversation a few hundred tokens are mostly
+        # attention, whose launches fill the GPU whole: at 1,500 positions 512 20.9 -> 20.8, 768 29.7 -> 29.4, 1,500 61.0 -> 61.7; 224 12.9 -> 12.3, 2,048
+        # 89.2 -> 87.6.  (Other shapes take these lines and the next as they are: two shapes are what they were drawn from.)
         if not (n <= 256 or n >= 1024 or self.pos < 1024 and (n >= 800 or n <= 512)):
             return False
         # A small model's launches are over before the next is queued, so twice as many of them only cost (the Qwen2.5-0.5B
-        # shape: 384 tokens 2.8 -> 3.0 ms, 512 3.28 -> 3.15, 1,024 6.7 -> 5.7; at 1,500 positions 1,536 tokens 16.8 -> 18.4,
-        # 2,048 even): a half must bring so many products of a weight and a token to a layer.
+        # shape: 384 tokens 2.34 -> 2.77 ms, 480 2.70 -> 2.76, 512 as whole, 832 4.04 -> 3.94, 1,024 5.1 -> 4.7; at 1,500 positions 1,024
+        # 8.9 -> 8.6, 2,048 16.6 -> 18.7): a half must bring so many products of a weight and a token to a layer.
         return work >= (3.5e9 if self.pos < 1024 else 1.2e10)
 
     def argmax(self):
