@@ -491,12 +491,15 @@ hipError_t ilt_k_attn_scores_mm(const float* q, const float* kc, float* raw, int
 // Sixteen rows a wave once that leaves about six waves a CU (32 heads of 128 over 8 on 512 tokens, 2,048 waves: 95.7 us for the
 // chunk's attention against 97.6 with four; 1,250 at 1,250 893 against 1,102), else four: a wave's chain of positions, an
 // instruction every few cycles, is the launch's time (256 tokens 41 us against 43, 64 tokens 13.9 against 15.5, 14 heads of 64
-// over 2 on 1,250 121 against 137).  Further into a conversation than the chunk is long, where it also has the GPU to itself, sixteen as soon
-// as their chain, 53 ns a position, is over before the four times as many waves of four rows, 19 ns a position each, are through: by how
-// many waves they are and how much of the longest chain their average is (values, us, four and sixteen; 32 heads of 128 over 8: 128
+// over 2 on 1,250 121 against 137).  Further into a conversation than the chunk is long, sixteen as soon as their chain, 53 ns a position, is over
+// before the four times as many waves of four rows, 19 ns a position each, are through: by how many waves they are and how much of the longest chain
+// their average is (values, us, four and sixteen; 32 heads of 128 over 8: 128
 // tokens at 1,900, 502 by this count, 76 and 107; 200 at 1,200, 743, 90 and 78; 300 at 1,700, 1,110, 161 and 139; 380 at 600 87 and 69; 14 of
-// 64 over 2, 700 at 3,000, 556, 173 and 192).  Beside a chunk's other half four rows are better (256 at 256, 768 by this count: the prompt of
-// 512 11.6 ms against 12.1).  One row a wave up to 1,400 waves, a little more than the SIMDs (32 heads of 128 over 8 at 300
+// 64 over 2, 700 at 3,000, 556, 173 and 192).  So also beside a prompt's other half, where it lies as far in (whole prompts, ms, all its halves with four and
+// by this rule: 400 tokens at 600, as 256 and 144, 12.8 and 12.3; 512 at 900 17.3 and 16.2; 400 at 300 11.3 and 11.7); a half no further in than it is long has four
+// (512 at none, its second half 256 at 256, 768 by this count: 10.7 ms, with sixteen 11.0), alone the two are within 5 % there (32 heads of 128 over 8,
+// the chunk's attention: 300 at 200 67.8 us with four, 66.6 with sixteen; 28 over 4, 400 at 300 99.4 and 95.2).  One row a wave up to 1,400 waves, a little more
+// than the SIMDs (32 heads of 128 over 8 at 300
 // positions, 1,344 waves 17.6 us against 18.6, 2,112 21.1 against 19.3; 14 of 64 over 2, 1,400 19.8 against 20.9, 2,800 30.5 against
 // 29.1); its values three sets ahead up to 512 positions, four past them (3 tokens at 2,000: 35.5 against 39.7).
 hipError_t ilt_k_attn_values_mm(const float* prob, const float* vc, float* out, int nh, int nkv, int hd, int pos0, int ntok, int spitch, const IltRowsQuant* to,

@@ -1487,7 +1487,12 @@ hipError_t launch_i8r_group(const BfParams& p, long long total_rows, hipStream_t
 // to lie on the same two SIMDs of a CU: 1.4, then 2.35.)  The chip is taken to be empty: where another stream's launches run beside
 // (the halves of a prompt) a launch takes longer than this says -- down at the Qwen3-4B shape on 256 tokens 49 us here and alone, 60-70 beside the
 // other half -- and the choice is the one for a launch alone, but for the largest tiles, which do the most for an instruction: two on a CU take
-// 5.45 and 5.0 alone, and with those figures here 512 tokens as halves took 11.3 ms instead of 10.6, 2,000 50.1 instead of 48.5.
+// 5.45 and 5.0 alone, and with those figures here 512 tokens as halves take 11.2 ms instead of 10.7, 1,024 21.0 instead of 20.2 (2,048 50.3 instead of 50.5).
+// A product alone pays for that: of 260 random ones of each format (512 to 17,408 rows, 1,024 to 9,728 columns, 96 to 4,096 tokens) the tile taken is 1.3 %
+// (Q6_K 0.8) slower on average than the quickest of them, more than 5 % for 29 (20), at most 10; with 5.0 for both 0.9 (0.7), with 5.45 1.1 (1.3).
+// Of such products from 8 tokens on, 32 x 32 and 32 x 64 are the choice for one in 400 (Q6_K 600), where larger tiles leave most of a round empty (Q4_K 798 x
+// 2304 on 1,257 tokens 17.4 us, with four waves of 16 rows 19.9; 1685 x 8960 on 1,198 75, with 64 x 64 87), 64 x 128 for one in 600 and within 4 % of
+// 64 x 64 there (Q4_K 1085 x 1792 on 3,673 28.9 and 27.7, Q6_K 1284 x 1280 on 3,020 23.7 and 24.0), reg_split2 for one in 1,200 (Q6_K 130).
 struct RegTile { int rows, tokens, fit; float us[2][5]; };
 constexpr RegTile kRegTiles[] = {
   {32, 32, 5, {{1.1f, 1.18f, 1.3f, 1.35f, 2.0f}, {1.4f, 1.5f, 1.65f, 1.8f, 4.0f}}},       // (Q6_K: four fit, a fifth is a second round)
